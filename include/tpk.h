@@ -375,6 +375,16 @@ int tpk_gridding_grad_f64(int b, int n_pts, int n_grid_vertices, const double* g
                           const int32_t* grid_pt_indexes, const double* grad_grid, double* grad_ptcloud,
                           void* stream);
 
+/* The reference's front end gridding(ptcloud, scale) (torch_points_kernels/gridding.py:34-60) for a whole batch:
+ * coordinates times `scale`, grids over [-scale, scale - 1] per axis, points whose three products sum to zero
+ * (padding) left out cloud by cloud.  The gradient takes the same ptcloud and scale (padding: zeros). */
+int tpk_gridding_batch_f32(int b, int n_pts, double scale, const float* ptcloud, float* grid_weights, void* stream);
+int tpk_gridding_batch_f64(int b, int n_pts, double scale, const double* ptcloud, double* grid_weights, void* stream);
+int tpk_gridding_batch_grad_f32(int b, int n_pts, double scale, const float* ptcloud, const float* grad_grid,
+                                float* grad_ptcloud, void* stream);
+int tpk_gridding_batch_grad_f64(int b, int n_pts, double scale, const double* ptcloud, const double* grad_grid,
+                                double* grad_ptcloud, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * Cubic feature sampling (GRNet): the features of the grid vertices around every point.
  * Replaces cubic_feature_sampling_kernel_wrapper(scale, neighborhood_size, ptcloud,

@@ -1211,6 +1211,29 @@ def test_gridding_front_end_and_gradcheck(tpk, oracle, dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+# sums in LDS with one part, many parts, rows that do not divide; more points than its atomics are taken for (global)
+@pytest.mark.parametrize("B,n,scale", [(3, 1, 1), (5, 333, 3), (1, 5000, 16), (2, 700, 33), (1, 9000, 64), (1, 20000, 2)])
+def test_gridding_batch_parity(tpk, oracle, dev, dtype, B, n, scale):
+    g = torch.Generator().manual_seed(n + scale)
+    p = torch.rand(B, n, 3, generator=g, dtype=torch.float64).mul(2.02).sub(1.01).to(dtype)
+    p[0, n // 2 :] = 0  # padding
+    p[:, ::7, 0] = 0.25  # a wall: many points share one plane
+    x = p.to(dev).requires_grad_()
+    grid = tpk.gridding(x, scale)
+    r = torch.randn(B, (2 * scale) ** 3, generator=g, dtype=torch.float64).to(dtype)
+    grad = torch.autograd.grad(grid, x, r.to(dev))[0]
+    tol = 2e-5 if dtype == torch.float32 else 1e-12
+    for b in range(B):
+        q = p[b] * scale
+        kept = (q[:, 0] + q[:, 2]) + q[:, 1] != 0
+        wg, ww, wi = oracle.gridding(q[kept].unsqueeze(0).numpy(), scale)
+        np.testing.assert_allclose(_np(grid)[b], wg[0], rtol=tol, atol=tol * max(1.0, float(np.abs(wg).max())))
+        want = np.zeros((n, 3), p.numpy().dtype)
+        want[kept.numpy()] = oracle.gridding_grad(ww, wi, r[b : b + 1].numpy())[0] * p.numpy().dtype.type(scale)
+        np.testing.assert_array_equal(_np(grad)[b], want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("B,n,c,scale,ns", [(2, 64, 4, 8, 1), (2, 32, 2, 8, 2), (1, 32, 2, 16, 3), (2, 2048, 64, 16, 1), (1, 300, 7, 4, 2)])
 def test_cubic_feature_sampling_parity(tpk, oracle, dev, dtype, B, n, c, scale, ns):
     native = __import__("torch_points_kernels._native", fromlist=["native"]).native()

@@ -525,6 +525,49 @@ at::Tensor gridding_grad(at::Tensor grid_pt_weights, at::Tensor grid_pt_indexes,
     return grad;
 }
 
+// torch_points_kernels/gridding.py:34-60 (the reference's front end, a loop over the clouds there) for the whole
+// batch: one launch forward, one backward (tpk_gridding_batch_f32).
+at::Tensor gridding_batch_forward(const at::Tensor& ptcloud, double scale)
+{
+    check_gpu(ptcloud, "ptcloud");
+    TORCH_CHECK(ptcloud.scalar_type() == at::kFloat || ptcloud.scalar_type() == at::kDouble,
+                "ptcloud must be float32 or float64");
+    TORCH_CHECK(ptcloud.dim() == 3 && ptcloud.size(2) == 3, "ptcloud must have shape (B, n_pts, 3)");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(ptcloud.device());
+    const int b = as_int(ptcloud.size(0), "batch size"), n = as_int(ptcloud.size(1), "number of points");
+    const int64_t side = static_cast<int>(static_cast<float>(scale - 1) - static_cast<float>(-scale) + 1);
+    TORCH_CHECK(side > 0, "gridding: empty grid");
+    at::Tensor grid = at::empty({b, side * side * side}, ptcloud.options());
+    if (ptcloud.scalar_type() == at::kFloat)
+        check_status(tpk_gridding_batch_f32(b, n, scale, ptcloud.data_ptr<float>(), grid.data_ptr<float>(),
+                                            current_stream(ptcloud)),
+                     "gridding");
+    else
+        check_status(tpk_gridding_batch_f64(b, n, scale, ptcloud.data_ptr<double>(), grid.data_ptr<double>(),
+                                            current_stream(ptcloud)),
+                     "gridding");
+    return grid;
+}
+
+at::Tensor gridding_batch_backward(const at::Tensor& ptcloud, double scale, const at::Tensor& grad_grid)
+{
+    check_gpu(grad_grid, "grad_grid");
+    check_same_device(ptcloud, grad_grid, "ptcloud and grad_grid");
+    TORCH_CHECK(grad_grid.scalar_type() == ptcloud.scalar_type(), "grad_grid and ptcloud differ in dtype");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(ptcloud.device());
+    const int b = as_int(ptcloud.size(0), "batch size"), n = as_int(ptcloud.size(1), "number of points");
+    at::Tensor grad = at::empty_like(ptcloud);
+    if (ptcloud.scalar_type() == at::kFloat)
+        check_status(tpk_gridding_batch_grad_f32(b, n, scale, ptcloud.data_ptr<float>(), grad_grid.data_ptr<float>(),
+                                                 grad.data_ptr<float>(), current_stream(ptcloud)),
+                     "gridding_grad");
+    else
+        check_status(tpk_gridding_batch_grad_f64(b, n, scale, ptcloud.data_ptr<double>(), grad_grid.data_ptr<double>(),
+                                                 grad.data_ptr<double>(), current_stream(ptcloud)),
+                     "gridding_grad");
+    return grad;
+}
+
 // cuda/src/cubic_feature_sampling.cpp:4-16 -> {point_features, grid_pt_indexes}
 std::vector<at::Tensor> cubic_feature_sampling(int scale, int neighborhood_size, at::Tensor ptcloud,
                                                at::Tensor cubic_features)
@@ -806,6 +849,8 @@ std::vector<torch::Tensor> chamfer_dist_grad(torch::Tensor xyz1, torch::Tensor x
     return {grad_xyz1, grad_xyz2};
 }
 
+#include "differentiable.h"
+
 } // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
@@ -817,6 +862,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("instance_iou_cuda", &instance_iou_cuda);
     m.def("gridding", &gridding);
     m.def("gridding_grad", &gridding_grad);
+    m.def("gridding_batch", &gridding_batch);
     m.def("cubic_feature_sampling", &cubic_feature_sampling);
     m.def("cubic_feature_sampling_grad", &cubic_feature_sampling_grad);
     m.def("three_interpolate", &three_interpolate);
