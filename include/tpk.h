@@ -326,6 +326,40 @@ int tpk_grow_proximity(int64_t n, int nsample, const int64_t* neighbours, int64_
                        int member_order, int64_t* members, int64_t* starts, int64_t* found,
                        void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same clusters, the reference's member order, for callers that walk on host threads (csrc/grow_walk.h is the
+ * walk): the matrix is cut into pieces that no entry crosses - the components of its entries taken both ways, those
+ * below min_cluster_size dropped - and every piece becomes a compact block of rows.
+ *   tpk_grow_components: found (3, HOST memory) = pieces kept, their points, points of the largest.  Waits for the
+ *     stream once.  Leaves what tpk_grow_rows needs in the workspace (tpk_grow_components_workspace_bytes(n), 256-byte
+ *     aligned; 0 as for tpk_grow_proximity).
+ *   tpk_grow_rows (found[0] > 0): starts (found[0] + 1) int64, first place of every piece and the total;
+ *     positions (found[1]) the point at every place, ascending inside a piece, pieces in the order of their first
+ *     points; rows (found[1], nsample) of uint16 (entry_bytes 2, pieces up to 65536 points) or uint32 (4): entries as
+ *     places inside the piece, in row order, the place itself behind the row's end.  The outputs may lie in device
+ *     memory or in host memory the device can address. */
+size_t tpk_grow_components_workspace_bytes(int64_t n);
+int tpk_grow_components(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, int64_t* found,
+                        void* workspace, size_t workspace_bytes, void* stream);
+int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, void* rows,
+                  int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes, void* stream);
+
+/* region_grow(): the points label by label (ascending, ignored labels left out), inside a label in their order; every
+ * (label, sample) becomes a cloud of its own, so that one packed self query and one growth serve all labels (the
+ * reference loops over them, torch_points_kernels/cluster.py:84-107).
+ *   found (2, HOST memory): points kept; 1 if the outputs were written, 0 if the points already stand in that order
+ *     (one label, none ignored) or none is left.  order (n) int32: the point at every position; pos_out (n, 3);
+ *     ids (n) int64: ascending cloud ids.  batch must be sorted.  At most TPK_REGION_IGNORED ignored labels (HOST
+ *     array), labels spanning less than 2^31 (else TPK_ERR_UNSUPPORTED).  Waits for the stream once.
+ * tpk_region_members: members[i] = order[positions[i]] (order NULL: positions[i]); positions of 4 or 8 bytes, in place
+ * if they are `members`. */
+#define TPK_REGION_IGNORED 32
+size_t tpk_region_order_workspace_bytes(int64_t n);
+int tpk_region_order(int64_t n, const int64_t* labels, const int64_t* batch, const float* pos, int ignored_count,
+                     const int64_t* ignored_labels, int64_t* found, int32_t* order, float* pos_out, int64_t* ids,
+                     void* workspace, size_t workspace_bytes, void* stream);
+int tpk_region_members(int64_t count, const int32_t* order, int position_bytes, const void* positions, int64_t* members,
+                       void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * IoU between proposed instances and ground-truth instances.
  * Replaces instance_iou_kernel_wrapper(total_gt_instances, max_gt_instances, nInstance,

@@ -1087,6 +1087,30 @@ def test_region_grow_parity(tpk, oracle, dev):
         np.testing.assert_array_equal(_np(a), b)
 
 
+@pytest.mark.parametrize("n,kinds,ignored", [(40, 1, []), (3000, 1, []), (3000, 7, [5]), (20000, 40, list(range(0, 60, 3))), (9000, 50, list(range(45)))])
+@pytest.mark.parametrize("spread_labels", [1, 10**10])
+def test_region_grow_all_labels_at_once(tpk, oracle, dev, n, kinds, ignored, spread_labels):
+    """One label (no reordering), labels mixed point by point, more ignored labels than the device takes as values,
+    labels too far apart for sort keys, nothing left, other label types."""
+    from torch_points_kernels.cluster import region_grow
+
+    g = torch.Generator().manual_seed(n + kinds)
+    pos, batch = _blobs(g, 3, n, 0.05)
+    labels = (torch.randint(0, kinds, (pos.shape[0],), generator=g) - 3) * spread_labels
+    ignored = [(v - 3) * spread_labels for v in ignored]
+    for order in ("reference", "index"):
+        want = oracle.region_grow(pos.numpy(), labels.numpy(), batch.numpy(), ignore_labels=ignored, radius=0.06, min_cluster_size=5)
+        got = region_grow(pos.to(dev), labels.to(dev), batch.to(dev), ignored, radius=0.06, min_cluster_size=5, member_order=order)
+        assert len(got) == len(want)
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(_np(a), b if order == "reference" else np.sort(b))
+    if spread_labels == 1:
+        for kind in (torch.int32, torch.float32):
+            other = region_grow(pos.to(dev), labels.to(kind).to(dev), batch.to(dev), ignored, radius=0.06, min_cluster_size=5, member_order=order)
+            assert len(other) == len(got) and all(torch.equal(a, b) for a, b in zip(got, other))
+        assert region_grow(pos.to(dev), labels.to(dev), batch.to(dev), sorted(set(labels.tolist())), radius=0.06) == []
+
+
 def test_grow_proximity_any_matrix(tpk, oracle, dev):
     """Matrices that no ball query produces: rows ending early, entries after a -1 (ignored, the row has ended), chains
     in both directions, points nobody lists, no columns at all."""

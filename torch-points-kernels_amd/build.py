@@ -97,11 +97,12 @@ def build_extension(force=False):
 
     src = os.path.join(CSRC, "points_cuda.cpp")
     out = os.path.join(PKG, "points_cuda.so")
-    deps = [src, os.path.join(CSRC, "differentiable.h"), os.path.join(INCLUDE, "tpk.h")]
+    deps = [src, os.path.join(INCLUDE, "tpk.h")] + [os.path.join(CSRC, h) for h in ("differentiable.h", "grow_walk.h")]
     if not force and _newer(out, deps):
         return out
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+    # -fopenmp: at::parallel_for, which the host half of region growing uses
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-fopenmp",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=points_cuda",
            "-DTORCH_API_INCLUDE_EXTENSION_H",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]

@@ -27,6 +27,12 @@
 //
 // The entry point blocks the host: the number of sweeps and the sizes of the outputs depend on
 // the data.
+//
+// The reference's member order has a second path, tpk_grow_components / tpk_grow_rows, for callers
+// with host threads at hand (the Python layer's): a stack walk is a chain of dependent steps, 0.8 us
+// each on the device (row load, compare-and-swap, stack load: three trips to the L2) and 10-20 ns on
+// a host core whose cache holds the cluster's rows.  The device cuts the problem into pieces that no
+// entry crosses and lays each out as one compact block, the host walks the blocks side by side.
 #include <cstring>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -341,17 +347,169 @@ __global__ void __launch_bounds__(CL_THREADS)
         number[v] = -1;
 }
 
-// Sort keys: the number of the point's cluster, `clusters` for points of dropped clusters.
-__global__ void __launch_bounds__(CL_THREADS)
-    cluster_keys_kernel(int n, int clusters, const int* __restrict__ label, const int* __restrict__ number,
-                        unsigned* keys, unsigned* values)
+// ---- a stable sort by small keys -----------------------------------------------------------------
+// Clusters, pieces and labels are few, and what has to be sorted is point numbers that stand in order: one
+// counting pass over `bins` keys does it - a histogram per block of 2048 points, a prefix sum over
+// (key, block), a placement that keeps the order.  3 launches, 26 us for 300000 points and 150 keys, where the
+// merge sort rocPRIM picks at this size takes 20 launches and 105 us; it stays for more keys than the
+// tables are made for.
+constexpr int CS_WAVES = 4;
+constexpr int CS_STEPS = 8;
+constexpr int CS_BLOCK = CS_WAVES * CS_STEPS * TPK_WAVE;
+constexpr int CS_BINS = 1024;
+constexpr int CS_SCAN_THREADS = 1024;
+constexpr int64_t CS_TABLE = 1 << 18; // (key, block) pairs the one workgroup of the prefix sum goes through
+
+// The number of the point's cluster, `clusters` for points of dropped clusters.
+struct ClusterKeys
+{
+    int clusters;
+    const int* label;
+    const int* number;
+    __device__ __forceinline__ unsigned operator()(int v) const
+    {
+        const int c = number[label[v]];
+        return c < 0 ? (unsigned)clusters : (unsigned)c;
+    }
+};
+
+template <typename Keys>
+__global__ void __launch_bounds__(CS_WAVES * TPK_WAVE) counting_histogram_kernel(int n, int bins, Keys key_of, unsigned* keys, unsigned* table)
+{
+    __shared__ unsigned count[CS_BINS];
+    for (int k = threadIdx.x; k < bins; k += CS_WAVES * TPK_WAVE)
+        count[k] = 0;
+    __syncthreads();
+    const int begin = blockIdx.x * CS_BLOCK;
+    for (int i = begin + threadIdx.x; i < n && i < begin + CS_BLOCK; i += CS_WAVES * TPK_WAVE)
+    {
+        const unsigned k = key_of(i);
+        keys[i] = k;
+        atomicAdd(&count[k], 1u);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < bins; k += CS_WAVES * TPK_WAVE)
+        table[(int64_t)k * gridDim.x + blockIdx.x] = count[k];
+}
+
+// Exclusive prefix sum of the table in place, one workgroup: every thread sums a run of entries, the runs are
+// added up wavefront by wavefront.
+__global__ void __launch_bounds__(CS_SCAN_THREADS) counting_scan_kernel(int entries, unsigned* table)
+{
+    __shared__ int waves[CS_SCAN_THREADS / TPK_WAVE];
+    const int per = (entries + CS_SCAN_THREADS - 1) / CS_SCAN_THREADS;
+    const int begin = min(entries, (int)threadIdx.x * per), end = min(entries, begin + per);
+    int sum = 0;
+    for (int i = begin; i < end; ++i)
+        sum += (int)table[i];
+    int before = wave_exclusive_sum(sum);
+    const int wave = threadIdx.x / TPK_WAVE;
+    if (threadIdx.x % TPK_WAVE == TPK_WAVE - 1)
+        waves[wave] = before + sum;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w)
+        before += waves[w];
+    for (int i = begin; i < end; ++i)
+    {
+        const unsigned c = table[i];
+        table[i] = (unsigned)before;
+        before += (int)c;
+    }
+}
+
+__global__ void __launch_bounds__(CS_WAVES * TPK_WAVE)
+    counting_place_kernel(int n, int bins, int bits, const unsigned* __restrict__ keys, const unsigned* __restrict__ table,
+                          unsigned* __restrict__ keys_out, unsigned* __restrict__ values_out)
+{
+    __shared__ unsigned next[CS_WAVES][CS_BINS];
+    const int wave = threadIdx.x / TPK_WAVE, lane = threadIdx.x % TPK_WAVE;
+    for (int k = threadIdx.x; k < CS_WAVES * CS_BINS; k += CS_WAVES * TPK_WAVE)
+        (&next[0][0])[k] = 0;
+    __syncthreads();
+    const int begin = blockIdx.x * CS_BLOCK + wave * CS_STEPS * TPK_WAVE + lane;
+    unsigned mine[CS_STEPS];
+#pragma unroll
+    for (int step = 0; step < CS_STEPS; ++step)
+    {
+        const int i = begin + step * TPK_WAVE;
+        mine[step] = i < n ? keys[i] : ~0u;
+        if (i < n)
+            atomicAdd(&next[wave][mine[step]], 1u);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < bins; k += CS_WAVES * TPK_WAVE)
+    {
+        unsigned at = table[(int64_t)k * gridDim.x + blockIdx.x];
+        for (int w = 0; w < CS_WAVES; ++w)
+        {
+            const unsigned c = next[w][k];
+            next[w][k] = at;
+            at += c;
+        }
+    }
+    __syncthreads();
+    // a wavefront's steps follow each other, so its counters need no atomics: the lanes of one key take
+    // consecutive places, their last lane moves the counter on
+#pragma unroll
+    for (int step = 0; step < CS_STEPS; ++step)
+    {
+        const int i = begin + step * TPK_WAVE;
+        const unsigned k = mine[step];
+        u64 same = __ballot(i < n);
+        for (int bit = 0; bit < bits; ++bit)
+        {
+            const u64 set = __ballot((k >> bit) & 1u);
+            same &= (k >> bit) & 1u ? set : ~set;
+        }
+        if (i < n)
+        {
+            const unsigned at = next[wave][k] + tpk_prefix_count(same);
+            keys_out[at] = k;
+            values_out[at] = (unsigned)i;
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (i < n && (same >> lane) == 1)
+            next[wave][k] += __builtin_popcountll(same);
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <typename Keys>
+__global__ void __launch_bounds__(CL_THREADS) sort_keys_kernel(int n, Keys key_of, unsigned* keys, unsigned* values)
 {
     const int v = blockIdx.x * CL_THREADS + threadIdx.x;
     if (v >= n)
         return;
-    const int c = number[label[v]];
-    keys[v] = c < 0 ? (unsigned)clusters : (unsigned)c;
+    keys[v] = key_of(v);
     values[v] = (unsigned)v;
+}
+
+struct SortSpace
+{
+    unsigned *keys_in, *keys_out, *values_in, *values_out;
+    void* temp; // at least CS_TABLE entries
+    size_t temp_bytes;
+};
+
+// Point numbers 0 .. n-1 sorted by key_of (values below `bins`), equal keys in ascending order.
+template <typename Keys>
+hipError_t sort_points(int n, unsigned bins, const Keys& key_of, const SortSpace& space, hipStream_t s)
+{
+    const unsigned bits = bins > 1 ? 32u - (unsigned)__builtin_clz(bins - 1) : 1u;
+    const int64_t blocks = tpk_ceil_div(n, CS_BLOCK);
+    if (bins <= (unsigned)CS_BINS && blocks * bins <= CS_TABLE)
+    {
+        unsigned* table = static_cast<unsigned*>(space.temp);
+        counting_histogram_kernel<<<(unsigned)blocks, CS_WAVES * TPK_WAVE, 0, s>>>(n, (int)bins, key_of, space.keys_in, table);
+        counting_scan_kernel<<<1, CS_SCAN_THREADS, 0, s>>>((int)(blocks * bins), table);
+        counting_place_kernel<<<(unsigned)blocks, CS_WAVES * TPK_WAVE, 0, s>>>(n, (int)bins, (int)bits, space.keys_in, table, space.keys_out,
+                                                                                space.values_out);
+        return hipGetLastError();
+    }
+    sort_keys_kernel<<<(unsigned)tpk_ceil_div(n, CL_THREADS), CL_THREADS, 0, s>>>(n, key_of, space.keys_in, space.values_in);
+    size_t temp_size = space.temp_bytes;
+    return rocprim::radix_sort_pairs(space.temp, temp_size, space.keys_in, space.keys_out, space.values_in, space.values_out, (size_t)n,
+                                     0u, bits, s);
 }
 
 __global__ void __launch_bounds__(CL_THREADS) cluster_widen_kernel(int count, const unsigned* __restrict__ values, int64_t* members)
@@ -430,6 +588,324 @@ __global__ void __launch_bounds__(CL_THREADS)
     }
 }
 
+// ---- pieces for the walk on the host ----------------------------------------------------------
+
+// First parents, and the middle and last valid entry of every row for the two rounds of links below.  Rows
+// of an unsorted ball query list ascending indices, so the first entry is the smallest point the row names.
+// A parent is never above its point, so chains end.
+__global__ void __launch_bounds__(CL_THREADS)
+    component_init_kernel(int n, int nsample, const int64_t* __restrict__ neighbours, int* parent, int* picks, int* size, int* largest)
+{
+    const int64_t t = (int64_t)blockIdx.x * CL_THREADS + threadIdx.x;
+    if (t == 0)
+        *largest = 0;
+    const int64_t point = t / CL_ROW_LANES;
+    const int g = (int)(t % CL_ROW_LANES);
+    if (point >= n)
+        return; // the whole group of lanes leaves together
+    const int shift = (int)(tpk_lane_id() & (TPK_WAVE - CL_ROW_LANES)); // first lane of this row's group
+    const int64_t* row = neighbours + point * nsample;
+    int count = 0;
+    for (int first = 0; first < nsample; first += CL_ROW_LANES)
+    {
+        bool row_ends;
+        count += entries_before_end(first + g < nsample ? row[first + g] : -1, shift, &row_ends);
+        if (row_ends)
+            break;
+    }
+    const int v = (int)point;
+    if (g >= 3)
+        return;
+    const int64_t nei = count > 0 ? row[g == 0 ? 0 : g == 1 ? count - 1 : count / 2] : -1;
+    const bool usable = nei >= 0 && nei < n;
+    if (g == 0)
+    {
+        parent[v] = usable && nei < v ? (int)nei : v;
+        size[v] = 0;
+    }
+    else
+        picks[(int64_t)(g - 1) * n + v] = usable ? (int)nei : v;
+}
+
+// Joins the trees of two points: the higher root is hung under the lower by compare-and-swap.  The dies'
+// L2s do not see each other's stores within a kernel, so a root found by plain reads may have been hung
+// meanwhile; it is looked at once more past the caches before the swap is tried, because failing swaps of
+// thousands of entries on one address are what this would otherwise spend its time on.  What is found there
+// is strictly lower, so the loop ends.
+__device__ __forceinline__ void join_trees(int* parent, int a, int b)
+{
+    a = find_root(parent, a);
+    b = find_root(parent, b);
+    while (a != b)
+    {
+        const int high = max(a, b), low = min(a, b);
+        int above = __hip_atomic_load(&parent[high], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (above == high)
+            above = atomicCAS(&parent[high], high, low);
+        if (above == high)
+            return;
+        a = find_root(parent, above);
+        b = low;
+    }
+}
+
+// One entry of every row.
+__global__ void __launch_bounds__(CL_THREADS) component_link_kernel(int n, const int* __restrict__ picks, int* parent)
+{
+    const int u = blockIdx.x * CL_THREADS + threadIdx.x;
+    if (u >= n)
+        return;
+    const int nei = picks[u];
+    if (parent[nei] != parent[u])
+        join_trees(parent, u, nei);
+}
+
+// Every entry joins the trees of its two points, whatever its direction.  The rounds before have left one
+// tree for most of every component and flattened it, so for nearly all entries this is one comparison of
+// two parents.
+__global__ void __launch_bounds__(CL_THREADS)
+    component_join_kernel(int n, int nsample, const int64_t* __restrict__ neighbours, int* parent)
+{
+    const int64_t t = (int64_t)blockIdx.x * CL_THREADS + threadIdx.x;
+    const int64_t point = t / CL_ROW_LANES;
+    const int g = (int)(t % CL_ROW_LANES);
+    if (point >= n)
+        return; // the whole group of lanes leaves together
+    const int u = (int)point;
+    const int shift = (int)(tpk_lane_id() & (TPK_WAVE - CL_ROW_LANES)); // first lane of this row's group
+    const int mine = parent[u];
+    for (int first = 0; first < nsample; first += CL_ROW_LANES)
+    {
+        const int j = first + g;
+        const int64_t nei = j < nsample ? neighbours[(int64_t)u * nsample + j] : -1;
+        bool row_ends;
+        const int valid = entries_before_end(nei, shift, &row_ends);
+        if (g < valid && nei >= 0 && nei < n && nei != u && parent[nei] != mine)
+            join_trees(parent, u, (int)nei);
+        if (row_ends)
+            break;
+    }
+}
+
+// Every point directly under its root (stores of other threads only move a point further up).
+__global__ void __launch_bounds__(CL_THREADS) component_flatten_kernel(int n, int* parent)
+{
+    const int v = blockIdx.x * CL_THREADS + threadIdx.x;
+    if (v >= n)
+        return;
+    const int root = find_root(parent, v);
+    if (root < parent[v])
+        parent[v] = root;
+}
+
+// The root of every point, and the points per root.  Neighbouring points share few roots, so the counts are
+// gathered in LDS first (a small open table; what finds no place there is added outside): device-scope atomics
+// on one address pass one at a time.
+constexpr int CL_ROOT_THREADS = 1024;
+constexpr int CL_ROOT_POINTS = 4 * CL_ROOT_THREADS; // per workgroup
+constexpr int CL_ROOT_SLOTS = 512;
+
+__global__ void __launch_bounds__(CL_ROOT_THREADS)
+    component_roots_kernel(int n, const int* __restrict__ parent, int* __restrict__ root, int* size)
+{
+    __shared__ int slot_root[CL_ROOT_SLOTS], slot_count[CL_ROOT_SLOTS];
+    for (int i = threadIdx.x; i < CL_ROOT_SLOTS; i += CL_ROOT_THREADS)
+    {
+        slot_root[i] = -1;
+        slot_count[i] = 0;
+    }
+    __syncthreads();
+    const int begin = blockIdx.x * CL_ROOT_POINTS + threadIdx.x;
+    for (int v = begin; v < n && v < begin + CL_ROOT_POINTS; v += CL_ROOT_THREADS)
+    {
+        const int r = find_root(parent, v);
+        root[v] = r;
+        bool counted = false;
+        for (int probe = 0; probe < 4 && !counted; ++probe)
+        {
+            const int slot = (int)((unsigned)r * 0x9E3779B1u >> 23) + probe & (CL_ROOT_SLOTS - 1);
+            int holds = slot_root[slot];
+            if (holds == -1)
+                holds = atomicCAS(&slot_root[slot], -1, r);
+            if (holds == -1 || holds == r)
+            {
+                atomicAdd(&slot_count[slot], 1);
+                counted = true;
+            }
+        }
+        if (!counted)
+            atomicAdd(&size[r], 1);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < CL_ROOT_SLOTS; i += CL_ROOT_THREADS)
+        if (slot_count[i] > 0)
+            atomicAdd(&size[slot_root[i]], slot_count[i]);
+}
+
+// cluster_kept_kernel's scan input, and the size of the largest piece.
+__global__ void __launch_bounds__(CL_THREADS)
+    component_kept_kernel(int n, int min_size, const int* __restrict__ root, const int* __restrict__ size, u64* packed, int* largest)
+{
+    const int v = blockIdx.x * CL_THREADS + threadIdx.x;
+    if (v > n)
+        return;
+    u64 p = 0;
+    if (v < n && root[v] == v && size[v] >= min_size)
+    {
+        p = ((u64)1 << 32) | (unsigned)size[v];
+        atomicMax(largest, size[v]);
+    }
+    packed[v] = p;
+}
+
+// info = {pieces, points in them, largest piece}
+__global__ void component_info_kernel(int n, const u64* __restrict__ scanned, const int* __restrict__ largest, int64_t* info)
+{
+    info[0] = (int64_t)(scanned[n] >> 32);
+    info[1] = (int64_t)(scanned[n] & 0xffffffffu);
+    info[2] = *largest;
+}
+
+__global__ void __launch_bounds__(CL_THREADS)
+    component_places_kernel(int count, const unsigned* __restrict__ values, int* place, int32_t* positions)
+{
+    const int i = blockIdx.x * CL_THREADS + threadIdx.x;
+    if (i >= count)
+        return;
+    const int v = (int)values[i];
+    place[v] = i;
+    positions[i] = v;
+}
+
+// Row i: the entries of the point at place i, as places inside its piece; what lies behind the row's end,
+// or outside the matrix, becomes the point itself, which the walk has always seen already - so it needs no
+// test for the end of a row.
+template <typename E>
+__global__ void __launch_bounds__(CL_THREADS)
+    component_rows_kernel(int n, int count, int nsample, const int64_t* __restrict__ neighbours, const unsigned* __restrict__ values,
+                          const unsigned* __restrict__ keys, const int64_t* __restrict__ starts, const int* __restrict__ place, E* rows)
+{
+    const int64_t t = (int64_t)blockIdx.x * CL_THREADS + threadIdx.x;
+    const int64_t slot = t / CL_ROW_LANES;
+    const int g = (int)(t % CL_ROW_LANES);
+    if (slot >= count)
+        return; // the whole group of lanes leaves together
+    const int shift = (int)(tpk_lane_id() & (TPK_WAVE - CL_ROW_LANES));
+    const int64_t u = values[slot];
+    const int base = (int)starts[keys[slot]];
+    bool ended = false;
+    for (int first = 0; first < nsample; first += CL_ROW_LANES)
+    {
+        const int j = first + g;
+        const int64_t nei = j < nsample ? neighbours[u * nsample + j] : -1;
+        bool row_ends;
+        const int valid = entries_before_end(nei, shift, &row_ends);
+        int entry = (int)slot;
+        if (!ended && g < valid && nei >= 0 && nei < n)
+            entry = place[nei];
+        if (j < nsample)
+            rows[slot * nsample + j] = (E)(entry - base);
+        ended |= row_ends;
+    }
+}
+
+// ---- the points of a labelled cloud, label by label ---------------------------------------------
+
+constexpr int RG_RANGE_BLOCKS = 128;
+
+struct Ignored
+{
+    int count;
+    int64_t value[TPK_REGION_IGNORED];
+};
+
+struct LabelRange
+{
+    int64_t low, high, kept;
+};
+
+__device__ __forceinline__ bool is_ignored(const Ignored& ignored, int64_t label)
+{
+    for (int i = 0; i < ignored.count; ++i)
+        if (ignored.value[i] == label)
+            return true;
+    return false;
+}
+
+// Smallest and largest label that is not ignored and how many points carry one, per block.
+__global__ void __launch_bounds__(CL_THREADS)
+    region_range_kernel(int n, const int64_t* __restrict__ labels, Ignored ignored, LabelRange* ranges)
+{
+    __shared__ LabelRange shared[CL_THREADS];
+    LabelRange r{INT64_MAX, INT64_MIN, 0};
+    for (int i = blockIdx.x * CL_THREADS + threadIdx.x; i < n; i += RG_RANGE_BLOCKS * CL_THREADS)
+    {
+        const int64_t label = labels[i];
+        if (is_ignored(ignored, label))
+            continue;
+        r.low = min(r.low, label);
+        r.high = max(r.high, label);
+        r.kept += 1;
+    }
+    shared[threadIdx.x] = r;
+    for (int half = CL_THREADS / 2; half > 0; half /= 2)
+    {
+        __syncthreads();
+        if ((int)threadIdx.x < half)
+        {
+            LabelRange& a = shared[threadIdx.x];
+            const LabelRange& b = shared[threadIdx.x + half];
+            a.low = min(a.low, b.low);
+            a.high = max(a.high, b.high);
+            a.kept += b.kept;
+        }
+    }
+    if (threadIdx.x == 0)
+        ranges[blockIdx.x] = shared[0];
+}
+
+struct RegionKeys
+{
+    int64_t low;
+    unsigned beyond; // key of the points left out
+    const int64_t* labels;
+    Ignored ignored;
+    __device__ __forceinline__ unsigned operator()(int i) const
+    {
+        const int64_t label = labels[i];
+        return is_ignored(ignored, label) ? beyond : (unsigned)(label - low);
+    }
+};
+
+// Points of one label and one sample form a cloud; its id grows with (label, sample), which is the order
+// the rows stand in.
+__global__ void __launch_bounds__(CL_THREADS)
+    region_gather_kernel(int n, int kept, const unsigned* __restrict__ keys, const unsigned* __restrict__ values,
+                         const int64_t* __restrict__ batch, const float* __restrict__ pos, int32_t* order, float* pos_out, int64_t* ids)
+{
+    const int i = blockIdx.x * CL_THREADS + threadIdx.x;
+    if (i >= kept)
+        return;
+    const int64_t first = batch[0], span = batch[n - 1] - first + 1;
+    const int64_t v = values[i];
+    order[i] = (int32_t)v;
+    ids[i] = (int64_t)keys[i] * span + (batch[v] - first);
+    pos_out[(int64_t)i * 3 + 0] = pos[v * 3 + 0];
+    pos_out[(int64_t)i * 3 + 1] = pos[v * 3 + 1];
+    pos_out[(int64_t)i * 3 + 2] = pos[v * 3 + 2];
+}
+
+template <typename P>
+__global__ void __launch_bounds__(CL_THREADS)
+    region_members_kernel(int64_t count, const int32_t* __restrict__ order, const P* positions, int64_t* members)
+{
+    const int64_t i = (int64_t)blockIdx.x * CL_THREADS + threadIdx.x;
+    if (i >= count)
+        return;
+    const int64_t p = (int64_t)positions[i];
+    members[i] = order ? (int64_t)order[p] : p;
+}
+
 struct Layout
 {
     size_t parent, mutual, label, size, number, seeds, stack, keys_in, keys_out, values_in, values_out, packed, scanned, changed,
@@ -459,6 +935,8 @@ bool temp_bytes(int64_t n, size_t* bytes)
     if (rocprim::radix_sort_pairs(nullptr, sort, p32, p32, p32, p32, (size_t)n, 0u, 32u) != hipSuccess)
         return false;
     *bytes = scan > sort ? scan : sort;
+    if (*bytes < CS_TABLE * sizeof(unsigned))
+        *bytes = CS_TABLE * sizeof(unsigned);
     return true;
 }
 
@@ -494,7 +972,243 @@ bool layout(int64_t n, int nsample, Layout* l)
     return true;
 }
 
+struct ComponentLayout
+{
+    size_t parent, root, size, number, seeds, keys_in, keys_out, values_in, values_out, packed, scanned, starts, largest, info, temp,
+        temp_bytes, total;
+};
+
+bool component_layout(int64_t n, ComponentLayout* l)
+{
+    size_t temp = 0;
+    if (!temp_bytes(n, &temp))
+        return false;
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t here = at;
+        at += aligned(bytes);
+        return here;
+    };
+    const size_t ints = (size_t)n * 4;
+    l->parent = take(ints);
+    l->root = take(ints);
+    l->size = take(ints);
+    l->number = take(ints);
+    l->seeds = take(ints);
+    l->keys_in = take(ints);
+    l->keys_out = take(ints);
+    l->values_in = take(ints);
+    l->values_out = take(ints);
+    l->packed = take(((size_t)n + 1) * 8);
+    l->scanned = take(((size_t)n + 1) * 8);
+    l->starts = take(((size_t)n + 1) * 8);
+    l->largest = take(4);
+    l->info = take(24);
+    l->temp = take(temp);
+    l->temp_bytes = temp;
+    l->total = at;
+    return true;
+}
+
+struct RegionLayout
+{
+    size_t keys_in, keys_out, values_in, values_out, ranges, temp, temp_bytes, total;
+};
+
+bool region_layout(int64_t n, RegionLayout* l)
+{
+    size_t temp = 0;
+    if (!temp_bytes(n, &temp))
+        return false;
+    const size_t ints = aligned((size_t)n * 4);
+    l->keys_in = 0;
+    l->keys_out = ints;
+    l->values_in = 2 * ints;
+    l->values_out = 3 * ints;
+    l->ranges = 4 * ints;
+    l->temp = l->ranges + aligned(RG_RANGE_BLOCKS * sizeof(LabelRange));
+    l->temp_bytes = temp;
+    l->total = l->temp + aligned(temp);
+    return true;
+}
+
 } // namespace
+
+extern "C" size_t tpk_grow_components_workspace_bytes(int64_t n)
+{
+    ComponentLayout l;
+    if (n <= 0 || n > CL_MAX_POINTS || !component_layout(n, &l))
+        return 0;
+    return l.total;
+}
+
+extern "C" int tpk_grow_components(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, int64_t* found,
+                                   void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (n <= 0 || nsample <= 0 || !found || !neighbours)
+        return TPK_ERR_INVALID_ARG;
+    if (n > CL_MAX_POINTS)
+        return TPK_ERR_UNSUPPORTED;
+    ComponentLayout l;
+    if (!component_layout(n, &l))
+        return TPK_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0)
+        return TPK_ERR_WORKSPACE;
+    hipStream_t s = tpk_stream(stream);
+    char* ws = static_cast<char*>(workspace);
+    int* parent = reinterpret_cast<int*>(ws + l.parent);
+    int* root = reinterpret_cast<int*>(ws + l.root);
+    int* size = reinterpret_cast<int*>(ws + l.size);
+    int* number = reinterpret_cast<int*>(ws + l.number);
+    unsigned* keys_in = reinterpret_cast<unsigned*>(ws + l.keys_in);
+    unsigned* keys_out = reinterpret_cast<unsigned*>(ws + l.keys_out);
+    unsigned* values_in = reinterpret_cast<unsigned*>(ws + l.values_in);
+    unsigned* values_out = reinterpret_cast<unsigned*>(ws + l.values_out);
+    u64* packed = reinterpret_cast<u64*>(ws + l.packed);
+    u64* scanned = reinterpret_cast<u64*>(ws + l.scanned);
+    int64_t* starts = reinterpret_cast<int64_t*>(ws + l.starts);
+    int* largest = reinterpret_cast<int*>(ws + l.largest);
+    int64_t* info = reinterpret_cast<int64_t*>(ws + l.info);
+    const int ni = (int)n;
+    const unsigned blocks = (unsigned)tpk_ceil_div(n, CL_THREADS);
+    const unsigned blocks1 = (unsigned)tpk_ceil_div(n + 1, CL_THREADS);
+    const unsigned row_blocks = (unsigned)tpk_ceil_div(n * CL_ROW_LANES, CL_THREADS);
+    const int min_size = (int)(min_cluster_size > n ? n + 1 : (min_cluster_size < 1 ? 1 : min_cluster_size));
+    int* picks = reinterpret_cast<int*>(ws + l.packed); // (2 n ints; the counts come later)
+    component_init_kernel<<<row_blocks, CL_THREADS, 0, s>>>(ni, nsample, neighbours, parent, picks, size, largest);
+    component_flatten_kernel<<<blocks, CL_THREADS, 0, s>>>(ni, parent);
+    for (int round = 0; round < 2; ++round)
+    {
+        component_link_kernel<<<blocks, CL_THREADS, 0, s>>>(ni, picks + (size_t)round * n, parent);
+        component_flatten_kernel<<<blocks, CL_THREADS, 0, s>>>(ni, parent);
+    }
+    component_join_kernel<<<row_blocks, CL_THREADS, 0, s>>>(ni, nsample, neighbours, parent);
+    component_roots_kernel<<<(unsigned)tpk_ceil_div(n, CL_ROOT_POINTS), CL_ROOT_THREADS, 0, s>>>(ni, parent, root, size);
+    component_kept_kernel<<<blocks1, CL_THREADS, 0, s>>>(ni, min_size, root, size, packed, largest);
+    size_t temp_size = l.temp_bytes;
+    hipError_t e = rocprim::exclusive_scan(ws + l.temp, temp_size, packed, scanned, (u64)0, (size_t)n + 1, rocprim::plus<u64>(), s);
+    if (e != hipSuccess)
+        return (int)e;
+    component_info_kernel<<<1, 1, 0, s>>>(ni, scanned, largest, info);
+    cluster_describe_kernel<<<blocks1, CL_THREADS, 0, s>>>(ni, packed, scanned, number, reinterpret_cast<int*>(ws + l.seeds), starts);
+    e = static_cast<hipError_t>(tpk_read_back(found, info, 24, s));
+    if (e != hipSuccess || found[0] == 0)
+        return (int)e;
+    e = sort_points(ni, (unsigned)found[0] + 1u, ClusterKeys{(int)found[0], root, number},
+                    SortSpace{keys_in, keys_out, values_in, values_out, ws + l.temp, l.temp_bytes}, s);
+    return e != hipSuccess ? (int)e : tpk_launch_status();
+}
+
+extern "C" int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, void* rows,
+                             int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (n <= 0 || n > CL_MAX_POINTS || nsample <= 0 || !neighbours || !found || !rows || !positions || !starts || found[0] < 1 ||
+        found[1] < 1 || found[1] > n || (entry_bytes != 2 && entry_bytes != 4) || (entry_bytes == 2 && found[2] > 65536))
+        return TPK_ERR_INVALID_ARG;
+    ComponentLayout l;
+    if (!component_layout(n, &l))
+        return TPK_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0)
+        return TPK_ERR_WORKSPACE;
+    hipStream_t s = tpk_stream(stream);
+    char* ws = static_cast<char*>(workspace);
+    const unsigned* keys = reinterpret_cast<const unsigned*>(ws + l.keys_out);
+    const unsigned* values = reinterpret_cast<const unsigned*>(ws + l.values_out);
+    int* place = reinterpret_cast<int*>(ws + l.parent); // (the trees are done with)
+    const int count = (int)found[1];
+    const unsigned blocks = (unsigned)tpk_ceil_div(count, CL_THREADS);
+    const unsigned row_blocks = (unsigned)tpk_ceil_div((int64_t)count * CL_ROW_LANES, CL_THREADS);
+    component_places_kernel<<<blocks, CL_THREADS, 0, s>>>(count, values, place, positions);
+    const int64_t* from = reinterpret_cast<const int64_t*>(ws + l.starts);
+    if (entry_bytes == 2)
+        component_rows_kernel<uint16_t><<<row_blocks, CL_THREADS, 0, s>>>((int)n, count, nsample, neighbours, values, keys, from, place,
+                                                                           static_cast<uint16_t*>(rows));
+    else
+        component_rows_kernel<uint32_t><<<row_blocks, CL_THREADS, 0, s>>>((int)n, count, nsample, neighbours, values, keys, from, place,
+                                                                           static_cast<uint32_t*>(rows));
+    const hipError_t e = hipMemcpyAsync(starts, from, (size_t)(found[0] + 1) * 8, hipMemcpyDefault, s);
+    return e != hipSuccess ? (int)e : tpk_launch_status();
+}
+
+extern "C" size_t tpk_region_order_workspace_bytes(int64_t n)
+{
+    RegionLayout l;
+    if (n <= 0 || n > CL_MAX_POINTS || !region_layout(n, &l))
+        return 0;
+    return l.total;
+}
+
+extern "C" int tpk_region_order(int64_t n, const int64_t* labels, const int64_t* batch, const float* pos, int ignored_count,
+                                const int64_t* ignored_labels, int64_t* found, int32_t* order, float* pos_out, int64_t* ids,
+                                void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (n <= 0 || !labels || !batch || !pos || !found || !order || !pos_out || !ids || ignored_count < 0 ||
+        ignored_count > TPK_REGION_IGNORED || (ignored_count > 0 && !ignored_labels))
+        return TPK_ERR_INVALID_ARG;
+    if (n > CL_MAX_POINTS)
+        return TPK_ERR_UNSUPPORTED;
+    RegionLayout l;
+    if (!region_layout(n, &l))
+        return TPK_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0)
+        return TPK_ERR_WORKSPACE;
+    hipStream_t s = tpk_stream(stream);
+    char* ws = static_cast<char*>(workspace);
+    Ignored ignored{};
+    ignored.count = ignored_count;
+    for (int i = 0; i < ignored_count; ++i)
+        ignored.value[i] = ignored_labels[i];
+    LabelRange* ranges = reinterpret_cast<LabelRange*>(ws + l.ranges);
+    region_range_kernel<<<RG_RANGE_BLOCKS, CL_THREADS, 0, s>>>((int)n, labels, ignored, ranges);
+    LabelRange host[RG_RANGE_BLOCKS], all{INT64_MAX, INT64_MIN, 0};
+    hipError_t e = static_cast<hipError_t>(tpk_read_back(host, ranges, sizeof(host), s));
+    if (e != hipSuccess)
+        return (int)e;
+    for (const LabelRange& r : host)
+    {
+        all.low = r.low < all.low ? r.low : all.low;
+        all.high = r.high > all.high ? r.high : all.high;
+        all.kept += r.kept;
+    }
+    found[0] = all.kept;
+    found[1] = 0;
+    if (all.kept == 0)
+        return TPK_OK;
+    if (all.low == all.high && all.kept == n)
+        return TPK_OK; // one label: the points stand in their order already
+    if ((uint64_t)all.high - (uint64_t)all.low >= (uint64_t)0x7fffffff)
+        return TPK_ERR_UNSUPPORTED;
+    unsigned* keys_in = reinterpret_cast<unsigned*>(ws + l.keys_in);
+    unsigned* keys_out = reinterpret_cast<unsigned*>(ws + l.keys_out);
+    unsigned* values_in = reinterpret_cast<unsigned*>(ws + l.values_in);
+    unsigned* values_out = reinterpret_cast<unsigned*>(ws + l.values_out);
+    const unsigned beyond = (unsigned)(all.high - all.low) + 1u;
+    e = sort_points((int)n, beyond + 1u, RegionKeys{all.low, beyond, labels, ignored},
+                    SortSpace{keys_in, keys_out, values_in, values_out, ws + l.temp, l.temp_bytes}, s);
+    if (e != hipSuccess)
+        return (int)e;
+    region_gather_kernel<<<(unsigned)tpk_ceil_div(all.kept, CL_THREADS), CL_THREADS, 0, s>>>((int)n, (int)all.kept, keys_out, values_out,
+                                                                                             batch, pos, order, pos_out, ids);
+    found[1] = 1;
+    return tpk_launch_status();
+}
+
+extern "C" int tpk_region_members(int64_t count, const int32_t* order, int position_bytes, const void* positions, int64_t* members,
+                                  void* stream)
+{
+    if (count < 0 || (position_bytes != 4 && position_bytes != 8))
+        return TPK_ERR_INVALID_ARG;
+    if (count == 0)
+        return TPK_OK;
+    if (!positions || !members)
+        return TPK_ERR_INVALID_ARG;
+    const unsigned blocks = (unsigned)tpk_ceil_div(count, CL_THREADS);
+    if (position_bytes == 4)
+        region_members_kernel<int32_t><<<blocks, CL_THREADS, 0, tpk_stream(stream)>>>(count, order, static_cast<const int32_t*>(positions), members);
+    else
+        region_members_kernel<int64_t><<<blocks, CL_THREADS, 0, tpk_stream(stream)>>>(count, order, static_cast<const int64_t*>(positions), members);
+    return tpk_launch_status();
+}
 
 extern "C" size_t tpk_grow_proximity_workspace_bytes(int64_t n, int nsample)
 {
@@ -598,10 +1312,8 @@ extern "C" int tpk_grow_proximity(int64_t n, int nsample, const int64_t* neighbo
         return tpk_launch_status();
     if (member_order == TPK_MEMBERS_BY_INDEX)
     {
-        cluster_keys_kernel<<<blocks, CL_THREADS, 0, s>>>(ni, clusters, label, number, keys_in, values_in);
-        const unsigned bits = 32u - (unsigned)__builtin_clz((unsigned)clusters);
-        temp_size = l.temp_bytes;
-        e = rocprim::radix_sort_pairs(temp, temp_size, keys_in, keys_out, values_in, values_out, (size_t)n, 0u, bits, s);
+        e = sort_points(ni, (unsigned)clusters + 1u, ClusterKeys{clusters, label, number},
+                        SortSpace{keys_in, keys_out, values_in, values_out, temp, l.temp_bytes}, s);
         if (e != hipSuccess)
             return (int)e;
         cluster_widen_kernel<<<(unsigned)tpk_ceil_div(kept_points, CL_THREADS), CL_THREADS, 0, s>>>(kept_points, values_out, members);

@@ -1,0 +1,93 @@
+// The reference's stack walk (torch_points_kernels/cluster.py:9-37) on host threads, over the compact pieces that
+// tpk_grow_rows lays out: a piece is a block of rows whose entries are places inside the piece, so a core's cache holds
+// what its walk touches, and pieces are independent of each other.
+//
+// A step takes a point off the stack and collects which of its row's entries are unseen in a bit mask, 16 entries at a
+// time and without a branch; what is left to do per set bit happens once per point in all.  (Writing every entry to the
+// stack and the cluster and moving their ends on only for unseen ones has no branch at all, but 48 stores a step:
+// 14 ns per point against 7.)  The same step takes 0.8 us on the device.
+#pragma once
+
+#include <cstdint>
+#include <cstring>
+#include <vector>
+
+namespace grow_walk {
+
+// A cluster as the walk left it: its first point (the order clusters are numbered by) and its members in `places`.
+struct Cluster
+{
+    int32_t first_position;
+    int64_t at, size;
+};
+
+struct Scratch
+{
+    std::vector<uint8_t> unseen;
+    std::vector<uint32_t> stack, members;
+};
+
+// Walks one piece of `count` points.  Clusters of at least min_size members go to `found`, their members - as
+// positions - to places[at ...], which never takes more than the piece's own range.
+template <typename E>
+void walk_piece(const E* rows, int nsample, const int32_t* positions, int64_t base, int64_t count, int64_t min_size,
+                Scratch& scratch, int32_t* places, std::vector<Cluster>& found)
+{
+    // The rows have just arrived from the device and lie in no cache: read once in order they come at memory speed,
+    // where the walk itself would wait for them one line at a time.
+    const char* first_row = reinterpret_cast<const char*>(rows);
+    uint64_t touched = 0;
+    for (int64_t at = 0; at < count * nsample * static_cast<int64_t>(sizeof(E)); at += 64)
+        touched += static_cast<unsigned char>(first_row[at]);
+    asm volatile("" : : "r"(touched));
+    scratch.unseen.assign(static_cast<size_t>(count), 1);
+    if (scratch.stack.size() < static_cast<size_t>(count))
+    {
+        scratch.stack.resize(static_cast<size_t>(count));
+        scratch.members.resize(static_cast<size_t>(count));
+    }
+    uint8_t* unseen = scratch.unseen.data();
+    uint32_t* stack = scratch.stack.data();
+    uint32_t* members = scratch.members.data();
+    int64_t written = base;
+    for (int64_t seed = 0; seed < count; ++seed)
+    {
+        if (!unseen[seed])
+            continue;
+        unseen[seed] = 0;
+        members[0] = static_cast<uint32_t>(seed);
+        stack[0] = static_cast<uint32_t>(seed);
+        int64_t size = 1, top = 1;
+        while (top > 0)
+        {
+            const E* row = rows + static_cast<int64_t>(stack[--top]) * nsample;
+            for (int first = 0; first < nsample; first += 16)
+            {
+                uint32_t fresh = 0;
+                if (first + 16 <= nsample)
+                    for (int j = 0; j < 16; ++j)
+                        fresh |= static_cast<uint32_t>(unseen[row[first + j]]) << j;
+                else
+                    for (int j = 0; first + j < nsample; ++j)
+                        fresh |= static_cast<uint32_t>(unseen[row[first + j]]) << j;
+                for (; fresh != 0; fresh &= fresh - 1)
+                {
+                    const uint32_t e = row[first + __builtin_ctz(fresh)];
+                    if (!unseen[e])
+                        continue; // (the row has named it twice)
+                    unseen[e] = 0;
+                    stack[top++] = e;
+                    members[size++] = e;
+                }
+            }
+        }
+        if (size < min_size)
+            continue;
+        for (int64_t i = 0; i < size; ++i)
+            places[written + i] = positions[members[i]];
+        found.push_back(Cluster{positions[seed], written, size});
+        written += size;
+    }
+}
+
+} // namespace grow_walk

@@ -6,13 +6,18 @@
 // no kernels and no CPU implementation: without a GPU tensor it raises.
 #include <torch/extension.h>
 
+#include <ATen/Parallel.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <algorithm>
+#include <atomic>
+#include <tuple>
 #include <utility>
 #include <vector>
 
 #include "../../include/tpk.h"
+#include "grow_walk.h"
 
 namespace {
 
@@ -156,6 +161,111 @@ std::pair<at::Tensor, at::Tensor> dense_knn(at::Tensor support, at::Tensor query
     return std::make_pair(idx, dist2);
 }
 
+// Host memory the device can address (torch's pool of such blocks: a block given back is reused by the next call).
+at::Tensor pinned(int64_t bytes)
+{
+    return at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+}
+
+// Clusters in the reference's member order: pieces from the device, walked on host threads.  members: one tensor on the
+// device, clusters one after the other, as indices (order: what tpk_region_order put at every position; may be
+// undefined); sizes: theirs.
+template <typename E>
+void walk_pieces(const E* rows, int nsample, const int32_t* positions, const int64_t* starts, int64_t pieces, int64_t points,
+                 int64_t min_cluster_size, int32_t* places, int32_t* members, std::vector<int64_t>* sizes)
+{
+    std::vector<int64_t> turn(static_cast<size_t>(pieces));
+    for (int64_t p = 0; p < pieces; ++p)
+        turn[p] = p;
+    // the longest walks first: the end of the last one is what the caller waits for
+    std::stable_sort(turn.begin(), turn.end(), [&](int64_t a, int64_t b) { return starts[a + 1] - starts[a] > starts[b + 1] - starts[b]; });
+    // (below 16384 points the walk takes less time than waking the other threads)
+    const int64_t threads = points < 16384 ? 1 : std::min<int64_t>(at::get_num_threads(), pieces);
+    std::vector<std::vector<grow_walk::Cluster>> found(static_cast<size_t>(threads));
+    std::atomic<int64_t> next{0};
+    auto work = [&](int64_t t) {
+        grow_walk::Scratch scratch;
+        for (int64_t i = next.fetch_add(1); i < pieces; i = next.fetch_add(1))
+        {
+            const int64_t base = starts[turn[i]], count = starts[turn[i] + 1] - base;
+            grow_walk::walk_piece(rows + base * nsample, nsample, positions + base, base, count, min_cluster_size, scratch,
+                                  places, found[t]);
+        }
+    };
+    if (threads == 1)
+        work(0);
+    else
+        at::parallel_for(0, threads, 1, [&](int64_t begin, int64_t end) {
+            for (int64_t t = begin; t < end; ++t)
+                work(t);
+        });
+    std::vector<grow_walk::Cluster> all;
+    for (const auto& f : found)
+        all.insert(all.end(), f.begin(), f.end());
+    std::sort(all.begin(), all.end(), [](const grow_walk::Cluster& a, const grow_walk::Cluster& b) { return a.first_position < b.first_position; });
+    sizes->clear();
+    for (const grow_walk::Cluster& c : all)
+    {
+        std::memcpy(members, places + c.at, static_cast<size_t>(c.size) * sizeof(int32_t));
+        members += c.size;
+        sizes->push_back(c.size);
+    }
+}
+
+at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluster_size, const at::Tensor& order,
+                                std::vector<int64_t>* sizes)
+{
+    const int64_t n = neighbours.size(0);
+    const int nsample = as_int(neighbours.size(1), "nsample");
+    auto bytes_on_device = at::device(neighbours.device()).dtype(at::kByte);
+    auto longs = at::device(neighbours.device()).dtype(at::kLong);
+    void* stream = current_stream(neighbours);
+    sizes->clear();
+    const size_t ws_bytes = tpk_grow_components_workspace_bytes(n);
+    TORCH_CHECK(ws_bytes > 0, "grow_proximity: too many points");
+    at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes)}, bytes_on_device);
+    int64_t found[3] = {0, 0, 0};
+    check_status(tpk_grow_components(n, nsample, neighbours.data_ptr<int64_t>(), min_cluster_size, found, ws.data_ptr(), ws_bytes,
+                                     stream),
+                 "grow_proximity (components)");
+    const int64_t pieces = found[0], points = found[1];
+    if (pieces == 0)
+        return at::empty({0}, longs);
+    const int64_t entry = found[2] <= 65536 ? 2 : 4;
+    // one block for all three: starts, positions, rows
+    const int64_t at_positions = (pieces + 1) * 8, at_rows = (at_positions + points * 4 + 15) / 16 * 16;
+    at::Tensor staged = at::empty({at_rows + points * nsample * entry}, bytes_on_device);
+    uint8_t* d = staged.data_ptr<uint8_t>();
+    check_status(tpk_grow_rows(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), d + at_rows,
+                               reinterpret_cast<int32_t*>(d + at_positions), reinterpret_cast<int64_t*>(d), ws.data_ptr(), ws_bytes,
+                               stream),
+                 "grow_proximity (rows)");
+    at::Tensor host = pinned(staged.numel());
+    host.copy_(staged, /*non_blocking=*/true);
+    c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(neighbours.get_device()).synchronize();
+    const uint8_t* h = host.data_ptr<uint8_t>();
+    const int64_t* starts = reinterpret_cast<const int64_t*>(h);
+    const int32_t* positions = reinterpret_cast<const int32_t*>(h + at_positions);
+    // (both halves from the pool: fresh memory would cost a page fault per 4 KiB)
+    at::Tensor walked = pinned(points * 8);
+    int32_t* out = reinterpret_cast<int32_t*>(walked.data_ptr<uint8_t>());
+    int32_t* places = out + points;
+    if (entry == 2)
+        walk_pieces(reinterpret_cast<const uint16_t*>(h + at_rows), nsample, positions, starts, pieces, points, min_cluster_size, places, out, sizes);
+    else
+        walk_pieces(reinterpret_cast<const uint32_t*>(h + at_rows), nsample, positions, starts, pieces, points, min_cluster_size, places, out, sizes);
+    int64_t total = 0;
+    for (int64_t v : *sizes)
+        total += v;
+    at::Tensor members = at::empty({total}, longs);
+    at::Tensor uploaded = at::empty({total * 4}, bytes_on_device);
+    uploaded.copy_(walked.narrow(0, 0, total * 4), /*non_blocking=*/true);
+    check_status(tpk_region_members(total, order.defined() ? order.data_ptr<int32_t>() : nullptr, 4, uploaded.data_ptr(),
+                                    members.data_ptr<int64_t>(), stream),
+                 "grow_proximity (members)");
+    return members;
+}
+
 // torch_points_kernels/cluster.py:9-37 (_grow_proximity_core; host code in the reference)
 // -> (members, starts): clusters one after the other and their offsets (one more than clusters).
 std::pair<at::Tensor, at::Tensor> grow_proximity(at::Tensor neighbours, int64_t min_cluster_size,
@@ -171,6 +281,15 @@ std::pair<at::Tensor, at::Tensor> grow_proximity(at::Tensor neighbours, int64_t 
     at::Tensor members = torch::empty({n}, options);
     at::Tensor starts = torch::empty({n + 1}, options);
     int64_t found[2] = {0, 0};
+    if (n > 0 && reference_order && neighbours.size(1) > 0)
+    {
+        std::vector<int64_t> sizes;
+        members = grow_reference_order(neighbours, min_cluster_size, at::Tensor(), &sizes);
+        std::vector<int64_t> ends(1, 0);
+        for (int64_t v : sizes)
+            ends.push_back(ends.back() + v);
+        return std::make_pair(members, at::tensor(ends, at::kLong).to(neighbours.device()));
+    }
     if (n > 0)
     {
         const size_t ws_bytes = tpk_grow_proximity_workspace_bytes(n, as_int(neighbours.size(1), "nsample"));
@@ -423,6 +542,91 @@ std::pair<at::Tensor, at::Tensor> ball_query_partial_dense(at::Tensor x, at::Ten
                                             ws_bytes, current_stream(x)),
                  "ball_query_partial_dense");
     return std::make_pair(idx, dist);
+}
+
+// torch_points_kernels/cluster.py:48-109 for all labels at once: the points label by label, every (label, sample) a cloud
+// of one packed self query, one growth.  Returns the clusters label after label, ordered by first point inside a label.
+std::vector<at::Tensor> region_grow(at::Tensor pos, at::Tensor labels, at::Tensor batch, std::vector<int64_t> ignore_labels,
+                                    int64_t nsample, double radius, int64_t min_cluster_size, bool reference_order)
+{
+    check_gpu(pos, "pos");
+    check_f32(pos, "pos");
+    check_points(pos, 2, "pos");
+    check_same_device(pos, labels, "pos and labels");
+    check_same_device(pos, batch, "pos and batch");
+    check_dtype(labels, at::kLong, "labels");
+    check_dtype(batch, at::kLong, "batch");
+    const int64_t n = pos.size(0);
+    TORCH_CHECK(labels.dim() == 1 && labels.size(0) == n && batch.dim() == 1 && batch.size(0) == n,
+                "pos, labels and batch differ in length");
+    TORCH_CHECK(ignore_labels.size() <= TPK_REGION_IGNORED, "region_grow: too many labels to ignore");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(pos.device());
+    if (n == 0)
+        return {};
+    pos = pos.contiguous();
+    labels = labels.contiguous();
+    batch = batch.contiguous();
+    void* stream = current_stream(pos);
+    at::Tensor order = at::empty({n}, pos.options().dtype(at::kInt));
+    at::Tensor sorted = at::empty({n, 3}, pos.options());
+    at::Tensor ids = at::empty({n}, batch.options());
+    int64_t found[2] = {0, 0};
+    {
+        const size_t ws_bytes = tpk_region_order_workspace_bytes(n);
+        TORCH_CHECK(ws_bytes > 0, "region_grow: too many points");
+        at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes)}, pos.options().dtype(at::kByte));
+        const int status = tpk_region_order(n, labels.data_ptr<int64_t>(), batch.data_ptr<int64_t>(), pos.data_ptr<float>(),
+                                            static_cast<int>(ignore_labels.size()), ignore_labels.data(), found,
+                                            order.data_ptr<int32_t>(), sorted.data_ptr<float>(), ids.data_ptr<int64_t>(),
+                                            ws.data_ptr(), ws_bytes, stream);
+        if (status == TPK_ERR_UNSUPPORTED)
+        {
+            // labels far apart: their ranks instead
+            at::Tensor values, ranks;
+            std::tie(values, ranks) = at::_unique(labels, /*sorted=*/true, /*return_inverse=*/true);
+            values = values.cpu();
+            std::vector<int64_t> ignored_ranks;
+            for (int64_t i = 0; i < values.numel(); ++i)
+                if (std::count(ignore_labels.begin(), ignore_labels.end(), values.data_ptr<int64_t>()[i]))
+                    ignored_ranks.push_back(i);
+            return region_grow(pos, ranks, batch, ignored_ranks, nsample, radius, min_cluster_size, reference_order);
+        }
+        check_status(status, "region_grow (order)");
+    }
+    const int64_t kept = found[0];
+    if (kept == 0)
+        return {};
+    if (found[1])
+    {
+        sorted = sorted.narrow(0, 0, kept);
+        ids = ids.narrow(0, 0, kept);
+    }
+    else
+    {
+        sorted = pos;
+        ids = batch;
+        order = at::Tensor();
+    }
+    at::Tensor neighbours =
+        ball_query_partial_dense(sorted, sorted, ids, ids, static_cast<float>(radius), as_int(nsample, "nsample"), false).first;
+    std::vector<int64_t> sizes;
+    at::Tensor members;
+    if (reference_order && nsample > 0)
+        members = grow_reference_order(neighbours, min_cluster_size, order, &sizes);
+    else
+    {
+        at::Tensor starts;
+        std::tie(members, starts) = grow_proximity(neighbours, min_cluster_size, false);
+        if (order.defined())
+            check_status(tpk_region_members(members.numel(), order.data_ptr<int32_t>(), 8, members.data_ptr<int64_t>(),
+                                            members.data_ptr<int64_t>(), stream),
+                         "region_grow (members)");
+        const at::Tensor ends = starts.cpu();
+        const int64_t* e = ends.data_ptr<int64_t>();
+        for (int64_t c = 0; c + 1 < ends.numel(); ++c)
+            sizes.push_back(e[c + 1] - e[c]);
+    }
+    return members.split_with_sizes(sizes);
 }
 
 // cuda/src/metrics.cpp:12-52
@@ -858,7 +1062,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("furthest_point_sampling", &furthest_point_sampling);
     m.def("three_nn", &three_nn);
     m.def("dense_knn", &dense_knn);
-    m.def("grow_proximity", &grow_proximity);
+    m.def("grow_proximity", &grow_proximity, pybind11::call_guard<pybind11::gil_scoped_release>());
+    m.def("region_grow", &region_grow, pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("instance_iou_cuda", &instance_iou_cuda);
     m.def("gridding", &gridding);
     m.def("gridding_grad", &gridding_grad);
