@@ -382,6 +382,20 @@ int tpk_instance_iou(int64_t total_gt_instances, int64_t n_proposals, int64_t n_
                      const int64_t* offset_num_gt_instances, const int64_t* batch,
                      const int64_t* instance_pointnum, float* proposals_iou, void* stream);
 
+/* The same for proposals that lie in arrays of their own, with the description of the ground truth - which the
+ * reference's front end (torch_points_kernels/metrics.py:60-80) gathers sample by sample - formed on the device.
+ *   tpk_instance_counts: counts (1 + TPK_IOU_SAMPLES) int64, device: [0] = samples (the last point's + 1), [1 + s] =
+ *     instances of sample s (its largest label, at least 0).  tpk_instance_counts_read copies it to the host and waits;
+ *     more than TPK_IOU_SAMPLES samples are not served by the call below.
+ *   tpk_instance_iou_lists: table (n_proposals, 2) int64, device: address and length of every proposal's int64 indices;
+ *     sizes (total_gt_instances) int32, scratch. */
+#define TPK_IOU_SAMPLES 1024
+int tpk_instance_counts(int64_t n_points, const int64_t* labels, const int64_t* batch, int64_t* counts, void* stream);
+int tpk_instance_counts_read(const int64_t* counts, int64_t* host_counts, void* stream);
+int tpk_instance_iou_lists(int64_t total_gt_instances, int64_t n_proposals, int64_t n_points, int64_t n_samples,
+                           const int64_t* table, const int64_t* labels, const int64_t* batch, const int64_t* counts,
+                           int32_t* sizes, float* proposals_iou, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * Gridding (GRNet): point clouds to occupancy grids by trilinear weights, and the gradient.
  * Replaces gridding_kernel_warpper(min_x, max_x, min_y, max_y, min_z, max_z, ptcloud, stream)

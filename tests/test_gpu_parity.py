@@ -1186,6 +1186,27 @@ def test_instance_iou_parity(tpk, oracle, dev, samples, points, instances, propo
     assert (want > 0).any()
 
 
+def test_instance_iou_lists_edges(tpk, oracle, dev):
+    """Empty and strided proposals, proposals of another integer type, samples without instances, workgroups whose
+    points belong to many samples, more samples than the kernels count: the native list path and the general one agree."""
+    from torch_points_kernels.metrics import instance_iou
+
+    g = torch.Generator().manual_seed(12)
+    for points, samples in ((1, 1), (50, 40), (9000, 700), (3000, 1100)):
+        batch = torch.sort(torch.cat([torch.arange(samples), torch.randint(0, samples, (points - min(points, samples),), generator=g)])[:points])[0]
+        gt = torch.randint(-2, 4, (points,), generator=g)
+        gt[batch % 3 == 1] = 0
+        gt[torch.cat([torch.ones(1, dtype=torch.bool), batch[1:] != batch[:-1]])] = 0  # (no sample of negative labels alone)
+        props = [torch.randint(0, points, (k,), generator=g) for k in (1, 7, 300)] + [torch.zeros(0, dtype=torch.long)]
+        want = oracle.instance_iou([p.numpy() for p in props], gt.numpy(), batch.numpy())
+        for kind in (torch.int64, torch.int32):
+            got = instance_iou([p.to(kind).to(dev) for p in props], gt.to(dev), batch.to(dev))
+            assert got.shape == want.shape
+            np.testing.assert_array_equal(_np(got), want)
+        wide = torch.stack([props[1], props[1]], 1).to(dev)
+        np.testing.assert_array_equal(_np(instance_iou([wide[:, 0]], gt.to(dev), batch.to(dev)))[0], want[1])
+
+
 # ------------------------------------------------------------------ gridding, cubic feature sampling
 
 

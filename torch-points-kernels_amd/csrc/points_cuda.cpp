@@ -663,6 +663,64 @@ at::Tensor instance_iou_cuda(at::Tensor instance_idx, at::Tensor instance_offset
     return output;
 }
 
+// torch_points_kernels/metrics.py:37-104 for index tensors on the device: None where a proposal is not a contiguous
+// int64 vector there, or the samples are more than the kernels count (the general path serves those).  The table of the
+// proposals is made while the device counts the instances; the host waits once, for the width of the output.
+pybind11::object instance_iou_lists(const pybind11::list& proposals, const at::Tensor& gt_instances, const at::Tensor& batch)
+{
+    const at::Tensor* all[] = {&gt_instances, &batch};
+    const char* names[] = {"gt_instances", "batch"};
+    for (int i = 0; i < 2; ++i)
+    {
+        check_contiguous(*all[i], names[i]);
+        check_gpu(*all[i], names[i]);
+        check_dtype(*all[i], at::kLong, names[i]);
+        TORCH_CHECK(all[i]->dim() == 1, names[i], " must have one dimension");
+    }
+    check_same_device(gt_instances, batch, "gt_instances and batch");
+    TORCH_CHECK(batch.size(0) == gt_instances.size(0), "batch and gt_instances differ in length");
+    const int64_t n = gt_instances.size(0), rows = static_cast<int64_t>(pybind11::len(proposals));
+    if (n == 0 || rows == 0)
+        return pybind11::none();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(gt_instances.device());
+    void* stream = current_stream(gt_instances);
+    at::Tensor counts = at::empty({1 + TPK_IOU_SAMPLES}, gt_instances.options());
+    check_status(tpk_instance_counts(n, gt_instances.data_ptr<int64_t>(), batch.data_ptr<int64_t>(), counts.data_ptr<int64_t>(), stream),
+                 "instance_iou (counts)");
+    at::Tensor table = at::empty({rows, 2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+    int64_t* entry = table.data_ptr<int64_t>();
+    for (int64_t p = 0; p < rows; ++p, entry += 2)
+    {
+        PyObject* o = PyList_GET_ITEM(proposals.ptr(), p);
+        if (!THPVariable_Check(o))
+            return pybind11::none();
+        const at::Tensor& t = THPVariable_Unpack(o);
+        if (t.dim() != 1 || t.scalar_type() != at::kLong || t.device() != gt_instances.device() || (t.size(0) > 1 && t.stride(0) != 1))
+            return pybind11::none();
+        entry[0] = reinterpret_cast<int64_t>(t.const_data_ptr());
+        entry[1] = t.size(0);
+    }
+    const at::Tensor on_device = table.to(gt_instances.device(), /*non_blocking=*/true);
+    int64_t found[1 + TPK_IOU_SAMPLES];
+    {
+        pybind11::gil_scoped_release waiting;
+        check_status(tpk_instance_counts_read(counts.data_ptr<int64_t>(), found, stream), "instance_iou (counts)");
+    }
+    const int64_t samples = std::max<int64_t>(found[0], 0);
+    if (samples > TPK_IOU_SAMPLES)
+        return pybind11::none();
+    int64_t total = 0;
+    for (int64_t s = 0; s < samples; ++s)
+        total += found[1 + s];
+    at::Tensor sizes = at::empty({total}, gt_instances.options().dtype(at::kInt));
+    at::Tensor iou = at::empty({rows, total}, gt_instances.options().dtype(at::kFloat));
+    check_status(tpk_instance_iou_lists(total, rows, n, samples, on_device.data_ptr<int64_t>(), gt_instances.data_ptr<int64_t>(),
+                                        batch.data_ptr<int64_t>(), counts.data_ptr<int64_t>(), sizes.data_ptr<int32_t>(),
+                                        iou.data_ptr<float>(), stream),
+                 "instance_iou");
+    return pybind11::cast(iou);
+}
+
 // cuda/src/gridding.cpp:4-12 -> {grid_weights, grid_pt_weights, grid_pt_indexes}
 std::vector<at::Tensor> gridding(float min_x, float max_x, float min_y, float max_y, float min_z, float max_z,
                                  at::Tensor ptcloud)
@@ -1065,6 +1123,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("grow_proximity", &grow_proximity, pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("region_grow", &region_grow, pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("instance_iou_cuda", &instance_iou_cuda);
+    m.def("instance_iou_lists", &instance_iou_lists);
     m.def("gridding", &gridding);
     m.def("gridding_grad", &gridding_grad);
     m.def("gridding_batch", &gridding_batch);
