@@ -453,6 +453,19 @@ int tpk_cubic_feature_sampling_f32(int b, int n_pts, int channels, int scale, in
 int tpk_cubic_feature_sampling_f64(int b, int n_pts, int channels, int scale, int neighborhood_size,
                                    const double* ptcloud, const double* cubic_features, double* point_features,
                                    int32_t* grid_pt_indexes, void* stream);
+/* The same with a workspace, in which the maps are turned so that a vertex' features lie side by side
+ * (tpk_cubic_feature_sampling_workspace_bytes, element_bytes 4 or 8; 0: the call wants none; 16-byte aligned).
+ * mapped != 0: ptcloud in [-1, 1), taken to x * scale / 2 + scale / 2 first (the reference's front end,
+ * torch_points_kernels/cubic_feature_sampling.py:57). */
+size_t tpk_cubic_feature_sampling_workspace_bytes(int b, int n_pts, int channels, int scale, int neighborhood_size,
+                                                  int element_bytes);
+int tpk_cubic_feature_sampling_ws_f32(int b, int n_pts, int channels, int scale, int neighborhood_size, int mapped,
+                                      const float* ptcloud, const float* cubic_features, float* point_features,
+                                      int32_t* grid_pt_indexes, void* workspace, size_t workspace_bytes, void* stream);
+int tpk_cubic_feature_sampling_ws_f64(int b, int n_pts, int channels, int scale, int neighborhood_size, int mapped,
+                                      const double* ptcloud, const double* cubic_features, double* point_features,
+                                      int32_t* grid_pt_indexes, void* workspace, size_t workspace_bytes, void* stream);
+/* grad_ptcloud NULL: not wanted. */
 int tpk_cubic_feature_sampling_grad_f32(int b, int n_pts, int channels, int scale, int neighborhood_size,
                                         const float* grad_point_features, const int32_t* grid_pt_indexes,
                                         float* grad_ptcloud, float* grad_cubic_features, void* stream);

@@ -1298,6 +1298,30 @@ def test_cubic_feature_sampling_parity(tpk, oracle, dev, dtype, B, n, c, scale, 
     np.testing.assert_allclose(_np(grad_f), wf, rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+# turned maps: channels beyond a block of 64, odd ones, maps that do not fill their spans; many points on one vertex (lists
+# sorted in several rounds, runs that share a cell); a map of more spans than are worth looking through
+@pytest.mark.parametrize("B,n,c,scale,crowd", [(3, 900, 70, 12, 0), (4, 2500, 33, 8, 0), (1, 4100, 20, 7, 3900), (8, 700, 130, 16, 500), (1, 9000, 12, 26, 0)])
+def test_cubic_feature_sampling_spans(tpk, oracle, dev, dtype, B, n, c, scale, crowd):
+    g = torch.Generator().manual_seed(n + c)
+    p = (torch.rand(B, n, 3, generator=g, dtype=torch.float64) * 2.2 - 1.1).to(dtype)
+    p[:, :crowd] = torch.tensor([0.1, 0.2, -0.3], dtype=dtype)
+    feats = torch.rand(B, c, scale, scale, scale, generator=g, dtype=torch.float64).to(dtype)
+    maps = feats.to(dev).requires_grad_()
+    x = p.to(dev).requires_grad_()
+    out = tpk.cubic_feature_sampling(x, maps, 1)
+    wo, wi = oracle.cubic_feature_sampling((p * (scale / 2) + scale / 2).numpy(), feats.numpy(), 1)
+    np.testing.assert_array_equal(_np(out), wo)
+    go = torch.randn(out.shape, generator=g, dtype=torch.float64).to(dtype)
+    gx, gm = torch.autograd.grad(out, (x, maps), go.to(dev), retain_graph=True)
+    assert (_np(gx) == 0).all()
+    wf = oracle.cubic_feature_sampling_grad(scale, 1, go.double().numpy(), wi)[1]
+    size = oracle.cubic_feature_sampling_grad(scale, 1, go.double().abs().numpy(), wi)[1]
+    unit = 2.0 ** (-23 if dtype == torch.float32 else -52)
+    assert (np.abs(_np(gm) - wf) <= (4 + crowd / 16) * unit * size).all()
+    assert torch.equal(torch.autograd.grad(out, maps, go.to(dev))[0].isnan(), torch.zeros_like(maps, dtype=torch.bool))
+
+
 def test_cubic_feature_sampling_front_end_and_gradcheck(tpk, oracle, dev):
     from torch_points_kernels.cubic_feature_sampling import CubicFeatureSamplingFunction, cubic_feature_sampling
 

@@ -295,33 +295,48 @@ __global__ __launch_bounds__(GR_THREADS) void gridding_batch_grad_kernel(
     grad_ptcloud[j * 3 + 2] = gz * factor;
 }
 
-// cuda/src/cubic_feature_sampling_gpu.cu:23-105.  First kernel: the vertex indices of every
-// point (-1 outside the grid); second kernel: one thread per output element, channel fastest.
+// ---- cubic feature sampling: cuda/src/cubic_feature_sampling_gpu.cu:23-210 ---------------------
+//
+// A point's vertices are floor - (ns - 1) .. floor + ns per axis (the upper plane lies one above the
+// lower one whether or not the coordinate is integral), x slowest.
+
+// Coordinates as the front end maps them (reference cubic_feature_sampling.py:57: x * half + half), or as they are.
 template <typename T>
-__global__ __launch_bounds__(GR_THREADS) void cubic_indexes_kernel(int64_t total_pts, int scale, int neighborhood_size,
-                                                                   int n_vertices, const T* __restrict__ ptcloud,
-                                                                   int* __restrict__ grid_pt_indexes)
+struct CubicFrame
 {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * GR_THREADS + threadIdx.x;
-    if (i >= total_pts)
-        return;
-    int lx, ux, ly, uy, lz, uz;
-    planes(ptcloud[i * 3 + 0], &lx, &ux);
-    planes(ptcloud[i * 3 + 1], &ly, &uy);
-    planes(ptcloud[i * 3 + 2], &lz, &uz);
-    const int ns = neighborhood_size - 1;
-    int at = 0;
-    for (int j = lx - ns; j <= ux + ns; ++j)
-        for (int k = ly - ns; k <= uy + ns; ++k)
-            for (int m = lz - ns; m <= uz + ns; ++m)
-            {
-                const bool outside = j < 0 || j >= scale || k < 0 || k >= scale || m < 0 || m >= scale;
-                if (at < n_vertices)
-                    grid_pt_indexes[i * n_vertices + at] = outside ? -1 : j * scale * scale + k * scale + m;
-                ++at;
-            }
+    T half;
+    bool mapped;
+    __device__ __forceinline__ T operator()(T v) const { return mapped ? v * half + half : v; }
+};
+
+// Vertex `v` of the point whose lower planes are (x, y, z); -1 outside the map.
+__device__ __forceinline__ int cubic_vertex(int x, int y, int z, int v, int side, int scale)
+{
+    const int first = 1 - side / 2;
+    const int vz = v % side, vy = v / side % side, vx = v / (side * side);
+    const int j = x + first + vx, k = y + first + vy, m = z + first + vz;
+    const bool outside = j < 0 || j >= scale || k < 0 || k >= scale || m < 0 || m >= scale;
+    return outside ? -1 : (j * scale + k) * scale + m;
 }
 
+// The vertex indices of every point, for the gather below.
+template <typename T>
+__global__ __launch_bounds__(GR_THREADS) void cubic_indexes_kernel(int64_t total_rows, int scale, int side, int n_vertices,
+                                                                   CubicFrame<T> frame, const T* __restrict__ ptcloud,
+                                                                   int* __restrict__ grid_pt_indexes)
+{
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * GR_THREADS + threadIdx.x;
+    if (row >= total_rows)
+        return;
+    const int64_t i = row / n_vertices;
+    const int x = static_cast<int>(floor(frame(ptcloud[i * 3 + 0])));
+    const int y = static_cast<int>(floor(frame(ptcloud[i * 3 + 1])));
+    const int z = static_cast<int>(floor(frame(ptcloud[i * 3 + 2])));
+    grid_pt_indexes[row] = cubic_vertex(x, y, z, static_cast<int>(row - i * n_vertices), side, scale);
+}
+
+// Small calls: one thread per output element, channel fastest, straight from the maps - a lane's read is
+// a line of its own, 1.7 clocks of a compute unit's address path each.
 template <typename T>
 __global__ __launch_bounds__(GR_THREADS) void cubic_gather_kernel(
     int64_t total, int n_pts, int n_vertices, int channels, int64_t cub_scale, const T* __restrict__ cubic_features,
@@ -338,7 +353,109 @@ __global__ __launch_bounds__(GR_THREADS) void cubic_gather_kernel(
     point_features[e] = vertex < 0 ? T(0) : cubic_features[(cloud * channels + k) * cub_scale + vertex];
 }
 
-// cuda/src/cubic_feature_sampling_gpu.cu:138-175
+// Otherwise the maps are turned first, (c, cells) -> (cells, c), so that what a vertex contributes is one run
+// of consecutive values: the gather then reads and writes whole rows.
+constexpr int CT_TILE = 64;
+constexpr int CT_THREADS = 256;
+
+// WIDE: 16 bytes per lane on both sides (cells and channels multiples of that).
+template <typename T, bool WIDE>
+__global__ __launch_bounds__(CT_THREADS) void cubic_turn_kernel(int channels, int64_t cub_scale, int cell_tiles, int channel_tiles,
+                                                                const T* __restrict__ maps, T* __restrict__ turned)
+{
+    constexpr int V = WIDE ? 16 / static_cast<int>(sizeof(T)) : 1;
+    __shared__ T tile[CT_TILE][CT_TILE + 1];
+    const unsigned block = xcd_local_block(blockIdx.x, gridDim.x);
+    const int channel_tile = static_cast<int>(block % channel_tiles);
+    const unsigned rest = block / channel_tiles;
+    const int64_t cell0 = static_cast<int64_t>(rest % cell_tiles) * CT_TILE;
+    const int64_t cloud = rest / cell_tiles;
+    const int c0 = channel_tile * CT_TILE;
+    const T* from = maps + cloud * channels * cub_scale;
+    T* to = turned + cloud * channels * cub_scale;
+    constexpr int ACROSS = CT_TILE / V, STEP = CT_THREADS / ACROSS;
+    const int x = threadIdx.x % ACROSS * V, y = threadIdx.x / ACROSS;
+    struct alignas(sizeof(T) * V) Piece
+    {
+        T v[V];
+    };
+    Piece piece[CT_TILE / STEP];
+#pragma unroll
+    for (int r = 0; r < CT_TILE; r += STEP)
+        if (c0 + y + r < channels && cell0 + x < cub_scale)
+            piece[r / STEP] = *reinterpret_cast<const Piece*>(from + static_cast<int64_t>(c0 + y + r) * cub_scale + cell0 + x);
+#pragma unroll
+    for (int r = 0; r < CT_TILE; r += STEP)
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+            tile[y + r][x + i] = piece[r / STEP].v[i];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < CT_TILE; r += STEP)
+        if (cell0 + y + r < cub_scale && c0 + x < channels)
+        {
+            Piece out;
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+                out.v[i] = tile[x + i][y + r];
+            *reinterpret_cast<Piece*>(to + (cell0 + y + r) * channels + c0 + x) = out;
+        }
+}
+
+// A workgroup finds the vertices of its rows once, in LDS, and copies: bound by the stores of the rows, which
+// pass the caches by so that these hold the turned maps.  V: what a lane copies at a time (16 bytes where the
+// channels are a multiple of that); magic: 2^32 / per_row rounded up.
+constexpr int CR_ROWS = 256; // at most, per workgroup
+
+template <typename T, typename V>
+__global__ __launch_bounds__(GR_THREADS) void cubic_rows_kernel(int64_t total_rows, int rows_per_block, int n_pts, int n_vertices, int side,
+                                                                unsigned per_row, unsigned magic, int scale, CubicFrame<T> frame,
+                                                                const T* __restrict__ ptcloud, const V* __restrict__ turned,
+                                                                V* __restrict__ point_features, int* __restrict__ grid_pt_indexes)
+{
+    __shared__ int64_t from[CR_ROWS]; // first element of the row's source, -1: zeros
+    const int64_t row0 = static_cast<int64_t>(xcd_local_block(blockIdx.x, gridDim.x)) * rows_per_block;
+    const int rows = static_cast<int>(tpk_min64(rows_per_block, total_rows - row0));
+    const int64_t cub_scale = static_cast<int64_t>(scale) * scale * scale;
+    if (static_cast<int>(threadIdx.x) < rows)
+    {
+        const int64_t row = row0 + threadIdx.x, i = row / n_vertices;
+        const int x = static_cast<int>(floor(frame(ptcloud[i * 3 + 0])));
+        const int y = static_cast<int>(floor(frame(ptcloud[i * 3 + 1])));
+        const int z = static_cast<int>(floor(frame(ptcloud[i * 3 + 2])));
+        const int vertex = cubic_vertex(x, y, z, static_cast<int>(row - i * n_vertices), side, scale);
+        grid_pt_indexes[row] = vertex;
+        from[threadIdx.x] = vertex < 0 ? -1 : (i / n_pts * cub_scale + vertex) * per_row;
+    }
+    __syncthreads();
+    V* out = point_features + row0 * per_row;
+    const unsigned pieces = static_cast<unsigned>(rows) * per_row;
+    constexpr unsigned UNROLL = 8;
+    for (unsigned first = threadIdx.x; first < pieces; first += UNROLL * GR_THREADS)
+    {
+        V value[UNROLL];
+#pragma unroll
+        for (unsigned u = 0; u < UNROLL; ++u)
+        {
+            const unsigned e = first + u * GR_THREADS;
+            value[u] = V{};
+            if (e < pieces)
+            {
+                const unsigned row = per_row == 1 ? e : __umulhi(e, magic);
+                const int64_t at = from[row];
+                if (at >= 0)
+                    value[u] = turned[at + (e - row * per_row)];
+            }
+        }
+#pragma unroll
+        for (unsigned u = 0; u < UNROLL; ++u)
+            if (first + u * GR_THREADS < pieces)
+                __builtin_nontemporal_store(value[u], &out[first + u * GR_THREADS]);
+    }
+}
+
+// cuda/src/cubic_feature_sampling_gpu.cu:138-175, for maps of fewer cells than a workgroup below is worth
+// having and as the reference's scatter: one atomic per term, in no fixed order.
 template <typename T>
 __global__ __launch_bounds__(GR_THREADS) void cubic_scatter_kernel(
     int64_t total, int n_pts, int n_vertices, int channels, int64_t cub_scale,
@@ -356,46 +473,205 @@ __global__ __launch_bounds__(GR_THREADS) void cubic_scatter_kernel(
         atomicAdd(&grad_cubic_features[(cloud * channels + k) * cub_scale + vertex], grad_point_features[e]);
 }
 
-// The same sum with the destination in LDS: a workgroup owns `group` channels of one cloud's
-// feature map (group * scale^3 accumulators), walks all (point, vertex) entries of the cloud
-// and adds its channels' gradients with LDS atomics, then writes the map out in order.  One
-// global atomic per term (a cache line each, at device scope) is what makes the kernel above slow.
-constexpr int CS_THREADS = 1024; // LDS atomics are slow: many wavefronts keep the unit busy
+// The gradient of the maps as a gather.  A workgroup owns a span of cells of one cloud: it sorts the cloud's
+// (point, vertex) entries that lie in the span by cell (counting sort in LDS, the indices come from the L2),
+// then walks the sorted list - equal runs of it per group of LANES lanes, a lane per channel, the rows of
+// the gradient coming in as whole lines, 16 in flight - adds up while the cell stays the same and puts a
+// finished sum into LDS; what runs share at their ends is added there atomically.  The span leaves as whole lines
+// per channel.  (One pass that keeps the indices in registers between counting and placing spills: 52 us; three
+// 32-bit divisions per index instead of masks, and entries handled lane by lane instead of in scalars: 59 us.)
+// Every row of the gradient is read once and every element of the maps written once, where
+// sums by LDS atomics (194 clocks per 64 terms) bounded the version before: 32 clouds of 2048 points, 64
+// channels, 16^3 cells 219 us, 44 us this way.  Bound: the stream of gradient rows.
+constexpr int CB_THREADS = 1024;
+constexpr int CB_LIST = 2048;   // entries sorted at a time
+constexpr int CB_CHANNELS = 64; // channels summed at a time
+constexpr int CB_LINE = 16;     // cells that stay together: 64 bytes of a channel
 
 template <typename T>
-__global__ __launch_bounds__(CS_THREADS) void cubic_scatter_lds_kernel(
-    int n_pts, int n_vertices, int channels, int group, int64_t cub_scale, const T* __restrict__ grad_point_features,
-    const int* __restrict__ grid_pt_indexes, T* __restrict__ grad_cubic_features)
+struct CubicSpan
+{
+    static constexpr int CELLS = sizeof(T) == 4 ? 256 : 128; // (two workgroups per compute unit)
+    T sums[CELLS][CB_CHANNELS + 1];
+    unsigned entry[CB_LIST];
+    unsigned short cell[CB_LIST];
+    int count[CELLS + 1];
+    int total;
+};
+
+// (float32, a lane per channel: two workgroups per compute unit, 8 wavefronts per SIMD; the other forms need the
+// registers of one)
+template <typename T, int LANES>
+__global__ __launch_bounds__(CB_THREADS, sizeof(T) == 4 && LANES == TPK_WAVE ? 8 : 4) void cubic_spans_kernel(
+                                                                 int n_pts, int n_vertices, int channels, int64_t cub_scale, int spans,
+                                                                 const T* __restrict__ grad_point_features,
+                                                                 const int* __restrict__ grid_pt_indexes,
+                                                                 T* __restrict__ grad_cubic_features)
 {
     extern __shared__ __align__(16) unsigned char cubic_lds[];
-    T* sums = reinterpret_cast<T*>(cubic_lds);
-    // the workgroups of one cloud read the same lines of the gradient (each its own channels): they
-    // are kept on one die, so that one L2 serves them
-    const int groups = (channels + group - 1) / group;
+    CubicSpan<T>& lds = *reinterpret_cast<CubicSpan<T>*>(cubic_lds);
+    constexpr int CELLS = CubicSpan<T>::CELLS;
     const int block = static_cast<int>(xcd_local_block(blockIdx.x, gridDim.x));
-    const int cloud = block / groups;
-    const int k0 = (block - cloud * groups) * group;
-    const int width = min(group, channels - k0);
-    const int64_t cells = static_cast<int64_t>(width) * cub_scale;
-    for (int64_t t = threadIdx.x; t < cells; t += CS_THREADS)
-        sums[t] = T(0);
-    __syncthreads();
+    const int cloud = block / spans;
+    const int span = block - cloud * spans, span_bits = 31 - __builtin_clz(spans); // (a power of two)
+    // Cell c lies in line c / LINE; lines are dealt out spans at a time, every turn starting one span further on, so
+    // that no plane of the map - where a flat cloud's points would be - falls to one workgroup.
+    const unsigned lines = static_cast<unsigned>((cub_scale + CB_LINE - 1) / CB_LINE);
+    const int cells = static_cast<int>((lines + spans - 1) / spans) * CB_LINE; // places, some beyond the map
     const int64_t entries = static_cast<int64_t>(n_pts) * n_vertices;
     const int* indexes = grid_pt_indexes + cloud * entries;
     const T* grads = grad_point_features + cloud * entries * channels;
-    // consecutive threads take the channels of one entry, then the next entry
-    for (int64_t t = threadIdx.x; t < entries * width; t += CS_THREADS)
+    constexpr int WALKERS = CB_THREADS / LANES;
+    const int walker = threadIdx.x / LANES, lane = threadIdx.x % LANES;
+
+    // the span's entries among [begin, end): f(entry, cell of the span); BATCH indices per thread on their way at a time
+    auto own_entries = [&](int64_t begin, int64_t end, auto&& f) {
+        constexpr int BATCH = 8;
+        for (; begin < end; begin += BATCH * CB_THREADS)
+        {
+            const int* from = indexes + begin;
+            const int length = static_cast<int>(tpk_min64(end - begin, BATCH * CB_THREADS));
+            unsigned index[BATCH];
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i)
+                index[i] = static_cast<int>(threadIdx.x) < length - i * CB_THREADS ? (from + i * CB_THREADS)[threadIdx.x] : -1;
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i)
+            {
+                const unsigned line = index[i] / CB_LINE, turn = line >> span_bits;
+                if (index[i] < static_cast<unsigned>(cub_scale) && ((line + turn) & (spans - 1)) == static_cast<unsigned>(span))
+                    f(begin + threadIdx.x + i * CB_THREADS, static_cast<int>(turn * CB_LINE + index[i] % CB_LINE));
+            }
+        }
+    };
+    auto count = [&](int64_t begin, int64_t end) {
+        __syncthreads();
+        for (int t = threadIdx.x; t < CELLS; t += CB_THREADS)
+            lds.count[t] = 0;
+        __syncthreads();
+        own_entries(begin, end, [&](int64_t, int c) { atomicAdd(&lds.count[c], 1); });
+        __syncthreads();
+        if (threadIdx.x < TPK_WAVE)
+        {
+            int before = 0;
+            for (int at = 0; at < CELLS; at += TPK_WAVE)
+            {
+                const int v = lds.count[at + threadIdx.x];
+                const int ahead = wave_exclusive_sum(v);
+                lds.count[at + threadIdx.x] = before + ahead;
+                before += tpk_read_lane(ahead + v, TPK_WAVE - 1);
+            }
+            if (threadIdx.x == 0)
+                lds.total = before;
+        }
+        __syncthreads();
+        return lds.total;
+    };
+
+    for (int c0 = 0; c0 < channels; c0 += CB_CHANNELS)
     {
-        const int64_t entry = t / width;
-        const int k = static_cast<int>(t - entry * width);
-        const int vertex = indexes[entry];
-        if (vertex >= 0 && vertex < cub_scale)
-            atomicAdd(&sums[k * cub_scale + vertex], grads[entry * channels + k0 + k]);
+        const int width = min(CB_CHANNELS, channels - c0);
+        for (int t = threadIdx.x; t < CELLS * (CB_CHANNELS + 1); t += CB_THREADS)
+            (&lds.sums[0][0])[t] = T(0);
+        int64_t begin = 0, size = entries;
+        while (begin < entries)
+        {
+            int64_t end = tpk_min64(begin + size, entries);
+            int have = count(begin, end);
+            while (have > CB_LIST)
+            {
+                // fewer entries at a time: what should give three quarters of a list, in any case no more than a list
+                size = tpk_min64(size / 2, size * (3 * CB_LIST / 4) / have);
+                size = size < CB_LIST ? CB_LIST : size;
+                end = tpk_min64(begin + size, entries);
+                have = count(begin, end);
+            }
+            own_entries(begin, end, [&](int64_t e, int c) {
+                const int at = atomicAdd(&lds.count[c], 1);
+                lds.entry[at] = static_cast<unsigned>(e - begin);
+                lds.cell[at] = static_cast<unsigned short>(c);
+            });
+            __syncthreads();
+            // Runs end where a cell ends, if that is not far: a sum that two runs share goes through an LDS atomic, 192
+            // clocks for 64 lanes.  (LANES = 64: what follows is the same for a wavefront's lanes and kept in scalars;
+            // the walk is bound by instruction issue.)
+            auto same_for_group = [&](int v) { return LANES == TPK_WAVE ? __builtin_amdgcn_readfirstlane(v) : v; };
+            auto run_start = [&](int w) {
+                const int even = static_cast<int>(static_cast<int64_t>(have) * w / WALKERS);
+                for (int q = even; q < even + 32; ++q)
+                    if (q == 0 || q >= have || lds.cell[q] != lds.cell[q - 1])
+                        return q < have ? q : have;
+                return even;
+            };
+            const int q0 = same_for_group(run_start(walker)), q1 = same_for_group(run_start(walker + 1));
+            int shared_start = same_for_group(q0 > 0 && q0 < q1 && lds.cell[q0] == lds.cell[q0 - 1]);
+            const int shared_end = same_for_group(q1 > q0 && q1 < have && lds.cell[q1] == lds.cell[q1 - 1]);
+            // (lanes beyond the channels go along: theirs are entries of the list too)
+            const char* column = reinterpret_cast<const char*>(grads + begin * channels + c0 + min(lane, width - 1));
+            const unsigned row_bytes = static_cast<unsigned>(channels) * static_cast<unsigned>(sizeof(T));
+            int open = same_for_group(q0 < q1 ? lds.cell[q0] : 0);
+            T sum = T(0);
+            auto put = [&](int shared) {
+                if (lane >= width)
+                    return;
+                if (shared)
+                    atomicAdd(&lds.sums[open][lane], sum);
+                else
+                    lds.sums[open][lane] += sum;
+            };
+            // A group takes up its entries a lane each; rows are asked for AHEAD entries before they are added.
+            constexpr int AHEAD = sizeof(T) == 4 ? 16 : 8;
+            for (int q = q0; q < q1; q += LANES)
+            {
+                const int n = min(LANES, q1 - q);
+                // (beyond the end: the last entry again, to a cell that is none - no branch around a load, behind one the
+                // compiler waits for all loads in flight)
+                const int mine = q + min(lane, n - 1);
+                const int my_offset = static_cast<int>(lds.entry[mine] * row_bytes);
+                const int my_cell = lds.cell[mine];
+                auto of = [&](int v, int i) {
+                    i = min(i, LANES - 1);
+                    return LANES == TPK_WAVE ? __builtin_amdgcn_readlane(v, i) : __shfl(v, i, LANES);
+                };
+                auto row = [&](int i) { return *reinterpret_cast<const T*>(column + static_cast<unsigned>(of(my_offset, i))); };
+                T value[AHEAD];
+#pragma unroll
+                for (int a = 0; a < AHEAD; ++a)
+                    value[a] = row(a);
+                for (int first = 0; first < n; first += AHEAD)
+#pragma unroll
+                    for (int a = 0; a < AHEAD; ++a)
+                    {
+                        const T v = value[a];
+                        value[a] = row(first + a + AHEAD);
+                        if (first + a < n)
+                        {
+                            const int c = of(my_cell, first + a);
+                            if (c != open)
+                            {
+                                put(shared_start);
+                                shared_start = 0;
+                                open = c;
+                                sum = T(0);
+                            }
+                            sum += v;
+                        }
+                    }
+            }
+            if (q0 < q1)
+                put(shared_start | shared_end);
+            begin = end;
+        }
+        __syncthreads();
+        T* out = grad_cubic_features + (static_cast<int64_t>(cloud) * channels + c0) * cub_scale;
+        const int place = threadIdx.x % CELLS; // (the same in every turn of the loop)
+        const unsigned turn = place / CB_LINE, line = turn * spans + ((span - turn) & (spans - 1));
+        const int64_t c = static_cast<int64_t>(line) * CB_LINE + place % CB_LINE;
+        if (place < cells && c < cub_scale)
+            for (int k = threadIdx.x / CELLS; k < width; k += CB_THREADS / CELLS)
+                out[k * cub_scale + c] = lds.sums[place][k];
+        __syncthreads();
     }
-    __syncthreads();
-    T* out = grad_cubic_features + (static_cast<int64_t>(cloud) * channels + k0) * cub_scale;
-    for (int64_t t = threadIdx.x; t < cells; t += CS_THREADS)
-        out[t] = sums[t];
 }
 
 // How many workgroups share a grid in gridding_lds_kernel, and their LDS; 0: take gridding_kernel.
@@ -539,9 +815,19 @@ int64_t cubic_vertices(int neighborhood_size)
     return side * side * side;
 }
 
+// Whether the maps are turned first: an element gathered from them as they are costs 2.8 ps, from turned ones 0.7 ps,
+// turning 1.6 ps per element of the maps and a launch.
+bool cubic_turns(int b, int n_pts, int channels, int scale, int64_t nv)
+{
+    const double per_cell = static_cast<double>(b) * channels;
+    const double rows = per_cell * n_pts * static_cast<double>(nv), cells = per_cell * scale * static_cast<double>(scale) * scale;
+    return rows > 0.8 * cells + 1.5e6 && cells < 2.0e9 && channels < 65536;
+}
+
 template <typename T>
-int cubic_fwd(int b, int n_pts, int channels, int scale, int neighborhood_size, const T* ptcloud,
-              const T* cubic_features, T* point_features, int32_t* grid_pt_indexes, hipStream_t s)
+int cubic_fwd(int b, int n_pts, int channels, int scale, int neighborhood_size, bool mapped, const T* ptcloud,
+              const T* cubic_features, T* point_features, int32_t* grid_pt_indexes, void* workspace, size_t workspace_bytes,
+              hipStream_t s)
 {
     const int64_t nv = cubic_vertices(neighborhood_size);
     if (b < 0 || n_pts < 0 || channels < 0 || scale <= 0 || nv < 0 || scale > 1290)
@@ -550,19 +836,69 @@ int cubic_fwd(int b, int n_pts, int channels, int scale, int neighborhood_size, 
         return TPK_OK;
     if (!ptcloud || !grid_pt_indexes || (channels > 0 && (!cubic_features || !point_features)))
         return TPK_ERR_INVALID_ARG;
-    const int64_t total_pts = static_cast<int64_t>(b) * n_pts;
-    const int64_t total = total_pts * nv * channels;
-    const int64_t blocks_pts = tpk_ceil_div(total_pts, GR_THREADS), blocks = tpk_ceil_div(total, GR_THREADS);
-    if (blocks > 0x7fffffffLL || nv > 0x7fffffffLL)
+    const int64_t total_rows = static_cast<int64_t>(b) * n_pts * nv;
+    const int64_t total = total_rows * channels;
+    const int64_t blocks_rows = tpk_ceil_div(total_rows, GR_THREADS), blocks = tpk_ceil_div(total, GR_THREADS);
+    if (blocks > 0x7fffffffLL || blocks_rows > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(cubic_indexes_kernel<T>, dim3(static_cast<unsigned>(blocks_pts)), dim3(GR_THREADS), 0, s,
-                       total_pts, scale, neighborhood_size, static_cast<int>(nv), ptcloud, grid_pt_indexes);
+    const int side = 2 * neighborhood_size, vertices = static_cast<int>(nv);
+    const int64_t cub = static_cast<int64_t>(scale) * scale * scale;
+    const CubicFrame<T> frame{static_cast<T>(scale / 2.0), mapped};
+    if (total > 0 && workspace && cubic_turns(b, n_pts, channels, scale, nv))
+    {
+        if (workspace_bytes < static_cast<size_t>(b * channels * cub) * sizeof(T) || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
+            return TPK_ERR_WORKSPACE;
+        const int64_t cell_tiles = tpk_ceil_div(cub, CT_TILE), channel_tiles = tpk_ceil_div(channels, CT_TILE);
+        const int64_t tiles = cell_tiles * channel_tiles * b;
+        if (tiles > 0x7fffffffLL)
+            return TPK_ERR_UNSUPPORTED;
+        T* turned = static_cast<T*>(workspace);
+        constexpr int WIDE = 16 / static_cast<int>(sizeof(T));
+        typedef unsigned Quad __attribute__((ext_vector_type(4)));
+        const bool wide = channels % WIDE == 0 && ((reinterpret_cast<uintptr_t>(point_features) | reinterpret_cast<uintptr_t>(cubic_features)) & 15) == 0;
+        const auto turn = wide && cub % WIDE == 0 ? cubic_turn_kernel<T, true> : cubic_turn_kernel<T, false>;
+        hipLaunchKernelGGL(turn, dim3(static_cast<unsigned>(tiles)), dim3(CT_THREADS), 0, s, channels, cub,
+                           static_cast<int>(cell_tiles), static_cast<int>(channel_tiles), cubic_features, turned);
+        const int per_row = wide ? channels / WIDE : channels;
+        // (about 4096 pieces per workgroup; below 2^16, where the multiplication by `magic` is exact)
+        const int rows = per_row >= 4096 ? 1 : 4096 / per_row > CR_ROWS ? CR_ROWS : 4096 / per_row;
+        if (static_cast<int64_t>(rows) * per_row >= 65536)
+            return TPK_ERR_UNSUPPORTED;
+        const unsigned magic = static_cast<unsigned>(((uint64_t(1) << 32) + per_row - 1) / per_row);
+        const unsigned grid = static_cast<unsigned>(tpk_ceil_div(total_rows, rows));
+        if (wide)
+            hipLaunchKernelGGL((cubic_rows_kernel<T, Quad>), dim3(grid), dim3(GR_THREADS), 0, s, total_rows, rows, n_pts, vertices, side,
+                               static_cast<unsigned>(per_row), magic, scale, frame, ptcloud, reinterpret_cast<const Quad*>(turned),
+                               reinterpret_cast<Quad*>(point_features), grid_pt_indexes);
+        else
+            hipLaunchKernelGGL((cubic_rows_kernel<T, T>), dim3(grid), dim3(GR_THREADS), 0, s, total_rows, rows, n_pts, vertices, side,
+                               static_cast<unsigned>(per_row), magic, scale, frame, ptcloud, turned, point_features, grid_pt_indexes);
+        return tpk_launch_status();
+    }
+    hipLaunchKernelGGL(cubic_indexes_kernel<T>, dim3(static_cast<unsigned>(blocks_rows)), dim3(GR_THREADS), 0, s,
+                       total_rows, scale, side, vertices, frame, ptcloud, grid_pt_indexes);
     int st = tpk_launch_status();
     if (st != TPK_OK || total == 0)
         return st;
     hipLaunchKernelGGL(cubic_gather_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(GR_THREADS), 0, s, total, n_pts,
-                       static_cast<int>(nv), channels, static_cast<int64_t>(scale) * scale * scale, cubic_features,
-                       grid_pt_indexes, point_features);
+                       vertices, channels, cub, cubic_features, grid_pt_indexes, point_features);
+    return tpk_launch_status();
+}
+
+template <typename T, int LANES>
+int launch_spans(int b, int n_pts, int nv, int channels, int64_t cub, const T* grad, const int32_t* indexes, T* grad_maps, hipStream_t s)
+{
+    int64_t spans = 1;
+    while (spans * CubicSpan<T>::CELLS < cub)
+        spans *= 2;
+    const int64_t blocks = spans * b;
+    if (blocks > 0x7fffffffLL)
+        return TPK_ERR_UNSUPPORTED;
+    const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(cubic_spans_kernel<T, LANES>), sizeof(CubicSpan<T>));
+    if (allowed != TPK_OK)
+        return allowed;
+    hipLaunchKernelGGL((cubic_spans_kernel<T, LANES>), dim3(static_cast<unsigned>(blocks)), dim3(CB_THREADS), sizeof(CubicSpan<T>), s,
+                       n_pts, nv, channels, cub, static_cast<int>(spans), grad, indexes, grad_maps);
     return tpk_launch_status();
 }
 
@@ -576,36 +912,27 @@ int cubic_bwd(int b, int n_pts, int channels, int scale, int neighborhood_size, 
     if (b == 0)
         return TPK_OK;
     const int64_t cub = static_cast<int64_t>(scale) * scale * scale;
-    if ((n_pts > 0 && !grad_ptcloud) || (channels > 0 && !grad_cubic_features))
+    if (channels > 0 && !grad_cubic_features)
         return TPK_ERR_INVALID_ARG;
     // the coordinates only choose the vertices (floor and ceil): their gradient is zero
     // (cuda/src/cubic_feature_sampling_gpu.cu:165-170)
-    int st = fill_zero<T>(static_cast<int64_t>(b) * n_pts * 3, grad_ptcloud, s);
+    int st = grad_ptcloud ? fill_zero<T>(static_cast<int64_t>(b) * n_pts * 3, grad_ptcloud, s) : TPK_OK;
     if (st != TPK_OK)
         return st;
-    const int64_t total = static_cast<int64_t>(b) * n_pts * nv * channels;
+    const int64_t entries = static_cast<int64_t>(n_pts) * nv;
+    const int64_t total = entries * b * channels;
     if (total > 0 && (!grad_point_features || !grid_pt_indexes))
         return TPK_ERR_INVALID_ARG;
-    // Feature maps that fit in LDS (at least one channel of scale^3 sums in 128 KiB) are summed there.
-    const int64_t fit = (128 * 1024) / (cub * static_cast<int64_t>(sizeof(T)));
-    if (fit >= 1 && channels > 0 && nv <= 0x7fffffffLL)
+    // Every span of 256 cells looks through all entries of its cloud: worth it while those are not many times the
+    // span's own - up to 64 spans (maps of 25^3 cells) - or while a span's look is short.
+    const int64_t spans = tpk_ceil_div(cub, CubicSpan<T>::CELLS);
+    if (channels > 0 && total > 0 && entries * channels * static_cast<int64_t>(sizeof(T)) < (int64_t(1) << 32) && (spans <= 64 || entries <= 65536))
     {
-        // as many channels per workgroup as fit (the fewer workgroups share a line of the gradient, the
-        // less often it is read), but a workgroup for every compute unit
-        int64_t group = fit < channels ? fit : channels;
-        while (group > 1 && static_cast<int64_t>(b) * tpk_ceil_div(channels, group) < 256)
-            group = (group + 1) / 2;
-        const int64_t blocks = static_cast<int64_t>(b) * tpk_ceil_div(channels, group);
-        if (blocks <= 0x7fffffffLL)
-        {
-            const size_t lds = static_cast<size_t>(group * cub) * sizeof(T);
-            const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(cubic_scatter_lds_kernel<T>), lds);
-            if (allowed != TPK_OK)
-                return allowed;
-            hipLaunchKernelGGL(cubic_scatter_lds_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(CS_THREADS), lds, s, n_pts, static_cast<int>(nv), channels,
-                               static_cast<int>(group), cub, grad_point_features, grid_pt_indexes, grad_cubic_features);
-            return tpk_launch_status();
-        }
+        if (channels > 32)
+            return launch_spans<T, 64>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
+        if (channels > 16)
+            return launch_spans<T, 32>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
+        return launch_spans<T, 16>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
     }
     st = fill_zero<T>(static_cast<int64_t>(b) * channels * cub, grad_cubic_features, s);
     if (st != TPK_OK || total == 0)
@@ -674,20 +1001,46 @@ extern "C" int tpk_gridding_batch_grad_f64(int b, int n_pts, double scale, const
     return gridding_batch_grad<double>(b, n_pts, scale, ptcloud, grad_grid, grad_ptcloud, tpk_stream(stream));
 }
 
+extern "C" size_t tpk_cubic_feature_sampling_workspace_bytes(int b, int n_pts, int channels, int scale, int neighborhood_size,
+                                                             int element_bytes)
+{
+    const int64_t nv = cubic_vertices(neighborhood_size);
+    if (b <= 0 || n_pts <= 0 || channels <= 0 || scale <= 0 || scale > 1290 || nv < 0 || (element_bytes != 4 && element_bytes != 8) ||
+        !cubic_turns(b, n_pts, channels, scale, nv))
+        return 0;
+    return static_cast<size_t>(b) * channels * (static_cast<size_t>(scale) * scale * scale) * element_bytes;
+}
+
 extern "C" int tpk_cubic_feature_sampling_f32(int b, int n_pts, int channels, int scale, int neighborhood_size,
                                               const float* ptcloud, const float* cubic_features, float* point_features,
                                               int32_t* grid_pt_indexes, void* stream)
 {
-    return cubic_fwd<float>(b, n_pts, channels, scale, neighborhood_size, ptcloud, cubic_features, point_features,
-                            grid_pt_indexes, tpk_stream(stream));
+    return cubic_fwd<float>(b, n_pts, channels, scale, neighborhood_size, false, ptcloud, cubic_features, point_features,
+                         grid_pt_indexes, nullptr, 0, tpk_stream(stream));
+}
+
+extern "C" int tpk_cubic_feature_sampling_ws_f32(int b, int n_pts, int channels, int scale, int neighborhood_size, int mapped,
+                                                const float* ptcloud, const float* cubic_features, float* point_features,
+                                                int32_t* grid_pt_indexes, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return cubic_fwd<float>(b, n_pts, channels, scale, neighborhood_size, mapped != 0, ptcloud, cubic_features, point_features,
+                         grid_pt_indexes, workspace, workspace_bytes, tpk_stream(stream));
 }
 
 extern "C" int tpk_cubic_feature_sampling_f64(int b, int n_pts, int channels, int scale, int neighborhood_size,
-                                              const double* ptcloud, const double* cubic_features,
-                                              double* point_features, int32_t* grid_pt_indexes, void* stream)
+                                              const double* ptcloud, const double* cubic_features, double* point_features,
+                                              int32_t* grid_pt_indexes, void* stream)
 {
-    return cubic_fwd<double>(b, n_pts, channels, scale, neighborhood_size, ptcloud, cubic_features, point_features,
-                             grid_pt_indexes, tpk_stream(stream));
+    return cubic_fwd<double>(b, n_pts, channels, scale, neighborhood_size, false, ptcloud, cubic_features, point_features,
+                         grid_pt_indexes, nullptr, 0, tpk_stream(stream));
+}
+
+extern "C" int tpk_cubic_feature_sampling_ws_f64(int b, int n_pts, int channels, int scale, int neighborhood_size, int mapped,
+                                                const double* ptcloud, const double* cubic_features, double* point_features,
+                                                int32_t* grid_pt_indexes, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return cubic_fwd<double>(b, n_pts, channels, scale, neighborhood_size, mapped != 0, ptcloud, cubic_features, point_features,
+                         grid_pt_indexes, workspace, workspace_bytes, tpk_stream(stream));
 }
 
 extern "C" int tpk_cubic_feature_sampling_grad_f32(int b, int n_pts, int channels, int scale, int neighborhood_size,

@@ -831,8 +831,9 @@ at::Tensor gridding_batch_backward(const at::Tensor& ptcloud, double scale, cons
 }
 
 // cuda/src/cubic_feature_sampling.cpp:4-16 -> {point_features, grid_pt_indexes}
-std::vector<at::Tensor> cubic_feature_sampling(int scale, int neighborhood_size, at::Tensor ptcloud,
-                                               at::Tensor cubic_features)
+// mapped: ptcloud in [-1, 1), as the front end takes it.
+std::vector<at::Tensor> sample_cubes(int scale, int neighborhood_size, const at::Tensor& ptcloud, const at::Tensor& cubic_features,
+                                     bool mapped)
 {
     check_gpu(ptcloud, "ptcloud");
     check_gpu(cubic_features, "cubic_features");
@@ -853,22 +854,34 @@ std::vector<at::Tensor> cubic_feature_sampling(int scale, int neighborhood_size,
     const int64_t side = 2 * static_cast<int64_t>(neighborhood_size), vertices = side * side * side;
     at::Tensor features = torch::empty({b, n, vertices, channels}, ptcloud.options());
     at::Tensor indexes = torch::empty({b, n, vertices}, ptcloud.options().dtype(at::kInt));
-    if (ptcloud.scalar_type() == at::kFloat)
-        check_status(tpk_cubic_feature_sampling_f32(b, n, channels, scale, neighborhood_size, ptcloud.data_ptr<float>(),
-                                                    cubic_features.data_ptr<float>(), features.data_ptr<float>(),
-                                                    indexes.data_ptr<int32_t>(), current_stream(ptcloud)),
+    const bool single = ptcloud.scalar_type() == at::kFloat;
+    const size_t ws_bytes = tpk_cubic_feature_sampling_workspace_bytes(b, n, channels, scale, neighborhood_size, single ? 4 : 8);
+    at::Tensor ws;
+    if (ws_bytes)
+        ws = at::empty({static_cast<int64_t>(ws_bytes)}, ptcloud.options().dtype(at::kByte));
+    void* wsp = ws_bytes ? ws.data_ptr() : nullptr;
+    if (single)
+        check_status(tpk_cubic_feature_sampling_ws_f32(b, n, channels, scale, neighborhood_size, mapped, ptcloud.data_ptr<float>(),
+                                                       cubic_features.data_ptr<float>(), features.data_ptr<float>(),
+                                                       indexes.data_ptr<int32_t>(), wsp, ws_bytes, current_stream(ptcloud)),
                      "cubic_feature_sampling");
     else
-        check_status(tpk_cubic_feature_sampling_f64(b, n, channels, scale, neighborhood_size, ptcloud.data_ptr<double>(),
-                                                    cubic_features.data_ptr<double>(), features.data_ptr<double>(),
-                                                    indexes.data_ptr<int32_t>(), current_stream(ptcloud)),
+        check_status(tpk_cubic_feature_sampling_ws_f64(b, n, channels, scale, neighborhood_size, mapped, ptcloud.data_ptr<double>(),
+                                                       cubic_features.data_ptr<double>(), features.data_ptr<double>(),
+                                                       indexes.data_ptr<int32_t>(), wsp, ws_bytes, current_stream(ptcloud)),
                      "cubic_feature_sampling");
     return {features, indexes};
 }
 
+std::vector<at::Tensor> cubic_feature_sampling(int scale, int neighborhood_size, at::Tensor ptcloud,
+                                               at::Tensor cubic_features)
+{
+    return sample_cubes(scale, neighborhood_size, ptcloud, cubic_features, false);
+}
+
 // cuda/src/cubic_feature_sampling.cpp:18-30 -> {grad_ptcloud, grad_cubic_features}
-std::vector<at::Tensor> cubic_feature_sampling_grad(int scale, int neighborhood_size, at::Tensor grad_point_features,
-                                                    at::Tensor grid_pt_indexes)
+std::vector<at::Tensor> sample_cubes_grad(int scale, int neighborhood_size, const at::Tensor& grad_point_features,
+                                          const at::Tensor& grid_pt_indexes, bool points_too)
 {
     check_gpu(grad_point_features, "grad_point_features");
     check_gpu(grid_pt_indexes, "grid_pt_indexes");
@@ -887,21 +900,29 @@ std::vector<at::Tensor> cubic_feature_sampling_grad(int scale, int neighborhood_
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(grad_point_features.device());
     const int b = as_int(grad_point_features.size(0), "batch size"), n = as_int(grid_pt_indexes.size(1), "number of points");
     const int channels = as_int(grad_point_features.size(3), "channels");
-    at::Tensor grad_ptcloud = torch::empty({b, n, 3}, grad_point_features.options());
+    at::Tensor grad_ptcloud;
+    if (points_too)
+        grad_ptcloud = torch::empty({b, n, 3}, grad_point_features.options());
     at::Tensor grad_cubic = torch::empty({b, channels, scale, scale, scale}, grad_point_features.options());
     if (grad_point_features.scalar_type() == at::kFloat)
         check_status(tpk_cubic_feature_sampling_grad_f32(b, n, channels, scale, neighborhood_size,
                                                          grad_point_features.data_ptr<float>(),
-                                                         grid_pt_indexes.data_ptr<int32_t>(), grad_ptcloud.data_ptr<float>(),
+                                                         grid_pt_indexes.data_ptr<int32_t>(), points_too ? grad_ptcloud.data_ptr<float>() : nullptr,
                                                          grad_cubic.data_ptr<float>(), current_stream(grad_point_features)),
                      "cubic_feature_sampling_grad");
     else
         check_status(tpk_cubic_feature_sampling_grad_f64(b, n, channels, scale, neighborhood_size,
                                                          grad_point_features.data_ptr<double>(),
-                                                         grid_pt_indexes.data_ptr<int32_t>(), grad_ptcloud.data_ptr<double>(),
+                                                         grid_pt_indexes.data_ptr<int32_t>(), points_too ? grad_ptcloud.data_ptr<double>() : nullptr,
                                                          grad_cubic.data_ptr<double>(), current_stream(grad_point_features)),
                      "cubic_feature_sampling_grad");
     return {grad_ptcloud, grad_cubic};
+}
+
+std::vector<at::Tensor> cubic_feature_sampling_grad(int scale, int neighborhood_size, at::Tensor grad_point_features,
+                                                    at::Tensor grid_pt_indexes)
+{
+    return sample_cubes_grad(scale, neighborhood_size, grad_point_features, grid_pt_indexes, true);
 }
 
 // No counterpart in the reference's native module: its grouping_operation is
@@ -1127,6 +1148,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("gridding", &gridding);
     m.def("gridding_grad", &gridding_grad);
     m.def("gridding_batch", &gridding_batch);
+    m.def("cubic_sampling", &cubic_sampling);
     m.def("cubic_feature_sampling", &cubic_feature_sampling);
     m.def("cubic_feature_sampling_grad", &cubic_feature_sampling_grad);
     m.def("three_interpolate", &three_interpolate);
