@@ -1142,6 +1142,30 @@ def test_grow_proximity_any_matrix(tpk, oracle, dev):
                 assert got == (want if reference_order else [sorted(c) for c in want])
 
 
+# ------------------------------------------------------------------ sampling pools
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 960, 961, 1920, 1921, 3840, 3841, 5760, 5761, 11520, 11521, 16384])
+def test_fps_pools_at_the_edges_of_the_shapes(tpk, oracle, dev, n):
+    """Sizes on both sides of every register shape; clouds without ties, with every point held twice (ties inside a pool),
+    with 100 copies of ten far points (more equal minima than a pool takes), all but a few points near the origin
+    (nothing left above zero), and a coordinate that is not finite (a point that never falls to zero)."""
+    g = torch.Generator().manual_seed(n)
+    plain = torch.rand(n, 3, generator=g) + 0.1
+    twice = plain[: (n + 1) // 2].repeat(2, 1)[:n]
+    crowd = plain.clone()
+    copies = torch.arange(min(n, 1000))
+    crowd[n - copies.numel() :] = 3.0 + (copies % 10).float().unsqueeze(1) * torch.tensor([1.0, 0.5, 0.25])
+    few = 0.001 * plain
+    few[:: max(1, n // 7)] += 1.0
+    odd = plain.clone()
+    odd[n // 2, 1] = float("nan")
+    clouds = torch.stack([plain, twice, crowd, few, odd])
+    npoint = min(n, 700)
+    got = tpk.furthest_point_sample(clouds.to(dev), npoint)
+    np.testing.assert_array_equal(_np(got), oracle.furthest_point_sample(clouds.numpy(), npoint))
+
+
 # ------------------------------------------------------------------ instance IoU
 
 

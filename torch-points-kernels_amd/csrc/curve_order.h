@@ -205,9 +205,9 @@ __device__ __forceinline__ void curve_order(const float* __restrict__ xyz, int n
     for (int i = tid; i < CURVE_BINS; i += THREADS)
     {
         bins[i] = 0;
-        // curve position of every cell of the 16^3 grid, computed once per cell instead of once
-        // per point; the table borrows sort_keys, which the scatter fills only later
-        sort_keys[i] = curve_bin_of_cell(i & 15, (i >> 4) & 15, i >> 8);
+        // curve position of every cell of the 16^3 grid, from the table made at compile time (computed here it was
+        // 4 us of a kernel); its copy borrows sort_keys, which the scatter fills only later
+        sort_keys[i] = curve_bin_table.bin[i];
     }
     __syncthreads();
     {

@@ -2,21 +2,17 @@
 // the chosen set, pick the point whose distance is largest".
 //
 // One workgroup (one compute unit) owns a cloud for the whole call; the rounds of a cloud
-// depend on each other, so a call runs as many workgroups as there are clouds.  Four kernels
+// depend on each other, so a call runs as many workgroups as there are clouds.  Three kernels
 // by cloud size:
-//   up to 512 points     fps_resident_kernel: one point per lane in registers, every point
-//                        updated every round, one 24-byte LDS record per wavefront and one
-//                        barrier per round (records double buffered);
-//   up to 16384 points   fps_pruned_kernel: up to 32 points per lane in registers, cloud
-//                        ordered along a space filling curve so that most updates can be
-//                        skipped exactly (described at the kernel);
+//   up to 16384 points   fps_pool_kernel: up to 18 points per lane in registers, cloud ordered along
+//                        a space filling curve so that most updates can be skipped exactly; one
+//                        wavefront takes dozens of samples per round from a pool (described at the kernel);
 //   up to 163840 points  fps_cells_batched_kernel: the cloud ordered along the curve into cells of 64
 //                        points that stay in memory (the caller's workspace); boxes, largest
 //                        distance and best point of every cell in LDS; a round touches only
 //                        the cells the new sample can change (described at the kernel);
-//   larger clouds        fps_streaming_kernel: the selection code of the first kernel over
-//                        points streamed from global memory, running minima in a workspace
-//                        provided by the caller.
+//   larger clouds        fps_streaming_kernel: every point updated every round, points streamed from
+//                        global memory, running minima in a workspace provided by the caller.
 // In all of them the chosen point's coordinates travel through LDS with the selection: the
 // chosen point is never re-read from memory.
 //
@@ -109,185 +105,42 @@ __device__ __forceinline__ bool eligible(float x, float y, float z)
     return !(static_cast<double>(mag) <= 1e-3);
 }
 
-// First slot whose value equals `value` (per lane; used only when lanes tie).
-template <int PPT>
-__device__ __forceinline__ int first_slot_equal(const int (&t)[PPT], int value)
-{
-    int slot = PPT - 1;
-#pragma unroll
-    for (int i = PPT - 2; i >= 0; --i)
-        slot = t[i] == value ? i : slot;
-    return slot;
-}
-
-template <int PPT, int THREADS>
-__global__ __launch_bounds__(THREADS) void fps_resident_kernel(
-    int n, int npoint, int log2_bs, int groups, const float* __restrict__ xyz,
-    int32_t* __restrict__ out)
-{
-    constexpr int WAVES = THREADS / TPK_WAVE;
-    constexpr int NG = PPT >= 4 ? PPT / 4 : 1; // slots are searched in groups of GS
-    constexpr int GS = PPT / NG;
-    __shared__ WaveRecord records[2][WAVES];
-
-    xyz += static_cast<int64_t>(blockIdx.x) * n * 3;
-    out += static_cast<int64_t>(blockIdx.x) * npoint;
-    const int tid = threadIdx.x;
-    const int lane = tid & (TPK_WAVE - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
-
-    // Lane `tid` owns points tid, tid + THREADS, ...: ascending slot = ascending tie key
-    // (THREADS is a multiple of the reference's block size).  The running minimum of a point
-    // is held as the bit pattern of a non-negative float, which orders like a signed
-    // integer; an ineligible or absent point holds the pattern of -1.0f (negative as an
-    // integer), which an integer min against any distance keeps forever.
-    float x[PPT], y[PPT], z[PPT];
-    int t[PPT];
-#pragma unroll
-    for (int i = 0; i < PPT; ++i)
-    {
-        const int k = tid + THREADS * i;
-        bool ok = false;
-        float px = 0.f, py = 0.f, pz = 0.f;
-        if (k < n)
-        {
-            px = xyz[k * 3 + 0];
-            py = xyz[k * 3 + 1];
-            pz = xyz[k * 3 + 2];
-            ok = eligible(px, py, pz);
-        }
-        x[i] = ok ? px : 0.f;
-        y[i] = ok ? py : 0.f;
-        z[i] = ok ? pz : 0.f;
-        t[i] = ordered_bits(ok ? 1e10f : -1.0f);
-    }
-
-    const unsigned bs_mask = (1u << log2_bs) - 1u;
-    const unsigned rev = log2_bs ? (__brev(tid & bs_mask) >> (32 - log2_bs)) : 0u;
-    const unsigned tk_base = rev * static_cast<unsigned>(groups);
-
-    const float p0x = xyz[0], p0y = xyz[1], p0z = xyz[2];
-    float sx = p0x, sy = p0y, sz = p0z;
-    if (tid == 0)
-        out[0] = 0;
-
-    for (int j = 1; j < npoint; ++j)
-    {
-        // 1. distance update: 8 double-rate fp32 operations + one integer min per point
-        const float vx = to_vector_register(sx);
-        const float vy = to_vector_register(sy);
-        const float vz = to_vector_register(sz);
-        int g[NG];
-#pragma unroll
-        for (int gi = 0; gi < NG; ++gi)
-        {
-#pragma unroll
-            for (int e = 0; e < GS; ++e)
-            {
-                const int i = gi * GS + e;
-                const float d = tpk_dist2(x[i], y[i], z[i], vx, vy, vz);
-                t[i] = min(t[i], ordered_bits(d));
-                g[gi] = e == 0 ? t[i] : max(g[gi], t[i]);
-            }
-        }
-        int best = g[0];
-#pragma unroll
-        for (int gi = 1; gi < NG; ++gi)
-            best = max(best, g[gi]);
-
-        // 2. wavefront maximum and the lane that owns it
-        const int wave_val = wave_max_i32(best);
-        const unsigned long long top = __ballot(best == wave_val);
-        int wl;
-        if (__builtin_popcountll(top) == 1)
-        {
-            wl = __builtin_ctzll(top);
-        }
-        else
-        {
-            // several lanes hold the maximum: the smallest tie key decides
-            const int bi = first_slot_equal<PPT>(t, best);
-            const unsigned my_tk = tk_base + (static_cast<unsigned>(tid + THREADS * bi) >> log2_bs);
-            const unsigned cand = best == wave_val ? my_tk : 0xFFFFFFFFu;
-            const unsigned lowest = wave_min_u32(cand);
-            wl = __builtin_ctzll(__ballot(cand == lowest));
-        }
-        // first slot of lane wl holding the maximum: its group first, then inside the group
-        // (wave-uniform control flow; only lane reads, no per-lane bookkeeping in step 1)
-        int grp = NG - 1;
-#pragma unroll
-        for (int gi = NG - 2; gi >= 0; --gi)
-            grp = __builtin_amdgcn_readlane(g[gi], wl) == wave_val ? gi : grp;
-        int slot = 0;
-        float cx = 0.f, cy = 0.f, cz = 0.f;
-#pragma unroll
-        for (int gi = 0; gi < NG; ++gi)
-            if (grp == gi)
-            {
-                int e_sel = GS - 1;
-#pragma unroll
-                for (int e = GS - 2; e >= 0; --e)
-                    e_sel = __builtin_amdgcn_readlane(t[gi * GS + e], wl) == wave_val ? e : e_sel;
-#pragma unroll
-                for (int e = 0; e < GS; ++e)
-                    if (e_sel == e)
-                    {
-                        slot = gi * GS + e;
-                        cx = tpk_read_lane(x[gi * GS + e], wl);
-                        cy = tpk_read_lane(y[gi * GS + e], wl);
-                        cz = tpk_read_lane(z[gi * GS + e], wl);
-                    }
-            }
-        const int win_tid = wave * TPK_WAVE + wl;
-        const int win_k = win_tid + THREADS * slot;
-        const unsigned win_rev = log2_bs ? (__brev(win_tid & bs_mask) >> (32 - log2_bs)) : 0u;
-        WaveRecord r;
-        r.val = wave_val;
-        r.tk = win_rev * static_cast<unsigned>(groups) + (static_cast<unsigned>(win_k) >> log2_bs);
-        r.k = win_k;
-        r.x = cx;
-        r.y = cy;
-        r.z = cz;
-        if (lane == 0)
-            records[j & 1][wave] = r;
-        __syncthreads();
-
-        // 3. all wavefronts reduce the records
-        int k;
-        int gv_unused;
-        reduce_records<WAVES>(records[j & 1], lane, p0x, p0y, p0z, k, sx, sy, sz, gv_unused);
-        if (tid == 0)
-            out[j] = k;
-    }
-}
-
 // ---------------------------------------------------------------------------------------
-// Register-resident kernel with exact pruning, for clouds of a few thousand to 16384 points.
+// Register-resident kernel with exact pruning and pools of samples, for clouds up to 16384 points.
 //
-// Pruning.  A point's running minimum changes in a round only if its distance to the new
-// sample is smaller than that minimum, and no minimum exceeds the value that won the previous
-// round.  So a set of points whose bounding box is further from the new sample than the square
-// root of the previous winning value cannot change, and its update can be skipped without
-// changing any result.  To make such sets exist, the kernel first orders the cloud along a
-// Hilbert curve (12-bit position of its cell in a 16^3 grid, counting sort in LDS) and cuts the curve into cells of
-// 64 * GS consecutive points.  A cell is GS registers of the 64 lanes of one wavefront; every
-// wavefront holds NG cells, taken round-robin along the curve so that the cells around a
-// sample belong to different wavefronts.  A wavefront tests its NG boxes at once, lane g
-// testing the box of its group g, and updates only the live groups (wave-uniform branches).
-// The fp32 box distance is compared with a relative margin of 2e-6, several times the rounding
-// error of either side, so a skipped update is provably a no-op.
+// Pools.  A round takes many samples.  After its updates let the pool be all points whose running
+// minimum lies above some floor; no point outside it holds more than the floor, and minima only
+// fall.  So as long as the largest minimum inside the pool lies above the floor, it is the largest
+// of the cloud, its point is the next sample, and only the pool's minima have to be brought up to date
+// to find the one after it.  A pool of at most 64 points is a lane each of ONE wavefront, and the
+// whole sequence runs in its registers: maximum over the lanes, the point's coordinates by lane
+// reads, one distance per lane - a chain of 40 dependent instructions, 0.1 us, without a barrier or
+// a trip to LDS.  On the clouds this was made for a pool of 44 gives about 31 samples.  (The version before
+// let every wavefront offer its two best points and took those that did not change each other: 8
+// samples per round, 0.37 us each; now 0.2.  Two points per lane in the pool would save two rounds of five and
+// cost every step a third more.)
 //
-// Selection.  Each lane keeps the largest and second largest running minimum of every group; a
-// wavefront publishes its two best points of different lanes (value, coordinates, sorted
-// position: found per lane by compare/select, then through wave-uniform, GPR-indexed register
-// reads) and the largest minimum it keeps to itself, and a round takes as many of the published
-// points as follow each other as samples (described where the loop begins): several samples per
-// round, each round's box tests one instruction sequence whatever their number.
+// Two kinds of wavefronts.  Wavefront 0 samples pools and holds no points.  The others hold the cloud,
+// PPT points per lane; while wavefront 0 samples they bring their points up to date with the samples
+// it has published so far (8 at a time, through LDS), and when it reports the end of the pool they gather
+// the next one.  What share below the largest minimum makes a pool of the wanted size is carried from round
+// to round; a pool that came out empty or too full is gathered again.
 //
-// Equal maxima.  When several points hold the maximum, or no point is eligible, the round takes one
-// sample by the reference's tie key over all points holding the maximum, through a copy of the
-// running minima in LDS (slots are not in index order here, so the key is computed from the
-// original index kept in the sort keys).
+// Pruning.  A point's running minimum changes only if its distance to the new sample is smaller
+// than that minimum, and no minimum exceeds the one the round's first sample held.  So a set of
+// points whose bounding box is further from the sample than the square root of that value cannot
+// change, and its update can be skipped without changing any result.  To make such sets exist, the
+// kernel first orders the cloud along a Hilbert curve (12-bit position of its cell in a 16^3 grid,
+// counting sort in LDS) and cuts the curve into cells of 64 * GS consecutive points.  A cell is GS
+// registers of the 64 lanes of one wavefront; cells go round-robin to the wavefronts, so the cells around a
+// sample belong to different ones.  A wavefront tests its up to 8 boxes against 8 samples at
+// once, a lane per pair, and updates only what is reached (wave-uniform branches).  The fp32 box
+// distance is compared with a relative margin of 2e-6, several times the rounding error of either
+// side, so a skipped update is provably a no-op.
+//
+// Equal maxima inside a pool go by the reference's tie key.  When more points hold the same value than
+// a pool takes, when nothing above zero is left, or when a coordinate is not finite (such a point never
+// falls to zero), rounds take one sample by the tie key over all points holding the maximum.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ unsigned tie_key(int k, int log2_bs, int ref_groups)
 {
@@ -296,23 +149,11 @@ __device__ __forceinline__ unsigned tie_key(int k, int log2_bs, int ref_groups)
     return rev * static_cast<unsigned>(ref_groups) + (static_cast<unsigned>(k) >> log2_bs);
 }
 
-// Register arrays of the sorted kernel are vector types: the winner's slot is a wave-uniform
-// number known only at run time, and indexing a vector register tuple with a uniform index
-// is one move in GPR-index mode (an array would be indexed through scratch memory).
-template <int N>
-struct RegisterVector
-{
-    typedef float floats __attribute__((ext_vector_type(N)));
-    typedef int ints __attribute__((ext_vector_type(N)));
-};
-
 // The words of LDS through which the wavefronts of a workgroup agree on a round's winner.
 struct RoundWords
 {
     int max_val;      // atomic max of the running minima (bit patterns), starts at INT_MIN
-    int winners;      // 1 when exactly one point holds max_val, more when several may
-    unsigned min_tie; // atomic min of the tie keys of the points holding max_val (ties only)
-    int pad;
+    unsigned min_tie; // atomic min of the tie keys of the points holding max_val
 };
 
 // LDS atomics without return value, issued as written: one instruction for the active lanes
@@ -326,56 +167,91 @@ __device__ __forceinline__ void lds_atomic_max_i32(int* p, int v)
 {
     asm volatile("ds_max_i32 %0, %1" ::"v"(lds_offset(p)), "v"(v) : "memory");
 }
-__device__ __forceinline__ void lds_atomic_add_u32(int* p, int v)
+
+// Largest value of the wavefront as a scalar: DPP maxima inside the rows of 16 lanes, then from row to row; six
+// dependent steps and one lane read.
+__device__ __forceinline__ int wave_max_to_scalar(int v)
 {
-    asm volatile("ds_add_u32 %0, %1" ::"v"(lds_offset(p)), "v"(v) : "memory");
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true));  // quad_perm [1,0,3,2]
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true));  // quad_perm [2,3,0,1]
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true)); // row_half_mirror
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true)); // row_mirror
+    v = max(v, __builtin_amdgcn_update_dpp(INT_MIN, v, 0x142, 0xA, 0xF, false)); // row_bcast:15 into rows 1 and 3
+    v = max(v, __builtin_amdgcn_update_dpp(INT_MIN, v, 0x143, 0xC, 0xF, false)); // row_bcast:31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(v, TPK_WAVE - 1);
 }
 
-// Position on the sorted curve of member `e` of group `g` held by lane `lane` of wavefront `wave`.
-template <int WAVES, int GS>
-__device__ __forceinline__ int sorted_position(int g, int wave, int e, int lane)
+// Position on the sorted curve of member `e` of group `g` held by lane `lane` of worker `worker`.
+template <int WORKERS, int GS>
+__device__ __forceinline__ int sorted_position(int g, int worker, int e, int lane)
 {
-    return ((g * WAVES + wave) * GS + e) * TPK_WAVE + lane;
+    return ((g * WORKERS + worker) * GS + e) * TPK_WAVE + lane;
 }
 
-template <int PPT, int THREADS, int GS>
-__global__ __launch_bounds__(THREADS) void fps_pruned_kernel(
+constexpr int POOL_CAPACITY = 2 * TPK_WAVE; // points gathered at most; the best 64 are sampled
+constexpr int POOL_TARGET = 60;
+constexpr int POOL_TRIES = 8;
+constexpr int POOL_BATCH = 8;   // samples published at a time: one per lane of a row of 8
+constexpr int POOL_DONE = 1 << 16;
+
+// ORDERED: the cloud is ordered along the curve and updates are pruned.  Small clouds are taken as they come: all their
+// points can be brought up to date in less time than a sample takes, and the ordering alone is 8 us.
+template <int PPT, int WAVES, int GS, bool ORDERED>
+__global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
     int n, int npoint, int log2_bs, int ref_groups, int key_capacity,
     const float* __restrict__ xyz, int32_t* __restrict__ out)
 {
-    constexpr int WAVES = THREADS / TPK_WAVE;
+    constexpr int THREADS = WAVES * TPK_WAVE;
+    constexpr int WORKERS = WAVES - 1;
     constexpr int NG = PPT / GS;
-    static_assert(NG <= 16, "one DPP row of lanes tests the group boxes");
-    static_assert(WAVES >= 2, "a cloud without eligible points must count several winners");
-    // key_capacity keys (curve position << 20) | index in curve order, kept for the whole kernel; then
-    // PPT * THREADS words (the unsorted keys during set-up, later the copy of the running minima
-    // made when equal maxima have to be resolved); then the bins of the counting sort
+    static_assert(NG * GS == PPT && NG * POOL_BATCH <= TPK_WAVE, "a row of 8 lanes tests each group");
+    // key_capacity keys (curve position << 20) | index in curve order, kept for the whole kernel; then, during
+    // set-up, key_capacity unsorted keys and the bins of the counting sort
     extern __shared__ unsigned sort_keys[];
-    int* const t_copy = reinterpret_cast<int*>(sort_keys + key_capacity);
     unsigned* const unsorted = sort_keys + key_capacity;
-    int* const bins = t_copy + PPT * THREADS; // CURVE_BINS words
+    int* const bins = reinterpret_cast<int*>(unsorted + key_capacity); // CURVE_BINS words
     __shared__ int wave_totals[WAVES];
     __shared__ RoundWords words[2];
     __shared__ int cloud_box[6];      // ordered ints: min x,y,z then max x,y,z
-    __shared__ int group_box[WAVES * NG * 6]; // the same per (wavefront, group) cell
+    __shared__ __align__(16) float4 group_lo[WORKERS * NG], group_hi[WORKERS * NG]; // box of every (worker, group) cell
+    __shared__ __align__(16) float4 pool[POOL_CAPACITY]; // x, y, z, sorted position of the pool's points
+    __shared__ int pool_min[POOL_CAPACITY];              // their running minima
+    __shared__ int pool_count[3];                   // one per attempt, in turn
+    __shared__ __align__(16) float4 taken[TPK_WAVE]; // the round's samples
+    // By round: how many of them stand in taken[] (POOL_DONE: there will be no more), the first one's minimum,
+    // what no minimum exceeds when all their updates are made; last the exclusive or of the three.
+    __shared__ __align__(16) int4 published[2];
+    __shared__ int pool_best[TPK_WAVE]; // where its best 64 stand, if it holds more
+    __shared__ int not_finite;
 
     xyz += static_cast<int64_t>(blockIdx.x) * n * 3;
     out += static_cast<int64_t>(blockIdx.x) * npoint;
     const int tid = threadIdx.x;
     const int lane = tid & (TPK_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
+    const int worker = wave - 1;
+    auto original_index = [&](int position) { return ORDERED ? static_cast<int>(sort_keys[position] & 0x3FFFu) : position; };
 
     // ---- set-up 1 and 2: order the cloud along the curve (curve_order.h)
     if (tid < 2)
-        words[tid] = RoundWords{INT_MIN, 0, 0xFFFFFFFFu, 0};
-    curve_order<THREADS>(xyz, n, sort_keys, unsorted, bins, cloud_box, wave_totals);
+    {
+        words[tid] = RoundWords{INT_MIN, 0xFFFFFFFFu};
+        published[tid] = int4{0, 0, 0, 0};
+    }
+    if (tid < 3)
+        pool_count[tid] = 0;
+    if (tid == 0)
+        not_finite = 0;
+    if constexpr (ORDERED)
+        curve_order<THREADS>(xyz, n, sort_keys, unsorted, bins, cloud_box, wave_totals);
+    else
+        __syncthreads();
 
     // ---- set-up 3: this lane's points.  The curve is cut into cells of 64 * GS consecutive
-    // points; cell c belongs to wavefront c % WAVES as its group c / WAVES (neighbouring cells
-    // go to different wavefronts, which spreads the work around a sample).  Slot i of a lane =
+    // points; cell c belongs to worker c % WORKERS as its group c / WORKERS.  Slot i of a lane =
     // group (i / GS), member (i % GS); see sorted_position().
-    typename RegisterVector<PPT>::floats x, y, z;
-    typename RegisterVector<PPT>::ints t;
+    float x[PPT], y[PPT], z[PPT];
+    int t[PPT];
 #pragma unroll
     for (int gi = 0; gi < NG; ++gi)
     {
@@ -385,10 +261,12 @@ __global__ __launch_bounds__(THREADS) void fps_pruned_kernel(
         for (int e = 0; e < GS; ++e)
         {
             const int i = gi * GS + e;
-            const int q = sorted_position<WAVES, GS>(gi, wave, e, lane);
-            const int k = static_cast<int>(sort_keys[q < n ? q : 0] & 0x3FFFu);
+            const int q = worker >= 0 ? sorted_position<WORKERS, GS>(gi, worker, e, lane) : n;
+            const int k = original_index(q < n ? q : 0);
             const float px = xyz[k * 3 + 0], py = xyz[k * 3 + 1], pz = xyz[k * 3 + 2];
             const bool ok = q < n && eligible(px, py, pz);
+            if (ok && !(px - px == 0.f && py - py == 0.f && pz - pz == 0.f))
+                not_finite = 1;
             x[i] = ok ? px : 0.f;
             y[i] = ok ? py : 0.f;
             z[i] = ok ? pz : 0.f;
@@ -400,289 +278,313 @@ __global__ __launch_bounds__(THREADS) void fps_pruned_kernel(
             hi[1] = ok ? fmaxf(hi[1], py) : hi[1];
             hi[2] = ok ? fmaxf(hi[2], pz) : hi[2];
         }
+        if constexpr (!ORDERED)
+            continue;
         // the cell belongs to this wavefront alone: reduce over its lanes, plain store
 #pragma unroll
         for (int a = 0; a < 3; ++a)
         {
-            const int cell_lo = wave_min_i32(float_to_ordered_int(lo[a]));
-            const int cell_hi = wave_max_i32(float_to_ordered_int(hi[a]));
-            if (lane == 0)
-            {
-                group_box[(wave * NG + gi) * 6 + a] = cell_lo;
-                group_box[(wave * NG + gi) * 6 + 3 + a] = cell_hi;
-            }
+            lo[a] = ordered_int_to_float(wave_min_i32(float_to_ordered_int(lo[a])));
+            hi[a] = ordered_int_to_float(wave_max_i32(float_to_ordered_int(hi[a])));
+        }
+        if (lane == 0 && worker >= 0)
+        {
+            group_lo[worker * NG + gi] = make_float4(lo[0], lo[1], lo[2], 0.f);
+            group_hi[worker * NG + gi] = make_float4(hi[0], hi[1], hi[2], 0.f);
         }
     }
     __syncthreads();
-    // lane g of every 16-lane row tests this wavefront's group g; lanes beyond NG hold an empty box
-    // (row g of the lanes tests group g, its lane k against sample k of the round)
-    static_assert(NG <= 4, "one row of lanes per group");
-    const int my_group = lane >> 4;
-    float blo[3], bhi[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-    {
-        blo[a] = my_group < NG ? ordered_int_to_float(group_box[(wave * NG + my_group) * 6 + a]) : __builtin_inff();
-        bhi[a] = my_group < NG ? ordered_int_to_float(group_box[(wave * NG + my_group) * 6 + 3 + a]) : -__builtin_inff();
-    }
-
-    int g[NG]; // per-lane maximum of each group, kept across rounds
-#pragma unroll
-    for (int gi = 0; gi < NG; ++gi)
-    {
-        g[gi] = t[gi * GS];
-#pragma unroll
-        for (int e = 1; e < GS; ++e)
-            g[gi] = max(g[gi], t[gi * GS + e]);
-    }
-
     const float p0x = xyz[0], p0y = xyz[1], p0z = xyz[2];
-    int bound = ordered_bits(__builtin_inff()); // no running minimum exceeds this
-    const bool row_head = (lane & 15) == 0;
-    int best = g[0]; // this lane's largest running minimum and that of its row of 16 lanes
-#pragma unroll
-    for (int gi = 1; gi < NG; ++gi)
-        best = max(best, g[gi]);
     if (tid == 0)
+    {
         out[0] = 0;
+        taken[0] = make_float4(p0x, p0y, p0z, 0.f);
+    }
+    const bool one_by_one = __builtin_amdgcn_readfirstlane(not_finite) != 0;
+    __syncthreads();
     TPK_WORK_DECL
 
-    {
-        // Several samples per round.  After a round's updates let c0 > c1 > c2 ... be the points in the order of
-        // their running minima.  c0 is the next sample.  If c1's minimum is not changed by c0 (c0 is no closer
-        // to it than its minimum), then after c0's update c1 still holds what it held, nothing holds more, and
-        // c1 is the sample after c0 - and so on: ck follows as long as none of c0 .. c(k-1) changes its minimum.
-        // The largest minima sit in different corners of the cloud, far from each other, and a round takes eight
-        // samples on average.  Every wavefront publishes its two best points and the largest minimum it does
-        // not publish; after a barrier wavefront 0 sorts out the list - candidates above everything unpublished,
-        // strictly ordered (equal minima are left to the exact resolution below, one sample at a time), each
-        // unchanged by those before it - and after a second barrier all wavefronts apply the new samples'
-        // updates together: which of a wavefront's groups a sample can change is one box test per (group,
-        // sample), all of a round's in one instruction sequence.
-        constexpr int FPB_T = WAVES >= 16 ? 16 : 8; // samples per round at most (16: one lane of a row each in the box tests)
-        static_assert(FPB_T <= 16 && TPK_WAVE % FPB_T == 0, "the pair tests take whole rows of lanes");
-        constexpr int FPB_PUB = 2; // points a wavefront publishes per round (3: 1 % faster at best)
-        constexpr int CANDS = WAVES * FPB_PUB;
-        static_assert(CANDS % 4 == 0 && CANDS <= TPK_WAVE && CANDS > FPB_T, "one lane per published point");
-        __shared__ float4 cand_rec[2][CANDS];                // x, y, z, sorted position of the published points
-        __shared__ __align__(16) int cand_val[2][CANDS];     // their running minima (INT_MIN: nothing published)
-        __shared__ int hidden[2][WAVES];          // per wavefront: the largest minimum not published
-        int g2[NG]; // per lane: second largest of each group (g: the largest)
+    // The updates of samples first .. first + count - 1 (at most POOL_BATCH) of taken[]; `bound`: no running minimum
+    // exceeds it.  (Bit patterns of non-negative floats throughout.)
+    auto update = [&](int first, int count, int bound) __attribute__((always_inline)) {
+        // row r of 8 lanes tests this wavefront's group r, its lane k against sample k
+        const int k = lane % POOL_BATCH, group = lane / POOL_BATCH, cell = worker * NG + (group < NG ? group : 0);
+        const float4 s = taken[first + (k < count ? k : 0)];
+        if constexpr (!ORDERED)
+        {
+            for (int from = 0; from < count; ++from)
+            {
+                const float sx = to_vector_register(tpk_read_lane(s.x, from)), sy = to_vector_register(tpk_read_lane(s.y, from));
+                const float sz = to_vector_register(tpk_read_lane(s.z, from));
+                TPK_WORK_ADD(PPT);
+#pragma unroll
+                for (int i = 0; i < PPT; ++i)
+                    t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], sx, sy, sz)));
+            }
+            return;
+        }
+        const float4 lo = group_lo[cell], hi = group_hi[cell];
+        const float dx = fmaxf(fmaxf(lo.x - s.x, s.x - hi.x), 0.f);
+        const float dy = fmaxf(fmaxf(lo.y - s.y, s.y - hi.y), 0.f);
+        const float dz = fmaxf(fmaxf(lo.z - s.z, s.z - hi.z), 0.f);
+        const float lb = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)) * 0.999998f;
+        // an empty box gives lb = +inf (never live); NaN compares false -> live
+        const unsigned long long live = __ballot(k < count && group < NG && !(lb >= __int_as_float(bound)));
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi)
-        {
-            int a1 = INT_MIN, a2 = INT_MIN;
-#pragma unroll
-            for (int e = 0; e < GS; ++e)
+            for (unsigned reach = static_cast<unsigned>(live >> (gi * POOL_BATCH)) & 0xFFu; reach != 0; reach &= reach - 1)
             {
-                const int v = t[gi * GS + e];
-                a2 = max(a2, min(a1, v));
-                a1 = max(a1, v);
-            }
-            g2[gi] = a2;
-        }
-        // the samples whose updates are due: the round before's published points in the order of their minima
-        // (first: point 0), and which of them may follow each other
-        static_assert(FPB_PUB * CANDS <= TPK_WAVE && FPB_T <= WAVES, "a wavefront ranks its points in one step; one wavefront per place");
-        __shared__ int order[2][CANDS];             // published point of every place
-        __shared__ __align__(16) float4 taken[2][FPB_T]; // x, y, z, sorted position of the point of place k
-        __shared__ int follows[2][FPB_T];           // 1: the point of place k may follow those before it
-        __shared__ int largest[2];                  // the round's largest minimum
-        if (tid == 0)
-            taken[0][0] = make_float4(p0x, p0y, p0z, 0.f);
-        __syncthreads();
-        int ns = 1, from = 0;
-        // Clouds with equal minima at the top in round after round (lattices, repeated points) gain nothing from the
-        // list: after a round that had to fall back on the exact resolution the next `pause` rounds go there at
-        // once, twice as many each time it happens again, until a round takes several samples.
-        int pause = 0, penalty = 1, which = 0;
-        int j = 1;
-        for (int round = 1; j < npoint; ++round)
-        {
-            const int par = round & 1;
-            // 1. the updates of the round before's samples.  Which groups can change?  Lane k < FPB_T fetches
-            // sample k; row g of the lanes tests its lane's sample against group g.
-            const float4 fetched = taken[from][lane < ns ? lane : 0];
-            unsigned long long live;
-            {
-                const int k = lane & 15;
-                const float sx = __shfl(fetched.x, k, TPK_WAVE), sy = __shfl(fetched.y, k, TPK_WAVE), sz = __shfl(fetched.z, k, TPK_WAVE);
-                const float dx = fmaxf(fmaxf(blo[0] - sx, sx - bhi[0]), 0.f);
-                const float dy = fmaxf(fmaxf(blo[1] - sy, sy - bhi[1]), 0.f);
-                const float dz = fmaxf(fmaxf(blo[2] - sz, sz - bhi[2]), 0.f);
-                const float lb = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)) * 0.999998f;
-                // an empty box gives lb = +inf (never live); NaN compares false -> live
-                live = __ballot(k < ns && !(lb >= __int_as_float(bound)));
-            }
-#pragma unroll
-            for (int gi = 0; gi < NG; ++gi)
-            {
-                // samples that reach group gi, one bit each
-                unsigned reach = static_cast<unsigned>(live >> (gi * 16)) & 0xFFFFu;
-                if (reach == 0)
-                    continue; // (uniform over the wavefront)
-                while (reach != 0)
-                {
-                    const int k = __builtin_ctz(reach);
-                    reach &= reach - 1;
-                    const float sx = to_vector_register(tpk_read_lane(fetched.x, k)), sy = to_vector_register(tpk_read_lane(fetched.y, k));
-                    const float sz = to_vector_register(tpk_read_lane(fetched.z, k));
-                    TPK_WORK_ADD(GS);
-#pragma unroll
-                    for (int e = 0; e < GS; ++e)
-                    {
-                        const int i = gi * GS + e;
-                        t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], sx, sy, sz)));
-                    }
-                }
-                int a1 = INT_MIN, a2 = INT_MIN;
+                const int from = __builtin_ctz(reach); // (lanes 0 .. 7 hold samples 0 .. 7)
+                const float sx = to_vector_register(tpk_read_lane(s.x, from)), sy = to_vector_register(tpk_read_lane(s.y, from));
+                const float sz = to_vector_register(tpk_read_lane(s.z, from));
+                TPK_WORK_ADD(GS);
 #pragma unroll
                 for (int e = 0; e < GS; ++e)
                 {
-                    const int v = t[gi * GS + e];
-                    a2 = max(a2, min(a1, v));
-                    a1 = max(a1, v);
+                    const int i = gi * GS + e;
+                    t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], sx, sy, sz)));
                 }
-                g[gi] = a1;
-                g2[gi] = a2;
             }
-            // 2. the lane's largest and second largest minimum
-            int b1 = INT_MIN, b2 = INT_MIN;
-#pragma unroll
-            for (int gi = 0; gi < NG; ++gi)
-            {
-                b2 = max(max(b2, min(b1, g[gi])), g2[gi]);
-                b1 = max(b1, g[gi]);
-            }
-            best = b1;
-            if (pause == 0)
-            {
-                // 3. the wavefront's FPB_PUB best points (of different lanes) and the largest minimum it keeps to itself
-                // the slot of a lane's best point: group, then member (uniform indices into the registers)
-                auto publish = [&](int from_lane, int place) __attribute__((always_inline)) {
-                    int my_grp = 0;
-#pragma unroll
-                    for (int gi = NG - 1; gi >= 0; --gi)
-                        my_grp = g[gi] == b1 ? gi : my_grp;
-                    const int grp = __builtin_amdgcn_readlane(my_grp, from_lane);
-                    int my_e = 0;
-#pragma unroll
-                    for (int e = GS - 1; e >= 0; --e)
-                        my_e = t[grp * GS + e] == b1 ? e : my_e;
-                    const int ce = __builtin_amdgcn_readlane(my_e, from_lane);
-                    const int slot = grp * GS + ce;
-                    const float cx = x[slot], cy = y[slot], cz = z[slot];
-                    if (lane == from_lane)
-                    {
-                        cand_rec[par][place] = make_float4(cx, cy, cz, __int_as_float(sorted_position<WAVES, GS>(grp, wave, ce, lane)));
-                        cand_val[par][place] = b1;
-                    }
-                };
-                {
-                    int left = b1;                   // the lane's best point not yet published
-                    unsigned long long gone = 0ull;  // lanes whose best point is published
-                    int most = wave_max_i32(left);
-#pragma unroll
-                    for (int p = 0; p < FPB_PUB; ++p)
-                    {
-                        const int from_lane = __builtin_ctzll(__ballot(left == most));
-                        // (a lane's second point is not published: with it the list ends)
-                        const bool fresh = ((gone >> from_lane) & 1ull) == 0ull;
-                        if (fresh)
-                        {
-                            publish(from_lane, wave * FPB_PUB + p);
-                            gone |= 1ull << from_lane;
-                            left = lane == from_lane ? b2 : left;
-                            most = wave_max_i32(left);
-                        }
-                        else if (lane == 0)
-                            cand_val[par][wave * FPB_PUB + p] = INT_MIN;
-                    }
-                    if (lane == 0)
-                        hidden[par][wave] = most;
-                }
-                lds_barrier();
-                // 4. the list is sorted out by all wavefronts together, in two short steps.  First every wavefront
-                // finds the places of its own published points among all of them (lane (c, o): is point o above my
-                // point c? - equal values: the lower number first, so the places are distinct).
-                {
-                    const int c = lane / CANDS, o = lane % CANDS;
-                    const int mine = wave * FPB_PUB + (c < FPB_PUB ? c : 0);
-                    const int my_val = cand_val[par][mine], other = cand_val[par][o];
-                    const unsigned long long above = __ballot(c < FPB_PUB && (other > my_val || (other == my_val && o < mine)));
-                    if (o == 0 && c < FPB_PUB)
-                        order[par][__builtin_popcountll((above >> (c * CANDS)) & ((1ull << CANDS) - 1ull))] = mine;
-                }
-                lds_barrier();
-                // Then wavefront k looks at the point of place k: it may follow when its minimum is above everything
-                // unpublished, strictly above the next one's (equal minima are left to the exact resolution below)
-                // and a real minimum (>= 0), and when none of the points before it changes it (lane i: point i).
-                if (wave < FPB_T)
-                {
-                    const int at = order[par][wave], next = order[par][wave + 1], before = order[par][lane < wave ? lane : 0];
-                    const int val = cand_val[par][at], val_next = cand_val[par][next];
-                    const float4 rec = cand_rec[par][at], earlier = cand_rec[par][before];
-                    const int kept = wave_max_i32(lane < WAVES ? hidden[par][lane] : INT_MIN);
-                    const bool spoiled = lane < wave && ordered_bits(tpk_dist2(rec.x, rec.y, rec.z, earlier.x, earlier.y, earlier.z)) < val;
-                    // (after place 0 above 0: the samples before it drop to 0, and equal minima go by tie keys)
-                    const bool may = __ballot(spoiled) == 0ull && val > kept && val > val_next && val >= (wave == 0 ? 0 : 1);
-                    if (lane == 0)
-                    {
-                        taken[par][wave] = rec;
-                        follows[par][wave] = may ? 1 : 0;
-                        if (wave == 0)
-                            largest[par] = val;
-                    }
-                }
-                lds_barrier();
-                const int accept = min(static_cast<int>(__builtin_ctzll(~__ballot(lane < FPB_T && follows[par][lane < FPB_T ? lane : 0] != 0))), npoint - j);
-                if (accept > 0)
-                {
-                    if (wave == 0 && lane < accept) // (the others are on their way already)
-                        out[j + lane] = static_cast<int>(sort_keys[__float_as_int(taken[par][lane].w)] & 0x3FFFu);
-                    ns = accept;
-                    from = par;
-                    j += accept;
-                    // (no minimum exceeds the round's largest; the new samples still hold theirs until their own updates)
-                    bound = __builtin_amdgcn_readfirstlane(largest[par]);
-                    penalty = accept > 1 ? 1 : penalty;
-                    continue;
-                }
-                pause = penalty;
-                penalty = min(2 * penalty, 32);
-            }
-            else
-                --pause;
+    };
+    if (worker >= 0)
+        update(0, 1, ordered_bits(__builtin_inff()));
 
-            // Equal minima at the top, or nothing eligible: one sample by the reference's tie key over all points
-            // that hold the maximum (the key comes from the original index kept in the sort keys).
-            if (tid == 0)
-                words[which ^ 1] = RoundWords{INT_MIN, 0, 0xFFFFFFFFu, 0}; // (for the next time)
-            const int row_best = row_all_max_i32(b1);
-            if (row_head)
-                lds_atomic_max_i32(&words[which].max_val, row_best);
-            lds_barrier();
-            const int gv = __builtin_amdgcn_readfirstlane(words[which].max_val);
-            if (gv < 0)
+    int most_left = 0;       // no running minimum exceeds this
+    float gap = 0.1f;        // the pool takes what lies within this share below it
+    int pause = 1, penalty = 1; // rounds to take one by one; the first finds the largest minimum
+    int which = 0, attempt = 0, round = 0;
+    int j = 1;
+    while (j < npoint)
+    {
+        // 1. the pool: all points whose minimum lies above `floor_bits`, at most 64
+        int count = 0, floor_bits = 0;
+        bool pooled = false;
+        const bool paused = pause > 0 || one_by_one;
+        if (paused)
+            --pause;
+        else
+            for (int tries = 0; tries < POOL_TRIES && !pooled; ++tries)
             {
-                // No eligible point in the whole cloud: the reference's reduction yields index 0.
-                if (tid == 0)
+                floor_bits = ordered_bits(fmaxf(__int_as_float(most_left) * (1.0f - gap), 0.f));
+                if (floor_bits >= most_left)
+                    break; // nothing above zero, or more equal minima than a pool holds
+                const int slot = attempt % 3;
+                if (worker >= 0)
                 {
-                    taken[par][0] = make_float4(p0x, p0y, p0z, 0.f);
-                    out[j] = 0;
+                    unsigned long long above[PPT];
+                    int own = 0;
+#pragma unroll
+                    for (int i = 0; i < PPT; ++i)
+                    {
+                        above[i] = __ballot(t[i] > floor_bits);
+                        own += __builtin_popcountll(above[i]);
+                    }
+                    if (own > 0) // (uniform over the wavefront)
+                    {
+                        int at = 0;
+                        if (lane == 0)
+                            at = atomicAdd(&pool_count[slot], own);
+                        at = __builtin_amdgcn_readfirstlane(at);
+                        if (at + own <= POOL_CAPACITY)
+                        {
+#pragma unroll
+                            for (int i = 0; i < PPT; ++i)
+                                if (above[i] != 0)
+                                {
+                                    if (t[i] > floor_bits)
+                                    {
+                                        const int to = at + static_cast<int>(tpk_prefix_count(above[i]));
+                                        pool[to] = make_float4(x[i], y[i], z[i], __int_as_float(sorted_position<WORKERS, GS>(i / GS, worker, i % GS, lane)));
+                                        pool_min[to] = t[i];
+                                    }
+                                    at += __builtin_popcountll(above[i]);
+                                }
+                        }
+                    }
                 }
+                lds_barrier();
+                count = __builtin_amdgcn_readfirstlane(pool_count[slot]);
+                if (tid == 0)
+                    pool_count[(attempt + 2) % 3] = 0; // (the one before: everybody has read it)
+                ++attempt;
+                pooled = count > 0 && count <= POOL_CAPACITY;
+                if (count == 0 && floor_bits == 0)
+                    break; // nothing above zero
+                const float wanted = count == 0 ? 2.0f : static_cast<float>(POOL_TARGET) / static_cast<float>(count);
+                gap *= pooled ? fminf(fmaxf(wanted, 0.5f), 2.0f) : fmaxf(wanted, 0.02f);
+            }
+        if (pooled)
+        {
+            const int par = round & 1;
+            int taken_now = 0; // (none: more than 64 hold the largest minimum)
+            ++round;
+            if (wave == 0)
+            {
+                // 2a. the samples, one after the other (what a step costs is its instructions, a chain of dependent
+                // ones; the others' work goes into its gaps).  A point taken falls to zero, so a step takes a new one.
+                __builtin_amdgcn_s_setprio(3);
+                int at = lane < count ? lane : 0, left = lane < count ? pool_min[lane] : INT_MIN;
+                int number = -1; // this lane's point was the number-th to be taken
+                if (count > TPK_WAVE)
+                {
+                    // a floor that leaves at most 64, and not many fewer if that can be had: between the pool's own (more)
+                    // and its largest minimum (none), first where they would lie if they were evenly spread
+                    const int second = lane + TPK_WAVE < count ? pool_min[lane + TPK_WAVE] : INT_MIN;
+                    int high = wave_max_to_scalar(max(left, second)), low = floor_bits;
+                    unsigned long long first_ones = 0ull, second_ones = 0ull;
+                    int share = (TPK_WAVE - 4) * 256 / count;
+                    for (int tries = 0; tries < 6; ++tries)
+                    {
+                        const int middle = high - static_cast<int>(static_cast<long long>(high - low) * share / 256);
+                        const unsigned long long f = __ballot(left > middle), g = __ballot(second > middle);
+                        const int have = __builtin_popcountll(f) + __builtin_popcountll(g);
+                        if (have > TPK_WAVE)
+                            low = middle;
+                        else
+                        {
+                            high = middle;
+                            first_ones = f;
+                            second_ones = g;
+                            if (have >= TPK_WAVE - 12)
+                                break;
+                        }
+                        share = 128;
+                    }
+                    floor_bits = high;
+                    count = __builtin_popcountll(first_ones) + __builtin_popcountll(second_ones); // 0: too many are equal
+                    if (left > floor_bits && count > 0)
+                        pool_best[tpk_prefix_count(first_ones)] = lane;
+                    if (second > floor_bits && count > 0)
+                        pool_best[__builtin_popcountll(first_ones) + tpk_prefix_count(second_ones)] = lane + TPK_WAVE;
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    at = lane < count ? pool_best[lane] : 0;
+                    left = lane < count ? pool_min[at] : INT_MIN;
+                }
+                const float4 rec = pool[at];
+                int most = wave_max_to_scalar(left), now = 0;
+                const int top = most;
+                if (lane == 0)
+                    published[par ^ 1] = int4{0, 0, 0, 0}; // (the round before: everybody has left it)
+                auto publish = [&](int from, int flags) __attribute__((always_inline)) {
+                    if (number >= from)
+                        taken[number] = rec;
+                    // (a wavefront's LDS accesses are executed in order: nothing to wait for)
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    if (lane == 0)
+                        published[par] = int4{now | flags, top, floor_bits, (now | flags) ^ top ^ floor_bits};
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                };
+                while (true)
+                {
+                    const int from = now;
+#pragma unroll
+                    for (int u = 0; u < POOL_BATCH; ++u)
+                        if (__builtin_expect(most > floor_bits, 1))
+                        {
+                            unsigned long long holders = __ballot(left == most);
+                            if (__builtin_expect(__builtin_popcountll(holders) != 1, 0))
+                            {
+                                const unsigned key = left == most ? tie_key(original_index(__float_as_int(rec.w)), log2_bs, ref_groups) : 0xFFFFFFFFu;
+                                holders = __ballot(key == wave_min_u32(key));
+                            }
+                            const int l = __builtin_ctzll(holders);
+                            const float d = tpk_dist2(rec.x, rec.y, rec.z, tpk_read_lane(rec.x, l), tpk_read_lane(rec.y, l), tpk_read_lane(rec.z, l));
+                            number = lane == l ? now : number;
+                            left = min(left, ordered_bits(d));
+                            ++now;
+                            most = wave_max_to_scalar(left);
+                        }
+                    if (most <= floor_bits)
+                    {
+                        publish(from, POOL_DONE);
+                        break;
+                    }
+                    publish(from, 0);
+                }
+                __builtin_amdgcn_s_setprio(0);
+                if (number >= 0 && j + number < npoint)
+                    out[j + number] = original_index(__float_as_int(rec.w));
+                taken_now = now;
             }
             else
             {
-                unsigned my_tk = 0xFFFFFFFFu;
-                int my_q = 0;
+                // 2b. meanwhile the updates of the samples published so far
+                const volatile int4* const word = &published[par];
+                int seen = 0;
+                while (true)
+                {
+                    const int state = __builtin_amdgcn_readfirstlane(word->x), top = __builtin_amdgcn_readfirstlane(word->y);
+                    const int floor_now = __builtin_amdgcn_readfirstlane(word->z);
+                    if ((state ^ top ^ floor_now) != __builtin_amdgcn_readfirstlane(word->w))
+                        continue; // (read while it was being written)
+                    floor_bits = floor_now;
+                    const int ready = state & (POOL_DONE - 1);
+                    if (seen < ready)
+                    {
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                        for (; seen < ready; seen = min(seen + POOL_BATCH, ready))
+                            update(seen, min(POOL_BATCH, ready - seen), top);
+                    }
+                    else if ((state & POOL_DONE) == 0)
+                        __builtin_amdgcn_s_sleep(1);
+                    if (state & POOL_DONE)
+                        break;
+                }
+                taken_now = seen;
+            }
+            if (taken_now > 0)
+            {
+                j += taken_now;
+                penalty = taken_now > 1 ? 1 : penalty;
+                most_left = floor_bits;
+                continue;
+            }
+        }
+        if (!paused)
+        {
+            pause = penalty;
+            penalty = min(2 * penalty, 32);
+            gap = 0.02f;
+        }
+
+        // More equal minima at the top than a pool holds, or nothing above zero: one sample by the reference's tie key
+        // over all points that hold the maximum (the key comes from the original index kept in the sort keys).
+        if (tid == 0)
+            words[which ^ 1] = RoundWords{INT_MIN, 0xFFFFFFFFu}; // (for the next time)
+        if (worker >= 0)
+        {
+            int best = t[0];
+#pragma unroll
+            for (int i = 1; i < PPT; ++i)
+                best = max(best, t[i]);
+            const int row_best = row_all_max_i32(best);
+            if ((lane & 15) == 0)
+                lds_atomic_max_i32(&words[which].max_val, row_best);
+        }
+        lds_barrier();
+        const int gv = __builtin_amdgcn_readfirstlane(words[which].max_val);
+        if (gv < 0)
+        {
+            // No eligible point in the whole cloud: the reference's reduction yields index 0.
+            if (tid == 0)
+            {
+                taken[0] = make_float4(p0x, p0y, p0z, 0.f);
+                out[j] = 0;
+            }
+        }
+        else
+        {
+            unsigned my_tk = 0xFFFFFFFFu;
+            int my_q = 0;
+            if (worker >= 0)
+            {
 #pragma unroll
                 for (int i = 0; i < PPT; ++i)
                 {
-                    const int q = sorted_position<WAVES, GS>(i / GS, wave, i % GS, lane);
+                    const int q = sorted_position<WORKERS, GS>(i / GS, worker, i % GS, lane);
                     if (t[i] == gv && q < n)
                     {
-                        const unsigned tk = tie_key(static_cast<int>(sort_keys[q] & 0x3FFFu), log2_bs, ref_groups);
+                        const unsigned tk = tie_key(original_index(q), log2_bs, ref_groups);
                         if (tk < my_tk)
                         {
                             my_tk = tk;
@@ -692,24 +594,24 @@ __global__ __launch_bounds__(THREADS) void fps_pruned_kernel(
                 }
                 if (my_tk != 0xFFFFFFFFu)
                     atomicMin(&words[which].min_tie, my_tk);
-                lds_barrier();
-                if (my_tk == words[which].min_tie) // tie keys are distinct: exactly one lane
-                {
-                    const int k = static_cast<int>(sort_keys[my_q] & 0x3FFFu);
-                    taken[par][0] = make_float4(xyz[k * 3 + 0], xyz[k * 3 + 1], xyz[k * 3 + 2], __int_as_float(my_q));
-                    out[j] = k;
-                }
             }
             lds_barrier();
-            which ^= 1;
-            ns = 1;
-            from = par;
-            j += 1;
-            bound = gv < 0 ? bound : gv;
+            if (worker >= 0 && my_tk == words[which].min_tie) // tie keys are distinct: exactly one lane
+            {
+                const int k = original_index(my_q);
+                taken[0] = make_float4(xyz[k * 3 + 0], xyz[k * 3 + 1], xyz[k * 3 + 2], __int_as_float(my_q));
+                out[j] = k;
+            }
         }
-        TPK_WORK_FLUSH
-        return;
+        lds_barrier();
+        which ^= 1;
+        j += 1;
+        most_left = max(gv, 0);
+        if (worker >= 0)
+            update(0, 1, gv < 0 ? ordered_bits(__builtin_inff()) : gv);
+        lds_barrier(); // (taken[] may be written again)
     }
+    TPK_WORK_FLUSH
 }
 
 constexpr int FPS_CELL_WINDOW = CURVE_MAX_POINTS;            // points ordered together
@@ -1158,26 +1060,18 @@ int reference_log2_block(int n)
     return l;
 }
 
-template <int PPT, int THREADS>
-void launch_resident(int b, int n, int npoint, int log2_bs, int groups, const float* xyz,
-                     int32_t* out, hipStream_t s)
+template <int PPT, int WAVES, int GS, bool ORDERED>
+int launch_pool(int b, int n, int npoint, int log2_bs, int groups, const float* xyz, int32_t* out, hipStream_t s)
 {
-    hipLaunchKernelGGL((fps_resident_kernel<PPT, THREADS>), dim3(b), dim3(THREADS), 0, s, n,
-                       npoint, log2_bs, groups, xyz, out);
-}
-
-
-template <int PPT, int THREADS, int GS>
-int launch_pruned(int b, int n, int npoint, int log2_bs, int groups, const float* xyz,
-                  int32_t* out, hipStream_t s)
-{
+    if (n > PPT * (WAVES - 1) * TPK_WAVE || n > FPS_REGISTER_POINTS)
+        return TPK_ERR_UNSUPPORTED;
     const int key_capacity = n > CURVE_BINS ? (n + 63) & ~63 : CURVE_BINS; // (the ordering borrows CURVE_BINS words)
-    const size_t lds = (static_cast<size_t>(key_capacity) + static_cast<size_t>(PPT) * THREADS + CURVE_BINS) * sizeof(unsigned);
-    auto kernel = fps_pruned_kernel<PPT, THREADS, GS>;
+    const size_t lds = ORDERED ? (2 * static_cast<size_t>(key_capacity) + CURVE_BINS) * sizeof(unsigned) : 0;
+    auto kernel = fps_pool_kernel<PPT, WAVES, GS, ORDERED>;
     const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(kernel), lds);
     if (allowed != TPK_OK)
         return allowed;
-    hipLaunchKernelGGL(kernel, dim3(b), dim3(THREADS), lds, s, n, npoint, log2_bs, groups, key_capacity,
+    hipLaunchKernelGGL(kernel, dim3(b), dim3(WAVES * TPK_WAVE), lds, s, n, npoint, log2_bs, groups, key_capacity,
                        xyz, out);
     return tpk_launch_status();
 }
@@ -1247,22 +1141,22 @@ extern "C" int tpk_fps_f32(int b, int n, int npoint, const float* xyz, void* wor
     const int log2_bs = reference_log2_block(n);
     const int groups = static_cast<int>(tpk_ceil_div(n, 1 << log2_bs));
 
-    // Tiny clouds: one point per lane, no sorting.  Up to 16384 points: registers of a workgroup of 512 or
-    // 1024 lanes, curve order and pruning (cells of 64, 128 or 256 points).  Shapes as measured: sixteen
-    // wavefronts with half as many points each shorten a round (fewer cells per wavefront to update, fewer
-    // groups for the winner to search) except between 4097 and 8192 points.
-    if (n <= 512)
-        launch_resident<1, FPS_THREADS>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 512 * 2)
-        return launch_pruned<2, 512, 1>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 512 * 4)
-        return launch_pruned<2, 1024, 2>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 512 * 8)
-        return launch_pruned<4, 1024, 4>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 512 * 16)
-        return launch_pruned<16, 512, 4>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    // Up to 16384 points: registers of the workers of a workgroup, with one wavefront more that samples.  Sixteen
+    // wavefronts throughout (eight with twice the points each: 4 - 20 us more), cells of 64 to 192 points.  Measured with a
+    // quarter of the points sampled (16 clouds; the version before): 400 points 45 us (68), 1024 82 (114), 2048 134 (204),
+    // 4096 234 (359), 8192 430 (768), 16384 843 (1293).
+    if (n <= 15 * 64)
+        return launch_pool<1, 16, 1, false>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 2 * 15 * 64)
+        return launch_pool<2, 16, 2, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 4 * 15 * 64)
+        return launch_pool<4, 16, 2, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 6 * 15 * 64)
+        return launch_pool<6, 16, 3, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 12 * 15 * 64)
+        return launch_pool<12, 16, 3, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
     else if (n <= FPS_REGISTER_POINTS)
-        return launch_pruned<16, 1024, 4>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+        return launch_pool<18, 16, 3, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
     else if (n <= FPS_CELL_POINTS && workspace && workspace_bytes >= cell_layout(b, n).total)
     {
         // Cells of 64 points in memory, their summaries in LDS.
