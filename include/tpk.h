@@ -151,6 +151,8 @@ int tpk_ball_query_sorted_partial_f32(int64_t size_x, int64_t size_y, float radi
  * that grid, are ordered along a space filling curve and only nearby cells are searched; with
  * workspace == NULL the grid answers uneven clouds as well (slower there), and for other shapes
  * all pairs are tested.  Same results every way.
+ * tpk_three_nn_distance_f32: the same with the distances instead of their squares (the square root,
+ * correctly rounded, as the results are written).
  * tpk_three_nn_all_pairs_f32: the scan of all pairs itself, for any shape (what the reference
  * kernel does; here for measurements and as a check).
  * ------------------------------------------------------------------------------------- */
@@ -158,6 +160,9 @@ size_t tpk_three_nn_workspace_bytes(int b, int n, int m);
 int tpk_three_nn_f32(int b, int n, int m, const float* unknown, const float* known,
                      float* dist2, int32_t* idx, void* workspace, size_t workspace_bytes,
                      void* stream);
+int tpk_three_nn_distance_f32(int b, int n, int m, const float* unknown, const float* known,
+                              float* dist, int32_t* idx, void* workspace, size_t workspace_bytes,
+                              void* stream);
 int tpk_three_nn_all_pairs_f32(int b, int n, int m, const float* unknown, const float* known,
                                float* dist2, int32_t* idx, void* stream);
 
@@ -278,6 +283,10 @@ int tpk_group_grad_lists_f32(int b, int c, int n, int npoint, int nsample, const
  * arguments are kept for callers written against earlier versions and are ignored): the points
  * that chose a point as nearest neighbour are chained to it in LDS.  Clouds of more than about
  * 38000 points scatter with hardware float atomics instead.
+ * tpk_chamfer_loss_*: *loss = mean(dist1) + mean(dist2) of the whole batch, summed in float64 in a
+ * fixed order (`workspace`: tpk_chamfer_loss_workspace_bytes() bytes, 8-byte aligned; NaN where a
+ * mean is over nothing).  tpk_chamfer_loss_bwd_*: the backward pass for that loss: grad_loss is one
+ * number on the device, and every distance's gradient is grad_loss over the number of distances.
  * ------------------------------------------------------------------------------------- */
 size_t tpk_chamfer_fwd_workspace_bytes(int b, int n, int m);
 int tpk_chamfer_fwd_f32(int b, int n, int m, const float* xyz1, const float* xyz2, float* dist1,
@@ -295,6 +304,17 @@ int tpk_chamfer_bwd_f64(int b, int n, int m, const double* xyz1, const double* x
                         const int32_t* idx1, const int32_t* idx2, const double* grad_dist1,
                         const double* grad_dist2, double* grad_xyz1, double* grad_xyz2,
                         void* workspace, size_t workspace_bytes, void* stream);
+size_t tpk_chamfer_loss_workspace_bytes(int b, int n, int m);
+int tpk_chamfer_loss_f32(int b, int n, int m, const float* dist1, const float* dist2, float* loss,
+                         void* workspace, size_t workspace_bytes, void* stream);
+int tpk_chamfer_loss_f64(int b, int n, int m, const double* dist1, const double* dist2, double* loss,
+                         void* workspace, size_t workspace_bytes, void* stream);
+int tpk_chamfer_loss_bwd_f32(int b, int n, int m, const float* xyz1, const float* xyz2,
+                             const int32_t* idx1, const int32_t* idx2, const float* grad_loss,
+                             float* grad_xyz1, float* grad_xyz2, void* stream);
+int tpk_chamfer_loss_bwd_f64(int b, int n, int m, const double* xyz1, const double* xyz2,
+                             const int32_t* idx1, const int32_t* idx2, const double* grad_loss,
+                             double* grad_xyz1, double* grad_xyz2, void* stream);
 
 /* ---------------------------------------------------------------------------------------
  * Clusters grown over a neighbour matrix (PointGroup's region growing).

@@ -679,6 +679,19 @@ def test_three_nn_cell_search_parity(tpk, oracle, dev, B, n, m):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
+@pytest.mark.parametrize("B,n,m", [(2, 700, 600), (1, 900, 16384), (2, 600, 1024)])
+def test_three_nn_distances(tpk, dev, B, n, m):
+    # the square root taken as the results are written: by the cell search, and behind the grid in LDS for a cloud it
+    # hands over (clusters)
+    from torch_points_kernels._native import native
+    g = torch.Generator().manual_seed(m)
+    unknown, known = torch.rand(B, n, 3, generator=g).to(dev), _clustered(g, B, m).to(dev)
+    dist2, idx = native().three_nn(unknown, known)
+    dist, same = tpk.three_nn(unknown, known)
+    assert torch.equal(same, idx)
+    np.testing.assert_array_equal(_np(dist), np.sqrt(_np(dist2)))
+
+
 def test_three_nn_cell_search_ties(tpk, oracle, dev):
     # equal distances in every triple: tripled known points, lattices, a collapsed cloud
     native = __import__("torch_points_kernels._native", fromlist=["native"]).native()
@@ -1459,6 +1472,32 @@ def test_chamfer_backward_skewed_indices(tpk, dev, dtype):
     else:
         _assert_scatter_sum_close(_np(ga), wa.astype(np.float32), ma.astype(np.float32), "chamfer backward, skewed indices, xyz1")
         _assert_scatter_sum_close(_np(gb), wb.astype(np.float32), mb.astype(np.float32), "chamfer backward, skewed indices, xyz2")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,n,m", [(1, 1, 1), (2, 4096, 1), (1, 4096, 4096), (1, 4097, 4096), (3, 2731, 2000), (1, 40000, 700), (2, 0, 5)])
+def test_chamfer_loss_as_one_node(tpk, dev, dtype, B, n, m):
+    # means by one workgroup (up to 8192 distances) or shares of several, and the backward pass that is given one
+    # gradient for all distances (in LDS, or scattered for clouds beyond it), against the distances' own node and
+    # float64 means; a pair without points gives NaN and no gradient
+    g = torch.Generator().manual_seed(n + m)
+    a = torch.rand(B, n, 3, generator=g, dtype=dtype).to(dev).requires_grad_()
+    b = torch.rand(B, m, 3, generator=g, dtype=dtype).to(dev).requires_grad_()
+    loss = tpk.chamfer_dist.chamfer_dist(a, b)
+    assert loss.dtype == dtype and loss.shape == () and loss.requires_grad
+    ga, gb = torch.autograd.grad(loss * -3, (a, b))
+    d1, d2 = tpk.ChamferFunction.apply(a, b)
+    want = d1.double().mean() + d2.double().mean()
+    wa, wb = torch.autograd.grad(want * -3, (a, b))
+    tol = 1e-12 if dtype == torch.float64 else 1e-6
+    np.testing.assert_allclose(_np(loss), _np(want).astype(_np(loss).dtype), rtol=tol)
+    for got, exact in ((ga, wa), (gb, wb)):
+        assert got.shape == exact.shape
+        if n:
+            np.testing.assert_allclose(_np(got), _np(exact), rtol=10 * tol, atol=10 * tol * float(exact.abs().max()))
+    with torch.no_grad():
+        plain = tpk.chamfer_dist.chamfer_dist(a, b)
+    assert not plain.requires_grad and (torch.equal(plain, loss) or n == 0)
 
 
 def test_chamfer_ties_take_lowest_index(tpk, oracle, dev):

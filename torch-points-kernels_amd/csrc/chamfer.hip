@@ -201,8 +201,16 @@ __global__ __launch_bounds__(CH_THREADS) void chamfer_fwd_kernel(
     }
 }
 
+// The gradients of the distances a backward pass starts from: an array per direction, or (UNIFORM: the distances were
+// averaged) one number for all of them, divided by how many distances a direction has.
+template <typename T, bool UNIFORM>
+__device__ __forceinline__ T twice_gradient(const T* __restrict__ grad_dist, int64_t p, int64_t count)
+{
+    return (UNIFORM ? grad_dist[0] / static_cast<T>(count) : grad_dist[p]) * 2;
+}
+
 // Own term of every point: grad[j] = 2 * grad_dist[j] * (p[j] - other[idx[j]]), stored.
-template <typename T>
+template <typename T, bool UNIFORM>
 __global__ __launch_bounds__(256) void chamfer_bwd_own_kernel(
     int64_t total1, int64_t total2, int n, int m, const T* __restrict__ xyz1,
     const T* __restrict__ xyz2, const int32_t* __restrict__ idx1,
@@ -221,7 +229,7 @@ __global__ __launch_bounds__(256) void chamfer_bwd_own_kernel(
         const T* a = (second ? xyz2 : xyz1) + p * 3;
         const int j2 = (second ? idx2 : idx1)[p];
         const T* o = (second ? xyz1 : xyz2) + (cloud * nother + j2) * 3;
-        const T g = (second ? grad_dist2 : grad_dist1)[p] * 2;
+        const T g = twice_gradient<T, UNIFORM>(second ? grad_dist2 : grad_dist1, p, second ? total2 : total1);
         T* out = (second ? grad_xyz2 : grad_xyz1) + p * 3;
         out[0] = g * (a[0] - o[0]);
         out[1] = g * (a[1] - o[1]);
@@ -230,7 +238,7 @@ __global__ __launch_bounds__(256) void chamfer_bwd_own_kernel(
 }
 
 // Scattered term: grad_other[idx[j]] += -(2 * grad_dist[j] * (p[j] - other[idx[j]])).
-template <typename T>
+template <typename T, bool UNIFORM>
 __global__ __launch_bounds__(256) void chamfer_bwd_scatter_kernel(
     int64_t total1, int64_t total2, int n, int m, const T* __restrict__ xyz1,
     const T* __restrict__ xyz2, const int32_t* __restrict__ idx1,
@@ -250,7 +258,7 @@ __global__ __launch_bounds__(256) void chamfer_bwd_scatter_kernel(
         const int j2 = (second ? idx2 : idx1)[p];
         const int64_t op = cloud * nother + j2;
         const T* o = (second ? xyz1 : xyz2) + op * 3;
-        const T g = (second ? grad_dist2 : grad_dist1)[p] * 2;
+        const T g = twice_gradient<T, UNIFORM>(second ? grad_dist2 : grad_dist1, p, second ? total2 : total1);
         T* out = (second ? grad_xyz1 : grad_xyz2) + op * 3;
         unsafeAtomicAdd(out + 0, -(g * (a[0] - o[0])));
         unsafeAtomicAdd(out + 1, -(g * (a[1] - o[1])));
@@ -280,14 +288,16 @@ __global__ __launch_bounds__(256) void chamfer_bwd_scatter_kernel(
 constexpr int CHB_THREADS = 1024;
 constexpr int CHB_LDS_INTS = 38912; // 152 KiB
 
-// LDS words of one entry: four values and the link.
-template <typename T>
+// Values of an entry (x, y, z and, unless all are the same, 2 g), and LDS words of it: the values and the link.
+template <bool UNIFORM>
+constexpr int CHB_VALUES = UNIFORM ? 3 : 4;
+template <typename T, bool UNIFORM>
 constexpr int chb_entry_ints()
 {
-    return 4 * static_cast<int>(sizeof(T) / sizeof(int)) + 1;
+    return CHB_VALUES<UNIFORM> * static_cast<int>(sizeof(T) / sizeof(int)) + 1;
 }
 
-template <typename T>
+template <typename T, bool UNIFORM>
 __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
     int n, int m, int clouds, int splits, int range1, int range2, int lds_ints, const T* __restrict__ xyz1,
     const T* __restrict__ xyz2, const int32_t* __restrict__ idx1, const int32_t* __restrict__ idx2,
@@ -315,14 +325,17 @@ __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
     const T* __restrict__ other = (second ? xyz1 : xyz2) + static_cast<int64_t>(cloud) * nother * 3;
     const int32_t* __restrict__ own_idx = (second ? idx2 : idx1) + static_cast<int64_t>(cloud) * npts;
     const int32_t* __restrict__ other_idx = (second ? idx1 : idx2) + static_cast<int64_t>(cloud) * nother;
-    const T* __restrict__ own_g = (second ? grad_dist2 : grad_dist1) + static_cast<int64_t>(cloud) * npts;
-    const T* __restrict__ other_g = (second ? grad_dist1 : grad_dist2) + static_cast<int64_t>(cloud) * nother;
+    const T* __restrict__ own_g = (second ? grad_dist2 : grad_dist1) + (UNIFORM ? 0 : static_cast<int64_t>(cloud) * npts);
+    const T* __restrict__ other_g = (second ? grad_dist1 : grad_dist2) + (UNIFORM ? 0 : static_cast<int64_t>(cloud) * nother);
+    const T every_own = UNIFORM ? twice_gradient<T, true>(own_g, 0, static_cast<int64_t>(clouds) * npts) : T(0);
+    const T every_other = UNIFORM ? twice_gradient<T, true>(other_g, 0, static_cast<int64_t>(clouds) * nother) : T(0);
+    constexpr int V = CHB_VALUES<UNIFORM>;
     T* __restrict__ out = (second ? grad_xyz2 : grad_xyz1) + static_cast<int64_t>(cloud) * npts * 3;
 
-    // entries in LDS: values [capacity][4], links [capacity], heads [range]
-    const int capacity = min(nother, (lds_ints - range) / chb_entry_ints<T>());
+    // entries in LDS: values [capacity][V], links [capacity], heads [range]
+    const int capacity = min(nother, (lds_ints - range) / chb_entry_ints<T, UNIFORM>());
     T* const values = reinterpret_cast<T*>(chain_lds);
-    int* const links = chain_lds + capacity * (chb_entry_ints<T>() - 1);
+    int* const links = chain_lds + capacity * (chb_entry_ints<T, UNIFORM>() - 1);
     int* head = links + capacity;
     for (int t = tid; t < t1 - t0; t += CHB_THREADS)
         head[t] = -1;
@@ -349,7 +362,7 @@ __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
             ox[u] = other[j * 3 + 0];
             oy[u] = other[j * 3 + 1];
             oz[u] = other[j * 3 + 2];
-            og[u] = other_g[j] * 2;
+            og[u] = UNIFORM ? every_other : other_g[j] * 2;
         }
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
@@ -361,10 +374,11 @@ __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
                 if (e < capacity)
                 {
                     links[e] = atomicExch(&head[k[u] - t0], e);
-                    values[e * 4 + 0] = ox[u];
-                    values[e * 4 + 1] = oy[u];
-                    values[e * 4 + 2] = oz[u];
-                    values[e * 4 + 3] = og[u];
+                    values[e * V + 0] = ox[u];
+                    values[e * V + 1] = oy[u];
+                    values[e * V + 2] = oz[u];
+                    if (!UNIFORM)
+                        values[e * V + 3] = og[u];
                 }
             }
     }
@@ -413,7 +427,7 @@ __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
                 py[u] = own[k * 3 + 1];
                 pz[u] = own[k * 3 + 2];
                 j2[u] = own_idx[k];
-                g[u] = own_g[k] * 2;
+                g[u] = UNIFORM ? every_own : own_g[k] * 2;
                 j[u] = kb + u * CHB_THREADS < t1 ? head[k - t0] : -1;
             }
             T qx[TPT], qy[TPT], qz[TPT];
@@ -433,7 +447,8 @@ __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
                 int e = j[u];
                 while (e >= 0)
                 {
-                    const T vx = values[e * 4 + 0], vy = values[e * 4 + 1], vz = values[e * 4 + 2], vg = values[e * 4 + 3];
+                    const T vx = values[e * V + 0], vy = values[e * V + 1], vz = values[e * V + 2];
+                    const T vg = UNIFORM ? every_other : values[e * V + 3];
                     e = links[e];
                     ax = ax + -(vg * (vx - px[u]));
                     ay = ay + -(vg * (vy - py[u]));
@@ -454,7 +469,7 @@ __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
     {
         const T px = own[k * 3 + 0], py = own[k * 3 + 1], pz = own[k * 3 + 2];
         const int j2 = own_idx[k];
-        const T g = own_g[k] * 2;
+        const T g = UNIFORM ? every_own : own_g[k] * 2;
         int j = head[k - t0];
         T ax = g * (px - other[j2 * 3 + 0]);
         T ay = g * (py - other[j2 * 3 + 1]);
@@ -477,7 +492,7 @@ __global__ __launch_bounds__(CHB_THREADS) void chamfer_bwd_chains_kernel(
                 for (int l = 0; l < CHAIN; ++l)
                 {
                     const int jj = link[l] >= 0 ? link[l] : 0;
-                    gj[l] = other_g[jj] * 2;
+                    gj[l] = UNIFORM ? every_other : other_g[jj] * 2;
                     ox[l] = other[jj * 3 + 0];
                     oy[l] = other[jj * 3 + 1];
                     oz[l] = other[jj * 3 + 2];
@@ -545,10 +560,10 @@ int chamfer_fwd(int b, int n, int m, const T* xyz1, const T* xyz2, T* dist1, T* 
     return launch_fwd<T, 1>(b, n, m, xyz1, xyz2, dist1, dist2, idx1, idx2, s);
 }
 
-template <typename T>
+template <typename T, bool UNIFORM>
 int chamfer_bwd(int b, int n, int m, const T* xyz1, const T* xyz2, const int32_t* idx1,
                 const int32_t* idx2, const T* grad_dist1, const T* grad_dist2, T* grad_xyz1,
-                T* grad_xyz2, void* workspace, size_t workspace_bytes, void* stream)
+                T* grad_xyz2, void* stream)
 {
     if (b < 0 || n < 0 || m < 0)
         return TPK_ERR_INVALID_ARG;
@@ -570,8 +585,6 @@ int chamfer_bwd(int b, int n, int m, const T* xyz1, const T* xyz2, const int32_t
         hipLaunchKernelGGL(fill_zero_kernel<T>, dim3(blocks), dim3(256), 0, s, p, count);
         return tpk_launch_status();
     }
-    (void)workspace;
-    (void)workspace_bytes;
     // Chains in LDS (no workspace): as many target ranges per cloud as give every compute unit one
     // workgroup and none a second (config 5: 256 workgroups 19.7 us, 320 or 1024: 24 us, 512: 20.4 us),
     // each of at least 1024 targets; clouds too large for LDS scatter with atomics.
@@ -586,7 +599,7 @@ int chamfer_bwd(int b, int n, int m, const T* xyz1, const T* xyz2, const int32_t
         // (room for the entries a range expects - its share of the other cloud - and a third more)
         auto with_entries = [&](int parts) {
             const int64_t range = tpk_ceil_div(larger, parts);
-            return range + chb_entry_ints<T>() * (range + range / 3 + 64);
+            return range + chb_entry_ints<T, UNIFORM>() * (range + range / 3 + 64);
         };
         while (with_entries(splits) > CHB_LDS_INTS && splits < most)
             ++splits;
@@ -596,13 +609,13 @@ int chamfer_bwd(int b, int n, int m, const T* xyz1, const T* xyz2, const int32_t
         if (larger + range <= CHB_LDS_INTS && groups <= 0x7fffffffLL && static_cast<int64_t>(larger) * 3 <= 0x7fffffffLL)
         {
             // every point of the other cloud as an entry where that fits; else all of the LDS
-            const int64_t all = range + static_cast<int64_t>(chb_entry_ints<T>()) * larger;
+            const int64_t all = range + static_cast<int64_t>(chb_entry_ints<T, UNIFORM>()) * larger;
             const int lds_ints = static_cast<int>(all <= CHB_LDS_INTS ? (all > larger + range ? all : larger + range) : CHB_LDS_INTS);
             const size_t lds = static_cast<size_t>(lds_ints) * sizeof(int);
-            const int allowed = allow_lds(chamfer_bwd_chains_kernel<T>, lds);
+            const int allowed = allow_lds(chamfer_bwd_chains_kernel<T, UNIFORM>, lds);
             if (allowed != TPK_OK)
                 return allowed;
-            hipLaunchKernelGGL(chamfer_bwd_chains_kernel<T>, dim3(static_cast<unsigned>(groups)), dim3(CHB_THREADS), lds, s,
+            hipLaunchKernelGGL((chamfer_bwd_chains_kernel<T, UNIFORM>), dim3(static_cast<unsigned>(groups)), dim3(CHB_THREADS), lds, s,
                                n, m, b, splits, range1, range2, lds_ints, xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2,
                                grad_xyz1, grad_xyz2);
             return tpk_launch_status();
@@ -610,15 +623,109 @@ int chamfer_bwd(int b, int n, int m, const T* xyz1, const T* xyz2, const int32_t
     }
     const unsigned blocks =
         static_cast<unsigned>(tpk_min64(tpk_ceil_div(total1 + total2, 256), 1 << 20));
-    hipLaunchKernelGGL(chamfer_bwd_own_kernel<T>, dim3(blocks), dim3(256), 0, s, total1, total2,
+    hipLaunchKernelGGL((chamfer_bwd_own_kernel<T, UNIFORM>), dim3(blocks), dim3(256), 0, s, total1, total2,
                        n, m, xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2, grad_xyz1,
                        grad_xyz2);
     int st = tpk_launch_status();
     if (st != TPK_OK)
         return st;
-    hipLaunchKernelGGL(chamfer_bwd_scatter_kernel<T>, dim3(blocks), dim3(256), 0, s, total1,
+    hipLaunchKernelGGL((chamfer_bwd_scatter_kernel<T, UNIFORM>), dim3(blocks), dim3(256), 0, s, total1,
                        total2, n, m, xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2, grad_xyz1,
                        grad_xyz2);
+    return tpk_launch_status();
+}
+
+// Mean of the distances of both directions, added.  One workgroup for up to CHM_PER_BLOCK distances; for more, one per
+// CHM_PER_BLOCK of them up to CHM_BLOCKS, each leaving its share, and a workgroup behind them that adds the shares: every
+// sum is formed in float64 and in an order that depends on the sizes only.  The distances come from the cache the search
+// left them in (4 MB for 32 pairs of 16384 points), so the two launches are latency: 7 us, where two means and an
+// addition by torch took 17.
+constexpr int CHM_THREADS = 1024;
+constexpr int CHM_PER_BLOCK = 8 * CHM_THREADS;
+constexpr int CHM_BLOCKS = 256;
+
+inline int mean_blocks(int64_t distances)
+{
+    return static_cast<int>(tpk_min64(tpk_ceil_div(distances > 0 ? distances : 1, CHM_PER_BLOCK), CHM_BLOCKS));
+}
+
+// Sum over the workgroup, in every lane of the first wavefront.
+__device__ __forceinline__ double mean_block_sum(double v)
+{
+    __shared__ double sums[CHM_THREADS / TPK_WAVE];
+    for (int step = TPK_WAVE / 2; step > 0; step >>= 1)
+        v += __shfl_xor(v, step);
+    if ((threadIdx.x & (TPK_WAVE - 1)) == 0)
+        sums[threadIdx.x / TPK_WAVE] = v;
+    __syncthreads();
+    double total = 0;
+    for (int w = 0; w < CHM_THREADS / TPK_WAVE; ++w)
+        total += sums[w];
+    return total;
+}
+
+template <typename T>
+__device__ __forceinline__ double mean_share(const T* __restrict__ dist, int64_t count)
+{
+    constexpr int BATCH = 8; // loads in flight per lane
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * CHM_THREADS;
+    double sum = 0;
+    for (int64_t first = static_cast<int64_t>(blockIdx.x) * CHM_THREADS + threadIdx.x; first < count; first += BATCH * stride)
+    {
+        T v[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+        {
+            const int64_t at = first + u * stride;
+            v[u] = at < count ? dist[at] : T(0);
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+            sum += v[u];
+    }
+    return sum / static_cast<double>(count); // (0 / 0, NaN, over nothing)
+}
+
+template <typename T>
+__global__ __launch_bounds__(CHM_THREADS) void chamfer_mean_kernel(int64_t total1, int64_t total2, const T* __restrict__ dist1,
+                                                                   const T* __restrict__ dist2, double* __restrict__ shares,
+                                                                   T* __restrict__ loss)
+{
+    const double sum = mean_block_sum(mean_share(dist1, total1) + mean_share(dist2, total2));
+    if (threadIdx.x == 0)
+    {
+        if (gridDim.x == 1)
+            loss[0] = static_cast<T>(sum);
+        else
+            shares[blockIdx.x] = sum;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(CHM_THREADS) void chamfer_mean_total_kernel(int blocks, const double* __restrict__ shares, T* __restrict__ loss)
+{
+    const int at = threadIdx.x;
+    const double sum = mean_block_sum(at < blocks ? shares[at] : 0.0);
+    if (at == 0)
+        loss[0] = static_cast<T>(sum);
+}
+
+template <typename T>
+int chamfer_loss(int b, int n, int m, const T* dist1, const T* dist2, T* loss, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (b < 0 || n < 0 || m < 0 || !loss)
+        return TPK_ERR_INVALID_ARG;
+    const int64_t total1 = static_cast<int64_t>(b) * n, total2 = static_cast<int64_t>(b) * m;
+    if ((total1 > 0 && !dist1) || (total2 > 0 && !dist2))
+        return TPK_ERR_INVALID_ARG;
+    const int blocks = mean_blocks(total1 + total2);
+    if (blocks > 1 && (!workspace || workspace_bytes < tpk_chamfer_loss_workspace_bytes(b, n, m) || (reinterpret_cast<uintptr_t>(workspace) & 7u)))
+        return TPK_ERR_WORKSPACE;
+    hipStream_t s = tpk_stream(stream);
+    double* const shares = static_cast<double*>(workspace);
+    hipLaunchKernelGGL(chamfer_mean_kernel<T>, dim3(blocks), dim3(CHM_THREADS), 0, s, total1, total2, dist1, dist2, shares, loss);
+    if (blocks > 1)
+        hipLaunchKernelGGL(chamfer_mean_total_kernel<T>, dim3(1), dim3(CHM_THREADS), 0, s, blocks, shares, loss);
     return tpk_launch_status();
 }
 
@@ -657,8 +764,10 @@ extern "C" int tpk_chamfer_bwd_f32(int b, int n, int m, const float* xyz1, const
                                    float* grad_xyz1, float* grad_xyz2, void* workspace,
                                    size_t workspace_bytes, void* stream)
 {
-    return chamfer_bwd<float>(b, n, m, xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2, grad_xyz1,
-                            grad_xyz2, workspace, workspace_bytes, stream);
+    (void)workspace;
+    (void)workspace_bytes;
+    return chamfer_bwd<float, false>(b, n, m, xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2, grad_xyz1,
+                                     grad_xyz2, stream);
 }
 
 extern "C" int tpk_chamfer_bwd_f64(int b, int n, int m, const double* xyz1, const double* xyz2,
@@ -667,8 +776,10 @@ extern "C" int tpk_chamfer_bwd_f64(int b, int n, int m, const double* xyz1, cons
                                    double* grad_xyz1, double* grad_xyz2, void* workspace,
                                    size_t workspace_bytes, void* stream)
 {
-    return chamfer_bwd<double>(b, n, m, xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2, grad_xyz1,
-                            grad_xyz2, workspace, workspace_bytes, stream);
+    (void)workspace;
+    (void)workspace_bytes;
+    return chamfer_bwd<double, false>(b, n, m, xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2, grad_xyz1,
+                                     grad_xyz2, stream);
 }
 
 extern "C" size_t tpk_chamfer_bwd_workspace_bytes(int b, int n, int m)
@@ -677,4 +788,38 @@ extern "C" size_t tpk_chamfer_bwd_workspace_bytes(int b, int n, int m)
     (void)n;
     (void)m;
     return 0; // the backward pass keeps its chains in LDS
+}
+
+extern "C" size_t tpk_chamfer_loss_workspace_bytes(int b, int n, int m)
+{
+    if (b <= 0 || n < 0 || m < 0)
+        return 0;
+    const int blocks = mean_blocks(static_cast<int64_t>(b) * n + static_cast<int64_t>(b) * m);
+    return blocks > 1 ? blocks * sizeof(double) : 0;
+}
+
+extern "C" int tpk_chamfer_loss_f32(int b, int n, int m, const float* dist1, const float* dist2, float* loss,
+                                    void* workspace, size_t workspace_bytes, void* stream)
+{
+    return chamfer_loss<float>(b, n, m, dist1, dist2, loss, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tpk_chamfer_loss_f64(int b, int n, int m, const double* dist1, const double* dist2, double* loss,
+                                    void* workspace, size_t workspace_bytes, void* stream)
+{
+    return chamfer_loss<double>(b, n, m, dist1, dist2, loss, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tpk_chamfer_loss_bwd_f32(int b, int n, int m, const float* xyz1, const float* xyz2,
+                                        const int32_t* idx1, const int32_t* idx2, const float* grad_loss,
+                                        float* grad_xyz1, float* grad_xyz2, void* stream)
+{
+    return chamfer_bwd<float, true>(b, n, m, xyz1, xyz2, idx1, idx2, grad_loss, grad_loss, grad_xyz1, grad_xyz2, stream);
+}
+
+extern "C" int tpk_chamfer_loss_bwd_f64(int b, int n, int m, const double* xyz1, const double* xyz2,
+                                        const int32_t* idx1, const int32_t* idx2, const double* grad_loss,
+                                        double* grad_xyz1, double* grad_xyz2, void* stream)
+{
+    return chamfer_bwd<double, true>(b, n, m, xyz1, xyz2, idx1, idx2, grad_loss, grad_loss, grad_xyz1, grad_xyz2, stream);
 }

@@ -454,7 +454,7 @@ __device__ __forceinline__ void scan_cell3_few(const float4* __restrict__ cand, 
 __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
     int n, int m, int qcells, int ccells, int clouds, const float4* __restrict__ sorted_unknown,
     const float4* __restrict__ sorted_known, const float4* __restrict__ boxes_known, float* __restrict__ dist2,
-    int32_t* __restrict__ idx, const int* __restrict__ only)
+    int32_t* __restrict__ idx, bool root, const int* __restrict__ only)
 {
     __shared__ float4 stages[NG_SCAN_THREADS / TPK_WAVE][NG_CELL];
     extern __shared__ float lows_all[]; // [wavefronts][candidate cells, in whole groups of 64]
@@ -545,9 +545,9 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
     TPK_WORK_FLUSH
     if (qindex != 0x7FFFFFFF)
     {
-        dist2[qindex * 3 + 0] = s.b1;
-        dist2[qindex * 3 + 1] = s.b2;
-        dist2[qindex * 3 + 2] = s.b3;
+        dist2[qindex * 3 + 0] = root ? sqrtf(s.b1) : s.b1;
+        dist2[qindex * 3 + 1] = root ? sqrtf(s.b2) : s.b2;
+        dist2[qindex * 3 + 2] = root ? sqrtf(s.b3) : s.b3;
         idx[qindex * 3 + 0] = s.i1;
         idx[qindex * 3 + 1] = s.i2;
         idx[qindex * 3 + 2] = s.i3;
@@ -1141,7 +1141,7 @@ int* tpk_grid_three_nn_flags(int b, int n, int m, void* workspace, size_t worksp
 }
 
 int tpk_grid_three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2,
-                      int32_t* idx, void* workspace, size_t workspace_bytes, bool flagged, hipStream_t s)
+                      int32_t* idx, bool root, void* workspace, size_t workspace_bytes, bool flagged, hipStream_t s)
 {
     if (!grid_supported(b, n, m) || static_cast<int64_t>(b) * 2 > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
@@ -1166,7 +1166,7 @@ int tpk_grid_three_nn(int b, int n, int m, const float* unknown, const float* kn
     const size_t lds = static_cast<size_t>(NG_SCAN_THREADS / TPK_WAVE) * ((ccells + NG_CELL - 1) / NG_CELL * NG_CELL) *
                        sizeof(float);
     hipLaunchKernelGGL(three_nn_grid_kernel, dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), lds, s, n,
-                       m, qcells, ccells, b, a.sorted, c.sorted, c.boxes, dist2, idx, only);
+                       m, qcells, ccells, b, a.sorted, c.sorted, c.boxes, dist2, idx, root, only);
     return tpk_launch_status();
 }
 

@@ -91,8 +91,7 @@ at::Tensor furthest_point_sampling(at::Tensor points, const int nsamples)
     return output;
 }
 
-// cuda/src/interpolate.cpp:12-32
-std::vector<at::Tensor> three_nn(at::Tensor unknowns, at::Tensor knows)
+std::vector<at::Tensor> three_nearest(const at::Tensor& unknowns, const at::Tensor& knows, bool root)
 {
     check_contiguous(unknowns, "unknowns");
     check_contiguous(knows, "knows");
@@ -117,12 +116,23 @@ std::vector<at::Tensor> three_nn(at::Tensor unknowns, at::Tensor knows)
     at::Tensor ws;
     if (ws_bytes)
         ws = torch::empty({static_cast<int64_t>(ws_bytes)}, unknowns.options().dtype(torch::kUInt8));
-    check_status(tpk_three_nn_f32(b, n, m, unknowns.data_ptr<float>(), knows.data_ptr<float>(),
-                                  dist2.data_ptr<float>(), idx.data_ptr<int32_t>(),
-                                  ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
-                                  current_stream(unknowns)),
+    check_status((root ? tpk_three_nn_distance_f32 : tpk_three_nn_f32)(
+                     b, n, m, unknowns.data_ptr<float>(), knows.data_ptr<float>(), dist2.data_ptr<float>(), idx.data_ptr<int32_t>(),
+                     ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, current_stream(unknowns)),
                  "three_nn");
     return {dist2, idx};
+}
+
+// cuda/src/interpolate.cpp:12-32
+std::vector<at::Tensor> three_nn(at::Tensor unknowns, at::Tensor knows)
+{
+    return three_nearest(unknowns, knows, false);
+}
+
+// What the reference's torchpoints.py:64 makes of it: the distances, their square root taken as they are written.
+std::vector<at::Tensor> three_nn_distance(at::Tensor unknowns, at::Tensor knows)
+{
+    return three_nearest(unknowns, knows, true);
 }
 
 // cpu/src/knn.cpp:43-62 (dense_knn; the reference has it for CPU tensors only)
@@ -1132,6 +1142,73 @@ std::vector<torch::Tensor> chamfer_dist_grad(torch::Tensor xyz1, torch::Tensor x
     return {grad_xyz1, grad_xyz2};
 }
 
+// mean(dist1) + mean(dist2) over the whole batch, what the reference's chamfer_dist.py:25-54 makes of the distances, and
+// the nearest neighbours its gradient needs: {loss, idx1 (b, n) then idx2 (b, m) in one array}.
+std::vector<at::Tensor> chamfer_loss_forward(const at::Tensor& xyz1, const at::Tensor& xyz2)
+{
+    check_gpu(xyz1, "xyz1");
+    check_gpu(xyz2, "xyz2");
+    check_same_device(xyz1, xyz2, "xyz1 and xyz2");
+    check_points(xyz1, 3, "xyz1");
+    check_points(xyz2, 3, "xyz2");
+    TORCH_CHECK(xyz1.size(0) == xyz2.size(0), "xyz1 and xyz2 differ in batch size");
+    TORCH_CHECK(xyz1.scalar_type() == xyz2.scalar_type(), "xyz1 and xyz2 differ in dtype");
+    TORCH_CHECK(xyz1.scalar_type() == at::kFloat || xyz1.scalar_type() == at::kDouble, "chamfer_dist supports float32 and float64");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(xyz1.device());
+    const int b = as_int(xyz1.size(0), "batch size"), n = as_int(xyz1.size(1), "points of xyz1"), m = as_int(xyz2.size(1), "points of xyz2");
+    const bool narrow = xyz1.scalar_type() == at::kFloat;
+    const size_t total1 = static_cast<size_t>(b) * n, total2 = static_cast<size_t>(b) * m;
+    // one scratch: the search's workspace, the sums' workspace, the distances
+    const size_t ws_bytes = narrow ? tpk_chamfer_fwd_workspace_bytes(b, n, m) : 0, sum_bytes = tpk_chamfer_loss_workspace_bytes(b, n, m);
+    const size_t sums_at = (ws_bytes + 255) & ~static_cast<size_t>(255), dist_at = (sums_at + sum_bytes + 255) & ~static_cast<size_t>(255);
+    at::Tensor scratch = torch::empty({static_cast<int64_t>(dist_at + (total1 + total2) * xyz1.element_size())}, xyz1.options().dtype(at::kByte));
+    at::Tensor idx = torch::empty({static_cast<int64_t>(total1 + total2)}, xyz1.options().dtype(at::kInt));
+    at::Tensor loss = torch::empty({}, xyz1.options());
+    char* const bytes = static_cast<char*>(scratch.data_ptr());
+    int32_t* const idx1 = idx.data_ptr<int32_t>();
+    void* const ws = ws_bytes ? bytes : nullptr;
+    void* const sums = sum_bytes ? bytes + sums_at : nullptr;
+    void* const s = current_stream(xyz1);
+    if (narrow)
+    {
+        float* const dist1 = reinterpret_cast<float*>(bytes + dist_at);
+        check_status(tpk_chamfer_fwd_f32(b, n, m, xyz1.data_ptr<float>(), xyz2.data_ptr<float>(), dist1, dist1 + total1, idx1, idx1 + total1,
+                                         ws, ws_bytes, s),
+                     "chamfer_dist");
+        check_status(tpk_chamfer_loss_f32(b, n, m, dist1, dist1 + total1, loss.data_ptr<float>(), sums, sum_bytes, s), "chamfer_dist");
+    }
+    else
+    {
+        double* const dist1 = reinterpret_cast<double*>(bytes + dist_at);
+        check_status(tpk_chamfer_fwd_f64(b, n, m, xyz1.data_ptr<double>(), xyz2.data_ptr<double>(), dist1, dist1 + total1, idx1,
+                                         idx1 + total1, s),
+                     "chamfer_dist");
+        check_status(tpk_chamfer_loss_f64(b, n, m, dist1, dist1 + total1, loss.data_ptr<double>(), sums, sum_bytes, s), "chamfer_dist");
+    }
+    return {loss, idx};
+}
+
+std::vector<at::Tensor> chamfer_loss_backward(const at::Tensor& xyz1, const at::Tensor& xyz2, const at::Tensor& idx, const at::Tensor& grad_loss)
+{
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(xyz1.device());
+    check_gpu(grad_loss, "the gradient of the loss");
+    TORCH_CHECK(grad_loss.scalar_type() == xyz1.scalar_type() && grad_loss.numel() == 1, "the gradient of the loss is one number of its type");
+    const int b = as_int(xyz1.size(0), "batch size"), n = as_int(xyz1.size(1), "points of xyz1"), m = as_int(xyz2.size(1), "points of xyz2");
+    at::Tensor grad_xyz1 = torch::empty_like(xyz1), grad_xyz2 = torch::empty_like(xyz2);
+    const int32_t* const idx1 = idx.data_ptr<int32_t>();
+    const int32_t* const idx2 = idx1 + static_cast<int64_t>(b) * n;
+    void* const s = current_stream(xyz1);
+    if (xyz1.scalar_type() == at::kFloat)
+        check_status(tpk_chamfer_loss_bwd_f32(b, n, m, xyz1.data_ptr<float>(), xyz2.data_ptr<float>(), idx1, idx2, grad_loss.data_ptr<float>(),
+                                              grad_xyz1.data_ptr<float>(), grad_xyz2.data_ptr<float>(), s),
+                     "chamfer_dist_grad");
+    else
+        check_status(tpk_chamfer_loss_bwd_f64(b, n, m, xyz1.data_ptr<double>(), xyz2.data_ptr<double>(), idx1, idx2,
+                                              grad_loss.data_ptr<double>(), grad_xyz1.data_ptr<double>(), grad_xyz2.data_ptr<double>(), s),
+                     "chamfer_dist_grad");
+    return {grad_xyz1, grad_xyz2};
+}
+
 #include "differentiable.h"
 
 } // namespace
@@ -1140,6 +1217,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.def("furthest_point_sampling", &furthest_point_sampling);
     m.def("three_nn", &three_nn);
+    m.def("three_nn_distance", &three_nn_distance);
     m.def("dense_knn", &dense_knn);
     m.def("grow_proximity", &grow_proximity, pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("region_grow", &region_grow, pybind11::call_guard<pybind11::gil_scoped_release>());
@@ -1166,5 +1244,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("grouping_operation_grad_lists", &grouping_operation_grad_lists);
     m.def("chamfer_dist", &chamfer_dist);
     m.def("chamfer_dist_grad", &chamfer_dist_grad);
+    m.def("interpolate_features", &interpolate_features);
+    m.def("group_features", &group_features);
+    m.def("chamfer_loss", &chamfer_loss);
     m.def("tpk_version", &tpk_version);
 }

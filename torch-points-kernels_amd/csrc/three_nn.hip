@@ -26,7 +26,7 @@ constexpr int NN_TILE = 1024; // known points per LDS tile (16 KiB)
 template <int Q>
 __global__ __launch_bounds__(NN_THREADS) void three_nn_kernel(
     int n, int m, int blocks_per_cloud, const float* __restrict__ unknown,
-    const float* __restrict__ known, float* __restrict__ dist2, int32_t* __restrict__ idx)
+    const float* __restrict__ known, float* __restrict__ dist2, int32_t* __restrict__ idx, bool root)
 {
     __shared__ float4 tile[NN_TILE];
 
@@ -111,9 +111,9 @@ __global__ __launch_bounds__(NN_THREADS) void three_nn_kernel(
         const int j = j0 + q * NN_THREADS;
         if (j < n)
         {
-            dist2[j * 3 + 0] = b1[q];
-            dist2[j * 3 + 1] = b2[q];
-            dist2[j * 3 + 2] = b3[q];
+            dist2[j * 3 + 0] = root ? sqrtf(b1[q]) : b1[q];
+            dist2[j * 3 + 1] = root ? sqrtf(b2[q]) : b2[q];
+            dist2[j * 3 + 2] = root ? sqrtf(b3[q]) : b3[q];
             idx[j * 3 + 0] = i1[q];
             idx[j * 3 + 1] = i2[q];
             idx[j * 3 + 2] = i3[q];
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(NN_THREADS) void three_nn_kernel(
 
 template <int Q>
 int launch_three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2,
-                    int32_t* idx, hipStream_t stream)
+                    int32_t* idx, bool root, hipStream_t stream)
 {
     const int64_t blocks_per_cloud = tpk_ceil_div(n, NN_THREADS * Q);
     const int64_t blocks = blocks_per_cloud * b;
@@ -131,7 +131,7 @@ int launch_three_nn(int b, int n, int m, const float* unknown, const float* know
         return TPK_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(three_nn_kernel<Q>, dim3(static_cast<unsigned>(blocks)), dim3(NN_THREADS),
                        0, stream, n, m, static_cast<int>(blocks_per_cloud), unknown, known, dist2,
-                       idx);
+                       idx, root);
     return tpk_launch_status();
 }
 
@@ -169,7 +169,7 @@ struct Best3
 
 __global__ __launch_bounds__(LG_THREADS) void three_nn_cells_kernel(
     int n, int m, int blocks_per_cloud, int queries_per_block, const float* __restrict__ unknown,
-    const float* __restrict__ known, float* __restrict__ dist2, int32_t* __restrict__ idx, int* __restrict__ general)
+    const float* __restrict__ known, float* __restrict__ dist2, int32_t* __restrict__ idx, bool root, int* __restrict__ general)
 {
     extern __shared__ __align__(16) unsigned char tnc_lds[];
     const int tid = threadIdx.x;
@@ -209,9 +209,10 @@ __global__ __launch_bounds__(LG_THREADS) void three_nn_cells_kernel(
             lds_grid_scan_all(grid, m, qx, qy, qz, best TPK_WORK_ARG);
         else
             lds_grid_search(grid, qx, qy, qz, best TPK_WORK_ARG);
-        dist2[j * 3 + 0] = __int_as_float(static_cast<int>(best.k1 >> 32));
-        dist2[j * 3 + 1] = __int_as_float(static_cast<int>(best.k2 >> 32));
-        dist2[j * 3 + 2] = best.bound();
+        const float d1 = __int_as_float(static_cast<int>(best.k1 >> 32)), d2 = __int_as_float(static_cast<int>(best.k2 >> 32));
+        dist2[j * 3 + 0] = root ? sqrtf(d1) : d1;
+        dist2[j * 3 + 1] = root ? sqrtf(d2) : d2;
+        dist2[j * 3 + 2] = root ? sqrtf(best.bound()) : best.bound();
         idx[j * 3 + 0] = static_cast<int>(best.k1 & 0xFFFFFFFFu);
         idx[j * 3 + 1] = static_cast<int>(best.k2 & 0xFFFFFFFFu);
         idx[j * 3 + 2] = static_cast<int>(best.k3 & 0xFFFFFFFFu);
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(LG_THREADS) void three_nn_cells_kernel(
 }
 
 int launch_three_nn_cells(int b, int n, int m, const float* unknown, const float* known, float* dist2, int32_t* idx,
-                          int* general, hipStream_t stream)
+                          bool root, int* general, hipStream_t stream)
 {
     // one workgroup per compute unit where the queries allow it (every workgroup sorts its cloud)
     const int64_t per_cloud = std::max<int64_t>(1, std::min<int64_t>(tpk_ceil_div(n, LG_THREADS), TPK_COMPUTE_UNITS / b));
@@ -233,20 +234,33 @@ int launch_three_nn_cells(int b, int n, int m, const float* unknown, const float
     if (st != TPK_OK)
         return st;
     hipLaunchKernelGGL(three_nn_cells_kernel, dim3(static_cast<unsigned>(bpc * b)), dim3(LG_THREADS), lds, stream, n, m,
-                       static_cast<int>(bpc), per_block, unknown, known, dist2, idx, general);
+                       static_cast<int>(bpc), per_block, unknown, known, dist2, idx, root, general);
     return tpk_launch_status();
 }
 
-} // namespace
-
-extern "C" size_t tpk_three_nn_workspace_bytes(int b, int n, int m)
+// (root: distances instead of their squares)
+int all_pairs(int b, int n, int m, const float* unknown, const float* known, float* dist2, int32_t* idx, bool root, void* stream)
 {
-    return tpk_grid_three_nn_workspace_bytes(b, n, m);
+    if (b < 0 || n < 0 || m < 0)
+        return TPK_ERR_INVALID_ARG;
+    if (b == 0 || n == 0)
+        return TPK_OK;
+    if (!unknown || !dist2 || !idx || (m > 0 && !known))
+        return TPK_ERR_INVALID_ARG;
+    if (static_cast<int64_t>(n) * 3 > 0x7fffffffLL || static_cast<int64_t>(m) * 3 > 0x7fffffffLL)
+        return TPK_ERR_UNSUPPORTED;
+    hipStream_t s = tpk_stream(stream);
+    // Queries per lane: as many as still leave a few workgroups per compute unit.
+    const int64_t queries = static_cast<int64_t>(b) * n;
+    if (queries >= 4LL * NN_THREADS * 2048)
+        return launch_three_nn<4>(b, n, m, unknown, known, dist2, idx, root, s);
+    if (queries >= 2LL * NN_THREADS * 2048)
+        return launch_three_nn<2>(b, n, m, unknown, known, dist2, idx, root, s);
+    return launch_three_nn<1>(b, n, m, unknown, known, dist2, idx, root, s);
 }
 
-extern "C" int tpk_three_nn_f32(int b, int n, int m, const float* unknown, const float* known,
-                                float* dist2, int32_t* idx, void* workspace, size_t workspace_bytes,
-                                void* stream)
+int three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2, int32_t* idx, bool root, void* workspace,
+             size_t workspace_bytes, void* stream)
 {
     if (b < 0 || n < 0 || m < 0)
         return TPK_ERR_INVALID_ARG;
@@ -262,40 +276,46 @@ extern "C" int tpk_three_nn_f32(int b, int n, int m, const float* unknown, const
         // The known cloud fits in LDS: a grid there, one lane per query.  It notes the clouds it gives up (uneven
         // density) in the workspace, and the search over curve-ordered cells, enqueued behind it, answers those.
         int* const general = tpk_grid_three_nn_flags(b, n, m, workspace, workspace_bytes);
-        const int st = launch_three_nn_cells(b, n, m, unknown, known, dist2, idx, general, s);
+        const int st = launch_three_nn_cells(b, n, m, unknown, known, dist2, idx, root, general, s);
         if (st != TPK_OK || !general)
             return st;
-        return tpk_grid_three_nn(b, n, m, unknown, known, dist2, idx, workspace, workspace_bytes, true, s);
+        return tpk_grid_three_nn(b, n, m, unknown, known, dist2, idx, root, workspace, workspace_bytes, true, s);
     }
     if (workspace)
     {
         // Search over curve-ordered cells where it applies; otherwise all pairs.
-        const int st = tpk_grid_three_nn(b, n, m, unknown, known, dist2, idx, workspace, workspace_bytes, false, s);
+        const int st = tpk_grid_three_nn(b, n, m, unknown, known, dist2, idx, root, workspace, workspace_bytes, false, s);
         if (st != TPK_ERR_UNSUPPORTED)
             return st;
     }
-    return tpk_three_nn_all_pairs_f32(b, n, m, unknown, known, dist2, idx, stream);
+    return all_pairs(b, n, m, unknown, known, dist2, idx, root, stream);
+}
+
+} // namespace
+
+extern "C" size_t tpk_three_nn_workspace_bytes(int b, int n, int m)
+{
+    return tpk_grid_three_nn_workspace_bytes(b, n, m);
+}
+
+extern "C" int tpk_three_nn_f32(int b, int n, int m, const float* unknown, const float* known,
+                                float* dist2, int32_t* idx, void* workspace, size_t workspace_bytes,
+                                void* stream)
+{
+    return three_nn(b, n, m, unknown, known, dist2, idx, false, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tpk_three_nn_distance_f32(int b, int n, int m, const float* unknown, const float* known,
+                                         float* dist, int32_t* idx, void* workspace, size_t workspace_bytes,
+                                         void* stream)
+{
+    return three_nn(b, n, m, unknown, known, dist, idx, true, workspace, workspace_bytes, stream);
 }
 
 extern "C" int tpk_three_nn_all_pairs_f32(int b, int n, int m, const float* unknown, const float* known,
                                           float* dist2, int32_t* idx, void* stream)
 {
-    if (b < 0 || n < 0 || m < 0)
-        return TPK_ERR_INVALID_ARG;
-    if (b == 0 || n == 0)
-        return TPK_OK;
-    if (!unknown || !dist2 || !idx || (m > 0 && !known))
-        return TPK_ERR_INVALID_ARG;
-    if (static_cast<int64_t>(n) * 3 > 0x7fffffffLL || static_cast<int64_t>(m) * 3 > 0x7fffffffLL)
-        return TPK_ERR_UNSUPPORTED;
-    hipStream_t s = tpk_stream(stream);
-    // Queries per lane: as many as still leave a few workgroups per compute unit.
-    const int64_t queries = static_cast<int64_t>(b) * n;
-    if (queries >= 4LL * NN_THREADS * 2048)
-        return launch_three_nn<4>(b, n, m, unknown, known, dist2, idx, s);
-    if (queries >= 2LL * NN_THREADS * 2048)
-        return launch_three_nn<2>(b, n, m, unknown, known, dist2, idx, s);
-    return launch_three_nn<1>(b, n, m, unknown, known, dist2, idx, s);
+    return all_pairs(b, n, m, unknown, known, dist2, idx, false, stream);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -36,9 +36,9 @@ def three_nn(unknown, known):
     if unknown.shape[1] < 3:
         raise ValueError("Not enough points. unknown should ahve at least 3 points.")
     if unknown.is_cuda:
-        dist2, idx = native().three_nn(unknown, known)
-    else:
-        idx, dist2 = knn(known, unknown, 3)
+        dist, idx = native().three_nn_distance(unknown, known)
+        return dist, idx
+    idx, dist2 = knn(known, unknown, 3)
     return torch.sqrt(dist2), idx
 
 
@@ -75,6 +75,8 @@ class ThreeInterpolate(Function):
 def three_interpolate(features, idx, weight):
     r"""features (B, c, m), idx (B, n, 3) (int32 on the GPU, int64 on the CPU: what three_nn returns there),
     weight (B, n, 3) -> (B, c, n) (reference: torchpoints.py:109-126)."""
+    if features.is_cuda:
+        return native().interpolate_features(features, idx, weight)
     return ThreeInterpolate.apply(features, idx, weight)
 
 
@@ -107,7 +109,7 @@ def grouping_operation(features, idx):
     (reference: torchpoints.py:129-146).  float32 tensors on the GPU take the native kernels; every other
     device and dtype is served, as in the reference, by torch's own gather (and its autograd)."""
     if features.is_cuda and features.dtype == torch.float32 and idx.dtype == torch.int64:
-        return GroupingOperation.apply(features, idx)
+        return native().group_features(features, idx)
     b, c = features.shape[0], features.shape[1]
     columns = idx.reshape(b, 1, -1).expand(b, c, -1)
     return torch.gather(features, 2, columns).reshape(b, c, idx.shape[1], idx.shape[2])
