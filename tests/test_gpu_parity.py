@@ -1002,6 +1002,48 @@ def test_knn_parity(tpk, oracle, dev, B, n, m, k):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
+@pytest.mark.parametrize("kind", ["uniform", "clusters", "flat", "one_point", "lattice", "outlier", "queries_outside", "non_finite"])
+@pytest.mark.parametrize("B,n,m,k", [(2, 1, 3, 1), (2, 65, 40, 48), (1, 3000, 150, 49), (1, 8192, 200, 17), (2, 8193, 90, 48), (1, 40000, 60, 4)])
+def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
+    # up to 48 neighbours: a grid in LDS (up to 8192 points) or in memory, its block of cells grown until it holds k, the
+    # cells of the ball around it, and merging where many distances are equal or too few are finite; 49: lists
+    g = torch.Generator().manual_seed(n + k)
+    support, query = torch.rand(B, n, 3, generator=g), torch.rand(B, m, 3, generator=g)
+    if kind == "clusters":
+        support, query = _clustered(g, B, n), _clustered(g, B, m)
+    elif kind == "flat":
+        support[..., 1] = 0.25
+    elif kind == "one_point":
+        support[:] = 0.5
+    elif kind == "lattice":
+        support, query = (support * 12).round(), (query * 24).round() / 2
+    elif kind == "outlier":
+        support[:, n // 3] = torch.tensor([400.0, -300.0, 1e6])
+    elif kind == "queries_outside":
+        query[:, ::2] += 5.0
+        query[:, 1::2, 1] = -40.0
+    elif kind == "non_finite" and n > 64:
+        support[:, 5, 0] = float("nan")
+        support[:, 7, 1] = float("inf")
+        support[:, 9] = float("-inf")
+        query[:, 0, 2] = float("inf")
+    idx, dist2 = tpk.knn(support.to(dev), query.to(dev), k)
+    if kind == "non_finite" and n > 64:
+        # behind the finite distances come the infinite ones by index; a slot no candidate fills holds (inf, 2^31 - 1)
+        d = (query[:, :, None] - support[:, None]).pow(2).sum(3)
+        infinite = torch.isinf(d).sum(2)
+        finite = torch.isfinite(d).sum(2)
+        place = torch.arange(k)
+        assert torch.equal(torch.isfinite(dist2.cpu()), place < finite[..., None])
+        assert torch.equal(idx.cpu() == 2 ** 31 - 1, place >= (finite + infinite)[..., None])
+        query, idx, dist2 = query[:, 1:], idx[:, 1:, : min(k, n - 3)], dist2[:, 1:, : min(k, n - 3)]
+        support[:, [5, 7, 9]] = 1e18  # (the oracle's scan: far, and last)
+        k = min(k, n - 3)
+    wi, wd = oracle.knn(support.numpy(), query.contiguous().numpy(), k)
+    np.testing.assert_array_equal(_np(idx), wi)
+    np.testing.assert_array_equal(_np(dist2), wd)
+
+
 def test_knn_ties_and_errors(tpk, oracle, dev):
     # reference test/test_knn.py:14-23
     support = torch.tensor([[[0, 0, 0], [1, 0, 0], [2, 0, 0]]]).float().to(dev)

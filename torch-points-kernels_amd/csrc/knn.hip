@@ -8,18 +8,26 @@
 // exactly equal distances is unspecified.  k must not exceed the number of support points
 // (cpu/src/knn.cpp:12-14 raises).
 //
-// With a workspace, clouds of 512..163840 points are searched over curve-ordered cells
-// (nn_grid.hip).  Otherwise all pairs are tested: one lane owns one query and keeps its list in
-// registers (topk.h); the support points of the cloud stream through LDS in tiles of float4, read
-// by all lanes at the same address.  k above 32 is served in rounds of 32 entries.
+// Up to KNC_MAX_K neighbours are found by a wavefront per query (survivors.h): in clouds that fit into LDS over a grid there
+// (below), in larger ones, given a workspace, over such a grid in memory.  More neighbours, and large clouds without a
+// workspace: one lane owns one query and keeps its list in registers (topk.h), 32 entries a round - over
+// curve-ordered cells for clouds of 512..163840 points with a workspace, otherwise testing all pairs: the support points of
+// the cloud stream through LDS in tiles of float4, read by all lanes at the same address.
 #include "ball_cells.h"
+#include "lds_grid.h"
 #include "nn_grid.h"
+#include "survivors.h"
 #include "topk.h"
+
+#include <algorithm>
+#include <cmath>
 
 namespace {
 
 constexpr int KNN_THREADS = 256;
 constexpr int KNN_TILE = 1024; // support points per LDS tile (16 KiB)
+
+constexpr int KNG_AXIS = 128; // cells per axis of a grid in memory at most (LG_AXIS of one in LDS)
 
 constexpr int KNN_GROUP = 8;   // candidates whose distances are formed together
 
@@ -147,6 +155,403 @@ int launch_knn(int b, int n, int m, int k, float limit, const float* query, cons
     return TPK_OK;
 }
 
+// One query by one wavefront over a grid of cells: the 27 cells around it hold k points or the block grows; the k-th of
+// them bounds the ball the answer lies in, and the cells that ball touches outside the block are examined too (one query
+// in three).  The lanes find the candidates of the wavefront's rows of cells by a running maximum: each row's lane leaves
+// its number at its first candidate's place.  Returns the lane's key of the answer and its place there (>= k: none).
+// m: records in `points`, for the queries no distance separates.
+__device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4* points, const int* starts, int m, int k, int lane, float qx,
+                                               float qy, float qz, Survivors& s, u64& mine TPK_WORK_PARAM)
+{
+    const int cx = grid.cells[0], cy = grid.cells[1], cz = grid.cells[2];
+    const float q[3] = {qx, qy, qz};
+    s.clear();
+    bool separated = true; // every selection so far found its distance
+
+    // The candidates of up to 64 rows of cells, a row per lane (start, size), offered.
+    auto walk = [&](int start, int size, int before, int total, bool ball) __attribute__((always_inline)) {
+        const int origin = start - before; // candidate c of the walk lies at origin + c, for the c of this lane's row
+        for (int c0 = 0; c0 < total && separated; c0 += TPK_WAVE)
+        {
+            // the row of candidate c0, and every row that starts behind it in this step at its first candidate
+            const int first = __builtin_ctzll(__ballot(size > 0 && before <= c0 && before + size > c0));
+            const bool starts_here = size > 0 && before > c0 && before < c0 + TPK_WAVE;
+            const int mark = __builtin_amdgcn_ds_permute((starts_here ? before - c0 : 0) << 2, starts_here ? lane : 0);
+            const int row = max(wave_inclusive_max_i32(lane == 0 ? 0 : mark), first);
+            const int at = __shfl(origin, row) + c0 + lane;
+            const bool has = c0 + lane < total;
+            const float4 p = points[has ? at : 0];
+            TPK_WORK_ADD(1);
+            separated = s.offer(has, tpk_dist2(qx, qy, qz, p.x, p.y, p.z), __float_as_int(p.w), ball);
+        }
+    };
+
+    // ---- the block of cells around the query that holds k points ----
+    int c[3];
+    for (int a = 0; a < 3; ++a)
+        c[a] = __builtin_amdgcn_readfirstlane(lg_cell((q[a] - grid.lo[a]) * grid.inv[a], grid.cells[a]));
+    int xl, xh, yl, yh, zl, zh;
+    // (a crowded cell may do alone: its 26 neighbours would be as crowded)
+    const int own = c[0] + cx * (c[1] + cy * c[2]);
+    for (int ring = starts[own + 1] - starts[own] >= 2 * k ? 0 : 1;; ++ring)
+    {
+        const bool all = ring > 3; // (7 x 7 rows are the most a lane each can take)
+        xl = all ? 0 : max(c[0] - ring, 0), xh = all ? cx - 1 : min(c[0] + ring, cx - 1);
+        yl = all ? 0 : max(c[1] - ring, 0), yh = all ? cy - 1 : min(c[1] + ring, cy - 1);
+        zl = all ? 0 : max(c[2] - ring, 0), zh = all ? cz - 1 : min(c[2] + ring, cz - 1);
+        const int ny = yh - yl + 1, rows = ny * (zh - zl + 1);
+        if (all)
+        {
+            // a query with hardly any point near it: every row
+            for (int row0 = 0; row0 < rows && separated; row0 += TPK_WAVE)
+            {
+                const int c0 = min(row0 + lane, rows - 1) * cx;
+                const int start = starts[c0], size = row0 + lane < rows ? starts[c0 + cx] - start : 0;
+                const int before = wave_exclusive_sum(size);
+                walk(start, size, before, __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1), false);
+            }
+            break;
+        }
+        int start = 0, size = 0;
+        if (lane < rows)
+        {
+            const int iz = static_cast<int>((static_cast<float>(lane) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(ny)));
+            const int c0 = xl + cx * ((yl + lane - iz * ny) + cy * (zl + iz));
+            start = starts[c0];
+            size = starts[c0 + (xh - xl + 1)] - start;
+        }
+        const int before = wave_exclusive_sum(size);
+        const int total = __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1);
+        if (total < k)
+            continue;
+        walk(start, size, before, total, false);
+        break;
+    }
+
+    // ---- the k-th so far bounds the ball; the cells it touches outside the block ----
+    mine = ~0ull;
+    int place = KNC_MOST;
+    separated = separated && s.count >= k && (s.count <= KNC_MOST || s.select(__builtin_inff(), 0, false));
+    if (separated)
+    {
+        place = s.rank(mine);
+        const int kth = __builtin_ctzll(__ballot(place == k - 1));
+        const float bound = tpk_read_lane(__int_as_float(static_cast<int>(mine >> 32)), kth);
+        const float radius = sqrtf(bound) * 1.000001f;
+        int from[3], to[3];
+        for (int a = 0; a < 3; ++a)
+        {
+            // (the ends a few ulps out, so that no point the rounded distances accept is left out)
+            const float slack = (fabsf(q[a]) + radius) * 1e-6f + 1e-30f;
+            from[a] = __builtin_amdgcn_readfirstlane(lg_cell(((q[a] - radius) - slack - grid.lo[a]) * grid.inv[a], grid.cells[a]));
+            to[a] = __builtin_amdgcn_readfirstlane(lg_cell(((q[a] + radius) + slack - grid.lo[a]) * grid.inv[a], grid.cells[a]));
+        }
+        if (from[0] < xl || to[0] > xh || from[1] < yl || to[1] > yh || from[2] < zl || to[2] > zh)
+        {
+            // Distance along axis a from the query to a cell, a lower bound.
+            auto apart = [&](int a, int at) __attribute__((always_inline)) {
+                const float t = (q[a] - grid.lo[a]) * grid.inv[a];
+                const float gap = fmaxf(static_cast<float>(at) - t, t - static_cast<float>(at + 1));
+                return fmaxf(gap - 1e-5f * (fabsf(t) + static_cast<float>(KNG_AXIS)), 0.0f) * grid.width[a];
+            };
+            // the k kept in order, then the rest of the ball: two pieces for a row that crosses the block
+            if (place < k)
+                s.keys[place] = mine;
+            s.count = k;
+            s.reach = bound;
+            const int ny = to[1] - from[1] + 1, pieces = 2 * ny * (to[2] - from[2] + 1);
+            for (int piece0 = 0; piece0 < pieces && separated; piece0 += TPK_WAVE)
+            {
+                const int e = piece0 + lane;
+                int start = 0, size = 0;
+                if (e < pieces)
+                {
+                    const int row = e >> 1;
+                    const int iz = static_cast<int>((static_cast<float>(row) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(ny)));
+                    const int y = from[1] + row - iz * ny, z = from[2] + iz;
+                    const bool crosses = y >= yl && y <= yh && z >= zl && z <= zh;
+                    const int x0 = (e & 1) ? xh + 1 : from[0];
+                    const int x1 = (e & 1) ? (crosses ? to[0] : x0 - 1) : (crosses ? xl - 1 : to[0]);
+                    const float dy = apart(1, y), dz = apart(2, z);
+                    if (x1 >= x0 && dy * dy + dz * dz <= bound * 1.00001f)
+                    {
+                        const int c0 = cx * (y + cy * z);
+                        start = starts[c0 + x0];
+                        size = starts[c0 + x1 + 1] - start;
+                    }
+                }
+                const int before = wave_exclusive_sum(size);
+                walk(start, size, before, __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1), true);
+            }
+            separated = separated && (s.count <= KNC_MOST || s.select(__builtin_inff(), 0, true));
+            if (separated && (s.count > k || s.reach != bound)) // (else none came along, and the k lie in order)
+                place = s.rank(mine);
+            else if (separated)
+                place = lane < k ? lane : KNC_MOST, mine = s.keys[lane < k ? lane : 0];
+        }
+    }
+    if (!separated)
+    {
+        mine = nearest_by_merging(m, k, lane, qx, qy, qz, [&](int at) { return points[at]; } TPK_WORK_ARG);
+        place = lane;
+    }
+    return place;
+}
+
+// Points per cell: a fifth of k, so that the 27 cells around a query hold five times k and the ball inside them rather more
+// than k.  (0.15 and 0.32 of k: within 4 % on even clouds; on a sphere 0.32 is 8 to 12 % slower.)
+inline float knn_per_cell(int k)
+{
+    return fmaxf(1.0f, 0.2f * static_cast<float>(k));
+}
+
+// Clouds of up to LG_MAX_POINTS points: every workgroup builds the grid in LDS (lds_grid.h) and serves a stretch of queries.
+__global__ __launch_bounds__(LG_THREADS) void knn_cells_kernel(
+    int n, int m, int k, int blocks_per_cloud, int queries_per_block, float per_cell, const float* __restrict__ query,
+    const float* __restrict__ support, float* __restrict__ dist2, int64_t* __restrict__ idx)
+{
+    extern __shared__ __align__(16) unsigned char knc_lds[];
+    const int tid = threadIdx.x;
+    const int lane = tid & (TPK_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
+    const int cloud = blockIdx.x / blocks_per_cloud;
+    const int blk = blockIdx.x - cloud * blocks_per_cloud;
+    query += static_cast<int64_t>(cloud) * n * 3;
+    support += static_cast<int64_t>(cloud) * m * 3;
+    dist2 += static_cast<int64_t>(cloud) * n * k;
+    idx += static_cast<int64_t>(cloud) * n * k;
+    TPK_WORK_DECL
+
+    u64* const all_keys = reinterpret_cast<u64*>(knc_lds);
+    LdsGrid grid;
+    lds_grid_build(grid, knc_lds + LG_WAVES * KNC_ROOM * sizeof(u64), support, m, 0, per_cell);
+    Survivors s;
+    s.keys = all_keys + wave * KNC_ROOM;
+    s.lane = lane;
+    s.k = k;
+
+    const int q_end = min(n, (blk + 1) * queries_per_block);
+    for (int j = blk * queries_per_block + wave; j < q_end; j += LG_WAVES)
+    {
+        const float qx = to_vector_register(query[j * 3 + 0]), qy = to_vector_register(query[j * 3 + 1]), qz = to_vector_register(query[j * 3 + 2]);
+        u64 mine;
+        const int place = nearest_in_grid(grid, grid.points, grid.starts, m, k, lane, qx, qy, qz, s, mine TPK_WORK_ARG);
+        if (place < k)
+        {
+            dist2[static_cast<int64_t>(j) * k + place] = __int_as_float(static_cast<int>(mine >> 32));
+            idx[static_cast<int64_t>(j) * k + place] = static_cast<int64_t>(mine & 0xFFFFFFFFu);
+        }
+    }
+    TPK_WORK_FLUSH
+}
+
+int launch_knn_cells(int b, int n, int m, int k, const float* query, const float* support, float* dist2, int64_t* idx, hipStream_t stream)
+{
+    // one workgroup per compute unit where the queries allow it (every workgroup sorts its cloud), a query per wavefront
+    // at a time
+    const int64_t per_cloud = std::max<int64_t>(1, std::min<int64_t>(tpk_ceil_div(n, LG_WAVES), TPK_COMPUTE_UNITS / b));
+    const int per_block = static_cast<int>(tpk_ceil_div(n, per_cloud));
+    const int64_t bpc = tpk_ceil_div(n, per_block);
+    if (bpc * b > 0x7fffffffLL)
+        return TPK_ERR_UNSUPPORTED;
+    const size_t lds = lg_lds_bytes(m) + LG_WAVES * KNC_ROOM * sizeof(u64);
+    const int st = tpk_allow_lds(reinterpret_cast<const void*>(&knn_cells_kernel), lds);
+    if (st != TPK_OK)
+        return st;
+    hipLaunchKernelGGL(knn_cells_kernel, dim3(static_cast<unsigned>(bpc * b)), dim3(LG_THREADS), lds, stream, n, m, k,
+                       static_cast<int>(bpc), per_block, knn_per_cell(k), query, support, dist2, idx);
+    return tpk_launch_status();
+}
+
+// Larger clouds: the grid in memory, built by one workgroup per cloud.  Two passes over the points - their box, then
+// their cells' counts in LDS -, a prefix sum, and a third that writes every point's record to its cell.
+constexpr int KNG_CELLS = 32768; // cells at most (their counts lie in LDS)
+
+// Per cloud: the records [m], the cells' first places [KNG_CELLS + 64], the shape [16].
+struct KnnGridLayout
+{
+    size_t starts, shape, total;
+};
+inline KnnGridLayout knn_grid_layout(int m)
+{
+    KnnGridLayout l;
+    l.starts = (static_cast<size_t>(m) * sizeof(float4) + 255) & ~static_cast<size_t>(255);
+    l.shape = l.starts + (KNG_CELLS + TPK_WAVE) * sizeof(int);
+    l.total = l.shape + 256;
+    return l;
+}
+
+__global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float per_cell, KnnGridLayout layout,
+                                                                    const float* __restrict__ support, unsigned char* __restrict__ workspace)
+{
+    extern __shared__ __align__(16) int kng_counts[]; // [KNG_CELLS]
+    __shared__ int box[6];
+    __shared__ float shape[12];
+    __shared__ int wave_totals[LG_WAVES];
+    constexpr int BATCH = 8; // points in flight per lane
+    const int tid = threadIdx.x;
+    const int lane = tid & (TPK_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
+    support += static_cast<int64_t>(blockIdx.x) * m * 3;
+    workspace += blockIdx.x * layout.total;
+    float4* __restrict__ const records = reinterpret_cast<float4*>(workspace);
+    int* __restrict__ const starts = reinterpret_cast<int*>(workspace + layout.starts);
+
+    // f(point number, x, y, z) for every point of the cloud
+    auto each = [&](auto f) __attribute__((always_inline)) {
+        for (int first = tid; first < m; first += BATCH * LG_THREADS)
+        {
+            float px[BATCH], py[BATCH], pz[BATCH];
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+            {
+                const int t = min(first + u * LG_THREADS, m - 1);
+                px[u] = support[static_cast<int64_t>(t) * 3 + 0];
+                py[u] = support[static_cast<int64_t>(t) * 3 + 1];
+                pz[u] = support[static_cast<int64_t>(t) * 3 + 2];
+            }
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+                if (first + u * LG_THREADS < m)
+                    f(first + u * LG_THREADS, px[u], py[u], pz[u]);
+        }
+    };
+    if (tid < 6)
+        box[tid] = tid < 3 ? 0x7FFFFFFF : INT_MIN;
+    const float inf = __builtin_inff();
+    float lows[3] = {inf, inf, inf}, highs[3] = {-inf, -inf, -inf};
+    each([&](int, float x, float y, float z) {
+        const float v[3] = {x, y, z};
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+        {
+            const bool finite = fabsf(v[a]) < inf;
+            lows[a] = lg_min(lows[a], finite ? v[a] : inf);
+            highs[a] = lg_max(highs[a], finite ? v[a] : -inf);
+        }
+    });
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        const int low = ~wave_max_i32(~lg_ordered(lows[a])), high = wave_max_i32(lg_ordered(highs[a]));
+        if (lane == 0)
+        {
+            atomicMin(&box[a], low);
+            atomicMax(&box[3 + a], high);
+        }
+    }
+    __syncthreads();
+    if (wave == 0)
+        lg_shape(box, m, per_cell, KNG_AXIS, KNG_CELLS, lane, shape);
+    __syncthreads();
+    const float lo[3] = {shape[0], shape[1], shape[2]}, inv[3] = {shape[3], shape[4], shape[5]};
+    const int cx = __float_as_int(shape[9]), cy = __float_as_int(shape[10]), cz = __float_as_int(shape[11]);
+    const int cells = cx * cy * cz;
+    if (tid < 12)
+        reinterpret_cast<float*>(workspace + layout.shape)[tid] = shape[tid];
+    const int steps = (cells + 4 * LG_THREADS - 1) / (4 * LG_THREADS); // of the prefix sum, four cells per lane
+    for (int c = tid; c < steps * LG_THREADS; c += LG_THREADS)
+        reinterpret_cast<int4*>(kng_counts)[c] = make_int4(0, 0, 0, 0);
+    __syncthreads();
+    auto cell_of = [&](float x, float y, float z) __attribute__((always_inline)) {
+        return lg_cell((x - lo[0]) * inv[0], cx) + cx * (lg_cell((y - lo[1]) * inv[1], cy) + cy * lg_cell((z - lo[2]) * inv[2], cz));
+    };
+    each([&](int, float x, float y, float z) { atomicAdd(&kng_counts[cell_of(x, y, z)], 1); });
+    __syncthreads();
+    int placed = 0; // points in the cells of the steps before
+    for (int step = 0; step < steps; ++step)
+    {
+        int4* const four = reinterpret_cast<int4*>(kng_counts) + step * LG_THREADS + tid;
+        const int4 c4 = *four;
+        const int own = c4.x + c4.y + c4.z + c4.w;
+        const int before = wave_exclusive_sum(own);
+        if (lane == TPK_WAVE - 1)
+            wave_totals[wave] = before + own;
+        __syncthreads();
+        const int total = lane < LG_WAVES ? wave_totals[lane] : 0;
+        const int totals_before = wave_exclusive_sum(total);
+        int at = placed + __builtin_amdgcn_readlane(totals_before, wave) + before;
+        placed += __builtin_amdgcn_readlane(totals_before + total, LG_WAVES - 1);
+        int4 s4;
+        s4.x = at;
+        s4.y = at += c4.x;
+        s4.z = at += c4.y;
+        s4.w = at += c4.z;
+        *four = s4;
+        reinterpret_cast<int4*>(starts)[step * LG_THREADS + tid] = s4; // (also those behind the last cell: the end)
+        __syncthreads();
+    }
+    if (tid == 0)
+        starts[steps * 4 * LG_THREADS] = m;
+    each([&](int t, float x, float y, float z) {
+        records[atomicAdd(&kng_counts[cell_of(x, y, z)], 1)] = make_float4(x, y, z, __int_as_float(t));
+    });
+}
+
+__global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t queries, int n, int m, int k, KnnGridLayout layout,
+                                                                      const float* __restrict__ query, const unsigned char* __restrict__ workspace,
+                                                                      float* __restrict__ dist2, int64_t* __restrict__ idx)
+{
+    __shared__ u64 keys[KNN_THREADS / TPK_WAVE][KNC_ROOM];
+    const int lane = threadIdx.x & (TPK_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TPK_WAVE);
+    const int64_t j = static_cast<int64_t>(xcd_local_block(blockIdx.x, gridDim.x)) * (KNN_THREADS / TPK_WAVE) + wave;
+    if (j >= queries)
+        return; // (no workgroup barrier anywhere in this kernel)
+    workspace += (j / n) * layout.total;
+    const float qx = to_vector_register(query[j * 3 + 0]), qy = to_vector_register(query[j * 3 + 1]), qz = to_vector_register(query[j * 3 + 2]);
+    const float* __restrict__ const shape = reinterpret_cast<const float*>(workspace + layout.shape);
+    TPK_WORK_DECL
+    LdsGrid grid;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        grid.lo[a] = shape[a];
+        grid.inv[a] = shape[3 + a];
+        grid.width[a] = shape[6 + a];
+        grid.cells[a] = __float_as_int(shape[9 + a]);
+    }
+    Survivors s;
+    s.keys = keys[wave];
+    s.lane = lane;
+    s.k = k;
+    u64 mine;
+    const int place = nearest_in_grid(grid, reinterpret_cast<const float4*>(workspace), reinterpret_cast<const int*>(workspace + layout.starts), m, k,
+                                      lane, qx, qy, qz, s, mine TPK_WORK_ARG);
+    if (place < k)
+    {
+        dist2[j * k + place] = __int_as_float(static_cast<int>(mine >> 32));
+        idx[j * k + place] = static_cast<int64_t>(mine & 0xFFFFFFFFu);
+    }
+    TPK_WORK_FLUSH
+}
+
+size_t knn_grid_workspace_bytes(int b, int m)
+{
+    return b > 0 && m > LG_MAX_POINTS ? b * knn_grid_layout(m).total : 0;
+}
+
+int launch_knn_grid(int b, int n, int m, int k, const float* query, const float* support, float* dist2, int64_t* idx, void* workspace,
+                    size_t workspace_bytes, hipStream_t stream)
+{
+    const int64_t queries = static_cast<int64_t>(b) * n, blocks = tpk_ceil_div(queries, KNN_THREADS / TPK_WAVE);
+    if (blocks > 0x7fffffffLL)
+        return TPK_ERR_UNSUPPORTED;
+    if (workspace_bytes < knn_grid_workspace_bytes(b, m) || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+        return TPK_ERR_WORKSPACE;
+    const size_t lds = KNG_CELLS * sizeof(int);
+    const int st = tpk_allow_lds(reinterpret_cast<const void*>(&knn_grid_build_kernel), lds);
+    if (st != TPK_OK)
+        return st;
+    const KnnGridLayout layout = knn_grid_layout(m);
+    unsigned char* const w = static_cast<unsigned char*>(workspace);
+    hipLaunchKernelGGL(knn_grid_build_kernel, dim3(b), dim3(LG_THREADS), lds, stream, m, knn_per_cell(k), layout, support, w);
+    hipLaunchKernelGGL(knn_grid_search_kernel, dim3(static_cast<unsigned>(blocks)), dim3(KNN_THREADS), 0, stream, queries, n, m, k, layout,
+                       query, w, dist2, idx);
+    return tpk_launch_status();
+}
+
 // The k nearest support points closer than `limit` (squared), for every query: search over
 // curve-ordered cells where it applies and a workspace is given, otherwise all pairs.
 int nearest_within(int b, int n_support, int m_query, int k, float limit, const float* support, const float* query,
@@ -172,7 +577,8 @@ int nearest_within(int b, int n_support, int m_query, int k, float limit, const 
 
 extern "C" size_t tpk_knn_workspace_bytes(int b, int n_support, int m_query)
 {
-    return tpk_grid_knn_workspace_bytes(b, m_query, n_support);
+    // (a list per lane; a wavefront per query)
+    return m_query > 0 ? std::max(tpk_grid_knn_workspace_bytes(b, m_query, n_support), knn_grid_workspace_bytes(b, n_support)) : 0;
 }
 
 extern "C" int tpk_knn_f32(int b, int n_support, int m_query, int k, const float* support,
@@ -187,6 +593,10 @@ extern "C" int tpk_knn_f32(int b, int n_support, int m_query, int k, const float
         return TPK_ERR_INVALID_ARG;
     if (static_cast<int64_t>(n_support) * 3 > 0x7fffffffLL || static_cast<int64_t>(m_query) * 3 > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
+    if (k <= KNC_MAX_K && n_support <= LG_MAX_POINTS)
+        return launch_knn_cells(b, m_query, n_support, k, query, support, dist2, idx, tpk_stream(stream));
+    if (k <= KNC_MAX_K && workspace)
+        return launch_knn_grid(b, m_query, n_support, k, query, support, dist2, idx, workspace, workspace_bytes, tpk_stream(stream));
     return nearest_within(b, n_support, m_query, k, __builtin_inff(), support, query, idx, dist2, workspace,
                           workspace_bytes, tpk_stream(stream));
 }

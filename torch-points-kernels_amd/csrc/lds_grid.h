@@ -1,8 +1,8 @@
 // A grid over a cloud of up to LG_MAX_POINTS points, built in LDS by a workgroup of LG_THREADS lanes, and the
-// search for a query's nearest points in it, one lane per query (three_nn.hip).
+// search for a query's nearest points in it, one lane per query (three_nn.hip; knn.hip searches it by wavefronts).
 //
 // Build: bounding box of the finite coordinates, up to LG_AXIS cells per axis and LG_CELLS in all sized for
-// about LG_PER_CELL points per cell (a flat cloud gets a flat grid), a count per cell (LDS atomics that also
+// about per_cell points per cell (a flat cloud gets a flat grid), a count per cell (LDS atomics that also
 // hand every point its place inside its cell), a prefix sum, the points written cell by cell as records
 // (x, y, z, index) of 16 bytes.  Search: cells are numbered x first, so the (up to) three cells of a row (y, z)
 // are one run of consecutive places; a lane walks the runs around its query point by point - its own cell first, a row is
@@ -28,7 +28,7 @@ constexpr int LG_PER_THREAD = LG_MAX_POINTS / LG_THREADS;
 constexpr int LG_AXIS = 64;    // cells per axis at most
 constexpr int LG_CELLS = 4096; // cells in all at most
 constexpr int LG_STARTS = LG_CELLS + TPK_WAVE; // the cells' first places, one more for the end, padded
-constexpr float LG_PER_CELL = 2.0f;            // points per cell aimed at (1 / 1.5 / 3: 9 / 6 / 1 % slower on three_nn)
+constexpr float LG_PER_CELL = 2.0f;            // points per cell three_nn aims at (1 / 1.5 / 3: 9 / 6 / 1 % slower)
 
 // Dynamic LDS a grid over m points takes.
 inline size_t lg_lds_bytes(int m)
@@ -89,20 +89,69 @@ __device__ __forceinline__ unsigned long long lg_key(float d, int i)
     return (static_cast<unsigned long long>(static_cast<unsigned>(__float_as_int(d))) << 32) | static_cast<unsigned>(i);
 }
 
+// The grid's shape, by one wavefront: lo, 1 / width, width and number of cells along each axis (shape[0 .. 11]) for about
+// per_cell of m points per cell, cells as cubic as `axis` per axis (at most 128) and `most` in all allow (a flat cloud
+// gets a flat grid).  box: ordered ints, min x, y, z then max x, y, z.  The lanes try 64 sizes at a time.
+__device__ __forceinline__ void lg_shape(const int* box, int m, float per_cell, int axis, int most, int lane, float* shape)
+{
+            float low[3], extent[3], longest = 0.0f;
+    #pragma unroll
+            for (int a = 0; a < 3; ++a)
+            {
+                low[a] = lg_unordered(box[a]);
+                extent[a] = lg_unordered(box[3 + a]) - low[a]; // (NaN or -inf for a cloud without finite coordinates)
+                extent[a] = extent[a] > 0.0f ? extent[a] : 0.0f;
+                longest = fmaxf(longest, extent[a]);
+            }
+            float share[3]; // of the longest axis
+    #pragma unroll
+            for (int a = 0; a < 3; ++a)
+                share[a] = longest > 0.0f ? extent[a] / longest : 0.0f;
+            // cells per axis for `along` cells along the longest axis, and their product
+            auto fit = [&](float along, int (&count)[3]) __attribute__((always_inline)) {
+                int all = 1;
+    #pragma unroll
+                for (int a = 0; a < 3; ++a)
+                {
+                    const float f = longest > 0.0f ? fminf(share[a] * along + 0.5f, static_cast<float>(axis)) : 1.0f;
+                    count[a] = f >= 1.0f ? static_cast<int>(f) : 1;
+                    all *= count[a];
+                }
+                return all;
+            };
+            // (the product grows with `along`: the largest of the sizes tried that stays within the cells wanted, in
+            // steps of 2 up to 128, then in steps of 1 / 32 inside the step found)
+            const int wanted = static_cast<int>(fminf(static_cast<float>(most), fmaxf(static_cast<float>(m) / per_cell, 1.0f)));
+            int count[3];
+            const int coarse = __builtin_popcountll(__ballot(fit(2.0f * static_cast<float>(lane + 1), count) <= wanted));
+            const int fine = __builtin_popcountll(__ballot(fit(2.0f * static_cast<float>(coarse) + static_cast<float>(lane + 1) * (1.0f / 32.0f), count) <= wanted));
+            fit(2.0f * static_cast<float>(coarse) + static_cast<float>(fine) * (1.0f / 32.0f), count);
+            if (lane < 3)
+            {
+                const float e = lane == 0 ? extent[0] : lane == 1 ? extent[1] : extent[2];
+                const float l = lane == 0 ? low[0] : lane == 1 ? low[1] : low[2];
+                const int k = lane == 0 ? count[0] : lane == 1 ? count[1] : count[2];
+                shape[lane] = e > 0.0f ? l : 0.0f;
+                shape[3 + lane] = e > 0.0f ? static_cast<float>(k) / e : 0.0f;
+                shape[6 + lane] = e / static_cast<float>(k);
+                shape[9 + lane] = __int_as_float(k);
+            }
+}
+
 struct LdsGrid
 {
     float4* points;      // [m] the points cell by cell: x, y, z, index
     int* starts;         // [LG_STARTS] first place of every cell, then the number of points
     float lo[3], inv[3], width[3];
     int cells[3];
-    float crowd;         // points per cell as a point sees them (3 in a cloud of even density, LG_PER_CELL + 1)
+    float crowd;         // points per cell as a point sees them (per_cell + 1 in a cloud of even density)
 };
 
 // Builds the grid over known[0 .. m) (m <= LG_MAX_POINTS) in `lds` (lg_lds_bytes(m) bytes, 16-byte aligned); the
-// points are recorded under index_base + their number.  Every lane of the workgroup calls it; it starts and ends
+// points are recorded under index_base + their number, the cells sized for per_cell points each.  Every lane of the workgroup calls it; it starts and ends
 // with a barrier, so it may follow searches in an earlier grid at the same place.
 __device__ __forceinline__ void lds_grid_build(LdsGrid& g, unsigned char* lds, const float* __restrict__ known, int m,
-                                               int index_base)
+                                               int index_base, float per_cell)
 {
     float4* const points = g.points = reinterpret_cast<float4*>(lds);
     int* const starts = g.starts = reinterpret_cast<int*>(points + m);
@@ -160,53 +209,10 @@ __device__ __forceinline__ void lds_grid_build(LdsGrid& g, unsigned char* lds, c
     }
     __syncthreads();
 
-    // ---- the grid: about LG_PER_CELL points per cell, cells as cubic as LG_AXIS per axis and LG_CELLS in
-    // all allow (a flat cloud gets a flat grid of up to 64 x 64 cells).  The first wavefront works it out, its
-    // lanes trying 64 sizes at a time. ----
+    // ---- the grid: the first wavefront works its shape out ----
     if (wave == 0)
     {
-        float low[3], extent[3], longest = 0.0f;
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-        {
-            low[a] = lg_unordered(box[a]);
-            extent[a] = lg_unordered(box[3 + a]) - low[a]; // (NaN or -inf for a cloud without finite coordinates)
-            extent[a] = extent[a] > 0.0f ? extent[a] : 0.0f;
-            longest = fmaxf(longest, extent[a]);
-        }
-        float share[3]; // of the longest axis
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-            share[a] = longest > 0.0f ? extent[a] / longest : 0.0f;
-        // cells per axis for `along` cells along the longest axis, and their product
-        auto fit = [&](float along, int (&count)[3]) __attribute__((always_inline)) {
-            int all = 1;
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-            {
-                const float f = longest > 0.0f ? fminf(share[a] * along + 0.5f, static_cast<float>(LG_AXIS)) : 1.0f;
-                count[a] = f >= 1.0f ? static_cast<int>(f) : 1;
-                all *= count[a];
-            }
-            return all;
-        };
-        // (the product grows with `along`: the largest of the sizes tried that stays within the cells wanted, in
-        // steps of 2 up to 2 * LG_AXIS, then in steps of 1 / 32 inside the step found)
-        const int wanted = static_cast<int>(fminf(static_cast<float>(LG_CELLS), fmaxf(static_cast<float>(m) / LG_PER_CELL, 1.0f)));
-        int count[3];
-        const int coarse = __builtin_popcountll(__ballot(fit(2.0f * static_cast<float>(lane + 1), count) <= wanted));
-        const int fine = __builtin_popcountll(__ballot(fit(2.0f * static_cast<float>(coarse) + static_cast<float>(lane + 1) * (1.0f / 32.0f), count) <= wanted));
-        fit(2.0f * static_cast<float>(coarse) + static_cast<float>(fine) * (1.0f / 32.0f), count);
-        if (lane < 3)
-        {
-            const float e = lane == 0 ? extent[0] : lane == 1 ? extent[1] : extent[2];
-            const float l = lane == 0 ? low[0] : lane == 1 ? low[1] : low[2];
-            const int k = lane == 0 ? count[0] : lane == 1 ? count[1] : count[2];
-            shape[lane] = e > 0.0f ? l : 0.0f;
-            shape[3 + lane] = e > 0.0f ? static_cast<float>(k) / e : 0.0f;
-            shape[6 + lane] = e / static_cast<float>(k);
-            shape[9 + lane] = __int_as_float(k);
-        }
+        lg_shape(box, m, per_cell, LG_AXIS, LG_CELLS, lane, shape);
     }
     __syncthreads();
     float lo[3], inv[3], width[3];

@@ -1423,12 +1423,6 @@ int tpk_grid_knn(int b, int n, int m, int k, float limit, const float* query, co
     if (st != TPK_OK)
         return st;
     const int qcells = grid_cells(n), ccells = grid_cells(m);
-    if (k <= 4)
-        return launch_knn_grid<4>(b, n, k, limit, qcells, ccells, a, c, dist2, idx, s);
-    if (k <= 8)
-        return launch_knn_grid<8>(b, n, k, limit, qcells, ccells, a, c, dist2, idx, s);
-    if (k <= 16)
-        return launch_knn_grid<16>(b, n, k, limit, qcells, ccells, a, c, dist2, idx, s);
     return launch_knn_grid<KNN_MAX_K>(b, n, k, limit, qcells, ccells, a, c, dist2, idx, s);
 }
 

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(LG_THREADS) void three_nn_cells_kernel(
     TPK_WORK_DECL
 
     LdsGrid grid;
-    lds_grid_build(grid, tnc_lds, known, m, 0);
+    lds_grid_build(grid, tnc_lds, known, m, 0, LG_PER_CELL);
     // Points per cell as a point sees them (3 in a cloud of even density): above TNC_CROWDED the grid is a poor
     // fit - dense cells cost their queries many candidates, empty ones many steps of widening - and, where the
     // caller enqueues it behind this kernel, the search over curve-ordered cells answers the cloud instead.
