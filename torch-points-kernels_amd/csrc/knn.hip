@@ -166,10 +166,11 @@ __device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4
     const int cx = grid.cells[0], cy = grid.cells[1], cz = grid.cells[2];
     const float q[3] = {qx, qy, qz};
     s.clear();
+    s.unit = 0.0f;
     bool separated = true; // every selection so far found its distance
 
     // The candidates of up to 64 rows of cells, a row per lane (start, size), offered.
-    auto walk = [&](int start, int size, int before, int total, bool ball) __attribute__((always_inline)) {
+    auto walk = [&](int start, int size, int before, int total) __attribute__((always_inline)) {
         const int origin = start - before; // candidate c of the walk lies at origin + c, for the c of this lane's row
         for (int c0 = 0; c0 < total && separated; c0 += TPK_WAVE)
         {
@@ -182,14 +183,18 @@ __device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4
             const bool has = c0 + lane < total;
             const float4 p = points[has ? at : 0];
             TPK_WORK_ADD(1);
-            separated = s.offer(has, tpk_dist2(qx, qy, qz, p.x, p.y, p.z), __float_as_int(p.w), ball);
+            separated = s.offer(has, tpk_dist2(qx, qy, qz, p.x, p.y, p.z), __float_as_int(p.w));
         }
     };
 
     // ---- the block of cells around the query that holds k points ----
     int c[3];
+    float t[3]; // in cells
     for (int a = 0; a < 3; ++a)
-        c[a] = __builtin_amdgcn_readfirstlane(lg_cell((q[a] - grid.lo[a]) * grid.inv[a], grid.cells[a]));
+    {
+        t[a] = (q[a] - grid.lo[a]) * grid.inv[a];
+        c[a] = __builtin_amdgcn_readfirstlane(lg_cell(t[a], grid.cells[a]));
+    }
     int xl, xh, yl, yh, zl, zh;
     // (a crowded cell may do alone: its 26 neighbours would be as crowded)
     const int own = c[0] + cx * (c[1] + cy * c[2]);
@@ -208,7 +213,7 @@ __device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4
                 const int c0 = min(row0 + lane, rows - 1) * cx;
                 const int start = starts[c0], size = row0 + lane < rows ? starts[c0 + cx] - start : 0;
                 const int before = wave_exclusive_sum(size);
-                walk(start, size, before, __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1), false);
+                walk(start, size, before, __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1));
             }
             break;
         }
@@ -224,35 +229,41 @@ __device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4
         const int total = __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1);
         if (total < k)
             continue;
-        walk(start, size, before, total, false);
+        // a ball that holds one of them, of the block's volume: 3 / (4 pi) x cells / total (a flat cloud's cells: as wide as
+        // they are long)
+        const float longest = fmaxf(fmaxf(grid.width[0], grid.width[1]), grid.width[2]);
+        float volume = 0.2387f * static_cast<float>(rows * (xh - xl + 1)) * __builtin_amdgcn_rcpf(static_cast<float>(total));
+        for (int a = 0; a < 3; ++a)
+            volume *= grid.width[a] > 0.0f ? grid.width[a] : longest;
+        s.unit = s.volume_ratio(volume);
+        walk(start, size, before, total);
         break;
     }
 
     // ---- the k-th so far bounds the ball; the cells it touches outside the block ----
     mine = ~0ull;
     int place = KNC_MOST;
-    separated = separated && s.count >= k && (s.count <= KNC_MOST || s.select(__builtin_inff(), 0, false));
+    separated = separated && s.count >= k && (s.count <= KNC_MOST || s.select(__builtin_inff(), 0));
     if (separated)
     {
         place = s.rank(mine);
         const int kth = __builtin_ctzll(__ballot(place == k - 1));
         const float bound = tpk_read_lane(__int_as_float(static_cast<int>(mine >> 32)), kth);
-        const float radius = sqrtf(bound) * 1.000001f;
+        const float radius = __builtin_amdgcn_sqrtf(bound) * 1.00001f;
         int from[3], to[3];
         for (int a = 0; a < 3; ++a)
         {
-            // (the ends a few ulps out, so that no point the rounded distances accept is left out)
-            const float slack = (fabsf(q[a]) + radius) * 1e-6f + 1e-30f;
-            from[a] = __builtin_amdgcn_readfirstlane(lg_cell(((q[a] - radius) - slack - grid.lo[a]) * grid.inv[a], grid.cells[a]));
-            to[a] = __builtin_amdgcn_readfirstlane(lg_cell(((q[a] + radius) + slack - grid.lo[a]) * grid.inv[a], grid.cells[a]));
+            // (the ends further out than rounding may have moved a point's cell by)
+            const float span = radius * grid.inv[a] + 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS));
+            from[a] = __builtin_amdgcn_readfirstlane(lg_cell(t[a] - span, grid.cells[a]));
+            to[a] = __builtin_amdgcn_readfirstlane(lg_cell(t[a] + span, grid.cells[a]));
         }
         if (from[0] < xl || to[0] > xh || from[1] < yl || to[1] > yh || from[2] < zl || to[2] > zh)
         {
             // Distance along axis a from the query to a cell, a lower bound.
             auto apart = [&](int a, int at) __attribute__((always_inline)) {
-                const float t = (q[a] - grid.lo[a]) * grid.inv[a];
-                const float gap = fmaxf(static_cast<float>(at) - t, t - static_cast<float>(at + 1));
-                return fmaxf(gap - 1e-5f * (fabsf(t) + static_cast<float>(KNG_AXIS)), 0.0f) * grid.width[a];
+                const float gap = fmaxf(static_cast<float>(at) - t[a], t[a] - static_cast<float>(at + 1));
+                return fmaxf(gap - 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS)), 0.0f) * grid.width[a];
             };
             // the k kept in order, then the rest of the ball: two pieces for a row that crosses the block
             if (place < k)
@@ -281,9 +292,9 @@ __device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4
                     }
                 }
                 const int before = wave_exclusive_sum(size);
-                walk(start, size, before, __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1), true);
+                walk(start, size, before, __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1));
             }
-            separated = separated && (s.count <= KNC_MOST || s.select(__builtin_inff(), 0, true));
+            separated = separated && (s.count <= KNC_MOST || s.select(__builtin_inff(), 0));
             if (separated && (s.count > k || s.reach != bound)) // (else none came along, and the k lie in order)
                 place = s.rank(mine);
             else if (separated)
@@ -397,23 +408,32 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
     float4* __restrict__ const records = reinterpret_cast<float4*>(workspace);
     int* __restrict__ const starts = reinterpret_cast<int*>(workspace + layout.starts);
 
-    // f(point number, x, y, z) for every point of the cloud
-    auto each = [&](auto f) __attribute__((always_inline)) {
-        for (int first = tid; first < m; first += BATCH * LG_THREADS)
-        {
-            float px[BATCH], py[BATCH], pz[BATCH];
+    // f(point number, x, y, z) for every point of the cloud; a lane's first BATCH points stay in its registers
+    float hx[BATCH], hy[BATCH], hz[BATCH];
+    auto load = [&](int first, float (&px)[BATCH], float (&py)[BATCH], float (&pz)[BATCH]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u)
-            {
-                const int t = min(first + u * LG_THREADS, m - 1);
-                px[u] = support[static_cast<int64_t>(t) * 3 + 0];
-                py[u] = support[static_cast<int64_t>(t) * 3 + 1];
-                pz[u] = support[static_cast<int64_t>(t) * 3 + 2];
-            }
+        for (int u = 0; u < BATCH; ++u)
+        {
+            const int64_t t = min(first + u * LG_THREADS, m - 1);
+            px[u] = support[t * 3 + 0];
+            py[u] = support[t * 3 + 1];
+            pz[u] = support[t * 3 + 2];
+        }
+    };
+    load(tid, hx, hy, hz);
+    auto each = [&](auto f) __attribute__((always_inline)) {
+        auto batch = [&](int first, const float (&px)[BATCH], const float (&py)[BATCH], const float (&pz)[BATCH]) __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
                 if (first + u * LG_THREADS < m)
                     f(first + u * LG_THREADS, px[u], py[u], pz[u]);
+        };
+        batch(tid, hx, hy, hz);
+        for (int first = tid + BATCH * LG_THREADS; first < m; first += BATCH * LG_THREADS)
+        {
+            float px[BATCH], py[BATCH], pz[BATCH];
+            load(first, px, py, pz);
+            batch(first, px, py, pz);
         }
     };
     if (tid < 6)
@@ -527,9 +547,18 @@ __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t qu
     TPK_WORK_FLUSH
 }
 
-size_t knn_grid_workspace_bytes(int b, int m)
+// The grid in LDS saves a launch and the one workgroup per cloud in front of the search; the grid in memory leaves room for
+// twice as many wavefronts.  (16 queries per wavefront of the chip: k = 16, 4 x 4000: 25.3 and 26.3 us, 8 x 4099: 42.8 and
+// 39.6 us, 8 x 8192: 73.8 and 65.4 us.)
+constexpr int64_t KNC_LDS_QUERIES = 16384;
+inline bool knn_in_lds(int b, int m, int n, bool workspace)
 {
-    return b > 0 && m > LG_MAX_POINTS ? b * knn_grid_layout(m).total : 0;
+    return m <= LG_MAX_POINTS && (static_cast<int64_t>(b) * n <= KNC_LDS_QUERIES || !workspace);
+}
+
+size_t knn_grid_workspace_bytes(int b, int m, int n)
+{
+    return b > 0 && n > 0 && !knn_in_lds(b, m, n, true) ? b * knn_grid_layout(m).total : 0;
 }
 
 int launch_knn_grid(int b, int n, int m, int k, const float* query, const float* support, float* dist2, int64_t* idx, void* workspace,
@@ -538,7 +567,7 @@ int launch_knn_grid(int b, int n, int m, int k, const float* query, const float*
     const int64_t queries = static_cast<int64_t>(b) * n, blocks = tpk_ceil_div(queries, KNN_THREADS / TPK_WAVE);
     if (blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    if (workspace_bytes < knn_grid_workspace_bytes(b, m) || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+    if (workspace_bytes < knn_grid_workspace_bytes(b, m, n) || (reinterpret_cast<uintptr_t>(workspace) & 255u))
         return TPK_ERR_WORKSPACE;
     const size_t lds = KNG_CELLS * sizeof(int);
     const int st = tpk_allow_lds(reinterpret_cast<const void*>(&knn_grid_build_kernel), lds);
@@ -578,7 +607,7 @@ int nearest_within(int b, int n_support, int m_query, int k, float limit, const 
 extern "C" size_t tpk_knn_workspace_bytes(int b, int n_support, int m_query)
 {
     // (a list per lane; a wavefront per query)
-    return m_query > 0 ? std::max(tpk_grid_knn_workspace_bytes(b, m_query, n_support), knn_grid_workspace_bytes(b, n_support)) : 0;
+    return m_query > 0 ? std::max(tpk_grid_knn_workspace_bytes(b, m_query, n_support), knn_grid_workspace_bytes(b, n_support, m_query)) : 0;
 }
 
 extern "C" int tpk_knn_f32(int b, int n_support, int m_query, int k, const float* support,
@@ -593,7 +622,7 @@ extern "C" int tpk_knn_f32(int b, int n_support, int m_query, int k, const float
         return TPK_ERR_INVALID_ARG;
     if (static_cast<int64_t>(n_support) * 3 > 0x7fffffffLL || static_cast<int64_t>(m_query) * 3 > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    if (k <= KNC_MAX_K && n_support <= LG_MAX_POINTS)
+    if (k <= KNC_MAX_K && knn_in_lds(b, n_support, m_query, workspace != nullptr))
         return launch_knn_cells(b, m_query, n_support, k, query, support, dist2, idx, tpk_stream(stream));
     if (k <= KNC_MAX_K && workspace)
         return launch_knn_grid(b, m_query, n_support, k, query, support, dist2, idx, workspace, workspace_bytes, tpk_stream(stream));

@@ -28,11 +28,17 @@ struct Survivors
     u64* keys; // [KNC_ROOM] in LDS, the wavefront's own
     int lane, k, count;
     float reach; // candidates beyond this squared distance do not matter
+    float unit;  // about the squared distance within which one candidate lies, before reach is known
 
     __device__ __forceinline__ void clear()
     {
         count = 0;
         reach = __builtin_inff();
+    }
+    // Ratio of squared distances to a ratio of volumes.
+    __device__ __forceinline__ float volume_ratio(float counts) const
+    {
+        return __builtin_amdgcn_exp2f(0.66667f * __builtin_amdgcn_logf(counts));
     }
     __device__ __forceinline__ int within(const float (&v)[3], float t) const
     {
@@ -41,8 +47,9 @@ struct Survivors
     }
     // Reduces the survivors and this step's candidates (d; +inf for none) to between k and `most`, and `reach` with
     // them.  False when no distance separates so few (equal distances): the caller starts over another way.
-    // ball: the candidates fill a ball around the query (else a block of cells).
-    __device__ __forceinline__ bool select(float d, int i, bool ball)
+    // The count within a distance grows about as the volume does: the first guess comes from `unit`, the later ones from
+    // the last count.
+    __device__ __forceinline__ bool select(float d, int i)
     {
         const float inf = __builtin_inff();
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -50,32 +57,28 @@ struct Survivors
         float v[3] = {lane < count ? __int_as_float(static_cast<int>(k0 >> 32)) : inf,
                       lane + TPK_WAVE < count ? __int_as_float(static_cast<int>(k1 >> 32)) : inf, d};
         const int most = min(k + KNC_SPARE, KNC_MOST);
-        float far = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 3; ++u)
-            far = fmaxf(far, v[u] < inf ? v[u] : 0.0f);
-        float hi = __int_as_float(wave_max_i32(__float_as_int(far))), lo = 0.0f;
-        int in_hi = within(v, hi);
-        // the count grows about as the volume does, with the distance to the third
         const float target = static_cast<float>(k + (most - k) / 2);
-        float guess = hi;
-        int in_guess = in_hi;
-        float scale = ball ? 1.0f : 0.4f; // (a block of 27 cells: its corners are further away than its faces)
+        float lo = 0.0f, hi = __builtin_inff(), guess = reach; // (reach: all of them, or +inf before the first selection)
+        int in_guess = TPK_WAVE + count;
+        if (reach == inf)
+        {
+            guess = tpk_read_lane(unit * volume_ratio(target), 0);
+            in_guess = within(v, guess);
+        }
         for (int tries = 0; in_guess < k || in_guess > most; ++tries)
         {
             if (tries > 40)
                 return false;
-            // from the nearer side of the bracket; bisection of the bit patterns when that leaves it
-            float next = guess * scale * __builtin_amdgcn_exp2f(0.66667f * __builtin_amdgcn_logf(target * __builtin_amdgcn_rcpf(fmaxf(static_cast<float>(in_guess), 0.5f))));
-            scale = 1.0f;
-            if (!(next > lo && next < hi) || tries > 5)
-                next = __int_as_float((__float_as_int(lo) + __float_as_int(hi)) >> 1);
-            guess = tpk_read_lane(next, 0);
-            in_guess = within(v, guess);
             if (in_guess < k)
                 lo = guess;
             else
                 hi = guess;
+            // from the last guess; bisection of the bit patterns when that leaves the bracket, or after a few
+            float next = guess * volume_ratio(target * __builtin_amdgcn_rcpf(fmaxf(static_cast<float>(in_guess), 0.5f)));
+            if (!(next > lo && next < hi) || tries > 5)
+                next = __int_as_float((__float_as_int(lo) + __float_as_int(hi)) >> 1);
+            guess = tpk_read_lane(next, 0);
+            in_guess = within(v, guess);
         }
         reach = guess;
         count = 0;
@@ -92,14 +95,14 @@ struct Survivors
         count += __builtin_popcountll(mask);
     }
     // One candidate per lane (in = false: none).
-    __device__ __forceinline__ bool offer(bool in, float d, int i, bool ball)
+    __device__ __forceinline__ bool offer(bool in, float d, int i)
     {
         in = in && d <= reach && d < __builtin_inff();
         const int more = __builtin_popcountll(__ballot(in));
         if (more == 0)
             return true;
         if (count + more > KNC_ROOM)
-            return select(in ? d : __builtin_inff(), i, ball);
+            return select(in ? d : __builtin_inff(), i);
         put(in, knn_key(d, i));
         return true;
     }
