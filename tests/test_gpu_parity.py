@@ -966,6 +966,19 @@ def test_grouping_grad_long_rows(tpk, oracle, dev, N, npoint, nsample, C):
     _assert_scatter_sum_close(_np(f.grad), want, oracle.grouping_operation_grad(gout.abs().numpy(), idx.numpy(), N))
 
 
+@pytest.mark.parametrize("columns", [1, 1023, 1024, 1025, 5121])
+def test_gather_full_grids(tpk, oracle, dev, columns):
+    # grids with a workgroup for every compute unit: each starts at another run of 1024 columns and wraps around
+    g = torch.Generator().manual_seed(columns)
+    feats = torch.randn(8, 66, 300, generator=g)
+    idx = torch.randint(0, 300, (8, columns, 1), generator=g)
+    out = tpk.grouping_operation(feats.to(dev), idx.to(dev))
+    np.testing.assert_array_equal(_np(out), oracle.grouping_operation(feats.numpy(), idx.numpy()))
+    feats, idx, w, _ = _interp_case(32, 66, 300, columns, columns)
+    out = tpk.three_interpolate(feats.to(dev), idx.to(dev), w.to(dev))
+    np.testing.assert_array_equal(_np(out), oracle.three_interpolate(feats.numpy(), idx.numpy(), w.numpy()))
+
+
 def test_grouping_full_config3b(tpk, oracle, dev):
     w = W.cfg3b_grouping()
     f = w["features"].to(dev).requires_grad_(True)

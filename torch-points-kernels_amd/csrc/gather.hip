@@ -37,6 +37,7 @@ namespace {
 
 constexpr int G_MAX_ROWS = 8;
 constexpr int G_LDS_BUDGET = 131072; // bytes of LDS for the staged rows
+constexpr unsigned G_FULL_GRID = 256;  // a workgroup for every compute unit
 constexpr int G_PLAIN_BLOCKS = 1024; // workgroups the plain gather aims at (four per compute unit, two at a time)
 
 template <int K, bool WEIGHTED, typename IdxT>
@@ -133,14 +134,22 @@ __device__ __forceinline__ void stage_copy(float* dst, const float* __restrict__
 }
 
 // grid: (clouds * row_blocks * jsplit).  dynamic LDS: R * m floats.
-template <int K, bool WEIGHTED, typename IdxT, bool XCD_LOCAL>
+//
+// Bound by the output's way to memory.  All workgroups write rows that lie a multiple of the row length apart: where
+// they walk the columns in step and that length is a power of two, their stores meet in the same few memory channels.
+// Every workgroup therefore starts at another run of G_THREADS columns and wraps around (xcd_local_block keeps a
+// cloud's workgroups, and the indices they share, on one die).  Measured behind a pass over other memory (16 clouds,
+// 128 channels): rows of 32768 columns, plain, 99 -> 60 us (348 MB: 5.8 TB/s; a large copy here moves 5.3), without
+// the dies 64; rows of 16384 columns, three weighted neighbours, 54 -> 41 us (174 MB), without the dies 49.
+template <int K, bool WEIGHTED, typename IdxT>
 __global__ __launch_bounds__(G_THREADS) void gather_fwd_lds_kernel(
     int c, int m, int64_t n, int rows_per_block, int row_blocks, int jsplit, int64_t jlen,
     const float* __restrict__ src, const IdxT* __restrict__ idx,
     const float* __restrict__ weight, float* __restrict__ out)
 {
     extern __shared__ float rows[];
-    int bid = XCD_LOCAL ? static_cast<int>(xcd_local_block(blockIdx.x, gridDim.x)) : static_cast<int>(blockIdx.x);
+    const unsigned block = xcd_local_block(blockIdx.x, gridDim.x);
+    int bid = static_cast<int>(block);
     const int jpart = bid % jsplit;
     bid /= jsplit;
     const int rb = bid % row_blocks;
@@ -155,39 +164,42 @@ __global__ __launch_bounds__(G_THREADS) void gather_fwd_lds_kernel(
     const int64_t jbeg = static_cast<int64_t>(jpart) * jlen;
     const int64_t jend = tpk_min64(n, jbeg + jlen);
     const float* __restrict__ s = src + (static_cast<int64_t>(cloud) * c + c0) * m;
+    if (jbeg >= jend)
+        return; // (rounding of jlen: a part without columns)
 
-    if (WEIGHTED)
-    {
-        // Bound by the random LDS reads: a column's indices and weights are requested one column ahead, the
-        // first before the rows are staged, so that no lane waits for them between its reads.
-        int64_t j = jbeg + threadIdx.x;
-        Column<K, WEIGHTED, IdxT> next;
-        if (j < jend)
-            next.load(idx, weight, j);
-        stage_copy(rows, s, static_cast<unsigned>(nrows) * static_cast<unsigned>(m));
-        __syncthreads();
-        for (; j < jend; j += G_THREADS)
-        {
-            const Column<K, WEIGHTED, IdxT> col = next;
-            next.load(idx, weight, tpk_min64(j + G_THREADS, jend - 1));
-#pragma unroll
-            for (int r = 0; r < G_MAX_ROWS; ++r)
-                if (r < nrows)
-                    o[static_cast<int64_t>(r) * n + j] = col.combine(rows + r * m);
-        }
-        return;
-    }
+    // The runs of G_THREADS columns of this part, from run `first` on and around.  (A grid that leaves compute units idle
+    // is bound by latency, and its workgroups gain from asking for the same indices together.)
+    const unsigned runs = static_cast<unsigned>((jend - jbeg + G_THREADS - 1) / G_THREADS);
+    const unsigned first = gridDim.x >= G_FULL_GRID ? block % runs : 0u;
+    auto column = [&](unsigned i) __attribute__((always_inline)) {
+        const unsigned run = first + i < runs ? first + i : first + i - runs;
+        return jbeg + static_cast<int64_t>(run) * G_THREADS + threadIdx.x;
+    };
+    // A column's indices (and weights) are requested one run ahead of the one whose rows are read, the first before the
+    // rows are staged: no lane waits for them between its LDS reads.
+    Column<K, WEIGHTED, IdxT> next;
+    next.load(idx, weight, tpk_min64(column(0), jend - 1));
     stage_copy(rows, s, static_cast<unsigned>(nrows) * static_cast<unsigned>(m));
     __syncthreads();
-    for (int64_t j = jbeg + threadIdx.x; j < jend; j += G_THREADS)
+    for (unsigned i = 0; i < runs; ++i)
     {
-        Column<K, WEIGHTED, IdxT> col;
-        col.load(idx, weight, j);
+        const int64_t j = column(i);
+        const Column<K, WEIGHTED, IdxT> col = next;
+        if (i + 1 < runs)
+            next.load(idx, weight, tpk_min64(column(i + 1), jend - 1));
+        if (j >= jend)
+            continue;
 #pragma unroll
         for (int r = 0; r < G_MAX_ROWS; ++r)
             if (r < nrows)
-                // (written once, read by nobody here: past the caches, -3 % on config 3b)
-                __builtin_nontemporal_store(col.combine(rows + r * m), &o[static_cast<int64_t>(r) * n + j]);
+            {
+                const float v = col.combine(rows + r * m);
+                float* const to = &o[static_cast<int64_t>(r) * n + j];
+                if constexpr (WEIGHTED)
+                    *to = v;
+                else
+                    __builtin_nontemporal_store(v, to); // (written once, read by nobody here: past the caches)
+            }
     }
 }
 
@@ -700,8 +712,8 @@ int gather_fwd(int b, int c, int m, int64_t n, const float* src, const IdxT* idx
     // The plain gather is bound by its stores and gains from two workgroups per compute unit that stage and store
     // at different times, and from row blocks that are not split by columns (every split stages the rows again):
     // fewer rows per workgroup while that gives more workgroups, down to two rows (with one row the indices, read
-    // once per row block, become the larger stream).  Config 3b: 8 rows x 2 column parts 62 us, 4 rows 59, 2 rows 55,
-    // 1 row 78.
+    // once per row block, become the larger stream).  16 clouds of 4096 points, 128 channels, 32768 columns: 2 rows
+    // 60 us, 4 rows 63, 1 row 70.
     if (!WEIGHTED)
         while (r > 2 && static_cast<int64_t>(b) * tpk_ceil_div(c, r) < G_PLAIN_BLOCKS)
             r = (r + 1) / 2;
@@ -721,10 +733,7 @@ int gather_fwd(int b, int c, int m, int64_t n, const float* src, const IdxT* idx
         if (blocks > 0x7fffffffLL)
             return TPK_ERR_UNSUPPORTED;
         const size_t lds = static_cast<size_t>(r) * m * sizeof(float);
-        // Measured on MI355X: the weighted 3-neighbour gather (LDS-read bound) is fastest with one
-        // workgroup per compute unit and die-local cloud placement; the plain gather (store
-        // bound) with two workgroups per compute unit at a time and the default placement.
-        auto kernel = gather_fwd_lds_kernel<K, WEIGHTED, IdxT, WEIGHTED>;
+        auto kernel = gather_fwd_lds_kernel<K, WEIGHTED, IdxT>;
         int st = allow_lds(kernel, lds);
         if (st != TPK_OK)
             return st;
