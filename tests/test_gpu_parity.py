@@ -931,6 +931,32 @@ def test_backward_over_lists_built_in_the_forward_pass(tpk, oracle, dev):
                               oracle.three_interpolate_grad(gout.abs().numpy(), idx.numpy(), w.numpy(), 60000))
 
 
+@pytest.mark.parametrize("sort", [False, True])
+@pytest.mark.parametrize("rest", [0, 4, 40])
+def test_ball_query_packed_long_bins(tpk, oracle, dev, rest, sort):
+    # clusters of 47 .. 129 points about a bin apart (steps that are full, nearly full and begun), and clusters of `rest`
+    # points: how many of them a query touches decides whether it walks its bins one after the other or together
+    g = torch.Generator().manual_seed(rest)
+    sizes = [47, 48, 63, 64, 65, 127, 128, 129] * 6
+    spots = torch.randperm(16 ** 3, generator=g)
+    where = [torch.full((n,), int(spots[i])) for i, n in enumerate(sizes)]
+    where += [torch.full((rest,), int(v)) for v in spots[len(sizes) : len(sizes) + 200]]
+    where = torch.cat(where)
+    where = where[torch.randperm(where.numel(), generator=g)]
+    where = where.repeat(-(-9000 // where.numel()))
+    x = torch.stack([where % 16, (where // 16) % 16, where // 256], 1).float() + 0.8 * torch.rand(where.numel(), 3, generator=g)
+    bx = torch.arange(2).repeat_interleave(torch.tensor([5000, x.shape[0] - 5000]))
+    q = torch.arange(0, x.shape[0], 7)
+    y, by = (x[q] + 0.3 * torch.rand(q.numel(), 3, generator=g)).contiguous(), bx[q].contiguous()
+    idx, dist = tpk.ball_query(0.35, 20, x.to(dev), y.to(dev), mode="partial_dense", batch_x=bx.to(dev), batch_y=by.to(dev), sort=sort)
+    if sort:
+        wi, wd = oracle.ball_query_sorted_partial(0.35, 20, x.numpy(), y.numpy(), bx.numpy(), by.numpy())
+    else:
+        wi, wd = oracle.ball_query_partial_dense(0.35, 20, x.numpy(), y.numpy(), bx.numpy(), by.numpy())
+    np.testing.assert_array_equal(_np(idx), wi)
+    np.testing.assert_array_equal(_np(dist), wd)
+
+
 # ------------------------------------------------------------------ grouping
 
 

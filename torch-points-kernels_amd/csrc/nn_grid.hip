@@ -756,6 +756,13 @@ constexpr int BQB_HITS = TPK_WAVE; // hits a wavefront collects before it falls 
 constexpr int BQB_DENSE_MIN_POINTS = 8192; // dense layout: clouds above this take the bin walk (smaller ones fit in LDS whole)
 constexpr int64_t BQB_DENSE_MIN_PAIRS = 40000000; // ... when the call has at least this many (query, point) pairs
 
+// Points per touched bin from which the bins are walked one after the other: a step of 64 candidates of one bin needs a
+// third of the instructions of a step of 64 from all of them (which has to find out whose each candidate is), but a
+// bin's last step is only partly filled.  300000 queries of 24 clouds (12500 points, bins of about 100): 294 us mixed,
+// 266 one after the other from 48 points on, 277 from 32, 290 from 16 (the prefix sums' new last steps: 254).  Scenes
+// with 4 points a bin: no difference.
+constexpr int BQB_LONG_BIN = 48;
+
 // Range of 16^3-grid cells along one axis that [v - r, v + r] can touch.  The interval is widened
 // by a few ulps of its ends so that a point the fp32 radius test accepts is never left out.
 __device__ __forceinline__ void bin_range(float v, float r, float lo, float scale, int& first, int& last)
@@ -854,15 +861,17 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
         auto walk_pairs = [&](int pair0) __attribute__((always_inline)) {
             // one descriptor per pair, written by the window's lane: a window's block holds a few bins, so a loop
             // is cheaper here than the marks used for the candidates below (64.6 against 62 us on 58750 queries)
-            // (volatile: what a lane reads back was written by other lanes)
-            volatile int* const marks = slots;
+            // (What a lane reads back was written by other lanes: fences for the compiler, no instructions.  Accesses
+            // through a volatile pointer were flat ones that wait for all memory: 300000 queries of 24 clouds 275 us
+            // for the whole call, 264 without.)
             for (int i = max(0, pair0 - pairs_before); i < nbins && pairs_before + i < pair0 + TPK_WAVE; ++i)
-                marks[pairs_before + i - pair0] = block | (i << 20);
+                slots[pairs_before + i - pair0] = block | (i << 20);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             // lane p: where the points of pair pair0 + p start in the ordered array, and how many
             int start = 0, size = 0;
             if (pair0 + lane < pairs)
             {
-                const int d = marks[lane];
+                const int d = slots[lane];
                 const int i = (d >> 20) & 63, window = (d >> 26) & 63;
                 const int fx = d & 15, fy = (d >> 4) & 15, fz = (d >> 8) & 15;
                 const int nx = ((d >> 12) & 15) + 1, ny = ((d >> 16) & 15) + 1;
@@ -881,31 +890,20 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
             }
             const int before = wave_exclusive_sum(size);
             const int total = __builtin_amdgcn_readlane(before + size, TPK_WAVE - 1);
-            const int origin = start - before; // candidate c of this walk lies at origin + c, for the c of this lane's pair
-            for (int c0 = 0; c0 < total && !serial; c0 += TPK_WAVE)
-            {
-                // Which pair does candidate c0 + lane belong to?  Every pair's lane marks the slot of its first
-                // candidate in this step with its own number; a running maximum over the slots carries the
-                // number on to the pair's other candidates.
-                marks[lane] = 0;
-                if (size > 0 && before < c0 + TPK_WAVE && before + size > c0)
-                    marks[max(before - c0, 0)] = lane;
-                const int mark = marks[lane];
-                const bool has = c0 + lane < total;
-                const int at_x = __shfl(origin, wave_inclusive_max_i32(mark)) + c0 + lane;
-                const float4 p = sorted_x[has ? at_x : 0];
+            // one candidate per lane (of those that have one)
+            auto test = [&](const float4 p, bool has) __attribute__((always_inline)) {
                 const float d = tpk_dist2(qx, qy, qz, p.x, p.y, p.z);
                 TPK_WORK_ADD(1);
                 const int row = __float_as_int(p.w);
                 if constexpr (SORTED)
                 {
                     offer(has && d < radius2 && row >= s0 && row < s1, d, row);
-                    continue;
+                    return;
                 }
                 const bool hit = has && (DENSE ? d < radius2 : d <= radius2) && row >= s0 && row < s1;
                 const unsigned long long mask = __ballot(hit);
                 if (mask == 0)
-                    continue;
+                    return;
                 const int at = cnt + static_cast<int>(tpk_prefix_count(mask));
                 if (hit && at < BQB_HITS)
                 {
@@ -914,6 +912,57 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
                 }
                 cnt += __builtin_popcountll(mask);
                 serial = cnt > BQB_HITS;
+            };
+            unsigned long long live = __ballot(size > 0);
+            if (total >= BQB_LONG_BIN * __builtin_popcountll(live) && total > 0)
+            {
+                // Long bins: one after the other, 64 points per step, the points of a step requested a step ahead.
+                int at = 0, end = 0; // (wave-uniform: what is left of the bin at hand)
+                auto next_step = [&]() __attribute__((always_inline)) {
+                    at += TPK_WAVE;
+                    if (at < end)
+                        return true;
+                    if (live == 0)
+                        return false;
+                    const int pair = __builtin_ctzll(live);
+                    live &= live - 1;
+                    at = __builtin_amdgcn_readlane(start, pair);
+                    end = at + __builtin_amdgcn_readlane(size, pair);
+                    return true;
+                };
+                bool more = next_step();
+                float4 ahead = sorted_x[min(at + lane, end - 1)];
+                bool ahead_has = at + lane < end;
+                while (more && !serial)
+                {
+                    const float4 p = ahead;
+                    const bool has = ahead_has;
+                    more = next_step();
+                    if (more)
+                    {
+                        ahead = sorted_x[min(at + lane, end - 1)];
+                        ahead_has = at + lane < end;
+                    }
+                    test(p, has);
+                }
+                return;
+            }
+            const int origin = start - before; // candidate c of this walk lies at origin + c, for the c of this lane's pair
+            for (int c0 = 0; c0 < total && !serial; c0 += TPK_WAVE)
+            {
+                // Which pair does candidate c0 + lane belong to?  Every pair's lane marks the slot of its first
+                // candidate in this step with its own number; a running maximum over the slots carries the
+                // number on to the pair's other candidates.
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                slots[lane] = 0;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (size > 0 && before < c0 + TPK_WAVE && before + size > c0)
+                    slots[max(before - c0, 0)] = lane;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const int mark = slots[lane];
+                const bool has = c0 + lane < total;
+                const int at_x = __builtin_amdgcn_ds_bpermute(wave_inclusive_max_i32(mark) * 4, origin) + c0 + lane;
+                test(sorted_x[has ? at_x : 0], has);
             }
         };
         if (!serial)

