@@ -208,6 +208,7 @@ constexpr int GB_STAGE_FLOATS = 32768; // at most this many of them hold the sta
 constexpr int GB_FETCH = GB_STAGE_FLOATS / 4 / G_THREADS; // 16-byte loads per lane that bring in a piece: 8
 constexpr int GB_AHEAD = 8;            // rows of list entries a wavefront has requested ahead of the one it adds
 constexpr int GB_HOLD = 36;            // rows of list entries a lane keeps in registers where a piece's entries are held
+constexpr int GB_BUSY_GRID = 128;      // workgroups below which a call takes fewer rows per workgroup
 // The walk that holds a piece's entries in registers: one row per pass, 4-byte entries.
 template <int K, bool WEIGHTED, int R>
 constexpr bool GB_HOLD_FOR = K == 1 && !WEIGHTED && R == 1;
@@ -860,9 +861,19 @@ int gather_bwd_from_lists(int b, int c, int m, int64_t n, const float* grad_out,
         return TPK_ERR_WORKSPACE;
     const Lists<WEIGHTED> lists =
         lists_at<WEIGHTED>(lists_memory, static_cast<int64_t>(b) * sh.parts, m, static_cast<int64_t>(sh.part_len) * K);
-    if (sh.rows == 4)
+    // Fewer rows together where a call would leave most compute units idle: a workgroup then stages and finishes less, and
+    // reads the lists as often as before on a compute unit of its own.  (The lists do not depend on the rows.)  Measured:
+    // 2 x 64 rows of 8192 columns 13.3 -> 10.3 us, 7 x 33 weighted rows of 5001 columns 20.6 -> 11.9, 1 x 128 of 16384
+    // 17.1 -> 15.6; a limit of 64 workgroups keeps the old time for the last and for 4 x 64 rows, 256 is the same as 128.
+    // One plain row alone holds its entries in registers, GB_HOLD requests however few they are: not below 4096 columns
+    // (256 columns: 8.1 us, and 9.1 that way).
+    const int fewest = GB_HOLD_FOR<K, WEIGHTED, 1> && n < 4096 ? 2 : 1;
+    int rows = sh.rows;
+    while (rows > fewest && static_cast<int64_t>(b) * tpk_ceil_div(c, rows) < GB_BUSY_GRID)
+        rows /= 2;
+    if (rows == 4)
         return launch_bwd_lists<K, WEIGHTED, 4>(b, c, m, n, sh, grad_out, lists, grad_src, s);
-    if (sh.rows == 2)
+    if (rows == 2)
         return launch_bwd_lists<K, WEIGHTED, 2>(b, c, m, n, sh, grad_out, lists, grad_src, s);
     return launch_bwd_lists<K, WEIGHTED, 1>(b, c, m, n, sh, grad_out, lists, grad_src, s);
 }
