@@ -1008,7 +1008,8 @@ def test_gather_full_grids(tpk, oracle, dev, columns):
 @pytest.mark.parametrize("columns", [1, 255, 4095, 4096, 4097, 8192])
 @pytest.mark.parametrize("B,C", [(1, 1), (2, 31), (2, 64), (8, 62), (8, 64)])
 def test_gather_grad_rows_together(tpk, oracle, dev, B, C, columns):
-    # one, two or four rows of grad_out are walked together: calls around the grids where the number changes
+    # one, two or four rows of grad_out are walked together, and two, four or eight rows interpolated by a workgroup:
+    # calls around the grids where the numbers change
     g = torch.Generator().manual_seed(columns + C)
     feats = torch.randn(B, C, 50, generator=g)
     idx = torch.randint(0, 50, (B, columns, 1), generator=g)
@@ -1019,7 +1020,9 @@ def test_gather_grad_rows_together(tpk, oracle, dev, B, C, columns):
     _assert_scatter_sum_close(_np(f.grad), want, oracle.grouping_operation_grad(gout.abs().numpy(), idx.numpy(), 50))
     feats, idx, w, gout = _interp_case(B, C, 50, columns, columns)
     f = feats.to(dev).requires_grad_(True)
-    tpk.three_interpolate(f, idx.to(dev), w.to(dev)).backward(gout.to(dev))
+    out = tpk.three_interpolate(f, idx.to(dev), w.to(dev))
+    np.testing.assert_array_equal(_np(out), oracle.three_interpolate(feats.numpy(), idx.numpy(), w.numpy()))
+    out.backward(gout.to(dev))
     want = oracle.three_interpolate_grad(gout.numpy(), idx.numpy(), w.numpy(), 50)
     _assert_scatter_sum_close(_np(f.grad), want, oracle.three_interpolate_grad(gout.abs().numpy(), idx.numpy(), w.numpy(), 50))
 

@@ -38,6 +38,7 @@ namespace {
 constexpr int G_MAX_ROWS = 8;
 constexpr int G_LDS_BUDGET = 131072; // bytes of LDS for the staged rows
 constexpr unsigned G_FULL_GRID = 256;  // a workgroup for every compute unit
+constexpr int G_BUSY_GRID = 192;       // workgroups below which the weighted gather takes fewer rows per workgroup
 constexpr int G_PLAIN_BLOCKS = 1024; // workgroups the plain gather aims at (four per compute unit, two at a time)
 
 template <int K, bool WEIGHTED, typename IdxT>
@@ -710,6 +711,15 @@ int gather_fwd(int b, int c, int m, int64_t n, const float* src, const IdxT* idx
     if (!src || !idx || !out || (WEIGHTED && !weight))
         return TPK_ERR_INVALID_ARG;
     int r = rows_for(m, c);
+    // parts of a row's columns, each at least as long as a row, so that staging a row block stays the smaller share
+    const int64_t whole_parts = n / (m > G_THREADS ? m : G_THREADS), max_split = whole_parts < 1 ? 1 : whole_parts;
+    // The weighted gather, where it would leave compute units idle: fewer rows per workgroup, down to two.  Measured:
+    // 1 cloud, 128 rows of 16384 columns from 4096 points 15.9 -> 10.6 us, 2 x 32 rows of 8192 from 2048 10.8 -> 7.9,
+    // 7 x 33 of 5001 from 1250 9.7 -> 8.5 (a second step, from 252 workgroups to 357: 9.9; 3 x 77 of 9000 from 600, from
+    // 240 to 300: 9.2 -> 10.3).
+    if (WEIGHTED)
+        while (r > 2 && static_cast<int64_t>(b) * tpk_ceil_div(c, r) * max_split < G_BUSY_GRID)
+            r = (r + 1) / 2;
     // The plain gather is bound by its stores and gains from two workgroups per compute unit that stage and store
     // at different times, and from row blocks that are not split by columns (every split stages the rows again):
     // fewer rows per workgroup while that gives more workgroups, down to two rows (with one row the indices, read
@@ -721,10 +731,8 @@ int gather_fwd(int b, int c, int m, int64_t n, const float* src, const IdxT* idx
     if (r > 0)
     {
         const int row_blocks = static_cast<int>(tpk_ceil_div(c, r));
-        // Split the columns so that a few hundred workgroups exist, but keep each part at
-        // least as long as a row (so staging a row block stays the smaller share of traffic).
+        // Split the columns so that a few hundred workgroups exist.
         int64_t jsplit = tpk_ceil_div(WEIGHTED ? 256 : G_PLAIN_BLOCKS, static_cast<int64_t>(row_blocks) * b);
-        const int64_t max_split = n / (m > G_THREADS ? m : G_THREADS);
         if (jsplit > max_split)
             jsplit = max_split;
         if (jsplit < 1)
