@@ -34,6 +34,16 @@ def test_header_declares_the_expected_entry_points():
         assert want in names
 
 
+def test_knn_grid_workspace_is_its_own_size():
+    """The grid in memory has a size function of its own: what tpk_knn_workspace_bytes() says stays the curve search's."""
+    lib = ctypes.CDLL(LIB)
+    size = lib.tpk_knn_grid_workspace_bytes
+    size.restype = ctypes.c_size_t
+    assert size(0, 1000, 1000) == 0 and size(2, 0, 1000) == 0 and size(2, 1000, 0) == 0
+    assert size(1, 8192, 16384) == 0  # few queries of a cloud that fits in LDS
+    assert size(1, 8192, 16385) >= 8192 * 16 and size(2, 200000, 1000) >= 2 * 200000 * 16
+
+
 def test_counting_build_exports_the_same_abi_plus_its_reader():
     """libtpk_hip_counting.so (measurement only) carries the whole C ABI and tpk_work_read_reset; the
     shipping library carries no counter."""

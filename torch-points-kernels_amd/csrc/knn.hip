@@ -604,10 +604,16 @@ int nearest_within(int b, int n_support, int m_query, int k, float limit, const 
 
 } // namespace
 
+// (a list per lane over curve-ordered cells)
 extern "C" size_t tpk_knn_workspace_bytes(int b, int n_support, int m_query)
 {
-    // (a list per lane; a wavefront per query)
-    return m_query > 0 ? std::max(tpk_grid_knn_workspace_bytes(b, m_query, n_support), knn_grid_workspace_bytes(b, n_support, m_query)) : 0;
+    return tpk_grid_knn_workspace_bytes(b, m_query, n_support);
+}
+
+// (a wavefront per query over a grid in memory)
+extern "C" size_t tpk_knn_grid_workspace_bytes(int b, int n_support, int m_query)
+{
+    return n_support > 0 ? knn_grid_workspace_bytes(b, n_support, m_query) : 0;
 }
 
 extern "C" int tpk_knn_f32(int b, int n_support, int m_query, int k, const float* support,
@@ -622,9 +628,10 @@ extern "C" int tpk_knn_f32(int b, int n_support, int m_query, int k, const float
         return TPK_ERR_INVALID_ARG;
     if (static_cast<int64_t>(n_support) * 3 > 0x7fffffffLL || static_cast<int64_t>(m_query) * 3 > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    if (k <= KNC_MAX_K && knn_in_lds(b, n_support, m_query, workspace != nullptr))
+    const bool grid = workspace && workspace_bytes >= knn_grid_workspace_bytes(b, n_support, m_query);
+    if (k <= KNC_MAX_K && knn_in_lds(b, n_support, m_query, grid))
         return launch_knn_cells(b, m_query, n_support, k, query, support, dist2, idx, tpk_stream(stream));
-    if (k <= KNC_MAX_K && workspace)
+    if (k <= KNC_MAX_K && grid)
         return launch_knn_grid(b, m_query, n_support, k, query, support, dist2, idx, workspace, workspace_bytes, tpk_stream(stream));
     return nearest_within(b, n_support, m_query, k, __builtin_inff(), support, query, idx, dist2, workspace,
                           workspace_bytes, tpk_stream(stream));

@@ -160,7 +160,7 @@ std::pair<at::Tensor, at::Tensor> dense_knn(at::Tensor support, at::Tensor query
     const int b = as_int(query.size(0), "batch size");
     const int n = as_int(support.size(1), "number of support points");
     const int m = as_int(query.size(1), "number of query points");
-    const size_t ws_bytes = tpk_knn_workspace_bytes(b, n, m);
+    const size_t ws_bytes = std::max(tpk_knn_workspace_bytes(b, n, m), tpk_knn_grid_workspace_bytes(b, n, m));
     at::Tensor ws;
     if (ws_bytes)
         ws = torch::empty({static_cast<int64_t>(ws_bytes)}, query.options().dtype(torch::kUInt8));
