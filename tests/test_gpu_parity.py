@@ -957,6 +957,32 @@ def test_ball_query_packed_long_bins(tpk, oracle, dev, rest, sort):
     np.testing.assert_array_equal(_np(dist), wd)
 
 
+@pytest.mark.parametrize("record", [True, False])
+def test_forward_mode_is_refused(tpk, dev, record):
+    # no operator has a forward mode: a tangent is an error, not a result without one
+    import torch.autograd.forward_ad as fw
+
+    def dual(t):
+        return fw.make_dual(t.to(dev), torch.ones_like(t).to(dev))
+
+    pts = torch.rand(2, 40, 3) - 0.5
+    feats, idx, w, _ = _interp_case(2, 3, 20, 30, 0)
+    calls = [
+        lambda: tpk.three_interpolate(dual(feats), idx.to(dev), w.to(dev)),
+        lambda: tpk.three_interpolate(feats.to(dev), idx.to(dev), dual(w)),
+        lambda: tpk.grouping_operation(dual(feats), idx.long().to(dev)),
+        lambda: tpk.chamfer_dist.chamfer_dist(dual(pts), pts.to(dev)),
+        lambda: tpk.chamfer_dist.chamfer_dist(pts.to(dev), dual(pts)),
+        lambda: tpk.gridding(dual(pts), 4),
+        lambda: tpk.cubic_feature_sampling(dual(pts), torch.rand(2, 3, 4, 4, 4).to(dev)),
+        lambda: tpk.cubic_feature_sampling(pts.to(dev), dual(torch.rand(2, 3, 4, 4, 4))),
+    ]
+    with fw.dual_level(), torch.set_grad_enabled(record):
+        for call in calls:
+            with pytest.raises(RuntimeError):
+                call()
+
+
 # ------------------------------------------------------------------ grouping
 
 

@@ -5,9 +5,11 @@
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
+// Whether a call has to go through its node.  (With a forward-mode tangent too, whether or not gradients are recorded:
+// none of the nodes has a forward mode, and the node says so, where the kernels alone would lose the tangent in silence.)
 inline bool records(const at::Tensor& t)
 {
-    return at::GradMode::is_enabled() && t.requires_grad();
+    return (at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(/*level=*/0).defined();
 }
 
 struct GriddingBatch : torch::autograd::Function<GriddingBatch>
