@@ -957,6 +957,25 @@ def test_ball_query_packed_long_bins(tpk, oracle, dev, rest, sort):
     np.testing.assert_array_equal(_np(dist), wd)
 
 
+@pytest.mark.parametrize("name", ["interpolate", "group", "chamfer", "gridding", "cubic"])
+def test_traces_follow_their_inputs(tpk, dev, name):
+    # a trace made with one input computes with the next one's values, as a call does
+    g = torch.Generator().manual_seed(3)
+    r = lambda *shape: torch.rand(*shape, generator=g).to(dev)
+    idx = torch.randint(0, 20, (2, 2, 30, 3), generator=g).to(dev)
+    op, inputs = {
+        "interpolate": (lambda f, i, w: tpk.three_interpolate(f, i.int(), w), (r(2, 2, 4, 20), idx, r(2, 2, 30, 3))),
+        "group": (tpk.grouping_operation, (r(2, 2, 4, 20), idx)),
+        "chamfer": (tpk.chamfer_dist.chamfer_dist, (r(2, 2, 40, 3), r(2, 2, 50, 3))),
+        "gridding": (lambda p: tpk.gridding(p, 4), (r(2, 2, 40, 3) - 0.5,)),
+        "cubic": (lambda p, m: tpk.cubic_feature_sampling(p, m), (r(2, 2, 40, 3) - 0.5, r(2, 2, 3, 4, 4, 4))),
+    }[name]
+    traced = torch.jit.trace(op, tuple(v[0] for v in inputs), check_trace=False)
+    got, want = traced(*(v[1] for v in inputs)), op(*(v[1] for v in inputs))
+    # (sums of at most 320 terms in another order: 320 * 2^-24 of their size)
+    torch.testing.assert_close(got, want, rtol=2e-5, atol=2e-5 * float(want.abs().max()))
+
+
 @pytest.mark.parametrize("record", [True, False])
 def test_forward_mode_is_refused(tpk, dev, record):
     # no operator has a forward mode: a tangent is an error, not a result without one

@@ -75,7 +75,7 @@ class ThreeInterpolate(Function):
 def three_interpolate(features, idx, weight):
     r"""features (B, c, m), idx (B, n, 3) (int32 on the GPU, int64 on the CPU: what three_nn returns there),
     weight (B, n, 3) -> (B, c, n) (reference: torchpoints.py:109-126)."""
-    if features.is_cuda:
+    if features.is_cuda and not torch.jit.is_tracing():  # (a trace records the Python function, not the native call)
         return native().interpolate_features(features, idx, weight)
     return ThreeInterpolate.apply(features, idx, weight)
 
@@ -109,6 +109,8 @@ def grouping_operation(features, idx):
     (reference: torchpoints.py:129-146).  float32 tensors on the GPU take the native kernels; every other
     device and dtype is served, as in the reference, by torch's own gather (and its autograd)."""
     if features.is_cuda and features.dtype == torch.float32 and idx.dtype == torch.int64:
+        if torch.jit.is_tracing():
+            return GroupingOperation.apply(features, idx)
         return native().group_features(features, idx)
     b, c = features.shape[0], features.shape[1]
     columns = idx.reshape(b, 1, -1).expand(b, c, -1)
