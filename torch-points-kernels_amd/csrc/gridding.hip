@@ -2,9 +2,9 @@
 // gradient) and cubic feature sampling (features of the grid vertices around a point, and its
 // gradient).  Reference: cuda/src/gridding_gpu.cu:29-331, cuda/src/cubic_feature_sampling_gpu.cu:
 // 23-210.  The reference runs one block per cloud; here every launch spreads over all points
-// (or output elements) of all clouds.  Sums into the grid are float / double atomics in no fixed
-// order, as in the reference; the gridding gradient of a point is one thread's sum in the
-// reference's order, so it is reproduced bit for bit.
+// (or output elements) of all clouds.  Sums into the grid are formed in no fixed order, as in the
+// reference (float / double atomics in memory or, for a batch, in LDS); the gridding gradient of a
+// point is one thread's sum in the reference's order, so it is reproduced bit for bit.
 //
 // Gridding comes in two forms over the same arithmetic: the reference's native pair, which takes
 // coordinates in grid units and hands the factors of every (point, vertex) from the forward to the

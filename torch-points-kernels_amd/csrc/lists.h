@@ -62,7 +62,11 @@ static_assert(static_cast<uint32_t>(L_NOTHING) * 1u >= TPK_LDS_BYTES && static_c
 constexpr int L_SPANS = G_THREADS / TPK_WAVE; // spans of targets per cloud: one per wavefront of the walker
 constexpr int L_MAX_SPAN = 15360;             // targets of a span: their bookkeeping (2 ints each) fits in LDS
 constexpr int L_REGION_GAP = 128;             // entry slots between the regions of consecutive spans
-constexpr int L_CACHED = 48;                  // index values a thread keeps in registers between the two passes
+// Index values a thread keeps in registers between the two passes: all of the longest part that is walked whole (32768
+// columns of one entry, or 16384 of three).  (48 for both spilled with 64-bit indices: 16 clouds of 32768 entries 18.1 us,
+// 17.6 with 32.)
+template <int K>
+constexpr int L_CACHED = K == 1 ? 32 : 48;
 constexpr int L_QUEUE = 128;                  // places of a wavefront's queue of entries inside the span (a power of two >= 128)
 
 template <bool WEIGHTED>
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED
     __syncthreads();
 
     // First pass.  Entry e of the part is read by thread e % G_THREADS in its round e / G_THREADS.
-    int cached[L_CACHED];
+    int cached[L_CACHED<K>];
     int below = 0; // valid entries whose target lies before this span
     auto count_one = [&](int v) {
         below += (v >= 0 && v < i0) ? 1 : 0;
@@ -173,9 +177,9 @@ __global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED
         return (e < total && v >= 0 && v < m) ? static_cast<int>(v) : -1;
     };
     constexpr int BATCH = 16; // index loads in flight per thread
-    static_assert(L_CACHED % BATCH == 0, "the cached rounds are whole batches");
+    static_assert(L_CACHED<K> % BATCH == 0, "the cached rounds are whole batches");
 #pragma unroll
-    for (int b = 0; b < L_CACHED; b += BATCH)
+    for (int b = 0; b < L_CACHED<K>; b += BATCH)
     {
         if (b * G_THREADS < total) // (wave-uniform)
         {
@@ -193,7 +197,7 @@ __global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED
                 cached[b + u] = -1;
         }
     }
-    for (int e0 = L_CACHED * G_THREADS + tid; e0 < total; e0 += BATCH * G_THREADS)
+    for (int e0 = L_CACHED<K> * G_THREADS + tid; e0 < total; e0 += BATCH * G_THREADS)
     {
         int iv[BATCH];
 #pragma unroll
@@ -325,7 +329,7 @@ __global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED
             place_queued(TPK_WAVE);
     };
 #pragma unroll
-    for (int b = 0; b < L_CACHED; b += BATCH)
+    for (int b = 0; b < L_CACHED<K>; b += BATCH)
         if (b * G_THREADS < total) // (wave-uniform)
         {
 #pragma unroll
@@ -333,7 +337,7 @@ __global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED
                 enqueue((b + u) * G_THREADS + tid, cached[b + u]);
         }
     // (the rounds behind the cached ones; the trip count is the same for every lane of a wavefront)
-    for (int e0 = L_CACHED * G_THREADS + tid; e0 - tid < total; e0 += BATCH * G_THREADS)
+    for (int e0 = L_CACHED<K> * G_THREADS + tid; e0 - tid < total; e0 += BATCH * G_THREADS)
     {
         int iv[BATCH];
 #pragma unroll
