@@ -719,7 +719,7 @@ def test_three_nn_cell_search_ties(tpk, oracle, dev):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
-@pytest.mark.parametrize("kind", ["uniform", "clusters", "flat", "one_point", "outlier", "queries_outside", "non_finite", "line",
+@pytest.mark.parametrize("kind", ["uniform", "clusters", "flat", "one_point", "outlier", "overflow", "queries_outside", "non_finite", "line",
                                   "lattice", "tripled", "offset_1e5", "two_points"])
 @pytest.mark.parametrize("B,n,m", [(2, 700, 1024), (1, 5000, 4096), (3, 300, 8192), (300, 40, 1500), (1, 2100, 3000)])
 def test_three_nn_grid_in_lds(tpk, oracle, dev, kind, B, n, m):
@@ -740,6 +740,9 @@ def test_three_nn_grid_in_lds(tpk, oracle, dev, kind, B, n, m):
         known[:] = 0.5
     elif kind == "outlier":
         known[:, m // 3] = torch.tensor([400.0, -300.0, 1e6])
+    elif kind == "overflow":  # finite coordinates whose range is not, on every axis
+        known[:, m // 3] = 2e38
+        known[:, m // 2] = -2e38
     elif kind == "queries_outside":
         unknown[:, ::3] += 5.0
         unknown[:, 1::3, 1] = -40.0
@@ -1108,7 +1111,7 @@ def test_knn_parity(tpk, oracle, dev, B, n, m, k):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
-@pytest.mark.parametrize("kind", ["uniform", "clusters", "flat", "one_point", "lattice", "outlier", "queries_outside", "non_finite"])
+@pytest.mark.parametrize("kind", ["uniform", "clusters", "flat", "one_point", "lattice", "outlier", "overflow", "queries_outside", "non_finite"])
 @pytest.mark.parametrize("B,n,m,k", [(2, 1, 3, 1), (2, 65, 40, 48), (1, 3000, 150, 49), (1, 8192, 200, 17), (2, 8193, 90, 48), (1, 40000, 60, 4)])
 def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
     # up to 48 neighbours: a grid in LDS (up to 8192 points) or in memory, its block of cells grown until it holds k, the
@@ -1125,6 +1128,9 @@ def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
         support, query = (support * 12).round(), (query * 24).round() / 2
     elif kind == "outlier":
         support[:, n // 3] = torch.tensor([400.0, -300.0, 1e6])
+    elif kind == "overflow":  # finite coordinates whose range is not, on every axis
+        support[:, n // 3] = 2e38
+        support[:, n // 2] = -2e38
     elif kind == "queries_outside":
         query[:, ::2] += 5.0
         query[:, 1::2, 1] = -40.0

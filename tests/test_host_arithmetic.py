@@ -1,0 +1,82 @@
+"""Arithmetic the kernels share with the host (csrc headers without device code), compiled here with g++ and tried over
+inputs a GPU test cannot afford to get wrong: what it returns sizes LDS and workspaces."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "torch-points-kernels_amd", "csrc")
+
+SHIM = r"""
+#include "grid_shape.h"
+
+extern "C" void grid_of(const float* low, const float* high, int m, float per_cell, int axis, int most, float* extent, int* along)
+{
+    float e[3];
+    for (int a = 0; a < 3; ++a)
+        extent[a] = e[a] = grid_extent(low[a], high[a]);
+    const GridCounts counts = grid_counts(e, m, per_cell, axis, most, [](auto f) {
+        int fitting = 0;
+        for (int lane = 0; lane < 64; ++lane)
+            fitting += f(lane) ? 1 : 0;
+        return fitting;
+    });
+    for (int a = 0; a < 3; ++a)
+        along[a] = counts.along[a];
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("shim")
+    source, library = str(folder / "shim.cpp"), str(folder / "shim.so")
+    with open(source, "w") as f:
+        f.write(SHIM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-Wall", "-Werror", "-shared", "-fPIC", "-I" + CSRC, source, "-o", library],
+                   check=True)
+    return ctypes.CDLL(library)
+
+
+def _grid(shim, low, high, m, per_cell, axis, most):
+    low, high = (np.asarray(v, np.float32) for v in (low, high))
+    extent, along = np.zeros(3, np.float32), np.zeros(3, np.int32)
+    pointer = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    shim.grid_of(pointer(low), pointer(high), m, ctypes.c_float(per_cell), axis, most, pointer(extent), pointer(along))
+    return extent, along
+
+
+# (the grid in LDS: 64 cells per axis, 4096 in all; the one in memory: 128 and 32768)
+@pytest.mark.parametrize("axis,most", [(64, 4096), (128, 32768)])
+@pytest.mark.parametrize("m,per_cell", [(1, 2.0), (7, 1.0), (8192, 1.0), (8192, 3.2), (16384, 9.6), (1 << 24, 1.0)])
+def test_a_grid_has_no_more_cells_than_there_is_room(shim, axis, most, m, per_cell):
+    inf = float("inf")
+    sides = (0.0, 1e-45, 1e-38, 1e-20, 1e-7, 1.0, 2.0 ** 40, 1.7e38, 2e38, 3.4028235e38)
+    spans = [(-a, b) for a in sides for b in (0.0, 1.0, 2e38, 3.4028235e38)] + [(a, a) for a in sides]
+    # a cloud without a finite coordinate on an axis: the box of nothing
+    spans += [(inf, -inf)]
+    for x in spans:
+        for y in spans[:: 3] + [x]:
+            for z in (x, y, (0.0, 1.0), (-2e38, 2e38)):
+                low, high = zip(x, y, z)
+                extent, along = _grid(shim, low, high, m, per_cell, axis, most)
+                assert (along >= 1).all() and (along <= axis).all(), (low, high, along)
+                assert int(along.astype(np.int64).prod()) <= most, (low, high, along)
+                assert np.isfinite(extent).all()
+                assert np.isfinite(along[extent > 0] / extent[extent > 0]).all(), (low, high, along)
+                assert (along[extent == 0] == 1).all()
+
+
+def test_a_grid_follows_the_cloud(shim):
+    """An even cloud gets about per_cell points per cell, a flat one a flat grid, a scaled one the same grid."""
+    _, cube = _grid(shim, [0, 0, 0], [1, 1, 1], 8192, 2.0, 64, 4096)
+    assert list(cube) == [16, 16, 16]
+    for scale in (1e-12, 1e12, 1e37):
+        _, along = _grid(shim, [0, 0, 0], [scale] * 3, 8192, 2.0, 64, 4096)
+        assert list(along) == list(cube)
+    _, flat = _grid(shim, [0, 0, 5], [1, 2, 5], 4096, 2.0, 64, 4096)
+    assert flat[2] == 1 and flat[1] == 2 * flat[0] and 1800 <= flat.prod() <= 2048
+    _, thin = _grid(shim, [0, 0, 0], [1, 1e-3, 1e-3], 8192, 2.0, 64, 4096)
+    assert list(thin) == [64, 1, 1]

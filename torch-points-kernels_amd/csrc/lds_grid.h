@@ -17,6 +17,7 @@
 // per candidate (four arrays x, y, z, index: 2.5 us more per call on 16 clouds of 4096 points, 16384 queries each).
 #pragma once
 
+#include "grid_shape.h"
 #include "tpk_device.h"
 
 namespace {
@@ -94,48 +95,25 @@ __device__ __forceinline__ unsigned long long lg_key(float d, int i)
 // gets a flat grid).  box: ordered ints, min x, y, z then max x, y, z.  The lanes try 64 sizes at a time.
 __device__ __forceinline__ void lg_shape(const int* box, int m, float per_cell, int axis, int most, int lane, float* shape)
 {
-            float low[3], extent[3], longest = 0.0f;
-    #pragma unroll
-            for (int a = 0; a < 3; ++a)
-            {
-                low[a] = lg_unordered(box[a]);
-                extent[a] = lg_unordered(box[3 + a]) - low[a]; // (NaN or -inf for a cloud without finite coordinates)
-                extent[a] = extent[a] > 0.0f ? extent[a] : 0.0f;
-                longest = fmaxf(longest, extent[a]);
-            }
-            float share[3]; // of the longest axis
-    #pragma unroll
-            for (int a = 0; a < 3; ++a)
-                share[a] = longest > 0.0f ? extent[a] / longest : 0.0f;
-            // cells per axis for `along` cells along the longest axis, and their product
-            auto fit = [&](float along, int (&count)[3]) __attribute__((always_inline)) {
-                int all = 1;
-    #pragma unroll
-                for (int a = 0; a < 3; ++a)
-                {
-                    const float f = longest > 0.0f ? fminf(share[a] * along + 0.5f, static_cast<float>(axis)) : 1.0f;
-                    count[a] = f >= 1.0f ? static_cast<int>(f) : 1;
-                    all *= count[a];
-                }
-                return all;
-            };
-            // (the product grows with `along`: the largest of the sizes tried that stays within the cells wanted, in
-            // steps of 2 up to 128, then in steps of 1 / 32 inside the step found)
-            const int wanted = static_cast<int>(fminf(static_cast<float>(most), fmaxf(static_cast<float>(m) / per_cell, 1.0f)));
-            int count[3];
-            const int coarse = __builtin_popcountll(__ballot(fit(2.0f * static_cast<float>(lane + 1), count) <= wanted));
-            const int fine = __builtin_popcountll(__ballot(fit(2.0f * static_cast<float>(coarse) + static_cast<float>(lane + 1) * (1.0f / 32.0f), count) <= wanted));
-            fit(2.0f * static_cast<float>(coarse) + static_cast<float>(fine) * (1.0f / 32.0f), count);
-            if (lane < 3)
-            {
-                const float e = lane == 0 ? extent[0] : lane == 1 ? extent[1] : extent[2];
-                const float l = lane == 0 ? low[0] : lane == 1 ? low[1] : low[2];
-                const int k = lane == 0 ? count[0] : lane == 1 ? count[1] : count[2];
-                shape[lane] = e > 0.0f ? l : 0.0f;
-                shape[3 + lane] = e > 0.0f ? static_cast<float>(k) / e : 0.0f;
-                shape[6 + lane] = e / static_cast<float>(k);
-                shape[9 + lane] = __int_as_float(k);
-            }
+    float low[3], extent[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        low[a] = lg_unordered(box[a]);
+        extent[a] = grid_extent(low[a], lg_unordered(box[3 + a]));
+    }
+    const GridCounts counts = grid_counts(extent, m, per_cell, axis, most,
+                                          [lane](auto f) { return static_cast<int>(__builtin_popcountll(__ballot(f(lane)))); });
+    if (lane < 3)
+    {
+        const float e = lane == 0 ? extent[0] : lane == 1 ? extent[1] : extent[2];
+        const float l = lane == 0 ? low[0] : lane == 1 ? low[1] : low[2];
+        const int k = lane == 0 ? counts.along[0] : lane == 1 ? counts.along[1] : counts.along[2];
+        shape[lane] = e > 0.0f ? l : 0.0f;
+        shape[3 + lane] = e > 0.0f ? static_cast<float>(k) / e : 0.0f;
+        shape[6 + lane] = e / static_cast<float>(k);
+        shape[9 + lane] = __int_as_float(k);
+    }
 }
 
 struct LdsGrid
