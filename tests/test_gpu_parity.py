@@ -1491,8 +1491,10 @@ def test_cubic_feature_sampling_parity(tpk, oracle, dev, dtype, B, n, c, scale, 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 # turned maps: channels beyond a block of 64, odd ones, maps that do not fill their spans; many points on one vertex (lists
-# sorted in several rounds, runs that share a cell); a map of more spans than are worth looking through
-@pytest.mark.parametrize("B,n,c,scale,crowd", [(3, 900, 70, 12, 0), (4, 2500, 33, 8, 0), (1, 4100, 20, 7, 3900), (8, 700, 130, 16, 500), (1, 9000, 12, 26, 0)])
+# sorted in several rounds, runs that share a cell); maps of more spans than are worth looking through, summed in memory or,
+# with enough channels (of 26^3 in float32, of 21^3 in float64), in LDS
+@pytest.mark.parametrize("B,n,c,scale,crowd", [(3, 900, 70, 12, 0), (4, 2500, 33, 8, 0), (1, 4100, 20, 7, 3900), (8, 700, 130, 16, 500), (1, 9000, 12, 26, 0),
+                                               (2, 9000, 40, 26, 0), (2, 8500, 33, 21, 400)])
 def test_cubic_feature_sampling_spans(tpk, oracle, dev, dtype, B, n, c, scale, crowd):
     g = torch.Generator().manual_seed(n + c)
     p = (torch.rand(B, n, 3, generator=g, dtype=torch.float64) * 2.2 - 1.1).to(dtype)
@@ -1511,6 +1513,24 @@ def test_cubic_feature_sampling_spans(tpk, oracle, dev, dtype, B, n, c, scale, c
     unit = 2.0 ** (-23 if dtype == torch.float32 else -52)
     assert (np.abs(_np(gm) - wf) <= (4 + crowd / 16) * unit * size).all()
     assert torch.equal(torch.autograd.grad(out, maps, go.to(dev))[0].isnan(), torch.zeros_like(maps, dtype=torch.bool))
+
+
+def test_cubic_feature_sampling_grad_beyond_32_bits(tpk, dev):
+    """A cloud whose gradient takes 4 GiB: offsets into it need more than 32 bits, and two channels share a workgroup."""
+    native = __import__("torch_points_kernels._native", fromlist=["native"]).native()
+    n, nv, c, scale = 32768, 64, 512, 8
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    go = torch.randn(1, n, nv, c, generator=g, device=dev)
+    vertices = torch.randint(-1, scale ** 3, (1, n, nv), generator=g, device=dev, dtype=torch.int32)
+    got = native.cubic_feature_sampling_grad(scale, 2, go, vertices)[1].view(c, scale ** 3)
+    rows = torch.where(vertices < 0, scale ** 3, vertices).view(-1).long()
+    for c0 in range(0, c, 64):
+        terms = go[..., c0 : c0 + 64].reshape(-1, 64)
+        want = torch.zeros(scale ** 3 + 1, 64, dtype=torch.float64, device=dev).index_add_(0, rows, terms.double())[:-1].t()
+        size = torch.zeros(scale ** 3 + 1, 64, dtype=torch.float64, device=dev).index_add_(0, rows, terms.abs().double())[:-1].t()
+        # about 4096 terms a sum, each addition off by at most half a unit of the sum so far: four standard deviations
+        assert ((got[c0 : c0 + 64] - want).abs() <= 4 * 64 * 2.0 ** -24 * size).all()
 
 
 def test_cubic_feature_sampling_front_end_and_gradcheck(tpk, oracle, dev):

@@ -18,6 +18,9 @@
 // and contributes no gradient.
 #include "tpk_device.h"
 
+#include <algorithm>
+#include <cmath>
+
 namespace {
 
 constexpr int GR_THREADS = 256;
@@ -454,8 +457,8 @@ __global__ __launch_bounds__(GR_THREADS) void cubic_rows_kernel(int64_t total_ro
     }
 }
 
-// cuda/src/cubic_feature_sampling_gpu.cu:138-175, for maps of fewer cells than a workgroup below is worth
-// having and as the reference's scatter: one atomic per term, in no fixed order.
+// cuda/src/cubic_feature_sampling_gpu.cu:138-175 as the reference's scatter, one atomic per term, in no fixed order: what
+// neither of the two kernels below takes.
 template <typename T>
 __global__ __launch_bounds__(GR_THREADS) void cubic_scatter_kernel(
     int64_t total, int n_pts, int n_vertices, int channels, int64_t cub_scale,
@@ -471,6 +474,48 @@ __global__ __launch_bounds__(GR_THREADS) void cubic_scatter_kernel(
     const int vertex = grid_pt_indexes[pv];
     if (vertex >= 0 && vertex < cub_scale)
         atomicAdd(&grad_cubic_features[(cloud * channels + k) * cub_scale + vertex], grad_point_features[e]);
+}
+
+// The same sums in LDS: a workgroup owns `group` channels of one cloud's maps (group * scale^3 sums), walks all entries of
+// the cloud, adds its channels' terms with LDS atomics and writes the maps out in order.  Bound: the atomics, 1.3 ns of a
+// compute unit per term (3 clocks), where one in memory costs the chip 24 ps.
+constexpr int CS_THREADS = 1024;
+constexpr int64_t CS_BYTES = 128 * 1024; // sums per workgroup at most
+
+template <typename T>
+__global__ __launch_bounds__(CS_THREADS) void cubic_scatter_lds_kernel(
+    int n_pts, int n_vertices, int channels, int group, int64_t cub_scale, const T* __restrict__ grad_point_features,
+    const int* __restrict__ grid_pt_indexes, T* __restrict__ grad_cubic_features)
+{
+    extern __shared__ __align__(16) unsigned char cubic_lds[];
+    T* sums = reinterpret_cast<T*>(cubic_lds);
+    // the workgroups of one cloud read the same lines of the gradient (each its own channels): they
+    // are kept on one die, so that one L2 serves them
+    const int groups = (channels + group - 1) / group;
+    const int block = static_cast<int>(xcd_local_block(blockIdx.x, gridDim.x));
+    const int cloud = block / groups;
+    const int k0 = (block - cloud * groups) * group;
+    const int width = min(group, channels - k0);
+    const int64_t cells = static_cast<int64_t>(width) * cub_scale;
+    for (int64_t t = threadIdx.x; t < cells; t += CS_THREADS)
+        sums[t] = T(0);
+    __syncthreads();
+    const int64_t entries = static_cast<int64_t>(n_pts) * n_vertices;
+    const int* indexes = grid_pt_indexes + cloud * entries;
+    const T* grads = grad_point_features + cloud * entries * channels;
+    // consecutive threads take the channels of one entry, then the next entry
+    for (int64_t t = threadIdx.x; t < entries * width; t += CS_THREADS)
+    {
+        const int64_t entry = t / width;
+        const int k = static_cast<int>(t - entry * width);
+        const int vertex = indexes[entry];
+        if (vertex >= 0 && vertex < cub_scale)
+            atomicAdd(&sums[k * cub_scale + vertex], grads[entry * channels + k0 + k]);
+    }
+    __syncthreads();
+    T* out = grad_cubic_features + (static_cast<int64_t>(cloud) * channels + k0) * cub_scale;
+    for (int64_t t = threadIdx.x; t < cells; t += CS_THREADS)
+        out[t] = sums[t];
 }
 
 // The gradient of the maps as a gather.  A workgroup owns a span of cells of one cloud: it sorts the cloud's
@@ -902,6 +947,55 @@ int launch_spans(int b, int n_pts, int nv, int channels, int64_t cub, const T* g
     return tpk_launch_status();
 }
 
+// What the three ways to the gradient of the maps take, in ns beyond a launch (infinite: not possible or not considered).
+// Measured over 1 .. 32 clouds of 128 .. 16384 points, 4 .. 128 channels, 4^3 .. 32^3 cells, points spread over the map and over a
+// sphere (uneven spans): the way taken is the quicker one or within a tenth of it in 97 of 100 calls.
+struct CubicWays
+{
+    double spans, sums, atomics;
+    int64_t group; // channels whose sums a workgroup of cubic_scatter_lds_kernel holds
+};
+
+template <typename T>
+CubicWays cubic_ways(int b, int channels, int64_t entries, int64_t cub)
+{
+    CubicWays w{HUGE_VAL, HUGE_VAL, HUGE_VAL, 1};
+    const double terms = static_cast<double>(entries) * channels; // of a cloud
+    const double bytes = terms * sizeof(T);
+    int64_t spans = 1;
+    while (spans * CubicSpan<T>::CELLS < cub)
+        spans *= 2;
+    // Spans: every workgroup looks through all entries of its cloud (0.26 ns each) and adds its own rows (13 ns each), once per
+    // CB_CHANNELS channels; offsets into the gradient are 32 bits.
+    const bool addressable = bytes < 4294967296.0;
+    if (addressable)
+    {
+        const double rounds = std::max(1.0, static_cast<double>(b) * spans / TPK_COMPUTE_UNITS);
+        w.spans = rounds * tpk_ceil_div(channels, CB_CHANNELS) * (5500.0 + entries * (0.26 + 13.0 / spans));
+    }
+    // Sums in LDS: a workgroup takes a clock or so per sum and three per term; in float64, where the unit keeps up, what counts is
+    // whether the gradients of the clouds on a die stay in its 4 MiB of L2.
+    const int64_t fit = CS_BYTES / (cub * static_cast<int64_t>(sizeof(T)));
+    if (fit > 0)
+    {
+        // as many channels per workgroup as fit (the fewer workgroups share a line of the gradient, the
+        // less often it is read), but a workgroup for every compute unit
+        w.group = std::min<int64_t>(fit, channels);
+        while (w.group > 1 && b * tpk_ceil_div(channels, w.group) < TPK_COMPUTE_UNITS)
+            w.group = (w.group + 1) / 2;
+        const double rounds = static_cast<double>(tpk_ceil_div(b * tpk_ceil_div(channels, w.group), TPK_COMPUTE_UNITS));
+        const double term = sizeof(T) == 4 ? 1.3 : bytes * tpk_ceil_div(b, 8) > 4194304.0 ? 0.9 : 0.45;
+        w.sums = rounds * w.group * (entries * term + cub * 0.13);
+    }
+    // Atomics in memory, 22 ps of the chip each (25 to 45 where they queue up on few addresses): where a span's
+    // look is long and there are many spans.  (32 channels in float32: 8 x 16384 points, 32^3 cells 806 us, sums in LDS 193; 40^3
+    // 850, spans 301; 2 x 65536, 32^3 798, sums 766, spans 222; 4 channels, 8 x 16384, 32^3 107, sums 166; 8 channels
+    // 240, sums 187.)
+    if (!addressable || (spans > 64 && entries > 65536))
+        w.atomics = 0.022 * terms * b;
+    return w;
+}
+
 template <typename T>
 int cubic_bwd(int b, int n_pts, int channels, int scale, int neighborhood_size, const T* grad_point_features,
               const int32_t* grid_pt_indexes, T* grad_ptcloud, T* grad_cubic_features, hipStream_t s)
@@ -923,16 +1017,30 @@ int cubic_bwd(int b, int n_pts, int channels, int scale, int neighborhood_size, 
     const int64_t total = entries * b * channels;
     if (total > 0 && (!grad_point_features || !grid_pt_indexes))
         return TPK_ERR_INVALID_ARG;
-    // Every span of 256 cells looks through all entries of its cloud: worth it while those are not many times the
-    // span's own - up to 64 spans (maps of 25^3 cells) - or while a span's look is short.
-    const int64_t spans = tpk_ceil_div(cub, CubicSpan<T>::CELLS);
-    if (channels > 0 && total > 0 && entries * channels * static_cast<int64_t>(sizeof(T)) < (int64_t(1) << 32) && (spans <= 64 || entries <= 65536))
+    if (total > 0)
     {
-        if (channels > 32)
-            return launch_spans<T, 64>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
-        if (channels > 16)
-            return launch_spans<T, 32>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
-        return launch_spans<T, 16>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
+        const CubicWays ways = cubic_ways<T>(b, channels, entries, cub);
+        if (ways.spans <= ways.sums && ways.spans <= ways.atomics)
+        {
+            if (channels > 32)
+                return launch_spans<T, 64>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
+            if (channels > 16)
+                return launch_spans<T, 32>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
+            return launch_spans<T, 16>(b, n_pts, static_cast<int>(nv), channels, cub, grad_point_features, grid_pt_indexes, grad_cubic_features, s);
+        }
+        if (ways.sums <= ways.atomics)
+        {
+            const int64_t blocks = b * tpk_ceil_div(channels, ways.group);
+            if (blocks > 0x7fffffffLL)
+                return TPK_ERR_UNSUPPORTED;
+            const size_t lds = static_cast<size_t>(ways.group * cub) * sizeof(T);
+            const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(cubic_scatter_lds_kernel<T>), lds);
+            if (allowed != TPK_OK)
+                return allowed;
+            hipLaunchKernelGGL(cubic_scatter_lds_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(CS_THREADS), lds, s, n_pts,
+                               static_cast<int>(nv), channels, static_cast<int>(ways.group), cub, grad_point_features, grid_pt_indexes, grad_cubic_features);
+            return tpk_launch_status();
+        }
     }
     st = fill_zero<T>(static_cast<int64_t>(b) * channels * cub, grad_cubic_features, s);
     if (st != TPK_OK || total == 0)
