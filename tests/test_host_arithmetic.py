@@ -10,7 +10,9 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "torch-points-kernels_amd", "csrc")
 
 SHIM = r"""
+#include "bracket.h"
 #include "grid_shape.h"
+#include <cmath>
 
 extern "C" void grid_of(const float* low, const float* high, int m, float per_cell, int axis, int most, float* extent, int* along)
 {
@@ -25,6 +27,29 @@ extern "C" void grid_of(const float* low, const float* high, int m, float per_ce
     });
     for (int a = 0; a < 3; ++a)
         along[a] = counts.along[a];
+}
+
+// The guesses until between k and `most` of the distances lie within one; -1: none found.
+extern "C" int guesses(const float* distance, int count, int k, int most, float first)
+{
+    auto within = [&](float t) {
+        int in = 0;
+        for (int i = 0; i < count; ++i)
+            in += distance[i] <= t ? 1 : 0;
+        return in;
+    };
+    Bracket bracket;
+    float guess = first;
+    int in = within(guess), tries = 0;
+    for (; in < k || in > most; ++tries)
+    {
+        if (tries >= BRACKET_TRIES)
+            return -1;
+        const float estimate = guess * std::pow((k + (most - k) / 2) / std::fmax(static_cast<float>(in), 0.5f), 2.0f / 3.0f);
+        guess = bracket.next(guess, in < k, estimate, tries);
+        in = within(guess);
+    }
+    return tries;
 }
 """
 
@@ -80,3 +105,23 @@ def test_a_grid_follows_the_cloud(shim):
     assert flat[2] == 1 and flat[1] == 2 * flat[0] and 1800 <= flat.prod() <= 2048
     _, thin = _grid(shim, [0, 0, 0], [1, 1e-3, 1e-3], 8192, 2.0, 64, 4096)
     assert list(thin) == [64, 1, 1]
+
+
+# (a first guess of 0 comes from a cloud without volume, one of +inf from a cell beyond float32; a query at 300 cloud sizes sees
+# all points at about the same distance, far beyond the distance of neighbouring points)
+@pytest.mark.parametrize("first", [0.0, 1e-30, 1e-3, 1.0, 1e20, float("inf")])
+@pytest.mark.parametrize("offset,spread", [(0.0, 1.0), (0.0, 1e-30), (270000.0, 300.0), (3e37, 1e36), (0.0, 3e38)])
+@pytest.mark.parametrize("k", [1, 16, 40, 48])
+def test_a_selection_finds_a_distance(shim, first, offset, spread, k):
+    rng = np.random.default_rng(k)
+    for count in (65, 100, 144):
+        distance = np.unique((offset + spread * rng.random(count)).astype(np.float32))
+        rng.shuffle(distance)
+        most = min(k + 24, 64)
+        tries = shim.guesses(distance.ctypes.data_as(ctypes.c_void_p), len(distance), k, most, ctypes.c_float(first))
+        assert 0 <= tries <= 6 + 31, (count, tries)
+
+
+def test_a_selection_gives_up_on_equal_distances(shim):
+    distance = np.full(100, 0.5, np.float32)
+    assert shim.guesses(distance.ctypes.data_as(ctypes.c_void_p), 100, 16, 40, ctypes.c_float(1.0)) == -1

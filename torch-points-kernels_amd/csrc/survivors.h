@@ -1,6 +1,7 @@
 // The survivors of a k-nearest search by a wavefront (knn.hip).
 #pragma once
 
+#include "bracket.h"
 #include "topk.h"
 
 namespace {
@@ -58,7 +59,8 @@ struct Survivors
                       lane + TPK_WAVE < count ? __int_as_float(static_cast<int>(k1 >> 32)) : inf, d};
         const int most = min(k + KNC_SPARE, KNC_MOST);
         const float target = static_cast<float>(k + (most - k) / 2);
-        float lo = 0.0f, hi = __builtin_inff(), guess = reach; // (reach: all of them, or +inf before the first selection)
+        Bracket bracket;
+        float guess = reach; // (all of them, or +inf before the first selection)
         int in_guess = TPK_WAVE + count;
         if (reach == inf)
         {
@@ -67,17 +69,10 @@ struct Survivors
         }
         for (int tries = 0; in_guess < k || in_guess > most; ++tries)
         {
-            if (tries > 40)
+            if (tries >= BRACKET_TRIES)
                 return false;
-            if (in_guess < k)
-                lo = guess;
-            else
-                hi = guess;
-            // from the last guess; bisection of the bit patterns when that leaves the bracket, or after a few
-            float next = guess * volume_ratio(target * __builtin_amdgcn_rcpf(fmaxf(static_cast<float>(in_guess), 0.5f)));
-            if (!(next > lo && next < hi) || tries > 5)
-                next = __int_as_float((__float_as_int(lo) + __float_as_int(hi)) >> 1);
-            guess = tpk_read_lane(next, 0);
+            const float estimate = guess * volume_ratio(target * __builtin_amdgcn_rcpf(fmaxf(static_cast<float>(in_guess), 0.5f)));
+            guess = tpk_read_lane(bracket.next(guess, in_guess < k, estimate, tries), 0);
             in_guess = within(v, guess);
         }
         reach = guess;
