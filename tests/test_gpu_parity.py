@@ -1111,14 +1111,16 @@ def test_knn_parity(tpk, oracle, dev, B, n, m, k):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
-@pytest.mark.parametrize("kind", ["uniform", "clusters", "flat", "one_point", "lattice", "outlier", "overflow", "queries_outside", "non_finite"])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "clusters", "flat", "one_point", "lattice", "outlier", "overflow", "queries_outside", "non_finite"])
 @pytest.mark.parametrize("B,n,m,k", [(2, 1, 3, 1), (2, 65, 40, 48), (1, 3000, 150, 49), (1, 8192, 200, 17), (2, 8193, 90, 48), (1, 40000, 60, 4)])
 def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
     # up to 48 neighbours: a grid in LDS (up to 8192 points) or in memory, its block of cells grown until it holds k, the
     # cells of the ball around it, and merging where many distances are equal or too few are finite; 49: lists
     g = torch.Generator().manual_seed(n + k)
     support, query = torch.rand(B, n, 3, generator=g), torch.rand(B, m, 3, generator=g)
-    if kind == "clusters":
+    if kind == "normal":  # (queries whose block of cells grows beyond the rows of one step)
+        support, query = torch.randn(B, n, 3, generator=g), 1.5 * torch.randn(B, m, 3, generator=g)
+    elif kind == "clusters":
         support, query = _clustered(g, B, n), _clustered(g, B, m)
     elif kind == "flat":
         support[..., 1] = 0.25
@@ -2047,6 +2049,46 @@ def test_counting_build_counts_executed_pairs(oracle, dev):
     pruned = run(2, 4096, 2048, True)
     assert 2 * 4096 * 3 <= pruned < 2 * 4096 * 2048 // 2
     assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0 and count.value == 0
+
+
+@pytest.mark.parametrize("kind", ["uniform", "normal", "flat", "queries_far", "queries_around"])
+def test_knn_looks_at_few_points(oracle, dev, kind):
+    """The searches over a grid look at a small part of the cloud, also where the queries lie far outside or the points are
+    spread unevenly: 1 to 11 steps of 64 points per query on average, where a scan of the cloud takes 256 (in LDS 94)."""
+    import ctypes
+    import os
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip_counting.so"))
+    lib.tpk_knn_grid_workspace_bytes.restype = ctypes.c_size_t
+    count = ctypes.c_ulonglong(0)
+    g = torch.Generator().manual_seed(3)
+    for b, n, m, k in ((1, 16384, 17000, 16), (1, 16384, 17000, 4), (1, 6000, 1000, 16)):
+        support, query = torch.rand(b, n, 3, generator=g), torch.rand(b, m, 3, generator=g)
+        if kind == "normal":
+            support, query = torch.randn(b, n, 3, generator=g), torch.randn(b, m, 3, generator=g)
+        elif kind == "flat":
+            support[..., 2] *= 1e-3
+            query[..., 2] *= 1e-3
+        elif kind == "queries_far":
+            query += 300.0
+        elif kind == "queries_around":
+            query = query * 3 - 1
+        s, q = support.to(dev), query.to(dev)
+        dist2 = torch.empty(b, m, k, device=dev)
+        idx = torch.empty(b, m, k, dtype=torch.int64, device=dev)
+        nbytes = lib.tpk_knn_grid_workspace_bytes(b, n, m)
+        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
+        assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0
+        st = lib.tpk_knn_f32(b, n, m, k, ctypes.c_void_p(s.data_ptr()), ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(idx.data_ptr()),
+                             ctypes.c_void_p(dist2.data_ptr()), ctypes.c_void_p(ws.data_ptr()) if nbytes else None, ctypes.c_size_t(nbytes),
+                             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert st == 0
+        assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0
+        wi, wd = oracle.knn(support.numpy(), query[:, :300].contiguous().numpy(), k)
+        np.testing.assert_array_equal(_np(idx)[:, :300], wi)
+        steps = count.value / (64 * b * m)
+        assert steps < 20, (n, k, steps)
 
 
 def test_extension_rejects_bad_tensors(tpk, dev):

@@ -90,9 +90,9 @@ __device__ __forceinline__ unsigned long long lg_key(float d, int i)
     return (static_cast<unsigned long long>(static_cast<unsigned>(__float_as_int(d))) << 32) | static_cast<unsigned>(i);
 }
 
-// The grid's shape, by one wavefront: lo, 1 / width, width and number of cells along each axis (shape[0 .. 11]) for about
-// per_cell of m points per cell, cells as cubic as `axis` per axis (at most 128) and `most` in all allow (a flat cloud
-// gets a flat grid).  box: ordered ints, min x, y, z then max x, y, z.  The lanes try 64 sizes at a time.
+// The grid's shape, by one wavefront: lo, 1 / width, width and number of cells along each axis (shape[0 .. 11]) and the volume of a
+// cell (shape[12]; one of a flat cloud counts as wide as it is long) for about per_cell of m points per cell, cells as cubic as
+// `axis` per axis (at most 128) and `most` in all allow (a flat cloud gets a flat grid).  box: ordered ints, min x, y, z then max x, y, z.  The lanes try 64 sizes at a time.
 __device__ __forceinline__ void lg_shape(const int* box, int m, float per_cell, int axis, int most, int lane, float* shape)
 {
     float low[3], extent[3];
@@ -104,23 +104,29 @@ __device__ __forceinline__ void lg_shape(const int* box, int m, float per_cell, 
     }
     const GridCounts counts = grid_counts(extent, m, per_cell, axis, most,
                                           [lane](auto f) { return static_cast<int>(__builtin_popcountll(__ballot(f(lane)))); });
+    const float e = lane == 0 ? extent[0] : lane == 1 ? extent[1] : extent[2];
+    const float l = lane == 0 ? low[0] : lane == 1 ? low[1] : low[2];
+    const int k = lane == 0 ? counts.along[0] : lane == 1 ? counts.along[1] : counts.along[2];
+    const float width = e / static_cast<float>(k);
     if (lane < 3)
     {
-        const float e = lane == 0 ? extent[0] : lane == 1 ? extent[1] : extent[2];
-        const float l = lane == 0 ? low[0] : lane == 1 ? low[1] : low[2];
-        const int k = lane == 0 ? counts.along[0] : lane == 1 ? counts.along[1] : counts.along[2];
         shape[lane] = e > 0.0f ? l : 0.0f;
         shape[3 + lane] = e > 0.0f ? static_cast<float>(k) / e : 0.0f;
-        shape[6 + lane] = e / static_cast<float>(k);
+        shape[6 + lane] = width;
         shape[9 + lane] = __int_as_float(k);
     }
+    const float wx = tpk_read_lane(width, 0), wy = tpk_read_lane(width, 1), wz = tpk_read_lane(width, 2), longest = fmaxf(fmaxf(wx, wy), wz);
+    if (lane == 0)
+        shape[12] = (wx > 0.0f ? wx : longest) * (wy > 0.0f ? wy : longest) * (wz > 0.0f ? wz : longest);
 }
+
+constexpr int LG_SHAPE = 13; // floats of a shape
 
 struct LdsGrid
 {
     float4* points;      // [m] the points cell by cell: x, y, z, index
     int* starts;         // [LG_STARTS] first place of every cell, then the number of points
-    float lo[3], inv[3], width[3];
+    float lo[3], inv[3], width[3], volume;
     int cells[3];
     float crowd;         // points per cell as a point sees them (per_cell + 1 in a cloud of even density)
 };
@@ -134,7 +140,7 @@ __device__ __forceinline__ void lds_grid_build(LdsGrid& g, unsigned char* lds, c
     float4* const points = g.points = reinterpret_cast<float4*>(lds);
     int* const starts = g.starts = reinterpret_cast<int*>(points + m);
     __shared__ int box[6];      // ordered ints: min x, y, z then max x, y, z of the finite coordinates
-    __shared__ float shape[12]; // lo, inv, width, cells of the grid, from the first wavefront
+    __shared__ float shape[LG_SHAPE]; // from the first wavefront
     __shared__ int wave_totals[LG_WAVES];
     __shared__ int crowding; // sum over the cells of count^2
     const int tid = threadIdx.x;
@@ -249,6 +255,7 @@ __device__ __forceinline__ void lds_grid_build(LdsGrid& g, unsigned char* lds, c
         }
     __syncthreads();
     g.crowd = static_cast<float>(crowding) / static_cast<float>(m);
+    g.volume = shape[12];
 #pragma unroll
     for (int a = 0; a < 3; ++a)
     {
