@@ -1111,7 +1111,7 @@ def test_knn_parity(tpk, oracle, dev, B, n, m, k):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
-@pytest.mark.parametrize("kind", ["uniform", "normal", "clusters", "flat", "one_point", "lattice", "outlier", "overflow", "queries_outside", "non_finite"])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "clusters", "flat", "one_point", "lattice", "outlier", "outliers", "overflow", "queries_outside", "non_finite"])
 @pytest.mark.parametrize("B,n,m,k", [(2, 1, 3, 1), (2, 65, 40, 48), (1, 3000, 150, 49), (1, 8192, 200, 17), (2, 8193, 90, 48), (1, 40000, 60, 4)])
 def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
     # up to 48 neighbours: a grid in LDS (up to 8192 points) or in memory, its block of cells grown until it holds k, the
@@ -1130,6 +1130,13 @@ def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
         support, query = (support * 12).round(), (query * 24).round() / 2
     elif kind == "outlier":
         support[:, n // 3] = torch.tensor([400.0, -300.0, 1e6])
+    elif kind == "outliers":  # the grid's box is trimmed: on one side and on both, queries beyond it and at the points there
+        far = min(n, 7)
+        support[:, :far] = support[:, :far] * torch.tensor([1e3, 1.0, 1.0]) + torch.tensor([0.0, 50.0, -2e5])
+        support[:, n - 1, 2] = 3e7
+        query[:, 0] = support[:, 0]
+        query[:, 1] = support[:, n - 1] * 0.5
+        query[:, 2] = -1e4
     elif kind == "overflow":  # finite coordinates whose range is not, on every axis
         support[:, n // 3] = 2e38
         support[:, n // 2] = -2e38
@@ -2051,7 +2058,7 @@ def test_counting_build_counts_executed_pairs(oracle, dev):
     assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0 and count.value == 0
 
 
-@pytest.mark.parametrize("kind", ["uniform", "normal", "flat", "queries_far", "queries_around"])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "flat", "outlier", "outliers", "queries_far", "queries_around"])
 def test_knn_looks_at_few_points(oracle, dev, kind):
     """The searches over a grid look at a small part of the cloud, also where the queries lie far outside or the points are
     spread unevenly: 1 to 11 steps of 64 points per query on average, where a scan of the cloud takes 256 (in LDS 94)."""
@@ -2070,6 +2077,12 @@ def test_knn_looks_at_few_points(oracle, dev, kind):
         elif kind == "flat":
             support[..., 2] *= 1e-3
             query[..., 2] *= 1e-3
+        elif kind in ("outlier", "outliers"):
+            if n < 8192:
+                continue  # (in LDS nothing trims the grid: a scan of few points there)
+            support[:, n // 3] = 1000.0
+            if kind == "outliers":
+                support[:, ::1000, 1] = -1e6
         elif kind == "queries_far":
             query += 300.0
         elif kind == "queries_around":

@@ -128,6 +128,7 @@ struct LdsGrid
     int* starts;         // [LG_STARTS] first place of every cell, then the number of points
     float lo[3], inv[3], width[3], volume;
     int cells[3];
+    float below[3], above[3]; // where the cloud ends, in cells (of a grid in memory only: knn.hip)
     float crowd;         // points per cell as a point sees them (per_cell + 1 in a cloud of even density)
 };
 
