@@ -198,9 +198,9 @@ int tpk_three_nn_static_f32(int b, int n, int m, const float* unknown, const flo
  * rule of three_nn (nanoflann leaves that order open).  k > n_support is TPK_ERR_INVALID_ARG
  * (cpu/src/knn.cpp:12-14 raises).  `workspace` (tpk_knn_workspace_bytes() bytes - 0 for shapes
  * not served that way -, 256-byte aligned): search over curve-ordered cells instead of all
- * pairs, same results.  Up to 48 neighbours are found in a grid of cells: in the workspace where
- * it has tpk_knn_grid_workspace_bytes() bytes too (the larger of the two serves every k; 0 for
- * small calls), otherwise in LDS for clouds of up to 8192 points.
+ * pairs, same results.  Up to 48 neighbours are found in a grid of cells: in the workspace, which
+ * holds all the cells a large cloud can use with tpk_knn_grid_workspace_bytes() bytes (0 for small
+ * calls; the larger of the two sizes serves every k best), or in LDS for clouds of up to 8192 points.
  * ------------------------------------------------------------------------------------- */
 size_t tpk_knn_workspace_bytes(int b, int n_support, int m_query);
 size_t tpk_knn_grid_workspace_bytes(int b, int n_support, int m_query);

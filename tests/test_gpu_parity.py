@@ -2058,17 +2058,41 @@ def test_counting_build_counts_executed_pairs(oracle, dev):
     assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0 and count.value == 0
 
 
-@pytest.mark.parametrize("kind", ["uniform", "normal", "flat", "outlier", "outliers", "queries_far", "queries_around"])
-def test_knn_looks_at_few_points(oracle, dev, kind):
-    """The searches over a grid look at a small part of the cloud, also where the queries lie far outside or the points are
-    spread unevenly: 1 to 11 steps of 64 points per query on average, where a scan of the cloud takes 256 (in LDS 94)."""
+def _knn_steps(oracle, dev, support, query, k, workspace="grid"):
+    """Steps of 64 points per query that the counting build takes; the answers are checked on the way.  workspace: the size the
+    grid in memory wants, or the one for curve-ordered cells."""
     import ctypes
     import os
 
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip_counting.so"))
-    lib.tpk_knn_grid_workspace_bytes.restype = ctypes.c_size_t
+    size = lib.tpk_knn_grid_workspace_bytes if workspace == "grid" else lib.tpk_knn_workspace_bytes
+    size.restype = ctypes.c_size_t
     count = ctypes.c_ulonglong(0)
+    (b, n, _), m = support.shape, query.shape[1]
+    s, q = support.to(dev), query.to(dev)
+    dist2 = torch.empty(b, m, k, device=dev)
+    idx = torch.empty(b, m, k, dtype=torch.int64, device=dev)
+    nbytes = size(b, n, m)
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
+    guard = torch.full((1 << 20,), 7, dtype=torch.uint8, device=dev)
+    assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0
+    st = lib.tpk_knn_f32(b, n, m, k, ctypes.c_void_p(s.data_ptr()), ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(idx.data_ptr()),
+                         ctypes.c_void_p(dist2.data_ptr()), ctypes.c_void_p(ws.data_ptr()) if nbytes else None, ctypes.c_size_t(nbytes),
+                         ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == 0
+    assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0
+    assert (guard == 7).all()
+    wi, wd = oracle.knn(support.numpy(), query[:, :300].contiguous().numpy(), k)
+    np.testing.assert_array_equal(_np(idx)[:, :300], wi)
+    np.testing.assert_array_equal(_np(dist2)[:, :300], wd)
+    return count.value / (64 * b * m)
+
+
+@pytest.mark.parametrize("kind", ["uniform", "normal", "flat", "outlier", "outliers", "queries_far", "queries_around"])
+def test_knn_looks_at_few_points(oracle, dev, kind):
+    """The searches over a grid look at a small part of the cloud, also where the queries lie far outside or the points are
+    spread unevenly: 1 to 11 steps of 64 points per query on average, where a scan of the cloud takes 256 (in LDS 94)."""
     g = torch.Generator().manual_seed(3)
     for b, n, m, k in ((1, 16384, 17000, 16), (1, 16384, 17000, 4), (1, 6000, 1000, 16)):
         support, query = torch.rand(b, n, 3, generator=g), torch.rand(b, m, 3, generator=g)
@@ -2087,21 +2111,19 @@ def test_knn_looks_at_few_points(oracle, dev, kind):
             query += 300.0
         elif kind == "queries_around":
             query = query * 3 - 1
-        s, q = support.to(dev), query.to(dev)
-        dist2 = torch.empty(b, m, k, device=dev)
-        idx = torch.empty(b, m, k, dtype=torch.int64, device=dev)
-        nbytes = lib.tpk_knn_grid_workspace_bytes(b, n, m)
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-        assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0
-        st = lib.tpk_knn_f32(b, n, m, k, ctypes.c_void_p(s.data_ptr()), ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(idx.data_ptr()),
-                             ctypes.c_void_p(dist2.data_ptr()), ctypes.c_void_p(ws.data_ptr()) if nbytes else None, ctypes.c_size_t(nbytes),
-                             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-        assert st == 0
-        assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0
-        wi, wd = oracle.knn(support.numpy(), query[:, :300].contiguous().numpy(), k)
-        np.testing.assert_array_equal(_np(idx)[:, :300], wi)
-        steps = count.value / (64 * b * m)
+        steps = _knn_steps(oracle, dev, support, query, k)
         assert steps < 20, (n, k, steps)
+
+
+@pytest.mark.parametrize("b,n,m", [(1, 8193, 512), (1, 12000, 1000), (3, 16384, 600), (2, 30000, 515), (1, 60000, 512)])
+@pytest.mark.parametrize("k", [4, 16])
+def test_knn_in_a_workspace_for_curve_ordered_cells(oracle, dev, b, n, m, k):
+    """A caller with the smaller workspace gets a grid of as many cells as fit there: a few steps per query, counted by the search
+    over a grid alone."""
+    g = torch.Generator().manual_seed(n)
+    support, query = torch.rand(b, n, 3, generator=g), torch.rand(b, m, 3, generator=g)
+    steps = _knn_steps(oracle, dev, support, query, k, "curve")
+    assert 1 <= steps < 5, steps
 
 
 def test_extension_rejects_bad_tensors(tpk, dev):

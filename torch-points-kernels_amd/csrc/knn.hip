@@ -428,18 +428,19 @@ int launch_knn_cells(int b, int n, int m, int k, const float* query, const float
 // their cells' counts in LDS -, a prefix sum, and a third that writes every point's record to its cell.
 constexpr int KNG_CELLS = 32768; // cells at most (their counts lie in LDS)
 
-// Per cloud: the records [m], the cells' first places [KNG_CELLS + 64], the shape [LG_SHAPE],
-// where the cloud ends [6].
+// Per cloud: the records [m], the cells' first places [cells + 64], the shape [LG_SHAPE], where the cloud ends [6].
 struct KnnGridLayout
 {
     size_t starts, shape, total;
+    int cells; // at most; a multiple of 4096, the places a step of the builder's prefix sum writes
 };
-inline KnnGridLayout knn_grid_layout(int m)
+inline KnnGridLayout knn_grid_layout(int m, int cells)
 {
     KnnGridLayout l;
     l.starts = (static_cast<size_t>(m) * sizeof(float4) + 255) & ~static_cast<size_t>(255);
-    l.shape = l.starts + (KNG_CELLS + TPK_WAVE) * sizeof(int);
+    l.shape = l.starts + (static_cast<size_t>(cells) + TPK_WAVE) * sizeof(int);
     l.total = l.shape + 256;
+    l.cells = cells;
     return l;
 }
 
@@ -572,7 +573,7 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
     for (int zooms = 0;; ++zooms)
     {
         if (wave == 0)
-            lg_shape(box, m, per_cell, KNG_AXIS, KNG_CELLS, lane, shape);
+            lg_shape(box, m, per_cell, KNG_AXIS, layout.cells, lane, shape);
         __syncthreads();
 #pragma unroll
         for (int a = 0; a < 3; ++a)
@@ -733,22 +734,39 @@ inline bool knn_in_lds(int b, int m, int n, bool workspace)
 
 size_t knn_grid_workspace_bytes(int b, int m, int n)
 {
-    return b > 0 && n > 0 && !knn_in_lds(b, m, n, true) ? b * knn_grid_layout(m).total : 0;
+    return b > 0 && n > 0 && !knn_in_lds(b, m, n, true) ? b * knn_grid_layout(m, KNG_CELLS).total : 0;
 }
 
-int launch_knn_grid(int b, int n, int m, int k, const float* query, const float* support, float* dist2, int64_t* idx, void* workspace,
-                    size_t workspace_bytes, hipStream_t stream)
+// The cells of the grid that a workspace has room for (0: none).  One for the search over curve-ordered cells
+// (tpk_knn_workspace_bytes) holds 18.5 bytes per point, which leaves a smaller cloud fewer than KNG_CELLS beside its records, but
+// hardly fewer than it has use for: 1000 queries in a cloud of 12000 points, k = 4 and 16: lists over curve-ordered cells 224 and
+// 671 us (lists of 32 entries 1505), this way 24.
+int knn_grid_cells(int b, int m, int n, size_t workspace_bytes)
+{
+    if (workspace_bytes >= knn_grid_workspace_bytes(b, m, n))
+        return KNG_CELLS;
+    const size_t lists = tpk_grid_knn_workspace_bytes(b, n, m);
+    if (lists == 0 || workspace_bytes < lists)
+        return 0;
+    int cells = KNG_CELLS;
+    while (cells > 0 && b * knn_grid_layout(m, cells).total > workspace_bytes)
+        cells -= 4 * LG_THREADS;
+    return cells;
+}
+
+int launch_knn_grid(int b, int n, int m, int k, int cells, const float* query, const float* support, float* dist2, int64_t* idx, void* workspace,
+                    hipStream_t stream)
 {
     const int64_t queries = static_cast<int64_t>(b) * n, blocks = tpk_ceil_div(queries, KNN_THREADS / TPK_WAVE);
     if (blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    if (workspace_bytes < knn_grid_workspace_bytes(b, m, n) || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+    if (reinterpret_cast<uintptr_t>(workspace) & 255u)
         return TPK_ERR_WORKSPACE;
     const size_t lds = KNG_CELLS * sizeof(int);
     const int st = tpk_allow_lds(reinterpret_cast<const void*>(&knn_grid_build_kernel), lds);
     if (st != TPK_OK)
         return st;
-    const KnnGridLayout layout = knn_grid_layout(m);
+    const KnnGridLayout layout = knn_grid_layout(m, cells);
     unsigned char* const w = static_cast<unsigned char*>(workspace);
     hipLaunchKernelGGL(knn_grid_build_kernel, dim3(b), dim3(LG_THREADS), lds, stream, m, knn_per_cell(k), layout, support, w);
     hipLaunchKernelGGL(knn_grid_search_kernel, dim3(static_cast<unsigned>(blocks)), dim3(KNN_THREADS), 0, stream, queries, n, m, k, layout,
@@ -803,11 +821,11 @@ extern "C" int tpk_knn_f32(int b, int n_support, int m_query, int k, const float
         return TPK_ERR_INVALID_ARG;
     if (static_cast<int64_t>(n_support) * 3 > 0x7fffffffLL || static_cast<int64_t>(m_query) * 3 > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    const bool grid = workspace && workspace_bytes >= knn_grid_workspace_bytes(b, n_support, m_query);
-    if (k <= KNC_MAX_K && knn_in_lds(b, n_support, m_query, grid))
+    const int cells = workspace ? knn_grid_cells(b, n_support, m_query, workspace_bytes) : 0; // of a grid in it
+    if (k <= KNC_MAX_K && knn_in_lds(b, n_support, m_query, cells > 0))
         return launch_knn_cells(b, m_query, n_support, k, query, support, dist2, idx, tpk_stream(stream));
-    if (k <= KNC_MAX_K && grid)
-        return launch_knn_grid(b, m_query, n_support, k, query, support, dist2, idx, workspace, workspace_bytes, tpk_stream(stream));
+    if (k <= KNC_MAX_K && cells > 0)
+        return launch_knn_grid(b, m_query, n_support, k, cells, query, support, dist2, idx, workspace, tpk_stream(stream));
     return nearest_within(b, n_support, m_query, k, __builtin_inff(), support, query, idx, dist2, workspace,
                           workspace_bytes, tpk_stream(stream));
 }
