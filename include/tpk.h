@@ -448,9 +448,12 @@ int tpk_gridding_grad_f64(int b, int n_pts, int n_grid_vertices, const double* g
 
 /* The reference's front end gridding(ptcloud, scale) (torch_points_kernels/gridding.py:34-60) for a whole batch:
  * coordinates times `scale`, grids over [-scale, scale - 1] per axis, points whose three products sum to zero
- * (padding) left out cloud by cloud.  The gradient takes the same ptcloud and scale (padding: zeros). */
+ * (padding) left out cloud by cloud.  The gradient takes the same ptcloud and scale (padding: zeros).
+ * _keep_: the forward pass also copies ptcloud to kept (b, n_pts, 3), for a gradient of the points as they were. */
 int tpk_gridding_batch_f32(int b, int n_pts, double scale, const float* ptcloud, float* grid_weights, void* stream);
 int tpk_gridding_batch_f64(int b, int n_pts, double scale, const double* ptcloud, double* grid_weights, void* stream);
+int tpk_gridding_batch_keep_f32(int b, int n_pts, double scale, const float* ptcloud, float* grid_weights, float* kept, void* stream);
+int tpk_gridding_batch_keep_f64(int b, int n_pts, double scale, const double* ptcloud, double* grid_weights, double* kept, void* stream);
 int tpk_gridding_batch_grad_f32(int b, int n_pts, double scale, const float* ptcloud, const float* grad_grid,
                                 float* grad_ptcloud, void* stream);
 int tpk_gridding_batch_grad_f64(int b, int n_pts, double scale, const double* ptcloud, const double* grad_grid,

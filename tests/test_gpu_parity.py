@@ -1479,6 +1479,28 @@ def test_gridding_batch_parity(tpk, oracle, dev, dtype, B, n, scale):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,n,scale", [(2, 700, 8), (1, 1, 2), (1, 5000, 16), (1, 20000, 2)])
+def test_gridding_backward_takes_the_points_as_they_were(tpk, dev, dtype, B, n, scale):
+    # (a caller that moves the cloud in place between the passes, openly or through .data)
+    g = torch.Generator().manual_seed(n)
+    p = (torch.rand(B, n, 3, generator=g, dtype=torch.float64) * 1.9 - 0.95).to(dtype)
+    p[0, n // 2 + 1 :] = 0  # padding
+    r = torch.randn(B, (2 * scale) ** 3, generator=g, dtype=torch.float64).to(dtype).to(dev)
+    x = p.to(dev).requires_grad_()
+    want = torch.autograd.grad(tpk.gridding(x, scale), x, r)[0]
+    for change in ("open", "data"):
+        x = p.to(dev).requires_grad_()
+        cloud = x.clone()
+        grid = tpk.gridding(cloud, scale)
+        if change == "open":
+            with torch.no_grad():
+                cloud.mul_(0.5)
+        else:
+            cloud.data.mul_(0.5)
+        assert torch.equal(torch.autograd.grad(grid, x, r)[0], want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("B,n,c,scale,ns", [(2, 64, 4, 8, 1), (2, 32, 2, 8, 2), (1, 32, 2, 16, 3), (2, 2048, 64, 16, 1), (1, 300, 7, 4, 2)])
 def test_cubic_feature_sampling_parity(tpk, oracle, dev, dtype, B, n, c, scale, ns):
     native = __import__("torch_points_kernels._native", fromlist=["native"]).native()

@@ -12,13 +12,16 @@ inline bool records(const at::Tensor& t)
     return (at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(/*level=*/0).defined();
 }
 
+// (The backward pass needs the points; it gets a copy that the forward kernel makes, so that the caller's may be changed in place.)
 struct GriddingBatch : torch::autograd::Function<GriddingBatch>
 {
     static at::Tensor forward(AutogradContext* ctx, const at::Tensor& ptcloud, double scale)
     {
-        ctx->save_for_backward({ptcloud});
+        at::Tensor kept;
+        at::Tensor grid = gridding_batch_forward(ptcloud, scale, &kept);
+        ctx->save_for_backward({kept});
         ctx->saved_data["scale"] = scale;
-        return gridding_batch_forward(ptcloud, scale);
+        return grid;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {

@@ -11,7 +11,8 @@
 // backward pass, and the form of its Python front end (reference gridding.py:34-60) for a whole
 // batch at once: coordinates times `factor`, points whose three products sum to zero (padding)
 // left out, and a backward pass that forms the factors again from the 12 bytes of a point instead
-// of reading the 128 bytes they take.
+// of reading the 128 bytes they take - of the points as the forward pass found them: it copies
+// them on the way, so that a caller may change the cloud in between, as with the factors kept.
 //
 // Vertices outside the grid: the reference forms the linear index regardless (and writes out of
 // bounds or into a neighbouring row); here such a vertex gets index -1, adds nothing to the grid
@@ -132,19 +133,31 @@ __device__ __forceinline__ void store_factors(int64_t j, const GridBox& box, con
     }
 }
 
+// What the front end's forward pass keeps of a point, as it was given.
+template <typename T>
+__device__ __forceinline__ void keep_point(T* kept, T x, T y, T z)
+{
+    kept[0] = x;
+    kept[1] = y;
+    kept[2] = z;
+}
+
 // cuda/src/gridding_gpu.cu:29-191.  One thread per point, sums in the zeroed grid itself: for grids
 // that the kernel below cannot hold, and for more points than its LDS atomics are quick for.
 template <typename T>
 __global__ __launch_bounds__(GR_THREADS) void gridding_kernel(
     int64_t total_pts, int n_pts, int n_grid_vertices, GridBox box, T factor, bool drop_padding,
     const T* __restrict__ ptcloud, T* __restrict__ grid_weights, T* __restrict__ grid_pt_weights,
-    int* __restrict__ grid_pt_indexes)
+    int* __restrict__ grid_pt_indexes, T* __restrict__ kept)
 {
     const int64_t j = static_cast<int64_t>(blockIdx.x) * GR_THREADS + threadIdx.x;
     if (j >= total_pts)
         return;
     T* grid = grid_weights + (j / n_pts) * n_grid_vertices;
-    const T px = ptcloud[j * 3 + 0] * factor, py = ptcloud[j * 3 + 1] * factor, pz = ptcloud[j * 3 + 2] * factor;
+    const T x = ptcloud[j * 3 + 0], y = ptcloud[j * 3 + 1], z = ptcloud[j * 3 + 2];
+    if (kept)
+        keep_point(kept + j * 3, x, y, z);
+    const T px = x * factor, py = y * factor, pz = z * factor;
     if (drop_padding && is_padding(px, py, pz))
         return;
     const Trilinear<T> p = trilinear(px, py, pz, box.min_x, box.min_y, box.min_z);
@@ -173,7 +186,7 @@ constexpr int GRL_THREADS = 1024;
 template <typename T>
 __global__ __launch_bounds__(GRL_THREADS) void gridding_lds_kernel(
     int n_pts, int parts, int rows_per_x, GridBox box, T factor, bool drop_padding, const T* __restrict__ ptcloud,
-    T* __restrict__ grid_weights, T* __restrict__ grid_pt_weights, int* __restrict__ grid_pt_indexes)
+    T* __restrict__ grid_weights, T* __restrict__ grid_pt_weights, int* __restrict__ grid_pt_indexes, T* __restrict__ kept)
 {
     extern __shared__ __align__(16) unsigned char gridding_lds[];
     T* sums = reinterpret_cast<T*>(gridding_lds);
@@ -188,12 +201,15 @@ __global__ __launch_bounds__(GRL_THREADS) void gridding_lds_kernel(
     const T* points = ptcloud + static_cast<int64_t>(cloud) * n_pts * 3;
     for (int i = threadIdx.x; i < n_pts; i += GRL_THREADS)
     {
-        const T px = points[static_cast<int64_t>(i) * 3 + 0] * factor, py = points[static_cast<int64_t>(i) * 3 + 1] * factor;
-        const T pz = points[static_cast<int64_t>(i) * 3 + 2] * factor;
+        const T x = points[static_cast<int64_t>(i) * 3 + 0], y = points[static_cast<int64_t>(i) * 3 + 1], z = points[static_cast<int64_t>(i) * 3 + 2];
+        const bool stores = ((i / TPK_WAVE) & (parts - 1)) == part; // (one workgroup of the cloud's)
+        if (kept && stores)
+            keep_point(kept + (static_cast<int64_t>(cloud) * n_pts + i) * 3, x, y, z);
+        const T px = x * factor, py = y * factor, pz = z * factor;
         if (drop_padding && is_padding(px, py, pz))
             continue;
         const Trilinear<T> p = trilinear(px, py, pz, box.min_x, box.min_y, box.min_z);
-        if (grid_pt_weights && ((i / TPK_WAVE) & (parts - 1)) == part)
+        if (grid_pt_weights && stores)
             store_factors(static_cast<int64_t>(cloud) * n_pts + i, box, p, grid_pt_weights, grid_pt_indexes);
 #pragma unroll
         for (int row = 0; row < 4; ++row)
@@ -752,7 +768,7 @@ bool grid_box(float min_x, float max_x, float min_y, float max_y, float min_z, f
 
 template <typename T>
 int gridding_fwd(int b, int n_pts, const GridBox& box, T factor, bool drop_padding, const T* ptcloud, T* grid_weights,
-                 T* grid_pt_weights, int32_t* grid_pt_indexes, hipStream_t s)
+                 T* grid_pt_weights, int32_t* grid_pt_indexes, T* kept, hipStream_t s)
 {
     const int64_t vertices = static_cast<int64_t>(box.len_x) * box.len_y * box.len_z;
     if (vertices > 0x7fffffffLL)
@@ -769,7 +785,7 @@ int gridding_fwd(int b, int n_pts, const GridBox& box, T factor, bool drop_paddi
             return allowed;
         hipLaunchKernelGGL(gridding_lds_kernel<T>, dim3(static_cast<unsigned>(b) * parts), dim3(GRL_THREADS), lds, s, n_pts,
                            parts, rows_per_x, box, factor, drop_padding, ptcloud, grid_weights, grid_pt_weights,
-                           grid_pt_indexes);
+                           grid_pt_indexes, kept);
         return tpk_launch_status();
     }
     int st = fill_zero<T>(static_cast<int64_t>(b) * vertices, grid_weights, s);
@@ -781,7 +797,7 @@ int gridding_fwd(int b, int n_pts, const GridBox& box, T factor, bool drop_paddi
         return TPK_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(gridding_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(GR_THREADS), 0, s, total, n_pts,
                        static_cast<int>(vertices), box, factor, drop_padding, ptcloud, grid_weights, grid_pt_weights,
-                       grid_pt_indexes);
+                       grid_pt_indexes, kept);
     return tpk_launch_status();
 }
 
@@ -795,12 +811,12 @@ int gridding_native(int b, int n_pts, float min_x, float max_x, float min_y, flo
         return TPK_ERR_INVALID_ARG;
     if (b > 0 && (!grid_weights || (n_pts > 0 && (!ptcloud || !grid_pt_weights || !grid_pt_indexes))))
         return TPK_ERR_INVALID_ARG;
-    return gridding_fwd<T>(b, n_pts, box, T(1), false, ptcloud, grid_weights, grid_pt_weights, grid_pt_indexes, s);
+    return gridding_fwd<T>(b, n_pts, box, T(1), false, ptcloud, grid_weights, grid_pt_weights, grid_pt_indexes, nullptr, s);
 }
 
 // The front end: a grid over [-scale, scale - 1] per axis, coordinates times `scale`.
 template <typename T>
-int gridding_batch(int b, int n_pts, double scale, const T* ptcloud, T* grid_weights, hipStream_t s)
+int gridding_batch(int b, int n_pts, double scale, const T* ptcloud, T* grid_weights, T* kept, hipStream_t s)
 {
     GridBox box;
     const float lo = static_cast<float>(-scale), hi = static_cast<float>(scale - 1);
@@ -808,7 +824,7 @@ int gridding_batch(int b, int n_pts, double scale, const T* ptcloud, T* grid_wei
         return TPK_ERR_INVALID_ARG;
     if (b > 0 && (!grid_weights || (n_pts > 0 && !ptcloud)))
         return TPK_ERR_INVALID_ARG;
-    return gridding_fwd<T>(b, n_pts, box, static_cast<T>(scale), true, ptcloud, grid_weights, nullptr, nullptr, s);
+    return gridding_fwd<T>(b, n_pts, box, static_cast<T>(scale), true, ptcloud, grid_weights, nullptr, nullptr, kept, s);
 }
 
 template <typename T>
@@ -1089,12 +1105,26 @@ extern "C" int tpk_gridding_grad_f64(int b, int n_pts, int n_grid_vertices, cons
 
 extern "C" int tpk_gridding_batch_f32(int b, int n_pts, double scale, const float* ptcloud, float* grid_weights, void* stream)
 {
-    return gridding_batch<float>(b, n_pts, scale, ptcloud, grid_weights, tpk_stream(stream));
+    return gridding_batch<float>(b, n_pts, scale, ptcloud, grid_weights, nullptr, tpk_stream(stream));
+}
+
+extern "C" int tpk_gridding_batch_keep_f32(int b, int n_pts, double scale, const float* ptcloud, float* grid_weights, float* kept, void* stream)
+{
+    if (b > 0 && n_pts > 0 && !kept)
+        return TPK_ERR_INVALID_ARG;
+    return gridding_batch<float>(b, n_pts, scale, ptcloud, grid_weights, kept, tpk_stream(stream));
 }
 
 extern "C" int tpk_gridding_batch_f64(int b, int n_pts, double scale, const double* ptcloud, double* grid_weights, void* stream)
 {
-    return gridding_batch<double>(b, n_pts, scale, ptcloud, grid_weights, tpk_stream(stream));
+    return gridding_batch<double>(b, n_pts, scale, ptcloud, grid_weights, nullptr, tpk_stream(stream));
+}
+
+extern "C" int tpk_gridding_batch_keep_f64(int b, int n_pts, double scale, const double* ptcloud, double* grid_weights, double* kept, void* stream)
+{
+    if (b > 0 && n_pts > 0 && !kept)
+        return TPK_ERR_INVALID_ARG;
+    return gridding_batch<double>(b, n_pts, scale, ptcloud, grid_weights, kept, tpk_stream(stream));
 }
 
 extern "C" int tpk_gridding_batch_grad_f32(int b, int n_pts, double scale, const float* ptcloud, const float* grad_grid,

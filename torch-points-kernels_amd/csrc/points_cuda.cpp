@@ -798,8 +798,8 @@ at::Tensor gridding_grad(at::Tensor grid_pt_weights, at::Tensor grid_pt_indexes,
 }
 
 // torch_points_kernels/gridding.py:34-60 (the reference's front end, a loop over the clouds there) for the whole
-// batch: one launch forward, one backward (tpk_gridding_batch_f32).
-at::Tensor gridding_batch_forward(const at::Tensor& ptcloud, double scale)
+// batch: one launch forward, one backward (tpk_gridding_batch_f32).  kept: receives a copy of the points, or nullptr.
+at::Tensor gridding_batch_forward(const at::Tensor& ptcloud, double scale, at::Tensor* kept = nullptr)
 {
     check_gpu(ptcloud, "ptcloud");
     TORCH_CHECK(ptcloud.scalar_type() == at::kFloat || ptcloud.scalar_type() == at::kDouble,
@@ -810,13 +810,19 @@ at::Tensor gridding_batch_forward(const at::Tensor& ptcloud, double scale)
     const int64_t side = static_cast<int>(static_cast<float>(scale - 1) - static_cast<float>(-scale) + 1);
     TORCH_CHECK(side > 0, "gridding: empty grid");
     at::Tensor grid = at::empty({b, side * side * side}, ptcloud.options());
+    if (kept)
+        *kept = at::empty_like(ptcloud);
     if (ptcloud.scalar_type() == at::kFloat)
-        check_status(tpk_gridding_batch_f32(b, n, scale, ptcloud.data_ptr<float>(), grid.data_ptr<float>(),
-                                            current_stream(ptcloud)),
+        check_status(kept ? tpk_gridding_batch_keep_f32(b, n, scale, ptcloud.data_ptr<float>(), grid.data_ptr<float>(),
+                                                        kept->data_ptr<float>(), current_stream(ptcloud))
+                          : tpk_gridding_batch_f32(b, n, scale, ptcloud.data_ptr<float>(), grid.data_ptr<float>(),
+                                                   current_stream(ptcloud)),
                      "gridding");
     else
-        check_status(tpk_gridding_batch_f64(b, n, scale, ptcloud.data_ptr<double>(), grid.data_ptr<double>(),
-                                            current_stream(ptcloud)),
+        check_status(kept ? tpk_gridding_batch_keep_f64(b, n, scale, ptcloud.data_ptr<double>(), grid.data_ptr<double>(),
+                                                        kept->data_ptr<double>(), current_stream(ptcloud))
+                          : tpk_gridding_batch_f64(b, n, scale, ptcloud.data_ptr<double>(), grid.data_ptr<double>(),
+                                                   current_stream(ptcloud)),
                      "gridding");
     return grid;
 }
