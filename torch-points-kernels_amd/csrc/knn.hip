@@ -446,9 +446,9 @@ inline KnnGridLayout knn_grid_layout(int m, int cells)
 
 // Trims every axis of the grid's box, by one wavefront, to the cells outside which a 128th of the m points lies on either side
 // (marginals: the points per cell along x, y, z).  The box before goes to `before`; *trimmed = whether it shrinks to KNG_KEPT or
-// less, otherwise `box` stays.  (A normal distribution sees 11 times the points of an even cloud, laser scans 20 to 30, clusters
-// hundreds; trimmed to a half from 8 times on, calls of theirs took up to twice as long.)
-constexpr float KNG_CROWDED = 32.0f; // points per cell as a point sees them, over those of an even cloud, from which the box is trimmed
+// less, otherwise `box` stays.  (A point sees 11 times an even cloud's points in its cell under a normal distribution, 20 to 30 times
+// in laser scans, hundreds in clusters: trimmed to a half from 8 times on, calls of theirs took up to twice as long.)
+constexpr float KNG_CROWDED = 32.0f; // a crowded cell's points, over those that a point of an even cloud sees in its cell
 constexpr float KNG_KEPT = 1.0f / 16.0f;
 constexpr int KNG_ZOOMS = 8; // times at most
 
@@ -489,9 +489,8 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
     __shared__ int box[6], box_before[6]; // ordered ints: min x, y, z then max x, y, z; of the zoom before
     __shared__ float shape[LG_SHAPE];
     __shared__ int wave_totals[LG_WAVES];
-    __shared__ float wave_squares[LG_WAVES];
-    __shared__ int marginals[3 * KNG_AXIS];
-    __shared__ int trimmed;
+    __shared__ int crowded; // points in crowded cells
+    __shared__ int marginals[3 * KNG_AXIS], trimmed;
     constexpr int BATCH = 8; // points in flight per lane
     const int tid = threadIdx.x;
     const int lane = tid & (TPK_WAVE - 1);
@@ -565,11 +564,11 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
     auto cell_of = [&](float x, float y, float z) __attribute__((always_inline)) {
         return lg_cell((x - lo[0]) * inv[0], cx) + cx * (lg_cell((y - lo[1]) * inv[1], cy) + cy * lg_cell((z - lo[2]) * inv[2], cz));
     };
-    // Uneven clouds.  A few points far out leave all others in a cell or two, whose queries would walk the whole cloud.  Where the
-    // cells are that crowded, as a point sees them, and most of the box holds hardly a point, the grid is laid over the rest of the
-    // box and its outermost cells take what lies beyond.  8 x 16384 points, one of them at 1000 cloud sizes, k = 16: 2040 us, this
-    // way 224; even clouds 1.7 us of 104 for the sum of squares.
-    float crowd_before = inf;
+    // Uneven clouds.  A few points far out leave all others in a cell or two, whose queries would walk the whole cloud.  Where half of
+    // the points lie in such cells, and most of the box holds hardly a point, the grid is laid over the rest of the box and its
+    // outermost cells take what lies beyond.  8 x 16384 points, one of them at 1000 cloud sizes, k = 16: 2040 us, this way 232.
+    const int crowd = static_cast<int>(KNG_CROWDED * (per_cell + 1.0f));
+    int crowded_before = m;
     for (int zooms = 0;; ++zooms)
     {
         if (wave == 0)
@@ -585,18 +584,19 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
         const int steps = (cx * cy * cz + 4 * LG_THREADS - 1) / (4 * LG_THREADS); // of the prefix sum, four cells per lane
         for (int c = tid; c < steps * LG_THREADS; c += LG_THREADS)
             reinterpret_cast<int4*>(kng_counts)[c] = make_int4(0, 0, 0, 0);
+        if (tid == 0)
+            crowded = 0;
         __syncthreads();
         each([&](int, float x, float y, float z) { atomicAdd(&kng_counts[cell_of(x, y, z)], 1); });
         __syncthreads();
         int placed = 0; // points in the cells of the steps before
-        float squares = 0.0f;
+        int in_crowds = 0;
         for (int step = 0; step < steps; ++step)
         {
             int4* const four = reinterpret_cast<int4*>(kng_counts) + step * LG_THREADS + tid;
             const int4 c4 = *four;
             const int own = c4.x + c4.y + c4.z + c4.w;
-            const float fx = static_cast<float>(c4.x), fy = static_cast<float>(c4.y), fz = static_cast<float>(c4.z), fw = static_cast<float>(c4.w);
-            squares += fx * fx + fy * fy + fz * fz + fw * fw;
+            in_crowds += (c4.x > crowd ? c4.x : 0) + (c4.y > crowd ? c4.y : 0) + (c4.z > crowd ? c4.z : 0) + (c4.w > crowd ? c4.w : 0);
             const int before = wave_exclusive_sum(own);
             if (lane == TPK_WAVE - 1)
                 wave_totals[wave] = before + own;
@@ -612,35 +612,31 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
             s4.w = at += c4.z;
             *four = s4;
             reinterpret_cast<int4*>(starts)[step * LG_THREADS + tid] = s4; // (also those behind the last cell: the end)
+            if (step == steps - 1 && __ballot(in_crowds != 0) != 0 && in_crowds != 0)
+                atomicAdd(&crowded, in_crowds);
             __syncthreads();
         }
         if (tid == 0)
             starts[steps * 4 * LG_THREADS] = m;
-        for (int off = 1; off < TPK_WAVE; off *= 2)
-            squares += __shfl_xor(squares, off);
-        if (lane == 0)
-            wave_squares[wave] = squares;
-        for (int c = tid; c < 3 * KNG_AXIS; c += LG_THREADS)
-            marginals[c] = 0;
-        __syncthreads();
-        float crowd = 0.0f;
-        for (int w = 0; w < LG_WAVES; ++w)
-            crowd += wave_squares[w];
-        crowd *= 1.0f / static_cast<float>(m);
         // (from here on everything is the same for the whole workgroup)
-        if (zooms > KNG_ZOOMS || crowd <= KNG_CROWDED * (per_cell + 1.0f))
+        const int crowded_now = crowded;
+        if (zooms > KNG_ZOOMS || crowded_now <= m / 2)
             break;
-        if (zooms == KNG_ZOOMS || crowd > crowd_before)
+        if (zooms == KNG_ZOOMS || crowded_now > crowded_before)
         {
-            // the last zoom made it worse: back to the box before
-            if (crowd <= crowd_before)
+            if (crowded_now <= crowded_before)
                 break;
+            // the last zoom made it worse: back to the box before
             if (tid < 6)
                 box[tid] = box_before[tid];
             zooms = KNG_ZOOMS;
             __syncthreads();
             continue;
         }
+        crowded_before = crowded_now;
+        for (int c = tid; c < 3 * KNG_AXIS; c += LG_THREADS)
+            marginals[c] = 0;
+        __syncthreads();
         // (the counts of planes and rows are differences of the prefix sums; neighbouring lanes add to neighbouring places)
         const int cells = cx * cy * cz;
         auto count_of = [&](int first, int end) __attribute__((always_inline)) { return (end < cells ? kng_counts[end] : m) - kng_counts[first]; };
@@ -661,7 +657,6 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
         __syncthreads();
         if (!trimmed)
             break;
-        crowd_before = crowd;
     }
     if (tid < LG_SHAPE)
         reinterpret_cast<float*>(workspace + layout.shape)[tid] = shape[tid];
