@@ -372,7 +372,7 @@ int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64
  *   found (2, HOST memory): points kept; 1 if the outputs were written, 0 if the points already stand in that order
  *     (one label, none ignored) or none is left.  order (n) int32: the point at every position; pos_out (n, 3);
  *     ids (n) int64: ascending cloud ids.  batch must be sorted.  At most TPK_REGION_IGNORED ignored labels (HOST
- *     array), labels spanning less than 2^31 (else TPK_ERR_UNSUPPORTED).  Waits for the stream once.
+ *     array), labels spanning less than 2^31, times the span of the sample ids less than 2^63 (else TPK_ERR_UNSUPPORTED).  Waits for the stream once.
  * tpk_region_members: members[i] = order[positions[i]] (order NULL: positions[i]); positions of 4 or 8 bytes, in place
  * if they are `members`. */
 #define TPK_REGION_IGNORED 32

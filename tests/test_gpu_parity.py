@@ -1287,6 +1287,24 @@ def test_region_grow_all_labels_at_once(tpk, oracle, dev, n, kinds, ignored, spr
         assert region_grow(pos.to(dev), labels.to(dev), batch.to(dev), sorted(set(labels.tolist())), radius=0.06) == []
 
 
+@pytest.mark.parametrize("label_step,ids", [(10 ** 6, [-(2 ** 62), 17, 2 ** 62]), (2 ** 28, [0, 5, 2 ** 40]), (1, [-(2 ** 63), 0, 2 ** 63 - 1])])
+def test_region_grow_sample_ids_far_apart(tpk, oracle, dev, label_step, ids):
+    """Sample ids that are hashes and labels spread wide: label times span of the ids does not fit 63 bits."""
+    from torch_points_kernels.cluster import region_grow
+
+    g = torch.Generator().manual_seed(9)
+    pos, batch = _blobs(g, 3, 2000, 0.05)
+    labels = torch.randint(0, 5, (pos.shape[0],), generator=g) * label_step
+    far = torch.tensor(ids)[batch]
+    want = oracle.region_grow(pos.numpy(), labels.numpy(), batch.numpy(), ignore_labels=[label_step], radius=0.06, min_cluster_size=5)
+    assert len(want) > 0
+    for order in ("reference", "index"):
+        got = region_grow(pos.to(dev), labels.to(dev), far.to(dev), [label_step], radius=0.06, min_cluster_size=5, member_order=order)
+        assert len(got) == len(want)
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(_np(a), b if order == "reference" else np.sort(b))
+
+
 def test_grow_proximity_any_matrix(tpk, oracle, dev):
     """Matrices that no ball query produces: rows ending early, entries after a -1 (ignored, the row has ended), chains
     in both directions, points nobody lists, no columns at all."""

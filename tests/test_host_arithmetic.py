@@ -11,6 +11,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 SHIM = r"""
 #include "bracket.h"
+#include "cloud_ids.h"
 #include "grid_shape.h"
 #include <cmath>
 
@@ -50,6 +51,11 @@ extern "C" int guesses(const float* distance, int count, int k, int most, float 
         in = within(guess);
     }
     return tries;
+}
+
+extern "C" int ids_fit(unsigned labels, unsigned long long span)
+{
+    return region_ids_fit(labels, span) ? 1 : 0;
 }
 """
 
@@ -125,3 +131,13 @@ def test_a_selection_finds_a_distance(shim, first, offset, spread, k):
 def test_a_selection_gives_up_on_equal_distances(shim):
     distance = np.full(100, 0.5, np.float32)
     assert shim.guesses(distance.ctypes.data_as(ctypes.c_void_p), 100, 16, 40, ctypes.c_float(1.0)) == -1
+
+
+def test_cloud_ids_are_refused_before_they_overflow(shim):
+    shim.ids_fit.argtypes = [ctypes.c_uint, ctypes.c_ulonglong]
+    for labels in (1, 2, 3, 1000, 2 ** 31 - 1, 2 ** 31):
+        for span in [1, 2, 1000] + [2 ** e + d for e in (31, 32, 33, 52, 61, 62, 63) for d in (-1, 0, 1)] + [2 ** 64 - 1]:
+            largest = labels * span - 1  # label labels - 1, sample span - 1
+            assert not shim.ids_fit(labels, span) or largest < 2 ** 63 - 1, (labels, span)
+            assert shim.ids_fit(labels, span) or largest >= 2 ** 63 - 1 - labels, (labels, span)
+        assert not shim.ids_fit(labels, 0)  # all 2^64 values

@@ -38,6 +38,7 @@
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
+#include "cloud_ids.h"
 #include "tpk_device.h"
 
 namespace
@@ -832,11 +833,14 @@ __device__ __forceinline__ bool is_ignored(const Ignored& ignored, int64_t label
     return false;
 }
 
-// Smallest and largest label that is not ignored and how many points carry one, per block.
+// Smallest and largest label that is not ignored and how many points carry one, per block; behind them the first and the last
+// sample id.
 __global__ void __launch_bounds__(CL_THREADS)
-    region_range_kernel(int n, const int64_t* __restrict__ labels, Ignored ignored, LabelRange* ranges)
+    region_range_kernel(int n, const int64_t* __restrict__ labels, const int64_t* __restrict__ batch, Ignored ignored, LabelRange* ranges)
 {
     __shared__ LabelRange shared[CL_THREADS];
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        ranges[RG_RANGE_BLOCKS] = LabelRange{batch[0], batch[n - 1], 0};
     LabelRange r{INT64_MAX, INT64_MIN, 0};
     for (int i = blockIdx.x * CL_THREADS + threadIdx.x; i < n; i += RG_RANGE_BLOCKS * CL_THREADS)
     {
@@ -878,15 +882,14 @@ struct RegionKeys
 };
 
 // Points of one label and one sample form a cloud; its id grows with (label, sample), which is the order
-// the rows stand in.
+// the rows stand in.  (span: of the sample ids; labels * span is below 2^63, or the caller numbers both anew)
 __global__ void __launch_bounds__(CL_THREADS)
-    region_gather_kernel(int n, int kept, const unsigned* __restrict__ keys, const unsigned* __restrict__ values,
+    region_gather_kernel(int kept, int64_t first, int64_t span, const unsigned* __restrict__ keys, const unsigned* __restrict__ values,
                          const int64_t* __restrict__ batch, const float* __restrict__ pos, int32_t* order, float* pos_out, int64_t* ids)
 {
     const int i = blockIdx.x * CL_THREADS + threadIdx.x;
     if (i >= kept)
         return;
-    const int64_t first = batch[0], span = batch[n - 1] - first + 1;
     const int64_t v = values[i];
     order[i] = (int32_t)v;
     ids[i] = (int64_t)keys[i] * span + (batch[v] - first);
@@ -1026,7 +1029,7 @@ bool region_layout(int64_t n, RegionLayout* l)
     l->values_in = 2 * ints;
     l->values_out = 3 * ints;
     l->ranges = 4 * ints;
-    l->temp = l->ranges + aligned(RG_RANGE_BLOCKS * sizeof(LabelRange));
+    l->temp = l->ranges + aligned((RG_RANGE_BLOCKS + 1) * sizeof(LabelRange));
     l->temp_bytes = temp;
     l->total = l->temp + aligned(temp);
     return true;
@@ -1159,13 +1162,14 @@ extern "C" int tpk_region_order(int64_t n, const int64_t* labels, const int64_t*
     for (int i = 0; i < ignored_count; ++i)
         ignored.value[i] = ignored_labels[i];
     LabelRange* ranges = reinterpret_cast<LabelRange*>(ws + l.ranges);
-    region_range_kernel<<<RG_RANGE_BLOCKS, CL_THREADS, 0, s>>>((int)n, labels, ignored, ranges);
-    LabelRange host[RG_RANGE_BLOCKS], all{INT64_MAX, INT64_MIN, 0};
+    region_range_kernel<<<RG_RANGE_BLOCKS, CL_THREADS, 0, s>>>((int)n, labels, batch, ignored, ranges);
+    LabelRange host[RG_RANGE_BLOCKS + 1], all{INT64_MAX, INT64_MIN, 0};
     hipError_t e = static_cast<hipError_t>(tpk_read_back(host, ranges, sizeof(host), s));
     if (e != hipSuccess)
         return (int)e;
-    for (const LabelRange& r : host)
+    for (int block = 0; block < RG_RANGE_BLOCKS; ++block)
     {
+        const LabelRange& r = host[block];
         all.low = r.low < all.low ? r.low : all.low;
         all.high = r.high > all.high ? r.high : all.high;
         all.kept += r.kept;
@@ -1178,17 +1182,21 @@ extern "C" int tpk_region_order(int64_t n, const int64_t* labels, const int64_t*
         return TPK_OK; // one label: the points stand in their order already
     if ((uint64_t)all.high - (uint64_t)all.low >= (uint64_t)0x7fffffff)
         return TPK_ERR_UNSUPPORTED;
+    const unsigned beyond = (unsigned)(all.high - all.low) + 1u;
+    const int64_t first = host[RG_RANGE_BLOCKS].low;
+    const uint64_t span = (uint64_t)host[RG_RANGE_BLOCKS].high - (uint64_t)first + 1; // (0: all of them)
+    if (!region_ids_fit(beyond, span))
+        return TPK_ERR_UNSUPPORTED;
     unsigned* keys_in = reinterpret_cast<unsigned*>(ws + l.keys_in);
     unsigned* keys_out = reinterpret_cast<unsigned*>(ws + l.keys_out);
     unsigned* values_in = reinterpret_cast<unsigned*>(ws + l.values_in);
     unsigned* values_out = reinterpret_cast<unsigned*>(ws + l.values_out);
-    const unsigned beyond = (unsigned)(all.high - all.low) + 1u;
     e = sort_points((int)n, beyond + 1u, RegionKeys{all.low, beyond, labels, ignored},
                     SortSpace{keys_in, keys_out, values_in, values_out, ws + l.temp, l.temp_bytes}, s);
     if (e != hipSuccess)
         return (int)e;
-    region_gather_kernel<<<(unsigned)tpk_ceil_div(all.kept, CL_THREADS), CL_THREADS, 0, s>>>((int)n, (int)all.kept, keys_out, values_out,
-                                                                                             batch, pos, order, pos_out, ids);
+    region_gather_kernel<<<(unsigned)tpk_ceil_div(all.kept, CL_THREADS), CL_THREADS, 0, s>>>((int)all.kept, first, (int64_t)span, keys_out,
+                                                                                             values_out, batch, pos, order, pos_out, ids);
     found[1] = 1;
     return tpk_launch_status();
 }

@@ -591,8 +591,9 @@ std::vector<at::Tensor> region_grow(at::Tensor pos, at::Tensor labels, at::Tenso
                                             ws.data_ptr(), ws_bytes, stream);
         if (status == TPK_ERR_UNSUPPORTED)
         {
-            // labels far apart: their ranks instead
+            // labels far apart, or sample ids too far apart for as many labels: the ranks of both instead
             at::Tensor values, ranks;
+            batch = std::get<1>(at::unique_consecutive(batch, /*return_inverse=*/true));
             std::tie(values, ranks) = at::_unique(labels, /*sorted=*/true, /*return_inverse=*/true);
             values = values.cpu();
             std::vector<int64_t> ignored_ranks;
