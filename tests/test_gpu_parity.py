@@ -1305,6 +1305,24 @@ def test_region_grow_sample_ids_far_apart(tpk, oracle, dev, label_step, ids):
             np.testing.assert_array_equal(_np(a), b if order == "reference" else np.sort(b))
 
 
+@pytest.mark.parametrize("n,nsample", [(4000, 16), (40000, 5), (70000, 3)])
+def test_grow_proximity_in_several_turns(tpk, dev, n, nsample):
+    """Rows that take more pinned memory than is allowed at a time are copied and walked in turns; a piece that alone takes more
+    comes through pageable memory.  (Entries of 2 bytes, and of 4 where a piece has more than 65536 points.)"""
+    native = __import__("torch_points_kernels._native", fromlist=["native"]).native()
+    g = torch.Generator().manual_seed(n)
+    pos, batch = _blobs(g, 2, n // 2, 0.03)
+    if n == 70000:
+        batch = torch.zeros_like(batch)
+    neighbours = tpk.ball_query(0.3 if n == 70000 else 0.02, nsample, pos.to(dev), pos.to(dev), mode="PARTIAL_DENSE",
+                                batch_x=batch.to(dev), batch_y=batch.to(dev))[0]
+    members, starts = native.grow_proximity(neighbours, 2, True)
+    assert starts.shape[0] > 1
+    for most in (1, 10 ** 4, 10 ** 5, 10 ** 6):
+        some, ends = native.grow_proximity(neighbours, 2, True, most)
+        assert torch.equal(some, members) and torch.equal(ends, starts)
+
+
 def test_grow_proximity_any_matrix(tpk, oracle, dev):
     """Matrices that no ball query produces: rows ending early, entries after a -1 (ignored, the row has ended), chains
     in both directions, points nobody lists, no columns at all."""

@@ -13,6 +13,7 @@ SHIM = r"""
 #include "bracket.h"
 #include "cloud_ids.h"
 #include "grid_shape.h"
+#include "grow_walk.h"
 #include <cmath>
 
 extern "C" void grid_of(const float* low, const float* high, int m, float per_cell, int axis, int most, float* extent, int* along)
@@ -51,6 +52,16 @@ extern "C" int guesses(const float* distance, int count, int k, int most, float 
         in = within(guess);
     }
     return tries;
+}
+
+extern "C" long long pieces_within(const int64_t* starts, long long pieces, long long begin, long long row_bytes, long long most)
+{
+    return grow_walk::pieces_within(starts, pieces, begin, row_bytes, most);
+}
+
+extern "C" long long most_staged()
+{
+    return grow_walk::MOST_STAGED;
 }
 
 extern "C" int ids_fit(unsigned labels, unsigned long long span)
@@ -141,3 +152,22 @@ def test_cloud_ids_are_refused_before_they_overflow(shim):
             assert not shim.ids_fit(labels, span) or largest < 2 ** 63 - 1, (labels, span)
             assert shim.ids_fit(labels, span) or largest >= 2 ** 63 - 1 - labels, (labels, span)
         assert not shim.ids_fit(labels, 0)  # all 2^64 values
+
+
+@pytest.mark.parametrize("row_bytes,most", [(32, 1), (32, 3200), (6, 10 ** 4), (256, 10 ** 6), (4, 2 ** 62)])
+def test_turns_of_pieces_stay_within_their_bytes(shim, row_bytes, most):
+    """Every piece in one turn, no turn above the bytes unless it is a single piece, none that could have taken the next one too."""
+    shim.pieces_within.restype = ctypes.c_longlong
+    shim.pieces_within.argtypes = [ctypes.c_void_p] + [ctypes.c_longlong] * 4
+    shim.most_staged.restype = ctypes.c_longlong
+    assert 2 ** 24 <= shim.most_staged() <= 2 ** 28
+    rng = np.random.default_rng(7)
+    for pieces in (1, 2, 77):
+        starts = np.concatenate([[0], np.cumsum(rng.integers(1, 200, pieces))]).astype(np.int64)
+        begin = 0
+        while begin < pieces:
+            end = shim.pieces_within(starts.ctypes.data_as(ctypes.c_void_p), pieces, begin, row_bytes, most)
+            assert begin < end <= pieces
+            assert end == begin + 1 or (starts[end] - starts[begin]) * row_bytes <= most
+            assert end == pieces or (starts[end + 1] - starts[begin]) * row_bytes > most
+            begin = end

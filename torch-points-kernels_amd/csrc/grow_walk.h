@@ -27,6 +27,10 @@ struct Scratch
     std::vector<uint32_t> stack, members;
 };
 
+// Bytes of pinned memory that hold rows at a time.  Such memory stays with the process (torch's pool of it gives nothing back), and
+// the rows of millions of points are gigabytes.
+constexpr int64_t MOST_STAGED = int64_t(256) << 20;
+
 // Walks one piece of `count` points.  Clusters of at least min_size members go to `found`, their members - as
 // positions - to places[at ...], which never takes more than the piece's own range.
 template <typename E>
@@ -88,6 +92,16 @@ void walk_piece(const E* rows, int nsample, const int32_t* positions, int64_t ba
         found.push_back(Cluster{positions[seed], written, size});
         written += size;
     }
+}
+
+// Pieces begin .. end (returned) whose rows, row_bytes per point, take no more than `most` bytes together; at least one piece,
+// whatever it takes.  starts: first place of every piece, then the total.
+inline int64_t pieces_within(const int64_t* starts, int64_t pieces, int64_t begin, int64_t row_bytes, int64_t most)
+{
+    int64_t end = begin + 1;
+    while (end < pieces && (starts[end + 1] - starts[begin]) <= most / row_bytes)
+        ++end;
+    return end;
 }
 
 } // namespace grow_walk

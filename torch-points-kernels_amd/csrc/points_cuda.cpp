@@ -171,22 +171,22 @@ std::pair<at::Tensor, at::Tensor> dense_knn(at::Tensor support, at::Tensor query
     return std::make_pair(idx, dist2);
 }
 
-// Host memory the device can address (torch's pool of such blocks: a block given back is reused by the next call).
-at::Tensor pinned(int64_t bytes)
+// Host memory for copies to and from the device: pinned up to `most` bytes (torch's pool of such blocks, one given back is reused by
+// the next call), pageable beyond, which the pool does not keep.
+at::Tensor host_bytes(int64_t bytes, int64_t most)
 {
-    return at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+    return at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(bytes <= most));
 }
 
-// Clusters in the reference's member order: pieces from the device, walked on host threads.  members: one tensor on the
-// device, clusters one after the other, as indices (order: what tpk_region_order put at every position; may be
-// undefined); sizes: theirs.
+// Walks the pieces begin .. end on host threads; rows: theirs, from the place starts[begin] on.  Adds to `all`.
 template <typename E>
-void walk_pieces(const E* rows, int nsample, const int32_t* positions, const int64_t* starts, int64_t pieces, int64_t points,
-                 int64_t min_cluster_size, int32_t* places, int32_t* members, std::vector<int64_t>* sizes)
+void walk_pieces(const E* rows, int nsample, const int32_t* positions, const int64_t* starts, int64_t begin, int64_t end,
+                 int64_t min_cluster_size, int32_t* places, std::vector<grow_walk::Cluster>* all)
 {
+    const int64_t pieces = end - begin, points = starts[end] - starts[begin];
     std::vector<int64_t> turn(static_cast<size_t>(pieces));
     for (int64_t p = 0; p < pieces; ++p)
-        turn[p] = p;
+        turn[p] = begin + p;
     // the longest walks first: the end of the last one is what the caller waits for
     std::stable_sort(turn.begin(), turn.end(), [&](int64_t a, int64_t b) { return starts[a + 1] - starts[a] > starts[b + 1] - starts[b]; });
     // (below 16384 points the walk takes less time than waking the other threads)
@@ -198,38 +198,34 @@ void walk_pieces(const E* rows, int nsample, const int32_t* positions, const int
         for (int64_t i = next.fetch_add(1); i < pieces; i = next.fetch_add(1))
         {
             const int64_t base = starts[turn[i]], count = starts[turn[i] + 1] - base;
-            grow_walk::walk_piece(rows + base * nsample, nsample, positions + base, base, count, min_cluster_size, scratch,
-                                  places, found[t]);
+            grow_walk::walk_piece(rows + (base - starts[begin]) * nsample, nsample, positions + base, base, count, min_cluster_size,
+                                  scratch, places, found[t]);
         }
     };
     if (threads == 1)
         work(0);
     else
-        at::parallel_for(0, threads, 1, [&](int64_t begin, int64_t end) {
-            for (int64_t t = begin; t < end; ++t)
+        at::parallel_for(0, threads, 1, [&](int64_t first, int64_t last) {
+            for (int64_t t = first; t < last; ++t)
                 work(t);
         });
-    std::vector<grow_walk::Cluster> all;
     for (const auto& f : found)
-        all.insert(all.end(), f.begin(), f.end());
-    std::sort(all.begin(), all.end(), [](const grow_walk::Cluster& a, const grow_walk::Cluster& b) { return a.first_position < b.first_position; });
-    sizes->clear();
-    for (const grow_walk::Cluster& c : all)
-    {
-        std::memcpy(members, places + c.at, static_cast<size_t>(c.size) * sizeof(int32_t));
-        members += c.size;
-        sizes->push_back(c.size);
-    }
+        all->insert(all->end(), f.begin(), f.end());
 }
 
+// Clusters in the reference's member order: pieces from the device, walked on host threads.  members: one tensor on the
+// device, clusters one after the other, as indices (order: what tpk_region_order put at every position; may be
+// undefined); sizes: theirs.  most: bytes of pinned memory at a time; pieces that together take more are copied and walked in
+// several turns.
 at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluster_size, const at::Tensor& order,
-                                std::vector<int64_t>* sizes)
+                                std::vector<int64_t>* sizes, int64_t most = grow_walk::MOST_STAGED)
 {
     const int64_t n = neighbours.size(0);
     const int nsample = as_int(neighbours.size(1), "nsample");
     auto bytes_on_device = at::device(neighbours.device()).dtype(at::kByte);
     auto longs = at::device(neighbours.device()).dtype(at::kLong);
     void* stream = current_stream(neighbours);
+    auto wait = [&] { c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(neighbours.get_device()).synchronize(); };
     sizes->clear();
     const size_t ws_bytes = tpk_grow_components_workspace_bytes(n);
     TORCH_CHECK(ws_bytes > 0, "grow_proximity: too many points");
@@ -241,35 +237,62 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     const int64_t pieces = found[0], points = found[1];
     if (pieces == 0)
         return at::empty({0}, longs);
-    const int64_t entry = found[2] <= 65536 ? 2 : 4;
+    const int64_t entry = found[2] <= 65536 ? 2 : 4, row_bytes = nsample * entry;
     // one block for all three: starts, positions, rows
     const int64_t at_positions = (pieces + 1) * 8, at_rows = (at_positions + points * 4 + 15) / 16 * 16;
-    at::Tensor staged = at::empty({at_rows + points * nsample * entry}, bytes_on_device);
+    at::Tensor staged = at::empty({at_rows + points * row_bytes}, bytes_on_device);
     uint8_t* d = staged.data_ptr<uint8_t>();
     check_status(tpk_grow_rows(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), d + at_rows,
                                reinterpret_cast<int32_t*>(d + at_positions), reinterpret_cast<int64_t*>(d), ws.data_ptr(), ws_bytes,
                                stream),
                  "grow_proximity (rows)");
-    at::Tensor host = pinned(staged.numel());
-    host.copy_(staged, /*non_blocking=*/true);
-    c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(neighbours.get_device()).synchronize();
+    // (at once where it fits; otherwise the rows come by themselves)
+    const bool at_once = staged.numel() <= most;
+    at::Tensor host = host_bytes(at_once ? staged.numel() : at_rows, most);
+    host.copy_(staged.narrow(0, 0, host.numel()), /*non_blocking=*/true);
+    wait();
     const uint8_t* h = host.data_ptr<uint8_t>();
     const int64_t* starts = reinterpret_cast<const int64_t*>(h);
     const int32_t* positions = reinterpret_cast<const int32_t*>(h + at_positions);
     // (both halves from the pool: fresh memory would cost a page fault per 4 KiB)
-    at::Tensor walked = pinned(points * 8);
+    at::Tensor walked = host_bytes(points * 8, most);
     int32_t* out = reinterpret_cast<int32_t*>(walked.data_ptr<uint8_t>());
     int32_t* places = out + points;
-    if (entry == 2)
-        walk_pieces(reinterpret_cast<const uint16_t*>(h + at_rows), nsample, positions, starts, pieces, points, min_cluster_size, places, out, sizes);
+    std::vector<grow_walk::Cluster> all;
+    auto walk = [&](const uint8_t* rows, int64_t begin, int64_t end) {
+        if (entry == 2)
+            walk_pieces(reinterpret_cast<const uint16_t*>(rows), nsample, positions, starts, begin, end, min_cluster_size, places, &all);
+        else
+            walk_pieces(reinterpret_cast<const uint32_t*>(rows), nsample, positions, starts, begin, end, min_cluster_size, places, &all);
+    };
+    if (at_once)
+        walk(h + at_rows, 0, pieces);
     else
-        walk_pieces(reinterpret_cast<const uint32_t*>(h + at_rows), nsample, positions, starts, pieces, points, min_cluster_size, places, out, sizes);
+    {
+        at::Tensor turn; // the rows of some pieces
+        for (int64_t begin = 0, end = 0; begin < pieces; begin = end)
+        {
+            end = grow_walk::pieces_within(starts, pieces, begin, row_bytes, most);
+            const int64_t bytes = (starts[end] - starts[begin]) * row_bytes;
+            if (!turn.defined() || turn.numel() < bytes)
+                turn = host_bytes(std::max(bytes, std::min(most, points * row_bytes)), most);
+            at::Tensor rows = turn.narrow(0, 0, bytes);
+            rows.copy_(staged.narrow(0, at_rows + starts[begin] * row_bytes, bytes), /*non_blocking=*/true);
+            wait();
+            walk(rows.data_ptr<uint8_t>(), begin, end);
+        }
+    }
+    std::sort(all.begin(), all.end(), [](const grow_walk::Cluster& a, const grow_walk::Cluster& b) { return a.first_position < b.first_position; });
     int64_t total = 0;
-    for (int64_t v : *sizes)
-        total += v;
+    for (const grow_walk::Cluster& c : all)
+    {
+        std::memcpy(out + total, places + c.at, static_cast<size_t>(c.size) * sizeof(int32_t));
+        total += c.size;
+        sizes->push_back(c.size);
+    }
     at::Tensor members = at::empty({total}, longs);
     at::Tensor uploaded = at::empty({total * 4}, bytes_on_device);
-    uploaded.copy_(walked.narrow(0, 0, total * 4), /*non_blocking=*/true);
+    uploaded.copy_(walked.narrow(0, 0, total * 4), /*non_blocking=*/walked.numel() <= most); // (a pageable block goes with this call)
     check_status(tpk_region_members(total, order.defined() ? order.data_ptr<int32_t>() : nullptr, 4, uploaded.data_ptr(),
                                     members.data_ptr<int64_t>(), stream),
                  "grow_proximity (members)");
@@ -278,8 +301,9 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
 
 // torch_points_kernels/cluster.py:9-37 (_grow_proximity_core; host code in the reference)
 // -> (members, starts): clusters one after the other and their offsets (one more than clusters).
-std::pair<at::Tensor, at::Tensor> grow_proximity(at::Tensor neighbours, int64_t min_cluster_size,
-                                                 bool reference_order)
+// most_staged: see grow_reference_order.
+std::pair<at::Tensor, at::Tensor> grow_proximity(at::Tensor neighbours, int64_t min_cluster_size, bool reference_order,
+                                                 int64_t most_staged)
 {
     check_contiguous(neighbours, "neighbours");
     check_dtype(neighbours, at::kLong, "neighbours");
@@ -294,7 +318,7 @@ std::pair<at::Tensor, at::Tensor> grow_proximity(at::Tensor neighbours, int64_t 
     if (n > 0 && reference_order && neighbours.size(1) > 0)
     {
         std::vector<int64_t> sizes;
-        members = grow_reference_order(neighbours, min_cluster_size, at::Tensor(), &sizes);
+        members = grow_reference_order(neighbours, min_cluster_size, at::Tensor(), &sizes, most_staged);
         std::vector<int64_t> ends(1, 0);
         for (int64_t v : sizes)
             ends.push_back(ends.back() + v);
@@ -627,7 +651,7 @@ std::vector<at::Tensor> region_grow(at::Tensor pos, at::Tensor labels, at::Tenso
     else
     {
         at::Tensor starts;
-        std::tie(members, starts) = grow_proximity(neighbours, min_cluster_size, false);
+        std::tie(members, starts) = grow_proximity(neighbours, min_cluster_size, false, grow_walk::MOST_STAGED);
         if (order.defined())
             check_status(tpk_region_members(members.numel(), order.data_ptr<int32_t>(), 8, members.data_ptr<int64_t>(),
                                             members.data_ptr<int64_t>(), stream),
@@ -1226,7 +1250,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("three_nn", &three_nn);
     m.def("three_nn_distance", &three_nn_distance);
     m.def("dense_knn", &dense_knn);
-    m.def("grow_proximity", &grow_proximity, pybind11::call_guard<pybind11::gil_scoped_release>());
+    m.def("grow_proximity", &grow_proximity, pybind11::arg("neighbours"), pybind11::arg("min_cluster_size"), pybind11::arg("reference_order"),
+          pybind11::arg("most_staged") = grow_walk::MOST_STAGED, pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("region_grow", &region_grow, pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("instance_iou_cuda", &instance_iou_cuda);
     m.def("instance_iou_lists", &instance_iou_lists);
