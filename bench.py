@@ -36,18 +36,23 @@ VALU_FILE = os.path.join(PROFILES, "distance_scans_valu_utilisation.txt")
 
 # Kernels whose HBM traffic adds up to one launch of an operator (names as rocprofv3 prints them).
 TRAFFIC_KERNELS = {
-    "fps": ["fps_pruned_kernel<16, 1024, 4>"],
-    "three_interpolate_fwd": ["gather_fwd_lds_kernel<3, true, int, true>"],
+    "fps": ["fps_pool_kernel<18, 16, 3, true>"],
+    "three_interpolate_fwd": ["gather_fwd_lds_kernel<3, true, int>"],
     "three_interpolate_bwd": ["build_lists_kernel<3, true, int>", "gather_bwd_lists_kernel<3, true, 2>"],
     "three_interpolate_bwd_lists": ["gather_bwd_lists_kernel<3, true, 2>"],
     "grouping_bwd_lists": ["gather_bwd_lists_kernel<1, false, 1>"],
-    "grouping_fwd": ["gather_fwd_lds_kernel<1, false, long, false>"],
+    "grouping_fwd": ["gather_fwd_lds_kernel<1, false, long>"],
     "grouping_bwd": ["build_lists_kernel<1, false, long>", "gather_bwd_lists_kernel<1, false, 1>"],
-    "chamfer_bwd": ["chamfer_bwd_chains_kernel<float>"],
+    "chamfer_bwd": ["chamfer_bwd_chains_kernel<float, false>"],
+    "gridding_fwd": ["gridding_lds_kernel<float>"],
+    "gridding_bwd": ["gridding_grad_kernel<float>"],
+    "cubic_fwd": ["cubic_turn_kernel<float, true>", "cubic_rows_kernel<float, unsigned int __vector(4)>"],
+    "cubic_bwd": ["fill_zero_kernel<float>", "cubic_spans_kernel<float, 64>"],
+    "instance_iou": ["instance_iou_kernel"],
 }
 # Kernels whose VALU counters describe a distance scan.
 VALU_KERNELS = {
-    "fps": "fps_pruned_kernel<16, 1024, 4>",
+    "fps": "fps_pool_kernel<18, 16, 3, true>",
     "ball_query_dense": "ball_query_dense_cells_kernel<false>",
     "ball_query_partial_dense": "ball_query_bins_kernel<false, false>",
     "three_nn": "three_nn_cells_kernel",
@@ -234,8 +239,8 @@ def _all_pairs_entry(call, pairs, steps, warmup, valu_kernel):
                         "valu_lane_utilisation_pct": table[valu_kernel].get("VALUUtilization"),
                         "source": "profiles/" + os.path.basename(VALU_FILE), "measured_at_commit": commit}
     return {"what": "the same configuration through the C ABI's scan of all pairs (workspace == NULL; three_nn: "
-                    "tpk_three_nn_all_pairs_f32): every query scans its whole cloud "
-                    "(the kernel the north star describes); same results", "kernel_ms": ev, "wall_ms": wall, "roofline": roof}
+                    "tpk_three_nn_all_pairs_f32): every query scans its whole cloud; "
+                    "same results", "kernel_ms": ev, "wall_ms": wall, "roofline": roof}
 
 
 COUNT_WORK = True  # --no-count: leave the counting build out (profiler runs: its kernels carry the same names)

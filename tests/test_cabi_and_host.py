@@ -293,3 +293,24 @@ def test_bench_line_is_short_and_parses():
     # a line that would be too long sheds the operators outside the BASELINE configurations first
     short = json.loads(bench.compact_line(full, bench.DETAIL_FILE, limit=2600))
     assert short["ops_dropped"] > 0 and "ball_query_dense" in short["ops"] and "roofline" in short
+
+
+def test_benchmark_names_kernels_that_exist():
+    """The counters bench.py reports come from the tracked profiles by kernel name: every name is a kernel of the library as it is
+    built and has its row there."""
+    import subprocess
+    import sys
+
+    sys.path.insert(0, ROOT)
+    import bench
+
+    symbols = subprocess.run(["nm", "-C", LIB], check=True, stdout=subprocess.PIPE, text=True).stdout
+    built = set(re.findall(r"__device_stub__(\w+(?:<.*>)?)\(", symbols))
+    assert "three_nn_cells_kernel" in built
+    traffic = {k for kernels in bench.TRAFFIC_KERNELS.values() for k in kernels}
+    for names, path, column in ((traffic, bench.TRAFFIC_FILE, "FETCH_SIZE"), (set(bench.VALU_KERNELS.values()), bench.VALU_FILE, "VALUBusy")):
+        rows, commit = bench._profile_table(path, (column,))
+        assert commit
+        for kernel in names:
+            assert kernel in built, kernel
+            assert column in rows.get(kernel, {}), kernel
