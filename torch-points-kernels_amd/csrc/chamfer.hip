@@ -638,8 +638,8 @@ int chamfer_bwd(int b, int n, int m, const T* xyz1, const T* xyz2, const int32_t
 // Mean of the distances of both directions, added.  One workgroup for up to CHM_PER_BLOCK distances; for more, one per
 // CHM_PER_BLOCK of them up to CHM_BLOCKS, each leaving its share, and a workgroup behind them that adds the shares: every
 // sum is formed in float64 and in an order that depends on the sizes only.  The distances come from the cache the search
-// left them in (4 MB for 32 pairs of 16384 points), so the two launches are latency: 7 us, where two means and an
-// addition by torch took 17.
+// left them in (4 MB for 32 pairs of 16384 points), so the two launches are latency: kernels of 4.9 and 4.6 us, where two
+// means and an addition by torch took 17 us.
 constexpr int CHM_THREADS = 1024;
 constexpr int CHM_PER_BLOCK = 8 * CHM_THREADS;
 constexpr int CHM_BLOCKS = 256;

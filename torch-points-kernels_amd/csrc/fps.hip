@@ -631,10 +631,10 @@ constexpr int FPS_LIVE_CAPACITY = (FPS_MAX_CELLS + FPS_THREADS - 1) / FPS_THREAD
 // minimum is skipped (margin for rounding as in the register kernel), exactly.  Cell c belongs
 // to wavefront c mod 16 (neighbours on the curve go to different wavefronts): the wavefront
 // tests the boxes of its cells (one per lane and step), then updates the live ones - 64 points
-// per cell, a few cells' loads in flight together - and renews their LDS entries.  After a
-// Every wavefront then finds the best of its cells and the results are exchanged through LDS.
-// Several samples are taken per round, as in fps_pruned_kernel: after a round's updates the points with the
-// largest running minima follow each other as samples as long as none of them changes the next one's minimum.
+// per cell, a few cells' loads in flight together - and renews their LDS entries.  Every wavefront then
+// finds the best of its cells, and these are exchanged through LDS.
+// Several samples are taken per round: the points with the largest running minima follow each other as samples
+// as long as none of them changes the next one's minimum, which has to be above all that is not among them.
 // Here the order is by (minimum, then the reference's tie key), which is strict - equal minima need no separate
 // path - and a candidate's coordinates are at hand in LDS (the best point of its cell).  LDS also keeps every
 // cell's SECOND best point's minimum and key: what a wavefront does not publish - the best points of its other

@@ -836,7 +836,7 @@ at::Tensor gridding_batch_forward(const at::Tensor& ptcloud, double scale, at::T
     TORCH_CHECK(side > 0, "gridding: empty grid");
     at::Tensor grid = at::empty({b, side * side * side}, ptcloud.options());
     if (kept)
-        *kept = at::empty_like(ptcloud);
+        *kept = at::empty(ptcloud.sizes(), ptcloud.options()); // (contiguous, as ptcloud is)
     if (ptcloud.scalar_type() == at::kFloat)
         check_status(kept ? tpk_gridding_batch_keep_f32(b, n, scale, ptcloud.data_ptr<float>(), grid.data_ptr<float>(),
                                                         kept->data_ptr<float>(), current_stream(ptcloud))
@@ -859,7 +859,7 @@ at::Tensor gridding_batch_backward(const at::Tensor& ptcloud, double scale, cons
     TORCH_CHECK(grad_grid.scalar_type() == ptcloud.scalar_type(), "grad_grid and ptcloud differ in dtype");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(ptcloud.device());
     const int b = as_int(ptcloud.size(0), "batch size"), n = as_int(ptcloud.size(1), "number of points");
-    at::Tensor grad = at::empty_like(ptcloud);
+    at::Tensor grad = at::empty(ptcloud.sizes(), ptcloud.options());
     if (ptcloud.scalar_type() == at::kFloat)
         check_status(tpk_gridding_batch_grad_f32(b, n, scale, ptcloud.data_ptr<float>(), grad_grid.data_ptr<float>(),
                                                  grad.data_ptr<float>(), current_stream(ptcloud)),
