@@ -5,7 +5,7 @@
  * Every entry point takes plain device pointers and sizes, launches on the HIP stream
  * passed as `stream` (a hipStream_t cast to void*; NULL = the null stream), never
  * allocates, never synchronises the host (exceptions, documented below: tpk_grow_proximity,
- * tpk_grow_components, tpk_region_order and tpk_ball_query_sorted_partial_f32 with a workspace and nsample > 64) and keeps no state between calls
+ * tpk_grow_components, tpk_region_order, tpk_instance_counts_read and tpk_ball_query_sorted_partial_f32 with a workspace and nsample > 64) and keeps no state between calls
  * (exception: tpk_three_nn_static_f32, whose scratch memory is an array inside the library that all calls on a GPU
  * share).  The first call of a kernel on a device makes a few runtime calls on the host (the kernel's LDS limit;
  * for tpk_three_nn_static_f32 also the address of its array): a caller that captures HIP graphs makes one call

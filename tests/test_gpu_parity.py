@@ -1111,7 +1111,7 @@ def test_knn_parity(tpk, oracle, dev, B, n, m, k):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
-@pytest.mark.parametrize("kind", ["uniform", "normal", "clusters", "flat", "one_point", "lattice", "outlier", "outliers", "overflow", "queries_outside", "non_finite"])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "clusters", "flat", "one_point", "lattice", "outlier", "outliers", "scattered", "overflow", "queries_outside", "non_finite"])
 @pytest.mark.parametrize("B,n,m,k", [(2, 1, 3, 1), (2, 65, 40, 48), (1, 3000, 150, 49), (1, 8192, 200, 17), (2, 8193, 90, 48), (1, 40000, 60, 4)])
 def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
     # up to 48 neighbours: a grid in LDS (up to 8192 points) or in memory, its block of cells grown until it holds k, the
@@ -1137,6 +1137,9 @@ def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
         query[:, 0] = support[:, 0]
         query[:, 1] = support[:, n - 1] * 0.5
         query[:, 2] = -1e4
+    elif kind == "scattered":  # (trimmed twice; queries among the few points beyond the grid)
+        support[:, ::20] *= 100.0
+        query[:, ::3] *= 100.0
     elif kind == "overflow":  # finite coordinates whose range is not, on every axis
         support[:, n // 3] = 2e38
         support[:, n // 2] = -2e38
@@ -2147,7 +2150,7 @@ def _knn_steps(oracle, dev, support, query, k, workspace="grid"):
     return count.value / (64 * b * m)
 
 
-@pytest.mark.parametrize("kind", ["uniform", "normal", "flat", "outlier", "outliers", "queries_far", "queries_around"])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "flat", "outlier", "outliers", "scattered", "queries_far", "queries_around"])
 def test_knn_looks_at_few_points(oracle, dev, kind):
     """The searches over a grid look at a small part of the cloud, also where the queries lie far outside or the points are
     spread unevenly: 1 to 11 steps of 64 points per query on average, where a scan of the cloud takes 256 (in LDS 94)."""
@@ -2159,10 +2162,13 @@ def test_knn_looks_at_few_points(oracle, dev, kind):
         elif kind == "flat":
             support[..., 2] *= 1e-3
             query[..., 2] *= 1e-3
-        elif kind in ("outlier", "outliers"):
+        elif kind in ("outlier", "outliers", "scattered"):
             if n < 8192:
                 continue  # (in LDS nothing trims the grid: a scan of few points there)
-            support[:, n // 3] = 1000.0
+            if kind == "scattered":
+                support[:, ::20] *= 100.0
+            else:
+                support[:, n // 3] = 1000.0
             if kind == "outliers":
                 support[:, ::1000, 1] = -1e6
         elif kind == "queries_far":

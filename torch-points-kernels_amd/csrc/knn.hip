@@ -444,17 +444,18 @@ inline KnnGridLayout knn_grid_layout(int m, int cells)
     return l;
 }
 
-// Trims every axis of the grid's box, by one wavefront, to the cells outside which a 128th of the m points lies on either side
+// Trims every axis of the grid's box, by one wavefront, to the cells outside which a 16th of the m points lies on either side
 // (marginals: the points per cell along x, y, z).  The box before goes to `before`; *trimmed = whether it shrinks to KNG_KEPT or
-// less, otherwise `box` stays.  (A point sees 11 times an even cloud's points in its cell under a normal distribution, 20 to 30 times
-// in laser scans, hundreds in clusters: trimmed to a half from 8 times on, calls of theirs took up to twice as long.)
+// less, otherwise `box` stays.  With a 128th instead, clouds with 5 % of their points scattered widely stayed untrimmed: 2 x
+// 100000 of those 16.0 ms, this way 1.2.  (A point sees 11 times an even cloud's points in its cell under a normal distribution, 20
+// to 30 times in laser scans, hundreds in clusters: trimmed to a half from 8 times on, calls of theirs took up to twice as long.)
 constexpr float KNG_CROWDED = 32.0f; // a crowded cell's points, over those that a point of an even cloud sees in its cell
 constexpr float KNG_KEPT = 1.0f / 16.0f;
 constexpr int KNG_ZOOMS = 8; // times at most
 
 __device__ __forceinline__ void trim_box(const int* marginals, int m, const float* shape, int lane, int* box, int* before, int* trimmed)
 {
-    const int drop = m / 128;
+    const int drop = m / 16;
     float kept = 1.0f;
     int low[3], high[3];
     for (int a = 0; a < 3; ++a)
@@ -489,7 +490,7 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
     __shared__ int box[6], box_before[6]; // ordered ints: min x, y, z then max x, y, z; of the zoom before
     __shared__ float shape[LG_SHAPE];
     __shared__ int wave_totals[LG_WAVES];
-    __shared__ int crowded; // points in crowded cells
+    __shared__ int crowded, fullest; // points in crowded cells; in the fullest of them
     __shared__ int marginals[3 * KNG_AXIS], trimmed;
     constexpr int BATCH = 8; // points in flight per lane
     const int tid = threadIdx.x;
@@ -568,7 +569,7 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
     // the points lie in such cells, and most of the box holds hardly a point, the grid is laid over the rest of the box and its
     // outermost cells take what lies beyond.  8 x 16384 points, one of them at 1000 cloud sizes, k = 16: 2040 us, this way 232.
     const int crowd = static_cast<int>(KNG_CROWDED * (per_cell + 1.0f));
-    int crowded_before = m;
+    int fullest_before = m;
     for (int zooms = 0;; ++zooms)
     {
         if (wave == 0)
@@ -585,18 +586,17 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
         for (int c = tid; c < steps * LG_THREADS; c += LG_THREADS)
             reinterpret_cast<int4*>(kng_counts)[c] = make_int4(0, 0, 0, 0);
         if (tid == 0)
-            crowded = 0;
+            crowded = fullest = 0;
         __syncthreads();
         each([&](int, float x, float y, float z) { atomicAdd(&kng_counts[cell_of(x, y, z)], 1); });
         __syncthreads();
         int placed = 0; // points in the cells of the steps before
-        int in_crowds = 0;
         for (int step = 0; step < steps; ++step)
         {
             int4* const four = reinterpret_cast<int4*>(kng_counts) + step * LG_THREADS + tid;
             const int4 c4 = *four;
             const int own = c4.x + c4.y + c4.z + c4.w;
-            in_crowds += (c4.x > crowd ? c4.x : 0) + (c4.y > crowd ? c4.y : 0) + (c4.z > crowd ? c4.z : 0) + (c4.w > crowd ? c4.w : 0);
+            const int in_crowds = (c4.x > crowd ? c4.x : 0) + (c4.y > crowd ? c4.y : 0) + (c4.z > crowd ? c4.z : 0) + (c4.w > crowd ? c4.w : 0);
             const int before = wave_exclusive_sum(own);
             if (lane == TPK_WAVE - 1)
                 wave_totals[wave] = before + own;
@@ -612,19 +612,22 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
             s4.w = at += c4.z;
             *four = s4;
             reinterpret_cast<int4*>(starts)[step * LG_THREADS + tid] = s4; // (also those behind the last cell: the end)
-            if (step == steps - 1 && __ballot(in_crowds != 0) != 0 && in_crowds != 0)
+            if (in_crowds != 0)
+            {
                 atomicAdd(&crowded, in_crowds);
+                atomicMax(&fullest, max(max(c4.x, c4.y), max(c4.z, c4.w)));
+            }
             __syncthreads();
         }
         if (tid == 0)
             starts[steps * 4 * LG_THREADS] = m;
         // (from here on everything is the same for the whole workgroup)
-        const int crowded_now = crowded;
-        if (zooms > KNG_ZOOMS || crowded_now <= m / 2)
+        const int fullest_now = fullest;
+        if (zooms > KNG_ZOOMS || crowded <= m / 2)
             break;
-        if (zooms == KNG_ZOOMS || crowded_now > crowded_before)
+        if (zooms == KNG_ZOOMS || fullest_now > fullest_before)
         {
-            if (crowded_now <= crowded_before)
+            if (fullest_now <= fullest_before)
                 break;
             // the last zoom made it worse: back to the box before
             if (tid < 6)
@@ -633,7 +636,7 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
             __syncthreads();
             continue;
         }
-        crowded_before = crowded_now;
+        fullest_before = fullest_now;
         for (int c = tid; c < 3 * KNG_AXIS; c += LG_THREADS)
             marginals[c] = 0;
         __syncthreads();
