@@ -1381,6 +1381,25 @@ def test_fps_pools_at_the_edges_of_the_shapes(tpk, oracle, dev, n):
     np.testing.assert_array_equal(_np(got), oracle.furthest_point_sample(clouds.numpy(), npoint))
 
 
+@pytest.mark.parametrize("n", [64, 128, 129, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 16383])
+def test_fps_orders_a_whole_pool_at_once(tpk, oracle, dev, n):
+    """Sizes on both sides of every shape; a ball's surface and a sheet (points lowered inside the pool, where a round is cut),
+    a fine and a coarse lattice (equal minima inside a pool, and more of them than a pool takes), 40 places held by all
+    points (nothing above zero after 40 samples), clusters far apart (a floor far below the largest minimum)."""
+    g = torch.Generator().manual_seed(7 * n)
+    ball = torch.randn(n, 3, generator=g)
+    ball = ball / ball.norm(dim=1, keepdim=True) + 0.01 * torch.randn(n, 3, generator=g)
+    sheet = torch.rand(n, 3, generator=g) * torch.tensor([2.0, 1.0, 0.0]) + 0.2
+    fine = torch.randint(0, 50, (n, 3), generator=g) * 0.25 + 1.0
+    coarse = torch.randint(0, 9, (n, 3), generator=g) * 0.25 + 1.0
+    places = torch.rand(40, 3, generator=g)[torch.randint(0, 40, (n,), generator=g)] + 0.1
+    apart = torch.randint(0, 4, (n, 1), generator=g) * 50.0 + torch.rand(n, 3, generator=g) + 0.1
+    clouds = torch.stack([ball, sheet, fine, coarse, places, apart]).float()
+    npoint = min(n, 900)
+    got = tpk.furthest_point_sample(clouds.to(dev), npoint)
+    np.testing.assert_array_equal(_np(got), oracle.furthest_point_sample(clouds.numpy(), npoint))
+
+
 # ------------------------------------------------------------------ instance IoU
 
 

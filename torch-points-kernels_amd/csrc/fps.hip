@@ -2,11 +2,12 @@
 // the chosen set, pick the point whose distance is largest".
 //
 // One workgroup (one compute unit) owns a cloud for the whole call; the rounds of a cloud
-// depend on each other, so a call runs as many workgroups as there are clouds.  Three kernels
+// depend on each other, so a call runs as many workgroups as there are clouds.  Four kernels
 // by cloud size:
-//   up to 16384 points   fps_pool_kernel: up to 18 points per lane in registers, cloud ordered along
-//                        a space filling curve so that most updates can be skipped exactly; one
-//                        wavefront takes dozens of samples per round from a pool (described at the kernel);
+//   up to 256 points     fps_wave_kernel: one wavefront, a sample at a time;
+//   up to 16384 points   fps_pool_kernel: up to 16 points per lane in registers, cloud ordered along
+//                        a space filling curve so that most updates can be skipped exactly; dozens of
+//                        samples per round from a pool (described at the kernel);
 //   up to 163840 points  fps_cells_batched_kernel: the cloud ordered along the curve into cells of 64
 //                        points that stay in memory (the caller's workspace); boxes, largest
 //                        distance and best point of every cell in LDS; a round touches only
@@ -106,41 +107,42 @@ __device__ __forceinline__ bool eligible(float x, float y, float z)
 }
 
 // ---------------------------------------------------------------------------------------
-// Register-resident kernel with exact pruning and pools of samples, for clouds up to 16384 points.
+// Register-resident kernel with exact pruning and pools of samples, for clouds of 257 to 16384 points.
 //
-// Pools.  A round takes many samples.  After its updates let the pool be all points whose running
-// minimum lies above some floor; no point outside it holds more than the floor, and minima only
-// fall.  So as long as the largest minimum inside the pool lies above the floor, it is the largest
-// of the cloud, its point is the next sample, and only the pool's minima have to be brought up to date
-// to find the one after it.  A pool of at most 64 points is a lane each of ONE wavefront, and the
-// whole sequence runs in its registers: maximum over the lanes, the point's coordinates by lane
-// reads, one distance per lane - a chain of 40 dependent instructions, 0.1 us, without a barrier or
-// a trip to LDS.  On the clouds this was made for a pool of 44 gives about 31 samples.  (The version before
-// let every wavefront offer its two best points and took those that did not change each other: 8
-// samples per round, 0.37 us each; now 0.2.  Two points per lane in the pool would save two rounds of five and
-// cost every step a third more.)
+// Pools.  A round takes many samples.  Let the pool be all points whose running minimum lies above some
+// floor; no point outside it holds more than the floor, and minima only fall.  So as long as the largest
+// minimum inside the pool lies above the floor, it is the largest of the cloud and its point the next sample.
+// What the pool's points do to each other decides the whole sequence at once: in the order of their minima
+// (equal ones by the tie key) a point is taken unless one taken before it is closer to it than its minimum.
+// Every wavefront forms the distances of its share of the pool's pairs and leaves, per point, a mask of who would
+// lower it; then all points whose lowering points are decided are decided together, two or three passes of a dozen
+// scalar instructions.  A point lowered by those taken, but not to the floor, would have its turn again: the round
+// is cut where the largest of these stands, and what lies below waits for the next pool.  A pool of 54 gives about 38
+// samples.  (The version before let one wavefront take sample after sample, a chain of 40 dependent instructions
+// each, while the others updated: 31 samples per round, 0.1 us each.)
 //
-// Two kinds of wavefronts.  Wavefront 0 samples pools and holds no points.  The others hold the cloud,
-// PPT points per lane; while wavefront 0 samples they bring their points up to date with the samples
-// it has published so far (8 at a time, through LDS), and when it reports the end of the pool they gather
-// the next one.  What share below the largest minimum makes a pool of the wanted size is carried from round
-// to round; a pool that came out empty or too full is gathered again.
+// A round is: gather the pool in LDS; barrier; (if it holds more than 64, one wavefront picks the best 64; barrier;)
+// the pairs; barrier; decide, in every wavefront alike; update this wavefront's points with all samples.  What
+// share below the largest minimum makes a pool of the wanted size is carried from round to round.  At 16384 points a round
+// takes 13000 clocks: updates 5000, gathering 2200, waiting for the busiest wavefront 2000, the pool 4000.
+// 16 clouds of 16384 points, 4096 samples: 853 -> 602 us (uneven clouds 938 -> 725); 4096 points 235 -> 158, 1024 85 -> 63.
 //
 // Pruning.  A point's running minimum changes only if its distance to the new sample is smaller
-// than that minimum, and no minimum exceeds the one the round's first sample held.  So a set of
+// than that minimum, and no minimum exceeds the one the sample held.  So a set of
 // points whose bounding box is further from the sample than the square root of that value cannot
 // change, and its update can be skipped without changing any result.  To make such sets exist, the
 // kernel first orders the cloud along a Hilbert curve (12-bit position of its cell in a 16^3 grid,
 // counting sort in LDS) and cuts the curve into cells of 64 * GS consecutive points.  A cell is GS
 // registers of the 64 lanes of one wavefront; cells go round-robin to the wavefronts, so the cells around a
-// sample belong to different ones.  A wavefront tests its up to 8 boxes against 8 samples at
-// once, a lane per pair, and updates only what is reached (wave-uniform branches).  The fp32 box
-// distance is compared with a relative margin of 2e-6, several times the rounding error of either
-// side, so a skipped update is provably a no-op.
+// sample belong to different ones.  A wavefront tests its boxes against all samples of a round, a lane each, and updates
+// only what is reached.  The fp32 box distance is compared with a relative margin of 3e-6, several times the rounding error
+// of either side, so a skipped update is provably a no-op.  (Cells of 64, 128, 256 points: 749 / 612 / 603 us on even clouds,
+// 806 / 736 / 720 on uneven ones at 16384 points, 181 / 169 / 174 and 193 / 186 / 213 at 4096.)
 //
-// Equal maxima inside a pool go by the reference's tie key.  When more points hold the same value than
-// a pool takes, when nothing above zero is left, or when a coordinate is not finite (such a point never
-// falls to zero), rounds take one sample by the tie key over all points holding the maximum.
+// One sample per round.  The first samples drop so many minima that a pool gives one to four of them; and when more
+// points hold the same value than a pool takes, when nothing above zero is left, or when a coordinate is not finite
+// (such a point never falls to zero), a pool gives none.  Then every wavefront offers its best point, one barrier, and all
+// find the best of those.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ unsigned tie_key(int k, int log2_bs, int ref_groups)
 {
@@ -149,13 +151,6 @@ __device__ __forceinline__ unsigned tie_key(int k, int log2_bs, int ref_groups)
     return rev * static_cast<unsigned>(ref_groups) + (static_cast<unsigned>(k) >> log2_bs);
 }
 
-// The words of LDS through which the wavefronts of a workgroup agree on a round's winner.
-struct RoundWords
-{
-    int max_val;      // atomic max of the running minima (bit patterns), starts at INT_MIN
-    unsigned min_tie; // atomic min of the tie keys of the points holding max_val
-};
-
 // LDS atomics without return value, issued as written: one instruction for the active lanes
 // (the compiler would otherwise wrap a same-address atomic in a loop over those lanes).
 __device__ __forceinline__ unsigned lds_offset(const void* p)
@@ -163,9 +158,9 @@ __device__ __forceinline__ unsigned lds_offset(const void* p)
     return static_cast<unsigned>(reinterpret_cast<unsigned long long>(
         (const __attribute__((address_space(3))) char*)p));
 }
-__device__ __forceinline__ void lds_atomic_max_i32(int* p, int v)
+__device__ __forceinline__ void lds_or_u32(unsigned* p, unsigned v)
 {
-    asm volatile("ds_max_i32 %0, %1" ::"v"(lds_offset(p)), "v"(v) : "memory");
+    asm volatile("ds_or_b32 %0, %1" ::"v"(lds_offset(p)), "v"(v) : "memory");
 }
 
 // Largest value of the wavefront as a scalar: DPP maxima inside the rows of 16 lanes, then from row to row; six
@@ -181,47 +176,63 @@ __device__ __forceinline__ int wave_max_to_scalar(int v)
     return __builtin_amdgcn_readlane(v, TPK_WAVE - 1);
 }
 
-// Position on the sorted curve of member `e` of group `g` held by lane `lane` of worker `worker`.
-template <int WORKERS, int GS>
-__device__ __forceinline__ int sorted_position(int g, int worker, int e, int lane)
+// `v`, of which the compiler shall not know that it stays the same: what is computed from it is computed where it is used
+// instead of once before the loop and kept in registers that the points need.
+__device__ __forceinline__ int not_hoisted(int v)
 {
-    return ((g * WORKERS + worker) * GS + e) * TPK_WAVE + lane;
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
-constexpr int POOL_CAPACITY = 2 * TPK_WAVE; // points gathered at most; the best 64 are sampled
-constexpr int POOL_TARGET = 60;
-constexpr int POOL_TRIES = 8;
-constexpr int POOL_BATCH = 8;   // samples published at a time: one per lane of a row of 8
-constexpr int POOL_DONE = 1 << 16;
+// Position on the sorted curve of member `e` of group `g` held by lane `lane` of wavefront `wave`.
+template <int WAVES, int GS>
+__device__ __forceinline__ int sorted_position(int g, int wave, int e, int lane)
+{
+    return ((g * WAVES + wave) * GS + e) * TPK_WAVE + lane;
+}
 
-// ORDERED: the cloud is ordered along the curve and updates are pruned.  Small clouds are taken as they come: all their
-// points can be brought up to date in less time than a sample takes, and the ordering alone is 8 us.
+constexpr int POOL_CAPACITY = 4 * TPK_WAVE; // points gathered at most; the best 64 are sampled
+constexpr int POOL_TARGET = 64;             // (56, 64, 72, 84: 611 / 603 / 601 / 606 us at 16384 points)
+constexpr int POOL_TRIES = 12;
+
+// ORDERED: the cloud is ordered along the curve and updates are pruned.  Small clouds are taken as they come.
 template <int PPT, int WAVES, int GS, bool ORDERED>
 __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
     int n, int npoint, int log2_bs, int ref_groups, int key_capacity,
     const float* __restrict__ xyz, int32_t* __restrict__ out)
 {
     constexpr int THREADS = WAVES * TPK_WAVE;
-    constexpr int WORKERS = WAVES - 1;
     constexpr int NG = PPT / GS;
-    static_assert(NG * GS == PPT && NG * POOL_BATCH <= TPK_WAVE, "a row of 8 lanes tests each group");
+    // samples taken one by one before the first pool (1, 8, 16, 32: 74 / 72 / 69 / 71 us for 256 of 1024 points, 625 / 610 / 606 /
+    // 611 for 4096 of 16384; 2048 points 102 / 98 / 102 / 106)
+    constexpr int OPENING = ORDERED && PPT <= 2 ? 8 : 16;
+    constexpr int ROWS = TPK_WAVE / WAVES; // rows of the pool's relation that a wavefront works out
+    static_assert(PPT <= 16 && NG * GS == PPT && ROWS * WAVES == TPK_WAVE && ROWS % 4 == 0, "whole groups, whole rows");
     // key_capacity keys (curve position << 20) | index in curve order, kept for the whole kernel; then, during
     // set-up, key_capacity unsorted keys and the bins of the counting sort
-    extern __shared__ unsigned sort_keys[];
+    extern __shared__ __align__(16) unsigned sort_keys[];
     unsigned* const unsorted = sort_keys + key_capacity;
     int* const bins = reinterpret_cast<int*>(unsorted + key_capacity); // CURVE_BINS words
     __shared__ int wave_totals[WAVES];
-    __shared__ RoundWords words[2];
     __shared__ int cloud_box[6];      // ordered ints: min x,y,z then max x,y,z
-    __shared__ __align__(16) float4 group_lo[WORKERS * NG], group_hi[WORKERS * NG]; // box of every (worker, group) cell
-    __shared__ __align__(16) float4 pool[POOL_CAPACITY]; // x, y, z, sorted position of the pool's points
-    __shared__ int pool_min[POOL_CAPACITY];              // their running minima
-    __shared__ int pool_count[3];                   // one per attempt, in turn
-    __shared__ __align__(16) float4 taken[TPK_WAVE]; // the round's samples
-    // By round: how many of them stand in taken[] (POOL_DONE: there will be no more), the first one's minimum,
-    // what no minimum exceeds when all their updates are made; last the exclusive or of the three.
-    __shared__ __align__(16) int4 published[2];
-    __shared__ int pool_best[TPK_WAVE]; // where its best 64 stand, if it holds more
+    __shared__ __align__(16) float4 group_lo[WAVES * NG], group_hi[WAVES * NG]; // box of every (wavefront, group) cell
+    // The pool's points (x, y, z, running minimum) and their places on the curve, rounds in turn: where the ordering had
+    // its unsorted keys
+    __shared__ __align__(16) float4 pool_room[ORDERED ? 1 : 2 * POOL_CAPACITY];
+    __shared__ int pool_place_room[ORDERED ? 1 : 2 * POOL_CAPACITY];
+    float4* const pools = ORDERED ? reinterpret_cast<float4*>(unsorted) : pool_room;
+    int* const pool_places = ORDERED ? reinterpret_cast<int*>(pools + 2 * POOL_CAPACITY) : pool_place_room;
+    static_assert(2 * POOL_CAPACITY * (sizeof(float4) + sizeof(int)) <= CURVE_BINS * sizeof(int), "room for the pools");
+    __shared__ __align__(16) float4 best[TPK_WAVE];      // the same of its best 64, if it holds more
+    __shared__ int best_place[TPK_WAVE];
+    __shared__ __align__(8) int2 best_of;                // how many they are, what they lie above
+    __shared__ int pool_count[3];                        // one per attempt, in turn
+    __shared__ __align__(8) uint2 pool_blockers[TPK_WAVE]; // per pool point: who, taken before it, lowers it
+    __shared__ __align__(8) uint2 pool_before[TPK_WAVE];   // per pool point: who comes before it
+    __shared__ __align__(8) uint2 pool_keepers[TPK_WAVE];  // per pool point with a bit in keeps[]: who lowers it, but not out of the pool
+    __shared__ __align__(8) unsigned keeps[2][2];          // rounds in turn
+    __shared__ __align__(16) float4 offers[2][WAVES]; // every wavefront's best point (x, y, z, running minimum), rounds in turn
+    __shared__ int offer_places[2][WAVES];            // and its place on the curve
     __shared__ int not_finite;
 
     xyz += static_cast<int64_t>(blockIdx.x) * n * 3;
@@ -229,17 +240,13 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & (TPK_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
-    const int worker = wave - 1;
     auto original_index = [&](int position) { return ORDERED ? static_cast<int>(sort_keys[position] & 0x3FFFu) : position; };
 
     // ---- set-up 1 and 2: order the cloud along the curve (curve_order.h)
-    if (tid < 2)
-    {
-        words[tid] = RoundWords{INT_MIN, 0xFFFFFFFFu};
-        published[tid] = int4{0, 0, 0, 0};
-    }
     if (tid < 3)
         pool_count[tid] = 0;
+    if (tid < 4)
+        keeps[tid / 2][tid % 2] = 0;
     if (tid == 0)
         not_finite = 0;
     if constexpr (ORDERED)
@@ -248,129 +255,191 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
         __syncthreads();
 
     // ---- set-up 3: this lane's points.  The curve is cut into cells of 64 * GS consecutive
-    // points; cell c belongs to worker c % WORKERS as its group c / WORKERS.  Slot i of a lane =
+    // points; cell c belongs to wavefront c % WAVES as its group c / WAVES.  Slot i of a lane =
     // group (i / GS), member (i % GS); see sorted_position().
     float x[PPT], y[PPT], z[PPT];
     int t[PPT];
+    bool finite = true;
 #pragma unroll
-    for (int gi = 0; gi < NG; ++gi)
+    for (int i = 0; i < PPT; ++i)
     {
-        float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
-        float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+        const int q = sorted_position<WAVES, GS>(i / GS, wave, i % GS, lane);
+        const int k = original_index(q < n ? q : 0);
+        x[i] = xyz[k * 3 + 0];
+        y[i] = xyz[k * 3 + 1];
+        z[i] = xyz[k * 3 + 2];
+    }
 #pragma unroll
-        for (int e = 0; e < GS; ++e)
-        {
-            const int i = gi * GS + e;
-            const int q = worker >= 0 ? sorted_position<WORKERS, GS>(gi, worker, e, lane) : n;
-            const int k = original_index(q < n ? q : 0);
-            const float px = xyz[k * 3 + 0], py = xyz[k * 3 + 1], pz = xyz[k * 3 + 2];
-            const bool ok = q < n && eligible(px, py, pz);
-            if (ok && !(px - px == 0.f && py - py == 0.f && pz - pz == 0.f))
-                not_finite = 1;
-            x[i] = ok ? px : 0.f;
-            y[i] = ok ? py : 0.f;
-            z[i] = ok ? pz : 0.f;
-            t[i] = ordered_bits(ok ? 1e10f : -1.0f);
-            lo[0] = ok ? fminf(lo[0], px) : lo[0];
-            lo[1] = ok ? fminf(lo[1], py) : lo[1];
-            lo[2] = ok ? fminf(lo[2], pz) : lo[2];
-            hi[0] = ok ? fmaxf(hi[0], px) : hi[0];
-            hi[1] = ok ? fmaxf(hi[1], py) : hi[1];
-            hi[2] = ok ? fmaxf(hi[2], pz) : hi[2];
-        }
-        if constexpr (!ORDERED)
-            continue;
-        // the cell belongs to this wavefront alone: reduce over its lanes, plain store
+    for (int i = 0; i < PPT; ++i)
+    {
+        const bool ok = sorted_position<WAVES, GS>(i / GS, wave, i % GS, lane) < n && eligible(x[i], y[i], z[i]);
+        finite = finite && (!ok || (x[i] - x[i] == 0.f && y[i] - y[i] == 0.f && z[i] - z[i] == 0.f));
+        t[i] = ordered_bits(ok ? 1e10f : -1.0f);
+    }
+    if (!finite)
+        not_finite = 1;
+    if constexpr (ORDERED)
+    {
+        // a cell belongs to this wavefront alone: reduce over its lanes, plain store
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
+        for (int gi = 0; gi < NG; ++gi)
         {
-            lo[a] = ordered_int_to_float(wave_min_i32(float_to_ordered_int(lo[a])));
-            hi[a] = ordered_int_to_float(wave_max_i32(float_to_ordered_int(hi[a])));
-        }
-        if (lane == 0 && worker >= 0)
-        {
-            group_lo[worker * NG + gi] = make_float4(lo[0], lo[1], lo[2], 0.f);
-            group_hi[worker * NG + gi] = make_float4(hi[0], hi[1], hi[2], 0.f);
+            float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
+            float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+#pragma unroll
+            for (int e = 0; e < GS; ++e)
+            {
+                const int i = gi * GS + e;
+                const bool ok = t[i] >= 0;
+                lo[0] = ok ? fminf(lo[0], x[i]) : lo[0];
+                lo[1] = ok ? fminf(lo[1], y[i]) : lo[1];
+                lo[2] = ok ? fminf(lo[2], z[i]) : lo[2];
+                hi[0] = ok ? fmaxf(hi[0], x[i]) : hi[0];
+                hi[1] = ok ? fmaxf(hi[1], y[i]) : hi[1];
+                hi[2] = ok ? fmaxf(hi[2], z[i]) : hi[2];
+            }
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+            {
+                lo[a] = ordered_int_to_float(wave_min_i32(float_to_ordered_int(lo[a])));
+                hi[a] = ordered_int_to_float(wave_max_i32(float_to_ordered_int(hi[a])));
+            }
+            // a cell without points that take part: a box at infinity, which nothing reaches
+            if (lane == 0)
+            {
+                const bool none = !(lo[0] <= hi[0]);
+                group_lo[wave * NG + gi] = none ? make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.f) : make_float4(lo[0], lo[1], lo[2], 0.f);
+                group_hi[wave * NG + gi] = none ? make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.f) : make_float4(hi[0], hi[1], hi[2], 0.f);
+            }
         }
     }
-    __syncthreads();
     const float p0x = xyz[0], p0y = xyz[1], p0z = xyz[2];
     if (tid == 0)
-    {
         out[0] = 0;
-        taken[0] = make_float4(p0x, p0y, p0z, 0.f);
-    }
-    const bool one_by_one = __builtin_amdgcn_readfirstlane(not_finite) != 0;
     __syncthreads();
+    const bool one_by_one = __builtin_amdgcn_readfirstlane(not_finite) != 0;
     TPK_WORK_DECL
 
-    // The updates of samples first .. first + count - 1 (at most POOL_BATCH) of taken[]; `bound`: no running minimum
-    // exceeds it.  (Bit patterns of non-negative floats throughout.)
-    auto update = [&](int first, int count, int bound) __attribute__((always_inline)) {
-        // row r of 8 lanes tests this wavefront's group r, its lane k against sample k
-        const int k = lane % POOL_BATCH, group = lane / POOL_BATCH, cell = worker * NG + (group < NG ? group : 0);
-        const float4 s = taken[first + (k < count ? k : 0)];
+    // The updates of the samples held by the lanes of `mask`, a lane each (and by samples[lane] in LDS); `bound`: no running
+    // minimum exceeds it when that sample is taken.  (Bit patterns of non-negative floats throughout.)
+    auto update = [&](float px, float py, float pz, int bound, unsigned long long mask, const float4* samples) __attribute__((always_inline)) {
+        // (two parts in a million and more above the bound: several times the rounding error of either side)
+        const float limit = __int_as_float(bound) * 1.000003f;
+        int cells = wave * NG;
+        unsigned long long reach[NG]; // who reaches a group
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi)
+        {
+            reach[gi] = mask;
+            if constexpr (ORDERED)
+            {
+                if (gi > 0 && gi % 4 == 0) // (four boxes in registers at a time)
+                    asm volatile("" : "+s"(cells) : "s"(reach[gi - 1]));
+                const float4 lo = group_lo[cells + gi], hi = group_hi[cells + gi];
+                const float dx = px - __builtin_amdgcn_fmed3f(px, lo.x, hi.x);
+                const float dy = py - __builtin_amdgcn_fmed3f(py, lo.y, hi.y);
+                const float dz = pz - __builtin_amdgcn_fmed3f(pz, lo.z, hi.z);
+                const float lb = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+                // (a box at infinity: lb = +inf, never live; NaN compares false -> live)
+                reach[gi] = __ballot(!(lb >= limit)) & mask;
+            }
+        }
         if constexpr (!ORDERED)
         {
-            for (int from = 0; from < count; ++from)
+            // (two samples at a time; every group is reached by all)
+            for (unsigned long long left = mask; left != 0; left &= left - 1)
             {
-                const float sx = to_vector_register(tpk_read_lane(s.x, from)), sy = to_vector_register(tpk_read_lane(s.y, from));
-                const float sz = to_vector_register(tpk_read_lane(s.z, from));
-                TPK_WORK_ADD(PPT);
+                const int first = __builtin_ctzll(left);
+                left &= left - 1;
+                const float4 s = samples[first], r = samples[left != 0 ? __builtin_ctzll(left) : first];
+                TPK_WORK_ADD(2 * PPT);
 #pragma unroll
                 for (int i = 0; i < PPT; ++i)
-                    t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], sx, sy, sz)));
+                    t[i] = min(min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], s.x, s.y, s.z))), ordered_bits(tpk_dist2(x[i], y[i], z[i], r.x, r.y, r.z)));
             }
             return;
         }
-        const float4 lo = group_lo[cell], hi = group_hi[cell];
-        const float dx = fmaxf(fmaxf(lo.x - s.x, s.x - hi.x), 0.f);
-        const float dy = fmaxf(fmaxf(lo.y - s.y, s.y - hi.y), 0.f);
-        const float dz = fmaxf(fmaxf(lo.z - s.z, s.z - hi.z), 0.f);
-        const float lb = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)) * 0.999998f;
-        // an empty box gives lb = +inf (never live); NaN compares false -> live
-        const unsigned long long live = __ballot(k < count && group < NG && !(lb >= __int_as_float(bound)));
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi)
-            for (unsigned reach = static_cast<unsigned>(live >> (gi * POOL_BATCH)) & 0xFFu; reach != 0; reach &= reach - 1)
+            for (unsigned long long left = reach[gi]; left != 0; left &= left - 1)
             {
-                const int from = __builtin_ctz(reach); // (lanes 0 .. 7 hold samples 0 .. 7)
-                const float sx = to_vector_register(tpk_read_lane(s.x, from)), sy = to_vector_register(tpk_read_lane(s.y, from));
-                const float sz = to_vector_register(tpk_read_lane(s.z, from));
+                float4 s = samples[__builtin_ctzll(left)];
+                asm volatile("" : "+v"(s.w));
                 TPK_WORK_ADD(GS);
 #pragma unroll
                 for (int e = 0; e < GS; ++e)
                 {
                     const int i = gi * GS + e;
-                    t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], sx, sy, sz)));
+                    t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], s.x, s.y, s.z)));
                 }
             }
     };
-    if (worker >= 0)
-        update(0, 1, ordered_bits(__builtin_inff()));
+    // The same for one sample: a lane tests each group.
+    auto update_one = [&](const float4 s, int bound) __attribute__((always_inline)) {
+        unsigned long long reach = ~0ull;
+        if constexpr (ORDERED)
+        {
+            const int cell = wave * NG + (lane < NG ? lane : 0);
+            const float4 lo = group_lo[cell], hi = group_hi[cell];
+            const float dx = s.x - __builtin_amdgcn_fmed3f(s.x, lo.x, hi.x);
+            const float dy = s.y - __builtin_amdgcn_fmed3f(s.y, lo.y, hi.y);
+            const float dz = s.z - __builtin_amdgcn_fmed3f(s.z, lo.z, hi.z);
+            reach = __ballot(!(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)) >= __int_as_float(bound) * 1.000003f));
+        }
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi)
+            if ((reach >> gi & 1ull) != 0ull)
+            {
+                TPK_WORK_ADD(GS);
+#pragma unroll
+                for (int e = 0; e < GS; ++e)
+                {
+                    const int i = gi * GS + e;
+                    t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], s.x, s.y, s.z)));
+                }
+            }
+    };
+    update_one(make_float4(p0x, p0y, p0z, 0.f), ordered_bits(__builtin_inff()));
 
     int most_left = 0;       // no running minimum exceeds this
-    float gap = 0.1f;        // the pool takes what lies within this share below it
-    int pause = 1, penalty = 1; // rounds to take one by one; the first finds the largest minimum
-    int which = 0, attempt = 0, round = 0;
+    // the pool takes what lies above this much less than it, in bit patterns: 2^23 is a factor of two
+    int gap = 1 << 21;
+    int pause = OPENING, penalty = 1; // samples to take one by one
+    int attempt = 0, par = 0, turn = 0;
+    bool keyed = false;
     int j = 1;
     while (j < npoint)
     {
+        float4* const pool = pools + par * POOL_CAPACITY;
+        int* const pool_place = pool_places + par * POOL_CAPACITY;
         // 1. the pool: all points whose minimum lies above `floor_bits`, at most 64
+        // Every wavefront reads ROWS of its points, a row of 16 lanes each, and all 64, 16 at a time.
+        constexpr int CHUNKS = TPK_WAVE / 16, PASSES = ROWS / 4;
+        float4 other[CHUNKS], mine[PASSES];
+        auto read_points = [&](const float4* points) __attribute__((always_inline)) {
+#pragma unroll
+            for (int c = 0; c < CHUNKS; ++c)
+                other[c] = points[c * 16 + lane % 16];
+#pragma unroll
+            for (int p = 0; p < PASSES; ++p)
+                mine[p] = points[wave * ROWS + p * 4 + lane / 16];
+        };
         int count = 0, floor_bits = 0;
         bool pooled = false;
         const bool paused = pause > 0 || one_by_one;
         if (paused)
             --pause;
         else
-            for (int tries = 0; tries < POOL_TRIES && !pooled; ++tries)
+        {
+            int narrow = 0, wide = 0; // gaps that gave no point, and too many
+            for (int tries = 0; tries < POOL_TRIES; ++tries)
             {
-                floor_bits = ordered_bits(fmaxf(__int_as_float(most_left) * (1.0f - gap), 0.f));
+                floor_bits = max(most_left - gap, 0);
                 if (floor_bits >= most_left)
                     break; // nothing above zero, or more equal minima than a pool holds
                 const int slot = attempt % 3;
-                if (worker >= 0)
                 {
+                    const int own_lane = not_hoisted(lane);
                     unsigned long long above[PPT];
                     int own = 0;
 #pragma unroll
@@ -389,20 +458,22 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
                         {
 #pragma unroll
                             for (int i = 0; i < PPT; ++i)
-                                if (above[i] != 0)
+                            {
                                 {
                                     if (t[i] > floor_bits)
                                     {
                                         const int to = at + static_cast<int>(tpk_prefix_count(above[i]));
-                                        pool[to] = make_float4(x[i], y[i], z[i], __int_as_float(sorted_position<WORKERS, GS>(i / GS, worker, i % GS, lane)));
-                                        pool_min[to] = t[i];
+                                        pool[to] = make_float4(x[i], y[i], z[i], __int_as_float(t[i]));
+                                        pool_place[to] = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
                                     }
                                     at += __builtin_popcountll(above[i]);
                                 }
+                            }
                         }
                     }
                 }
                 lds_barrier();
+                read_points(pool);
                 count = __builtin_amdgcn_readfirstlane(pool_count[slot]);
                 if (tid == 0)
                     pool_count[(attempt + 2) % 3] = 0; // (the one before: everybody has read it)
@@ -410,207 +481,415 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
                 pooled = count > 0 && count <= POOL_CAPACITY;
                 if (count == 0 && floor_bits == 0)
                     break; // nothing above zero
-                const float wanted = count == 0 ? 2.0f : static_cast<float>(POOL_TARGET) / static_cast<float>(count);
-                gap *= pooled ? fminf(fmaxf(wanted, 0.5f), 2.0f) : fmaxf(wanted, 0.02f);
+                if (pooled)
+                    break;
+                // the next gap: the number of points grows with the gap, and more than in proportion if it is far off
+                if (count == 0)
+                {
+                    narrow = gap;
+                    gap = wide > 0 ? narrow + (wide - narrow) / 2 : min(gap, 1 << 28) * 4;
+                }
+                else
+                {
+                    wide = gap;
+                    if (count > 8 * POOL_CAPACITY)
+                    {
+                        // (most likely equal minima: a sample by itself tells where the largest one is)
+                        gap = max(gap >> 3, 1 << 12);
+                        break;
+                    }
+                    const float share = __builtin_amdgcn_sqrtf(static_cast<float>(POOL_TARGET) * __builtin_amdgcn_rcpf(static_cast<float>(count)));
+                    const int next = __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<float>(gap) * share));
+                    gap = narrow > 0 ? max(next, narrow + (wide - narrow) / 2) : next;
+                }
             }
+        }
         if (pooled)
         {
-            const int par = round & 1;
-            int taken_now = 0; // (none: more than 64 hold the largest minimum)
-            ++round;
-            if (wave == 0)
+            const float4* points = pool;
+            const int* places = pool_place;
+            const int found = count;
+            if (count > TPK_WAVE)
             {
-                // 2a. the samples, one after the other (what a step costs is its instructions, a chain of dependent
-                // ones; the others' work goes into its gaps).  A point taken falls to zero, so a step takes a new one.
-                __builtin_amdgcn_s_setprio(3);
-                int at = lane < count ? lane : 0, left = lane < count ? pool_min[lane] : INT_MIN;
-                int number = -1; // this lane's point was the number-th to be taken
-                if (count > TPK_WAVE)
+                if (wave == 0)
                 {
-                    // a floor that leaves at most 64, and not many fewer if that can be had: between the pool's own (more)
-                    // and its largest minimum (none), first where they would lie if they were evenly spread
-                    const int second = lane + TPK_WAVE < count ? pool_min[lane + TPK_WAVE] : INT_MIN;
-                    int high = wave_max_to_scalar(max(left, second)), low = floor_bits;
-                    unsigned long long first_ones = 0ull, second_ones = 0ull;
-                    int share = (TPK_WAVE - 4) * 256 / count;
-                    for (int tries = 0; tries < 6; ++tries)
+                    // A floor that leaves at most 64, and not many fewer if that can be had: between the pool's own (more)
+                    // and its largest minimum (none).
+                    const int own_lane = not_hoisted(lane);
+                    int v[POOL_CAPACITY / TPK_WAVE], most = INT_MIN;
+                    unsigned long long kept[POOL_CAPACITY / TPK_WAVE] = {};
+#pragma unroll
+                    for (int u = 0; u < POOL_CAPACITY / TPK_WAVE; ++u)
                     {
+                        v[u] = u * TPK_WAVE + own_lane < count ? __float_as_int(pool[u * TPK_WAVE + own_lane].w) : INT_MIN;
+                        most = max(most, v[u]);
+                    }
+                    int high = wave_max_to_scalar(most), low = floor_bits, share = (TPK_WAVE - 6) * 256 / count;
+                    count = 0;
+                    for (int tries = 0; tries < 10; ++tries)
+                    {
+                        // (first where they would lie if they were evenly spread)
                         const int middle = high - static_cast<int>(static_cast<long long>(high - low) * share / 256);
-                        const unsigned long long f = __ballot(left > middle), g = __ballot(second > middle);
-                        const int have = __builtin_popcountll(f) + __builtin_popcountll(g);
+                        share = 128;
+                        unsigned long long above[POOL_CAPACITY / TPK_WAVE];
+                        int have = 0;
+#pragma unroll
+                        for (int u = 0; u < POOL_CAPACITY / TPK_WAVE; ++u)
+                        {
+                            above[u] = __ballot(v[u] > middle);
+                            have += __builtin_popcountll(above[u]);
+                        }
                         if (have > TPK_WAVE)
                             low = middle;
                         else
                         {
                             high = middle;
-                            first_ones = f;
-                            second_ones = g;
-                            if (have >= TPK_WAVE - 12)
+                            count = have;
+#pragma unroll
+                            for (int u = 0; u < POOL_CAPACITY / TPK_WAVE; ++u)
+                                kept[u] = above[u];
+                            if (have >= TPK_WAVE - 7)
                                 break;
                         }
-                        share = 128;
                     }
-                    floor_bits = high;
-                    count = __builtin_popcountll(first_ones) + __builtin_popcountll(second_ones); // 0: too many are equal
-                    if (left > floor_bits && count > 0)
-                        pool_best[tpk_prefix_count(first_ones)] = lane;
-                    if (second > floor_bits && count > 0)
-                        pool_best[__builtin_popcountll(first_ones) + tpk_prefix_count(second_ones)] = lane + TPK_WAVE;
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    at = lane < count ? pool_best[lane] : 0;
-                    left = lane < count ? pool_min[at] : INT_MIN;
-                }
-                const float4 rec = pool[at];
-                int most = wave_max_to_scalar(left), now = 0;
-                const int top = most;
-                if (lane == 0)
-                    published[par ^ 1] = int4{0, 0, 0, 0}; // (the round before: everybody has left it)
-                auto publish = [&](int from, int flags) __attribute__((always_inline)) {
-                    if (number >= from)
-                        taken[number] = rec;
-                    // (a wavefront's LDS accesses are executed in order: nothing to wait for)
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    if (lane == 0)
-                        published[par] = int4{now | flags, top, floor_bits, (now | flags) ^ top ^ floor_bits};
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                };
-                while (true)
-                {
-                    const int from = now;
+                    int to = 0;
 #pragma unroll
-                    for (int u = 0; u < POOL_BATCH; ++u)
-                        if (__builtin_expect(most > floor_bits, 1))
+                    for (int u = 0; u < POOL_CAPACITY / TPK_WAVE; ++u)
+                    {
+                        if (v[u] > high && count > 0) // (0 left: too many are equal)
                         {
-                            unsigned long long holders = __ballot(left == most);
-                            if (__builtin_expect(__builtin_popcountll(holders) != 1, 0))
-                            {
-                                const unsigned key = left == most ? tie_key(original_index(__float_as_int(rec.w)), log2_bs, ref_groups) : 0xFFFFFFFFu;
-                                holders = __ballot(key == wave_min_u32(key));
-                            }
-                            const int l = __builtin_ctzll(holders);
-                            const float d = tpk_dist2(rec.x, rec.y, rec.z, tpk_read_lane(rec.x, l), tpk_read_lane(rec.y, l), tpk_read_lane(rec.z, l));
-                            number = lane == l ? now : number;
-                            left = min(left, ordered_bits(d));
-                            ++now;
-                            most = wave_max_to_scalar(left);
+                            best[to + tpk_prefix_count(kept[u])] = pool[u * TPK_WAVE + own_lane];
+                            best_place[to + tpk_prefix_count(kept[u])] = pool_place[u * TPK_WAVE + own_lane];
                         }
-                    if (most <= floor_bits)
-                    {
-                        publish(from, POOL_DONE);
-                        break;
+                        to += __builtin_popcountll(kept[u]);
                     }
-                    publish(from, 0);
+                    if (lane == 0)
+                        best_of = int2{count, high};
                 }
-                __builtin_amdgcn_s_setprio(0);
-                if (number >= 0 && j + number < npoint)
-                    out[j + number] = original_index(__float_as_int(rec.w));
-                taken_now = now;
+                lds_barrier();
+                read_points(best);
+                const int2 trimmed = best_of;
+                count = __builtin_amdgcn_readfirstlane(trimmed.x);
+                floor_bits = __builtin_amdgcn_readfirstlane(trimmed.y);
+                points = best;
+                places = best_place;
             }
-            else
+            if (count > 0) // (0: more equal minima at the top than a pool takes)
             {
-                // 2b. meanwhile the updates of the samples published so far
-                const volatile int4* const word = &published[par];
-                int seen = 0;
-                while (true)
+                const unsigned long long everyone = ~0ull >> (TPK_WAVE - count);
+                const int own_lane = not_hoisted(lane);
+                // 3. its relation.  Point i comes before point r if it holds more (or as much, with a smaller tie key); it
+                // lowers r if it is closer than what r holds, and keeps it in the pool if it is further than the floor.
+                // (Bits of a ballot: four rows of 16 points.)
+#pragma unroll
+                for (int p = 0; p < PASSES; ++p)
                 {
-                    const int state = __builtin_amdgcn_readfirstlane(word->x), top = __builtin_amdgcn_readfirstlane(word->y);
-                    const int floor_now = __builtin_amdgcn_readfirstlane(word->z);
-                    if ((state ^ top ^ floor_now) != __builtin_amdgcn_readfirstlane(word->w))
-                        continue; // (read while it was being written)
-                    floor_bits = floor_now;
-                    const int ready = state & (POOL_DONE - 1);
-                    if (seen < ready)
+                    const int row = wave * ROWS + p * 4;
+                    const int held = __float_as_int(mine[p].w);
+                    unsigned long long before[CHUNKS], equal[CHUNKS], any_equal = 0ull;
+                    const unsigned long long rows = row + 4 <= count ? ~0ull : row < count ? (1ull << (16 * (count - row))) - 1ull : 0ull;
+#pragma unroll
+                    for (int c = 0; c < CHUNKS; ++c)
                     {
-                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                        for (; seen < ready; seen = min(seen + POOL_BATCH, ready))
-                            update(seen, min(POOL_BATCH, ready - seen), top);
+                        const unsigned long long valid = (static_cast<unsigned long long>(static_cast<unsigned>(everyone >> (c * 16)) & 0xFFFFu) * 0x0001000100010001ull) & rows;
+                        // (a point itself: bit row % 16 of its row in the chunk that holds it)
+                        const unsigned long long self = row / 16 == c ? 0x0008000400020001ull << (row % 16) : 0ull;
+                        const int theirs = __float_as_int(other[c].w);
+                        before[c] = __ballot(theirs > held) & valid;
+                        equal[c] = __ballot(theirs == held) & valid & ~self;
+                        any_equal |= equal[c];
                     }
-                    else if ((state & POOL_DONE) == 0)
-                        __builtin_amdgcn_s_sleep(1);
-                    if (state & POOL_DONE)
-                        break;
+                    if (__builtin_expect(any_equal != 0, 0))
+                    {
+                        const unsigned key = tie_key(original_index(places[min(row + own_lane / 16, count - 1)]), log2_bs, ref_groups);
+                        for (int c = 0; c < CHUNKS; ++c)
+                        {
+                            const unsigned theirs = tie_key(original_index(places[min(c * 16 + own_lane % 16, count - 1)]), log2_bs, ref_groups);
+                            const unsigned long long first = __ballot(theirs < key);
+#pragma unroll
+                            for (int k = 0; k < CHUNKS; ++k)
+                                before[k] |= k == c ? first & equal[k] : 0ull;
+                        }
+                    }
+                    unsigned long long lowers[CHUNKS], stays[CHUNKS], any_stays = 0ull;
+#pragma unroll
+                    for (int c = 0; c < CHUNKS; ++c)
+                    {
+                        const int d = ordered_bits(tpk_dist2(mine[p].x, mine[p].y, mine[p].z, other[c].x, other[c].y, other[c].z));
+                        TPK_WORK_ADD(row + lane / 16 < count && c * 16 + lane % 16 < count ? 1 : 0);
+                        lowers[c] = __ballot(d < held) & before[c];
+                        stays[c] = __ballot(d > floor_bits) & lowers[c];
+                        any_stays |= stays[c];
+                    }
+                    // (lane r < 4 puts the 16 bits of row r of every chunk together)
+                    const int shift = (own_lane % 4) * 16;
+                    auto row_mask = [&](const unsigned long long (&m)[CHUNKS]) __attribute__((always_inline)) {
+                        const unsigned a = static_cast<unsigned>(m[0] >> shift), b = static_cast<unsigned>(m[1] >> shift);
+                        const unsigned c = static_cast<unsigned>(m[2] >> shift), d = static_cast<unsigned>(m[3] >> shift);
+                        return uint2{__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(d, c, 0x05040100u)};
+                    };
+                    const uint2 row_lowers = row_mask(lowers), row_before = row_mask(before);
+                    if (own_lane < 4)
+                    {
+                        pool_blockers[row + own_lane] = row_lowers;
+                        pool_before[row + own_lane] = row_before;
+                    }
+                    if (any_stays != 0)
+                    {
+                        const uint2 row_stays = row_mask(stays);
+                        if (own_lane < 4 && (row_stays.x | row_stays.y) != 0)
+                        {
+                            pool_keepers[row + own_lane] = row_stays;
+                            lds_or_u32(&keeps[par][row / 32], 1u << ((row + own_lane) % 32));
+                        }
+                    }
                 }
-                taken_now = seen;
-            }
-            if (taken_now > 0)
-            {
-                j += taken_now;
-                penalty = taken_now > 1 ? 1 : penalty;
-                most_left = floor_bits;
-                continue;
+                if (wave == 0 && own_lane < 2)
+                    keeps[par ^ 1][own_lane] = 0; // (of the round before: everybody has read it)
+                lds_barrier();
+                // 4. who is taken: in the order of the pool a point is, unless one taken before it lowers it.  All points
+                // whose lowering sources are decided are decided together; the first undecided one always is.
+                const float4 rec = points[own_lane];
+                const uint2 blockers = pool_blockers[own_lane];
+                const unsigned kept_lo = keeps[par][0], kept_hi = keeps[par][1];
+                unsigned long long taken = ~__ballot((blockers.x | blockers.y) != 0u) & everyone, dead = 0ull, open = everyone & ~taken;
+                while (open != 0ull)
+                {
+                    const bool hit = ((blockers.x & static_cast<unsigned>(taken)) | (blockers.y & static_cast<unsigned>(taken >> 32))) != 0u;
+                    const bool waits = ((blockers.x & static_cast<unsigned>(~dead)) | (blockers.y & static_cast<unsigned>(~dead >> 32))) != 0u;
+                    const unsigned long long hits = __ballot(hit) & open, free = ~__ballot(waits) & open;
+                    if ((hits | free) == 0ull)
+                        break; // (cannot be: the order is strict)
+                    dead |= hits;
+                    taken |= free;
+                    open &= ~(hits | free);
+                }
+                // 5. a point lowered inside the pool would be taken once the largest minimum has come down to what it holds
+                // now: the round ends there
+                const unsigned long long kept = static_cast<unsigned long long>(static_cast<unsigned>(__builtin_amdgcn_readfirstlane(kept_hi))) << 32 |
+                                                static_cast<unsigned>(__builtin_amdgcn_readfirstlane(kept_lo));
+                if (kept != 0)
+                {
+                    const uint2 keepers = pool_keepers[own_lane];
+                    const unsigned taken_lo = static_cast<unsigned>(taken), taken_hi = static_cast<unsigned>(taken >> 32);
+                    const bool lowered = ((keepers.x & taken_lo) | (keepers.y & taken_hi)) != 0u;
+                    const bool out_of_it = ((blockers.x & ~keepers.x & taken_lo) | (blockers.y & ~keepers.y & taken_hi)) != 0u;
+                    for (unsigned long long back = __ballot(lowered && !out_of_it) & kept; back != 0; back &= back - 1)
+                    {
+                        const int l = __builtin_ctzll(back);
+                        const unsigned by_lo = __builtin_amdgcn_readlane(keepers.x, l), by_hi = __builtin_amdgcn_readlane(keepers.y, l);
+                        const int d = ordered_bits(tpk_dist2(rec.x, rec.y, rec.z, tpk_read_lane(rec.x, l), tpk_read_lane(rec.y, l), tpk_read_lane(rec.z, l)));
+                        const bool by = ((taken & (static_cast<unsigned long long>(by_hi) << 32 | by_lo)) >> lane & 1ull) != 0ull;
+                        floor_bits = max(floor_bits, -wave_max_to_scalar(by ? -d : INT_MIN));
+                    }
+                }
+                const int left = __float_as_int(rec.w);
+                taken &= __ballot(left > floor_bits);
+                par ^= 1;
+                if (taken != 0ull) // (its first point always is)
+                {
+                    if (wave == 0)
+                    {
+                        const uint2 first = pool_before[own_lane];
+                        const int number = j + __builtin_popcount(first.x & static_cast<unsigned>(taken)) + __builtin_popcount(first.y & static_cast<unsigned>(taken >> 32));
+                        if (((taken >> lane) & 1ull) && number < npoint)
+                            out[number] = original_index(places[lane]);
+                    }
+                    // the next gap: the number of points grows with the gap
+                    gap = min(max(gap + (gap >> 6) * (POOL_TARGET - found), gap >> 1), 1 << 29);
+                    // 6. their updates
+                    j += __builtin_popcountll(taken);
+                    penalty = __builtin_popcountll(taken) > 1 ? 1 : penalty;
+                    most_left = floor_bits;
+                    if (j < npoint)
+                        update(rec.x, rec.y, rec.z, left, taken, points);
+                    continue;
+                }
             }
         }
         if (!paused)
         {
             pause = penalty;
-            penalty = min(2 * penalty, 32);
-            gap = 0.02f;
+            penalty = min(2 * penalty, 64);
+            gap = max(gap, 1 << 12);
         }
 
-        // More equal minima at the top than a pool holds, or nothing above zero: one sample by the reference's tie key
-        // over all points that hold the maximum (the key comes from the original index kept in the sort keys).
-        if (tid == 0)
-            words[which ^ 1] = RoundWords{INT_MIN, 0xFFFFFFFFu}; // (for the next time)
-        if (worker >= 0)
-        {
-            int best = t[0];
+        // One sample: every wavefront offers the best of its points (of several that hold its maximum the one with the
+        // smallest tie key), and all of them find the best of those.
+        int most = t[0];
 #pragma unroll
-            for (int i = 1; i < PPT; ++i)
-                best = max(best, t[i]);
-            const int row_best = row_all_max_i32(best);
-            if ((lane & 15) == 0)
-                lds_atomic_max_i32(&words[which].max_val, row_best);
-        }
-        lds_barrier();
-        const int gv = __builtin_amdgcn_readfirstlane(words[which].max_val);
-        if (gv < 0)
+        for (int i = 1; i < PPT; ++i)
+            most = max(most, t[i]);
+        most = wave_max_to_scalar(most);
+        const int own_lane = not_hoisted(lane);
+        bool several = keyed; // (where there were some there will be more)
+        if (!keyed)
         {
-            // No eligible point in the whole cloud: the reference's reduction yields index 0.
-            if (tid == 0)
+            int held = 0;
+#pragma unroll
+            for (int i = 0; i < PPT; ++i)
+                held += __builtin_popcountll(__ballot(t[i] == most));
+            several = held > 1;
+        }
+        if (several && most >= 0)
+        {
+            if (!keyed)
             {
-                taken[0] = make_float4(p0x, p0y, p0z, 0.f);
-                out[j] = 0;
+                // (from the first such round on the sort keys of this wavefront's points hold tie key and index, 14 bits each)
+#pragma unroll
+                for (int i = 0; i < (ORDERED ? PPT : 0); ++i)
+                {
+                    const int q = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
+                    const int k = original_index(min(q, n - 1));
+                    if (q < n)
+                        sort_keys[q] = tie_key(k, log2_bs, ref_groups) << 14 | static_cast<unsigned>(k);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                keyed = true;
             }
+            constexpr int BATCH = PPT < 8 ? PPT : 8;
+            unsigned key = 0xFFFFFFFFu;
+#pragma unroll
+            for (int from = 0; from < PPT; from += BATCH)
+            {
+                unsigned k[BATCH];
+#pragma unroll
+                for (int i = 0; i < BATCH; ++i)
+                {
+                    const int q = min(sorted_position<WAVES, GS>((from + i) / GS, wave, (from + i) % GS, own_lane), n - 1);
+                    k[i] = ORDERED ? sort_keys[q] : tie_key(q, log2_bs, ref_groups) << 14;
+                }
+#pragma unroll
+                for (int i = 0; i < BATCH; ++i)
+                    key = t[from + i] == most ? min(key, k[i] << 4 | static_cast<unsigned>(from + i)) : key;
+            }
+            const unsigned lowest = wave_min_u32(key);
+            const int slot = static_cast<int>(lowest & 15u);
+#pragma unroll
+            for (int i = 0; i < PPT; ++i)
+                if (i == slot && key == lowest)
+                {
+                    offers[turn][wave] = make_float4(x[i], y[i], z[i], __int_as_float(most));
+                    offer_places[turn][wave] = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
+                }
         }
         else
         {
-            unsigned my_tk = 0xFFFFFFFFu;
-            int my_q = 0;
-            if (worker >= 0)
-            {
 #pragma unroll
-                for (int i = 0; i < PPT; ++i)
+            for (int i = 0; i < PPT; ++i)
+                if (t[i] == most)
                 {
-                    const int q = sorted_position<WORKERS, GS>(i / GS, worker, i % GS, lane);
-                    if (t[i] == gv && q < n)
-                    {
-                        const unsigned tk = tie_key(original_index(q), log2_bs, ref_groups);
-                        if (tk < my_tk)
-                        {
-                            my_tk = tk;
-                            my_q = q;
-                        }
-                    }
+                    offers[turn][wave] = make_float4(x[i], y[i], z[i], __int_as_float(most));
+                    offer_places[turn][wave] = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
                 }
-                if (my_tk != 0xFFFFFFFFu)
-                    atomicMin(&words[which].min_tie, my_tk);
-            }
-            lds_barrier();
-            if (worker >= 0 && my_tk == words[which].min_tie) // tie keys are distinct: exactly one lane
-            {
-                const int k = original_index(my_q);
-                taken[0] = make_float4(xyz[k * 3 + 0], xyz[k * 3 + 1], xyz[k * 3 + 2], __int_as_float(my_q));
-                out[j] = k;
-            }
         }
         lds_barrier();
-        which ^= 1;
+        const float4 offer = offers[turn][lane % WAVES];
+        const int place = offer_places[turn][lane % WAVES];
+        turn ^= 1;
+        const int gv = __builtin_amdgcn_readfirstlane(row_all_max_i32(__float_as_int(offer.w)));
+        unsigned long long first = __ballot(__float_as_int(offer.w) == gv) & ((1ull << WAVES) - 1ull);
+        if (gv >= 0 && (first & (first - 1)) != 0ull)
+        {
+            const unsigned key = (first >> lane & 1ull) != 0ull ? tie_key(original_index(place), log2_bs, ref_groups) : 0xFFFFFFFFu;
+            first = __ballot(key == wave_min_u32(key)) & first;
+        }
+        const int w = __builtin_ctzll(first);
+        float4 s = make_float4(tpk_read_lane(offer.x, w), tpk_read_lane(offer.y, w), tpk_read_lane(offer.z, w), 0.f);
+        const int chosen = __builtin_amdgcn_readlane(place, w);
+        if (gv < 0) // no eligible point in the whole cloud: the reference's reduction yields index 0
+            s = make_float4(p0x, p0y, p0z, 0.f);
+        if (tid == 0)
+            out[j] = gv < 0 ? 0 : original_index(chosen);
         j += 1;
         most_left = max(gv, 0);
-        if (worker >= 0)
-            update(0, 1, gv < 0 ? ordered_bits(__builtin_inff()) : gv);
-        lds_barrier(); // (taken[] may be written again)
+        update_one(s, gv < 0 ? ordered_bits(__builtin_inff()) : gv);
     }
+    TPK_WORK_FLUSH
+}
+
+// Clouds that one wavefront holds, PPT points per lane: a sample at a time, 0.2 to 0.3 us each, without barriers and LDS.
+// What it costs is its chain of dependent instructions.
+template <int PPT>
+__global__ __launch_bounds__(TPK_WAVE) void fps_wave_kernel(int n, int npoint, int log2_bs, int ref_groups,
+                                                            const float* __restrict__ xyz, int32_t* __restrict__ out)
+{
+    xyz += static_cast<int64_t>(blockIdx.x) * n * 3;
+    out += static_cast<int64_t>(blockIdx.x) * npoint;
+    const int lane = threadIdx.x;
+    float x[PPT], y[PPT], z[PPT];
+    int t[PPT];
+#pragma unroll
+    for (int i = 0; i < PPT; ++i)
+    {
+        const int k = min(i * TPK_WAVE + lane, n - 1);
+        x[i] = xyz[k * 3 + 0];
+        y[i] = xyz[k * 3 + 1];
+        z[i] = xyz[k * 3 + 2];
+    }
+#pragma unroll
+    for (int i = 0; i < PPT; ++i)
+        t[i] = ordered_bits(i * TPK_WAVE + lane < n && eligible(x[i], y[i], z[i]) ? 1e10f : -1.0f);
+    TPK_WORK_DECL
+    float sx = tpk_read_lane(x[0], 0), sy = tpk_read_lane(y[0], 0), sz = tpk_read_lane(z[0], 0);
+    int mine = 0; // sample number j of the 64 not yet written, in lane j % 64
+    for (int j = 1; j < npoint; ++j)
+    {
+        const float ux = to_vector_register(sx), uy = to_vector_register(sy), uz = to_vector_register(sz);
+        int best = INT_MIN;
+        TPK_WORK_ADD(PPT);
+#pragma unroll
+        for (int i = 0; i < PPT; ++i)
+        {
+            t[i] = min(t[i], ordered_bits(tpk_dist2(x[i], y[i], z[i], ux, uy, uz)));
+            best = max(best, t[i]);
+        }
+        const int most = wave_max_to_scalar(best);
+        unsigned long long holders[PPT];
+        int count = 0;
+#pragma unroll
+        for (int i = 0; i < PPT; ++i)
+        {
+            holders[i] = __ballot(t[i] == most);
+            count += __builtin_popcountll(holders[i]);
+        }
+        if (__builtin_expect(count != 1, 0))
+        {
+            // equal maxima: the smallest tie key
+            unsigned key = 0xFFFFFFFFu;
+#pragma unroll
+            for (int i = 0; i < PPT; ++i)
+                if (t[i] == most && i * TPK_WAVE + lane < n)
+                    key = min(key, tie_key(i * TPK_WAVE + lane, log2_bs, ref_groups));
+            const unsigned lowest = wave_min_u32(key);
+#pragma unroll
+            for (int i = 0; i < PPT; ++i)
+                holders[i] = __ballot(t[i] == most && i * TPK_WAVE + lane < n && tie_key(i * TPK_WAVE + lane, log2_bs, ref_groups) == lowest);
+        }
+        int k = 0;
+        if (most < 0)
+        {
+            // No eligible point in the whole cloud: the reference's reduction yields index 0.
+            sx = tpk_read_lane(x[0], 0), sy = tpk_read_lane(y[0], 0), sz = tpk_read_lane(z[0], 0);
+        }
+        else
+        {
+#pragma unroll
+            for (int i = 0; i < PPT; ++i)
+                if (holders[i] != 0)
+                {
+                    const int l = __builtin_ctzll(holders[i]);
+                    k = i * TPK_WAVE + l;
+                    sx = tpk_read_lane(x[i], l), sy = tpk_read_lane(y[i], l), sz = tpk_read_lane(z[i], l);
+                }
+        }
+        mine = lane == j % TPK_WAVE ? k : mine;
+        if (j % TPK_WAVE == TPK_WAVE - 1)
+            out[j - (TPK_WAVE - 1) + lane] = mine;
+    }
+    const int written = npoint / TPK_WAVE * TPK_WAVE;
+    if (written + lane < npoint)
+        out[written + lane] = mine;
     TPK_WORK_FLUSH
 }
 
@@ -1063,7 +1342,7 @@ int reference_log2_block(int n)
 template <int PPT, int WAVES, int GS, bool ORDERED>
 int launch_pool(int b, int n, int npoint, int log2_bs, int groups, const float* xyz, int32_t* out, hipStream_t s)
 {
-    if (n > PPT * (WAVES - 1) * TPK_WAVE || n > FPS_REGISTER_POINTS)
+    if (n > PPT * WAVES * TPK_WAVE || n > FPS_REGISTER_POINTS)
         return TPK_ERR_UNSUPPORTED;
     const int key_capacity = n > CURVE_BINS ? (n + 63) & ~63 : CURVE_BINS; // (the ordering borrows CURVE_BINS words)
     const size_t lds = ORDERED ? (2 * static_cast<size_t>(key_capacity) + CURVE_BINS) * sizeof(unsigned) : 0;
@@ -1073,6 +1352,15 @@ int launch_pool(int b, int n, int npoint, int log2_bs, int groups, const float* 
         return allowed;
     hipLaunchKernelGGL(kernel, dim3(b), dim3(WAVES * TPK_WAVE), lds, s, n, npoint, log2_bs, groups, key_capacity,
                        xyz, out);
+    return tpk_launch_status();
+}
+
+template <int PPT>
+int launch_wave(int b, int n, int npoint, int log2_bs, int groups, const float* xyz, int32_t* out, hipStream_t s)
+{
+    if (n > PPT * TPK_WAVE)
+        return TPK_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(fps_wave_kernel<PPT>, dim3(b), dim3(TPK_WAVE), 0, s, n, npoint, log2_bs, groups, xyz, out);
     return tpk_launch_status();
 }
 
@@ -1141,22 +1429,28 @@ extern "C" int tpk_fps_f32(int b, int n, int npoint, const float* xyz, void* wor
     const int log2_bs = reference_log2_block(n);
     const int groups = static_cast<int>(tpk_ceil_div(n, 1 << log2_bs));
 
-    // Up to 16384 points: registers of the workers of a workgroup, with one wavefront more that samples.  Sixteen
-    // wavefronts throughout (eight with twice the points each: 4 - 20 us more), cells of 64 to 192 points.  Measured with a
-    // quarter of the points sampled (16 clouds; the version before): 400 points 45 us (68), 1024 82 (114), 2048 134 (204),
-    // 4096 234 (359), 8192 430 (768), 16384 843 (1293).
-    if (n <= 15 * 64)
-        return launch_pool<1, 16, 1, false>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 2 * 15 * 64)
-        return launch_pool<2, 16, 2, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 4 * 15 * 64)
+    // Up to 256 points one wavefront (16 clouds, a quarter to half of the points sampled: 64 points 13 us, 128 17, 256 22 - 40;
+    // with pools 45 - 57; eight points per lane: 512 points 118 us against 55 with pools).  Up to 1024 points pools by eight
+    // wavefronts, above by sixteen (1024 points 63 / 69 us, 2048 110 / 98, 4096 187 / 159).  Up to there the cloud is taken as it comes: the
+    // ordering alone is 8 us.
+    if (n <= 64)
+        return launch_wave<1>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 2 * 64)
+        return launch_wave<2>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 4 * 64)
+        return launch_wave<4>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 8 * 64)
+        return launch_pool<1, 8, 1, false>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 2 * 8 * 64)
+        return launch_pool<2, 8, 2, false>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 2 * 16 * 64)
+        return launch_pool<2, 16, 1, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 4 * 16 * 64)
         return launch_pool<4, 16, 2, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 6 * 15 * 64)
-        return launch_pool<6, 16, 3, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
-    else if (n <= 12 * 15 * 64)
-        return launch_pool<12, 16, 3, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+    else if (n <= 8 * 16 * 64)
+        return launch_pool<8, 16, 2, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
     else if (n <= FPS_REGISTER_POINTS)
-        return launch_pool<18, 16, 3, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
+        return launch_pool<16, 16, 2, true>(b, n, npoint, log2_bs, groups, xyz, idx_out, s);
     else if (n <= FPS_CELL_POINTS && workspace && workspace_bytes >= cell_layout(b, n).total)
     {
         // Cells of 64 points in memory, their summaries in LDS.
