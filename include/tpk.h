@@ -243,6 +243,11 @@ int tpk_three_interpolate_lists_f32(int b, int n, int m, const int32_t* idx, con
 int tpk_three_interpolate_grad_lists_f32(int b, int c, int n, int m, const float* grad_out,
                                          void* lists, size_t lists_bytes, float* grad_points,
                                          void* stream);
+/* tpk_three_interpolate_f32 and tpk_three_interpolate_lists_f32 in one launch where both fit: the forward pass is bound by
+ * memory and the lists are not, so that they run beside each other.  Same `out`, same `lists`. */
+int tpk_three_interpolate_recording_f32(int b, int c, int m, int n, const float* points, const int32_t* idx,
+                                        const float* weight, float* out, void* lists, size_t lists_bytes,
+                                        void* stream);
 
 /* ---------------------------------------------------------------------------------------
  * Grouping (gather of feature columns), forward and backward.
@@ -266,6 +271,9 @@ int tpk_group_lists(int b, int n, int npoint, int nsample, const int64_t* idx, v
                     size_t lists_bytes, void* stream);
 int tpk_group_grad_lists_f32(int b, int c, int n, int npoint, int nsample, const float* grad_out,
                              void* lists, size_t lists_bytes, float* grad_features, void* stream);
+/* tpk_group_f32 and tpk_group_lists in one launch where both fit. */
+int tpk_group_recording_f32(int b, int c, int n, int npoint, int nsample, const float* features,
+                            const int64_t* idx, float* out, void* lists, size_t lists_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------------
  * Chamfer distance, forward (both directions) and backward.

@@ -1040,6 +1040,36 @@ def test_grouping_grad_long_rows(tpk, oracle, dev, N, npoint, nsample, C):
     _assert_scatter_sum_close(_np(f.grad), want, oracle.grouping_operation_grad(gout.abs().numpy(), idx.numpy(), N))
 
 
+@pytest.mark.parametrize("B,C,m,n", [(1, 1, 1, 1), (1, 3, 15, 1023), (2, 9, 16, 1024), (2, 5, 17, 1025), (1, 2, 300, 16385), (2, 2, 3000, 32768),
+                                     (1, 7, 4096, 32769), (1, 2, 20481, 4097), (16, 64, 1024, 4096)])
+@pytest.mark.parametrize("kind", ["spread", "one target", "last targets"])
+def test_gather_with_the_lists_of_its_gradient(tpk, dev, kind, B, C, m, n):
+    # the gather and the lists of its backward pass in one launch: the same bits as the gather alone, and - small integers
+    # throughout, whose sums are exact in any order - the exact gradient.  Sizes around a round of 1024 entries, a word of 32 rounds,
+    # the 16 spans and the rows that fit half of the LDS
+    g = torch.Generator().manual_seed(m + n)
+    idx = torch.randint(0, m, (B, n, 3), generator=g)
+    if kind == "one target":
+        idx[:] = m // 2
+    elif kind == "last targets":
+        idx = m - 1 - idx % min(m, 3)
+    feats = torch.randint(-8, 9, (B, C, m), generator=g).float()
+    weight = torch.randint(0, 5, (B, n, 3), generator=g).float()
+    gout = torch.randint(-8, 9, (B, C, n), generator=g).float()
+    index, weights = idx.to(dev), weight.to(dev)
+    for columns, run in ((idx[..., :1], lambda f: tpk.grouping_operation(f, index[..., :1].contiguous())),
+                         (idx, lambda f: tpk.three_interpolate(f, index.int(), weights))):
+        w = weight if columns.shape[2] == 3 else torch.ones(B, n, 1)
+        f = feats.to(dev).requires_grad_(True)
+        out = run(f)
+        assert torch.equal(out.detach(), run(feats.to(dev)))
+        out.backward(gout.to(dev).view(out.shape))
+        want = torch.zeros(B, C, m)
+        for k in range(columns.shape[2]):
+            want.scatter_add_(2, columns[:, None, :, k].expand(B, C, n), gout * w[:, None, :, k])
+        assert torch.equal(f.grad.cpu(), want), columns.shape
+
+
 @pytest.mark.parametrize("columns", [1, 1023, 1024, 1025, 5121])
 def test_gather_full_grids(tpk, oracle, dev, columns):
     # grids with a workgroup for every compute unit: each starts at another run of 1024 columns and wraps around

@@ -37,6 +37,8 @@ namespace {
 
 constexpr int G_MAX_ROWS = 8;
 constexpr int G_LDS_BUDGET = 131072; // bytes of LDS for the staged rows
+constexpr int G_SHARED_BUDGET = 81920; // ... where two workgroups share a compute unit
+constexpr int G_SHARED_GRID = 512;     // workgroups that fit the chip then
 constexpr unsigned G_FULL_GRID = 256;  // a workgroup for every compute unit
 constexpr int G_BUSY_GRID = 192;       // workgroups below which the weighted gather takes fewer rows per workgroup
 constexpr int G_PLAIN_BLOCKS = 1024; // workgroups the plain gather aims at (four per compute unit, two at a time)
@@ -134,7 +136,16 @@ __device__ __forceinline__ void stage_copy(float* dst, const float* __restrict__
     stage_rows_by<G_THREADS, 8>(dst, count, src, count, 1u, count, threadIdx.x);
 }
 
-// grid: (clouds * row_blocks * jsplit).  dynamic LDS: R * m floats.
+// How a forward pass is cut into workgroups: clouds * row_blocks * jsplit of them, each with `rows` rows of a cloud in LDS
+// and a part of jlen columns.
+struct FwdPlan
+{
+    int rows, row_blocks, jsplit; // rows == 0: a row does not fit
+    int64_t jlen, blocks;
+    size_t lds;
+};
+
+// The share of workgroup `block` of `blocks`.  LDS (`rows`): R * m floats.
 //
 // Bound by the output's way to memory.  All workgroups write rows that lie a multiple of the row length apart: where
 // they walk the columns in step and that length is a power of two, their stores meet in the same few memory channels.
@@ -143,13 +154,12 @@ __device__ __forceinline__ void stage_copy(float* dst, const float* __restrict__
 // 128 channels): rows of 32768 columns, plain, 99 -> 60 us (348 MB: 5.8 TB/s; a large copy here moves 5.3), without
 // the dies 64; rows of 16384 columns, three weighted neighbours, 54 -> 41 us (174 MB), without the dies 49.
 template <int K, bool WEIGHTED, typename IdxT>
-__global__ __launch_bounds__(G_THREADS) void gather_fwd_lds_kernel(
-    int c, int m, int64_t n, int rows_per_block, int row_blocks, int jsplit, int64_t jlen,
-    const float* __restrict__ src, const IdxT* __restrict__ idx,
-    const float* __restrict__ weight, float* __restrict__ out)
+__device__ __forceinline__ void gather_fwd_rows(
+    unsigned hardware_block, unsigned blocks, float* rows, int c, int m, int64_t n, int rows_per_block, int row_blocks, int jsplit,
+    int64_t jlen, const float* __restrict__ src, const IdxT* __restrict__ idx, const float* __restrict__ weight,
+    float* __restrict__ out)
 {
-    extern __shared__ float rows[];
-    const unsigned block = xcd_local_block(blockIdx.x, gridDim.x);
+    const unsigned block = xcd_local_block(hardware_block, blocks);
     int bid = static_cast<int>(block);
     const int jpart = bid % jsplit;
     bid /= jsplit;
@@ -171,7 +181,7 @@ __global__ __launch_bounds__(G_THREADS) void gather_fwd_lds_kernel(
     // The runs of G_THREADS columns of this part, from run `first` on and around.  (A grid that leaves compute units idle
     // is bound by latency, and its workgroups gain from asking for the same indices together.)
     const unsigned runs = static_cast<unsigned>((jend - jbeg + G_THREADS - 1) / G_THREADS);
-    const unsigned first = gridDim.x >= G_FULL_GRID ? block % runs : 0u;
+    const unsigned first = blocks >= G_FULL_GRID ? block % runs : 0u;
     auto column = [&](unsigned i) __attribute__((always_inline)) {
         const unsigned run = first + i < runs ? first + i : first + i - runs;
         return jbeg + static_cast<int64_t>(run) * G_THREADS + threadIdx.x;
@@ -202,6 +212,37 @@ __global__ __launch_bounds__(G_THREADS) void gather_fwd_lds_kernel(
                     __builtin_nontemporal_store(v, to); // (written once, read by nobody here: past the caches)
             }
     }
+}
+
+template <int K, bool WEIGHTED, typename IdxT>
+__global__ __launch_bounds__(G_THREADS) void gather_fwd_lds_kernel(
+    int c, int m, int64_t n, FwdPlan plan, const float* __restrict__ src, const IdxT* __restrict__ idx,
+    const float* __restrict__ weight, float* __restrict__ out)
+{
+    extern __shared__ float rows[];
+    gather_fwd_rows<K, WEIGHTED, IdxT>(blockIdx.x, gridDim.x, rows, c, m, n, plan.rows, plan.row_blocks, plan.jsplit, plan.jlen, src, idx,
+                                       weight, out);
+}
+
+// The forward pass of a call whose gradient will be asked for: the first job.workgroups workgroups build the lists of the
+// backward pass (lists.h), the others gather.  Neither needs the other, the gather waits for memory most of the time and the
+// builder for its instructions, and a workgroup of each fits a compute unit (64 registers, half of the LDS).  Measured with both
+// launches' time, apart and together: 16 clouds of 128 rows, 16384 x 3 entries on 2048 points 50.4 -> 42.3 us, on 4096 points 64
+// rows 40.9 -> 31.9; 32768 x 1 entries on 4096 points 80.4 -> 75.3; 16 x 100 from 20, all launch, 11.1 -> 7.7.
+template <int K, bool WEIGHTED, typename IdxT>
+__global__ __launch_bounds__(G_THREADS, 8) void gather_fwd_recording_kernel(
+    int c, int m, int64_t n, FwdPlan plan, const float* __restrict__ src, const IdxT* __restrict__ idx,
+    const float* __restrict__ weight, float* __restrict__ out, ListJob<WEIGHTED, IdxT> job)
+{
+    extern __shared__ float rows[];
+    const unsigned builders = static_cast<unsigned>(job.workgroups);
+    if (blockIdx.x < builders)
+    {
+        build_lists<K, WEIGHTED, IdxT>(job, static_cast<int>(blockIdx.x), reinterpret_cast<int*>(rows));
+        return;
+    }
+    gather_fwd_rows<K, WEIGHTED, IdxT>(blockIdx.x - builders, gridDim.x - builders, rows, c, m, n, plan.rows, plan.row_blocks, plan.jsplit,
+                                       plan.jlen, src, idx, weight, out);
 }
 
 constexpr int GB_LDS_FLOATS = TPK_LDS_BYTES / 4; // floats of LDS a workgroup of the backward walk may use (all 160 KiB)
@@ -685,32 +726,28 @@ __global__ __launch_bounds__(256) void fill_zero_f32_kernel(float* p, int64_t co
         p[t] = 0.0f;
 }
 
-// Rows staged per workgroup for rows of m floats; 0 = does not fit.
-int rows_for(int m, int c)
+// Rows staged per workgroup for rows of m floats in `budget` bytes of LDS; 0 = does not fit.
+int rows_for(int m, int c, int budget)
 {
     if (m <= 0)
         return 0;
-    int r = G_LDS_BUDGET / (4 * m);
+    int r = budget / (4 * m);
     if (r > G_MAX_ROWS)
         r = G_MAX_ROWS;
+    // (5 rows take longer than 4 and 4 again, for their stores: 16 clouds of 96 rows 60.0 us with 5 and 50.2 with 4)
+    if (budget == G_SHARED_BUDGET)
+        while ((r & (r - 1)) != 0)
+            --r;
     if (r > c)
         r = c;
     return r;
 }
 
-template <int K, bool WEIGHTED, typename IdxT>
-int gather_fwd(int b, int c, int m, int64_t n, const float* src, const IdxT* idx,
-               const float* weight, float* out, hipStream_t s)
+template <bool WEIGHTED>
+FwdPlan plan_fwd(int b, int c, int m, int64_t n, int budget)
 {
-    if (b < 0 || c < 0 || m < 0 || n < 0)
-        return TPK_ERR_INVALID_ARG;
-    if (b == 0 || c == 0 || n == 0)
-        return TPK_OK;
-    if (m == 0)
-        return TPK_ERR_INVALID_ARG; // columns to fill but nothing to gather from
-    if (!src || !idx || !out || (WEIGHTED && !weight))
-        return TPK_ERR_INVALID_ARG;
-    int r = rows_for(m, c);
+    FwdPlan plan{};
+    int r = rows_for(m, c, budget);
     // parts of a row's columns, each at least as long as a row, so that staging a row block stays the smaller share
     const int64_t whole_parts = n / (m > G_THREADS ? m : G_THREADS), max_split = whole_parts < 1 ? 1 : whole_parts;
     // The weighted gather, where it would leave compute units idle: fewer rows per workgroup, down to two.  Measured:
@@ -728,26 +765,41 @@ int gather_fwd(int b, int c, int m, int64_t n, const float* src, const IdxT* idx
     if (!WEIGHTED)
         while (r > 2 && static_cast<int64_t>(b) * tpk_ceil_div(c, r) < G_PLAIN_BLOCKS)
             r = (r + 1) / 2;
-    if (r > 0)
+    if (r == 0)
+        return plan;
+    plan.rows = r;
+    plan.row_blocks = static_cast<int>(tpk_ceil_div(c, r));
+    // Split the columns so that a few hundred workgroups exist.
+    const int64_t jsplit = tpk_min64(tpk_ceil_div(WEIGHTED ? 256 : G_PLAIN_BLOCKS, static_cast<int64_t>(plan.row_blocks) * b), max_split);
+    plan.jsplit = static_cast<int>(jsplit < 1 ? 1 : jsplit);
+    plan.jlen = tpk_ceil_div(n, plan.jsplit);
+    plan.blocks = static_cast<int64_t>(b) * plan.row_blocks * plan.jsplit;
+    plan.lds = static_cast<size_t>(r) * m * sizeof(float);
+    return plan;
+}
+
+template <int K, bool WEIGHTED, typename IdxT>
+int gather_fwd(int b, int c, int m, int64_t n, const float* src, const IdxT* idx,
+               const float* weight, float* out, hipStream_t s)
+{
+    if (b < 0 || c < 0 || m < 0 || n < 0)
+        return TPK_ERR_INVALID_ARG;
+    if (b == 0 || c == 0 || n == 0)
+        return TPK_OK;
+    if (m == 0)
+        return TPK_ERR_INVALID_ARG; // columns to fill but nothing to gather from
+    if (!src || !idx || !out || (WEIGHTED && !weight))
+        return TPK_ERR_INVALID_ARG;
+    const FwdPlan plan = plan_fwd<WEIGHTED>(b, c, m, n, G_LDS_BUDGET);
+    if (plan.rows > 0)
     {
-        const int row_blocks = static_cast<int>(tpk_ceil_div(c, r));
-        // Split the columns so that a few hundred workgroups exist.
-        int64_t jsplit = tpk_ceil_div(WEIGHTED ? 256 : G_PLAIN_BLOCKS, static_cast<int64_t>(row_blocks) * b);
-        if (jsplit > max_split)
-            jsplit = max_split;
-        if (jsplit < 1)
-            jsplit = 1;
-        const int64_t jlen = tpk_ceil_div(n, jsplit);
-        const int64_t blocks = static_cast<int64_t>(b) * row_blocks * jsplit;
-        if (blocks > 0x7fffffffLL)
+        if (plan.blocks > 0x7fffffffLL)
             return TPK_ERR_UNSUPPORTED;
-        const size_t lds = static_cast<size_t>(r) * m * sizeof(float);
         auto kernel = gather_fwd_lds_kernel<K, WEIGHTED, IdxT>;
-        int st = allow_lds(kernel, lds);
+        int st = allow_lds(kernel, plan.lds);
         if (st != TPK_OK)
             return st;
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(G_THREADS), lds, s, c,
-                           m, n, r, row_blocks, static_cast<int>(jsplit), jlen, src, idx, weight,
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(plan.blocks)), dim3(G_THREADS), plan.lds, s, c, m, n, plan, src, idx, weight,
                            out);
         return tpk_launch_status();
     }
@@ -854,6 +906,53 @@ int gather_lists(int b, int m, int64_t n, const IdxT* idx, const float* weight, 
     const int64_t part_total = static_cast<int64_t>(sh.part_len) * K;
     const Lists<WEIGHTED> lists = lists_at<WEIGHTED>(lists_memory, static_cast<int64_t>(b) * sh.parts, m, part_total);
     return launch_build_lists<K, WEIGHTED, IdxT>(b, m, n * K, part_total, idx, weight, lists, s);
+}
+
+// The forward pass and the lists of the backward pass.  TPK_ERR_UNSUPPORTED: the list path does not serve this shape
+// (nothing has been enqueued).
+template <int K, bool WEIGHTED, typename IdxT>
+int gather_fwd_recording(int b, int c, int m, int64_t n, const float* src, const IdxT* idx, const float* weight, float* out,
+                         void* lists_memory, size_t lists_bytes, hipStream_t s)
+{
+    if (b < 0 || c < 0 || m < 0 || n < 0)
+        return TPK_ERR_INVALID_ARG;
+    const BwdShape sh = list_shape<K>(b, m, n);
+    const size_t need = lists_workspace_bytes<K, WEIGHTED>(b, m, n);
+    if (sh.rows == 0 || need == 0)
+        return TPK_ERR_UNSUPPORTED;
+    if (!lists_memory || lists_bytes < need || (reinterpret_cast<uintptr_t>(lists_memory) & 15u))
+        return TPK_ERR_WORKSPACE;
+    if (!idx || (WEIGHTED && !weight) || (c > 0 && (!src || !out)))
+        return TPK_ERR_INVALID_ARG;
+    // Together where the gather's workgroups keep the rows they have on their own, or where there are so few of them that they
+    // find room beside the builders: with fewer rows each reads the indices more often.  Measured apart and together, 16384 x 3
+    // entries on 4096 points (8 rows apart, 4 together): 16 clouds of 64 rows (256 workgroups) 40.9 and 31.9 us, of 96 rows (384)
+    // 58.0 and 50.2, of 128 rows (512) 56.7 and 56.3, 8 clouds of 256 rows (512) 54.2 and 55.0, 32 of 128 (1024) 106.6 and 113.6.
+    const FwdPlan plan = plan_fwd<WEIGHTED>(b, c, m, n, G_SHARED_BUDGET);
+    if (b > 0 && c > 0 && n > 0 && plan.rows > 0 &&
+        (plan.blocks < G_SHARED_GRID || plan.rows == plan_fwd<WEIGHTED>(b, c, m, n, G_LDS_BUDGET).rows))
+    {
+        const int64_t part_total = static_cast<int64_t>(sh.part_len) * K;
+        const Lists<WEIGHTED> lists = lists_at<WEIGHTED>(lists_memory, static_cast<int64_t>(b) * sh.parts, m, part_total);
+        ListJob<WEIGHTED, IdxT> job;
+        int st = make_list_job<K, WEIGHTED, IdxT>(b, m, n * K, part_total, idx, weight, lists, &job);
+        if (st != TPK_OK)
+            return st;
+        const size_t list_lds = list_lds_bytes(job.span), lds = list_lds > plan.lds ? list_lds : plan.lds;
+        const int64_t blocks = plan.blocks + job.workgroups;
+        if (job.workgroups > 0 && list_lds <= static_cast<size_t>(G_SHARED_BUDGET) && blocks <= 0x7fffffffLL)
+        {
+            auto kernel = gather_fwd_recording_kernel<K, WEIGHTED, IdxT>;
+            st = allow_lds(kernel, lds);
+            if (st != TPK_OK)
+                return st;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(G_THREADS), lds, s, c, m, n, plan, src, idx, weight, out,
+                               job);
+            return tpk_launch_status();
+        }
+    }
+    const int st = gather_fwd<K, WEIGHTED, IdxT>(b, c, m, n, src, idx, weight, out, s);
+    return st != TPK_OK ? st : gather_lists<K, WEIGHTED, IdxT>(b, m, n, idx, weight, lists_memory, lists_bytes, s);
 }
 
 // The backward pass over lists that gather_lists() built for the same (b, n, m).
@@ -979,6 +1078,21 @@ extern "C" int tpk_three_interpolate_lists_f32(int b, int n, int m, const int32_
     if (b > 0 && n > 0 && m > 0 && (!idx || !weight))
         return TPK_ERR_INVALID_ARG;
     return gather_lists<3, true, int32_t>(b, m, n, idx, weight, lists, lists_bytes, tpk_stream(stream));
+}
+
+extern "C" int tpk_three_interpolate_recording_f32(int b, int c, int m, int n, const float* points, const int32_t* idx, const float* weight,
+                                                   float* out, void* lists, size_t lists_bytes, void* stream)
+{
+    return gather_fwd_recording<3, true, int32_t>(b, c, m, n, points, idx, weight, out, lists, lists_bytes, tpk_stream(stream));
+}
+
+extern "C" int tpk_group_recording_f32(int b, int c, int n, int npoint, int nsample, const float* features, const int64_t* idx, float* out,
+                                       void* lists, size_t lists_bytes, void* stream)
+{
+    if (npoint < 0 || nsample < 0)
+        return TPK_ERR_INVALID_ARG;
+    return gather_fwd_recording<1, false, int64_t>(b, c, n, static_cast<int64_t>(npoint) * nsample, features, idx, nullptr, out, lists,
+                                                   lists_bytes, tpk_stream(stream));
 }
 
 extern "C" int tpk_three_interpolate_grad_lists_f32(int b, int c, int n, int m, const float* grad_out, void* lists,

@@ -62,12 +62,11 @@ static_assert(static_cast<uint32_t>(L_NOTHING) * 1u >= TPK_LDS_BYTES && static_c
 constexpr int L_SPANS = G_THREADS / TPK_WAVE; // spans of targets per cloud: one per wavefront of the walker
 constexpr int L_MAX_SPAN = 15360;             // targets of a span: their bookkeeping (2 ints each) fits in LDS
 constexpr int L_REGION_GAP = 128;             // entry slots between the regions of consecutive spans
-// Index values a thread keeps in registers between the two passes: all of the longest part that is walked whole (32768
-// columns of one entry, or 16384 of three).  (48 for both spilled with 64-bit indices: 16 clouds of 32768 entries 18.1 us,
-// 17.6 with 32.)
 template <int K>
-constexpr int L_CACHED = K == 1 ? 32 : 48;
-constexpr int L_QUEUE = 128;                  // places of a wavefront's queue of entries inside the span (a power of two >= 128)
+constexpr int L_MAX_PART = K * 32768; // index entries of a part: columns that the walker takes whole
+constexpr int L_QUEUE = 512; // entries inside the span that a wavefront notes in LDS
+constexpr int L_ENTRY_BITS = 17, L_TARGET_BITS = 14; // ... as the number of the entry and the target's place in the span
+static_assert(L_MAX_PART<3> <= 1 << L_ENTRY_BITS && L_MAX_SPAN <= 1 << L_TARGET_BITS && L_ENTRY_BITS + L_TARGET_BITS <= 32, "a note's bits");
 
 template <bool WEIGHTED>
 struct Lists
@@ -124,29 +123,34 @@ struct ListJob
     Lists<WEIGHTED> lists;
 };
 
-// grid: (clouds * parts * L_SPANS); workgroup (cloud part, s) builds the lists of the targets
-// [s * span, (s + 1) * span).  It reads every index entry of its part (keeping the first
-// L_CACHED values per thread in registers for the second pass), counts those inside its span
-// with LDS integer atomics and those below it - their number fixes where its region starts, so
+// A workgroup's share: workgroup `block` of clouds * parts * L_SPANS, (cloud part, s), builds the lists of the targets
+// [s * span, (s + 1) * span).  It reads every index entry of its part and notes those inside its span in LDS, counts them
+// with LDS integer atomics and those below the span - their number fixes where its region starts, so
 // no workgroup waits for another -, prefix-sums the list lengths (empty lists count as one
-// entry) and places its entries in a second pass.  Index values outside [0, m) are dropped.
-// dynamic LDS: (2 * span + G_THREADS / 64 + 2) ints + the queues (L_QUEUE x 8 bytes per wavefront).
+// entry) and places its entries in a second pass over the notes.  Index values outside [0, m) are dropped.
+// LDS (`counters`): list_lds_bytes().
+//
+// Bound by the instructions of the first pass, as all but one entry in L_SPANS are read in vain, and by the stores of single
+// entries.  A part's workgroups run on one die, which reads its index once.  Keeping every index value in registers for a second
+// pass over all of them took 12900 + 15300 clocks for the two passes at 16384 x 3 entries (124 registers, 17.2 us), the notes
+// take 13300 + 6800 (42 registers, 12.6 us); a bit per entry instead of a note, and the index read again, 11300 + 20100.
 template <int K, bool WEIGHTED, typename IdxT>
-__global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED, IdxT> job)
+__device__ __forceinline__ void build_lists(const ListJob<WEIGHTED, IdxT>& job, int block, int* counters)
 {
     const int m = job.m, cloud_total = job.cloud_total, parts = job.parts, part_total = job.part_total, span = job.span;
     const IdxT* __restrict__ idx = job.idx;
     const float* __restrict__ weight = job.weight;
 
-    extern __shared__ int counters[];           // [span] list lengths, in the second pass the places still free
+    // counters: [span] list lengths, in the second pass the places still free
     int* const ends = counters + span;          // [span] rank behind every list's last entry inside the span
     int* const scan = ends + span;              // [G_THREADS / 64], then below_total
     int* const below_total = scan + G_THREADS / TPK_WAVE;
     const int tid = threadIdx.x;
     const int lane = tid & (TPK_WAVE - 1);
     const int wave = tid / TPK_WAVE;
-    const int cloud_part = blockIdx.x / L_SPANS;
-    const int s = blockIdx.x - cloud_part * L_SPANS;
+    block = static_cast<int>(xcd_local_block(static_cast<unsigned>(block), static_cast<unsigned>(job.workgroups)));
+    const int cloud_part = block / L_SPANS;
+    const int s = block - cloud_part * L_SPANS;
     const int part = cloud_part % parts;
     const int total = min(part_total, cloud_total - part * part_total);
     const int i0 = min(s * span, m);
@@ -163,55 +167,93 @@ __global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED
         *below_total = 0;
     __syncthreads();
 
-    // First pass.  Entry e of the part is read by thread e % G_THREADS in its round e / G_THREADS.
-    int cached[L_CACHED<K>];
-    int below = 0; // valid entries whose target lies before this span
-    auto count_one = [&](int v) {
-        below += (v >= 0 && v < i0) ? 1 : 0;
-        if (v >= i0 && v < i1)
-            atomicAdd(&counters[v - i0], 1);
+    // First pass.  Entry e of the part is read by thread e % G_THREADS in its round e / G_THREADS.  A wavefront notes those inside
+    // the span in its queue, in order.
+    // (a value that does not fit 32 bits is outside every cloud, like an entry behind the part's last)
+    constexpr unsigned OUTSIDE = ~0u;
+    auto index_value = [](IdxT v) {
+        if constexpr (sizeof(IdxT) == 8)
+            return (static_cast<unsigned long long>(v) >> 32) != 0 ? OUTSIDE : static_cast<unsigned>(v);
+        else
+            return static_cast<unsigned>(v);
     };
-    // (a value that does not fit 32 bits is outside every cloud: -1, like an entry behind the part's last)
-    auto index_value = [&](int e) {
-        const int64_t v = static_cast<int64_t>(idx[min(e, total - 1)]);
-        return (e < total && v >= 0 && v < m) ? static_cast<int>(v) : -1;
-    };
-    constexpr int BATCH = 16; // index loads in flight per thread
-    static_assert(L_CACHED<K> % BATCH == 0, "the cached rounds are whole batches");
-#pragma unroll
-    for (int b = 0; b < L_CACHED<K>; b += BATCH)
-    {
-        if (b * G_THREADS < total) // (wave-uniform)
+    constexpr int BATCH = 8; // rounds read together, while the batch before them is looked at
+    auto read_batch = [&](int first, IdxT* v) {
+        if (first + BATCH * G_THREADS <= total)
         {
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-                cached[b + u] = index_value((b + u) * G_THREADS + tid);
-#pragma unroll
-            for (int u = 0; u < BATCH; ++u)
-                count_one(cached[b + u]);
+                v[u] = (idx + (first + u * G_THREADS))[static_cast<unsigned>(tid)];
         }
         else
         {
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-                cached[b + u] = -1;
+            {
+                const int e = first + u * G_THREADS + tid;
+                v[u] = idx[min(e, total - 1)];
+                v[u] = e < total ? v[u] : static_cast<IdxT>(-1);
+            }
         }
-    }
-    for (int e0 = L_CACHED<K> * G_THREADS + tid; e0 < total; e0 += BATCH * G_THREADS)
-    {
-        int iv[BATCH];
+    };
+    auto read_entries = [&](auto&& take) { // (first entry of the thread in the batch, the batch's values)
+        IdxT v[BATCH], next[BATCH];
+        read_batch(0, next);
+        for (int first = 0; first < total; first += BATCH * G_THREADS)
+        {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+                v[u] = next[u];
+            if (first + BATCH * G_THREADS < total)
+                read_batch(first + BATCH * G_THREADS, next);
+            take(first + tid, v);
+        }
+    };
+    // (The values of a batch are counted per lane and their places in the queue follow from one prefix sum: with a ballot and
+    // its prefix count per value the wavefronts spent their time between the vector and the scalar unit.)
+    unsigned* const queue = reinterpret_cast<unsigned*>(below_total + 2) + wave * L_QUEUE;
+    int below = 0, queued = 0; // of this thread: entries before the span; of its wavefront: entries inside
+    read_entries([&](int e, const IdxT* v) {
+        unsigned t[BATCH];
+        int own = 0;
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
-            iv[u] = index_value(e0 + u * G_THREADS);
+        {
+            below += __builtin_sub_overflow(index_value(v[u]), static_cast<unsigned>(i0), &t[u]) ? 1 : 0;
+            own += t[u] < static_cast<unsigned>(width) ? 1 : 0;
+        }
+        const int before = wave_exclusive_sum(own);
+        const int all = __builtin_amdgcn_readlane(before + own, TPK_WAVE - 1);
+        if (queued + all <= L_QUEUE) // (wave-uniform)
+        {
+            unsigned* at = queue + queued + before;
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-            count_one(iv[u]);
-    }
+            for (int u = 0; u < BATCH; ++u)
+                if (t[u] < static_cast<unsigned>(width))
+                    *at++ = t[u] << L_ENTRY_BITS | static_cast<unsigned>(e + u * G_THREADS);
+        }
+        queued += all;
+    });
     {
         const int below_before = wave_exclusive_sum(below);
         if (lane == TPK_WAVE - 1)
             atomicAdd(below_total, below_before + below);
     }
+    const bool noted = __syncthreads_or(queued > L_QUEUE) == 0; // every entry of the span is in a queue
+    // Entries that crowd into one span: their targets are read again, without the queues.
+    if (noted)
+        for (int q = lane; q < queued; q += TPK_WAVE)
+            atomicAdd(&counters[queue[q] >> L_ENTRY_BITS], 1);
+    else
+        read_entries([&](int, const IdxT* v) {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+            {
+                const unsigned t = index_value(v[u]) - static_cast<unsigned>(i0);
+                if (t < static_cast<unsigned>(width))
+                    atomicAdd(&counters[t], 1);
+            }
+        });
     __syncthreads();
 
     // Prefix sum of the list lengths, an empty list counting as one entry (every thread owns a run of
@@ -283,72 +325,69 @@ __global__ __launch_bounds__(G_THREADS) void build_lists_kernel(ListJob<WEIGHTED
     }
     __syncthreads();
 
-    // Second pass.  Only one entry in L_SPANS lies inside the span: a wavefront first gathers those of its lanes
-    // into a queue of its own in LDS (ballot + prefix count), and whenever 64 are waiting every lane takes one:
-    // the next free place of its list, front to back.  `counters` holds the number of places still free, so the
-    // entry that takes the last one knows that it ends the list.
-    int2* const queue = reinterpret_cast<int2*>(below_total + 2) + wave * L_QUEUE;
-    int queued = 0, placed = 0; // (wave-uniform)
-    // An entry's weight is a trip to memory: the 64 entries taken from the queue wait for theirs while the next
-    // ones are queued, and go to their places when the queue has filled again (or at the end).
-    bool waiting = false; // per lane: an entry taken from the queue, not yet placed
-    int waiting_rank = 0, waiting_target = 0;
-    ListEntry<WEIGHTED> waiting_entry;
-    auto place_waiting = [&]() {
-        if (waiting)
-            place(waiting_rank, waiting_target, waiting_entry);
-        waiting = false;
+    // Second pass: an entry takes the next free place of its list, front to back.  `counters` holds the number of places
+    // still free, so the entry that takes the last one knows that it ends the list.
+    auto place_entry = [&](int e, unsigned t, [[maybe_unused]] float w) {
+        const int free_places = atomicSub(&counters[t], 1);
+        ListEntry<WEIGHTED> entry;
+        entry.j = ((e / K) * 4) | (free_places == 1 ? L_LAST : 0);
+        if constexpr (WEIGHTED)
+            entry.w = w;
+        place(ends[t] - free_places, i0 + static_cast<int>(t), entry);
     };
-    auto place_queued = [&](int count) {
-        place_waiting();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        if (lane < count)
+    if (noted)
+    {
+        constexpr int AT_ONCE = 4;
+        for (int first = lane; first < queued; first += AT_ONCE * TPK_WAVE)
         {
-            const int2 item = queue[(placed + lane) & (L_QUEUE - 1)];
-            const int e = item.x, t = item.y - i0;
-            const int left = atomicSub(&counters[t], 1); // places free before this entry took one
-            waiting_entry.j = ((e / K) * 4) | (left == 1 ? L_LAST : 0);
-            if constexpr (WEIGHTED)
-                waiting_entry.w = weight[e];
-            waiting_rank = ends[t] - left;
-            waiting_target = item.y;
-            waiting = true;
-        }
-        placed += count;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    };
-    auto enqueue = [&](int e, int v) {
-        const bool mine = v >= i0 && v < i1;
-        const unsigned long long mask = __ballot(mine);
-        if (mask == 0) // (wave-uniform)
-            return;
-        if (mine)
-            queue[(queued + static_cast<int>(tpk_prefix_count(mask))) & (L_QUEUE - 1)] = make_int2(e, v);
-        queued += __builtin_popcountll(mask);
-        if (queued - placed >= TPK_WAVE)
-            place_queued(TPK_WAVE);
-    };
+            unsigned note[AT_ONCE];
+            [[maybe_unused]] float w[AT_ONCE];
 #pragma unroll
-    for (int b = 0; b < L_CACHED<K>; b += BATCH)
-        if (b * G_THREADS < total) // (wave-uniform)
-        {
+            for (int u = 0; u < AT_ONCE; ++u)
+            {
+                note[u] = queue[min(first + u * TPK_WAVE, queued - 1)];
+                if constexpr (WEIGHTED)
+                    w[u] = weight[note[u] & ((1u << L_ENTRY_BITS) - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < AT_ONCE; ++u)
+                if (first + u * TPK_WAVE < queued)
+                {
+                    float own = 0.f;
+                    if constexpr (WEIGHTED)
+                        own = w[u];
+                    place_entry(static_cast<int>(note[u] & ((1u << L_ENTRY_BITS) - 1)), note[u] >> L_ENTRY_BITS, own);
+                }
+        }
+    }
+    else
+        read_entries([&](int e, const IdxT* v) {
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-                enqueue((b + u) * G_THREADS + tid, cached[b + u]);
-        }
-    // (the rounds behind the cached ones; the trip count is the same for every lane of a wavefront)
-    for (int e0 = L_CACHED<K> * G_THREADS + tid; e0 - tid < total; e0 += BATCH * G_THREADS)
-    {
-        int iv[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-            iv[u] = index_value(e0 + u * G_THREADS);
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-            enqueue(e0 + u * G_THREADS, iv[u]);
-    }
-    place_queued(queued - placed);
-    place_waiting();
+            {
+                const unsigned t = index_value(v[u]) - static_cast<unsigned>(i0);
+                if (t < static_cast<unsigned>(width))
+                {
+                    float own = 0.f;
+                    if constexpr (WEIGHTED)
+                        own = weight[e + u * G_THREADS];
+                    place_entry(e + u * G_THREADS, t, own);
+                }
+            }
+        });
+}
+
+template <int K, bool WEIGHTED, typename IdxT>
+__global__ __launch_bounds__(G_THREADS, 8) void build_lists_kernel(ListJob<WEIGHTED, IdxT> job)
+{
+    extern __shared__ int list_memory[];
+    build_lists<K, WEIGHTED, IdxT>(job, static_cast<int>(blockIdx.x), list_memory);
+}
+
+// Bytes of LDS a workgroup of the builder takes for spans of `span` targets.
+inline size_t list_lds_bytes(int span)
+{
+    return (2 * static_cast<size_t>(span) + G_THREADS / TPK_WAVE + 2 + G_THREADS / TPK_WAVE * L_QUEUE) * sizeof(int);
 }
 
 // Describes the job of building the lists of `clouds` clouds of `m` targets and `cloud_total`
@@ -366,8 +405,8 @@ int make_list_job(int clouds, int m, int64_t cloud_total, int64_t part_total, co
         return TPK_ERR_INVALID_ARG;
     const int64_t parts = tpk_ceil_div(cloud_total, part_total);
     const int64_t span = tpk_ceil_div(m, L_SPANS);
-    // (ranks inside a span must stay below 2^24 for the float division of the builder)
-    if (span > L_MAX_SPAN || part_total + span >= (1 << 24) || list_capacity(m, part_total) * 8 > 0x7fffffffLL ||
+    static_assert(L_MAX_PART<K> + L_MAX_SPAN < (1 << 24), "ranks inside a span: the builder divides them in float");
+    if (span > L_MAX_SPAN || part_total > L_MAX_PART<K> || list_capacity(m, part_total) * 8 > 0x7fffffffLL ||
         cloud_total > 0x7fffffffLL || clouds * parts * L_SPANS > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
     job->m = m;
@@ -390,8 +429,7 @@ int launch_build_lists(int clouds, int m, int64_t cloud_total, int64_t part_tota
     const int st = make_list_job<K, WEIGHTED, IdxT>(clouds, m, cloud_total, part_total, idx, weight, lists, &job);
     if (st != TPK_OK || job.workgroups == 0)
         return st;
-    const size_t lds = (2 * static_cast<size_t>(job.span) + G_THREADS / TPK_WAVE + 2) * sizeof(int) +
-                       static_cast<size_t>(G_THREADS / TPK_WAVE) * L_QUEUE * sizeof(int2);
+    const size_t lds = list_lds_bytes(job.span);
     auto build = build_lists_kernel<K, WEIGHTED, IdxT>;
     const int allowed = allow_lds(build, lds);
     if (allowed != TPK_OK)

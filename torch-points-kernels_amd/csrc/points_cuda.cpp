@@ -341,8 +341,7 @@ std::pair<at::Tensor, at::Tensor> grow_proximity(at::Tensor neighbours, int64_t 
     return std::make_pair(members.narrow(0, 0, found[1]), starts.narrow(0, 0, found[0] + 1));
 }
 
-// cuda/src/interpolate.cpp:34-54
-at::Tensor three_interpolate(at::Tensor points, at::Tensor idx, at::Tensor weight)
+void check_interpolate(const at::Tensor& points, const at::Tensor& idx, const at::Tensor& weight)
 {
     check_contiguous(points, "points");
     check_contiguous(idx, "idx");
@@ -359,6 +358,12 @@ at::Tensor three_interpolate(at::Tensor points, at::Tensor idx, at::Tensor weigh
     TORCH_CHECK(idx.dim() == 3 && idx.size(2) == 3 && idx.size(0) == points.size(0),
                 "idx must have shape (B, n, 3)");
     TORCH_CHECK(weight.sizes() == idx.sizes(), "weight must have the shape of idx");
+}
+
+// cuda/src/interpolate.cpp:34-54
+at::Tensor three_interpolate(at::Tensor points, at::Tensor idx, at::Tensor weight)
+{
+    check_interpolate(points, idx, weight);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(points.device());
 
     at::Tensor output = torch::empty({points.size(0), points.size(1), idx.size(1)},
@@ -419,25 +424,19 @@ at::Tensor three_interpolate_grad(at::Tensor grad_out, at::Tensor idx, at::Tenso
 // streams cost more than the 18 us they hide - 198 us per call against 52 us one after the other.)
 std::pair<at::Tensor, at::Tensor> three_interpolate_recording(at::Tensor points, at::Tensor idx, at::Tensor weight)
 {
-    check_contiguous(idx, "idx");
-    check_contiguous(weight, "weight");
-    check_gpu(points, "points");
-    check_gpu(idx, "idx");
-    check_gpu(weight, "weight");
-    check_dtype(idx, at::kInt, "idx");
-    check_f32(weight, "weight");
-    TORCH_CHECK(points.dim() == 3 && idx.dim() == 3 && idx.size(2) == 3 && weight.sizes() == idx.sizes(),
-                "points (B, c, m), idx and weight (B, n, 3) expected");
+    check_interpolate(points, idx, weight);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(points.device());
-    const int b = as_int(idx.size(0), "batch size"), n = as_int(idx.size(1), "n"), m = as_int(points.size(2), "m");
+    const int b = as_int(points.size(0), "batch size"), c = as_int(points.size(1), "channels"), m = as_int(points.size(2), "m");
+    const int n = as_int(idx.size(1), "n");
     const size_t bytes = tpk_three_interpolate_grad_workspace_bytes(b, n, m);
     if (bytes == 0)
         return {three_interpolate(points, idx, weight), torch::empty({0}, at::device(points.device()).dtype(at::kByte))};
     at::Tensor lists = torch::empty({static_cast<int64_t>(bytes)}, at::device(points.device()).dtype(at::kByte));
-    at::Tensor output = three_interpolate(points, idx, weight);
-    check_status(tpk_three_interpolate_lists_f32(b, n, m, idx.data_ptr<int32_t>(), weight.data_ptr<float>(), lists.data_ptr(),
-                                                 bytes, current_stream(points)),
-                 "three_interpolate (lists for the backward pass)");
+    at::Tensor output = torch::empty({points.size(0), points.size(1), idx.size(1)}, at::device(points.device()).dtype(at::kFloat));
+    check_status(tpk_three_interpolate_recording_f32(b, c, m, n, points.data_ptr<float>(), idx.data_ptr<int32_t>(),
+                                                     weight.data_ptr<float>(), output.data_ptr<float>(), lists.data_ptr(), bytes,
+                                                     current_stream(points)),
+                 "three_interpolate (with the lists for the backward pass)");
     return {output, lists};
 }
 
@@ -966,9 +965,7 @@ std::vector<at::Tensor> cubic_feature_sampling_grad(int scale, int neighborhood_
     return sample_cubes_grad(scale, neighborhood_size, grad_point_features, grid_pt_indexes, true);
 }
 
-// No counterpart in the reference's native module: its grouping_operation is
-// torch.gather on a repeated index (torch_points_kernels/torchpoints.py:129-146).
-at::Tensor grouping_operation(at::Tensor features, at::Tensor idx)
+void check_group(const at::Tensor& features, const at::Tensor& idx)
 {
     check_contiguous(features, "features");
     check_contiguous(idx, "idx");
@@ -980,6 +977,13 @@ at::Tensor grouping_operation(at::Tensor features, at::Tensor idx)
     TORCH_CHECK(features.dim() == 3, "features must have shape (B, C, N)");
     TORCH_CHECK(idx.dim() == 3 && idx.size(0) == features.size(0),
                 "idx must have shape (B, npoint, nsample)");
+}
+
+// No counterpart in the reference's native module: its grouping_operation is
+// torch.gather on a repeated index (torch_points_kernels/torchpoints.py:129-146).
+at::Tensor grouping_operation(at::Tensor features, at::Tensor idx)
+{
+    check_group(features, idx);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(features.device());
 
     at::Tensor out = torch::empty({features.size(0), features.size(1), idx.size(1), idx.size(2)},
@@ -1028,21 +1032,19 @@ at::Tensor grouping_operation_grad(at::Tensor grad_out, at::Tensor idx, const in
 // grouping_operation for a caller that will ask for the gradient: as three_interpolate_recording.
 std::pair<at::Tensor, at::Tensor> grouping_operation_recording(at::Tensor features, at::Tensor idx)
 {
-    check_contiguous(idx, "idx");
-    check_gpu(features, "features");
-    check_gpu(idx, "idx");
-    check_dtype(idx, at::kLong, "idx");
-    TORCH_CHECK(features.dim() == 3 && idx.dim() == 3, "features (B, C, N) and idx (B, npoint, nsample) expected");
+    check_group(features, idx);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(features.device());
-    const int b = as_int(idx.size(0), "batch size"), n = as_int(features.size(2), "N");
+    const int b = as_int(features.size(0), "batch size"), c = as_int(features.size(1), "channels"), n = as_int(features.size(2), "N");
     const int npoint = as_int(idx.size(1), "npoint"), nsample = as_int(idx.size(2), "nsample");
     const size_t bytes = tpk_group_grad_workspace_bytes(b, n, npoint, nsample);
     if (bytes == 0)
         return {grouping_operation(features, idx), torch::empty({0}, at::device(features.device()).dtype(at::kByte))};
     at::Tensor lists = torch::empty({static_cast<int64_t>(bytes)}, at::device(features.device()).dtype(at::kByte));
-    at::Tensor output = grouping_operation(features, idx);
-    check_status(tpk_group_lists(b, n, npoint, nsample, idx.data_ptr<int64_t>(), lists.data_ptr(), bytes, current_stream(features)),
-                 "grouping_operation (lists for the backward pass)");
+    at::Tensor output =
+        torch::empty({features.size(0), features.size(1), idx.size(1), idx.size(2)}, at::device(features.device()).dtype(at::kFloat));
+    check_status(tpk_group_recording_f32(b, c, n, npoint, nsample, features.data_ptr<float>(), idx.data_ptr<int64_t>(),
+                                         output.data_ptr<float>(), lists.data_ptr(), bytes, current_stream(features)),
+                 "grouping_operation (with the lists for the backward pass)");
     return {output, lists};
 }
 
