@@ -1728,6 +1728,42 @@ def test_chamfer_parity(tpk, oracle, dev, B, n, m, dtype):
     np.testing.assert_allclose(_np(gb), wb, rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("n,m", [(4095, 4096), (4097, 8192), (8193, 600), (12000, 16384), (16385, 20000)])
+@pytest.mark.parametrize("kind", ["even", "one place", "two places", "crowded"])
+def test_ordering_in_parts(dev, kind, n, m):
+    """The ordering of a window by several workgroups: sizes around the parts, and places that many points share, whose bin lies
+    across the parts' edges.  The search over the cells against the scan of all pairs."""
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_chamfer_fwd_workspace_bytes.restype = ctypes.c_size_t
+    g = torch.Generator().manual_seed(n + m)
+    clouds = []
+    for count in (n, m):
+        xyz = torch.rand(2, count, 3, generator=g)
+        if kind == "one place":
+            xyz[:] = 0.25
+        elif kind == "two places":
+            xyz = (torch.randint(0, 2, (2, count, 1), generator=g) * 0.5 + 0.25).expand(2, count, 3).contiguous()
+        elif kind == "crowded":
+            xyz[:, count // 5 : count // 5 * 4] = xyz[:, count // 5 : count // 5 * 4] * 1e-3 + 0.4
+        clouds.append(xyz.to(dev))
+    a, b = clouds
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    results = []
+    for nbytes in (lib.tpk_chamfer_fwd_workspace_bytes(2, n, m), 0):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+        out = [torch.full((2, k), -1, dtype=t, device=dev) for t in (torch.float32, torch.int32) for k in (n, m)]
+        st = lib.tpk_chamfer_fwd_f32(2, n, m, pointer(a), pointer(b), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None)
+        assert st == 0
+        torch.cuda.synchronize()
+        results.append([t.cpu() for t in out])
+    for cells, pairs in zip(*results):
+        assert torch.equal(cells, pairs)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_chamfer_backward_skewed_indices(tpk, dev, dtype):
     # The backward pass keeps, per range of points, the other cloud's points that chose one of them in LDS, with

@@ -4,12 +4,16 @@
 // sampling of clouds too large for registers (fps.hip).
 #pragma once
 
+#include <algorithm>
+
 #include "curve_order.h"
 
 namespace {
 
 constexpr int NG_CELL = 64;           // points per cell = lanes of a wavefront
 constexpr int NG_SORT_THREADS = 1024;
+constexpr int CURVE_STAGED = 4096;    // records of a window's part that are put in order in LDS (64 KB)
+constexpr int CURVE_PARTS = CURVE_MAX_POINTS / CURVE_STAGED; // parts of a window, at most
 constexpr int NG_BOX = 10;            // float4 per cell: box of the cell, then of its four runs of 16 points
 
 // A set of points to be ordered: `total` points in clouds of `cloud_points` consecutive points,
@@ -29,8 +33,9 @@ struct PointSet
     float4* boxes;        // [windows][cells][NG_BOX]: (lo.xyz, -), (hi.xyz, -) of the cell and of its quarters; or nullptr
     int* bin_ends;        // optional [windows][CURVE_BINS]: end of every bin of the counting sort
     float4* grid;         // optional [windows][2]: origin and scale of the window's 64^3 grid
-    int* wide_first;      // optional (with boxes) [windows][cells]: the window's cells, those with much wider boxes than
-                          // the window's average first - the cells whose queries take a search longest
+    int* wide_first;      // optional (with boxes) [windows][cells]: the cells of each of the window's parts (curve_parts()), those
+                          // with much wider boxes than the part's average first - the cells whose queries take a search longest;
+                          // the upper 16 bits of a part's first entry: how many of its cells are wide
     const int* only;      // optional [clouds]: a cloud whose word is 0 is left out (dense layout)
     const float4* records; // optional [total]: the points as (x, y, z, index) records to be read instead of xyz -
                            // an array that has been brought into a coarse order (coarse_order.h), whose records
@@ -118,42 +123,58 @@ __device__ __forceinline__ void cloud_rows_job(const CloudRows& job, int64_t gro
 
 constexpr float CURVE_WIDE_FACTOR = 3.0f; // a cell is wide when its box's squared diagonal exceeds this many times the window's average
 
-// One workgroup orders one window: the first windows_a blocks those of set_a, the rest set_b.
+// `parts` workgroups order one window: the first windows_a windows are those of set_a, the rest set_b.
 // `zero_word` (optional) is cleared by the first block: a counter used by the kernel that follows.
 // The window's points are read once and stay in registers (16 per thread): bounding box, curve
 // position of each point's cell of the 16^3 grid (a table in LDS), histogram and prefix sum over the
-// 4096 bins, and then every thread takes a place in its points' bins (LDS integer atomics) and stores
-// the records straight to their final positions.  The boxes of the cells are formed from the records
-// read back in order (one more trip to the L2 instead of random gathers of the coordinates).
+// 4096 bins, and then every thread takes a place in its points' bins (LDS integer atomics).
 // Inside a bin (1/16 of the window's extent per axis) the order is that in which the atomics were
 // served; it decides where a point sits inside its bin, never what a search over the cells returns.
-// dynamic LDS: (2 * CURVE_BINS + 24 * cells) words.
+//
+// STAGED: the workgroup keeps the places of its part of the window's cells, puts their records in order in LDS and writes them and
+// the boxes of their runs from there.  A record stored to its place by itself costs the compute unit's way to memory two clocks, as
+// much as all the counting, and of the launch's windows there are fewer than compute units: every part counts the whole window and
+// stores a share.  One window of 16384 points with boxes took 63000 clocks (18500 of them the stores, 20800 the boxes), a quarter of
+// it takes 41000; the ordering of 64 of them 32.0 -> 22.9 us, Chamfer forward of 32 x 16384 points 164 -> 146, of one cloud 72 -> 62.
+// Not STAGED (parts == 1; larger windows that are as many as compute units): the records go straight to their places, the boxes are
+// formed from the records read back in order (one more trip to the L2 instead of random gathers of the coordinates).
+// dynamic LDS: (2 * CURVE_BINS + 24 * cells of a part) words, STAGED also the part's records.
+template <bool STAGED>
 __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet set_a, PointSet set_b,
-                                                                      int windows_a, int windows, int* zero_word,
+                                                                      int windows_a, int windows, int parts, int* zero_word,
                                                                       CloudRows rows_job)
 {
+    constexpr int PER = CURVE_MAX_POINTS / NG_SORT_THREADS; // points per thread
     extern __shared__ unsigned bin_of_cell[];  // [CURVE_BINS] curve position of every cell of the 16^3 grid
     int* const bins = reinterpret_cast<int*>(bin_of_cell) + CURVE_BINS; // [CURVE_BINS]
-    int* const run_boxes = bins + CURVE_BINS;  // [cells * 4][6] ordered ints: boxes of the runs of 16 records
+    int* const run_boxes = bins + CURVE_BINS;  // [part's cells * 4][6] ordered ints: boxes of the runs of 16 records
+    float4* const stage = reinterpret_cast<float4*>(run_boxes); // (STAGED) [part's cells * 64] the records, before run_boxes
     __shared__ int cloud_box[6];
+    __shared__ int edge_bin[2], edge_start[2], edge_ends[2]; // the bins that hold the places before the part's first, and its last
+    __shared__ unsigned edge_totals[NG_SORT_THREADS / TPK_WAVE];
     __shared__ int wave_totals[NG_SORT_THREADS / TPK_WAVE];
     __shared__ float wide_sums[NG_SORT_THREADS / TPK_WAVE];
-    constexpr int PER = CURVE_MAX_POINTS / NG_SORT_THREADS; // points per thread
     static_assert(CURVE_BINS % NG_SORT_THREADS == 0, "every thread scans the same number of bins");
 
-    if (static_cast<int>(blockIdx.x) >= windows)
+    if (static_cast<int>(blockIdx.x) >= windows * parts)
     {
-        cloud_rows_job(rows_job, static_cast<int>(blockIdx.x) - windows, threadIdx.x);
+        cloud_rows_job(rows_job, static_cast<int>(blockIdx.x) - windows * parts, threadIdx.x);
         return;
     }
-    const bool first_set = static_cast<int>(blockIdx.x) < windows_a;
+    // (the workgroups of a window run on one die, which reads the window once: 14900 -> 6000 clocks for the loads)
+    const int task = static_cast<int>(xcd_local_block(blockIdx.x, static_cast<unsigned>(windows * parts)));
+    const int block = task / parts, part = task - block * parts;
+    const bool first_set = block < windows_a;
     const PointSet set = first_set ? set_a : set_b;
-    const int64_t window = first_set ? blockIdx.x : blockIdx.x - windows_a;
+    const int64_t window = first_set ? block : block - windows_a;
     const int per_cloud = set_windows_per_cloud(set);
     const int64_t in_cloud = (window % per_cloud) * static_cast<int64_t>(set.stride);
     const int64_t start = (window / per_cloud) * set.cloud_points + in_cloud;
     const int n = static_cast<int>(tpk_min64(set.stride, set.cloud_points - in_cloud));
     const int cells = set_cells(set);
+    // the cells of this part, and the places [place_lo, place_hi) of the points in them
+    const int part_cells = (cells + parts - 1) / parts, cell_lo = min(part * part_cells, cells), cell_hi = min(cell_lo + part_cells, cells);
+    const int place_lo = cell_lo * NG_CELL, place_hi = min(cell_hi * NG_CELL, n);
     const float* __restrict__ xyz = set.xyz + start * 3;
     const float4* __restrict__ records = set.records ? set.records + start : nullptr;
     const int64_t* __restrict__ group = set.group ? set.group + start : nullptr;
@@ -162,7 +183,7 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
     const int tid = threadIdx.x;
     const int lane = tid & (TPK_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
-    if (zero_word && blockIdx.x == 0 && tid == 0)
+    if (zero_word && task == 0 && tid == 0)
         *zero_word = 0;
     if (set.only && set.only[window / per_cloud] == 0)
         return; // (before the first barrier)
@@ -201,6 +222,8 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
     const int empty_hi = float_to_ordered_int(-__builtin_inff());
     if (tid < 6)
         cloud_box[tid] = tid < 3 ? empty_lo : empty_hi;
+    if (tid < 2)
+        edge_bin[tid] = -1;
     for (int i = tid; i < CURVE_BINS; i += NG_SORT_THREADS)
     {
         bins[i] = 0;
@@ -239,7 +262,7 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
 #pragma unroll
         for (int u = 0; u < PER; ++u)
         {
-            bin[u] = 0;
+            bin[u] = -2; // no point
             if (u * NG_SORT_THREADS >= n) // (uniform over the workgroup: a short window has fewer rounds)
                 continue;
             unsigned cell[3];
@@ -251,9 +274,11 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
             {
                 b = (static_cast<unsigned>(id_offset[u]) << 9) | (b >> 3);
             }
-            bin[u] = static_cast<int>(b);
             if (tid + u * NG_SORT_THREADS < n)
+            {
+                bin[u] = static_cast<int>(b);
                 atomicAdd(&bins[b], 1);
+            }
         }
     }
     __syncthreads();
@@ -277,17 +302,75 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
 #pragma unroll
         for (int i = 0; i < CURVE_BINS / NG_SORT_THREADS; ++i)
         {
-            bins[tid * (CURVE_BINS / NG_SORT_THREADS) + i] = run;
-            run += count[i];
+            const int b = tid * (CURVE_BINS / NG_SORT_THREADS) + i, end = run + count[i];
+            bins[b] = run;
+            run = end;
+            if constexpr (!STAGED)
+                continue;
+#pragma unroll
+            for (int edge = 0; edge < 2; ++edge)
+            {
+                const int at = edge == 0 ? place_lo : place_hi;
+                if (end - count[i] < at && end >= at)
+                {
+                    edge_bin[edge] = b;
+                    edge_start[edge] = end - count[i];
+                    edge_ends[edge] = end;
+                }
+            }
+            if (set.bin_ends && part == 0) // (the bin of a point is the leading 12 bits of its position on the curve: the cell
+                set.bin_ends[window * CURVE_BINS + b] = end; // of the 16^3 grid it lies in, curve_bin_of_cell())
         }
     }
     __syncthreads();
     // every point takes the next place of its bin; its record goes straight there
     {
+        // The part's bins.  A bin that also has places in the part before or behind is an edge of both; the places of its
+        // points follow from their numbers, the same in both.
+        const bool cut_lo = STAGED && edge_bin[0] >= 0 && edge_ends[0] > place_lo, cut_hi = STAGED && edge_bin[1] >= 0 && edge_ends[1] > place_hi;
+        const int bin_lo = STAGED ? edge_bin[0] + 1 : 0, bin_hi = !STAGED ? CURVE_BINS : place_lo < place_hi ? edge_bin[1] + (cut_hi ? 0 : 1) : 0;
         int place[PER];
 #pragma unroll
         for (int u = 0; u < PER; ++u)
-            place[u] = tid + u * NG_SORT_THREADS < n ? atomicAdd(&bins[bin[u]], 1) : -1;
+            place[u] = bin[u] >= bin_lo && bin[u] < bin_hi ? atomicAdd(&bins[bin[u]], 1) : -1;
+        if ((cut_lo || cut_hi) && place_lo < place_hi) // (uniform over the workgroup)
+        {
+            const int low = cut_lo ? edge_bin[0] : -1, high = cut_hi && edge_bin[1] != low ? edge_bin[1] : -1;
+            bool any = false;
+#pragma unroll
+            for (int u = 0; u < PER; ++u)
+                any = any || bin[u] == low || bin[u] == high;
+            const bool some = __ballot(any) != 0; // (a bin holds a handful of points: few wavefronts have one)
+            unsigned before = 0;                  // (points of the two edges in the halves of a word: at most 16384)
+            if (some)
+            {
+                unsigned own = 0;
+#pragma unroll
+                for (int u = 0; u < PER; ++u)
+                    own += (bin[u] == low ? 1u : 0u) + (bin[u] == high ? 0x10000u : 0u);
+                before = static_cast<unsigned>(wave_exclusive_sum(static_cast<int>(own)));
+                if (lane == TPK_WAVE - 1)
+                    edge_totals[wave] = before + own;
+            }
+            else if (lane == 0)
+                edge_totals[wave] = 0;
+            __syncthreads();
+            if (some)
+            {
+                for (int w = 0; w < wave; ++w)
+                    before += edge_totals[w];
+                const int start_lo = edge_start[0], start_hi = edge_start[1];
+#pragma unroll
+                for (int u = 0; u < PER; ++u)
+                {
+                    const bool in_low = bin[u] == low, in_high = bin[u] == high;
+                    const int at = in_low ? start_lo + static_cast<int>(before & 0xFFFFu) : start_hi + static_cast<int>(before >> 16);
+                    before += (in_low ? 1u : 0u) + (in_high ? 0x10000u : 0u);
+                    if ((in_low || in_high) && at >= place_lo && at < place_hi)
+                        place[u] = at;
+                }
+            }
+        }
         // (records: the number a point had before the coarse order - read once more, the line is still near)
         int number[PER];
 #pragma unroll
@@ -303,22 +386,67 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
 #pragma unroll
         for (int u = 0; u < PER; ++u)
             if (place[u] >= 0)
-                sorted[place[u]] = make_float4(p[u][0], p[u][1], p[u][2], __int_as_float(number[u]));
+            {
+                const float4 record = make_float4(p[u][0], p[u][1], p[u][2], __int_as_float(number[u]));
+                if constexpr (STAGED)
+                    stage[place[u] - place_lo] = record;
+                else
+                    sorted[place[u]] = record;
+            }
     }
-    const int padded = cells * NG_CELL;
+    const int padded = cell_hi * NG_CELL; // (of this part)
     {
         // records behind the last point: infinitely far away
         const float inf = __builtin_inff();
-        for (int q = n + tid; q < padded; q += NG_SORT_THREADS)
-            sorted[q] = make_float4(inf, inf, inf, __int_as_float(0x7FFFFFFF));
+        for (int q = max(n, place_lo) + tid; q < padded; q += NG_SORT_THREADS)
+        {
+            const float4 record = make_float4(inf, inf, inf, __int_as_float(0x7FFFFFFF));
+            if constexpr (STAGED)
+                stage[q - place_lo] = record;
+            else
+                sorted[q] = record;
+        }
     }
-    // Every place is taken: `bins` now holds the end of every bin, and the records have been stored.  The barrier
+    int* const runs = STAGED ? reinterpret_cast<int*>(stage + part_cells * NG_CELL) : run_boxes;
+    auto run_box_of = [&](int q, const float4& record) {
+        const bool real = __float_as_int(record.w) != 0x7FFFFFFF;
+        const float v[3] = {record.x, record.y, record.z};
+        int lo[3], hi[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+        {
+            const int ordered = float_to_ordered_int(v[a]);
+            lo[a] = row_all_min_i32(real ? ordered : 0x7FFFFFFF);
+            hi[a] = row_all_max_i32(real ? ordered : INT_MIN);
+        }
+        if ((lane & 15) == 0)
+        {
+            int* const run_box = runs + ((q - place_lo) / 16) * 6;
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+            {
+                run_box[a] = lo[a];
+                run_box[3 + a] = hi[a];
+            }
+        }
+    };
+    // Every place is taken.  Not staged, the records have been stored, and the barrier
     // orders memory at workgroup scope, which is all the read-back below needs: the wavefronts of a workgroup share
     // one L1, which holds no older copy of these lines (a wider fence would write the whole L2 back: 20 us).
     __syncthreads();
-    if (boxes)
+    if constexpr (STAGED)
     {
-        // The records in order, as the other wavefronts stored them: boxes of the runs of 16 (DPP row reductions).
+        for (int q = place_lo + tid; q < padded; q += NG_SORT_THREADS)
+        {
+            const float4 record = stage[q - place_lo];
+            sorted[q] = record;
+            if (boxes) // boxes of the runs of 16 (DPP row reductions)
+                run_box_of(q, record);
+        }
+    }
+    else if (boxes)
+    {
+        // The records in order, as the other wavefronts stored them.
         constexpr int BATCH = 16; // (all records of a thread are requested before the first is used: one trip to the L2)
         for (int q0 = tid; q0 < padded; q0 += NG_SORT_THREADS * BATCH)
         {
@@ -328,33 +456,8 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
                 rec[u] = sorted[min(q0 + u * NG_SORT_THREADS, padded - 1)];
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-            {
-                const int q = q0 + u * NG_SORT_THREADS;
-                if (q >= padded) // uniform over the wavefront: cells are whole
-                    continue;
-                const bool real = __float_as_int(rec[u].w) != 0x7FFFFFFF;
-                const float inf = __builtin_inff();
-                const float v[3] = {rec[u].x, rec[u].y, rec[u].z};
-                (void)inf;
-                int lo[3], hi[3];
-#pragma unroll
-                for (int a = 0; a < 3; ++a)
-                {
-                    const int ordered = float_to_ordered_int(v[a]);
-                    lo[a] = row_all_min_i32(real ? ordered : 0x7FFFFFFF);
-                    hi[a] = row_all_max_i32(real ? ordered : INT_MIN);
-                }
-                if ((lane & 15) == 0)
-                {
-                    int* const run_box = run_boxes + (q / 16) * 6;
-#pragma unroll
-                    for (int a = 0; a < 3; ++a)
-                    {
-                        run_box[a] = lo[a];
-                        run_box[3 + a] = hi[a];
-                    }
-                }
-            }
+                if (q0 + u * NG_SORT_THREADS < padded) // uniform over the wavefront: cells are whole
+                    run_box_of(q0 + u * NG_SORT_THREADS, rec[u]);
         }
     }
     if (boxes)
@@ -362,7 +465,7 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
         // one thread per cell: the boxes of its four runs, and their union, to memory
         float diagonal2 = -1.f;
         __syncthreads();
-        for (int c = tid; c < cells; c += NG_SORT_THREADS)
+        for (int c = cell_lo + tid; c < cell_hi; c += NG_SORT_THREADS)
         {
             // (an empty run keeps (INT_MAX, INT_MIN), which map to NaN patterns: written as (+inf, -inf))
             auto as_lo = [](int o) { return o == 0x7FFFFFFF ? __builtin_inff() : ordered_int_to_float(o); };
@@ -371,7 +474,7 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
 #pragma unroll
             for (int r = 0; r < 4; ++r)
             {
-                const int* const run_box = run_boxes + (c * 4 + r) * 6;
+                const int* const run_box = runs + ((c - cell_lo) * 4 + r) * 6;
                 boxes[c * NG_BOX + 2 + r * 2 + 0] = make_float4(as_lo(run_box[0]), as_lo(run_box[1]), as_lo(run_box[2]), 0.f);
                 boxes[c * NG_BOX + 2 + r * 2 + 1] = make_float4(as_hi(run_box[3]), as_hi(run_box[4]), as_hi(run_box[5]), 0.f);
 #pragma unroll
@@ -383,7 +486,7 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
             }
             boxes[c * NG_BOX + 0] = make_float4(as_lo(lo[0]), as_lo(lo[1]), as_lo(lo[2]), 0.f);
             boxes[c * NG_BOX + 1] = make_float4(as_hi(hi[0]), as_hi(hi[1]), as_hi(hi[2]), 0.f);
-            if (c == tid && lo[0] != 0x7FFFFFFF) // (a cell that holds points: the squared diagonal of its box)
+            if (c == cell_lo + tid && lo[0] != 0x7FFFFFFF) // (a cell that holds points: the squared diagonal of its box)
             {
                 const float dx = as_hi(hi[0]) - as_lo(lo[0]), dy = as_hi(hi[1]) - as_lo(lo[1]), dz = as_hi(hi[2]) - as_lo(lo[2]);
                 diagonal2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
@@ -420,22 +523,22 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
                 before += w < wave ? wave_totals[w] : 0;
                 all_wide += wave_totals[w];
             }
-            if (tid < cells)
-                set.wide_first[window * cells + (wide ? before : all_wide + tid - before)] = tid;
+            if (tid < cell_hi - cell_lo)
+            {
+                const int at = wide ? before : all_wide + tid - before;
+                set.wide_first[window * cells + cell_lo + at] = (cell_lo + tid) | (at == 0 ? all_wide << 16 : 0);
+            }
         }
     }
-    if (set.bin_ends)
+    if constexpr (!STAGED)
+        if (set.bin_ends) // bins[i] is the end of bin i on the curve: every place is taken
+            for (int i = tid; i < CURVE_BINS; i += NG_SORT_THREADS)
+                set.bin_ends[window * CURVE_BINS + i] = bins[i];
+    if (set.bin_ends && part == 0 && tid == 0)
     {
-        // bins[i] is the end of bin i on the curve; the bin of a point is the leading 12 bits of
-        // its position: the cell of the 16^3 grid it lies in (curve_bin_of_cell()).
-        for (int i = tid; i < CURVE_BINS; i += NG_SORT_THREADS)
-            set.bin_ends[window * CURVE_BINS + i] = bins[i];
-        if (tid == 0)
-        {
-            const CurveGrid grid = curve_grid(cloud_box);
-            set.grid[window * 2 + 0] = make_float4(grid.lo[0], grid.lo[1], grid.lo[2], 0.f);
-            set.grid[window * 2 + 1] = make_float4(grid.scale[0], grid.scale[1], grid.scale[2], 0.f);
-        }
+        const CurveGrid grid = curve_grid(cloud_box);
+        set.grid[window * 2 + 0] = make_float4(grid.lo[0], grid.lo[1], grid.lo[2], 0.f);
+        set.grid[window * 2 + 1] = make_float4(grid.scale[0], grid.scale[1], grid.scale[2], 0.f);
     }
 }
 
@@ -455,6 +558,14 @@ __device__ __forceinline__ float point_box_dist2(float x, float y, float z, floa
     return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
 }
 
+// Parts that the windows of a launch are cut into: such that a part's records fit in LDS, where the windows then still have a compute
+// unit per part; otherwise one.
+int curve_parts(const PointSet& a, const PointSet& c)
+{
+    const int64_t parts = tpk_ceil_div(std::max(a.stride, c.stride), CURVE_STAGED);
+    return (set_windows(a) + set_windows(c)) * parts <= TPK_COMPUTE_UNITS ? static_cast<int>(parts) : 1;
+}
+
 int launch_curve_cells(const PointSet& a, const PointSet& c, int* zero_word, hipStream_t s,
                        const CloudRows& rows_job = CloudRows{nullptr, nullptr, 0, 0, nullptr})
 {
@@ -463,16 +574,20 @@ int launch_curve_cells(const PointSet& a, const PointSet& c, int* zero_word, hip
         return TPK_ERR_UNSUPPORTED; // (a thread holds 16 points of a window: windows of at most 16384 points)
     const int64_t windows_a = set_windows(a), windows_c = set_windows(c);
     const int64_t row_groups = tpk_ceil_div(rows_job.size_y, NG_SORT_THREADS);
-    if (windows_a + windows_c + row_groups > 0x7fffffffLL)
+    if ((windows_a + windows_c) * CURVE_PARTS + row_groups > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    const size_t most_cells = static_cast<size_t>((largest + NG_CELL - 1) / NG_CELL);
-    const size_t lds = (2 * static_cast<size_t>(CURVE_BINS) + 24 * most_cells) * sizeof(unsigned);
-    const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(curve_cells_kernel), lds);
+    const int parts = curve_parts(a, c);
+    const int64_t part_cells = tpk_ceil_div(tpk_ceil_div(largest, NG_CELL), parts);
+    const bool staged = part_cells * NG_CELL <= CURVE_STAGED;
+    const size_t lds = (2 * static_cast<size_t>(CURVE_BINS) + 24 * static_cast<size_t>(part_cells)) * sizeof(unsigned) +
+                       (staged ? static_cast<size_t>(part_cells) * NG_CELL * sizeof(float4) : 0);
+    const auto kernel = staged ? curve_cells_kernel<true> : curve_cells_kernel<false>;
+    const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(kernel), lds);
     if (allowed != TPK_OK)
         return allowed;
-    hipLaunchKernelGGL(curve_cells_kernel, dim3(static_cast<unsigned>(windows_a + windows_c + row_groups)),
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((windows_a + windows_c) * parts + row_groups)),
                        dim3(NG_SORT_THREADS), lds, s, a, c, static_cast<int>(windows_a),
-                       static_cast<int>(windows_a + windows_c), zero_word, rows_job);
+                       static_cast<int>(windows_a + windows_c), parts, zero_word, rows_job);
     return tpk_launch_status();
 }
 

@@ -149,7 +149,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void chamfer_grid_kernel(
     const float4* __restrict__ sorted2, const float4* __restrict__ boxes1,
     const float4* __restrict__ boxes2, float* __restrict__ dist1, float* __restrict__ dist2,
     int32_t* __restrict__ idx1, int32_t* __restrict__ idx2, const int* __restrict__ wide1,
-    const int* __restrict__ wide2, int window_cells)
+    const int* __restrict__ wide2, int window_cells, int part_cells)
 {
     __shared__ float4 stages[NG_SCAN_THREADS / TPK_WAVE][NG_CELL];
     extern __shared__ float lows_all[]; // [wavefronts][largest number of candidate cells, in whole groups of 64]
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void chamfer_grid_kernel(
         // Wavefronts start in the order of their numbers, and the call lasts as long as the wavefront that ends
         // last: the cells with the widest boxes - whose queries search longest - go first.  The cells of both
         // clouds' windows are dealt out in groups of NG_DEAL windows, window after window, every window
-        // handing out its cells in the order the ordering kernel left: wide ones first.
+        // handing out its cells in the order the ordering kernel left: every part's wide ones first, then the others.
         const int per_cloud_windows = per_cloud / window_cells;
         const int64_t all_windows = static_cast<int64_t>(per_cloud_windows) * clouds;
         const int64_t group = task / (NG_DEAL * window_cells);
@@ -181,9 +181,29 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void chamfer_grid_kernel(
         const int windows1 = cells1 / window_cells;
         const bool in_second = k >= windows1;
         const int own = in_second ? k - windows1 : k; // the window's number in its cloud
-        const int* __restrict__ order = in_second ? wide2 + (static_cast<int64_t>(cloud) * (per_cloud_windows - windows1) + own) * window_cells
-                                                  : wide1 + (static_cast<int64_t>(cloud) * windows1 + own) * window_cells;
-        r = (in_second ? cells1 : 0) + own * window_cells + order[rank];
+        const int64_t at = in_second ? static_cast<int64_t>(cloud) * (per_cloud_windows - windows1) + own : static_cast<int64_t>(cloud) * windows1 + own;
+        const int* __restrict__ order = (in_second ? wide2 : wide1) + at * window_cells;
+        int wide_of[CURVE_PARTS]; // (parts that there are not: no cells)
+#pragma unroll
+        for (int p = 0; p < CURVE_PARTS; ++p)
+            wide_of[p] = p * part_cells < window_cells ? order[p * part_cells] >> 16 : 0;
+        int place = 0, left = rank; // the cell's place in `order`
+        bool found = false;
+#pragma unroll
+        for (int turn = 0; turn < 2; ++turn)
+#pragma unroll
+            for (int p = 0; p < CURVE_PARTS; ++p)
+            {
+                const int size = max(min(part_cells, window_cells - p * part_cells), 0);
+                const int count = turn == 0 ? wide_of[p] : size - wide_of[p];
+                if (!found && left < count)
+                {
+                    place = p * part_cells + (turn == 0 ? left : wide_of[p] + left);
+                    found = true;
+                }
+                left -= count;
+            }
+        r = (in_second ? cells1 : 0) + own * window_cells + (order[place] & 0xFFFF);
     }
     const bool second = r >= cells1;
     const int qcell = second ? r - cells1 : r;
@@ -1171,7 +1191,7 @@ int tpk_grid_chamfer_fwd(int b, int n, int m, const float* xyz1, const float* xy
                        ((std::max(cells1, cells2) + NG_CELL - 1) / NG_CELL * NG_CELL) * sizeof(float);
     hipLaunchKernelGGL(chamfer_grid_kernel, dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), lds, s, n,
                        m, cells1, cells2, b, a.sorted, c.sorted, a.boxes, c.boxes, dist1, dist2, idx1, idx2, a.wide_first,
-                       c.wide_first, window_cells);
+                       c.wide_first, window_cells, static_cast<int>(tpk_ceil_div(set_cells(a), curve_parts(a, c))));
     return tpk_launch_status();
 }
 
