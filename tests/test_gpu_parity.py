@@ -1728,6 +1728,39 @@ def test_chamfer_parity(tpk, oracle, dev, B, n, m, dtype):
     np.testing.assert_allclose(_np(gb), wb, rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("b,n,m", [(2, 1024, 1024), (3, 1025, 1024), (2, 4096, 4096), (2, 4097, 4097), (5, 16384, 8192), (2, 16385, 8192),
+                                   (200, 1500, 1024)])
+def test_three_nn_orders_the_clouds_it_gives_up(dev, b, n, m):
+    """Uneven clouds among even ones: their workgroups put them in order for the search that follows where they are enough,
+    a launch of its own does elsewhere.  Against the scan of all pairs."""
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_three_nn_workspace_bytes.restype = ctypes.c_size_t
+    g = torch.Generator().manual_seed(n + m)
+    unknown, known = torch.rand(b, n, 3, generator=g), torch.rand(b, m, 3, generator=g)
+    for cloud in range(1, b, 2):  # seven points in eight in a millionth of the volume
+        known[cloud, m // 8 :] = known[cloud, m // 8 :] * 1e-2 + 0.3
+        unknown[cloud, ::2] = unknown[cloud, ::2] * 1e-2 + 0.3
+    unknown, known = unknown.to(dev), known.to(dev)
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr())
+    nbytes = lib.tpk_three_nn_workspace_bytes(b, n, m)
+    assert nbytes > 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    results = []
+    for run in (lib.tpk_three_nn_f32, lib.tpk_three_nn_all_pairs_f32):
+        dist2 = torch.full((b, n, 3), -1.0, device=dev)
+        idx = torch.full((b, n, 3), -1, dtype=torch.int32, device=dev)
+        more = (pointer(ws), ctypes.c_size_t(nbytes)) if run is lib.tpk_three_nn_f32 else ()
+        assert run(b, n, m, pointer(unknown), pointer(known), pointer(dist2), pointer(idx), *more, None) == 0
+        torch.cuda.synchronize()
+        results.append((dist2.cpu(), idx.cpu()))
+    assert (ws[-256:].view(torch.int32)[: min(b, 64)].cpu() != 0).any() or b > 64  # (some cloud was given up)
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
 @pytest.mark.parametrize("n,m", [(4095, 4096), (4097, 8192), (8193, 600), (12000, 16384), (16385, 20000)])
 @pytest.mark.parametrize("kind", ["even", "one place", "two places", "crowded"])
 def test_ordering_in_parts(dev, kind, n, m):

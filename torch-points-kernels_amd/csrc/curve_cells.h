@@ -123,8 +123,7 @@ __device__ __forceinline__ void cloud_rows_job(const CloudRows& job, int64_t gro
 
 constexpr float CURVE_WIDE_FACTOR = 3.0f; // a cell is wide when its box's squared diagonal exceeds this many times the window's average
 
-// `parts` workgroups order one window: the first windows_a windows are those of set_a, the rest set_b.
-// `zero_word` (optional) is cleared by the first block: a counter used by the kernel that follows.
+// Orders part `part` of `parts` of a window of the set, by a workgroup of NG_SORT_THREADS; lds: curve_lds_bytes(), 16-byte aligned.
 // The window's points are read once and stay in registers (16 per thread): bounding box, curve
 // position of each point's cell of the 16^3 grid (a table in LDS), histogram and prefix sum over the
 // 4096 bins, and then every thread takes a place in its points' bins (LDS integer atomics).
@@ -138,14 +137,11 @@ constexpr float CURVE_WIDE_FACTOR = 3.0f; // a cell is wide when its box's squar
 // it takes 41000; the ordering of 64 of them 32.0 -> 22.9 us, Chamfer forward of 32 x 16384 points 164 -> 146, of one cloud 72 -> 62.
 // Not STAGED (parts == 1; larger windows that are as many as compute units): the records go straight to their places, the boxes are
 // formed from the records read back in order (one more trip to the L2 instead of random gathers of the coordinates).
-// dynamic LDS: (2 * CURVE_BINS + 24 * cells of a part) words, STAGED also the part's records.
 template <bool STAGED>
-__global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet set_a, PointSet set_b,
-                                                                      int windows_a, int windows, int parts, int* zero_word,
-                                                                      CloudRows rows_job)
+__device__ __forceinline__ void curve_cells_part(const PointSet& set, int64_t window, int part, int parts, unsigned* lds)
 {
     constexpr int PER = CURVE_MAX_POINTS / NG_SORT_THREADS; // points per thread
-    extern __shared__ unsigned bin_of_cell[];  // [CURVE_BINS] curve position of every cell of the 16^3 grid
+    unsigned* const bin_of_cell = lds;         // [CURVE_BINS] curve position of every cell of the 16^3 grid
     int* const bins = reinterpret_cast<int*>(bin_of_cell) + CURVE_BINS; // [CURVE_BINS]
     int* const run_boxes = bins + CURVE_BINS;  // [part's cells * 4][6] ordered ints: boxes of the runs of 16 records
     float4* const stage = reinterpret_cast<float4*>(run_boxes); // (STAGED) [part's cells * 64] the records, before run_boxes
@@ -156,17 +152,6 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
     __shared__ float wide_sums[NG_SORT_THREADS / TPK_WAVE];
     static_assert(CURVE_BINS % NG_SORT_THREADS == 0, "every thread scans the same number of bins");
 
-    if (static_cast<int>(blockIdx.x) >= windows * parts)
-    {
-        cloud_rows_job(rows_job, static_cast<int>(blockIdx.x) - windows * parts, threadIdx.x);
-        return;
-    }
-    // (the workgroups of a window run on one die, which reads the window once: 14900 -> 6000 clocks for the loads)
-    const int task = static_cast<int>(xcd_local_block(blockIdx.x, static_cast<unsigned>(windows * parts)));
-    const int block = task / parts, part = task - block * parts;
-    const bool first_set = block < windows_a;
-    const PointSet set = first_set ? set_a : set_b;
-    const int64_t window = first_set ? block : block - windows_a;
     const int per_cloud = set_windows_per_cloud(set);
     const int64_t in_cloud = (window % per_cloud) * static_cast<int64_t>(set.stride);
     const int64_t start = (window / per_cloud) * set.cloud_points + in_cloud;
@@ -183,10 +168,6 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
     const int tid = threadIdx.x;
     const int lane = tid & (TPK_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
-    if (zero_word && task == 0 && tid == 0)
-        *zero_word = 0;
-    if (set.only && set.only[window / per_cloud] == 0)
-        return; // (before the first barrier)
 
     // the points of this thread: tid, tid + 1024, ... (all loads issued before the first is used)
     float p[PER][3];
@@ -542,6 +523,39 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
     }
 }
 
+// The ordering of two sets: the first windows_a windows are those of set_a, the rest set_b.
+// `zero_word` (optional) is cleared by the first block: a counter used by the kernel that follows.
+template <bool STAGED>
+__global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet set_a, PointSet set_b,
+                                                                      int windows_a, int windows, int parts, int* zero_word,
+                                                                      CloudRows rows_job)
+{
+    extern __shared__ unsigned curve_lds[];
+    if (static_cast<int>(blockIdx.x) >= windows * parts)
+    {
+        cloud_rows_job(rows_job, static_cast<int>(blockIdx.x) - windows * parts, threadIdx.x);
+        return;
+    }
+    // (the workgroups of a window run on one die, which reads the window once: 14900 -> 6000 clocks for the loads)
+    const int task = static_cast<int>(xcd_local_block(blockIdx.x, static_cast<unsigned>(windows * parts)));
+    const int block = task / parts;
+    const bool first_set = block < windows_a;
+    const PointSet set = first_set ? set_a : set_b;
+    const int64_t window = first_set ? block : block - windows_a;
+    if (zero_word && task == 0 && threadIdx.x == 0)
+        *zero_word = 0;
+    if (set.only && set.only[window / set_windows_per_cloud(set)] == 0)
+        return;
+    curve_cells_part<STAGED>(set, window, task - block * parts, parts, curve_lds);
+}
+
+// Bytes of LDS for a part of `part_cells` cells.
+inline size_t curve_lds_bytes(int64_t part_cells, bool staged)
+{
+    return (2 * static_cast<size_t>(CURVE_BINS) + 24 * static_cast<size_t>(part_cells)) * sizeof(unsigned) +
+           (staged ? static_cast<size_t>(part_cells) * NG_CELL * sizeof(float4) : 0);
+}
+
 // Squared distance between two boxes / a point and a box (0 when they touch or overlap).
 __device__ __forceinline__ float box_box_dist2(float4 alo, float4 ahi, float4 blo, float4 bhi)
 {
@@ -579,8 +593,7 @@ int launch_curve_cells(const PointSet& a, const PointSet& c, int* zero_word, hip
     const int parts = curve_parts(a, c);
     const int64_t part_cells = tpk_ceil_div(tpk_ceil_div(largest, NG_CELL), parts);
     const bool staged = part_cells * NG_CELL <= CURVE_STAGED;
-    const size_t lds = (2 * static_cast<size_t>(CURVE_BINS) + 24 * static_cast<size_t>(part_cells)) * sizeof(unsigned) +
-                       (staged ? static_cast<size_t>(part_cells) * NG_CELL * sizeof(float4) : 0);
+    const size_t lds = curve_lds_bytes(part_cells, staged);
     const auto kernel = staged ? curve_cells_kernel<true> : curve_cells_kernel<false>;
     const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(kernel), lds);
     if (allowed != TPK_OK)

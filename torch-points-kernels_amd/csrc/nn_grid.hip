@@ -1209,8 +1209,16 @@ int* tpk_grid_three_nn_flags(int b, int n, int m, void* workspace, size_t worksp
     return reinterpret_cast<int*>(static_cast<char*>(workspace) + grid_layout(b, n, m).total);
 }
 
+GridCells tpk_grid_three_nn_cells(int b, int n, int m, void* workspace)
+{
+    const GridLayout l = grid_layout(b, n, m);
+    char* const w = static_cast<char*>(workspace);
+    return GridCells{reinterpret_cast<float4*>(w + l.sorted_a), reinterpret_cast<float4*>(w + l.sorted_b),
+                     reinterpret_cast<float4*>(w + l.boxes_b), grid_stride(n), grid_stride(m)};
+}
+
 int tpk_grid_three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2,
-                      int32_t* idx, bool root, void* workspace, size_t workspace_bytes, bool flagged, hipStream_t s)
+                      int32_t* idx, bool root, void* workspace, size_t workspace_bytes, bool flagged, bool ordered, hipStream_t s)
 {
     if (!grid_supported(b, n, m) || static_cast<int64_t>(b) * 2 > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
@@ -1220,13 +1228,17 @@ int tpk_grid_three_nn(int b, int n, int m, const float* unknown, const float* kn
     char* w = static_cast<char*>(workspace);
     const int* only = flagged ? reinterpret_cast<const int*>(w + l.total) : nullptr;
     // (the unknown points are only queried: no boxes of their cells - the search forms the box of its 64 queries)
-    PointSet a{unknown, nullptr, static_cast<int64_t>(b) * n, n, grid_stride(n), reinterpret_cast<float4*>(w + l.sorted_a),
+    const GridCells cells = tpk_grid_three_nn_cells(b, n, m, workspace);
+    PointSet a{unknown, nullptr, static_cast<int64_t>(b) * n, n, cells.window_unknown, cells.sorted_unknown,
                nullptr, nullptr, nullptr, nullptr, only};
-    PointSet c{known, nullptr, static_cast<int64_t>(b) * m, m, grid_stride(m), reinterpret_cast<float4*>(w + l.sorted_b),
-               reinterpret_cast<float4*>(w + l.boxes_b), nullptr, nullptr, nullptr, only};
-    int st = launch_curve_cells(a, c, nullptr, s);
-    if (st != TPK_OK)
-        return st;
+    PointSet c{known, nullptr, static_cast<int64_t>(b) * m, m, cells.window_known, cells.sorted_known,
+               cells.boxes_known, nullptr, nullptr, nullptr, only};
+    if (!ordered)
+    {
+        const int st = launch_curve_cells(a, c, nullptr, s);
+        if (st != TPK_OK)
+            return st;
+    }
     const int qcells = grid_cells(n), ccells = grid_cells(m);
     const int64_t waves = static_cast<int64_t>(qcells) * b;
     const int64_t blocks = tpk_ceil_div(waves, NG_SCAN_THREADS / TPK_WAVE);
