@@ -572,18 +572,24 @@ __device__ __forceinline__ float point_box_dist2(float x, float y, float z, floa
     return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
 }
 
+// (of sets that hold points)
+int largest_window(const PointSet& a, const PointSet& c)
+{
+    return std::max(a.total > 0 ? a.stride : 1, c.total > 0 ? c.stride : 1);
+}
+
 // Parts that the windows of a launch are cut into: such that a part's records fit in LDS, where the windows then still have a compute
 // unit per part; otherwise one.
 int curve_parts(const PointSet& a, const PointSet& c)
 {
-    const int64_t parts = tpk_ceil_div(std::max(a.stride, c.stride), CURVE_STAGED);
+    const int64_t parts = tpk_ceil_div(largest_window(a, c), CURVE_STAGED);
     return (set_windows(a) + set_windows(c)) * parts <= TPK_COMPUTE_UNITS ? static_cast<int>(parts) : 1;
 }
 
 int launch_curve_cells(const PointSet& a, const PointSet& c, int* zero_word, hipStream_t s,
                        const CloudRows& rows_job = CloudRows{nullptr, nullptr, 0, 0, nullptr})
 {
-    const int largest = a.stride > c.stride ? a.stride : c.stride;
+    const int largest = largest_window(a, c);
     if (largest > CURVE_MAX_POINTS)
         return TPK_ERR_UNSUPPORTED; // (a thread holds 16 points of a window: windows of at most 16384 points)
     const int64_t windows_a = set_windows(a), windows_c = set_windows(c);
