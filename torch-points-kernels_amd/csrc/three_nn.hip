@@ -254,8 +254,8 @@ __device__ __forceinline__ void three_nn_cells(
 }
 
 __global__ __launch_bounds__(LG_THREADS) void three_nn_cells_kernel(
-    int n, int m, int blocks_per_cloud, int queries_per_block, const float* unknown, const float* known, float* dist2, int32_t* idx,
-    bool root, int* general, HandOver over)
+    int n, int m, int blocks_per_cloud, int queries_per_block, const float* __restrict__ unknown, const float* __restrict__ known,
+    float* __restrict__ dist2, int32_t* __restrict__ idx, bool root, int* __restrict__ general, HandOver over)
 {
     three_nn_cells<true>(n, m, blocks_per_cloud, queries_per_block, unknown, known, dist2, idx, root, general, over);
 }
@@ -263,8 +263,8 @@ __global__ __launch_bounds__(LG_THREADS) void three_nn_cells_kernel(
 // Without the ordering of clouds that are given up, in half the registers, which lets the next workgroup onto a compute unit
 // before the last wavefront has ended: 300 clouds of 2048 points on 1024 take 110 us, 116 with the kernel above.
 __global__ __launch_bounds__(LG_THREADS) void three_nn_cells_many_kernel(
-    int n, int m, int blocks_per_cloud, int queries_per_block, const float* unknown, const float* known, float* dist2, int32_t* idx,
-    bool root, int* general, HandOver over)
+    int n, int m, int blocks_per_cloud, int queries_per_block, const float* __restrict__ unknown, const float* __restrict__ known,
+    float* __restrict__ dist2, int32_t* __restrict__ idx, bool root, int* __restrict__ general, HandOver over)
 {
     three_nn_cells<false>(n, m, blocks_per_cloud, queries_per_block, unknown, known, dist2, idx, root, general, over);
 }
