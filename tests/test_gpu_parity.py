@@ -1356,6 +1356,19 @@ def test_grow_proximity_in_several_turns(tpk, dev, n, nsample):
         assert torch.equal(some, members) and torch.equal(ends, starts)
 
 
+@pytest.mark.parametrize("n,clusters", [(1, 1), (2049, 3), (65536, 511), (65536, 1023), (65537, 1022), (140001, 1000)])
+def test_grow_proximity_many_clusters_by_index(dev, n, clusters):
+    # (cluster, block) tables around the 32768 entries that the prefix sum of the members' sort takes at a time: point i is listed
+    # with the points `clusters` before and behind it, so cluster c holds c, c + clusters, ...
+    native = __import__("torch_points_kernels._native", fromlist=["native"]).native()
+    i = torch.arange(n)
+    near = torch.stack([i, torch.where(i >= clusters, i - clusters, i), torch.where(i + clusters < n, i + clusters, i)], 1)
+    members, starts = native.grow_proximity(near.to(dev), 1, False, 1 << 28)
+    want = torch.cat([torch.arange(c, n, clusters) for c in range(min(clusters, n))])
+    sizes = torch.tensor([0] + [len(range(c, n, clusters)) for c in range(min(clusters, n))])
+    assert torch.equal(members.cpu(), want) and torch.equal(starts.cpu(), sizes.cumsum(0))
+
+
 def test_grow_proximity_any_matrix(tpk, oracle, dev):
     """Matrices that no ball query produces: rows ending early, entries after a -1 (ignored, the row has ended), chains
     in both directions, points nobody lists, no columns at all."""
