@@ -1443,6 +1443,27 @@ def test_fps_orders_a_whole_pool_at_once(tpk, oracle, dev, n):
     np.testing.assert_array_equal(_np(got), oracle.furthest_point_sample(clouds.numpy(), npoint))
 
 
+def test_fps_last_point_alone_among_equal_minima(tpk, oracle, dev):
+    """16384 points on the corners of a cube and, outside one of them, on two places side by side: point 0 and ten others on one,
+    the last point by itself on the other, so that it is taken when everything else has been.  Where the curve ends with those
+    two places the word that ranks the last point among equal minima is the largest there is."""
+    n = 16384
+    clouds = []
+    for corner in range(8):
+        for axis in range(3):
+            at = torch.tensor([(corner >> a) & 1 for a in range(3)], dtype=torch.float32)
+            outside = at + 0.1 * (2 * at - 1)
+            others = torch.arange(n) % 8
+            xyz = torch.stack([(others >> a) & 1 for a in range(3)], -1).float()
+            xyz[:1] = xyz[1000:1010] = outside
+            xyz[n - 1] = outside
+            xyz[n - 1, axis] = at[axis]
+            clouds.append(xyz + 1.0)
+    clouds = torch.stack(clouds)
+    got = tpk.furthest_point_sample(clouds.to(dev), 14)
+    np.testing.assert_array_equal(_np(got), oracle.furthest_point_sample(clouds.numpy(), 14))
+
+
 # ------------------------------------------------------------------ instance IoU
 
 

@@ -767,7 +767,7 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
             const int slot = static_cast<int>(lowest & 15u);
 #pragma unroll
             for (int i = 0; i < PPT; ++i)
-                if (i == slot && key == lowest)
+                if (i == slot && key == lowest && t[i] == most) // (the last of 16384 points in slot 15 has the key of the lanes without one)
                 {
                     offers[turn][wave] = make_float4(x[i], y[i], z[i], __int_as_float(most));
                     offer_places[turn][wave] = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
