@@ -1443,6 +1443,18 @@ def test_fps_orders_a_whole_pool_at_once(tpk, oracle, dev, n):
     np.testing.assert_array_equal(_np(got), oracle.furthest_point_sample(clouds.numpy(), npoint))
 
 
+@pytest.mark.parametrize("n,side", [(700, 12), (2048, 30), (4096, 12), (8192, 40), (16384, 24), (16384, 100)])
+def test_fps_distances_apart_by_their_rounding(tpk, oracle, dev, n, side):
+    """Lattices whose spacing is not a binary fraction: classes of minima a few units in the last place wide, of which a pool has to
+    take the upper part, and classes of exactly equal ones around the number that a pool takes."""
+    g = torch.Generator().manual_seed(n + side)
+    odd = (torch.randint(0, side, (n, 3), generator=g).float() + 0.5) / side
+    clouds = torch.stack([odd, odd * 0.1 + 0.7, torch.randint(0, side, (n, 3), generator=g) * 0.25 + 1.0])
+    npoint = min(n // 2, 1500)
+    got = tpk.furthest_point_sample(clouds.to(dev), npoint)
+    np.testing.assert_array_equal(_np(got), oracle.furthest_point_sample(clouds.numpy(), npoint))
+
+
 def test_fps_last_point_alone_among_equal_minima(tpk, oracle, dev):
     """16384 points on the corners of a cube and, outside one of them, on two places side by side: point 0 and ten others on one,
     the last point by itself on the other, so that it is taken when everything else has been.  Where the curve ends with those

@@ -524,9 +524,12 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
                         v[u] = u * TPK_WAVE + own_lane < count ? __float_as_int(pool[u * TPK_WAVE + own_lane].w) : INT_MIN;
                         most = max(most, v[u]);
                     }
+                    // (Ten halvings tell apart what lies a thousandth of the pool's range from each other.  On a lattice whose
+                    // distances differ by their rounding alone they left nothing, and a sample at a time was taken instead: 4096 of
+                    // 16384 points of a lattice of 100^3 3750 -> 1043 us, of 2048 points of one of 30^3 206 -> 128.)
                     int high = wave_max_to_scalar(most), low = floor_bits, share = (TPK_WAVE - 6) * 256 / count;
                     count = 0;
-                    for (int tries = 0; tries < 10; ++tries)
+                    for (int tries = 0; tries < 10 || (count == 0 && high - low > 1); ++tries)
                     {
                         // (first where they would lie if they were evenly spread)
                         const int middle = high - static_cast<int>(static_cast<long long>(high - low) * share / 256);
