@@ -28,6 +28,7 @@
 #include "coarse_order.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace {
 
@@ -182,6 +183,19 @@ __device__ __forceinline__ int not_hoisted(int v)
 {
     asm volatile("" : "+v"(v));
     return v;
+}
+
+// Calls f with the slot (LOW .. LOW + N - 1, the same in all lanes) as a constant: log2(N) branches instead of N in a row,
+// each of them 24 clocks of all wavefronts of a SIMD (1024 samples of 16384 points on 1728 places, taken one by one: 2590 -> 2297 us).
+template <int LOW, int N, typename F>
+__device__ __forceinline__ void with_slot(int slot, F&& f)
+{
+    if constexpr (N == 1)
+        f(std::integral_constant<int, LOW>{});
+    else if (slot < LOW + N / 2)
+        with_slot<LOW, N / 2>(slot, f);
+    else
+        with_slot<LOW + N / 2, N / 2>(slot, f);
 }
 
 // Position on the sorted curve of member `e` of group `g` held by lane `lane` of wavefront `wave`.
@@ -768,13 +782,14 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
             }
             const unsigned lowest = wave_min_u32(key);
             const int slot = static_cast<int>(lowest & 15u);
-#pragma unroll
-            for (int i = 0; i < PPT; ++i)
-                if (i == slot && key == lowest && t[i] == most) // (the last of 16384 points in slot 15 has the key of the lanes without one)
+            with_slot<0, PPT>(slot, [&](auto chosen) __attribute__((always_inline)) {
+                constexpr int i = chosen.value;
+                if (key == lowest && t[i] == most) // (the last of 16384 points in slot 15 has the key of the lanes without one)
                 {
                     offers[turn][wave] = make_float4(x[i], y[i], z[i], __int_as_float(most));
                     offer_places[turn][wave] = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
                 }
+            });
         }
         else
         {
