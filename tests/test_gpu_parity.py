@@ -1042,17 +1042,22 @@ def test_grouping_grad_long_rows(tpk, oracle, dev, N, npoint, nsample, C):
 
 @pytest.mark.parametrize("B,C,m,n", [(1, 1, 1, 1), (1, 3, 15, 1023), (2, 9, 16, 1024), (2, 5, 17, 1025), (1, 2, 300, 16385), (2, 2, 3000, 32768),
                                      (1, 7, 4096, 32769), (1, 2, 20481, 4097), (16, 64, 1024, 4096)])
-@pytest.mark.parametrize("kind", ["spread", "one target", "last targets"])
+@pytest.mark.parametrize("kind", ["spread", "one target", "last targets", "crowded first", "crowded last", "crowded in turn"])
 def test_gather_with_the_lists_of_its_gradient(tpk, dev, kind, B, C, m, n):
     # the gather and the lists of its backward pass in one launch: the same bits as the gather alone, and - small integers
     # throughout, whose sums are exact in any order - the exact gradient.  Sizes around a round of 1024 entries, a word of 32 rounds,
-    # the 16 spans and the rows that fit half of the LDS
+    # the 16 spans and the rows that fit half of the LDS; entries that crowd into the first span from the start, from somewhere on
+    # or for half of the wavefronts alone, more than a wavefront notes
     g = torch.Generator().manual_seed(m + n)
     idx = torch.randint(0, m, (B, n, 3), generator=g)
     if kind == "one target":
         idx[:] = m // 2
     elif kind == "last targets":
         idx = m - 1 - idx % min(m, 3)
+    elif kind.startswith("crowded"):
+        column = torch.arange(n)
+        crowd = {"first": column < n // 2, "last": column >= n // 3, "in turn": column % 1024 < 512}[kind[8:]]
+        idx[:, crowd] = idx[:, crowd] % max(1, m // 20)
     feats = torch.randint(-8, 9, (B, C, m), generator=g).float()
     weight = torch.randint(0, 5, (B, n, 3), generator=g).float()
     gout = torch.randint(-8, 9, (B, C, n), generator=g).float()

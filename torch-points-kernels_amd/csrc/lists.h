@@ -130,6 +130,12 @@ struct ListJob
 // entry) and places its entries in a second pass over the notes.  Index values outside [0, m) are dropped.
 // LDS (`counters`): list_lds_bytes().
 //
+// Where more entries of a wavefront crowd into the span than it can note, it counts the rest as it reads them and reads those once
+// more to place them.  The index of a padded ball query is like that: every empty slot repeats the lowest row of its ball, and the
+// first span of a cloud gets three to six times its share.  16 clouds, 32768 entries on 4096 targets, balls of 2, 4, 8, 16 points in
+// 32 slots 13, 16, 20, 21 us (even 12; with the whole part read twice more 21, 25, 30, 31; with all values in registers 15, 18, 23,
+// 24), 4 x 90000 weighted entries, Zipf exponent 0.7 and 1, 22 and 35 (42 and 45; 30 and 34).
+//
 // Bound by the instructions of the first pass, as all but one entry in L_SPANS are read in vain, and by the stores of single
 // entries.  A part's workgroups run on one die, which reads its index once.  Keeping every index value in registers for a second
 // pass over all of them took 12900 + 15300 clocks for the two passes at 16384 x 3 entries (124 registers, 17.2 us), the notes
@@ -196,10 +202,11 @@ __device__ __forceinline__ void build_lists(const ListJob<WEIGHTED, IdxT>& job, 
             }
         }
     };
-    auto read_entries = [&](auto&& take) { // (first entry of the thread in the batch, the batch's values)
+    auto read_entries = [&](int from, auto&& take) { // (first entry of the thread in the batch, the batch's values)
         IdxT v[BATCH], next[BATCH];
-        read_batch(0, next);
-        for (int first = 0; first < total; first += BATCH * G_THREADS)
+        if (from < total)
+            read_batch(from, next);
+        for (int first = from; first < total; first += BATCH * G_THREADS)
         {
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
@@ -212,8 +219,9 @@ __device__ __forceinline__ void build_lists(const ListJob<WEIGHTED, IdxT>& job, 
     // (The values of a batch are counted per lane and their places in the queue follow from one prefix sum: with a ballot and
     // its prefix count per value the wavefronts spent their time between the vector and the scalar unit.)
     unsigned* const queue = reinterpret_cast<unsigned*>(below_total + 2) + wave * L_QUEUE;
-    int below = 0, queued = 0; // of this thread: entries before the span; of its wavefront: entries inside
-    read_entries([&](int e, const IdxT* v) {
+    int below = 0, queued = 0; // of this thread: entries before the span; of its wavefront: entries noted
+    int noted = total;         // the batches of the wavefront from this entry on are not noted, but counted at once
+    read_entries(0, [&](int e, const IdxT* v) {
         unsigned t[BATCH];
         int own = 0;
 #pragma unroll
@@ -224,36 +232,32 @@ __device__ __forceinline__ void build_lists(const ListJob<WEIGHTED, IdxT>& job, 
         }
         const int before = wave_exclusive_sum(own);
         const int all = __builtin_amdgcn_readlane(before + own, TPK_WAVE - 1);
-        if (queued + all <= L_QUEUE) // (wave-uniform)
+        if (queued + all <= L_QUEUE && noted == total) // (wave-uniform)
         {
             unsigned* at = queue + queued + before;
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
                 if (t[u] < static_cast<unsigned>(width))
                     *at++ = t[u] << L_ENTRY_BITS | static_cast<unsigned>(e + u * G_THREADS);
+            queued += all;
         }
-        queued += all;
+        else
+        {
+            noted = min(noted, e - tid);
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+                if (t[u] < static_cast<unsigned>(width))
+                    atomicAdd(&counters[t[u]], 1);
+        }
     });
     {
         const int below_before = wave_exclusive_sum(below);
         if (lane == TPK_WAVE - 1)
             atomicAdd(below_total, below_before + below);
     }
-    const bool noted = __syncthreads_or(queued > L_QUEUE) == 0; // every entry of the span is in a queue
-    // Entries that crowd into one span: their targets are read again, without the queues.
-    if (noted)
-        for (int q = lane; q < queued; q += TPK_WAVE)
-            atomicAdd(&counters[queue[q] >> L_ENTRY_BITS], 1);
-    else
-        read_entries([&](int, const IdxT* v) {
-#pragma unroll
-            for (int u = 0; u < BATCH; ++u)
-            {
-                const unsigned t = index_value(v[u]) - static_cast<unsigned>(i0);
-                if (t < static_cast<unsigned>(width))
-                    atomicAdd(&counters[t], 1);
-            }
-        });
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (its own notes)
+    for (int q = lane; q < queued; q += TPK_WAVE)
+        atomicAdd(&counters[queue[q] >> L_ENTRY_BITS], 1);
     __syncthreads();
 
     // Prefix sum of the list lengths, an empty list counting as one entry (every thread owns a run of
@@ -335,7 +339,6 @@ __device__ __forceinline__ void build_lists(const ListJob<WEIGHTED, IdxT>& job, 
             entry.w = w;
         place(ends[t] - free_places, i0 + static_cast<int>(t), entry);
     };
-    if (noted)
     {
         constexpr int AT_ONCE = 4;
         for (int first = lane; first < queued; first += AT_ONCE * TPK_WAVE)
@@ -360,8 +363,9 @@ __device__ __forceinline__ void build_lists(const ListJob<WEIGHTED, IdxT>& job, 
                 }
         }
     }
-    else
-        read_entries([&](int e, const IdxT* v) {
+    // (what was not noted is read once more)
+    if (noted < total)
+        read_entries(noted, [&](int e, const IdxT* v) {
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
             {
