@@ -12,6 +12,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SHIM = r"""
 #include "bracket.h"
 #include "cloud_ids.h"
+#include "die_map.h"
 #include "grid_shape.h"
 #include "grow_walk.h"
 #include <cmath>
@@ -62,6 +63,19 @@ extern "C" long long pieces_within(const int64_t* starts, long long pieces, long
 extern "C" long long most_staged()
 {
     return grow_walk::MOST_STAGED;
+}
+
+// What each of the parts_grid() workgroups does; returns their number.
+extern "C" unsigned tasks(unsigned items, unsigned parts, unsigned* item, unsigned* part)
+{
+    const unsigned blocks = parts_grid(items, parts);
+    for (unsigned b = 0; b < blocks; ++b)
+    {
+        const PartTask task = part_task(b, items, parts);
+        item[b] = task.item;
+        part[b] = task.part;
+    }
+    return blocks;
 }
 
 extern "C" int ids_fit(unsigned labels, unsigned long long span)
@@ -152,6 +166,24 @@ def test_cloud_ids_are_refused_before_they_overflow(shim):
             assert not shim.ids_fit(labels, span) or largest < 2 ** 63 - 1, (labels, span)
             assert shim.ids_fit(labels, span) or largest >= 2 ** 63 - 1 - labels, (labels, span)
         assert not shim.ids_fit(labels, 0)  # all 2^64 values
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4])
+@pytest.mark.parametrize("items", [1, 2, 3, 7, 8, 9, 16, 29, 63, 64, 65, 96, 257])
+def test_the_parts_of_an_item_share_a_die(shim, items, parts):
+    """Workgroups go to the eight dies in turn: every part of every item is somebody's, all parts of an item on one die, and no die
+    has more items than an even share, rounded up."""
+    item, part = np.zeros(4096, np.uint32), np.zeros(4096, np.uint32)
+    blocks = shim.tasks(items, parts, *(a.ctypes.data_as(ctypes.c_void_p) for a in (item, part)))
+    assert items * parts <= blocks < (items + 8) * parts
+    die = np.arange(blocks) % 8
+    item, part = item[:blocks], part[:blocks]
+    done = item < items
+    assert sorted(zip(item[done], part[done])) == [(i, p) for i in range(items) for p in range(parts)]
+    for i in range(items):
+        assert len(set(die[item == i])) == 1
+    assert max(np.bincount(die[done], minlength=8)) == -(-items // 8) * parts
+    assert (np.diff(die[done][np.argsort(item[done], kind="stable")]) >= 0).all()
 
 
 @pytest.mark.parametrize("row_bytes,most", [(32, 1), (32, 3200), (6, 10 ** 4), (256, 10 ** 6), (4, 2 ** 62)])

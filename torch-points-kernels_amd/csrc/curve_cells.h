@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "curve_order.h"
+#include "die_map.h"
 
 namespace {
 
@@ -534,22 +535,27 @@ __global__ __launch_bounds__(NG_SORT_THREADS) void curve_cells_kernel(PointSet s
                                                                       CloudRows rows_job)
 {
     extern __shared__ unsigned curve_lds[];
-    if (static_cast<int>(blockIdx.x) >= windows * parts)
+    const unsigned ordering = parts_grid(static_cast<unsigned>(windows), static_cast<unsigned>(parts));
+    if (blockIdx.x >= ordering)
     {
-        cloud_rows_job(rows_job, static_cast<int>(blockIdx.x) - windows * parts, threadIdx.x);
+        cloud_rows_job(rows_job, blockIdx.x - ordering, threadIdx.x);
         return;
     }
-    // (the workgroups of a window run on one die, which reads the window once: 14900 -> 6000 clocks for the loads)
-    const int task = static_cast<int>(xcd_local_block(blockIdx.x, static_cast<unsigned>(windows * parts)));
-    const int block = task / parts;
+    // (The workgroups of a window run on one die, which reads the window once: 14900 -> 6000 clocks for the loads.  With blocks
+    // instead of windows dealt to the dies that held for some grids only: Chamfer forward of 1 x 5000 points 53.1 -> 51.4 us, 1 x 12000
+    // 66.4 -> 64.6, 3 x 5000 53.3 -> 52.1, 2 x 16384 90.0 -> 91.5.)
+    const PartTask task = part_task(blockIdx.x, static_cast<unsigned>(windows), static_cast<unsigned>(parts));
+    const int block = static_cast<int>(task.item);
+    if (zero_word && blockIdx.x == 0 && threadIdx.x == 0)
+        *zero_word = 0;
+    if (block >= windows)
+        return;
     const bool first_set = block < windows_a;
     const PointSet set = first_set ? set_a : set_b;
     const int64_t window = first_set ? block : block - windows_a;
-    if (zero_word && task == 0 && threadIdx.x == 0)
-        *zero_word = 0;
     if (set.only && set.only[window / set_windows_per_cloud(set)] == 0)
         return;
-    curve_cells_part<STAGED>(set, window, task - block * parts, parts, curve_lds);
+    curve_cells_part<STAGED>(set, window, static_cast<int>(task.part), parts, curve_lds);
 }
 
 // Bytes of LDS for a part of `part_cells` cells.
@@ -597,7 +603,7 @@ int launch_curve_cells(const PointSet& a, const PointSet& c, int* zero_word, hip
         return TPK_ERR_UNSUPPORTED; // (a thread holds 16 points of a window: windows of at most 16384 points)
     const int64_t windows_a = set_windows(a), windows_c = set_windows(c);
     const int64_t row_groups = tpk_ceil_div(rows_job.size_y, NG_SORT_THREADS);
-    if ((windows_a + windows_c) * CURVE_PARTS + row_groups > 0x7fffffffLL)
+    if ((windows_a + windows_c + DIES) * CURVE_PARTS + row_groups > 0x7fffffffLL || windows_a + windows_c >= 1LL << 29)
         return TPK_ERR_UNSUPPORTED;
     const int parts = curve_parts(a, c);
     const int64_t part_cells = tpk_ceil_div(tpk_ceil_div(largest, NG_CELL), parts);
@@ -607,7 +613,7 @@ int launch_curve_cells(const PointSet& a, const PointSet& c, int* zero_word, hip
     const int allowed = tpk_allow_lds(reinterpret_cast<const void*>(kernel), lds);
     if (allowed != TPK_OK)
         return allowed;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((windows_a + windows_c) * parts + row_groups)),
+    hipLaunchKernelGGL(kernel, dim3(parts_grid(static_cast<unsigned>(windows_a + windows_c), static_cast<unsigned>(parts)) + static_cast<unsigned>(row_groups)),
                        dim3(NG_SORT_THREADS), lds, s, a, c, static_cast<int>(windows_a),
                        static_cast<int>(windows_a + windows_c), parts, zero_word, rows_job);
     return tpk_launch_status();
