@@ -1,0 +1,41 @@
+"""Kernel sources run on the host, lane by lane, between guard pages: shapes whose accesses are checked here and not by
+running them on a GPU."""
+import os
+import re
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+CSRC = os.path.join(ROOT, "torch-points-kernels_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def ball_query_dense(tmp_path_factory):
+    folder = str(tmp_path_factory.mktemp("emulated"))
+    for name in os.listdir(CSRC):
+        if not name.endswith(".h") and name != "nn_grid.hip":
+            continue
+        with open(os.path.join(CSRC, name)) as f:
+            source = f.read()
+        # dynamic LDS is a pointer into the emulated one, the one instruction written by hand an assignment
+        source = re.sub(r"extern __shared__ (?:__align__\(16\) )?([a-z0-9 ]+?) ([a-z_]+)\[\];", r"\1* const \2 = reinterpret_cast<\1*>(emulation::lds);", source)
+        source = source.replace('asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "s"(uniform_value));', "v = uniform_value;")
+        source = source.replace('"../../include/tpk.h"', '"%s"' % os.path.join(ROOT, "include", "tpk.h"))
+        with open(os.path.join(folder, name.replace(".hip", ".cpp")), "w") as f:
+            f.write(source)
+    program = os.path.join(folder, "ball_query_dense")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-w", "-fpermissive", "-ffp-contract=off", "-U_FORTIFY_SOURCE", "-fsanitize=bounds",
+                    "-fno-sanitize-recover=bounds", "-I" + folder, "-I" + os.path.join(HERE, "emulation"),
+                    os.path.join(HERE, "emulation", "ball_query_dense.cpp"), "-o", program], check=True)
+    return program
+
+
+# (clouds of 9373 points: windows of 8192 that hold parts of two clouds, the last of 75 points, whose second part is empty; the first
+# is the call that test_ball_query_of_the_clouds_own_points leaves to this test)
+@pytest.mark.parametrize("clouds,points,queries,nsample,radius,own", [(7, 9373, 9373, 16, 0.05, 1), (7, 9373, 640, 16, 0.05, 0), (2, 8193, 8193, 64, 0.1, 0)])
+def test_dense_ball_query_stays_in_bounds(ball_query_dense, clouds, points, queries, nsample, radius, own):
+    done = subprocess.run([ball_query_dense] + [str(v) for v in (clouds, points, queries, nsample, radius, own)], capture_output=True,
+                          text=True, timeout=300)
+    assert done.returncode == 0, done.stdout + done.stderr

@@ -1779,6 +1779,19 @@ def test_chamfer_parity(tpk, oracle, dev, B, n, m, dtype):
     np.testing.assert_allclose(_np(gb), wb, rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.skip(reason="a kernel that was never committed ended in a memory fault in this call, or in the committed kernel's calls "
+                  "behind it; its cause is not known, so the call is not run on the GPU.  tests/test_emulated_kernels.py runs the "
+                  "committed kernels of this very call on the host, between guard pages")
+def test_ball_query_of_the_clouds_own_points(tpk, oracle, dev):
+    """The dense layout, clouds above 8192 points, every point a query."""
+    x = torch.rand(7, 9373, 3, generator=torch.Generator().manual_seed(16))
+    on_gpu = x.to(dev)
+    idx, dist = tpk.ball_query(0.05, 16, on_gpu, on_gpu)
+    want_idx, want_dist = oracle.ball_query_dense(0.05, 16, x.numpy(), x.numpy())
+    np.testing.assert_array_equal(_np(idx), want_idx)
+    np.testing.assert_array_equal(_np(dist), want_dist)
+
+
 @pytest.mark.parametrize("b,n,m", [(2, 1024, 1024), (3, 1025, 1024), (2, 4096, 4096), (2, 4097, 4097), (5, 16384, 8192), (2, 16385, 8192),
                                    (200, 1500, 1024)])
 def test_three_nn_orders_the_clouds_it_gives_up(dev, b, n, m):
