@@ -143,7 +143,8 @@ __device__ __forceinline__ bool eligible(float x, float y, float z)
 // One sample per round.  The first samples drop so many minima that a pool gives one to four of them; and when more
 // points hold the same value than a pool takes, when nothing above zero is left, or when a coordinate is not finite
 // (such a point never falls to zero), a pool gives none.  Then every wavefront offers its best point, one barrier, and all
-// find the best of those.
+// find the best of those: 4900 clocks a sample at 16384 points, most of them for the rank among equal minima that all
+// wavefronts look for in turn.  1024 of 16384 points on 1728 places, nearly all of them taken this way: 2300 us.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ unsigned tie_key(int k, int log2_bs, int ref_groups)
 {
@@ -186,7 +187,7 @@ __device__ __forceinline__ int not_hoisted(int v)
 }
 
 // Calls f with the slot (LOW .. LOW + N - 1, the same in all lanes) as a constant: log2(N) branches instead of N in a row,
-// each of them 24 clocks of all wavefronts of a SIMD (1024 samples of 16384 points on 1728 places, taken one by one: 2590 -> 2297 us).
+// each of them 24 clocks of all wavefronts of a SIMD (1024 of 16384 points on 1728 places, taken one by one: 2590 -> 2297 us).
 template <int LOW, int N, typename F>
 __device__ __forceinline__ void with_slot(int slot, F&& f)
 {
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
     {
         float4* const pool = pools + par * POOL_CAPACITY;
         int* const pool_place = pool_places + par * POOL_CAPACITY;
-        // 1. the pool: all points whose minimum lies above `floor_bits`, at most 64
+        // 1. the pool: all points whose minimum lies above `floor_bits`, at most POOL_CAPACITY
         // Every wavefront reads ROWS of its points, a row of 16 lanes each, and all 64, 16 at a time.
         constexpr int CHUNKS = TPK_WAVE / 16, PASSES = ROWS / 4;
         float4 other[CHUNKS], mine[PASSES];
@@ -523,7 +524,7 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
             const float4* points = pool;
             const int* places = pool_place;
             const int found = count;
-            if (count > TPK_WAVE)
+            if (count > TPK_WAVE) // 2. its best 64
             {
                 if (wave == 0)
                 {

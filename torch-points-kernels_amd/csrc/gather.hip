@@ -150,9 +150,10 @@ struct FwdPlan
 // Bound by the output's way to memory.  All workgroups write rows that lie a multiple of the row length apart: where
 // they walk the columns in step and that length is a power of two, their stores meet in the same few memory channels.
 // Every workgroup therefore starts at another run of G_THREADS columns and wraps around (xcd_local_block keeps a
-// cloud's workgroups, and the indices they share, on one die).  Measured behind a pass over other memory (16 clouds,
-// 128 channels): rows of 32768 columns, plain, 99 -> 60 us (348 MB: 5.8 TB/s; a large copy here moves 5.3), without
-// the dies 64; rows of 16384 columns, three weighted neighbours, 54 -> 41 us (174 MB), without the dies 49.
+// cloud's workgroups, and the indices they share, on one die, or on a few where the clouds are no multiple of eight).
+// Measured behind a pass over other memory (16 clouds, 128 channels): rows of 32768 columns, plain, 99 -> 60 us (348 MB:
+// 5.8 TB/s; a large copy here moves 5.3), without the dies 64; rows of 16384 columns, three weighted neighbours, 54 -> 41 us
+// (174 MB), without the dies 49.
 template <int K, bool WEIGHTED, typename IdxT>
 __device__ __forceinline__ void gather_fwd_rows(
     unsigned hardware_block, unsigned blocks, float* rows, int c, int m, int64_t n, int rows_per_block, int row_blocks, int jsplit,

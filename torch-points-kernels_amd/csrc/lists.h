@@ -137,9 +137,10 @@ struct ListJob
 // 24), 4 x 90000 weighted entries, Zipf exponent 0.7 and 1, 22 and 35 (42 and 45; 30 and 34).
 //
 // Bound by the instructions of the first pass, as all but one entry in L_SPANS are read in vain, and by the stores of single
-// entries.  A part's workgroups run on one die, which reads its index once.  Keeping every index value in registers for a second
-// pass over all of them took 12900 + 15300 clocks for the two passes at 16384 x 3 entries (124 registers, 17.2 us), the notes
-// take 13300 + 6800 (42 registers, 12.6 us); a bit per entry instead of a note, and the index read again, 11300 + 20100.
+// entries.  A part's workgroups run on one die, which reads its index once, where the parts are a multiple of eight, otherwise some
+// on a second one (a single part: on all).  Keeping every index value in registers for a second pass over all of them took
+// 12900 + 15300 clocks for the two passes at 16384 x 3 entries (124 registers; 16 clouds, 2048 targets 18.6 us), the notes take
+// 13300 + 6800 (38 registers, 14.9 us); a bit per entry instead of a note, and the index read again, 11300 + 20100.
 template <int K, bool WEIGHTED, typename IdxT>
 __device__ __forceinline__ void build_lists(const ListJob<WEIGHTED, IdxT>& job, int block, int* counters)
 {
