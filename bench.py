@@ -54,7 +54,7 @@ TRAFFIC_KERNELS = {
 VALU_KERNELS = {
     "fps": "fps_pool_kernel<16, 16, 2, true>",
     "ball_query_dense": "ball_query_dense_cells_kernel<false>",
-    "ball_query_partial_dense": "ball_query_bins_kernel<false, false>",
+    "ball_query_partial_dense": "bt_query_kernel",
     "three_nn": "three_nn_cells_kernel",
     "chamfer_fwd": "chamfer_grid_kernel",
 }
@@ -193,7 +193,7 @@ def _counting_lib():
         if not os.path.exists(path):
             sys.exit("bench.py: %s is not built (run torch-points-kernels_amd/build.py)" % path)
         lib = ctypes.CDLL(path)
-        for name in ("tpk_fps_workspace_bytes", "tpk_ball_query_partial_workspace_bytes", "tpk_three_nn_workspace_bytes",
+        for name in ("tpk_fps_workspace_bytes", "tpk_ball_query_partial_table_workspace_bytes", "tpk_three_nn_workspace_bytes",
                      "tpk_chamfer_fwd_workspace_bytes", "tpk_knn_workspace_bytes",
                      "tpk_ball_query_sorted_dense_workspace_bytes", "tpk_ball_query_sorted_partial_workspace_bytes"):
             getattr(lib, name).restype = ctypes.c_size_t
@@ -406,8 +406,8 @@ def bench_others(dev, steps, warmup, with_cpu):
     pairs = sum(a * b for a, b in zip(sizes, qsizes))
     bq_idx = torch.empty(nq, w["nsample"], dtype=torch.int64, device=dev)
     bq_dist = torch.empty(nq, w["nsample"], device=dev)
-    ws_bytes = _counting_lib().tpk_ball_query_partial_workspace_bytes(ctypes.c_int64(x.shape[0]), ctypes.c_int64(nq),
-                                                                      w["nsample"])
+    ws_bytes = _counting_lib().tpk_ball_query_partial_table_workspace_bytes(ctypes.c_int64(x.shape[0]), ctypes.c_int64(nq),
+                                                                            w["nsample"])
     ws = _ws(ws_bytes, dev)
     executed = _executed(lambda lib, st: lib.tpk_ball_query_partial_f32(
         ctypes.c_int64(x.shape[0]), ctypes.c_int64(nq), ctypes.c_float(w["radius"]), w["nsample"], _p(x), _p(y), _p(bx),

@@ -10,6 +10,7 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "torch-points-kernels_amd", "csrc")
 
 SHIM = r"""
+#include "ball_table.h"
 #include "bracket.h"
 #include "cloud_ids.h"
 #include "die_map.h"
@@ -30,6 +31,19 @@ extern "C" void grid_of(const float* low, const float* high, int m, float per_ce
     });
     for (int a = 0; a < 3; ++a)
         along[a] = counts.along[a];
+}
+
+extern "C" void table_cells(const float* v, int n, float inverse_width, int* cell)
+{
+    for (int i = 0; i < n; ++i)
+        cell[i] = bt_cell(v[i], inverse_width);
+}
+extern "C" float table_reach(float radius) { return bt_reach(radius); }
+extern "C" void table_bucket(int ix, int iy, int iz, int64_t cloud, uint32_t part_mask, uint32_t* part, uint32_t* bucket)
+{
+    const BtRow row = bt_row(iy, iz, cloud);
+    *part = row.part;
+    *bucket = bt_bucket(row, ix, part_mask);
 }
 
 // The guesses until between k and `most` of the distances lie within one; -1: none found.
@@ -203,3 +217,53 @@ def test_turns_of_pieces_stay_within_their_bytes(shim, row_bytes, most):
             assert end == begin + 1 or (starts[end] - starts[begin]) * row_bytes <= most
             assert end == pieces or (starts[end + 1] - starts[begin]) * row_bytes > most
             begin = end
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-3, 1.0, 5e3, 4e6, 3e30])
+@pytest.mark.parametrize("radius", [0.0, 1e-25, 1e-12, 0.05, 3.0, 1e19])
+def test_cells_of_the_ball_table_hold_every_accepted_point(shim, scale, radius):
+    """A coordinate the radius test accepts lies between the cells of the query's two ends, at every scale and radius."""
+    rng = np.random.default_rng(7)
+    reach = np.float32(_table_reach(shim, radius))
+    for width in (0.55, 2.2):
+        inverse = np.float32(1.0) / (np.float32(width) * reach)
+        q = ((rng.random(4000) - 0.5) * scale).astype(np.float32)
+        with np.errstate(over="ignore", under="ignore", invalid="ignore"):
+            step = np.concatenate([rng.uniform(-1.2, 1.2, 3000), np.repeat([-1.0, 1.0], 500)]) * radius
+            p = (q.astype(np.float64) + step).astype(np.float32)
+            d = p - q
+            accepted = d * d <= np.float32(radius) * np.float32(radius)
+            ends = [_table_cells(shim, v, inverse) for v in (q - reach, p, q + reach)]
+        assert accepted.any()
+        assert (ends[0] <= ends[1])[accepted].all() and (ends[1] <= ends[2])[accepted].all()
+
+
+def test_rows_of_the_ball_table_near_each_other_never_share_a_part(shim):
+    part, bucket = ctypes.c_uint32(), ctypes.c_uint32()
+    rng = np.random.default_rng(3)
+    for _ in range(50):
+        ix, iy, iz = (int(v) for v in rng.integers(-2**30, 2**30, 3))
+        cloud = int(rng.integers(-2**62, 2**62))
+        parts = set()
+        for dy in range(3):
+            for dz in range(3):
+                run = []
+                for dx in range(5):
+                    shim.table_bucket(ix + dx, iy + dy, iz + dz, ctypes.c_int64(cloud), 8191, ctypes.byref(part), ctypes.byref(bucket))
+                    assert bucket.value // 8192 == part.value < 16
+                    run.append(bucket.value % 8192)
+                parts.add(part.value)
+                assert all((b - a) % 8192 == 1 for a, b in zip(run, run[1:]))
+        assert len(parts) == 9
+
+
+def _table_reach(shim, radius):
+    shim.table_reach.restype = ctypes.c_float
+    return shim.table_reach(ctypes.c_float(radius))
+
+
+def _table_cells(shim, v, inverse):
+    v = np.ascontiguousarray(v, dtype=np.float32)
+    cell = np.empty(v.shape[0], dtype=np.int32)
+    shim.table_cells(v.ctypes.data_as(ctypes.c_void_p), v.shape[0], ctypes.c_float(inverse), cell.ctypes.data_as(ctypes.c_void_p))
+    return cell

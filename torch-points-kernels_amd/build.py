@@ -57,7 +57,7 @@ def _run(cmd):
 
 # Translation units that hold distance scans (and the counters' reader): compiled a second time
 # with -DTPK_COUNT_WORK for the counting library; the other objects are shared.
-COUNTING_UNITS = ("status", "ball_query", "three_nn", "chamfer", "knn", "nn_grid", "fps")
+COUNTING_UNITS = ("status", "ball_query", "ball_table", "three_nn", "chamfer", "knn", "nn_grid", "fps")
 
 
 def build_kernels(force=False):

@@ -745,6 +745,11 @@ extern "C" size_t tpk_ball_query_partial_workspace_bytes(int64_t size_x, int64_t
     return tpk_grid_ball_query_workspace_bytes(size_x, size_y, nsample);
 }
 
+extern "C" size_t tpk_ball_query_partial_table_workspace_bytes(int64_t size_x, int64_t size_y, int nsample)
+{
+    return tpk_table_ball_query_workspace_bytes(size_x, size_y, nsample);
+}
+
 extern "C" int tpk_ball_query_partial_f32(int64_t size_x, int64_t size_y, float radius,
                                           int nsample, const float* x, const float* y,
                                           const int64_t* batch_x, const int64_t* batch_y,
@@ -763,8 +768,12 @@ extern "C" int tpk_ball_query_partial_f32(int64_t size_x, int64_t size_y, float 
     const float radius2 = radius * radius;
     if (workspace)
     {
-        // Search over curve-ordered cells where it applies; otherwise all pairs.
-        const int st = tpk_grid_ball_query_partial(size_x, size_y, radius, radius2, nsample, false, x, y, batch_x, batch_y, idx,
+        // A table of cells where the workspace holds one, else the walk over bins where it applies; otherwise all pairs.
+        int st = tpk_table_ball_query_partial(size_x, size_y, radius, radius2, nsample, x, y, batch_x, batch_y, idx, dist, workspace,
+                                              workspace_bytes, tpk_stream(stream));
+        if (st != TPK_ERR_UNSUPPORTED)
+            return st;
+        st = tpk_grid_ball_query_partial(size_x, size_y, radius, radius2, nsample, false, x, y, batch_x, batch_y, idx,
                                                    dist, workspace, workspace_bytes, tpk_stream(stream));
         if (st != TPK_ERR_UNSUPPORTED)
             return st;

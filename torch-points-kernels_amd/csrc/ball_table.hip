@@ -1,0 +1,553 @@
+// Ball query, packed layout, over a hash table of cells (several clouds back to back, sorted cloud id per point).
+//
+// Space is cut into cells of 0.55 x 2.2 x 2.2 reaches (the reach: the radius and its rounding), and cell (ix, iy, iz) of a cloud
+// belongs to bucket row(iy, iz, cloud) + ix of a table with 2 .. 4 buckets per support point: the cells a ball touches are
+// at most four runs (two values of iy, two of iz; three each within rounding of an edge) of four or five consecutive buckets.  No
+// bounding box, no windows, no limit on a cloud's size: the launches in front of the queries clear the table, count the points
+// per bucket (the atomic that counts hands out the point's place in its bucket), turn the counts into places, and put the points
+// there as records (x, y, z, row).  Points of other cells that share a bucket fail the radius test or lie in another cloud's rows.
+//
+// A wavefront answers four queries, 16 lanes each, as wide as a row of the DPP network: a lane looks up a run, prefix sums
+// over the 16 give the query's candidates, which are tested 16 at a time.  Hits are collected in LDS and ranked by row,
+// which is the order a serial scan in index order that stops after nsample hits (cuda/src/ball_query_gpu.cu:54-95) meets them in.
+// A query with more than 128 keeps the nsample lowest rows and goes on.  Where that scan itself is likely to end sooner than the
+// walk - dense neighbourhoods -, or the query has more candidates than its cloud has rows, the wavefront scans.
+//
+// Measured against the walk over bins of windows (nn_grid.hip: windows of consecutive rows, each of which a query has to look
+// into), whole calls: 53000 queries of four scenes of 20000 .. 100000 points 50 -> 42 us (15 of them the queries, 37
+// before; clearing 3, counting 13, places 4, records 7, against 17 for the windows' ordering), all 212000 of their points as queries 117 ->
+// 61 (nsample 16, radius 0.04), 138 -> 75 (64, 0.1), 2300 -> 272 (64, 0.3: 60 points in a ball of a plane, which the walk over bins
+// left to the scan); 300000 queries of 24 clouds 257 -> 133.  An eighth of the points as queries: 38 -> 40 and 42 -> 40; 20000 points and
+// 3000 queries 21 -> 17 .. 22.  Slower where a ball holds a large part of its cloud and every query is scanned for: four scans per
+// wavefront are one after the other (radius 1 in rooms of 8: 12500 queries 150 -> 209, 100000 417 -> 448).
+// What bounds it: the counting its atomics, the queries instruction issue - 690 vector instructions per wavefront, 170 per query
+// with 16 hits each, of 1700 clocks a query before.
+// Cells of 1.1 and 0.28 reaches along x: the 300000 queries 96 and 94 us against 94, counting 15 and 13 against 13.
+#include <algorithm>
+#include <cmath>
+
+#include "ball_scan.h"
+#include "ball_table.h"
+#include "cloud_rows.h"
+#include "nn_grid.h"
+
+namespace {
+
+constexpr int BT_THREADS = 256;
+constexpr int BT_GROUP = 16;                       // lanes per query
+constexpr int BT_QUERIES = TPK_WAVE / BT_GROUP;    // queries per wavefront
+constexpr int BT_HITS = 2 * TPK_WAVE;              // hits a query holds when a step begins
+constexpr int BT_KEPT = TPK_WAVE;                  // slots of a call whose queries may keep their lowest rows when they hold more
+constexpr int BT_LONG = 8 * BT_HITS;               // candidates from which on a query may be scanned for at once
+constexpr int BT_HIT_STRIDE = BT_HITS + BT_GROUP + 2; // (the four queries of a wavefront read theirs at the same time: other banks)
+constexpr int BT_SCAN_THREADS = 1024;
+constexpr int BT_CHUNK = BT_SCAN_THREADS * 4;      // buckets whose places one workgroup hands out
+constexpr int BT_MOST_X = BT_CHUNK / 2;            // buckets of a run, at most: a run touches two chunks at most
+constexpr float BT_WIDTH_X = 0.55f, BT_WIDTH_YZ = 2.2f; // of a cell, in reaches
+
+struct CellScale
+{
+    float reach, inverse_x, inverse_yz;
+};
+
+__global__ void __launch_bounds__(BT_THREADS) bt_clear_kernel(int64_t quads, int4* table)
+{
+    const int64_t i = (int64_t)blockIdx.x * BT_THREADS + threadIdx.x;
+    if (i < quads)
+        table[i] = make_int4(0, 0, 0, 0);
+}
+
+__device__ __forceinline__ uint32_t bt_point_bucket(float x, float y, float z, int64_t cloud, const CellScale& scale, uint32_t part_mask)
+{
+    return bt_bucket(bt_row(bt_cell(y, scale.inverse_yz), bt_cell(z, scale.inverse_yz), cloud), bt_cell(x, scale.inverse_x), part_mask);
+}
+
+// counts: how many points every bucket holds; ranks: the place of every point among its bucket's.  Workgroups behind those of the
+// points find the rows of every query's cloud.  Bound by the atomics (16 to the nanosecond; 212000 points 13 us): lanes that share the bucket of the first lane - all of them where the radius is as
+// large as the cloud - share one.
+__global__ void __launch_bounds__(BT_THREADS)
+    bt_count_kernel(int n, unsigned point_blocks, const float* __restrict__ x, const int64_t* __restrict__ batch_x, CellScale scale, uint32_t part_mask,
+                    int* counts, int* __restrict__ ranks, int* __restrict__ placed, CloudRows rows)
+{
+    if (blockIdx.x >= point_blocks)
+    {
+        cloud_rows_job(rows, static_cast<int64_t>(blockIdx.x - point_blocks) * (BT_THREADS / TPK_WAVE) + threadIdx.x / TPK_WAVE,
+                       threadIdx.x & (TPK_WAVE - 1));
+        return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *placed = 0;
+    const int i = blockIdx.x * BT_THREADS + threadIdx.x;
+    if (i >= n)
+        return;
+    const uint32_t bucket = bt_point_bucket(x[(int64_t)i * 3 + 0], x[(int64_t)i * 3 + 1], x[(int64_t)i * 3 + 2], batch_x[i], scale, part_mask);
+    const bool same = bucket == static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(bucket)));
+    const unsigned long long sharing = __ballot(same);
+    int rank;
+    if (same)
+    {
+        const int first = __builtin_ctzll(sharing);
+        int base = 0;
+        if (static_cast<int>(threadIdx.x & (TPK_WAVE - 1)) == first)
+            base = atomicAdd(&counts[bucket], __builtin_popcountll(sharing));
+        rank = __builtin_amdgcn_readlane(base, first) + static_cast<int>(tpk_prefix_count(sharing));
+    }
+    else
+        rank = atomicAdd(&counts[bucket], 1);
+    ranks[i] = rank;
+}
+
+// Counts -> first places, in place.  Every workgroup sums a chunk of the table and takes its range of places with one atomic: the
+// chunks' ranges lie in no particular order, and a run of buckets that crosses from one chunk to the next is looked up as
+// two.  chunk_ends: where a chunk's last bucket ends.
+__global__ void __launch_bounds__(BT_SCAN_THREADS) bt_places_kernel(int4* table, int* __restrict__ chunk_ends, int* placed)
+{
+    __shared__ int waves[BT_SCAN_THREADS / TPK_WAVE];
+    __shared__ int base;
+    const int wave = threadIdx.x / TPK_WAVE, lane = threadIdx.x % TPK_WAVE;
+    const int64_t at = (int64_t)blockIdx.x * BT_SCAN_THREADS + threadIdx.x;
+    const int4 c = table[at];
+    const int mine = c.x + c.y + c.z + c.w;
+    const int before = wave_exclusive_sum(mine);
+    if (lane == TPK_WAVE - 1)
+        waves[wave] = before + mine;
+    __syncthreads();
+    if (wave == 0)
+    {
+        const int v = lane < BT_SCAN_THREADS / TPK_WAVE ? waves[lane] : 0;
+        const int sum = wave_exclusive_sum(v);
+        if (lane < BT_SCAN_THREADS / TPK_WAVE)
+            waves[lane] = sum;
+        if (lane == TPK_WAVE - 1)
+        {
+            base = atomicAdd(placed, sum + v);
+            chunk_ends[blockIdx.x] = base + sum + v;
+        }
+    }
+    __syncthreads();
+    const int first = base + waves[wave] + before;
+    table[at] = make_int4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
+}
+
+__global__ void __launch_bounds__(BT_THREADS)
+    bt_records_kernel(int n, const float* __restrict__ x, const int64_t* __restrict__ batch_x, CellScale scale, uint32_t part_mask,
+                      const int* __restrict__ table, const int* __restrict__ ranks, float4* __restrict__ records)
+{
+    const int i = blockIdx.x * BT_THREADS + threadIdx.x;
+    if (i >= n)
+        return;
+    const float px = x[(int64_t)i * 3 + 0], py = x[(int64_t)i * 3 + 1], pz = x[(int64_t)i * 3 + 2];
+    const uint32_t bucket = bt_point_bucket(px, py, pz, batch_x[i], scale, part_mask);
+    records[table[bucket] + ranks[i]] = make_float4(px, py, pz, __int_as_float(i));
+}
+
+// Sum of v over the lanes below this one in its row of 16.
+__device__ __forceinline__ int row_exclusive_sum(int v)
+{
+    int s = v;
+    s += __builtin_amdgcn_update_dpp(0, s, 0x111, 0xF, 0xF, false); // row_shr:1
+    s += __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false); // row_shr:2
+    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false); // row_shr:4
+    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false); // row_shr:8
+    return s - v;
+}
+
+// Largest of the values v >= 0 of this lane and the lanes below it in its row of 16.
+__device__ __forceinline__ int row_inclusive_max(int v)
+{
+    int s = v;
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x111, 0xF, 0xF, false));
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false));
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false));
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false));
+    return s;
+}
+
+// (value of the row's lane 15)
+__device__ __forceinline__ int row_last(int v, int lane)
+{
+    return __builtin_amdgcn_ds_bpermute((lane | (BT_GROUP - 1)) * 4, v);
+}
+
+// The largest of the four queries' values (each the same in the query's lanes).
+__device__ __forceinline__ int bt_most(int v)
+{
+    return max(max(tpk_read_lane(v, 0), tpk_read_lane(v, 16)), max(tpk_read_lane(v, 32), tpk_read_lane(v, 48)));
+}
+
+// (value of the row's lane L)
+template <int L>
+__device__ __forceinline__ int row_lane(int v)
+{
+    return __builtin_amdgcn_ds_swizzle(v, (L << 5) | 0x10); // and-mask 0x10, or-mask L: in every half wavefront, per row
+}
+
+// How many of the row's values are below `mine`, its own among them.
+template <int BY = 1>
+__device__ __forceinline__ int rank_among_row(int mine)
+{
+    if constexpr (BY == BT_GROUP)
+        return 0;
+    else
+        return (__builtin_amdgcn_update_dpp(0, mine, 0x120 + BY, 0xF, 0xF, true) < mine ? 1 : 0) + rank_among_row<BY + 1>(mine); // row_ror:BY
+}
+
+// Puts the first cnt hits of every query of the wavefront (int2 (row, distance); cnt is the same in a query's 16 lanes) in ascending order
+// of rows; those that are not among the nsample lowest go.  Up to 16 and 32 hits a query's own
+// lanes rank them, one or two each; above, the whole wavefront ranks one query's after the other's by lane reads, three instructions per hit.
+__device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, int nsample)
+{
+    const int group = lane / BT_GROUP, sub = lane % BT_GROUP;
+    int2* const hits = wave_hits + group * BT_HIT_STRIDE;
+    const int most = bt_most(cnt);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (most <= BT_GROUP)
+    {
+        const int2 hit = hits[sub];
+        const int mine = sub < cnt ? hit.x : 0x7fffffff;
+        const int rank = rank_among_row(mine);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (sub < cnt && rank < nsample)
+            hits[rank] = hit;
+    }
+    else if (most <= 2 * BT_GROUP)
+    {
+        const int2 hit0 = hits[sub], hit1 = hits[BT_GROUP + sub];
+        int rank0 = 0, rank1 = 0;
+        for (int i = 0; i < most; ++i)
+        {
+            const int other = i < cnt ? hits[i].x : 0x7fffffff;
+            rank0 += other < hit0.x ? 1 : 0;
+            rank1 += other < hit1.x ? 1 : 0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (sub < cnt && rank0 < nsample)
+            hits[rank0] = hit0;
+        if (BT_GROUP + sub < cnt && rank1 < nsample)
+            hits[rank1] = hit1;
+    }
+    else
+    {
+        for (int g = 0; g < BT_QUERIES; ++g)
+        {
+            int2* const of_g = wave_hits + g * BT_HIT_STRIDE;
+            const int count = tpk_read_lane(cnt, g * BT_GROUP);
+            if (count <= TPK_WAVE)
+            {
+                const int2 hit = of_g[lane];
+                const int mine = lane < count ? hit.x : 0x7fffffff;
+                int rank = 0;
+                for (int i = 0; i < count; ++i)
+                    rank += tpk_read_lane(mine, i) < mine ? 1 : 0;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (lane < count && rank < nsample)
+                    of_g[rank] = hit;
+                continue;
+            }
+            // (a query that is full: up to 144)
+            constexpr int PER = 3;
+            static_assert(PER * TPK_WAVE >= BT_HITS + BT_GROUP, "every hit has a register");
+            int2 hit[PER];
+            int rank[PER];
+#pragma unroll
+            for (int j = 0; j < PER; ++j)
+            {
+                hit[j] = of_g[min(j * TPK_WAVE + lane, BT_HIT_STRIDE - 1)];
+                rank[j] = 0;
+            }
+            for (int i = 0; i < count; ++i)
+            {
+                const int other = of_g[i].x;
+#pragma unroll
+                for (int j = 0; j < PER; ++j)
+                    rank[j] += other < hit[j].x ? 1 : 0;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int j = 0; j < PER; ++j)
+                if (j * TPK_WAVE + lane < count && rank[j] < nsample)
+                    of_g[rank[j]] = hit[j];
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Whether a scan of the cloud in index order is likely to take fewer instructions than a walk over `candidates` more, for a query with
+// about `hits` hits.  The scan meets nsample of them within rows * nsample / hits rows, 64 a step of 25 instructions; a step of the
+// walk takes 45 for 16 candidates of each of four queries.
+__device__ __forceinline__ bool scan_is_shorter(float rows, float nsample, float hits, float candidates)
+{
+    const float scan = fminf(rows, rows * nsample * __builtin_amdgcn_rcpf(hits)) * (25.0f / TPK_WAVE);
+    return candidates * (45.0f / (BT_GROUP * BT_QUERIES)) > scan;
+}
+
+__global__ void __launch_bounds__(BT_THREADS)
+    bt_query_kernel(int64_t size_y, CellScale scale, float radius2, int nsample, uint32_t part_mask, const float* __restrict__ x,
+                    const float* __restrict__ y, const int64_t* __restrict__ batch_y, const int2* __restrict__ cloud_rows,
+                    const float4* __restrict__ records, const int* __restrict__ table, const int* __restrict__ chunk_ends,
+                    int64_t* __restrict__ idx, float* __restrict__ dist)
+{
+    constexpr int WAVES = BT_THREADS / TPK_WAVE;
+    __shared__ int2 hits[WAVES][BT_QUERIES * BT_HIT_STRIDE]; // (row, bits of the squared distance)
+    __shared__ int marks[WAVES][TPK_WAVE];
+
+    const int lane = threadIdx.x & (TPK_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TPK_WAVE);
+    const int64_t q0 = (static_cast<int64_t>(blockIdx.x) * WAVES + wave) * BT_QUERIES;
+    if (q0 >= size_y)
+        return; // (no workgroup barrier anywhere in this kernel)
+    const int group = lane / BT_GROUP, sub = lane % BT_GROUP, group_lane = group * BT_GROUP;
+    const bool real = q0 + group < size_y;
+    const int64_t q = real ? q0 + group : q0;
+    int2* const my_hits = hits[wave] + group * BT_HIT_STRIDE;
+    int* const my_marks = marks[wave];
+    TPK_WORK_DECL
+
+    const float qx = y[q * 3 + 0], qy = y[q * 3 + 1], qz = y[q * 3 + 2];
+    const int2 cloud = cloud_rows[q];
+    const int s0 = cloud.x, s1 = real ? cloud.y : cloud.x;
+
+    // The runs of buckets that the cube around the ball touches, one per lane.
+    const float lx = (qx - scale.reach) * scale.inverse_x, hx = (qx + scale.reach) * scale.inverse_x;
+    const float ly = (qy - scale.reach) * scale.inverse_yz, hy = (qy + scale.reach) * scale.inverse_yz;
+    const float lz = (qz - scale.reach) * scale.inverse_yz, hz = (qz + scale.reach) * scale.inverse_yz;
+    int x0, y0, z0, nx, ny, nz;
+    // (cells so far out that a float has no fraction left are seldom)
+    const float farthest = fmaxf(fmaxf(fmaxf(-lx, hx), fmaxf(-ly, hy)), fmaxf(-lz, hz));
+    if (__ballot(!(farthest < BT_FAR && qx == qx && qy == qy && qz == qz)) == 0)
+    {
+        x0 = static_cast<int>(floorf(lx)), nx = static_cast<int>(floorf(hx)) - x0 + 1;
+        y0 = static_cast<int>(floorf(ly)), ny = static_cast<int>(floorf(hy)) - y0 + 1;
+        z0 = static_cast<int>(floorf(lz)), nz = static_cast<int>(floorf(hz)) - z0 + 1;
+    }
+    else
+    {
+        x0 = bt_scaled_cell(lx), nx = bt_scaled_cell(hx) - x0 + 1;
+        y0 = bt_scaled_cell(ly), ny = bt_scaled_cell(hy) - y0 + 1;
+        z0 = bt_scaled_cell(lz), nz = bt_scaled_cell(hz) - z0 + 1;
+    }
+    bool scan = !(nx >= 1 && nx <= BT_MOST_X && ny >= 1 && ny <= 3 && nz >= 1 && nz <= 3);
+    const int runs = scan ? 0 : ny * nz;
+    // (up to eight runs: the upper eight lanes take the second halves of runs that cross from one chunk to the next)
+    const int run = runs <= 8 ? sub & 7 : sub;
+    const bool second = runs <= 8 && sub >= 8;
+    int start = 0, size = 0;
+    bool crosses = false;
+    if (run < runs && s1 > s0)
+    {
+        const int iz = (run >= ny ? 1 : 0) + (run >= 2 * ny ? 1 : 0);
+        const BtRow row = bt_row(y0 + run - iz * ny, z0 + iz, batch_y[q]);
+        const uint32_t first = bt_bucket(row, x0, part_mask), last = bt_bucket(row, x0 + nx - 1, part_mask);
+        crosses = first / BT_CHUNK != last / BT_CHUNK;
+        if (!second || crosses)
+        {
+            const uint32_t from = second ? last & ~static_cast<uint32_t>(BT_CHUNK - 1) : first;
+            const uint32_t to = !second && crosses ? first | (BT_CHUNK - 1) : last;
+            start = table[from];
+            size = ((to + 1) % BT_CHUNK == 0 ? chunk_ends[to / BT_CHUNK] : table[to + 1]) - start;
+        }
+    }
+    if (runs > 8)
+        scan = ((__ballot(crosses) >> group_lane) & 0xffff) != 0;
+    const int before = row_exclusive_sum(size);
+    int total = row_last(before + size, lane);
+    // (a run of cells holds 5 to 13 times what the ball itself does, on a surface and in space)
+    scan = scan || total > s1 - s0 ||
+           (total > BT_LONG && scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), static_cast<float>(total) * 0.125f, static_cast<float>(total)));
+    if (scan)
+        total = 0;
+
+    int cnt = 0;             // hits kept so far, the same in all lanes of a query
+    unsigned wanted = s1 - s0; // rows s0 .. s0 + wanted are: the cloud's, or those below the nsample ones that are kept
+    const unsigned group_low = group < 2 ? 0xffffu << group_lane : 0, group_high = group < 2 ? 0 : 0xffffu << (group_lane - 32);
+    int most_total = bt_most(total);
+    auto record_at = [&](int at) __attribute__((always_inline)) {
+        // (below 2^32 bytes of records: a scalar base and a 32-bit offset)
+        return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(records) + static_cast<uint32_t>(at) * 16u);
+    };
+    const int origin = start - before; // candidate c of a query lies at origin + c, for the c of this lane's run
+    // Four runs at most, in the lanes 0 .. 3 of the query, nearly always: where they begin and lie, known to all its lanes.
+    const bool few = __ballot(crosses || runs > 4) == 0;
+    const int second_at = row_lane<1>(before), third_at = row_lane<2>(before), fourth_at = row_lane<3>(before);
+    const int o0 = row_lane<0>(origin), o1 = row_lane<1>(origin), o2 = row_lane<2>(origin), o3 = row_lane<3>(origin);
+    auto fetch = [&](int c0) __attribute__((always_inline)) {
+        const int c = c0 + sub;
+        int at = c;
+        if (few)
+            at += c < third_at ? (c < second_at ? o0 : o1) : (c < fourth_at ? o2 : o3);
+        else
+        {
+            // Whose candidate is c?  Every run's lane marks the slot of its first candidate of this step with its own
+            // number; a running maximum over the row carries the number on to the run's other candidates.  (What a lane reads
+            // back was written by other lanes: fences for the compiler, no instructions.)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            my_marks[lane] = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (size > 0 && before < c0 + BT_GROUP && before + size > c0)
+                my_marks[group_lane + max(before - c0, 0)] = sub;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            at += __builtin_amdgcn_ds_bpermute((group_lane + row_inclusive_max(my_marks[lane])) * 4, origin);
+        }
+        return record_at(c < total ? at : 0);
+    };
+    int c0 = 0;
+    float4 ahead = fetch(0);
+    for (;;)
+    {
+        for (; c0 < most_total; c0 += BT_GROUP)
+        {
+            const float4 p = ahead;
+            const bool has = c0 + sub < total;
+            if (c0 + BT_GROUP < most_total)
+                ahead = fetch(c0 + BT_GROUP);
+            const float d = tpk_dist2(qx, qy, qz, p.x, p.y, p.z);
+            TPK_WORK_ADD(has ? 1 : 0);
+            const int row = __float_as_int(p.w);
+            const bool hit = has && d <= radius2 && static_cast<unsigned>(row - s0) < wanted;
+            const unsigned long long all = __ballot(hit);
+            if (all == 0)
+                continue;
+            const unsigned low = static_cast<unsigned>(all) & group_low, high = static_cast<unsigned>(all >> 32) & group_high;
+            const unsigned slot = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, cnt));
+            if (hit)
+                my_hits[slot] = make_int2(row, __float_as_int(d));
+            cnt += __builtin_popcount(low) + __builtin_popcount(high);
+            if (__ballot(cnt > BT_HITS) != 0)
+            {
+                c0 += BT_GROUP;
+                break;
+            }
+        }
+        // Full: the nsample lowest rows are kept and the walk goes on, or the query is scanned for.  (Once rows are kept
+        // their number says nothing about the ball any more.)
+        const bool full = cnt > BT_HITS;
+        if (full && wanted == static_cast<unsigned>(s1 - s0))
+        {
+            const float tested = static_cast<float>(min(c0, total)), left = static_cast<float>(total) - tested;
+            const float ball = static_cast<float>(cnt) * static_cast<float>(total) * __builtin_amdgcn_rcpf(tested);
+            scan = nsample > BT_KEPT || scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), ball, left);
+            total = scan ? 0 : total;
+            cnt = scan ? 0 : cnt;
+        }
+        most_total = bt_most(total);
+        order_hits(hits[wave], cnt, lane, nsample);
+        if (cnt >= nsample)
+        {
+            cnt = nsample;
+            wanted = my_hits[nsample - 1].x - s0;
+        }
+        if (c0 >= most_total)
+            break;
+    }
+
+    // The hits in order, then the padding.
+    int64_t* const idx4 = idx + q0 * nsample;
+    float* const dist4 = dist + q0 * nsample;
+    if (real && !scan)
+        for (int s = sub; s < nsample; s += BT_GROUP)
+        {
+            const bool found = s < cnt;
+            const int2 hit = my_hits[found ? s : 0];
+            const uint32_t out = static_cast<uint32_t>(group * nsample + s);
+            idx4[out] = found ? hit.x : -1;
+            dist4[out] = found ? __int_as_float(hit.y) : -1.0f;
+        }
+
+    // The queries that were given up, one after the other by the whole wavefront.
+    unsigned long long left = __ballot(real && scan && sub == 0);
+    while (left != 0)
+    {
+        const int from = __builtin_ctzll(left);
+        left &= left - 1;
+        const int64_t out = static_cast<int64_t>(from / BT_GROUP) * nsample;
+        ball_scan_rows<false>(x, tpk_read_lane(s0, from), tpk_read_lane(s1, from), to_vector_register(tpk_read_lane(qx, from)),
+                              to_vector_register(tpk_read_lane(qy, from)), to_vector_register(tpk_read_lane(qz, from)), radius2, nsample,
+                              lane, idx4 + out, dist4 + out TPK_WORK_ARG);
+    }
+    TPK_WORK_FLUSH
+}
+
+struct TableLayout
+{
+    int64_t buckets;
+    size_t records, table, chunk_ends, ranks, cloud_rows, placed, total;
+};
+
+TableLayout table_layout(int64_t size_x, int64_t size_y)
+{
+    auto up = [](size_t v) { return (v + 255) & ~static_cast<size_t>(255); };
+    TableLayout l;
+    l.buckets = 2 * BT_CHUNK * BT_PARTS; // (a run that wraps around its part ends in another chunk than it starts in)
+    while (l.buckets < 2 * size_x)
+        l.buckets *= 2;
+    size_t pos = 0;
+    l.records = pos;
+    pos = up(pos + static_cast<size_t>(size_x) * sizeof(float4));
+    l.table = pos;
+    pos = up(pos + static_cast<size_t>(l.buckets) * sizeof(int));
+    l.chunk_ends = pos;
+    pos = up(pos + static_cast<size_t>(l.buckets / BT_CHUNK) * sizeof(int));
+    l.ranks = pos;
+    pos = up(pos + static_cast<size_t>(size_x) * sizeof(int));
+    l.cloud_rows = pos;
+    pos = up(pos + static_cast<size_t>(size_y) * sizeof(int2));
+    l.placed = pos;
+    pos = up(pos + sizeof(int));
+    l.total = pos;
+    return l;
+}
+
+bool table_supported(int64_t size_x, int64_t size_y, int nsample)
+{
+    // Small problems are served as fast by the all-pairs scan; the offsets of records are 32-bit here.
+    return size_x >= 8192 && size_y > 0 && nsample > 0 && size_x < (1LL << 28);
+}
+
+} // namespace
+
+size_t tpk_table_ball_query_workspace_bytes(int64_t size_x, int64_t size_y, int nsample)
+{
+    return table_supported(size_x, size_y, nsample) ? table_layout(size_x, size_y).total : 0;
+}
+
+int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, const float* x, const float* y,
+                                 const int64_t* batch_x, const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
+                                 size_t workspace_bytes, hipStream_t s)
+{
+    if (!table_supported(size_x, size_y, nsample) || !(radius2 < INFINITY)) // (an infinite square accepts points of any cell)
+        return TPK_ERR_UNSUPPORTED;
+    const TableLayout l = table_layout(size_x, size_y);
+    if (!workspace || workspace_bytes < l.total)
+        return TPK_ERR_UNSUPPORTED; // (the bin walk makes do with less)
+    if (reinterpret_cast<uintptr_t>(workspace) & 255u)
+        return TPK_ERR_WORKSPACE;
+    char* w = static_cast<char*>(workspace);
+    float4* records = reinterpret_cast<float4*>(w + l.records);
+    int* table = reinterpret_cast<int*>(w + l.table);
+    int* chunk_ends = reinterpret_cast<int*>(w + l.chunk_ends);
+    int* ranks = reinterpret_cast<int*>(w + l.ranks);
+    int* placed = reinterpret_cast<int*>(w + l.placed);
+    const CloudRows rows{batch_x, batch_y, static_cast<int>(size_x), size_y, reinterpret_cast<int2*>(w + l.cloud_rows)};
+    CellScale scale;
+    scale.reach = bt_reach(radius);
+    scale.inverse_x = 1.0f / (BT_WIDTH_X * scale.reach);
+    scale.inverse_yz = 1.0f / (BT_WIDTH_YZ * scale.reach);
+    const uint32_t part_mask = static_cast<uint32_t>(l.buckets / BT_PARTS - 1);
+    const int n = static_cast<int>(size_x);
+
+    const int64_t point_blocks = tpk_ceil_div(size_x, BT_THREADS), row_blocks = tpk_ceil_div(size_y, BT_THREADS);
+    const int64_t query_blocks = tpk_ceil_div(size_y, BT_THREADS / BT_GROUP);
+    if (query_blocks > 0x7fffffffLL || point_blocks + row_blocks > 0x7fffffffLL)
+        return TPK_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(bt_clear_kernel, dim3(static_cast<unsigned>(tpk_ceil_div(l.buckets / 4, BT_THREADS))), dim3(BT_THREADS), 0, s,
+                       l.buckets / 4, reinterpret_cast<int4*>(table));
+    hipLaunchKernelGGL(bt_count_kernel, dim3(static_cast<unsigned>(point_blocks + row_blocks)), dim3(BT_THREADS), 0, s, n,
+                       static_cast<unsigned>(point_blocks), x, batch_x, scale, part_mask, table, ranks, placed, rows);
+    hipLaunchKernelGGL(bt_places_kernel, dim3(static_cast<unsigned>(l.buckets / BT_CHUNK)), dim3(BT_SCAN_THREADS), 0, s,
+                       reinterpret_cast<int4*>(table), chunk_ends, placed);
+    hipLaunchKernelGGL(bt_records_kernel, dim3(static_cast<unsigned>(point_blocks)), dim3(BT_THREADS), 0, s, n, x, batch_x, scale, part_mask,
+                       table, ranks, records);
+    hipLaunchKernelGGL(bt_query_kernel, dim3(static_cast<unsigned>(query_blocks)), dim3(BT_THREADS), 0, s, size_y, scale, radius2, nsample, part_mask,
+                       x, y, batch_y, rows.rows, records, table, chunk_ends, idx, dist);
+    return tpk_launch_status();
+}

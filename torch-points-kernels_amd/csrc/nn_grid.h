@@ -63,3 +63,11 @@ size_t tpk_grid_ball_query_dense_workspace_bytes(int b, int n, int m, int nsampl
 int tpk_grid_ball_query_dense(int b, int n, int m, float radius, float radius2, int nsample, const float* new_xyz,
                               const float* xyz, int64_t* idx, float* dist, void* workspace, size_t workspace_bytes,
                               hipStream_t stream);
+
+// Ball query, packed layout, unsorted, over a hash table of cells (ball_table.hip): the results of tpk_grid_ball_query_partial,
+// in a larger workspace.  TPK_ERR_UNSUPPORTED (nothing launched) where the workspace is smaller than that, or the radius has no
+// finite square.
+size_t tpk_table_ball_query_workspace_bytes(int64_t size_x, int64_t size_y, int nsample);
+int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, const float* x, const float* y,
+                                 const int64_t* batch_x, const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
+                                 size_t workspace_bytes, hipStream_t stream);

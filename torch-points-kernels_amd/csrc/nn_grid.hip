@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include "ball_scan.h"
 #include "nn_grid.h"
 #include "topk.h"
 
@@ -744,7 +745,8 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void knn_grid_kernel(
 constexpr int NG_RUN = 16; // consecutive cells that share a second-level box in the wavefront-per-query search
 
 // ---------------------------------------------------------------------------------------
-// Ball query over bins, packed layout (several clouds back to back, sorted cloud id per point).
+// Ball query over bins, packed layout (several clouds back to back, sorted cloud id per point): with sorted neighbours, and for
+// workspaces that do not hold the table of ball_table.hip; dense layout above 8192 points.
 //
 // The support array is cut into windows of 8192 or 16384 (bqb_window_shift) consecutive rows, each ordered on its
 // own (curve_cells_kernel), which groups a window's points by the cell of a 16^3 grid over the
@@ -1057,46 +1059,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
         return;
     }
 
-    // Serial semantics directly: lanes hold 64 consecutive support rows; ballot + prefix count
-    // give the hits their slots in index order; stop after nsample hits.
-    cnt = 0;
-    int first_hit = -1; // (dense layout: the row that fills the slots behind the last hit)
-    constexpr int BATCH = 4; // loads of four steps in flight
-    for (int base = s0; base < s1 && cnt < nsample; base += BATCH * TPK_WAVE)
-    {
-        float px[BATCH], py[BATCH], pz[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-        {
-            const int64_t pos = min(base + u * TPK_WAVE + lane, s1 - 1);
-            px[u] = x[pos * 3 + 0];
-            py[u] = x[pos * 3 + 1];
-            pz[u] = x[pos * 3 + 2];
-        }
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-        {
-            const int pos = base + u * TPK_WAVE + lane;
-            const float d = tpk_dist2(qx, qy, qz, px[u], py[u], pz[u]);
-            TPK_WORK_ADD(1);
-            const bool hit = pos < s1 && (DENSE ? d < radius2 : d <= radius2);
-            const unsigned long long mask = __ballot(hit);
-            const int slot = cnt + static_cast<int>(tpk_prefix_count(mask));
-            if (hit && slot < nsample)
-            {
-                idx[out + slot] = DENSE ? pos - s0 : pos;
-                dist[out + slot] = d;
-            }
-            if (DENSE && first_hit < 0 && mask != 0)
-                first_hit = base + u * TPK_WAVE + __builtin_ctzll(mask) - s0;
-            cnt += __builtin_popcountll(mask);
-        }
-    }
-    for (int s = cnt + lane; s < nsample; s += TPK_WAVE)
-    {
-        idx[out + s] = DENSE ? max(first_hit, 0) : -1;
-        dist[out + s] = -1.0f;
-    }
+    ball_scan_rows<DENSE>(x, s0, s1, qx, qy, qz, radius2, nsample, lane, idx + out, dist + out TPK_WORK_ARG);
     TPK_WORK_FLUSH
 }
 

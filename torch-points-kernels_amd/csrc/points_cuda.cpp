@@ -563,7 +563,7 @@ std::pair<at::Tensor, at::Tensor> ball_query_partial_dense(at::Tensor x, at::Ten
                      "ball_query_partial_dense (sorted)");
         return std::make_pair(idx, dist);
     }
-    const size_t ws_bytes = tpk_ball_query_partial_workspace_bytes(x.size(0), y.size(0), nsample);
+    const size_t ws_bytes = tpk_ball_query_partial_table_workspace_bytes(x.size(0), y.size(0), nsample);
     at::Tensor ws;
     if (ws_bytes)
         ws = torch::empty({static_cast<int64_t>(ws_bytes)}, x.options().dtype(torch::kUInt8));
