@@ -54,7 +54,7 @@ TRAFFIC_KERNELS = {
 VALU_KERNELS = {
     "fps": "fps_pool_kernel<16, 16, 2, true>",
     "ball_query_dense": "ball_query_dense_cells_kernel<false>",
-    "ball_query_partial_dense": "bt_query_kernel",
+    "ball_query_partial_dense": "bt_query_kernel<false>",
     "three_nn": "three_nn_cells_kernel",
     "chamfer_fwd": "chamfer_grid_kernel",
 }

@@ -101,7 +101,7 @@ int tpk_ball_query_dense_ws_f32(int b, int n, int m, float radius, int nsample,
  * more than 16 neighbours in the radius are then answered by a scan in index order that stops
  * after nsample hits.  With workspace == NULL every query scans its whole cloud (same results).
  * A workspace of tpk_ball_query_partial_table_workspace_bytes() bytes or more (0 for sizes not served that way; 28 .. 36
- * bytes per support point and 8 per query) holds a hash table of cells instead, the fastest way (same results).
+ * bytes per support point and 8 per query) holds a hash table of cells instead, which calls with many queries take (same results).
  * ------------------------------------------------------------------------------------- */
 size_t tpk_ball_query_partial_workspace_bytes(int64_t size_x, int64_t size_y, int nsample);
 size_t tpk_ball_query_partial_table_workspace_bytes(int64_t size_x, int64_t size_y, int nsample);
@@ -124,8 +124,8 @@ int tpk_ball_query_partial_f32(int64_t size_x, int64_t size_y, float radius, int
  * space filling curve and a query only visits cells within its radius (clouds of 512 support
  * points or more; up to 64 neighbours one wavefront serves a query; dense layout, clouds of
  * 1024 .. 8192 points, up to 64 neighbours: buckets of cells in LDS, workspace not used), same results as the all
- * pairs scan used otherwise.  In the packed layout up to 64 neighbours are found by the walk
- * over bins of tpk_ball_query_partial_f32 (no wait for the stream); more than 64 cloud by
+ * pairs scan used otherwise.  In the packed layout up to 64 neighbours are found in the
+ * table of cells of tpk_ball_query_partial_f32 (no wait for the stream); more than 64 cloud by
  * cloud (clouds of up to 163840 points, cloud ids below 1024; others by all pairs), and only
  * then the call waits for the stream once, to read where the clouds start.
  * ------------------------------------------------------------------------------------- */

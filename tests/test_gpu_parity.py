@@ -390,20 +390,20 @@ def test_ball_query_partial_cell_search_parity(tpk, oracle, dev, sizes, qfrac, r
 @pytest.mark.parametrize(
     "sizes,queries,r,ns,scale,offset,ids",
     [
-        ((8192,), 1, 0.1, 16, 1.0, 0.0, (0,)),                  # the smallest table; a wavefront with one query
-        ((8191, 1), 4099, 0.1, 64, 1.0, -0.5, (-7, 2**62)),     # cells on both sides of zero; ids of any size; a cloud of one point
-        ((5000, 9000, 3), 999, 0.05, 32, 1.0, 0.0, (3, 4, 9)),
-        ((30000,), 2000, 0.3, 16, 1.0, 0.0, (1,)),              # full slots: the scan takes over
-        ((30000,), 2000, 0.05, 16, (1.0, 1.0, 0.01), 0.0, (1,)),  # ... or the lowest rows are kept and the walk goes on
-        ((30000,), 2000, 0.05, 32, (1.0, 1.0, 0.01), 0.0, (1,)),
-        ((30000,), 2000, 0.05, 33, (1.0, 1.0, 0.01), 0.0, (1,)),
-        ((30000,), 2000, 0.045, 100, (1.0, 1.0, 0.01), 0.0, (1,)),  # more than 64 slots
-        ((20000, 20000), 3001, 0.02, 20, 1.0, 3000.0, (0, 1)),  # cells far from the origin: three rows along an axis by rounding
-        ((20000,), 1000, 0.02, 20, 1.0, 300000.0, (0,)),        # hardly any fraction left
-        ((9000,), 500, 0.0, 4, 1.0, 0.0, (0,)),                 # radius 0: the point itself and its copies
-        ((9000,), 500, 1e-25, 4, 1.0, 0.0, (0,)),
-        ((9000,), 500, 1e20, 4, 1.0, 0.0, (0,)),                # radius squared overflows: all points
-        ((300000,), 3000, 0.004, 16, 1.0, 0.0, (0,)),           # many chunks: runs that cross from one to the next
+        ((8192,), 8193, 0.1, 16, 1.0, 0.0, (0,)),               # the smallest table; a wavefront with one query
+        ((8191, 1), 9999, 0.1, 64, 1.0, -0.5, (-7, 2**62)),     # cells on both sides of zero; ids of any size; a cloud of one point
+        ((5000, 9000, 3), 8194, 0.05, 32, 1.0, 0.0, (3, 4, 9)),
+        ((30000,), 8200, 0.3, 16, 1.0, 0.0, (1,)),              # full slots: the scan takes over
+        ((30000,), 8200, 0.05, 16, (1.0, 1.0, 0.01), 0.0, (1,)),  # ... or the lowest rows are kept and the walk goes on
+        ((30000,), 8200, 0.05, 32, (1.0, 1.0, 0.01), 0.0, (1,)),
+        ((30000,), 8200, 0.05, 33, (1.0, 1.0, 0.01), 0.0, (1,)),
+        ((30000,), 8200, 0.045, 100, (1.0, 1.0, 0.01), 0.0, (1,)),  # more than 64 slots
+        ((20000, 20000), 9001, 0.02, 20, 1.0, 3000.0, (0, 1)),  # cells far from the origin: three rows along an axis by rounding
+        ((20000,), 8192, 0.02, 20, 1.0, 300000.0, (0,)),        # hardly any fraction left
+        ((9000,), 8192, 0.0, 4, 1.0, 0.0, (0,)),                 # radius 0: the point itself and its copies
+        ((9000,), 8192, 1e-25, 4, 1.0, 0.0, (0,)),
+        ((9000,), 8192, 1e20, 4, 1.0, 0.0, (0,)),                # radius squared overflows: all points
+        ((300000,), 25003, 0.004, 16, 1.0, 0.0, (0,)),           # many chunks: runs that cross from one to the next
     ],
 )
 def test_ball_query_partial_table(tpk, oracle, dev, sizes, queries, r, ns, scale, offset, ids):
@@ -412,7 +412,7 @@ def test_ball_query_partial_table(tpk, oracle, dev, sizes, queries, r, ns, scale
     x = torch.rand(n, 3, generator=g) * torch.tensor(scale) + offset
     x[n // 2] = x[n // 2 - 1]
     bx = torch.repeat_interleave(torch.tensor(ids), torch.tensor(sizes))
-    pick = torch.sort(torch.randperm(n, generator=g)[:queries]).values
+    pick = torch.sort(torch.randint(0, n, (queries,), generator=g)).values
     y, by = x[pick].clone(), bx[pick]
     y[0] = float("nan")
     y[-1] = float("inf")
@@ -421,6 +421,34 @@ def test_ball_query_partial_table(tpk, oracle, dev, sizes, queries, r, ns, scale
     # (the checker numbers clouds from 0)
     wi, wd = oracle.ball_query_partial_dense(r, ns, x.numpy(), y.numpy(), torch.searchsorted(torch.tensor(ids), bx).numpy(),
                                              torch.searchsorted(torch.tensor(ids), by).numpy())
+    np.testing.assert_array_equal(_np(idx), wi)
+    np.testing.assert_array_equal(_np(dist), wd)
+
+
+@pytest.mark.parametrize(
+    "sizes,queries,r,ns,scale,offset",
+    [
+        ((8192,), 1, 0.1, 16, 1.0, 0.0),
+        ((8191, 1), 4099, 0.1, 64, 1.0, -0.5),
+        ((30000,), 2000, 0.3, 16, 1.0, 0.0),                # many times full: the nearest are kept
+        ((30000,), 2000, 0.05, 64, (1.0, 1.0, 0.01), 0.0),
+        ((20000, 20000), 3001, 0.02, 20, 1.0, 3000.0),      # copies: equal distances, the lower row first
+        ((9000,), 500, 2.0, 7, 1.0, 0.0),                   # more candidates than rows: the rows themselves
+        ((9000,), 50, 1e20, 64, 1.0, 0.0),                  # radius squared overflows
+        ((9000,), 500, 0.0, 4, 1.0, 0.0),                   # nothing is nearer than 0
+    ],
+)
+def test_ball_query_sorted_partial_table(tpk, oracle, dev, sizes, queries, r, ns, scale, offset):
+    g = torch.Generator().manual_seed(len(sizes) * 1000 + queries)
+    n = sum(sizes)
+    x = torch.rand(n, 3, generator=g) * torch.tensor(scale) + offset
+    x[n // 2] = x[n // 2 - 1]
+    bx = torch.repeat_interleave(torch.arange(len(sizes)), torch.tensor(sizes))
+    pick = torch.sort(torch.randperm(n, generator=g)[:queries]).values
+    y, by = x[pick].clone(), bx[pick]
+    y[0] = float("nan")
+    idx, dist = tpk.ball_query(r, ns, x.to(dev), y.to(dev), mode="partial_dense", batch_x=bx.to(dev), batch_y=by.to(dev), sort=True)
+    wi, wd = oracle.ball_query_sorted_partial(r, ns, x.numpy(), y.numpy(), bx.numpy(), by.numpy())
     np.testing.assert_array_equal(_np(idx), wi)
     np.testing.assert_array_equal(_np(dist), wd)
 

@@ -747,7 +747,10 @@ extern "C" size_t tpk_ball_query_partial_workspace_bytes(int64_t size_x, int64_t
 
 extern "C" size_t tpk_ball_query_partial_table_workspace_bytes(int64_t size_x, int64_t size_y, int nsample)
 {
-    return tpk_table_ball_query_workspace_bytes(size_x, size_y, nsample);
+    // (calls that the table does not pay for walk over bins in the same workspace)
+    const size_t table = tpk_table_ball_query_workspace_bytes(size_x, size_y, nsample);
+    const size_t bins = tpk_grid_ball_query_workspace_bytes(size_x, size_y, nsample);
+    return table > bins ? table : bins;
 }
 
 extern "C" int tpk_ball_query_partial_f32(int64_t size_x, int64_t size_y, float radius,
@@ -769,11 +772,11 @@ extern "C" int tpk_ball_query_partial_f32(int64_t size_x, int64_t size_y, float 
     if (workspace)
     {
         // A table of cells where the workspace holds one, else the walk over bins where it applies; otherwise all pairs.
-        int st = tpk_table_ball_query_partial(size_x, size_y, radius, radius2, nsample, x, y, batch_x, batch_y, idx, dist, workspace,
+        int st = tpk_table_ball_query_partial(size_x, size_y, radius, radius2, nsample, false, x, y, batch_x, batch_y, idx, dist, workspace,
                                               workspace_bytes, tpk_stream(stream));
         if (st != TPK_ERR_UNSUPPORTED)
             return st;
-        st = tpk_grid_ball_query_partial(size_x, size_y, radius, radius2, nsample, false, x, y, batch_x, batch_y, idx,
+        st = tpk_grid_ball_query_partial(size_x, size_y, radius, radius2, nsample, x, y, batch_x, batch_y, idx,
                                                    dist, workspace, workspace_bytes, tpk_stream(stream));
         if (st != TPK_ERR_UNSUPPORTED)
             return st;

@@ -22,6 +22,8 @@
 // wavefront are one after the other (radius 1 in rooms of 8: 12500 queries 150 -> 209, 100000 417 -> 448).
 // What bounds it: the counting its atomics, the queries instruction issue - 690 vector instructions per wavefront, 170 per query
 // with 16 hits each, of 1700 clocks a query before.
+// Sorted neighbours (calls against the walk over bins that merged a sorted list, us): 212000 queries of the four scenes 188 -> 69 (16 slots, radius
+// 0.04), 271 -> 85 (64, 0.1), 768 -> 366 (64, 0.3); an eighth of them 48 -> 37 and 67 -> 44.
 // Cells of 1.1 and 0.28 reaches along x: the 300000 queries 96 and 94 us against 94, counting 15 and 13 against 13.
 #include <algorithm>
 #include <cmath>
@@ -30,6 +32,7 @@
 #include "ball_table.h"
 #include "cloud_rows.h"
 #include "nn_grid.h"
+#include "topk.h"
 
 namespace {
 
@@ -182,21 +185,54 @@ __device__ __forceinline__ int row_lane(int v)
     return __builtin_amdgcn_ds_swizzle(v, (L << 5) | 0x10); // and-mask 0x10, or-mask L: in every half wavefront, per row
 }
 
+// What hits are ordered by: their rows, or (SORTED) squared distance and then row - the 64 bits of a hit as they lie in LDS.
+template <bool SORTED>
+struct HitKey;
+template <>
+struct HitKey<false>
+{
+    using type = int;
+    static constexpr type NONE = 0x7fffffff;
+    static __device__ __forceinline__ type of(int2 hit) { return hit.x; }
+    template <int BY>
+    static __device__ __forceinline__ type turned(type v) // row_ror:BY
+    {
+        return __builtin_amdgcn_update_dpp(0, v, 0x120 + BY, 0xF, 0xF, true);
+    }
+    static __device__ __forceinline__ type from_lane(type v, int lane) { return tpk_read_lane(v, lane); }
+};
+template <>
+struct HitKey<true>
+{
+    using type = u64;
+    static constexpr type NONE = ~0ull;
+    static __device__ __forceinline__ type of(int2 hit) { return static_cast<u64>(static_cast<unsigned>(hit.y)) << 32 | static_cast<unsigned>(hit.x); }
+    template <int BY>
+    static __device__ __forceinline__ type turned(type v)
+    {
+        return of(make_int2(HitKey<false>::turned<BY>(static_cast<int>(v)), HitKey<false>::turned<BY>(static_cast<int>(v >> 32))));
+    }
+    static __device__ __forceinline__ type from_lane(type v, int lane) { return read_lane_key(v, lane); }
+};
+
 // How many of the row's values are below `mine`, its own among them.
-template <int BY = 1>
-__device__ __forceinline__ int rank_among_row(int mine)
+template <bool SORTED, int BY = 1>
+__device__ __forceinline__ int rank_among_row(typename HitKey<SORTED>::type mine)
 {
     if constexpr (BY == BT_GROUP)
         return 0;
     else
-        return (__builtin_amdgcn_update_dpp(0, mine, 0x120 + BY, 0xF, 0xF, true) < mine ? 1 : 0) + rank_among_row<BY + 1>(mine); // row_ror:BY
+        return (HitKey<SORTED>::template turned<BY>(mine) < mine ? 1 : 0) + rank_among_row<SORTED, BY + 1>(mine);
 }
 
-// Puts the first cnt hits of every query of the wavefront (int2 (row, distance); cnt is the same in a query's 16 lanes) in ascending order
-// of rows; those that are not among the nsample lowest go.  Up to 16 and 32 hits a query's own
-// lanes rank them, one or two each; above, the whole wavefront ranks one query's after the other's by lane reads, three instructions per hit.
+// Puts the first cnt hits of every query of the wavefront (int2 (row, distance); cnt is the same in a query's 16 lanes) in ascending order;
+// those that are not among the nsample lowest go.  Up to 16 and 32 hits a query's own lanes rank them, one or two each; above, the
+// whole wavefront ranks one query's after the other's by lane reads, three instructions per hit.
+template <bool SORTED>
 __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, int nsample)
 {
+    using K = HitKey<SORTED>;
+    using Key = typename K::type;
     const int group = lane / BT_GROUP, sub = lane % BT_GROUP;
     int2* const hits = wave_hits + group * BT_HIT_STRIDE;
     const int most = bt_most(cnt);
@@ -204,8 +240,7 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
     if (most <= BT_GROUP)
     {
         const int2 hit = hits[sub];
-        const int mine = sub < cnt ? hit.x : 0x7fffffff;
-        const int rank = rank_among_row(mine);
+        const int rank = rank_among_row<SORTED>(sub < cnt ? K::of(hit) : K::NONE);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (sub < cnt && rank < nsample)
             hits[rank] = hit;
@@ -213,12 +248,13 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
     else if (most <= 2 * BT_GROUP)
     {
         const int2 hit0 = hits[sub], hit1 = hits[BT_GROUP + sub];
+        const Key mine0 = K::of(hit0), mine1 = K::of(hit1);
         int rank0 = 0, rank1 = 0;
         for (int i = 0; i < most; ++i)
         {
-            const int other = i < cnt ? hits[i].x : 0x7fffffff;
-            rank0 += other < hit0.x ? 1 : 0;
-            rank1 += other < hit1.x ? 1 : 0;
+            const Key other = i < cnt ? K::of(hits[i]) : K::NONE;
+            rank0 += other < mine0 ? 1 : 0;
+            rank1 += other < mine1 ? 1 : 0;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (sub < cnt && rank0 < nsample)
@@ -235,10 +271,10 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
             if (count <= TPK_WAVE)
             {
                 const int2 hit = of_g[lane];
-                const int mine = lane < count ? hit.x : 0x7fffffff;
+                const Key mine = lane < count ? K::of(hit) : K::NONE;
                 int rank = 0;
                 for (int i = 0; i < count; ++i)
-                    rank += tpk_read_lane(mine, i) < mine ? 1 : 0;
+                    rank += K::from_lane(mine, i) < mine ? 1 : 0;
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 if (lane < count && rank < nsample)
                     of_g[rank] = hit;
@@ -257,10 +293,10 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
             }
             for (int i = 0; i < count; ++i)
             {
-                const int other = of_g[i].x;
+                const Key other = K::of(of_g[i]);
 #pragma unroll
                 for (int j = 0; j < PER; ++j)
-                    rank[j] += other < hit[j].x ? 1 : 0;
+                    rank[j] += other < K::of(hit[j]) ? 1 : 0;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
@@ -281,8 +317,13 @@ __device__ __forceinline__ bool scan_is_shorter(float rows, float nsample, float
     return candidates * (45.0f / (BT_GROUP * BT_QUERIES)) > scan;
 }
 
-__global__ void __launch_bounds__(BT_THREADS)
-    bt_query_kernel(int64_t size_y, CellScale scale, float radius2, int nsample, uint32_t part_mask, const float* __restrict__ x,
+// SORTED: the nsample (<= 64) NEAREST points with squared distance < radius2, nearest first (equal distances: lower row first), instead
+// of the first nsample in row order with squared distance <= radius2.  Nothing ends a scan early then: a query that cannot walk takes
+// its cloud's rows themselves as candidates.
+// unbounded: the radius has no finite square, and accepts points of any cell.
+template <bool SORTED>
+__global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per SIMD; eight would spill the wider keys)
+    bt_query_kernel(int64_t size_y, CellScale scale, float radius2, bool unbounded, int nsample, uint32_t part_mask, const float* __restrict__ x,
                     const float* __restrict__ y, const int64_t* __restrict__ batch_y, const int2* __restrict__ cloud_rows,
                     const float4* __restrict__ records, const int* __restrict__ table, const int* __restrict__ chunk_ends,
                     int64_t* __restrict__ idx, float* __restrict__ dist)
@@ -326,7 +367,7 @@ __global__ void __launch_bounds__(BT_THREADS)
         y0 = bt_scaled_cell(ly), ny = bt_scaled_cell(hy) - y0 + 1;
         z0 = bt_scaled_cell(lz), nz = bt_scaled_cell(hz) - z0 + 1;
     }
-    bool scan = !(nx >= 1 && nx <= BT_MOST_X && ny >= 1 && ny <= 3 && nz >= 1 && nz <= 3);
+    bool scan = unbounded || !(nx >= 1 && nx <= BT_MOST_X && ny >= 1 && ny <= 3 && nz >= 1 && nz <= 3);
     const int runs = scan ? 0 : ny * nz;
     // (up to eight runs: the upper eight lanes take the second halves of runs that cross from one chunk to the next)
     const int run = runs <= 8 ? sub & 7 : sub;
@@ -353,18 +394,22 @@ __global__ void __launch_bounds__(BT_THREADS)
     int total = row_last(before + size, lane);
     // (a run of cells holds 5 to 13 times what the ball itself does, on a surface and in space)
     scan = scan || total > s1 - s0 ||
-           (total > BT_LONG && scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), static_cast<float>(total) * 0.125f, static_cast<float>(total)));
+           (!SORTED && total > BT_LONG && scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), static_cast<float>(total) * 0.125f, static_cast<float>(total)));
     if (scan)
-        total = 0;
+        total = SORTED ? s1 - s0 : 0;
 
     int cnt = 0;             // hits kept so far, the same in all lanes of a query
-    unsigned wanted = s1 - s0; // rows s0 .. s0 + wanted are: the cloud's, or those below the nsample ones that are kept
+    // Once nsample hits are kept, a candidate has to come before the last of them: in the order of rows s0 .. s0 + wanted, or
+    // (SORTED) with a smaller distance than `limit`, or that distance and a row below `limit_row`.
+    unsigned wanted = s1 - s0;
+    float limit = radius2;
+    int limit_row = 0;
     const unsigned group_low = group < 2 ? 0xffffu << group_lane : 0, group_high = group < 2 ? 0 : 0xffffu << (group_lane - 32);
     int most_total = bt_most(total);
     auto record_at = [&](int at) __attribute__((always_inline)) {
-        // (below 2^32 bytes of records: a scalar base and a 32-bit offset)
-        return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(records) + static_cast<uint32_t>(at) * 16u);
+        return records[static_cast<uint32_t>(at)];
     };
+    const bool any_rows = SORTED && __ballot(scan && s1 > s0) != 0;
     const int origin = start - before; // candidate c of a query lies at origin + c, for the c of this lane's run
     // Four runs at most, in the lanes 0 .. 3 of the query, nearly always: where they begin and lie, known to all its lanes.
     const bool few = __ballot(crosses || runs > 4) == 0;
@@ -388,6 +433,11 @@ __global__ void __launch_bounds__(BT_THREADS)
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             at += __builtin_amdgcn_ds_bpermute((group_lane + row_inclusive_max(my_marks[lane])) * 4, origin);
         }
+        if (any_rows && scan)
+        {
+            const int64_t row = s0 + min(c, total - 1);
+            return c < total ? make_float4(x[row * 3 + 0], x[row * 3 + 1], x[row * 3 + 2], __int_as_float(static_cast<int>(row))) : record_at(0);
+        }
         return record_at(c < total ? at : 0);
     };
     int c0 = 0;
@@ -403,7 +453,8 @@ __global__ void __launch_bounds__(BT_THREADS)
             const float d = tpk_dist2(qx, qy, qz, p.x, p.y, p.z);
             TPK_WORK_ADD(has ? 1 : 0);
             const int row = __float_as_int(p.w);
-            const bool hit = has && d <= radius2 && static_cast<unsigned>(row - s0) < wanted;
+            const bool near_enough = SORTED ? d < limit || (d == limit && row < limit_row) : d <= radius2;
+            const bool hit = has && near_enough && static_cast<unsigned>(row - s0) < wanted;
             const unsigned long long all = __ballot(hit);
             if (all == 0)
                 continue;
@@ -421,7 +472,7 @@ __global__ void __launch_bounds__(BT_THREADS)
         // Full: the nsample lowest rows are kept and the walk goes on, or the query is scanned for.  (Once rows are kept
         // their number says nothing about the ball any more.)
         const bool full = cnt > BT_HITS;
-        if (full && wanted == static_cast<unsigned>(s1 - s0))
+        if (!SORTED && full && wanted == static_cast<unsigned>(s1 - s0))
         {
             const float tested = static_cast<float>(min(c0, total)), left = static_cast<float>(total) - tested;
             const float ball = static_cast<float>(cnt) * static_cast<float>(total) * __builtin_amdgcn_rcpf(tested);
@@ -430,11 +481,18 @@ __global__ void __launch_bounds__(BT_THREADS)
             cnt = scan ? 0 : cnt;
         }
         most_total = bt_most(total);
-        order_hits(hits[wave], cnt, lane, nsample);
+        order_hits<SORTED>(hits[wave], cnt, lane, nsample);
         if (cnt >= nsample)
         {
             cnt = nsample;
-            wanted = my_hits[nsample - 1].x - s0;
+            const int2 last = my_hits[nsample - 1];
+            if constexpr (SORTED)
+            {
+                limit = __int_as_float(last.y);
+                limit_row = last.x;
+            }
+            else
+                wanted = last.x - s0;
         }
         if (c0 >= most_total)
             break;
@@ -443,7 +501,7 @@ __global__ void __launch_bounds__(BT_THREADS)
     // The hits in order, then the padding.
     int64_t* const idx4 = idx + q0 * nsample;
     float* const dist4 = dist + q0 * nsample;
-    if (real && !scan)
+    if (real && (SORTED || !scan))
         for (int s = sub; s < nsample; s += BT_GROUP)
         {
             const bool found = s < cnt;
@@ -454,7 +512,7 @@ __global__ void __launch_bounds__(BT_THREADS)
         }
 
     // The queries that were given up, one after the other by the whole wavefront.
-    unsigned long long left = __ballot(real && scan && sub == 0);
+    unsigned long long left = __ballot(!SORTED && real && scan && sub == 0);
     while (left != 0)
     {
         const int from = __builtin_ctzll(left);
@@ -497,10 +555,16 @@ TableLayout table_layout(int64_t size_x, int64_t size_y)
     return l;
 }
 
+// Five launches and an atomic per support point have to pay: with fewer queries, or with fewer than a twelfth as many as points, the walk
+// over bins (two launches) answers a call in row order as soon or sooner.  33000 points, 4100 queries 20.7 us over bins, 23 here,
+// 33000 queries 32 and 24; 100000 points, 12500 queries 30 and 25; 212000 points, 26600 queries 38 and 37.  (Sorted neighbours
+// have this way only: the same calls 23.1 and 24 us - a walk over bins that kept a sorted list -, 43 and 25, 48 and 37.)
+constexpr int64_t BT_MIN_QUERIES = 8192, BT_MOST_SHARE = 12;
+
 bool table_supported(int64_t size_x, int64_t size_y, int nsample)
 {
-    // Small problems are served as fast by the all-pairs scan; the offsets of records are 32-bit here.
-    return size_x >= 8192 && size_y > 0 && nsample > 0 && size_x < (1LL << 28);
+    // Small problems are served as fast by the all-pairs scan; rows and buckets are 32-bit here.
+    return size_x >= 8192 && size_y > 0 && nsample > 0 && size_x < (1LL << 30);
 }
 
 } // namespace
@@ -510,11 +574,12 @@ size_t tpk_table_ball_query_workspace_bytes(int64_t size_x, int64_t size_y, int 
     return table_supported(size_x, size_y, nsample) ? table_layout(size_x, size_y).total : 0;
 }
 
-int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, const float* x, const float* y,
-                                 const int64_t* batch_x, const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
+int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, bool sorted, const float* x,
+                                 const float* y, const int64_t* batch_x, const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
                                  size_t workspace_bytes, hipStream_t s)
 {
-    if (!table_supported(size_x, size_y, nsample) || !(radius2 < INFINITY)) // (an infinite square accepts points of any cell)
+    if (!table_supported(size_x, size_y, nsample) ||
+        (sorted ? nsample > TPK_WAVE : size_y < BT_MIN_QUERIES || size_y * BT_MOST_SHARE < size_x))
         return TPK_ERR_UNSUPPORTED;
     const TableLayout l = table_layout(size_x, size_y);
     if (!workspace || workspace_bytes < l.total)
@@ -547,7 +612,12 @@ int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, f
                        reinterpret_cast<int4*>(table), chunk_ends, placed);
     hipLaunchKernelGGL(bt_records_kernel, dim3(static_cast<unsigned>(point_blocks)), dim3(BT_THREADS), 0, s, n, x, batch_x, scale, part_mask,
                        table, ranks, records);
-    hipLaunchKernelGGL(bt_query_kernel, dim3(static_cast<unsigned>(query_blocks)), dim3(BT_THREADS), 0, s, size_y, scale, radius2, nsample, part_mask,
-                       x, y, batch_y, rows.rows, records, table, chunk_ends, idx, dist);
+    const bool unbounded = !(radius2 < INFINITY);
+    if (sorted)
+        hipLaunchKernelGGL((bt_query_kernel<true>), dim3(static_cast<unsigned>(query_blocks)), dim3(BT_THREADS), 0, s, size_y, scale, radius2, unbounded,
+                           nsample, part_mask, x, y, batch_y, rows.rows, records, table, chunk_ends, idx, dist);
+    else
+        hipLaunchKernelGGL((bt_query_kernel<false>), dim3(static_cast<unsigned>(query_blocks)), dim3(BT_THREADS), 0, s, size_y, scale, radius2, unbounded,
+                           nsample, part_mask, x, y, batch_y, rows.rows, records, table, chunk_ends, idx, dist);
     return tpk_launch_status();
 }

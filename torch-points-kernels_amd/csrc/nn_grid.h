@@ -48,10 +48,9 @@ int tpk_grid_ball_sorted(int b, int n, int m, int nsample, float limit, bool pac
 
 // Ball query, packed layout (a hit has squared distance <= radius2 = radius * radius as the caller
 // rounds it): same conventions.  Queries with dense neighbourhoods are answered by a scan in
-// index order inside the same kernel.  `sorted`: the nsample (<= 64) nearest points with squared
-// distance < radius2 instead, nearest first (equal distances: lower row first), -1 behind them.
+// index order inside the same kernel.
 size_t tpk_grid_ball_query_workspace_bytes(int64_t size_x, int64_t size_y, int nsample);
-int tpk_grid_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, bool sorted,
+int tpk_grid_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample,
                                 const float* x, const float* y, const int64_t* batch_x,
                                 const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
                                 size_t workspace_bytes, hipStream_t stream);
@@ -64,10 +63,11 @@ int tpk_grid_ball_query_dense(int b, int n, int m, float radius, float radius2, 
                               const float* xyz, int64_t* idx, float* dist, void* workspace, size_t workspace_bytes,
                               hipStream_t stream);
 
-// Ball query, packed layout, unsorted, over a hash table of cells (ball_table.hip): the results of tpk_grid_ball_query_partial,
-// in a larger workspace.  TPK_ERR_UNSUPPORTED (nothing launched) where the workspace is smaller than that, or the radius has no
-// finite square.
+// Ball query, packed layout, over a hash table of cells (ball_table.hip): the results of tpk_grid_ball_query_partial in a larger
+// workspace, and (`sorted`) the nsample (<= 64) nearest points with squared distance < radius2, nearest first (equal distances: lower
+// row first), -1 behind them.  TPK_ERR_UNSUPPORTED (nothing launched) where the workspace is too small, and for the few queries
+// in row order that the walk over bins answers as soon.
 size_t tpk_table_ball_query_workspace_bytes(int64_t size_x, int64_t size_y, int nsample);
-int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, const float* x, const float* y,
-                                 const int64_t* batch_x, const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
+int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, bool sorted, const float* x,
+                                 const float* y, const int64_t* batch_x, const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
                                  size_t workspace_bytes, hipStream_t stream);
