@@ -1427,6 +1427,36 @@ def test_grow_proximity_in_several_turns(tpk, dev, n, nsample):
         assert torch.equal(some, members) and torch.equal(ends, starts)
 
 
+@pytest.mark.parametrize("pieces,longest", [(1, 40000), (2, 9000), (1023, 60), (1024, 60), (1025, 60), (3000, 40), (7, 66000)])
+def test_grow_proximity_pieces_by_size(dev, pieces, longest):
+    """Up to 1024 pieces are laid out by size and walked while the later ones are being written (entries of 4 bytes above 65536
+    points); the clusters come out in the order of their first points all the same."""
+    from torch_points_kernels._native import host, native
+
+    rng = np.random.default_rng(pieces)
+    sizes = rng.integers(1, longest + 1, pieces)
+    sizes[pieces // 2] = longest
+    owner = rng.permutation(np.repeat(np.arange(pieces), sizes))
+    rows = np.full((owner.shape[0], 5), -1)
+    for p in range(pieces):
+        points = np.nonzero(owner == p)[0]
+        rows[points, 0] = points
+        for j, step in enumerate((1, 7, 30)):
+            rows[points, j + 1] = np.roll(points, -step)
+        rows[points[-1], 1:] = -1
+    for r in rows:  # (a row names a point once)
+        seen, keep = set(), []
+        for e in r:
+            if e >= 0 and e not in seen:
+                seen.add(e)
+                keep.append(e)
+        r[:] = keep + [-1] * (5 - len(keep))
+    rows = torch.from_numpy(rows)
+    want, ends = host().grow_proximity(rows, 3)
+    got, starts = native().grow_proximity(rows.to(dev), 3, True)
+    assert torch.equal(starts.cpu(), ends) and torch.equal(got.cpu(), want)
+
+
 @pytest.mark.parametrize("n,clusters", [(1, 1), (2049, 3), (65536, 511), (65536, 1023), (65537, 1022), (140001, 1000)])
 def test_grow_proximity_many_clusters_by_index(dev, n, clusters):
     # (cluster, block) tables around the 32768 entries that the prefix sum of the members' sort takes at a time: point i is listed

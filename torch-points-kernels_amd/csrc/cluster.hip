@@ -787,10 +787,38 @@ __global__ void component_info_kernel(int n, const u64* __restrict__ scanned, co
     info[2] = *largest;
 }
 
+// Numbers the pieces by size, the largest first: a caller that walks them on host threads has to wait for the end of the longest
+// walk, so the rows of the largest piece are the ones it wants first.  number: piece of every root; starts: first place of every piece,
+// then the total.  Every thread compares its piece with all others: 5 us for 150 pieces.
+constexpr int CL_RANKED = 1024; // pieces at most; more stay in the order of their first points
+__global__ void __launch_bounds__(CL_RANKED) component_rank_kernel(int pieces, const int* __restrict__ seeds, int* number, int64_t* starts)
+{
+    __shared__ int size[CL_RANKED];
+    const int i = threadIdx.x;
+    const int mine = i < pieces ? (int)(starts[i + 1] - starts[i]) : 0;
+    size[i] = mine;
+    __syncthreads();
+    if (i >= pieces)
+        return;
+    int rank = 0, at = 0;
+    for (int j = 0; j < pieces; ++j)
+    {
+        const int other = size[j];
+        const bool before = other > mine || (other == mine && j < i);
+        rank += before ? 1 : 0;
+        at += before ? other : 0;
+    }
+    starts[rank] = at;
+    number[seeds[i]] = rank;
+}
+
 __global__ void __launch_bounds__(CL_THREADS)
-    component_places_kernel(int count, const unsigned* __restrict__ values, int* place, int32_t* positions)
+    component_places_kernel(int count, const unsigned* __restrict__ values, int* place, int32_t* positions, int pieces,
+                            const int64_t* __restrict__ starts, int64_t* starts_out)
 {
     const int i = blockIdx.x * CL_THREADS + threadIdx.x;
+    if (i <= pieces) // (a piece has a point at least)
+        starts_out[i] = starts[i];
     if (i >= count)
         return;
     const int v = (int)values[i];
@@ -803,13 +831,13 @@ __global__ void __launch_bounds__(CL_THREADS)
 // test for the end of a row.
 template <typename E>
 __global__ void __launch_bounds__(CL_THREADS)
-    component_rows_kernel(int n, int count, int nsample, const int64_t* __restrict__ neighbours, const unsigned* __restrict__ values,
+    component_rows_kernel(int n, int first, int end, int nsample, const int64_t* __restrict__ neighbours, const unsigned* __restrict__ values,
                           const unsigned* __restrict__ keys, const int64_t* __restrict__ starts, const int* __restrict__ place, E* rows)
 {
     const int64_t t = (int64_t)blockIdx.x * CL_THREADS + threadIdx.x;
-    const int64_t slot = t / CL_ROW_LANES;
+    const int64_t slot = first + t / CL_ROW_LANES;
     const int g = (int)(t % CL_ROW_LANES);
-    if (slot >= count)
+    if (slot >= end)
         return; // the whole group of lanes leaves together
     const int shift = (int)(tpk_lane_id() & (TPK_WAVE - CL_ROW_LANES));
     const int64_t u = values[slot];
@@ -927,6 +955,30 @@ __global__ void __launch_bounds__(CL_THREADS)
         return;
     const int64_t p = (int64_t)positions[i];
     members[i] = order ? (int64_t)order[p] : p;
+}
+
+// Member i of the clusters, one after the other, as an index: the cluster it belongs to is found by halving the clusters' first
+// outputs; its row of the table says where its members lie in members_in and from which place its piece's places count.
+template <typename E>
+__global__ void __launch_bounds__(CL_THREADS)
+    grow_members_kernel(int64_t count, int clusters, const int64_t* __restrict__ table, const E* __restrict__ members_in,
+                        const int32_t* __restrict__ positions, const int32_t* __restrict__ order, int64_t* members)
+{
+    const int64_t i = (int64_t)blockIdx.x * CL_THREADS + threadIdx.x;
+    if (i >= count)
+        return;
+    int low = 0, high = clusters - 1; // (the first cluster's first output is 0)
+    while (low < high)
+    {
+        const int middle = (low + high + 1) / 2;
+        if (table[3 * middle] <= i)
+            low = middle;
+        else
+            high = middle - 1;
+    }
+    const int64_t* cluster = table + 3 * (int64_t)low;
+    const int32_t p = positions[cluster[2] + (int64_t)members_in[cluster[1] + (i - cluster[0])]];
+    members[i] = order ? (int64_t)order[p] : (int64_t)p;
 }
 
 struct Layout
@@ -1117,40 +1169,63 @@ extern "C" int tpk_grow_components(int64_t n, int nsample, const int64_t* neighb
     e = static_cast<hipError_t>(tpk_read_back(found, info, 24, s));
     if (e != hipSuccess || found[0] == 0)
         return (int)e;
+    if (found[0] > 1 && found[0] <= CL_RANKED)
+        component_rank_kernel<<<1, CL_RANKED, 0, s>>>((int)found[0], reinterpret_cast<const int*>(ws + l.seeds), number, starts);
     e = sort_points(ni, (unsigned)found[0] + 1u, ClusterKeys{(int)found[0], root, number},
                     SortSpace{keys_in, keys_out, values_in, values_out, ws + l.temp, l.temp_bytes}, s);
     return e != hipSuccess ? (int)e : tpk_launch_status();
 }
 
-extern "C" int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, void* rows,
-                             int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes, void* stream)
+extern "C" int tpk_grow_rows_part(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, int64_t first,
+                                  int64_t count, void* rows, void* workspace, size_t workspace_bytes, void* stream)
 {
-    if (n <= 0 || n > CL_MAX_POINTS || nsample <= 0 || !neighbours || !found || !rows || !positions || !starts || found[0] < 1 ||
-        found[1] < 1 || found[1] > n || (entry_bytes != 2 && entry_bytes != 4) || (entry_bytes == 2 && found[2] > 65536))
+    if (n <= 0 || n > CL_MAX_POINTS || nsample <= 0 || !neighbours || !found || !rows || found[0] < 1 || found[1] < 1 || found[1] > n ||
+        (entry_bytes != 2 && entry_bytes != 4) || (entry_bytes == 2 && found[2] > 65536) || first < 0 || count < 0 || first > found[1] - count)
         return TPK_ERR_INVALID_ARG;
     ComponentLayout l;
     if (!component_layout(n, &l))
         return TPK_ERR_UNSUPPORTED;
     if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0)
         return TPK_ERR_WORKSPACE;
+    if (count == 0)
+        return TPK_OK;
     hipStream_t s = tpk_stream(stream);
     char* ws = static_cast<char*>(workspace);
     const unsigned* keys = reinterpret_cast<const unsigned*>(ws + l.keys_out);
     const unsigned* values = reinterpret_cast<const unsigned*>(ws + l.values_out);
-    int* place = reinterpret_cast<int*>(ws + l.parent); // (the trees are done with)
-    const int count = (int)found[1];
-    const unsigned blocks = (unsigned)tpk_ceil_div(count, CL_THREADS);
-    const unsigned row_blocks = (unsigned)tpk_ceil_div((int64_t)count * CL_ROW_LANES, CL_THREADS);
-    component_places_kernel<<<blocks, CL_THREADS, 0, s>>>(count, values, place, positions);
+    const int* place = reinterpret_cast<const int*>(ws + l.parent);
     const int64_t* from = reinterpret_cast<const int64_t*>(ws + l.starts);
+    const unsigned row_blocks = (unsigned)tpk_ceil_div(count * CL_ROW_LANES, CL_THREADS);
+    const int end = (int)(first + count);
     if (entry_bytes == 2)
-        component_rows_kernel<uint16_t><<<row_blocks, CL_THREADS, 0, s>>>((int)n, count, nsample, neighbours, values, keys, from, place,
+        component_rows_kernel<uint16_t><<<row_blocks, CL_THREADS, 0, s>>>((int)n, (int)first, end, nsample, neighbours, values, keys, from, place,
                                                                            static_cast<uint16_t*>(rows));
     else
-        component_rows_kernel<uint32_t><<<row_blocks, CL_THREADS, 0, s>>>((int)n, count, nsample, neighbours, values, keys, from, place,
+        component_rows_kernel<uint32_t><<<row_blocks, CL_THREADS, 0, s>>>((int)n, (int)first, end, nsample, neighbours, values, keys, from, place,
                                                                            static_cast<uint32_t*>(rows));
-    const hipError_t e = hipMemcpyAsync(starts, from, (size_t)(found[0] + 1) * 8, hipMemcpyDefault, s);
-    return e != hipSuccess ? (int)e : tpk_launch_status();
+    return tpk_launch_status();
+}
+
+extern "C" int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, void* rows,
+                             int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (n <= 0 || n > CL_MAX_POINTS || nsample <= 0 || !neighbours || !found || !positions || !starts || found[0] < 1 ||
+        found[1] < found[0] || found[1] > n || (entry_bytes != 2 && entry_bytes != 4) || (entry_bytes == 2 && found[2] > 65536))
+        return TPK_ERR_INVALID_ARG;
+    ComponentLayout l;
+    if (!component_layout(n, &l))
+        return TPK_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0)
+        return TPK_ERR_WORKSPACE;
+    char* ws = static_cast<char*>(workspace);
+    int* place = reinterpret_cast<int*>(ws + l.parent); // (the trees are done with)
+    const int count = (int)found[1];
+    component_places_kernel<<<(unsigned)tpk_ceil_div((int64_t)count + 1, CL_THREADS), CL_THREADS, 0, tpk_stream(stream)>>>(
+        count, reinterpret_cast<const unsigned*>(ws + l.values_out), place, positions, (int)found[0], reinterpret_cast<const int64_t*>(ws + l.starts),
+        starts);
+    const int status = tpk_launch_status();
+    return status != TPK_OK || !rows ? status
+                                     : tpk_grow_rows_part(n, nsample, neighbours, found, entry_bytes, 0, count, rows, workspace, workspace_bytes, stream);
 }
 
 extern "C" size_t tpk_region_order_workspace_bytes(int64_t n)
@@ -1235,6 +1310,25 @@ extern "C" int tpk_region_members(int64_t count, const int32_t* order, int posit
         region_members_kernel<int32_t><<<blocks, CL_THREADS, 0, tpk_stream(stream)>>>(count, order, static_cast<const int32_t*>(positions), members);
     else
         region_members_kernel<int64_t><<<blocks, CL_THREADS, 0, tpk_stream(stream)>>>(count, order, static_cast<const int64_t*>(positions), members);
+    return tpk_launch_status();
+}
+
+extern "C" int tpk_grow_members(int64_t count, int64_t clusters, const int64_t* table, int entry_bytes, const void* entries,
+                                const int32_t* positions, const int32_t* order, int64_t* members, void* stream)
+{
+    if (count < 0 || clusters < 0 || clusters > CL_MAX_POINTS || (entry_bytes != 2 && entry_bytes != 4))
+        return TPK_ERR_INVALID_ARG;
+    if (count == 0 || clusters == 0)
+        return TPK_OK;
+    if (!table || !entries || !positions || !members)
+        return TPK_ERR_INVALID_ARG;
+    const unsigned blocks = (unsigned)tpk_ceil_div(count, CL_THREADS);
+    if (entry_bytes == 2)
+        grow_members_kernel<<<blocks, CL_THREADS, 0, tpk_stream(stream)>>>(count, (int)clusters, table, static_cast<const uint16_t*>(entries),
+                                                                           positions, order, members);
+    else
+        grow_members_kernel<<<blocks, CL_THREADS, 0, tpk_stream(stream)>>>(count, (int)clusters, table, static_cast<const uint32_t*>(entries),
+                                                                           positions, order, members);
     return tpk_launch_status();
 }
 

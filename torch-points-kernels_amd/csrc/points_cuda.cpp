@@ -9,9 +9,13 @@
 #include <ATen/Parallel.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/Event.h>
 
 #include <algorithm>
 #include <atomic>
+#include <exception>
+#include <mutex>
+#include <thread>
 #include <tuple>
 #include <utility>
 #include <vector>
@@ -178,16 +182,76 @@ at::Tensor host_bytes(int64_t bytes, int64_t most)
     return at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(bytes <= most));
 }
 
-// Walks the pieces begin .. end on host threads; rows: theirs, from the place starts[begin] on.  Adds to `all`.
+// What the device writes into host memory in parts, each followed by an event.  Threads that need what lies before some place wait for
+// the part that holds it: one of them for the event, the others for that one.
+class Arrivals
+{
+public:
+    explicit Arrivals(const at::Tensor& on) : device_(on.get_device()) {}
+    // All before `end` is there when the work enqueued so far is done.
+    void part(int64_t end)
+    {
+        ends_.push_back(end);
+        events_.emplace_back(c10::DeviceType::CUDA);
+        events_.back().record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device_).unwrap());
+    }
+    // Waits for all before `end`.  False: a wait failed, here or in another thread (rethrow() has the error).
+    bool wait(int64_t end)
+    {
+        while (there_.load(std::memory_order_acquire) < end)
+        {
+            if (failed_.load(std::memory_order_acquire))
+                return false;
+            std::unique_lock<std::mutex> lock(turn_, std::try_to_lock);
+            if (!lock.owns_lock())
+            {
+                std::this_thread::yield();
+                continue;
+            }
+            if (there_.load(std::memory_order_relaxed) >= end || failed_.load(std::memory_order_relaxed))
+                continue;
+            try
+            {
+                events_.at(next_).synchronize();
+                there_.store(ends_[next_++], std::memory_order_release);
+            }
+            catch (...)
+            {
+                error_ = std::current_exception();
+                failed_.store(true, std::memory_order_release);
+            }
+        }
+        return true;
+    }
+    void rethrow()
+    {
+        if (error_)
+            std::rethrow_exception(error_);
+    }
+
+private:
+    const c10::DeviceIndex device_;
+    std::vector<c10::Event> events_;
+    std::vector<int64_t> ends_;
+    size_t next_ = 0;
+    std::atomic<int64_t> there_{0};
+    std::atomic<bool> failed_{false};
+    std::exception_ptr error_;
+    std::mutex turn_;
+};
+
+// Walks the pieces begin .. end on host threads; rows: theirs, from the place starts[begin] on.  arrivals: the rows are still being
+// written, in the order of places (nullptr: they are there).  Adds to `all`.
 template <typename E>
-void walk_pieces(const E* rows, int nsample, const int32_t* positions, const int64_t* starts, int64_t begin, int64_t end,
-                 int64_t min_cluster_size, int32_t* places, std::vector<grow_walk::Cluster>* all)
+void walk_pieces(const E* rows, int nsample, const int64_t* starts, int64_t begin, int64_t end, int64_t min_cluster_size, E* entries,
+                 std::vector<grow_walk::Cluster>* all, Arrivals* arrivals)
 {
     const int64_t pieces = end - begin, points = starts[end] - starts[begin];
     std::vector<int64_t> turn(static_cast<size_t>(pieces));
     for (int64_t p = 0; p < pieces; ++p)
         turn[p] = begin + p;
-    // the longest walks first: the end of the last one is what the caller waits for
+    // The longest walks first: the end of the last one is what the caller waits for.  (Up to 1024 pieces lie in that order; more
+    // do not, and where they arrive in parts a thread may have to wait for the last one.)
     std::stable_sort(turn.begin(), turn.end(), [&](int64_t a, int64_t b) { return starts[a + 1] - starts[a] > starts[b + 1] - starts[b]; });
     // (below 16384 points the walk takes less time than waking the other threads)
     const int64_t threads = points < 16384 ? 1 : std::min<int64_t>(at::get_num_threads(), pieces);
@@ -198,8 +262,9 @@ void walk_pieces(const E* rows, int nsample, const int32_t* positions, const int
         for (int64_t i = next.fetch_add(1); i < pieces; i = next.fetch_add(1))
         {
             const int64_t base = starts[turn[i]], count = starts[turn[i] + 1] - base;
-            grow_walk::walk_piece(rows + (base - starts[begin]) * nsample, nsample, positions + base, base, count, min_cluster_size,
-                                  scratch, places, found[t]);
+            if (arrivals && !arrivals->wait(base + count))
+                return;
+            grow_walk::walk_piece(rows + (base - starts[begin]) * nsample, nsample, base, count, min_cluster_size, scratch, entries, found[t]);
         }
     };
     if (threads == 1)
@@ -209,6 +274,8 @@ void walk_pieces(const E* rows, int nsample, const int32_t* positions, const int
             for (int64_t t = first; t < last; ++t)
                 work(t);
         });
+    if (arrivals)
+        arrivals->rethrow();
     for (const auto& f : found)
         all->insert(all->end(), f.begin(), f.end());
 }
@@ -238,37 +305,68 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     if (pieces == 0)
         return at::empty({0}, longs);
     const int64_t entry = found[2] <= 65536 ? 2 : 4, row_bytes = nsample * entry;
-    // one block for all three: starts, positions, rows
+    // One block of pinned memory for starts, positions and rows, the rows written there by the kernel that makes them; where they take
+    // more than `most` they come by themselves.
     const int64_t at_positions = (pieces + 1) * 8, at_rows = (at_positions + points * 4 + 15) / 16 * 16;
-    at::Tensor staged = at::empty({at_rows + points * row_bytes}, bytes_on_device);
-    uint8_t* d = staged.data_ptr<uint8_t>();
-    check_status(tpk_grow_rows(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), d + at_rows,
-                               reinterpret_cast<int32_t*>(d + at_positions), reinterpret_cast<int64_t*>(d), ws.data_ptr(), ws_bytes,
-                               stream),
-                 "grow_proximity (rows)");
-    // (at once where it fits; otherwise the rows come by themselves)
-    const bool at_once = staged.numel() <= most;
-    at::Tensor host = host_bytes(at_once ? staged.numel() : at_rows, most);
-    host.copy_(staged.narrow(0, 0, host.numel()), /*non_blocking=*/true);
-    wait();
-    const uint8_t* h = host.data_ptr<uint8_t>();
+    const bool at_once = at_rows + points * row_bytes <= most;
+    at::Tensor host = host_bytes(at_once ? at_rows + points * row_bytes : at_rows, most);
+    uint8_t* h = host.data_ptr<uint8_t>();
     const int64_t* starts = reinterpret_cast<const int64_t*>(h);
     const int32_t* positions = reinterpret_cast<const int32_t*>(h + at_positions);
-    // (both halves from the pool: fresh memory would cost a page fault per 4 KiB)
-    at::Tensor walked = host_bytes(points * 8, most);
-    int32_t* out = reinterpret_cast<int32_t*>(walked.data_ptr<uint8_t>());
-    int32_t* places = out + points;
+    at::Tensor staged = at::empty({at_rows + (at_once ? 0 : points * row_bytes)}, bytes_on_device);
+    uint8_t* d = staged.data_ptr<uint8_t>();
+    check_status(tpk_grow_rows(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), at_once ? nullptr : d + at_rows,
+                               reinterpret_cast<int32_t*>(d + at_positions), reinterpret_cast<int64_t*>(at_once ? h : d), ws.data_ptr(),
+                               ws_bytes, stream),
+                 "grow_proximity (rows)");
+    // What the walk leaves: the clusters' members as entries, then a table of the clusters.  (From the pool: fresh memory would cost a page fault
+    // per 4 KiB.)
+    const int64_t at_table = (points * entry + 7) / 8 * 8, most_clusters = points / std::max<int64_t>(min_cluster_size, 1);
+    at::Tensor walked = host_bytes(at_table + most_clusters * 24, most);
+    uint8_t* entries = walked.data_ptr<uint8_t>();
     std::vector<grow_walk::Cluster> all;
-    auto walk = [&](const uint8_t* rows, int64_t begin, int64_t end) {
+    auto walk = [&](const uint8_t* rows, int64_t begin, int64_t end, Arrivals* arrivals) {
         if (entry == 2)
-            walk_pieces(reinterpret_cast<const uint16_t*>(rows), nsample, positions, starts, begin, end, min_cluster_size, places, &all);
+            walk_pieces(reinterpret_cast<const uint16_t*>(rows), nsample, starts, begin, end, min_cluster_size, reinterpret_cast<uint16_t*>(entries), &all,
+                        arrivals);
         else
-            walk_pieces(reinterpret_cast<const uint32_t*>(rows), nsample, positions, starts, begin, end, min_cluster_size, places, &all);
+            walk_pieces(reinterpret_cast<const uint32_t*>(rows), nsample, starts, begin, end, min_cluster_size, reinterpret_cast<uint32_t*>(entries), &all,
+                        arrivals);
     };
     if (at_once)
-        walk(h + at_rows, 0, pieces);
+    {
+        // The largest pieces lie first, so their walks, which end last, begin while the others' rows are being written.
+        // (Whatever is thrown on the way, the device must be done with the host block before it goes.)
+        Arrivals arrivals(neighbours);
+        try
+        {
+            const int64_t part = std::max(grow_walk::LEAST_PART / row_bytes, points / grow_walk::PARTS) + 1;
+            for (int64_t first = 0, count; first < points; first += count)
+            {
+                count = std::min(part, points - first);
+                check_status(tpk_grow_rows_part(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), first, count, h + at_rows,
+                                                ws.data_ptr(), ws_bytes, stream),
+                             "grow_proximity (rows)");
+                arrivals.part(first + count);
+            }
+            const int64_t bytes = points * 4;
+            host.narrow(0, at_positions, bytes).copy_(staged.narrow(0, at_positions, bytes), /*non_blocking=*/true);
+            arrivals.part(points + 1);
+            if (arrivals.wait(1))
+                walk(h + at_rows, 0, pieces, &arrivals);
+            arrivals.wait(points + 1);
+            arrivals.rethrow();
+        }
+        catch (...)
+        {
+            wait();
+            throw;
+        }
+    }
     else
     {
+        host.copy_(staged.narrow(0, 0, at_rows), /*non_blocking=*/true);
+        wait();
         at::Tensor turn; // the rows of some pieces
         for (int64_t begin = 0, end = 0; begin < pieces; begin = end)
         {
@@ -279,22 +377,28 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
             at::Tensor rows = turn.narrow(0, 0, bytes);
             rows.copy_(staged.narrow(0, at_rows + starts[begin] * row_bytes, bytes), /*non_blocking=*/true);
             wait();
-            walk(rows.data_ptr<uint8_t>(), begin, end);
+            walk(rows.data_ptr<uint8_t>(), begin, end, nullptr);
         }
     }
-    std::sort(all.begin(), all.end(), [](const grow_walk::Cluster& a, const grow_walk::Cluster& b) { return a.first_position < b.first_position; });
+    std::sort(all.begin(), all.end(), [&](const grow_walk::Cluster& a, const grow_walk::Cluster& b) { return positions[a.base + a.first] < positions[b.base + b.first]; });
+    int64_t* table = reinterpret_cast<int64_t*>(entries + at_table);
     int64_t total = 0;
-    for (const grow_walk::Cluster& c : all)
+    for (size_t c = 0; c < all.size(); ++c)
     {
-        std::memcpy(out + total, places + c.at, static_cast<size_t>(c.size) * sizeof(int32_t));
-        total += c.size;
-        sizes->push_back(c.size);
+        table[3 * c] = total;
+        table[3 * c + 1] = all[c].at;
+        table[3 * c + 2] = all[c].base;
+        total += all[c].size;
+        sizes->push_back(all[c].size);
     }
     at::Tensor members = at::empty({total}, longs);
-    at::Tensor uploaded = at::empty({total * 4}, bytes_on_device);
-    uploaded.copy_(walked.narrow(0, 0, total * 4), /*non_blocking=*/walked.numel() <= most); // (a pageable block goes with this call)
-    check_status(tpk_region_members(total, order.defined() ? order.data_ptr<int32_t>() : nullptr, 4, uploaded.data_ptr(),
-                                    members.data_ptr<int64_t>(), stream),
+    const int64_t clusters = static_cast<int64_t>(all.size()), bytes = at_table + clusters * 24;
+    at::Tensor uploaded = at::empty({bytes}, bytes_on_device);
+    uploaded.copy_(walked.narrow(0, 0, bytes), /*non_blocking=*/walked.numel() <= most); // (a pageable block goes with this call)
+    const uint8_t* u = uploaded.data_ptr<uint8_t>();
+    check_status(tpk_grow_members(total, clusters, reinterpret_cast<const int64_t*>(u + at_table), static_cast<int>(entry), u,
+                                  reinterpret_cast<const int32_t*>(d + at_positions), order.defined() ? order.data_ptr<int32_t>() : nullptr,
+                                  members.data_ptr<int64_t>(), stream),
                  "grow_proximity (members)");
     return members;
 }
