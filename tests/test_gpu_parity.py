@@ -1269,6 +1269,31 @@ def test_knn_by_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
     np.testing.assert_array_equal(_np(dist2), wd)
 
 
+@pytest.mark.parametrize("kind", ["uniform", "clusters", "lattice", "sparse_queries", "crowd"])
+@pytest.mark.parametrize("B,n,m,k", [(1, 8200, 32768, 1), (3, 8193, 10927, 8), (2, 4100, 16385, 9), (2, 9000, 16411, 16), (1, 8200, 32768, 17),
+                                     (1, 8200, 32767, 16), (80, 520, 411, 16), (1400, 512, 24, 3)])
+def test_knn_by_quarters_of_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
+    # from 32768 queries on, up to 16 neighbours: four queries of a cloud a wavefront, the last ones of a cloud fewer; one cell, eight
+    # and 27, more points than the lanes' registers, walks of more than 64 points, equal distances, queries with nothing near them
+    g = torch.Generator().manual_seed(n + k)
+    support, query = torch.rand(B, n, 3, generator=g), torch.rand(B, m, 3, generator=g)
+    if kind == "clusters":
+        support, query = _clustered(g, B, n), _clustered(g, B, m)
+    elif kind == "lattice":
+        support, query = (support * 9).round(), (query * 18).round() / 2
+    elif kind == "sparse_queries":
+        query = query * 4 - 1.5
+    elif kind == "crowd":  # half of the points and queries in a thousandth of the volume
+        support[:, ::2] *= 0.1
+        query[:, ::2] *= 0.1
+    idx, dist2 = tpk.knn(support.to(dev), query.to(dev), k)
+    idx, dist2 = _np(idx), _np(dist2)
+    for rows in (slice(0, 70), slice(max(0, m - 70), m)):
+        wi, wd = oracle.knn(support.numpy(), query[:, rows].contiguous().numpy(), k)
+        np.testing.assert_array_equal(idx[:, rows], wi)
+        np.testing.assert_array_equal(dist2[:, rows], wd)
+
+
 def test_knn_ties_and_errors(tpk, oracle, dev):
     # reference test/test_knn.py:14-23
     support = torch.tensor([[[0, 0, 0], [1, 0, 0], [2, 0, 0]]]).float().to(dev)

@@ -144,34 +144,6 @@ __global__ void __launch_bounds__(BT_THREADS)
     records[table[bucket] + ranks[i]] = make_float4(px, py, pz, __int_as_float(i));
 }
 
-// Sum of v over the lanes below this one in its row of 16.
-__device__ __forceinline__ int row_exclusive_sum(int v)
-{
-    int s = v;
-    s += __builtin_amdgcn_update_dpp(0, s, 0x111, 0xF, 0xF, false); // row_shr:1
-    s += __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false); // row_shr:2
-    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false); // row_shr:4
-    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false); // row_shr:8
-    return s - v;
-}
-
-// Largest of the values v >= 0 of this lane and the lanes below it in its row of 16.
-__device__ __forceinline__ int row_inclusive_max(int v)
-{
-    int s = v;
-    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x111, 0xF, 0xF, false));
-    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false));
-    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false));
-    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false));
-    return s;
-}
-
-// (value of the row's lane 15)
-__device__ __forceinline__ int row_last(int v, int lane)
-{
-    return __builtin_amdgcn_ds_bpermute((lane | (BT_GROUP - 1)) * 4, v);
-}
-
 // The largest of the four queries' values (each the same in the query's lanes).
 __device__ __forceinline__ int bt_most(int v)
 {

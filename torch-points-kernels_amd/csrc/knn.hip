@@ -155,6 +155,60 @@ int launch_knn(int b, int n, int m, int k, float limit, const float* query, cons
     return TPK_OK;
 }
 
+// Distance along axis a from a query (at t, in cells) to cell `at`, a lower bound.
+template <bool MEMORY>
+__device__ __forceinline__ float cell_apart(const LdsGrid& grid, const float* t, int a, int at)
+{
+    float near_end = static_cast<float>(at), far_end = static_cast<float>(at + 1);
+    if constexpr (MEMORY) // (its outermost cells hold all points that lie beyond them)
+    {
+        near_end = at == 0 ? grid.below[a] : near_end;
+        far_end = at == grid.cells[a] - 1 ? grid.above[a] : far_end;
+    }
+    const float gap = fmaxf(near_end - t[a], t[a] - far_end);
+    return fmaxf(gap - 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS)), 0.0f) * grid.width[a];
+}
+
+// The cells of row (y, z) within the ball of squared radius `bound` around the query: of what is left of the radius in this row (for a
+// query far from the cloud the ball is much wider than the stretch of a row that it reaches).  False: none.
+template <bool MEMORY>
+__device__ __forceinline__ bool ball_row(const LdsGrid& grid, const float* t, float bound, int y, int z, int& x_from, int& x_to)
+{
+    const float dy = cell_apart<MEMORY>(grid, t, 1, y), dz = cell_apart<MEMORY>(grid, t, 2, z);
+    const float rest = bound * 1.00001f - (dy * dy + dz * dz);
+    const float span = __builtin_amdgcn_sqrtf(fmaxf(rest, 0.0f)) * 1.00001f * grid.inv[0] + 1e-5f * (fabsf(t[0]) + static_cast<float>(KNG_AXIS));
+    x_from = lg_cell(t[0] - span, grid.cells[0]), x_to = lg_cell(t[0] + span, grid.cells[0]);
+    return rest >= 0.0f;
+}
+
+// Narrows the rows from[1 .. 2] to to[1 .. 2] of the ball around a query more than a cell outside the cloud to what the cloud's distance
+// along the other axes leaves of the ball's radius (a row's cells are trimmed by ball_row).  False: a query not so far out.
+__device__ __forceinline__ bool ball_rows_of_far_query(const LdsGrid& grid, const float* t, float bound, int* from, int* to)
+{
+    float gap[3]; // from the query to the cloud, in cells
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        gap[a] = fmaxf(grid.below[a] - t[a], t[a] - grid.above[a]);
+    if (!(fmaxf(fmaxf(gap[0], gap[1]), gap[2]) > 1.0f))
+        return false;
+    float out[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        const float apart = fmaxf(gap[a] - 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS)), 0.0f) * grid.width[a];
+        out[a] = apart * apart;
+    }
+#pragma unroll
+    for (int a = 1; a < 3; ++a)
+    {
+        const float left = __builtin_amdgcn_sqrtf(fmaxf(bound * 1.00001f - (out[0] + out[3 - a]), 0.0f)) * 1.00001f;
+        const float span = left * grid.inv[a] + 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS));
+        from[a] = lg_cell(t[a] - span, grid.cells[a]);
+        to[a] = lg_cell(t[a] + span, grid.cells[a]);
+    }
+    return true;
+}
+
 // One query by one wavefront over a grid of cells: the 27 cells around it hold k points or the block grows; the k-th of
 // them bounds the ball the answer lies in, and the cells that ball touches outside the block are examined too (one query
 // in three).  The lanes find the candidates of the wavefront's rows of cells by a running maximum: each row's lane leaves
@@ -277,38 +331,13 @@ __device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4
         {
             if constexpr (MEMORY)
             {
-                float gap[3]; // from the query to the cloud, in cells
-                for (int a = 0; a < 3; ++a)
-                    gap[a] = fmaxf(grid.below[a] - t[a], t[a] - grid.above[a]);
-                if (fmaxf(fmaxf(gap[0], gap[1]), gap[2]) > 1.0f)
-                {
-                    // What the cloud's distance along the other axes leaves of the ball's radius (a row's cells are trimmed below).
-                    float out[3];
-                    for (int a = 0; a < 3; ++a)
-                    {
-                        const float apart = fmaxf(gap[a] - 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS)), 0.0f) * grid.width[a];
-                        out[a] = apart * apart;
-                    }
+                if (ball_rows_of_far_query(grid, t, bound, from, to))
                     for (int a = 1; a < 3; ++a)
                     {
-                        const float left = __builtin_amdgcn_sqrtf(fmaxf(bound * 1.00001f - (out[0] + out[3 - a]), 0.0f)) * 1.00001f;
-                        const float span = left * grid.inv[a] + 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS));
-                        from[a] = __builtin_amdgcn_readfirstlane(lg_cell(t[a] - span, grid.cells[a]));
-                        to[a] = __builtin_amdgcn_readfirstlane(lg_cell(t[a] + span, grid.cells[a]));
+                        from[a] = __builtin_amdgcn_readfirstlane(from[a]);
+                        to[a] = __builtin_amdgcn_readfirstlane(to[a]);
                     }
-                }
             }
-            // Distance along axis a from the query to a cell, a lower bound.
-            auto apart = [&](int a, int at) __attribute__((always_inline)) {
-                float near_end = static_cast<float>(at), far_end = static_cast<float>(at + 1);
-                if constexpr (MEMORY) // (its outermost cells hold all points that lie beyond them)
-                {
-                    near_end = at == 0 ? grid.below[a] : near_end;
-                    far_end = at == grid.cells[a] - 1 ? grid.above[a] : far_end;
-                }
-                const float gap = fmaxf(near_end - t[a], t[a] - far_end);
-                return fmaxf(gap - 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS)), 0.0f) * grid.width[a];
-            };
             // the k kept in order, then the rest of the ball: two pieces for a row that crosses the block
             if (place < k)
                 s.keys[place] = mine;
@@ -326,15 +355,11 @@ __device__ __forceinline__ int nearest_in_grid(const LdsGrid& grid, const float4
                     const int iz = static_cast<int>((static_cast<float>(row) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(ny)));
                     const int y = from[1] + row - iz * ny, z = from[2] + iz;
                     const bool crosses = y >= yl && y <= yh && z >= zl && z <= zh;
-                    // the row's cells within the ball: of what is left of its radius in this row (for a query far from the cloud the
-                    // ball is much wider than the stretch of a row that it reaches)
-                    const float dy = apart(1, y), dz = apart(2, z);
-                    const float rest = bound * 1.00001f - (dy * dy + dz * dz);
-                    const float span = __builtin_amdgcn_sqrtf(fmaxf(rest, 0.0f)) * 1.00001f * grid.inv[0] + 1e-5f * (fabsf(t[0]) + static_cast<float>(KNG_AXIS));
-                    const int x_from = lg_cell(t[0] - span, cx), x_to = lg_cell(t[0] + span, cx);
+                    int x_from, x_to;
+                    const bool touched = ball_row<MEMORY>(grid, t, bound, y, z, x_from, x_to);
                     const int x0 = right ? max(xh + 1, x_from) : x_from;
                     const int x1 = right ? (crosses ? x_to : -1) : (crosses ? min(xl - 1, x_to) : x_to);
-                    if (rest >= 0.0f && x1 >= x0)
+                    if (touched && x1 >= x0)
                     {
                         const int c0 = cx * (y + cy * z);
                         start = starts[c0 + x0];
@@ -676,6 +701,22 @@ __global__ __launch_bounds__(LG_THREADS) void knn_grid_build_kernel(int m, float
     });
 }
 
+// The shape of a grid in memory, as its builder left it.
+__device__ __forceinline__ void knn_grid_read(LdsGrid& grid, const float* __restrict__ shape)
+{
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        grid.lo[a] = shape[a];
+        grid.inv[a] = shape[3 + a];
+        grid.width[a] = shape[6 + a];
+        grid.cells[a] = __float_as_int(shape[9 + a]);
+        grid.below[a] = shape[LG_SHAPE + a];
+        grid.above[a] = shape[LG_SHAPE + 3 + a];
+    }
+    grid.volume = shape[12];
+}
+
 __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t queries, int n, int m, int k, KnnGridLayout layout,
                                                                       const float* __restrict__ query, const unsigned char* __restrict__ workspace,
                                                                       float* __restrict__ dist2, int64_t* __restrict__ idx)
@@ -688,24 +729,9 @@ __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t qu
         return; // (no workgroup barrier anywhere in this kernel)
     workspace += (j / n) * layout.total;
     const float qx = to_vector_register(query[j * 3 + 0]), qy = to_vector_register(query[j * 3 + 1]), qz = to_vector_register(query[j * 3 + 2]);
-    const float* __restrict__ const shape = reinterpret_cast<const float*>(workspace + layout.shape);
     TPK_WORK_DECL
     LdsGrid grid;
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-    {
-        grid.lo[a] = shape[a];
-        grid.inv[a] = shape[3 + a];
-        grid.width[a] = shape[6 + a];
-        grid.cells[a] = __float_as_int(shape[9 + a]);
-    }
-    grid.volume = shape[12];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-    {
-        grid.below[a] = shape[LG_SHAPE + a];
-        grid.above[a] = shape[LG_SHAPE + 3 + a];
-    }
+    knn_grid_read(grid, reinterpret_cast<const float*>(workspace + layout.shape));
     Survivors s;
     s.keys = keys[wave];
     s.lane = lane;
@@ -717,6 +743,427 @@ __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t qu
     {
         dist2[j * k + place] = __int_as_float(static_cast<int>(mine >> 32));
         idx[j * k + place] = static_cast<int64_t>(mine & 0xFFFFFFFFu);
+    }
+    TPK_WORK_FLUSH
+}
+
+// Four queries of a cloud per wavefront, 16 lanes each, up to 16 neighbours.  A query looks at a block of cells - its own if that holds 2k
+// points, the eight whose common corner is nearest to it if they hold 4k, else the 27 around it -, has the block's first 16 * PER
+// points in its lanes' registers, PER each, and looks for a distance with k to k + KNQ_SPARE of them within it, all four at once.  The
+// rest of the block, and then the cells outside that the ball around the k nearest so far touches, are walked for points within
+// reach, 16 a step; longer walks by the whole wavefront, 64 a step, one query after the other.  Queries that need a larger block, with
+// too many equal distances or more than KNQ_PIECES rows of cells outside are left to nearest_in_grid.
+// Bound by instruction issue, most of which nearest_in_grid spends whatever the number of candidates: a wavefront that serves one
+// query has 86 of them in an even cloud (k = 16), a third of whose queries look outside.  Calls of k = 4 / 16, a wavefront a query and
+// this way: 8 x 16384 even 87 / 106 -> 63 / 75 us, on a sphere 104 / 118 -> 70 / 80, in clusters of sigma 0.05 121 / 183 -> 91 / 157;
+// 8 x 4099 even 30 / 34 -> 24 / 28, in those clusters 38 / 50 -> 34 / 49; 2 x 100000 even 219 / 241 -> 176 / 191.  Slower are clouds
+// with hundreds of points in most queries' cells (clusters of sigma 0.003: 8 x 16384 341 / 368 -> 355 / 420) and queries far outside
+// the cloud (8 x 16384 120 / 136 -> 84 / 194).
+// (Without the eight cells: 8 x 16384 on a sphere, k = 16, 111; without the walks by the wavefront in clusters 273; with four wavefronts
+// per SIMD instead of six, which spill two registers, 77 to 81 even.)  k = 32, with 16 points a lane, was 8 to 13 % faster in even clouds
+// and 10 to 20 % slower in clusters.  Of 16384 queries even clouds gained 4 to 8 %, 30000 in clusters of sigma 0.02 took 139 us instead of 124.
+constexpr int KNQ_MAX_K = 16;
+constexpr int64_t KNQ_LEAST = 32768; // queries: a wavefront each fills the chip's eight places per SIMD
+constexpr int KNQ_GROUP = 16, KNQ_QUERIES = TPK_WAVE / KNQ_GROUP;
+constexpr int KNQ_OWN = 2, KNQ_EIGHT = 4; // (3 for the eight: within 2 %)
+constexpr int KNQ_SPARE = 16;  // (8: within 2 %)
+constexpr int KNQ_TRIES = 12;  // guesses of the distance
+constexpr int KNQ_FULL = 48;   // keys kept between two steps at most; a step adds up to 64
+constexpr int KNQ_LONG = 64;   // points of a walk by 16 lanes at most (112: 2 % slower in clusters)
+constexpr int KNQ_PIECES = 256;
+
+// Puts the first cnt (<= 16 * HELD) keys of every query of the wavefront in ascending order, of which the k first stay.
+template <int HELD>
+__device__ __forceinline__ void order_kept(u64* mine, int cnt, int k, int sub)
+{
+    u64 key[HELD];
+    int rank[HELD];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (sub < 4)
+        mine[cnt + sub] = ~0ull; // (read four at a time)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int h = 0; h < HELD; ++h)
+    {
+        key[h] = h * KNQ_GROUP + sub < cnt ? mine[h * KNQ_GROUP + sub] : ~0ull;
+        rank[h] = 0;
+    }
+    for (int i = 0; i < cnt; i += 4)
+    {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+        {
+            const u64 other = mine[i + u];
+#pragma unroll
+            for (int h = 0; h < HELD; ++h)
+                rank[h] += other < key[h] ? 1 : 0;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int h = 0; h < HELD; ++h)
+        if (h * KNQ_GROUP + sub < cnt && rank[h] < k)
+            mine[rank[h]] = key[h];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// The same for one query's keys by the whole wavefront, up to two a lane.
+__device__ __forceinline__ void order_kept_by_wave(u64* mine, int cnt, int k, int lane)
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < 4)
+        mine[cnt + lane] = ~0ull;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const u64 key0 = lane < cnt ? mine[lane] : ~0ull, key1 = TPK_WAVE + lane < cnt ? mine[TPK_WAVE + lane] : ~0ull;
+    int rank0 = 0, rank1 = 0;
+    for (int i = 0; i < cnt; i += 4)
+    {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+        {
+            const u64 other = mine[i + u];
+            rank0 += other < key0 ? 1 : 0;
+            rank1 += other < key1 ? 1 : 0;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < cnt && rank0 < k)
+        mine[rank0] = key0;
+    if (TPK_WAVE + lane < cnt && rank1 < k)
+        mine[rank1] = key1;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// The largest of the four queries' values (each the same in the query's lanes).
+__device__ __forceinline__ int most_of_four(int v)
+{
+    return max(max(tpk_read_lane(v, 0), tpk_read_lane(v, 16)), max(tpk_read_lane(v, 32), tpk_read_lane(v, 48)));
+}
+
+template <int PER, int MAX_K>
+__global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, int m, int k, unsigned blocks_per_cloud, KnnGridLayout layout,
+                                                                    const float* __restrict__ query, const unsigned char* __restrict__ workspace,
+                                                                    float* __restrict__ dist2, int64_t* __restrict__ idx)
+{
+    constexpr int WAVES = KNN_THREADS / TPK_WAVE;
+    constexpr int MOST = PER * KNQ_GROUP;                              // a query's candidates
+    constexpr int ROOM = KNQ_FULL + TPK_WAVE + 4;
+    static_assert(MOST <= 256 && MAX_K + KNQ_SPARE <= KNQ_FULL, "");
+    __shared__ u64 keys[WAVES][KNC_ROOM];
+    __shared__ u64 kept[WAVES][KNQ_QUERIES][ROOM];
+    __shared__ unsigned marks[WAVES][KNQ_QUERIES][MOST / 4];
+    const int lane = threadIdx.x & (TPK_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TPK_WAVE);
+    const unsigned block = xcd_local_block(blockIdx.x, gridDim.x);
+    const unsigned cloud = block / blocks_per_cloud;
+    const int64_t j0 = (static_cast<int64_t>(block - cloud * blocks_per_cloud) * WAVES + wave) * KNQ_QUERIES;
+    if (j0 >= n)
+        return; // (no workgroup barrier anywhere in this kernel)
+    workspace += cloud * layout.total;
+    const float* __restrict__ const shape = reinterpret_cast<const float*>(workspace + layout.shape);
+    const int q0 = static_cast<int>(j0);
+    const int group = lane / KNQ_GROUP, sub = lane % KNQ_GROUP;
+    const bool real = q0 + group < n;
+    query += static_cast<int64_t>(cloud) * n * 3;
+    dist2 += static_cast<int64_t>(cloud) * n * k;
+    idx += static_cast<int64_t>(cloud) * n * k;
+    const int64_t j = real ? q0 + group : q0;
+    const float q[3] = {query[j * 3 + 0], query[j * 3 + 1], query[j * 3 + 2]};
+    const float4* __restrict__ const points = reinterpret_cast<const float4*>(workspace);
+    const int* __restrict__ const starts = reinterpret_cast<const int*>(workspace + layout.starts);
+    TPK_WORK_DECL
+    LdsGrid grid;
+    knn_grid_read(grid, shape);
+    Survivors s;
+    s.keys = keys[wave];
+    s.lane = lane;
+    s.k = k;
+
+    // ---- the block's rows of cells, one per lane ----
+    const int cx = grid.cells[0], cy = grid.cells[1];
+    float t[3]; // in cells
+    int c[3], low[3], high[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        t[a] = (q[a] - grid.lo[a]) * grid.inv[a];
+        c[a] = lg_cell(t[a], grid.cells[a]);
+    }
+    // The rows of the 27 cells around the query and of the eight whose common corner is nearest to it: both looked up at once.
+    auto rows_of = [&](const int* from, const int* to, int& start, int& size) __attribute__((always_inline)) {
+        const int ny = to[1] - from[1] + 1, rows = ny * (to[2] - from[2] + 1); // up to 9
+        start = size = 0;
+        if (sub < rows)
+        {
+            int row = sub + (c[1] - from[1]) + ny * (c[2] - from[2]); // (the query's own row first)
+            row -= row >= rows ? rows : 0;
+            const int iz = (row >= ny ? 1 : 0) + (row >= 2 * ny ? 1 : 0);
+            const int c0 = from[0] + cx * ((from[1] + row - iz * ny) + cy * (from[2] + iz));
+            start = starts[c0];
+            size = starts[c0 + to[0] - from[0] + 1] - start;
+        }
+    };
+    int low8[3], high8[3], start, size, start8, size8;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        low[a] = max(c[a] - 1, 0), high[a] = min(c[a] + 1, grid.cells[a] - 1);
+        const bool upper = t[a] - static_cast<float>(c[a]) >= 0.5f;
+        low8[a] = upper ? c[a] : low[a], high8[a] = upper ? high[a] : c[a];
+    }
+    rows_of(low, high, start, size);
+    rows_of(low8, high8, start8, size8);
+    const int own = c[0] + cx * (c[1] + cy * c[2]);
+    const int own_start = starts[own], own_size = starts[own + 1] - own_start;
+    const bool one = own_size >= KNQ_OWN * k, eight = row_last(row_exclusive_sum(size8) + size8, lane) >= KNQ_EIGHT * k;
+    start = one ? own_start : eight ? start8 : start;
+    size = one ? (sub == 0 ? own_size : 0) : eight ? size8 : size;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+        low[a] = one ? c[a] : eight ? low8[a] : low[a];
+        high[a] = one ? c[a] : eight ? high8[a] : high[a];
+    }
+    const int cells = (high[0] - low[0] + 1) * (high[1] - low[1] + 1) * (high[2] - low[2] + 1);
+    const int before = row_exclusive_sum(size);
+    const int total = row_last(before + size, lane);
+    bool good = real && total >= k, done = false;
+    if (__ballot(good) != 0)
+    {
+        // ---- its points: every row's lane marks the place of its first one, a running maximum finds the others' row ----
+        const int origin = start - before; // candidate i of a row's lane lies at origin + i
+        unsigned* const my_marks = marks[wave][group];
+        unsigned char* const mark = reinterpret_cast<unsigned char*>(my_marks);
+#pragma unroll
+        for (int i = 0; i < PER / 4; ++i)
+            my_marks[i * KNQ_GROUP + sub] = 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (good && size > 0 && before < MOST)
+            mark[before] = static_cast<unsigned char>(sub);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        float4 p[PER];
+        int carried = 0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+        {
+            const int at = i * KNQ_GROUP + sub;
+            const int row = max(row_inclusive_max(mark[at]), carried);
+            carried = row_last(row, lane);
+            const int place = __builtin_amdgcn_ds_bpermute((group * KNQ_GROUP + row) * 4, origin) + at;
+            p[i] = points[good && at < total ? place : 0];
+        }
+        float d[PER];
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+        {
+            TPK_WORK_ADD(1);
+            d[i] = good && i * KNQ_GROUP + sub < total ? tpk_dist2(q[0], q[1], q[2], p[i].x, p[i].y, p[i].z) : __builtin_inff();
+        }
+
+        // ---- a distance with k .. k + KNQ_SPARE of them within it (as Survivors::select) ----
+        const float target = static_cast<float>(k + KNQ_SPARE / 2);
+        float guess = s.volume_ratio(0.2387f * grid.volume * static_cast<float>(cells) * __builtin_amdgcn_rcpf(static_cast<float>(total)) * target);
+        Bracket bracket;
+        int within = 0, count = 0, held = 0;
+        for (int tries = 0;; ++tries)
+        {
+            count = 0;
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                count += d[i] <= guess && d[i] < __builtin_inff() ? 1 : 0;
+            within = row_exclusive_sum(count);
+            held = row_last(within + count, lane);
+            const bool fits = held >= k && held <= k + KNQ_SPARE;
+            if (tries == KNQ_TRIES || __ballot(good && !fits) == 0)
+            {
+                good = good && fits;
+                break;
+            }
+            const float estimate = guess * s.volume_ratio(target * __builtin_amdgcn_rcpf(fmaxf(static_cast<float>(held), 0.5f)));
+            const float next = bracket.next(guess, held < k, estimate, tries);
+            guess = fits ? guess : next;
+        }
+
+        u64* const mine = kept[wave][group];
+        int cnt = good ? held : 0; // kept so far
+        float reach = guess;       // the k-th lies within it
+        if (good)
+        {
+            int at = within;
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                if (d[i] <= guess && d[i] < __builtin_inff())
+                    mine[at++] = knn_key(d[i], __float_as_int(p[i].w));
+        }
+        auto order = [&]() __attribute__((always_inline)) {
+            if (most_of_four(cnt) <= 2 * KNQ_GROUP)
+                order_kept<2>(mine, cnt, k, sub);
+            else
+                order_kept<(KNQ_FULL + KNQ_GROUP) / KNQ_GROUP>(mine, cnt, k, sub);
+            if (cnt >= k)
+            {
+                cnt = k;
+                reach = __int_as_float(static_cast<int>(mine[k - 1] >> 32));
+            }
+        };
+        // The candidates from c0 on of the rows of cells that a query's lanes hold.
+        auto walk = [&](int start, int size, int before, int total, int c0) __attribute__((always_inline)) {
+            const int origin = start - before;
+            unsigned long long longer = __ballot(total - c0 > KNQ_LONG && sub == 0);
+            while (longer != 0)
+            {
+                const int first = __builtin_ctzll(longer); // the query's first lane
+                longer &= longer - 1;
+                unsigned char* const mark64 = reinterpret_cast<unsigned char*>(marks[wave][0]);
+                u64* const its = kept[wave][first / KNQ_GROUP];
+                const int its_total = tpk_read_lane(total, first);
+                const float x = to_vector_register(tpk_read_lane(q[0], first)), y = to_vector_register(tpk_read_lane(q[1], first)),
+                            z = to_vector_register(tpk_read_lane(q[2], first));
+                const bool row_here = first / KNQ_GROUP == group && size > 0;
+                int its_cnt = tpk_read_lane(cnt, first);
+                float its_reach = tpk_read_lane(reach, first);
+                auto fetch = [&](int c) __attribute__((always_inline)) {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    mark64[lane] = 0;
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    if (row_here && before < c + TPK_WAVE && before + size > c)
+                        mark64[max(before - c, 0)] = static_cast<unsigned char>(sub);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    const int place = __builtin_amdgcn_ds_bpermute((first + wave_inclusive_max_i32(mark64[lane])) * 4, origin) + c + lane;
+                    return points[c + lane < its_total ? place : 0];
+                };
+                float4 ahead = fetch(c0);
+                for (int c = c0; c < its_total; c += TPK_WAVE)
+                {
+                    const float4 p = ahead;
+                    if (c + TPK_WAVE < its_total)
+                        ahead = fetch(c + TPK_WAVE);
+                    TPK_WORK_ADD(1);
+                    const float d = tpk_dist2(x, y, z, p.x, p.y, p.z);
+                    const bool hit = c + lane < its_total && d <= its_reach && d < __builtin_inff();
+                    const unsigned long long all = __ballot(hit);
+                    if (all == 0)
+                        continue;
+                    if (hit)
+                        its[its_cnt + static_cast<int>(tpk_prefix_count(all))] = knn_key(d, __float_as_int(p.w));
+                    its_cnt += __builtin_popcountll(all);
+                    if (its_cnt > KNQ_FULL)
+                    {
+                        order_kept_by_wave(its, its_cnt, k, lane);
+                        its_cnt = k;
+                        its_reach = tpk_read_lane(__int_as_float(static_cast<int>(its[k - 1] >> 32)), 0);
+                    }
+                }
+                cnt = first / KNQ_GROUP == group ? its_cnt : cnt;
+                reach = first / KNQ_GROUP == group ? its_reach : reach;
+            }
+            total = total - c0 > KNQ_LONG ? 0 : total;
+            const int most = most_of_four(total);
+            auto fetch = [&](int c0) __attribute__((always_inline)) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                mark[sub] = 0;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (size > 0 && before < c0 + KNQ_GROUP && before + size > c0)
+                    mark[max(before - c0, 0)] = static_cast<unsigned char>(sub);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const int place = __builtin_amdgcn_ds_bpermute((group * KNQ_GROUP + row_inclusive_max(mark[sub])) * 4, origin) + c0 + sub;
+                return points[c0 + sub < total ? place : 0];
+            };
+            if (c0 >= most)
+                return;
+            float4 ahead = fetch(c0);
+            for (; c0 < most; c0 += KNQ_GROUP)
+            {
+                const float4 p = ahead;
+                if (c0 + KNQ_GROUP < most)
+                    ahead = fetch(c0 + KNQ_GROUP);
+                TPK_WORK_ADD(1);
+                const float d = tpk_dist2(q[0], q[1], q[2], p.x, p.y, p.z);
+                const bool hit = c0 + sub < total && d <= reach && d < __builtin_inff();
+                const unsigned long long all = __ballot(hit);
+                if (all == 0)
+                    continue;
+                const unsigned here = static_cast<unsigned>(all >> (group * KNQ_GROUP)) & 0xffffu;
+                if (hit)
+                    mine[cnt + __builtin_popcount(here & ((1u << sub) - 1u))] = knn_key(d, __float_as_int(p.w));
+                cnt += __builtin_popcount(here);
+                if (__ballot(cnt > KNQ_FULL) != 0)
+                    order();
+            }
+        };
+        walk(start, size, before, good ? total : 0, MOST);
+        order();
+
+        // ---- the cells outside the block that the ball around the k-th touches (the ends as in nearest_in_grid) ----
+        const float bound = reach;
+        const float radius = __builtin_amdgcn_sqrtf(bound) * 1.00001f;
+        int from[3], to[3];
+        bool inside = true;
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+        {
+            const float span = radius * grid.inv[a] + 1e-5f * (fabsf(t[a]) + static_cast<float>(KNG_AXIS));
+            from[a] = lg_cell(t[a] - span, grid.cells[a]);
+            to[a] = lg_cell(t[a] + span, grid.cells[a]);
+            inside = inside && from[a] >= low[a] && to[a] <= high[a];
+        }
+        if (!inside)
+            ball_rows_of_far_query(grid, t, bound, from, to);
+        const int wide = to[1] - from[1] + 1, pieces = 2 * wide * (to[2] - from[2] + 1); // (two for a row that crosses the block)
+        done = good && (inside || pieces <= KNQ_PIECES);
+        const bool wider = done && !inside;
+        for (int piece0 = 0; __ballot(wider && piece0 < pieces) != 0; piece0 += KNQ_GROUP)
+        {
+            const int e = piece0 + sub;
+            int start = 0, size = 0;
+            if (wider && e < pieces)
+            {
+                const bool right = e & 1;
+                const int row = e >> 1;
+                const int iz = static_cast<int>((static_cast<float>(row) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(wide)));
+                const int y = from[1] + row - iz * wide, z = from[2] + iz;
+                const bool crosses = y >= low[1] && y <= high[1] && z >= low[2] && z <= high[2];
+                int x_from, x_to;
+                const bool touched = ball_row<true>(grid, t, bound, y, z, x_from, x_to);
+                const int x0 = right ? max(high[0] + 1, x_from) : x_from;
+                const int x1 = right ? (crosses ? x_to : -1) : (crosses ? min(low[0] - 1, x_to) : x_to);
+                if (touched && x1 >= x0)
+                {
+                    const int c0 = cx * (y + cy * z);
+                    start = starts[c0 + x0];
+                    size = starts[c0 + x1 + 1] - start;
+                }
+            }
+            const int before = row_exclusive_sum(size);
+            walk(start, size, before, row_last(before + size, lane), 0);
+        }
+        if (__ballot(cnt > k) != 0)
+            order();
+    }
+
+    if (done)
+        for (int e = sub; e < k; e += KNQ_GROUP)
+        {
+            const u64 key = kept[wave][group][e];
+            dist2[j * k + e] = __int_as_float(static_cast<int>(key >> 32));
+            idx[j * k + e] = static_cast<int64_t>(key & 0xFFFFFFFFu);
+        }
+
+    unsigned long long left = __ballot(real && !done && sub == 0);
+    while (left != 0)
+    {
+        const int from = __builtin_ctzll(left);
+        left &= left - 1;
+        u64 mine;
+        const int place = nearest_in_grid<true>(grid, points, starts, m, k, lane, to_vector_register(tpk_read_lane(q[0], from)),
+                                                to_vector_register(tpk_read_lane(q[1], from)), to_vector_register(tpk_read_lane(q[2], from)),
+                                                s, mine TPK_WORK_ARG);
+        const int64_t out = static_cast<int64_t>(q0 + from / KNQ_GROUP) * k;
+        if (place < k)
+        {
+            dist2[out + place] = __int_as_float(static_cast<int>(mine >> 32));
+            idx[out + place] = static_cast<int64_t>(mine & 0xFFFFFFFFu);
+        }
     }
     TPK_WORK_FLUSH
 }
@@ -767,6 +1214,14 @@ int launch_knn_grid(int b, int n, int m, int k, int cells, const float* query, c
     const KnnGridLayout layout = knn_grid_layout(m, cells);
     unsigned char* const w = static_cast<unsigned char*>(workspace);
     hipLaunchKernelGGL(knn_grid_build_kernel, dim3(b), dim3(LG_THREADS), lds, stream, m, knn_per_cell(k), layout, support, w);
+    const int64_t per_cloud = tpk_ceil_div(n, KNQ_QUERIES * (KNN_THREADS / TPK_WAVE));
+    if (k <= KNQ_MAX_K && queries >= KNQ_LEAST && per_cloud * b <= 0x7fffffffLL)
+    {
+        auto* const kernel = k <= 8 ? &knn_grid_four_kernel<4, 8> : &knn_grid_four_kernel<8, KNQ_MAX_K>;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(per_cloud * b)), dim3(KNN_THREADS), 0, stream, n, m, k, static_cast<unsigned>(per_cloud),
+                           layout, query, w, dist2, idx);
+        return tpk_launch_status();
+    }
     hipLaunchKernelGGL(knn_grid_search_kernel, dim3(static_cast<unsigned>(blocks)), dim3(KNN_THREADS), 0, stream, queries, n, m, k, layout,
                        query, w, dist2, idx);
     return tpk_launch_status();

@@ -212,6 +212,34 @@ __device__ __forceinline__ int wave_inclusive_max_i32(int v)
     return s;
 }
 
+// Sum of v over the lanes below this one in its row of 16.
+__device__ __forceinline__ int row_exclusive_sum(int v)
+{
+    int s = v;
+    s += __builtin_amdgcn_update_dpp(0, s, 0x111, 0xF, 0xF, false); // row_shr:1
+    s += __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false); // row_shr:2
+    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false); // row_shr:4
+    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false); // row_shr:8
+    return s - v;
+}
+
+// Largest of the values v >= 0 of this lane and the lanes below it in its row of 16.
+__device__ __forceinline__ int row_inclusive_max(int v)
+{
+    int s = v;
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x111, 0xF, 0xF, false));
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x112, 0xF, 0xF, false));
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xF, false));
+    s = max(s, __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xF, false));
+    return s;
+}
+
+// (value of the row's lane 15)
+__device__ __forceinline__ int row_last(int v, int lane)
+{
+    return __builtin_amdgcn_ds_bpermute((lane | 15) * 4, v);
+}
+
 // Sum of v over the wavefront, the same value in every lane (row rotations, then the four row
 // totals added in lane order: the result does not depend on which lanes call it).
 __device__ __forceinline__ float wave_sum_f32(float v)
