@@ -763,8 +763,9 @@ __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t qu
 // rest of the block, and then the cells outside that the ball around the k nearest so far touches, are walked for points within
 // reach, 16 a step; longer walks by the whole wavefront, 64 a step, one query after the other.  Queries that need a larger block, with
 // too many equal distances or more than KNQ_PIECES rows of cells outside are left to nearest_in_grid.
-// Bound by instruction issue, most of which nearest_in_grid spends whatever the number of candidates: a wavefront that serves one
-// query has 86 of them in an even cloud (k = 16), a third of whose queries look outside.  Calls of k = 4 / 16, a wavefront a query and
+// Bound by instruction issue (8 x 16384 even, k = 16: 1010 vector instructions per wavefront, 252 per query, 55 of the kernel's 59 us), most of
+// which nearest_in_grid spends whatever the number of candidates: a wavefront that serves one query has 86 of them in an even cloud (k = 16),
+// a third of whose queries look outside.  Calls of k = 4 / 16, a wavefront a query and
 // this way: 8 x 16384 even 87 / 106 -> 63 / 75 us, on a sphere 104 / 118 -> 70 / 80, in clusters of sigma 0.05 121 / 183 -> 91 / 157;
 // 8 x 4099 even 30 / 34 -> 24 / 28, in those clusters 38 / 50 -> 34 / 49; 2 x 100000 even 219 / 241 -> 176 / 191.  Slower are clouds
 // with hundreds of points in most queries' cells (clusters of sigma 0.003: 8 x 16384 341 / 368 -> 355 / 420) and queries far outside
@@ -773,7 +774,7 @@ __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t qu
 // per SIMD instead of six, which spill two registers, 77 to 81 even.)  k = 32, with 16 points a lane, was 8 to 13 % faster in even clouds
 // and 10 to 20 % slower in clusters.  Of 16384 queries even clouds gained 4 to 8 %, 30000 in clusters of sigma 0.02 took 139 us instead of 124.
 constexpr int KNQ_MAX_K = 16;
-constexpr int64_t KNQ_LEAST = 32768; // queries: a wavefront each fills the chip's eight places per SIMD
+constexpr int64_t KNQ_LEAST = 32768; // queries: the chip has 8192 places for wavefronts
 constexpr int KNQ_GROUP = 16, KNQ_QUERIES = TPK_WAVE / KNQ_GROUP;
 constexpr int KNQ_OWN = 2, KNQ_EIGHT = 4; // (3 for the eight: within 2 %)
 constexpr int KNQ_SPARE = 16;  // (8: within 2 %)
