@@ -777,7 +777,7 @@ constexpr int KNQ_MAX_K = 16;
 constexpr int64_t KNQ_LEAST = 32768; // queries: the chip has 8192 places for wavefronts
 constexpr int KNQ_GROUP = 16, KNQ_QUERIES = TPK_WAVE / KNQ_GROUP;
 constexpr int KNQ_OWN = 2, KNQ_EIGHT = 4; // (3 for the eight: within 2 %)
-constexpr int KNQ_SPARE = 16;  // (8: within 2 %)
+constexpr int KNQ_SPARE = 16;  // (8: 1 to 3 % faster, but then nothing separates the 8 nearest on a lattice, where 7 and 19 points lie within a distance)
 constexpr int KNQ_TRIES = 12;  // guesses of the distance
 constexpr int KNQ_FULL = 48;   // keys kept between two steps at most; a step adds up to 64
 constexpr int KNQ_LONG = 64;   // points of a walk by 16 lanes at most (112: 2 % slower in clusters)
