@@ -17,6 +17,37 @@ SHIM = r"""
 #include "grid_shape.h"
 #include "grow_walk.h"
 #include <cmath>
+#include <stdexcept>
+
+// What happened to a block that the device was writing into when something was thrown, or not: 'w' the device was waited for, 'r' the
+// block went.
+extern "C" void block_given_up(int begun, int ended, int thrown, int wait_fails, char* log)
+{
+    struct Block
+    {
+        char*& log;
+        ~Block() { *log++ = 'r'; }
+    };
+    try
+    {
+        Block block{log};
+        auto wait = [&] {
+            *log++ = 'w';
+            if (wait_fails)
+                throw std::runtime_error("wait");
+        };
+        grow_walk::PendingWrites<decltype(wait)> writes(wait);
+        if (begun)
+            writes.begin();
+        if (thrown)
+            throw std::runtime_error("between");
+        if (ended)
+            writes.end();
+    }
+    catch (const std::runtime_error&)
+    {
+    }
+}
 
 extern "C" void grid_of(const float* low, const float* high, int m, float per_cell, int axis, int most, float* extent, int* along)
 {
@@ -217,6 +248,21 @@ def test_turns_of_pieces_stay_within_their_bytes(shim, row_bytes, most):
             assert end == begin + 1 or (starts[end] - starts[begin]) * row_bytes <= most
             assert end == pieces or (starts[end + 1] - starts[begin]) * row_bytes > most
             begin = end
+
+
+def test_a_block_goes_after_the_device_is_done_with_it(shim):
+    """The host block that the rows kernel writes into: the wait for the device comes before it goes back to its pool, whatever is
+    thrown behind the first launch that writes there."""
+    for begun, ended, thrown, fails, want in ((1, 0, 1, 0, b"wr"), (1, 0, 1, 1, b"wr"), (1, 0, 0, 0, b"wr"), (1, 1, 0, 0, b"r"), (0, 0, 1, 0, b"r")):
+        log = ctypes.create_string_buffer(8)
+        shim.block_given_up(begun, ended, thrown, fails, log)
+        assert log.value == want
+    with open(os.path.join(CSRC, "points_cuda.cpp")) as f:
+        body = f.read().split("at::Tensor grow_reference_order(")[1].split("\n}\n")[0]
+    # the guard lives behind the block and is set before the first launch that is handed the block
+    order = [body.index(s) for s in ("at::Tensor host =", "PendingWrites<decltype(wait)> writes(wait)", "writes.begin()", "tpk_grow_rows(",
+                                     "tpk_grow_rows_part(", "arrivals.wait(points + 1)", "writes.end()")]
+    assert order == sorted(order)
 
 
 @pytest.mark.parametrize("scale", [1e-30, 1e-3, 1.0, 5e3, 4e6, 3e30])

@@ -34,6 +34,35 @@ constexpr int64_t MOST_STAGED = int64_t(256) << 20;
 // all rows copied, then walked: 965; copied in 8 parts by the runtime, 32 us each: 938.
 constexpr int64_t PARTS = 5, LEAST_PART = int64_t(1) << 20;
 
+// Declared behind a host block that the device writes into by a kernel: whatever is thrown between begin() and end(), the wait for the
+// device comes before the block goes.  (The pool that owns such blocks knows of copies into them, not of kernels.)
+template <typename Wait>
+class PendingWrites
+{
+public:
+    explicit PendingWrites(const Wait& wait) : wait_(wait) {}
+    PendingWrites(const PendingWrites&) = delete;
+    PendingWrites& operator=(const PendingWrites&) = delete;
+    ~PendingWrites()
+    {
+        if (!pending_)
+            return;
+        try
+        {
+            wait_();
+        }
+        catch (...) // (the device is gone, and with it whatever it was writing)
+        {
+        }
+    }
+    void begin() { pending_ = true; }
+    void end() { pending_ = false; }
+
+private:
+    const Wait& wait_;
+    bool pending_ = false;
+};
+
 // Walks one piece of `count` points.  Clusters of at least min_size members go to `found`, their members - as
 // places inside the piece - to entries[at ...], which never takes more than the piece's own range (base and on).
 template <typename E>

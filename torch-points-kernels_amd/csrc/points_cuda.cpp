@@ -310,11 +310,14 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     const int64_t at_positions = (pieces + 1) * 8, at_rows = (at_positions + points * 4 + 15) / 16 * 16;
     const bool at_once = at_rows + points * row_bytes <= most;
     at::Tensor host = host_bytes(at_once ? at_rows + points * row_bytes : at_rows, most);
+    grow_walk::PendingWrites<decltype(wait)> writes(wait); // (gone before `host` is)
     uint8_t* h = host.data_ptr<uint8_t>();
     const int64_t* starts = reinterpret_cast<const int64_t*>(h);
     const int32_t* positions = reinterpret_cast<const int32_t*>(h + at_positions);
     at::Tensor staged = at::empty({at_rows + (at_once ? 0 : points * row_bytes)}, bytes_on_device);
     uint8_t* d = staged.data_ptr<uint8_t>();
+    if (at_once)
+        writes.begin();
     check_status(tpk_grow_rows(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), at_once ? nullptr : d + at_rows,
                                reinterpret_cast<int32_t*>(d + at_positions), reinterpret_cast<int64_t*>(at_once ? h : d), ws.data_ptr(),
                                ws_bytes, stream),
@@ -336,32 +339,24 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     if (at_once)
     {
         // The largest pieces lie first, so their walks, which end last, begin while the others' rows are being written.
-        // (Whatever is thrown on the way, the device must be done with the host block before it goes.)
         Arrivals arrivals(neighbours);
-        try
+        const int64_t part = std::max(grow_walk::LEAST_PART / row_bytes, points / grow_walk::PARTS) + 1;
+        for (int64_t first = 0, count; first < points; first += count)
         {
-            const int64_t part = std::max(grow_walk::LEAST_PART / row_bytes, points / grow_walk::PARTS) + 1;
-            for (int64_t first = 0, count; first < points; first += count)
-            {
-                count = std::min(part, points - first);
-                check_status(tpk_grow_rows_part(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), first, count, h + at_rows,
-                                                ws.data_ptr(), ws_bytes, stream),
-                             "grow_proximity (rows)");
-                arrivals.part(first + count);
-            }
-            const int64_t bytes = points * 4;
-            host.narrow(0, at_positions, bytes).copy_(staged.narrow(0, at_positions, bytes), /*non_blocking=*/true);
-            arrivals.part(points + 1);
-            if (arrivals.wait(1))
-                walk(h + at_rows, 0, pieces, &arrivals);
-            arrivals.wait(points + 1);
-            arrivals.rethrow();
+            count = std::min(part, points - first);
+            check_status(tpk_grow_rows_part(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), first, count, h + at_rows,
+                                            ws.data_ptr(), ws_bytes, stream),
+                         "grow_proximity (rows)");
+            arrivals.part(first + count);
         }
-        catch (...)
-        {
-            wait();
-            throw;
-        }
+        const int64_t bytes = points * 4;
+        host.narrow(0, at_positions, bytes).copy_(staged.narrow(0, at_positions, bytes), /*non_blocking=*/true);
+        arrivals.part(points + 1);
+        if (arrivals.wait(1))
+            walk(h + at_rows, 0, pieces, &arrivals);
+        arrivals.wait(points + 1);
+        arrivals.rethrow();
+        writes.end();
     }
     else
     {
