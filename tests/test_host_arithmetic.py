@@ -15,6 +15,7 @@ SHIM = r"""
 #include "cloud_ids.h"
 #include "die_map.h"
 #include "grid_shape.h"
+#include "grow_table.h"
 #include "grow_walk.h"
 #include <cmath>
 #include <stdexcept>
@@ -47,6 +48,19 @@ extern "C" void block_given_up(int begun, int ended, int thrown, int wait_fails,
     catch (const std::runtime_error&)
     {
     }
+}
+
+// The cluster of output i where cluster c's outputs begin at c * each; -1: a word outside the table was asked for.
+extern "C" int cluster_of(int clusters, long long each, long long i)
+{
+    bool outside = false;
+    const int c = grow_cluster_of(
+        [&](int64_t word) {
+            outside = outside || word < 0 || word >= int64_t(GROW_TABLE_ROW) * clusters || word % GROW_TABLE_ROW != 0;
+            return word / GROW_TABLE_ROW * each;
+        },
+        clusters, i);
+    return outside ? -1 : c;
 }
 
 extern "C" void grid_of(const float* low, const float* high, int m, float per_cell, int axis, int most, float* extent, int* along)
@@ -263,6 +277,17 @@ def test_a_block_goes_after_the_device_is_done_with_it(shim):
     order = [body.index(s) for s in ("at::Tensor host =", "PendingWrites<decltype(wait)> writes(wait)", "writes.begin()", "tpk_grow_rows(",
                                      "tpk_grow_rows_part(", "arrivals.wait(points + 1)", "writes.end()")]
     assert order == sorted(order)
+
+
+@pytest.mark.parametrize("clusters", [1, 2, 3, 1000, 715827882, 715827883, 2 ** 30])
+def test_an_outputs_cluster_is_found_in_a_table_of_any_size(shim, clusters):
+    """(from 715827883 clusters on a word's number takes more than 31 bits)"""
+    shim.cluster_of.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong]
+    for each in (1, 7):
+        for c in {0, 1, clusters // 3, clusters // 2, clusters - 2, clusters - 1}:
+            for i in (c * each, c * each + each - 1):
+                if 0 <= i < clusters * each:
+                    assert shim.cluster_of(clusters, each, i) == c
 
 
 @pytest.mark.parametrize("scale", [1e-30, 1e-3, 1.0, 5e3, 4e6, 3e30])

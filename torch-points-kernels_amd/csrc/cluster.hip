@@ -39,6 +39,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "cloud_ids.h"
+#include "grow_table.h"
 #include "tpk_device.h"
 
 namespace
@@ -957,8 +958,8 @@ __global__ void __launch_bounds__(CL_THREADS)
     members[i] = order ? (int64_t)order[p] : p;
 }
 
-// Member i of the clusters, one after the other, as an index: the cluster it belongs to is found by halving the clusters' first
-// outputs; its row of the table says where its members lie in members_in and from which place its piece's places count.
+// Member i of the clusters, one after the other, as an index: its cluster's row of the table says where the cluster's members lie in members_in
+// and from which place its piece's places count.
 template <typename E>
 __global__ void __launch_bounds__(CL_THREADS)
     grow_members_kernel(int64_t count, int clusters, const int64_t* __restrict__ table, const E* __restrict__ members_in,
@@ -967,16 +968,8 @@ __global__ void __launch_bounds__(CL_THREADS)
     const int64_t i = (int64_t)blockIdx.x * CL_THREADS + threadIdx.x;
     if (i >= count)
         return;
-    int low = 0, high = clusters - 1; // (the first cluster's first output is 0)
-    while (low < high)
-    {
-        const int middle = (low + high + 1) / 2;
-        if (table[3 * middle] <= i)
-            low = middle;
-        else
-            high = middle - 1;
-    }
-    const int64_t* cluster = table + 3 * (int64_t)low;
+    const int c = grow_cluster_of([&](int64_t word) { return table[word]; }, clusters, i);
+    const int64_t* cluster = table + GROW_TABLE_ROW * (int64_t)c;
     const int32_t p = positions[cluster[2] + (int64_t)members_in[cluster[1] + (i - cluster[0])]];
     members[i] = order ? (int64_t)order[p] : (int64_t)p;
 }
