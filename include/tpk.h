@@ -367,11 +367,14 @@ int tpk_grow_proximity(int64_t n, int nsample, const int64_t* neighbours, int64_
  *     stream once.  Leaves what tpk_grow_rows needs in the workspace (tpk_grow_components_workspace_bytes(n), 256-byte
  *     aligned; 0 as for tpk_grow_proximity).
  *   tpk_grow_rows (found[0] > 0): starts (found[0] + 1) int64, first place of every piece and the total;
- *     positions (found[1]) the point at every place, ascending inside a piece, up to 1024 pieces the largest first (then
- *     the one with the lower first point), more in the order of their first points; rows (found[1], nsample) of uint16 (entry_bytes 2, pieces up to 65536 points) or uint32 (4): entries as
+ *     positions (found[1]) the point at every place, ascending inside a piece, pieces in the order of their first
+ *     points; rows (found[1], nsample) of uint16 (entry_bytes 2, pieces up to 65536 points) or uint32 (4): entries as
  *     places inside the piece, in row order, the place itself behind the row's end.  The outputs may lie in device
- *     memory or in host memory the device can address.  rows NULL: starts and positions only, and the rows of the places
- *     first .. first + count by tpk_grow_rows_part behind it on the stream (`rows` is where place 0's would lie).
+ *     memory or in host memory the device can address.
+ *   tpk_grow_places, then tpk_grow_rows_part behind it on the stream: the same in parts - starts and positions only, then the
+ *     rows of the places first .. first + count (`rows` is where place 0's would lie).
+ *   tpk_grow_components_by_size: tpk_grow_components with up to 1024 pieces in the order of their sizes instead, the largest first
+ *     (equal sizes: lower first point first).
  *   tpk_grow_members: members (count) int64, the clusters the walk found one after the other: table (clusters, 3) int64,
  *     ascending, first output of every cluster (0 for the first), its first entry in entries, which holds its members as places
  *     inside their piece (uint16 or uint32), and the first place of that piece; positions as above; order: see
@@ -379,6 +382,10 @@ int tpk_grow_proximity(int64_t n, int nsample, const int64_t* neighbours, int64_
 size_t tpk_grow_components_workspace_bytes(int64_t n);
 int tpk_grow_components(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, int64_t* found,
                         void* workspace, size_t workspace_bytes, void* stream);
+int tpk_grow_components_by_size(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, int64_t* found,
+                                void* workspace, size_t workspace_bytes, void* stream);
+int tpk_grow_places(int64_t n, const int64_t* found, int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes,
+                    void* stream);
 int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, void* rows,
                   int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes, void* stream);
 int tpk_grow_rows_part(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, int64_t first,

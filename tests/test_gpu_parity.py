@@ -2201,6 +2201,55 @@ def test_gridding_last_cell_matches_the_reference_formula_inside_the_grid(tpk, d
     check_last_cell_behaviour(gridding)
 
 
+def test_c_abi_pieces_in_the_order_of_their_first_points(dev):
+    """tpk_grow_components / tpk_grow_rows lay the pieces out in the order of their first points, ..._by_size the largest first; the
+    rows in parts are the rows at once; no rows is an error."""
+    import ctypes
+    import os
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_grow_components_workspace_bytes.restype = ctypes.c_size_t
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    Z, L = ctypes.c_size_t, ctypes.c_int64
+    pieces = [[0, 5], [1, 2, 8, 9], [3], [4, 6, 7, 10, 11], [12, 13, 14, 15]]
+    n, nsample = 16, 3
+    rows = torch.full((n, nsample), -1, dtype=torch.int64)
+    for piece in pieces:
+        for i, p in enumerate(piece):
+            rows[p, 0] = p
+            if len(piece) > 1:
+                rows[p, 1] = piece[(i + 1) % len(piece)]
+    neighbours = rows.to(dev)
+    nbytes = lib.tpk_grow_components_workspace_bytes(L(n))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    stream = torch.cuda.current_stream()
+    S = ctypes.c_void_p(stream.cuda_stream)
+    by_first = [p for p in pieces if len(p) > 1]
+    for components, want in ((lib.tpk_grow_components, by_first), (lib.tpk_grow_components_by_size, sorted(by_first, key=lambda p: -len(p)))):
+        found = (ctypes.c_int64 * 3)()
+        assert components(L(n), nsample, P(neighbours), L(2), found, P(ws), Z(nbytes), S) == 0
+        assert list(found) == [4, 15, 5]
+        starts = torch.full((5,), -1, dtype=torch.int64, device=dev)
+        positions = torch.full((15,), -1, dtype=torch.int32, device=dev)
+        at_once = torch.full((15, nsample), 77, dtype=torch.int16, device=dev)
+        assert lib.tpk_grow_rows(L(n), nsample, P(neighbours), found, 2, None, P(positions), P(starts), P(ws), Z(nbytes), S) == -1
+        assert lib.tpk_grow_rows(L(n), nsample, P(neighbours), found, 2, P(at_once), P(positions), P(starts), P(ws), Z(nbytes), S) == 0
+        assert positions.tolist() == sum(want, [])
+        assert starts.tolist() == [0] + list(np.cumsum([len(p) for p in want]))
+        expect = [[i, (i + 1) % len(p), i] for p in want for i in range(len(p))]
+        assert at_once.tolist() == expect
+        for entry_bytes, dtype in ((2, torch.int16), (4, torch.int32)):
+            parts = torch.full((15, nsample), 77, dtype=dtype, device=dev)
+            starts.fill_(-1)
+            positions.fill_(-1)
+            assert lib.tpk_grow_places(L(n), found, P(positions), P(starts), P(ws), Z(nbytes), S) == 0
+            for first, count in ((11, 4), (0, 7), (7, 0), (7, 4)):
+                assert lib.tpk_grow_rows_part(L(n), nsample, P(neighbours), found, entry_bytes, L(first), L(count), P(parts), P(ws), Z(nbytes), S) == 0
+            assert parts.tolist() == expect and positions.tolist() == sum(want, [])
+            assert lib.tpk_grow_rows_part(L(n), nsample, P(neighbours), found, entry_bytes, L(12), L(4), P(parts), P(ws), Z(nbytes), S) == -1
+
+
 def test_c_abi_direct_call(oracle, dev):
     """libtpk_hip.so used without the extension: ctypes + raw device pointers + a stream."""
     import ctypes

@@ -274,14 +274,14 @@ def test_a_block_goes_after_the_device_is_done_with_it(shim):
     with open(os.path.join(CSRC, "points_cuda.cpp")) as f:
         body = f.read().split("at::Tensor grow_reference_order(")[1].split("\n}\n")[0]
     # the guard lives behind the block and is set before the first launch that is handed the block
-    order = [body.index(s) for s in ("at::Tensor host =", "PendingWrites<decltype(wait)> writes(wait)", "writes.begin()", "tpk_grow_rows(",
+    order = [body.index(s) for s in ("at::Tensor host =", "PendingWrites<decltype(wait)> writes(wait)", "writes.begin()", "tpk_grow_places(",
                                      "tpk_grow_rows_part(", "arrivals.wait(points + 1)", "writes.end()")]
     assert order == sorted(order)
 
 
-@pytest.mark.parametrize("clusters", [1, 2, 3, 1000, 715827882, 715827883, 2 ** 30])
+@pytest.mark.parametrize("clusters", [1, 2, 3, 1000, 715827883, 715827884, 2 ** 30])
 def test_an_outputs_cluster_is_found_in_a_table_of_any_size(shim, clusters):
-    """(from 715827883 clusters on a word's number takes more than 31 bits)"""
+    """(from 715827884 clusters on a word's number takes more than 31 bits)"""
     shim.cluster_of.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong]
     for each in (1, 7):
         for c in {0, 1, clusters // 3, clusters // 2, clusters - 2, clusters - 1}:

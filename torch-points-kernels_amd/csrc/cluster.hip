@@ -1110,8 +1110,11 @@ extern "C" size_t tpk_grow_components_workspace_bytes(int64_t n)
     return l.total;
 }
 
-extern "C" int tpk_grow_components(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, int64_t* found,
-                                   void* workspace, size_t workspace_bytes, void* stream)
+namespace {
+
+// largest_first: see tpk_grow_components_by_size.
+int grow_components(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, bool largest_first, int64_t* found,
+                    void* workspace, size_t workspace_bytes, void* stream)
 {
     if (n <= 0 || nsample <= 0 || !found || !neighbours)
         return TPK_ERR_INVALID_ARG;
@@ -1162,11 +1165,25 @@ extern "C" int tpk_grow_components(int64_t n, int nsample, const int64_t* neighb
     e = static_cast<hipError_t>(tpk_read_back(found, info, 24, s));
     if (e != hipSuccess || found[0] == 0)
         return (int)e;
-    if (found[0] > 1 && found[0] <= CL_RANKED)
+    if (largest_first && found[0] > 1 && found[0] <= CL_RANKED)
         component_rank_kernel<<<1, CL_RANKED, 0, s>>>((int)found[0], reinterpret_cast<const int*>(ws + l.seeds), number, starts);
     e = sort_points(ni, (unsigned)found[0] + 1u, ClusterKeys{(int)found[0], root, number},
                     SortSpace{keys_in, keys_out, values_in, values_out, ws + l.temp, l.temp_bytes}, s);
     return e != hipSuccess ? (int)e : tpk_launch_status();
+}
+
+} // namespace
+
+extern "C" int tpk_grow_components(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, int64_t* found,
+                                   void* workspace, size_t workspace_bytes, void* stream)
+{
+    return grow_components(n, nsample, neighbours, min_cluster_size, false, found, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tpk_grow_components_by_size(int64_t n, int nsample, const int64_t* neighbours, int64_t min_cluster_size, int64_t* found,
+                                           void* workspace, size_t workspace_bytes, void* stream)
+{
+    return grow_components(n, nsample, neighbours, min_cluster_size, true, found, workspace, workspace_bytes, stream);
 }
 
 extern "C" int tpk_grow_rows_part(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, int64_t first,
@@ -1199,11 +1216,10 @@ extern "C" int tpk_grow_rows_part(int64_t n, int nsample, const int64_t* neighbo
     return tpk_launch_status();
 }
 
-extern "C" int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, void* rows,
-                             int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes, void* stream)
+extern "C" int tpk_grow_places(int64_t n, const int64_t* found, int32_t* positions, int64_t* starts, void* workspace,
+                               size_t workspace_bytes, void* stream)
 {
-    if (n <= 0 || n > CL_MAX_POINTS || nsample <= 0 || !neighbours || !found || !positions || !starts || found[0] < 1 ||
-        found[1] < found[0] || found[1] > n || (entry_bytes != 2 && entry_bytes != 4) || (entry_bytes == 2 && found[2] > 65536))
+    if (n <= 0 || n > CL_MAX_POINTS || !found || !positions || !starts || found[0] < 1 || found[1] < found[0] || found[1] > n)
         return TPK_ERR_INVALID_ARG;
     ComponentLayout l;
     if (!component_layout(n, &l))
@@ -1216,9 +1232,18 @@ extern "C" int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, 
     component_places_kernel<<<(unsigned)tpk_ceil_div((int64_t)count + 1, CL_THREADS), CL_THREADS, 0, tpk_stream(stream)>>>(
         count, reinterpret_cast<const unsigned*>(ws + l.values_out), place, positions, (int)found[0], reinterpret_cast<const int64_t*>(ws + l.starts),
         starts);
-    const int status = tpk_launch_status();
-    return status != TPK_OK || !rows ? status
-                                     : tpk_grow_rows_part(n, nsample, neighbours, found, entry_bytes, 0, count, rows, workspace, workspace_bytes, stream);
+    return tpk_launch_status();
+}
+
+extern "C" int tpk_grow_rows(int64_t n, int nsample, const int64_t* neighbours, const int64_t* found, int entry_bytes, void* rows,
+                             int32_t* positions, int64_t* starts, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (nsample <= 0 || !neighbours || !found || !rows || (entry_bytes != 2 && entry_bytes != 4) || (entry_bytes == 2 && found[2] > 65536))
+        return TPK_ERR_INVALID_ARG;
+    const int status = tpk_grow_places(n, found, positions, starts, workspace, workspace_bytes, stream);
+    return status != TPK_OK
+               ? status
+               : tpk_grow_rows_part(n, nsample, neighbours, found, entry_bytes, 0, found[1], rows, workspace, workspace_bytes, stream);
 }
 
 extern "C" size_t tpk_region_order_workspace_bytes(int64_t n)

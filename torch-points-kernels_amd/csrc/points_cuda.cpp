@@ -298,8 +298,8 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     TORCH_CHECK(ws_bytes > 0, "grow_proximity: too many points");
     at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes)}, bytes_on_device);
     int64_t found[3] = {0, 0, 0};
-    check_status(tpk_grow_components(n, nsample, neighbours.data_ptr<int64_t>(), min_cluster_size, found, ws.data_ptr(), ws_bytes,
-                                     stream),
+    check_status(tpk_grow_components_by_size(n, nsample, neighbours.data_ptr<int64_t>(), min_cluster_size, found, ws.data_ptr(), ws_bytes,
+                                             stream),
                  "grow_proximity (components)");
     const int64_t pieces = found[0], points = found[1];
     if (pieces == 0)
@@ -316,12 +316,17 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     const int32_t* positions = reinterpret_cast<const int32_t*>(h + at_positions);
     at::Tensor staged = at::empty({at_rows + (at_once ? 0 : points * row_bytes)}, bytes_on_device);
     uint8_t* d = staged.data_ptr<uint8_t>();
+    int32_t* positions_out = reinterpret_cast<int32_t*>(d + at_positions);
     if (at_once)
+    {
         writes.begin();
-    check_status(tpk_grow_rows(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), at_once ? nullptr : d + at_rows,
-                               reinterpret_cast<int32_t*>(d + at_positions), reinterpret_cast<int64_t*>(at_once ? h : d), ws.data_ptr(),
-                               ws_bytes, stream),
-                 "grow_proximity (rows)");
+        check_status(tpk_grow_places(n, found, positions_out, reinterpret_cast<int64_t*>(h), ws.data_ptr(), ws_bytes, stream),
+                     "grow_proximity (places)");
+    }
+    else
+        check_status(tpk_grow_rows(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), d + at_rows, positions_out,
+                                   reinterpret_cast<int64_t*>(d), ws.data_ptr(), ws_bytes, stream),
+                     "grow_proximity (rows)");
     // What the walk leaves: the clusters' members as entries, then a table of the clusters.  (From the pool: fresh memory would cost a page fault
     // per 4 KiB.)
     const int64_t at_table = (points * entry + 7) / 8 * 8, most_clusters = points / std::max<int64_t>(min_cluster_size, 1);
