@@ -10,6 +10,7 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "torch-points-kernels_amd", "csrc")
 
 SHIM = r"""
+#include "arrivals.h"
 #include "ball_table.h"
 #include "bracket.h"
 #include "cloud_ids.h"
@@ -18,7 +19,56 @@ SHIM = r"""
 #include "grow_table.h"
 #include "grow_walk.h"
 #include <cmath>
+#include <atomic>
+#include <chrono>
+#include <ctime>
 #include <stdexcept>
+#include <thread>
+
+// `threads` wait for parts that come `apart` seconds after each other; fails: the event that throws, -1 for none.  Returns the
+// processor time the process took meanwhile; *right: how many threads got what they waited for, in time.
+extern "C" double parts_waited_for(int threads, int parts, double apart, int fails, int* right)
+{
+    using Clock = std::chrono::steady_clock;
+    struct Event
+    {
+        Clock::time_point at;
+        bool throws;
+        void synchronize()
+        {
+            std::this_thread::sleep_until(at);
+            if (throws)
+                throw std::runtime_error("event");
+        }
+    };
+    const auto start = Clock::now();
+    auto when = [&](int part) { return start + std::chrono::duration_cast<Clock::duration>(std::chrono::duration<double>(apart * (part + 1))); };
+    Arrivals<Event> arrivals;
+    for (int p = 0; p < parts; ++p)
+        arrivals.part(10 * (p + 1), Event{when(p), p == fails});
+    const std::clock_t before = std::clock();
+    std::atomic<int> good{0};
+    std::vector<std::thread> all;
+    for (int t = 0; t < threads; ++t)
+        all.emplace_back([&, t] {
+            const int part = t % parts;
+            const bool there = arrivals.wait(10 * part + 1 + t % 10);
+            good += (there ? Clock::now() >= when(part) && (fails < 0 || part < fails) : fails >= 0 && part >= fails) ? 1 : 0;
+        });
+    for (auto& t : all)
+        t.join();
+    *right = good;
+    try
+    {
+        arrivals.rethrow();
+        *right = fails < 0 ? *right : -1;
+    }
+    catch (const std::runtime_error&)
+    {
+        *right = fails < 0 ? -1 : *right;
+    }
+    return static_cast<double>(std::clock() - before) / CLOCKS_PER_SEC;
+}
 
 // What happened to a block that the device was writing into when something was thrown, or not: 'w' the device was waited for, 'r' the
 // block went.
@@ -150,7 +200,7 @@ def shim(tmp_path_factory):
     source, library = str(folder / "shim.cpp"), str(folder / "shim.so")
     with open(source, "w") as f:
         f.write(SHIM)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-Wall", "-Werror", "-shared", "-fPIC", "-I" + CSRC, source, "-o", library],
+    subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-Wall", "-Werror", "-shared", "-fPIC", "-pthread", "-I" + CSRC, source, "-o", library],
                    check=True)
     return ctypes.CDLL(library)
 
@@ -277,6 +327,18 @@ def test_a_block_goes_after_the_device_is_done_with_it(shim):
     order = [body.index(s) for s in ("at::Tensor host =", "PendingWrites<decltype(wait)> writes(wait)", "writes.begin()", "tpk_grow_places(",
                                      "tpk_grow_rows_part(", "arrivals.wait(points + 1)", "writes.end()")]
     assert order == sorted(order)
+
+
+@pytest.mark.parametrize("threads,parts,fails", [(1, 1, -1), (8, 5, -1), (16, 2, -1), (8, 5, 0), (8, 5, 3)])
+def test_threads_sleep_until_their_part_is_there(shim, threads, parts, fails):
+    """All threads get their part no sooner than it comes, or the error, and take no processor time while they wait (half of
+    one processor would do for a thread that asks for it again and again)."""
+    shim.parts_waited_for.restype = ctypes.c_double
+    shim.parts_waited_for.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.c_int, ctypes.c_void_p]
+    right, apart = ctypes.c_int(), 0.1
+    spent = shim.parts_waited_for(threads, parts, apart, fails, ctypes.addressof(right))
+    assert right.value == threads
+    assert spent < 0.5 * apart
 
 
 @pytest.mark.parametrize("clusters", [1, 2, 3, 1000, 715827883, 715827884, 2 ** 30])

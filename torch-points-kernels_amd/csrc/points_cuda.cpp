@@ -13,14 +13,12 @@
 
 #include <algorithm>
 #include <atomic>
-#include <exception>
-#include <mutex>
-#include <thread>
 #include <tuple>
 #include <utility>
 #include <vector>
 
 #include "../../include/tpk.h"
+#include "arrivals.h"
 #include "grow_walk.h"
 
 namespace {
@@ -182,69 +180,11 @@ at::Tensor host_bytes(int64_t bytes, int64_t most)
     return at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(bytes <= most));
 }
 
-// What the device writes into host memory in parts, each followed by an event.  Threads that need what lies before some place wait for
-// the part that holds it: one of them for the event, the others for that one.
-class Arrivals
-{
-public:
-    explicit Arrivals(const at::Tensor& on) : device_(on.get_device()) {}
-    // All before `end` is there when the work enqueued so far is done.
-    void part(int64_t end)
-    {
-        ends_.push_back(end);
-        events_.emplace_back(c10::DeviceType::CUDA);
-        events_.back().record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device_).unwrap());
-    }
-    // Waits for all before `end`.  False: a wait failed, here or in another thread (rethrow() has the error).
-    bool wait(int64_t end)
-    {
-        while (there_.load(std::memory_order_acquire) < end)
-        {
-            if (failed_.load(std::memory_order_acquire))
-                return false;
-            std::unique_lock<std::mutex> lock(turn_, std::try_to_lock);
-            if (!lock.owns_lock())
-            {
-                std::this_thread::yield();
-                continue;
-            }
-            if (there_.load(std::memory_order_relaxed) >= end || failed_.load(std::memory_order_relaxed))
-                continue;
-            try
-            {
-                events_.at(next_).synchronize();
-                there_.store(ends_[next_++], std::memory_order_release);
-            }
-            catch (...)
-            {
-                error_ = std::current_exception();
-                failed_.store(true, std::memory_order_release);
-            }
-        }
-        return true;
-    }
-    void rethrow()
-    {
-        if (error_)
-            std::rethrow_exception(error_);
-    }
-
-private:
-    const c10::DeviceIndex device_;
-    std::vector<c10::Event> events_;
-    std::vector<int64_t> ends_;
-    size_t next_ = 0;
-    std::atomic<int64_t> there_{0};
-    std::atomic<bool> failed_{false};
-    std::exception_ptr error_;
-    std::mutex turn_;
-};
-
 // Walks the pieces begin .. end on host threads; rows: theirs, from the place starts[begin] on.  arrivals: the rows are still being
 // written, in the order of places (nullptr: they are there).  Adds to `all`.
 template <typename E>
 void walk_pieces(const E* rows, int nsample, const int64_t* starts, int64_t begin, int64_t end, int64_t min_cluster_size, E* entries,
-                 std::vector<grow_walk::Cluster>* all, Arrivals* arrivals)
+                 std::vector<grow_walk::Cluster>* all, Arrivals<c10::Event>* arrivals)
 {
     const int64_t pieces = end - begin, points = starts[end] - starts[begin];
     std::vector<int64_t> turn(static_cast<size_t>(pieces));
@@ -333,7 +273,7 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     at::Tensor walked = host_bytes(at_table + most_clusters * 24, most);
     uint8_t* entries = walked.data_ptr<uint8_t>();
     std::vector<grow_walk::Cluster> all;
-    auto walk = [&](const uint8_t* rows, int64_t begin, int64_t end, Arrivals* arrivals) {
+    auto walk = [&](const uint8_t* rows, int64_t begin, int64_t end, Arrivals<c10::Event>* arrivals) {
         if (entry == 2)
             walk_pieces(reinterpret_cast<const uint16_t*>(rows), nsample, starts, begin, end, min_cluster_size, reinterpret_cast<uint16_t*>(entries), &all,
                         arrivals);
@@ -344,7 +284,12 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
     if (at_once)
     {
         // The largest pieces lie first, so their walks, which end last, begin while the others' rows are being written.
-        Arrivals arrivals(neighbours);
+        Arrivals<c10::Event> arrivals;
+        auto event = [&] { // happens when the work enqueued so far is done
+            c10::Event e(c10::DeviceType::CUDA);
+            e.record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(neighbours.get_device()).unwrap());
+            return e;
+        };
         const int64_t part = std::max(grow_walk::LEAST_PART / row_bytes, points / grow_walk::PARTS) + 1;
         for (int64_t first = 0, count; first < points; first += count)
         {
@@ -352,11 +297,11 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
             check_status(tpk_grow_rows_part(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), first, count, h + at_rows,
                                             ws.data_ptr(), ws_bytes, stream),
                          "grow_proximity (rows)");
-            arrivals.part(first + count);
+            arrivals.part(first + count, event());
         }
         const int64_t bytes = points * 4;
         host.narrow(0, at_positions, bytes).copy_(staged.narrow(0, at_positions, bytes), /*non_blocking=*/true);
-        arrivals.part(points + 1);
+        arrivals.part(points + 1, event());
         if (arrivals.wait(1))
             walk(h + at_rows, 0, pieces, &arrivals);
         arrivals.wait(points + 1);
