@@ -109,7 +109,8 @@ inline const uint64_t* exchange(uint64_t value)
     ++steps;
     if (++wave.arrived == wave.live)
     {
-        memcpy(wave.seen[turn & 1], wave.offered, sizeof wave.offered);
+        for (int i = 0; i < WAVE; ++i) // (lanes that have ended by now offer nothing; others may end before all have looked)
+            wave.seen[turn & 1][i] = fibres[now / WAVE * WAVE + i].done ? 0 : wave.offered[i];
         wave.arrived = 0;
         ++wave.turn;
     }
@@ -212,7 +213,7 @@ inline unsigned long long __ballot(bool p)
     const uint64_t* all = emulation::exchange(p);
     unsigned long long mask = 0;
     for (int i = 0; i < emulation::WAVE; ++i)
-        mask |= all[i] != 0 && !emulation::fibres[emulation::now / 64 * 64 + i].done ? 1ull << i : 0ull;
+        mask |= all[i] != 0 ? 1ull << i : 0ull;
     return mask;
 }
 template <typename T>
@@ -239,6 +240,17 @@ inline int __builtin_amdgcn_readlane(int v, int from)
 }
 inline int __builtin_amdgcn_readfirstlane(int v) { return emulation::exchanged(v, 0); }
 inline int __builtin_amdgcn_ds_bpermute(int address, int v) { return emulation::exchanged(v, address >> 2 & 63); }
+// (of the instruction's modes the one that masks the lane's number within its half of the wavefront)
+#define __builtin_amdgcn_ds_swizzle(v, pattern) emulation::swizzled(v, pattern)
+namespace emulation {
+inline int swizzled(int v, int pattern)
+{
+    if (pattern & 0x8000)
+        fail("a swizzle that is not emulated");
+    const int in_half = lane() % 32;
+    return exchanged(v, lane() - in_half + (((in_half & (pattern & 31)) | (pattern >> 5 & 31)) ^ (pattern >> 10 & 31)));
+}
+}
 inline int __builtin_amdgcn_update_dpp(int old, int v, int control, int rows, int banks, bool zero)
 {
     const int lane = emulation::lane(), row = lane / 16, in_row = lane % 16, by = control & 15;
@@ -280,11 +292,23 @@ inline unsigned __builtin_amdgcn_mbcnt_hi(unsigned mask, unsigned add)
     const int lane = emulation::lane() - 32;
     return add + __builtin_popcount(lane <= 0 ? 0u : mask & ((1u << lane) - 1u));
 }
+namespace emulation {
+inline const char *watched_begin, *watched_end; // atomics in here are counted
+inline long watched;
+}
 template <typename T, typename U>
 inline T atomicAdd(T* p, U v)
 {
+    const char* const at = reinterpret_cast<const char*>(p);
+    emulation::watched += at >= emulation::watched_begin && at < emulation::watched_end ? 1 : 0;
     const T old = *p;
     *p += v;
+    return old;
+}
+inline unsigned atomicCAS(unsigned* p, unsigned compare, unsigned v)
+{
+    const unsigned old = *p;
+    *p = old == compare ? v : old;
     return old;
 }
 inline int atomicMin(int* p, int v)

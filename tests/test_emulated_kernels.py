@@ -11,25 +11,33 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(ROOT, "torch-points-kernels_amd", "csrc")
 
 
-@pytest.fixture(scope="module")
-def ball_query_dense(tmp_path_factory):
-    folder = str(tmp_path_factory.mktemp("emulated"))
-    for name in os.listdir(CSRC):
-        if not name.endswith(".h") and name != "nn_grid.hip":
+def _emulated(folder, unit, name):
+    for source_name in os.listdir(CSRC):
+        if not source_name.endswith(".h") and source_name != unit + ".hip":
             continue
-        with open(os.path.join(CSRC, name)) as f:
+        with open(os.path.join(CSRC, source_name)) as f:
             source = f.read()
         # dynamic LDS is a pointer into the emulated one, the one instruction written by hand an assignment
         source = re.sub(r"extern __shared__ (?:__align__\(16\) )?([a-z0-9 ]+?) ([a-z_]+)\[\];", r"\1* const \2 = reinterpret_cast<\1*>(emulation::lds);", source)
         source = source.replace('asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "s"(uniform_value));', "v = uniform_value;")
         source = source.replace('"../../include/tpk.h"', '"%s"' % os.path.join(ROOT, "include", "tpk.h"))
-        with open(os.path.join(folder, name.replace(".hip", ".cpp")), "w") as f:
+        with open(os.path.join(folder, source_name.replace(".hip", ".cpp")), "w") as f:
             f.write(source)
-    program = os.path.join(folder, "ball_query_dense")
+    program = os.path.join(folder, name)
     subprocess.run(["g++", "-std=c++17", "-O2", "-w", "-fpermissive", "-ffp-contract=off", "-U_FORTIFY_SOURCE", "-fsanitize=bounds",
                     "-fno-sanitize-recover=bounds", "-I" + folder, "-I" + os.path.join(HERE, "emulation"),
-                    os.path.join(HERE, "emulation", "ball_query_dense.cpp"), "-o", program], check=True)
+                    os.path.join(HERE, "emulation", name + ".cpp"), "-o", program], check=True)
     return program
+
+
+@pytest.fixture(scope="module")
+def ball_query_dense(tmp_path_factory):
+    return _emulated(str(tmp_path_factory.mktemp("emulated")), "nn_grid", "ball_query_dense")
+
+
+@pytest.fixture(scope="module")
+def ball_query_packed(tmp_path_factory):
+    return _emulated(str(tmp_path_factory.mktemp("emulated")), "ball_table", "ball_query_packed")
 
 
 # (clouds of 9373 points: windows of 8192 that hold parts of two clouds, the last of 75 points, whose second part is empty; the first
@@ -39,3 +47,15 @@ def test_dense_ball_query_stays_in_bounds(ball_query_dense, clouds, points, quer
     done = subprocess.run([ball_query_dense] + [str(v) for v in (clouds, points, queries, nsample, radius, own)], capture_output=True,
                           text=True, timeout=300)
     assert done.returncode == 0, done.stdout + done.stderr
+
+
+# (radius 2: all points of a cloud in a few buckets; 0.02: hardly two in one; 12291 points: the last workgroup counts three)
+@pytest.mark.parametrize("clouds,points,queries,nsample,radius,sort", [(1, 12291, 8192, 16, 2.0, 0), (3, 8200, 8195, 5, 0.3, 0), (1, 9000, 8192, 16, 0.02, 0),
+                                                                       (2, 8192, 700, 64, 0.2, 1)])
+def test_packed_ball_query_counts_with_few_atomics(ball_query_packed, clouds, points, queries, nsample, radius, sort):
+    """In bounds and right; and however many points a bucket holds, 1024 consecutive ones that lie in it share one atomic (atomics on
+    one address wait for each other: an atomic per point took 550 us where a ball held a cloud of 100000)."""
+    done = subprocess.run([ball_query_packed] + [str(v) for v in (clouds, points, queries, nsample, radius, sort)], capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stdout + done.stderr
+    wrong, atomics, buckets, by_1024, chunks = (int(v) for v in re.findall(r"(\d+) (?:wrong|atomics|buckets|by 1024|chunks)", done.stdout))
+    assert wrong == 0 and atomics <= by_1024 + chunks

@@ -97,7 +97,7 @@ def build_extension(force=False):
 
     src = os.path.join(CSRC, "points_cuda.cpp")
     out = os.path.join(PKG, "points_cuda.so")
-    deps = [src, os.path.join(INCLUDE, "tpk.h")] + [os.path.join(CSRC, h) for h in ("differentiable.h", "grow_walk.h")]
+    deps = [src, os.path.join(INCLUDE, "tpk.h")] + [os.path.join(CSRC, h) for h in ("arrivals.h", "differentiable.h", "grow_walk.h")]
     if not force and _newer(out, deps):
         return out
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
