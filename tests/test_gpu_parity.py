@@ -1026,6 +1026,60 @@ def test_ball_query_packed_long_bins(tpk, oracle, dev, rest, sort):
     np.testing.assert_array_equal(_np(dist), wd)
 
 
+# (radius 1e25: every query is scanned for, of clouds of 1 .. 7 points up to four clouds' queries by a wavefront; 0.4 and 0.25 in a cube
+# of 1: queries with hundreds to thousands of candidates, some of which are scanned for and some walked; 0.08: walked)
+@pytest.mark.parametrize("radius,nsample", [(1e25, 3), (1e25, 8), (0.4, 1), (0.4, 16), (0.4, 65), (0.4, 300), (0.25, 16), (0.25, 64), (0.08, 20)])
+@pytest.mark.parametrize("sizes", ["small", "one", "three"])
+def test_ball_query_packed_scans_of_several_queries(tpk, oracle, dev, sizes, radius, nsample):
+    g = torch.Generator().manual_seed(nsample)
+    n = {"small": torch.randint(1, 8, (2300,), generator=g), "one": torch.tensor([8195]), "three": torch.tensor([4097, 70, 4033])}[sizes]
+    b = torch.arange(n.numel()).repeat_interleave(n)
+    x = torch.rand(b.numel(), 3, generator=g)
+    flat = torch.rand(b.numel(), generator=g) < 0.7  # most points on planes: queries beside them touch crowded cells
+    x[flat, 0] = 0.2 + 0.6 * (x[flat, 1] > 0.5)
+    y = (x + 0.2 * (torch.rand(x.shape, generator=g) < 0.2)).contiguous()
+    idx, dist = tpk.ball_query(radius, nsample, x.to(dev), y.to(dev), mode="partial_dense", batch_x=b.to(dev), batch_y=b.to(dev))
+    wi, wd = oracle.ball_query_partial_dense(radius, nsample, x.numpy(), y.numpy(), b.numpy(), b.numpy())
+    np.testing.assert_array_equal(_np(idx), wi)
+    np.testing.assert_array_equal(_np(dist), wd)
+
+
+@pytest.mark.parametrize("radius", [2.0, 6.0])
+def test_ball_query_packed_of_large_balls_is_not_left_behind(dev, radius):
+    """Balls that hold a large part of their cloud: the call over the table takes about as long as the one over bins in the smaller
+    workspace (1.0 times; an atomic per point and one scan after the other took 5 and 24 times as long)."""
+    import ctypes
+    import os
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip.so"))
+    P, L = lambda t: ctypes.c_void_p(t.data_ptr()), ctypes.c_int64
+    g = torch.Generator().manual_seed(1)
+    x = 8.0 * torch.rand(100000, 3, generator=g)
+    x[:80000, 0] = 1.0 + 6.0 * (x[:80000, 1] > 4.0)
+    x = x[torch.randperm(100000, generator=g)].to(dev)
+    y = x[:12500].contiguous()
+    b = torch.zeros(100000, dtype=torch.int64, device=dev)
+    idx, dist = torch.empty(12500, 16, dtype=torch.int64, device=dev), torch.empty(12500, 16, device=dev)
+    took = []
+    for size in (lib.tpk_ball_query_partial_workspace_bytes, lib.tpk_ball_query_partial_table_workspace_bytes):
+        size.restype = ctypes.c_size_t
+        nbytes = size(L(100000), L(12500), 16)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        times = []
+        for _ in range(20):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(4):
+                assert lib.tpk_ball_query_partial_f32(L(100000), L(12500), ctypes.c_float(radius), 16, P(x), P(y), P(b), P(b), P(idx), P(dist), P(ws),
+                                                      ctypes.c_size_t(nbytes), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        took.append(min(times))
+    assert took[1] < 2.5 * took[0], took
+
+
 @pytest.mark.parametrize("name", ["interpolate", "group", "chamfer", "gridding", "cubic"])
 def test_traces_follow_their_inputs(tpk, dev, name):
     # a trace made with one input computes with the next one's values, as a call does

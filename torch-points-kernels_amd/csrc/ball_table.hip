@@ -11,15 +11,20 @@
 // over the 16 give the query's candidates, which are tested 16 at a time.  Hits are collected in LDS and ranked by row,
 // which is the order a serial scan in index order that stops after nsample hits (cuda/src/ball_query_gpu.cu:54-95) meets them in.
 // A query with more than 128 keeps the nsample lowest rows and goes on.  Where that scan itself is likely to end sooner than the
-// walk - dense neighbourhoods -, or the query has more candidates than its cloud has rows, the wavefront scans.
+// walk - dense neighbourhoods -, or the query has more candidates than its cloud has rows, the wavefront scans, for all such queries of
+// a cloud among its four at once.
 //
 // Measured against the walk over bins of windows (nn_grid.hip: windows of consecutive rows, each of which a query has to look
-// into), whole calls: 53000 queries of four scenes of 20000 .. 100000 points 50 -> 42 us (15 of them the queries, 37
+// into), whole calls, us: 53000 queries of four scenes of 20000 .. 100000 points 50 -> 42 (15 of them the queries, 37
 // before; clearing 3, counting 13, places 4, records 7, against 17 for the windows' ordering), all 212000 of their points as queries 117 ->
 // 61 (nsample 16, radius 0.04), 138 -> 75 (64, 0.1), 2300 -> 272 (64, 0.3: 60 points in a ball of a plane, which the walk over bins
-// left to the scan); 300000 queries of 24 clouds 257 -> 133.  An eighth of the points as queries: 38 -> 40 and 42 -> 40; 20000 points and
-// 3000 queries 21 -> 17 .. 22.  Slower where a ball holds a large part of its cloud and every query is scanned for: four scans per
-// wavefront are one after the other (radius 1 in rooms of 8: 12500 queries 150 -> 209, 100000 417 -> 448).
+// left to the scan); 300000 queries of 24 clouds 257 -> 133.  By radius in rooms of 8, nsample 16 / 64:
+//     radius                        0.1                 0.3                   0.6                1                   1.4                2
+//     53000 of 4 clouds, 212000     58 / 59 -> 43 / 46  175 / 402 -> 86 / 92  327 / 678 -> 194 / 311  141 / 393 -> 142 / 331  71 / 182 -> 80 / 217  45 / 101 -> 46 / 93
+//     12500 of 1 cloud, 100000      33 / 34 -> 29 / 31  136 / 375 -> 59 / 74  147 / 310 -> 133 / 198  57 / 184 -> 106 / 227   35 / 77 -> 39 / 148   27 / 46 -> 29 / 48
+//     50000 of 1 cloud, 100000      57 / 58 -> 36 / 38  335 / 1035 -> 101 / 113  289 / 749 -> 211 / 378  112 / 367 -> 138 / 341  62 / 174 -> 60 / 223  44 / 97 -> 42 / 84
+// Still slower are balls of thousands of points, a hundredth of their cloud or more, whose queries are few: a wavefront that serves four
+// waits for the longest of their walks and then of their scans, on a chip that 3125 wavefronts do not fill.
 // What bounds it: the counting its atomics, the queries instruction issue - 690 vector instructions per wavefront, 170 per query
 // with 16 hits each, of 1700 clocks a query before.
 // Sorted neighbours (calls against the walk over bins that merged a sorted list, us): 212000 queries of the four scenes 188 -> 69 (16 slots, radius
@@ -42,6 +47,7 @@ constexpr int BT_QUERIES = TPK_WAVE / BT_GROUP;    // queries per wavefront
 constexpr int BT_HITS = 2 * TPK_WAVE;              // hits a query holds when a step begins
 constexpr int BT_KEPT = TPK_WAVE;                  // slots of a call whose queries may keep their lowest rows when they hold more
 constexpr int BT_LONG = 8 * BT_HITS;               // candidates from which on a query may be scanned for at once
+constexpr int BT_SAMPLES = 2;                      // of such a query's candidates, per lane, that tell how many of them lie in the ball
 constexpr int BT_HIT_STRIDE = BT_HITS + BT_GROUP + 2; // (the four queries of a wavefront read theirs at the same time: other banks)
 constexpr int BT_COUNT_THREADS = 1024;
 constexpr int BT_COUNT_SLOTS = 2 * BT_COUNT_THREADS; // of the table in LDS: every point of the workgroup may need one
@@ -300,13 +306,81 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// Whether a scan of the cloud in index order is likely to take fewer instructions than a walk over `candidates` more, for a query with
-// about `hits` hits.  The scan meets nsample of them within rows * nsample / hits rows, 64 a step of 25 instructions; a step of the
-// walk takes 45 for 16 candidates of each of four queries.
-__device__ __forceinline__ bool scan_is_shorter(float rows, float nsample, float hits, float candidates)
+// Whether a scan of the cloud in index order is likely to take less time than a walk over `candidates` more, for a query with
+// about `hits` hits.  The scan meets nsample of them within rows * nsample / hits rows, 64 a step of `per_step` instructions' time; a step
+// of the walk takes 45 instructions for 16 candidates of each of four queries.  A scan's step has about 10 (25 where it holds hits).  What
+// it counts for is fitted to calls of 12500 to 100000 queries with balls of 60 to 10000 points, where it is not instructions alone: before the
+// walk a step of a scan counts 8, since a long walk by 16 lanes waits for one load after the other; after 128 hits, when most of what is
+// left of a walk is short, 25.  (6 / 16: 100000 points in a room of 8, 12500 queries, radius 0.45 / 1 / 1.4: 137 / 99 / 38 us instead
+// of 107 / 106 / 39; 10 / 10: 103 / 116 / 38, and with 64 slots 170 / 234 / 168 instead of 139 / 227 / 148.)
+constexpr float BT_SCAN_STEP = 8.0f, BT_SCAN_STEP_LATER = 25.0f;
+__device__ __forceinline__ bool scan_is_shorter(float rows, float nsample, float hits, float candidates, float per_step)
 {
-    const float scan = fminf(rows, rows * nsample * __builtin_amdgcn_rcpf(hits)) * (25.0f / TPK_WAVE);
+    const float scan = fminf(rows, rows * nsample * __builtin_amdgcn_rcpf(hits)) * (per_step / TPK_WAVE);
     return candidates * (45.0f / (BT_GROUP * BT_QUERIES)) > scan;
+}
+
+// The support rows s0 .. s1 against those of the wavefront's four queries whose first lanes are set in `which`, as ball_scan_rows does
+// for one: a step's rows are loaded once for all of them.
+__device__ __forceinline__ void bt_scan_rows(const float* __restrict__ x, int s0, int s1, unsigned long long which, float qx, float qy, float qz,
+                                             float radius2, int nsample, int lane, int64_t* __restrict__ idx4, float* __restrict__ dist4 TPK_WORK_PARAM)
+{
+    constexpr int BATCH = 4; // loads of four steps in flight (6: 3 % slower; the next four requested ahead: nothing)
+    float x4[BT_QUERIES], y4[BT_QUERIES], z4[BT_QUERIES];
+    int cnt[BT_QUERIES];
+#pragma unroll
+    for (int g = 0; g < BT_QUERIES; ++g)
+    {
+        x4[g] = to_vector_register(tpk_read_lane(qx, g * BT_GROUP));
+        y4[g] = to_vector_register(tpk_read_lane(qy, g * BT_GROUP));
+        z4[g] = to_vector_register(tpk_read_lane(qz, g * BT_GROUP));
+        cnt[g] = which >> (g * BT_GROUP) & 1 ? 0 : nsample;
+    }
+    for (int base = s0; base < s1 && min(min(cnt[0], cnt[1]), min(cnt[2], cnt[3])) < nsample; base += BATCH * TPK_WAVE)
+    {
+        float px[BATCH], py[BATCH], pz[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+        {
+            const int64_t pos = min(base + u * TPK_WAVE + lane, s1 - 1);
+            px[u] = x[pos * 3 + 0];
+            py[u] = x[pos * 3 + 1];
+            pz[u] = x[pos * 3 + 2];
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+        {
+            const int pos = base + u * TPK_WAVE + lane;
+            const unsigned long long rows = __ballot(pos < s1);
+#pragma unroll
+            for (int g = 0; g < BT_QUERIES; ++g)
+            {
+                if (cnt[g] >= nsample)
+                    continue;
+                const float d = tpk_dist2(x4[g], y4[g], z4[g], px[u], py[u], pz[u]);
+                TPK_WORK_ADD(1);
+                const unsigned long long mask = rows & __ballot(d <= radius2);
+                if (mask == 0)
+                    continue; // (most steps of a long scan)
+                const bool hit = mask >> lane & 1;
+                const int slot = cnt[g] + static_cast<int>(tpk_prefix_count(mask));
+                if (hit && slot < nsample)
+                {
+                    idx4[g * nsample + slot] = pos;
+                    dist4[g * nsample + slot] = d;
+                }
+                cnt[g] += __builtin_popcountll(mask);
+            }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < BT_QUERIES; ++g)
+        if (which >> (g * BT_GROUP) & 1)
+            for (int s = cnt[g] + lane; s < nsample; s += TPK_WAVE)
+            {
+                idx4[g * nsample + s] = -1;
+                dist4[g * nsample + s] = -1.0f;
+            }
 }
 
 // SORTED: the nsample (<= 64) NEAREST points with squared distance < radius2, nearest first (equal distances: lower row first), instead
@@ -384,9 +458,7 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
         scan = ((__ballot(crosses) >> group_lane) & 0xffff) != 0;
     const int before = row_exclusive_sum(size);
     int total = row_last(before + size, lane);
-    // (a run of cells holds 5 to 13 times what the ball itself does, on a surface and in space)
-    scan = scan || total > s1 - s0 ||
-           (!SORTED && total > BT_LONG && scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), static_cast<float>(total) * 0.125f, static_cast<float>(total)));
+    scan = scan || total > s1 - s0;
     if (scan)
         total = SORTED ? s1 - s0 : 0;
 
@@ -407,11 +479,46 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
     const bool few = __ballot(crosses || runs > 4) == 0;
     const int second_at = row_lane<1>(before), third_at = row_lane<2>(before), fourth_at = row_lane<3>(before);
     const int o0 = row_lane<0>(origin), o1 = row_lane<1>(origin), o2 = row_lane<2>(origin), o3 = row_lane<3>(origin);
+    auto of_few = [&](int c) __attribute__((always_inline)) { return c + (c < third_at ? (c < second_at ? o0 : o1) : (c < fourth_at ? o2 : o3)); };
+    if constexpr (!SORTED)
+    {
+        // A run of cells holds 5 to 13 times what the ball itself does, on a surface and in space, but a query beside a surface whose
+        // cells it touches may have a hundredth: of long runs a few candidates at equal distances tell.  (Always an eighth: 12500
+        // queries of 100000 points, radius 0.6, 177 us instead of 133.)
+        const bool asks = total > BT_LONG;
+        if (__ballot(asks) != 0)
+        {
+            int in = 0;
+            if (few)
+            {
+                float4 p[BT_SAMPLES];
+                const int apart = total / (BT_SAMPLES * BT_GROUP);
+#pragma unroll
+                for (int j = 0; j < BT_SAMPLES; ++j)
+                    p[j] = record_at(asks ? of_few(apart * (j * BT_GROUP + sub)) : 0);
+#pragma unroll
+                for (int j = 0; j < BT_SAMPLES; ++j)
+                {
+                    const unsigned long long all = __ballot(tpk_dist2(qx, qy, qz, p[j].x, p[j].y, p[j].z) <= radius2);
+                    TPK_WORK_ADD(asks ? 1 : 0);
+                    in += __builtin_popcount(static_cast<unsigned>(all) & group_low) + __builtin_popcount(static_cast<unsigned>(all >> 32) & group_high);
+                }
+            }
+            const float share = few ? fmaxf(static_cast<float>(in), 0.5f) * (1.0f / (BT_SAMPLES * BT_GROUP)) : 0.125f;
+            const float candidates = static_cast<float>(total);
+            if (asks && scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), candidates * share, candidates, BT_SCAN_STEP))
+            {
+                scan = true;
+                total = 0;
+            }
+            most_total = bt_most(total);
+        }
+    }
     auto fetch = [&](int c0) __attribute__((always_inline)) {
         const int c = c0 + sub;
         int at = c;
         if (few)
-            at += c < third_at ? (c < second_at ? o0 : o1) : (c < fourth_at ? o2 : o3);
+            at = of_few(c);
         else
         {
             // Whose candidate is c?  Every run's lane marks the slot of its first candidate of this step with its own
@@ -468,7 +575,7 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
         {
             const float tested = static_cast<float>(min(c0, total)), left = static_cast<float>(total) - tested;
             const float ball = static_cast<float>(cnt) * static_cast<float>(total) * __builtin_amdgcn_rcpf(tested);
-            scan = nsample > BT_KEPT || scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), ball, left);
+            scan = nsample > BT_KEPT || scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), ball, left, BT_SCAN_STEP_LATER);
             total = scan ? 0 : total;
             cnt = scan ? 0 : cnt;
         }
@@ -503,16 +610,15 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
             dist4[out] = found ? __int_as_float(hit.y) : -1.0f;
         }
 
-    // The queries that were given up, one after the other by the whole wavefront.
+    // The queries that were given up, those of one cloud together.
     unsigned long long left = __ballot(!SORTED && real && scan && sub == 0);
     while (left != 0)
     {
         const int from = __builtin_ctzll(left);
-        left &= left - 1;
-        const int64_t out = static_cast<int64_t>(from / BT_GROUP) * nsample;
-        ball_scan_rows<false>(x, tpk_read_lane(s0, from), tpk_read_lane(s1, from), to_vector_register(tpk_read_lane(qx, from)),
-                              to_vector_register(tpk_read_lane(qy, from)), to_vector_register(tpk_read_lane(qz, from)), radius2, nsample,
-                              lane, idx4 + out, dist4 + out TPK_WORK_ARG);
+        const int first = tpk_read_lane(s0, from), end = tpk_read_lane(s1, from);
+        const unsigned long long with = left & __ballot(s0 == first && s1 == end);
+        left &= ~with;
+        bt_scan_rows(x, first, end, with, qx, qy, qz, radius2, nsample, lane, idx4, dist4 TPK_WORK_ARG);
     }
     TPK_WORK_FLUSH
 }
