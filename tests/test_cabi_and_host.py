@@ -44,6 +44,21 @@ def test_knn_grid_workspace_is_its_own_size():
     assert size(1, 8192, 16385) >= 8192 * 16 and size(2, 200000, 1000) >= 2 * 200000 * 16
 
 
+def test_sorted_packed_ball_query_builds_no_table_for_few_queries():
+    """A few queries of a large array walk over bins, whose workspace has no table of 2 .. 4 buckets per point (with one, 16 queries of a
+    million points took 111 us instead of 41); many, and all of a small array, take the table."""
+    lib = ctypes.CDLL(LIB)
+    sizes = [lib.tpk_ball_query_sorted_partial_workspace_bytes, lib.tpk_ball_query_partial_workspace_bytes, lib.tpk_ball_query_partial_table_workspace_bytes]
+    for size in sizes:
+        size.restype = ctypes.c_size_t
+    L = ctypes.c_int64
+    for n, m, table in ((1000000, 16, False), (1000000, 15624, False), (1000000, 15625, True), (1000000, 1000000, True), (65536, 1023, False), (65536, 1024, True),
+                        (65535, 1, True), (8192, 1, True)):
+        got, bins, with_table = sizes[0](L(n), L(m)), sizes[1](L(n), L(m), 64), sizes[2](L(n), L(m), 64)
+        assert bins < with_table
+        assert (got >= with_table) == table and got >= bins, (n, m)
+
+
 def test_counting_build_exports_the_same_abi_plus_its_reader():
     """libtpk_hip_counting.so (measurement only) carries the whole C ABI and tpk_work_read_reset; the
     shipping library carries no counter."""

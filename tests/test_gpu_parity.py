@@ -1044,6 +1044,22 @@ def test_ball_query_packed_scans_of_several_queries(tpk, oracle, dev, sizes, rad
     np.testing.assert_array_equal(_np(dist), wd)
 
 
+# (a few queries of 65536 points or more walk over bins: radius 0.03 a few bins, 0.3 more than 64 of a window, 1e25 every point; equal points)
+@pytest.mark.parametrize("radius,nsample", [(0.03, 64), (0.1, 16), (0.3, 1), (0.3, 33), (1e25, 5), (0.0, 4)])
+@pytest.mark.parametrize("sizes,queries", [([65536], 1), ([30000, 200, 40001], 500), ([70000], 1093), ([66000], 1031), ([66000], 1032)])
+def test_ball_query_packed_sorted_for_few_queries(tpk, oracle, dev, sizes, queries, radius, nsample):
+    g = torch.Generator().manual_seed(queries)
+    b = torch.arange(len(sizes)).repeat_interleave(torch.tensor(sizes))
+    x = torch.rand(b.numel(), 3, generator=g)
+    x[1::9] = x[0::9][: x[1::9].shape[0]]  # (some points twice)
+    pick = torch.sort(torch.randperm(b.numel(), generator=g)[:queries])[0]
+    y, by = x[pick].contiguous(), b[pick].contiguous()
+    idx, dist = tpk.ball_query(radius, nsample, x.to(dev), y.to(dev), mode="partial_dense", batch_x=b.to(dev), batch_y=by.to(dev), sort=True)
+    wi, wd = oracle.ball_query_sorted_partial(radius, nsample, x.numpy(), y.numpy(), b.numpy(), by.numpy())
+    np.testing.assert_array_equal(_np(idx), wi)
+    np.testing.assert_array_equal(_np(dist), wd)
+
+
 @pytest.mark.parametrize("radius", [2.0, 6.0])
 def test_ball_query_packed_of_large_balls_is_not_left_behind(dev, radius):
     """Balls that hold a large part of their cloud: the call over the table takes about as long as the one over bins in the smaller

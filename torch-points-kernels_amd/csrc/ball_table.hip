@@ -655,9 +655,17 @@ TableLayout table_layout(int64_t size_x, int64_t size_y)
 
 // Five launches and an atomic per support point have to pay: with fewer queries, or with fewer than a twelfth as many as points, the walk
 // over bins (two launches) answers a call in row order as soon or sooner.  33000 points, 4100 queries 20.7 us over bins, 23 here,
-// 33000 queries 32 and 24; 100000 points, 12500 queries 30 and 25; 212000 points, 26600 queries 38 and 37.  (Sorted neighbours
-// have this way only: the same calls 23.1 and 24 us - a walk over bins that kept a sorted list -, 43 and 25, 48 and 37.)
-constexpr int64_t BT_MIN_QUERIES = 8192, BT_MOST_SHARE = 12;
+// 33000 queries 32 and 24; 100000 points, 12500 queries 32 and 26; 212000 points, 13250 queries 33 and 35, 26600 queries 38 and 37.
+// Sorted neighbours cost the walk over bins more (a list of 64 keys, merged at every step with a hit), so it is the sooner one only for
+// few queries of a large array.  Over bins and here, us, radius 0.1 / 0.3 / 1.5 with 16 / 64 / 16 slots in rooms of 8:
+//     20000 points, 16 queries   23 / 22 / 81 and 19 / 24 / 55;  50000 points, 512 queries  24 / 26 / 123 and 21 / 27 / 109
+//     100000 points, 512 queries  25 / 31 / 157 and 24 / 34 / 186, 2048 queries  26 / 33 / 168 and 24 / 35 / 181
+//     200000 points, 2048 queries  31 / 50 / 223 and 33 / 47 / 319, 8192 queries  37 / 57 / 466 and 34 / 49 / 326
+//     400000 points, 512 queries  37 / 60 / 314 and 52 / 75 / 660, 8192 queries  51 / 88 / 656 and 53 / 84 / 626
+//     a million points, 16 queries  42 / 70 / 633 and 100 / 147 / 1557, 12500 queries  95 / 192 / 1771 and 103 / 198 / 2408
+// (In between, where a ball touches many bins of every window, the walk over bins is the slower one at every number of queries: a million points,
+// radius 0.6, 512 queries 630 and 347.  The host does not know the clouds' extent.)
+constexpr int64_t BT_MIN_QUERIES = 8192, BT_MOST_SHARE = 12, BT_SORTED_SHARE = 64, BT_SORTED_POINTS = 65536;
 
 bool table_supported(int64_t size_x, int64_t size_y, int nsample)
 {
@@ -672,12 +680,16 @@ size_t tpk_table_ball_query_workspace_bytes(int64_t size_x, int64_t size_y, int 
     return table_supported(size_x, size_y, nsample) ? table_layout(size_x, size_y).total : 0;
 }
 
+bool tpk_table_ball_query_pays(int64_t size_x, int64_t size_y, bool sorted)
+{
+    return sorted ? size_x < BT_SORTED_POINTS || size_y >= size_x / BT_SORTED_SHARE : size_y >= BT_MIN_QUERIES && size_y >= tpk_ceil_div(size_x, BT_MOST_SHARE);
+}
+
 int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, bool sorted, const float* x,
                                  const float* y, const int64_t* batch_x, const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
                                  size_t workspace_bytes, hipStream_t s)
 {
-    if (!table_supported(size_x, size_y, nsample) ||
-        (sorted ? nsample > TPK_WAVE : size_y < BT_MIN_QUERIES || size_y * BT_MOST_SHARE < size_x))
+    if (!table_supported(size_x, size_y, nsample) || !tpk_table_ball_query_pays(size_x, size_y, sorted) || (sorted && nsample > TPK_WAVE))
         return TPK_ERR_UNSUPPORTED;
     const TableLayout l = table_layout(size_x, size_y);
     if (!workspace || workspace_bytes < l.total)

@@ -1532,9 +1532,10 @@ extern "C" size_t tpk_ball_query_sorted_partial_workspace_bytes(int64_t size_x, 
     const size_t waves = tpk_grid_ball_sorted_workspace_bytes(1, most_x);
     const size_t grid = waves > lists ? waves : lists;
     // (up to 64 neighbours the packed array is searched as a whole: no wait)
-    const size_t table = tpk_table_ball_query_workspace_bytes(size_x, size_y, TPK_WAVE);
+    const size_t table = tpk_table_ball_query_pays(size_x, size_y, true) ? tpk_table_ball_query_workspace_bytes(size_x, size_y, TPK_WAVE) : 0;
+    const size_t bins = tpk_grid_ball_query_workspace_bytes(size_x, size_y, TPK_WAVE);
     const size_t cloudwise = grid ? NP_RANGES_BYTES + grid : 0;
-    return table > cloudwise ? table : cloudwise;
+    return std::max(std::max(table, bins), cloudwise);
 }
 
 extern "C" int tpk_ball_query_sorted_partial_f32(int64_t size_x, int64_t size_y, float radius, int nsample,
@@ -1562,10 +1563,13 @@ extern "C" int tpk_ball_query_sorted_partial_f32(int64_t size_x, int64_t size_y,
         return TPK_ERR_WORKSPACE;
     if (nsample <= TPK_WAVE)
     {
-        // A hash table of cells over the whole packed array, the rows of every query's cloud found on the device: no wait for the
-        // stream.
-        const int st = tpk_table_ball_query_partial(size_x, size_y, radius, limit, nsample, true, x, y, batch_x, batch_y,
-                                                   idx, dist, workspace, workspace_bytes, s);
+        // The whole packed array at once - a hash table of cells, for few queries windows of consecutive rows and their bins -, the
+        // rows of every query's cloud found on the device: no wait for the stream.
+        int st = tpk_table_ball_query_partial(size_x, size_y, radius, limit, nsample, true, x, y, batch_x, batch_y, idx, dist, workspace,
+                                              workspace_bytes, s);
+        if (st == TPK_ERR_UNSUPPORTED)
+            st = tpk_grid_ball_query_partial(size_x, size_y, radius, limit, nsample, true, x, y, batch_x, batch_y, idx, dist, workspace,
+                                             workspace_bytes, s);
         if (st != TPK_ERR_UNSUPPORTED)
             return st;
     }

@@ -745,7 +745,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void knn_grid_kernel(
 constexpr int NG_RUN = 16; // consecutive cells that share a second-level box in the wavefront-per-query search
 
 // ---------------------------------------------------------------------------------------
-// Ball query over bins, packed layout (several clouds back to back, sorted cloud id per point) for
+// Ball query over bins, packed layout (several clouds back to back, sorted cloud id per point): with sorted neighbours, and for
 // workspaces that do not hold the table of ball_table.hip; dense layout above 8192 points.
 //
 // The support array is cut into windows of 8192 or 16384 (bqb_window_shift) consecutive rows, each ordered on its
@@ -794,17 +794,22 @@ __device__ __forceinline__ void bin_range(float v, float r, float lo, float scal
     last = static_cast<int>(curve_grid_cell((v + r) + slack, lo, scale) >> 2);
 }
 
-// DENSE: the dense layout's rules instead (cuda/src/ball_query_gpu.cu:9-52) - clouds of dense_n
+// SORTED: the nsample (<= 64) NEAREST points with squared distance < radius2, nearest first, instead of the
+// first nsample in row order with squared distance <= radius2: the wavefront keeps its 64 best (distance, row)
+// keys sorted across the lanes and merges the hits of a step into them (as the wavefront-per-query kernel
+// further down does with the points of a cell).
+// DENSE (unsorted only): the dense layout's rules instead (cuda/src/ball_query_gpu.cu:9-52) - clouds of dense_n
 // consecutive rows with dense_m consecutive queries each (no cloud_rows), a hit has squared distance < radius2
 // (strict), indices count from the cloud's first row, and the slots behind the last hit repeat the first hit
 // (0 without any) with distance -1.
-template <bool DENSE>
+template <bool SORTED, bool DENSE>
 __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
     int size_x, int size_y, int window_shift, float radius, float radius2, int nsample, const float* __restrict__ x,
     const float* __restrict__ y, const float4* __restrict__ sorted_x, const int* __restrict__ bin_ends,
     const float4* __restrict__ grids, const int2* __restrict__ cloud_rows, int64_t* __restrict__ idx,
     float* __restrict__ dist, int dense_n, int dense_m)
 {
+    static_assert(!(SORTED && DENSE), "the sorted query of the dense layout has a kernel of its own");
     constexpr int WAVES = NG_SCAN_THREADS / TPK_WAVE;
     __shared__ int hit_rows[WAVES][BQB_HITS];
     __shared__ float hit_dists[WAVES][BQB_HITS];
@@ -839,6 +844,18 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
     // The walk is laid out so that dependent loads are few: all windows at once (one lane each),
     // then all (window, bin) pairs at once, then the candidates 64 at a time.
     int cnt = 0;
+    // SORTED: lane i holds the i-th smallest (distance, row) key so far; a hit must beat the nsample-th
+    constexpr u64 NONE = ~0ull;
+    u64 best = NONE, admit = NONE;
+    auto offer = [&](bool hit, float d, int row) __attribute__((always_inline)) {
+        u64 cand = hit ? knn_key(d, row) : NONE;
+        cand = cand < admit ? cand : NONE;
+        if (__ballot(cand != NONE) == 0)
+            return;
+        cand = wave_sort_keys(cand, lane, true);
+        best = wave_merge_ascending(best < cand ? best : cand, lane);
+        admit = read_lane_key(best, nsample - 1);
+    };
     const int wx0 = s0 >> window_shift;
     const int windows = s1 > s0 ? ((s1 - 1) >> window_shift) - wx0 + 1 : 0;
     bool serial = windows > TPK_WAVE; // answer by the scan in index order instead
@@ -900,6 +917,11 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
                 const float d = tpk_dist2(qx, qy, qz, p.x, p.y, p.z);
                 TPK_WORK_ADD(1);
                 const int row = __float_as_int(p.w);
+                if constexpr (SORTED)
+                {
+                    offer(has && d < radius2 && row >= s0 && row < s1, d, row);
+                    return;
+                }
                 const bool hit = has && (DENSE ? d < radius2 : d <= radius2) && row >= s0 && row < s1;
                 const unsigned long long mask = __ballot(hit);
                 if (mask == 0)
@@ -971,6 +993,42 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void ball_query_bins_kernel(
             walk_pairs(pair0);
     }
 
+    if constexpr (SORTED)
+    {
+        if (serial)
+        {
+            // too many windows or bins for the walk: every row of the cloud, 64 per step
+            constexpr int BATCH = 4;
+            for (int base = s0; base < s1; base += BATCH * TPK_WAVE)
+            {
+                float px[BATCH], py[BATCH], pz[BATCH];
+#pragma unroll
+                for (int u = 0; u < BATCH; ++u)
+                {
+                    const int64_t pos = min(base + u * TPK_WAVE + lane, s1 - 1);
+                    px[u] = x[pos * 3 + 0];
+                    py[u] = x[pos * 3 + 1];
+                    pz[u] = x[pos * 3 + 2];
+                }
+#pragma unroll
+                for (int u = 0; u < BATCH; ++u)
+                {
+                    const int pos = base + u * TPK_WAVE + lane;
+                    const float d = tpk_dist2(qx, qy, qz, px[u], py[u], pz[u]);
+                    TPK_WORK_ADD(1);
+                    offer(pos < s1 && d < radius2, d, pos);
+                }
+            }
+        }
+        if (lane < nsample)
+        {
+            const bool found = best != NONE;
+            idx[out + lane] = found ? static_cast<int64_t>(best & 0xFFFFFFFFu) : -1;
+            dist[out + lane] = found ? __int_as_float(static_cast<int>(best >> 32)) : -1.0f;
+        }
+        TPK_WORK_FLUSH
+        return;
+    }
     if (!serial)
     {
         // rank of every hit among the hits (rows are distinct), then hits in order, then -1
@@ -1451,12 +1509,12 @@ size_t tpk_grid_ball_query_workspace_bytes(int64_t size_x, int64_t size_y, int n
     return ball_bins_supported(size_x, size_y, nsample) ? ball_layout(size_x, size_y).total : 0;
 }
 
-int tpk_grid_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample,
+int tpk_grid_ball_query_partial(int64_t size_x, int64_t size_y, float radius, float radius2, int nsample, bool sorted,
                                 const float* x, const float* y, const int64_t* batch_x,
                                 const int64_t* batch_y, int64_t* idx, float* dist, void* workspace,
                                 size_t workspace_bytes, hipStream_t s)
 {
-    if (!ball_bins_supported(size_x, size_y, nsample))
+    if (!ball_bins_supported(size_x, size_y, nsample) || (sorted && nsample > TPK_WAVE))
         return TPK_ERR_UNSUPPORTED;
     const BallLayout l = ball_layout(size_x, size_y);
     if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255u))
@@ -1475,9 +1533,14 @@ int tpk_grid_ball_query_partial(int64_t size_x, int64_t size_y, float radius, fl
     const int64_t blocks = tpk_ceil_div(size_y, WAVES);
     if (blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((ball_query_bins_kernel<false>), dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), 0, s,
-                       static_cast<int>(size_x), static_cast<int>(size_y), window_shift, std::fabs(radius), radius2, nsample, x, y,
-                       px.sorted, px.bin_ends, px.grid, rows.rows, idx, dist, 0, 0);
+    if (sorted)
+        hipLaunchKernelGGL((ball_query_bins_kernel<true, false>), dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), 0, s,
+                           static_cast<int>(size_x), static_cast<int>(size_y), window_shift, std::fabs(radius), radius2, nsample, x, y,
+                           px.sorted, px.bin_ends, px.grid, rows.rows, idx, dist, 0, 0);
+    else
+        hipLaunchKernelGGL((ball_query_bins_kernel<false, false>), dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), 0, s,
+                           static_cast<int>(size_x), static_cast<int>(size_y), window_shift, std::fabs(radius), radius2, nsample, x, y,
+                           px.sorted, px.bin_ends, px.grid, rows.rows, idx, dist, 0, 0);
     return tpk_launch_status();
 }
 
@@ -1526,7 +1589,7 @@ int tpk_grid_ball_query_dense(int b, int n, int m, float radius, float radius2, 
     const int64_t blocks = tpk_ceil_div(size_y, WAVES);
     if (blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((ball_query_bins_kernel<true>), dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), 0, s,
+    hipLaunchKernelGGL((ball_query_bins_kernel<false, true>), dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), 0, s,
                        static_cast<int>(size_x), static_cast<int>(size_y), window_shift, std::fabs(radius), radius2, nsample, xyz,
                        new_xyz, px.sorted, px.bin_ends, px.grid, static_cast<const int2*>(nullptr), idx, dist, n, m);
     return tpk_launch_status();
