@@ -1364,6 +1364,57 @@ def test_knn_by_quarters_of_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
         np.testing.assert_array_equal(dist2[:, rows], wd)
 
 
+# (k = 8 and 9: the two shapes of the kernel; "axis": thousands of rows of cells for three or four of a wavefront's queries, "one in four" for
+# one of them; "shell": candidates at distances a few floats apart)
+@pytest.mark.parametrize("kind", ["far", "axis", "one in four", "around", "shell", "beyond float32"])
+@pytest.mark.parametrize("B,n,m,k", [(3, 8193, 10927, 8), (2, 9000, 16411, 16), (1, 60000, 32769, 3), (1, 20001, 32771, 9)])
+def test_knn_of_far_queries_by_quarters_of_wavefronts(tpk, oracle, dev, kind, B, n, m, k):
+    g = torch.Generator().manual_seed(n + k)
+    support, query = torch.rand(B, n, 3, generator=g), torch.rand(B, m, 3, generator=g)
+    if kind == "far":
+        query += 300
+    elif kind == "axis":
+        query[:, :, 0] += 300
+    elif kind == "one in four":
+        query[:, ::4, 1] -= 500
+    elif kind == "around":
+        query = 3 * query - 1
+    elif kind == "shell":
+        support = torch.nn.functional.normalize(support - 0.5, dim=2)
+        query *= 1e-4
+    else:
+        query[:, ::3] *= 1e19
+        query[:, 1::3] *= 1e25
+    idx, dist2 = tpk.knn(support.to(dev), query.to(dev), k)
+    idx, dist2 = _np(idx), _np(dist2)
+    for rows in (slice(0, 40), slice(m - 40, m)):
+        wi, wd = oracle.knn(support.numpy(), query[:, rows].contiguous().numpy(), k)
+        np.testing.assert_array_equal(idx[:, rows], wi)
+        np.testing.assert_array_equal(dist2[:, rows], wd)
+
+
+@pytest.mark.parametrize("kind", ["far"])
+def test_knn_by_quarters_of_wavefronts_is_not_left_behind(tpk, dev, kind):
+    """16 neighbours, four queries a wavefront, take no longer than 17, for which a wavefront serves a query (far queries: 0.8 times
+    as long, and 1.4 where their selections were given up)."""
+    g = torch.Generator().manual_seed(5)
+    support = torch.rand(8, 16384, 3, generator=g).to(dev)
+    query = (support + 300).contiguous()
+    took = []
+    for k in (16, 17):
+        times = []
+        for _ in range(20):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(4):
+                tpk.knn(support, query, k)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        took.append(min(times))
+    assert took[0] < 1.1 * took[1], took
+
+
 def test_knn_ties_and_errors(tpk, oracle, dev):
     # reference test/test_knn.py:14-23
     support = torch.tensor([[[0, 0, 0], [1, 0, 0], [2, 0, 0]]]).float().to(dev)

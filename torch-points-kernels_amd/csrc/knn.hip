@@ -781,7 +781,13 @@ constexpr int KNQ_SPARE = 16;  // (8: 1 to 3 % faster, but then nothing separate
 constexpr int KNQ_TRIES = 12;  // guesses of the distance
 constexpr int KNQ_FULL = 48;   // keys kept between two steps at most; a step adds up to 64
 constexpr int KNQ_LONG = 64;   // points of a walk by 16 lanes at most (112: 2 % slower in clusters)
-constexpr int KNQ_PIECES = 256;
+// The guess after which the distance of a selection is looked for between the nearest and the farthest candidate: seen from far away all
+// are about equally distant, which no estimate by volume finds.  (8 x 16384, queries 300 cloud sizes away, k = 16: 189 -> 107 us, a
+// quarter of them were given up after 12 guesses; a wavefront a query 135.  One guess earlier: 106, and 3 % slower on laser scans.)
+constexpr int KNQ_SPREAD = 2;
+// A single query with more rows of cells than this is given up, since the whole wavefront goes through them four times as fast; not where
+// most of the four have as many (8 x 16384, queries 300 cloud sizes away along one axis, k = 4 / 16: 833 / 761 -> 710 / 560 us).
+constexpr int KNQ_PIECES = 256, KNQ_TOGETHER = 3;
 
 // Puts the first cnt (<= 16 * HELD) keys of every query of the wavefront in ascending order, of which the k first stay.
 template <int HELD>
@@ -849,6 +855,20 @@ __device__ __forceinline__ void order_kept_by_wave(u64* mine, int cnt, int k, in
 __device__ __forceinline__ int most_of_four(int v)
 {
     return max(max(tpk_read_lane(v, 0), tpk_read_lane(v, 16)), max(tpk_read_lane(v, 32), tpk_read_lane(v, 48)));
+}
+
+// The smallest, or (LARGEST) the largest of the row's 16 values >= 0.
+template <bool LARGEST>
+__device__ __forceinline__ float row_extreme(float v)
+{
+    // (floats >= 0 order like their bits)
+    int s = __float_as_int(v);
+    auto with = [&](int turned) __attribute__((always_inline)) { s = LARGEST ? max(s, turned) : min(s, turned); };
+    with(__builtin_amdgcn_update_dpp(0, s, 0x128, 0xF, 0xF, true)); // row_ror:8
+    with(__builtin_amdgcn_update_dpp(0, s, 0x124, 0xF, 0xF, true));
+    with(__builtin_amdgcn_update_dpp(0, s, 0x122, 0xF, 0xF, true));
+    with(__builtin_amdgcn_update_dpp(0, s, 0x121, 0xF, 0xF, true));
+    return __int_as_float(s);
 }
 
 template <int PER, int MAX_K>
@@ -991,7 +1011,25 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
                 break;
             }
             const float estimate = guess * s.volume_ratio(target * __builtin_amdgcn_rcpf(fmaxf(static_cast<float>(held), 0.5f)));
-            const float next = bracket.next(guess, held < k, estimate, tries);
+            float next = bracket.next(guess, held < k, estimate, tries);
+            if (tries == KNQ_SPREAD)
+            {
+                float nearest = __builtin_inff(), farthest = 0.0f;
+#pragma unroll
+                for (int i = 0; i < PER; ++i)
+                {
+                    nearest = fminf(nearest, d[i]);
+                    farthest = d[i] < __builtin_inff() ? fmaxf(farthest, d[i]) : farthest;
+                }
+                nearest = row_extreme<false>(nearest);
+                farthest = row_extreme<true>(farthest);
+                const int candidates = min(total, MOST);
+                const float between = nearest + (farthest - nearest) * (target * __builtin_amdgcn_rcpf(static_cast<float>(candidates)));
+                const bool all = candidates <= k + KNQ_SPARE; // (these fit)
+                next = all ? farthest : between > bracket.lo && between < bracket.hi ? between : next;
+                bracket.lo = fmaxf(bracket.lo, nearest * 0.9999999f); // (the float below `nearest`: none lies within it)
+                bracket.hi = all ? bracket.hi : fminf(bracket.hi, farthest);
+            }
             guess = fits ? guess : next;
         }
 
@@ -1121,7 +1159,8 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
         if (!inside)
             ball_rows_of_far_query(grid, t, bound, from, to);
         const int wide = to[1] - from[1] + 1, pieces = 2 * wide * (to[2] - from[2] + 1); // (two for a row that crosses the block)
-        done = good && (inside || pieces <= KNQ_PIECES);
+        const int long_lists = __builtin_popcountll(__ballot(good && !inside && pieces > KNQ_PIECES && sub == 0));
+        done = good && (inside || pieces <= KNQ_PIECES || long_lists >= KNQ_TOGETHER);
         const bool wider = done && !inside;
         for (int piece0 = 0; __ballot(wider && piece0 < pieces) != 0; piece0 += KNQ_GROUP)
         {
