@@ -8,8 +8,8 @@
 // exactly equal distances is unspecified.  k must not exceed the number of support points
 // (cpu/src/knn.cpp:12-14 raises).
 //
-// Up to KNC_MAX_K neighbours are found by a wavefront per query (survivors.h): in clouds that fit into LDS over a grid there
-// (below), in larger ones, given a workspace, over such a grid in memory.  More neighbours, and large clouds without a
+// Up to KNC_MAX_K neighbours are found by a wavefront per query (survivors.h), over a grid in memory up to KNQ_MAX_K of many queries by a
+// quarter of one: in clouds that fit into LDS over a grid there (below), in larger ones, given a workspace, over such a grid in memory.  More neighbours, and large clouds without a
 // workspace: one lane owns one query and keeps its list in registers (topk.h), 32 entries a round - over
 // curve-ordered cells for clouds of 512..163840 points with a workspace, otherwise testing all pairs: the support points of
 // the cloud stream through LDS in tiles of float4, read by all lanes at the same address.
@@ -765,16 +765,30 @@ __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t qu
 // too many equal distances or more than KNQ_PIECES rows of cells outside are left to nearest_in_grid.
 // Bound by instruction issue (8 x 16384 even, k = 16: 1010 vector instructions per wavefront, 252 per query, 55 of the kernel's 59 us), most of
 // which nearest_in_grid spends whatever the number of candidates: a wavefront that serves one query has 86 of them in an even cloud (k = 16),
-// a third of whose queries look outside.  Calls of k = 4 / 16, a wavefront a query and
-// this way: 8 x 16384 even 87 / 106 -> 63 / 75 us, on a sphere 104 / 118 -> 70 / 80, in clusters of sigma 0.05 121 / 183 -> 91 / 157;
-// 8 x 4099 even 30 / 34 -> 24 / 28, in those clusters 38 / 50 -> 34 / 49; 2 x 100000 even 219 / 241 -> 176 / 191.  Slower are clouds
-// with hundreds of points in most queries' cells (clusters of sigma 0.003: 8 x 16384 341 / 368 -> 355 / 420) and queries far outside
-// the cloud (8 x 16384 120 / 136 -> 84 / 194).
+// a third of whose queries look outside.  Calls of k = 4 / 16, as many queries as points, a wavefront a query and this way, us:
+//                                            8 x 4099                8 x 16384                2 x 100000                 1 x 33000
+//     even                                30 / 35 -> 24 / 29       87 / 106 -> 58 / 70     219 / 240 -> 136 / 150      61 / 65 -> 44 / 46
+//     sphere                              33 / 35 -> 25 / 30      104 / 118 -> 64 / 75     254 / 298 -> 160 / 194      66 / 71 -> 47 / 49
+//     clusters of sigma 0.05              39 / 53 -> 32 / 50      125 / 192 -> 85 / 156    320 / 413 -> 246 / 325      75 / 97 -> 57 / 85
+//     clusters of sigma 0.02              44 / 56 -> 41 / 59      171 / 270 -> 147 / 253   566 / 713 -> 454 / 633      98 / 133 -> 89 / 131
+//     clusters of sigma 0.003             51 / 57 -> 55 / 63      338 / 365 -> 278 / 344  2234 / 2360 -> 1654 / 1787  194 / 199 -> 179 / 199
+//     laser scan (radius 1.5 to 50)       35 / 44 -> 31 / 47      102 / 138 -> 78 / 120    279 / 319 -> 206 / 256      67 / 79 -> 53 / 65
+//     queries 300 cloud sizes away        38 / 43 -> 45 / 37      117 / 135 -> 72 / 107    250 / 287 -> 145 / 187      68 / 67 -> 48 / 49
+//     the same along one axis             99 / 105 -> 111 / 100   692 / 619 -> 708 / 563  1946 / 2201 -> 1914 / 2300  307 / 260 -> 376 / 291
+//     queries over 3 times the width      39 / 45 -> 48 / 48      128 / 155 -> 124 / 157   272 / 346 -> 208 / 352      76 / 83 -> 77 / 85
+// What is still slower are small calls whose queries have long walks, which a quarter of the wavefronts then take one after the other.
 // (Without the eight cells: 8 x 16384 on a sphere, k = 16, 111; without the walks by the wavefront in clusters 273; with four wavefronts
-// per SIMD instead of six, which spill two registers, 77 to 81 even.)  k = 32, with 16 points a lane, was 8 to 13 % faster in even clouds
-// and 10 to 20 % slower in clusters.  Of 16384 queries even clouds gained 4 to 8 %, 30000 in clusters of sigma 0.02 took 139 us instead of 124.
+// per SIMD instead of six, which spill two registers, 77 to 81 even; seven and eight spill 14 and 33 and take 82 and more.)  k = 32, with 16
+// points a lane, was 8 to 13 % faster in even clouds and 10 to 20 % slower in clusters.
+// Built, measured, dropped: queries that are given up, or have hundreds of points to walk through or are far away, handed to a launch of
+// their own with a wavefront a query (8 x 4099, k = 16, even 30, clusters of sigma 0.003 80 to 105, far 53).
 constexpr int KNQ_MAX_K = 16;
-constexpr int64_t KNQ_LEAST = 32768; // queries: the chip has 8192 places for wavefronts
+// Queries from which on: with fewer the four wait for each other while wavefronts' places are empty - at six per SIMD there are 6144, 24576
+// queries -, and what uneven clouds and queries outside lose outweighs what even ones gain.  k = 4 / 16, time over a wavefront a query's, even,
+// clusters of sigma 0.05 and 0.003, queries over 3 times the width: 1 x 9000 0.98 / 1.00, 1.01 / 1.10, 1.17 / 1.28, 1.31 / 1.51; 4 x 5000 0.90 / 0.88,
+// 0.93 / 0.98, 1.09 / 1.13, 1.23 / 1.20; 7 x 4099 0.89 / 0.86, 0.90 / 0.99, 1.13 / 1.16, 1.19 / 1.09; 2 x 16000 0.88 / 0.87, 0.87 / 0.97, 0.99 / 1.09,
+// 1.20 / 1.25; 8 x 4099 0.79 / 0.81, 0.81 / 0.93, 1.08 / 1.11, 1.20 / 1.06; 8 x 16384 0.66 / 0.66, 0.68 / 0.81, 0.83 / 0.94, 0.96 / 1.01.
+constexpr int64_t KNQ_LEAST = 32768;
 constexpr int KNQ_GROUP = 16, KNQ_QUERIES = TPK_WAVE / KNQ_GROUP;
 constexpr int KNQ_OWN = 2, KNQ_EIGHT = 4; // (3 for the eight: within 2 %)
 constexpr int KNQ_SPARE = 16;  // (8: 1 to 3 % faster, but then nothing separates the 8 nearest on a lattice, where 7 and 19 points lie within a distance)
@@ -1055,8 +1069,8 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
                 reach = __int_as_float(static_cast<int>(mine[k - 1] >> 32));
             }
         };
-        // The candidates from c0 on of the rows of cells that a query's lanes hold.
-        auto walk = [&](int start, int size, int before, int total, int c0) __attribute__((always_inline)) {
+        // The candidates from c0 on of the rows of cells that a query's lanes hold (single: its first lane alone).
+        auto walk = [&](int start, int size, int before, int total, int c0, bool single) __attribute__((always_inline)) {
             const int origin = start - before;
             unsigned long long longer = __ballot(total - c0 > KNQ_LONG && sub == 0);
             while (longer != 0)
@@ -1071,7 +1085,12 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
                 const bool row_here = first / KNQ_GROUP == group && size > 0;
                 int its_cnt = tpk_read_lane(cnt, first);
                 float its_reach = tpk_read_lane(reach, first);
+                // (no looking up whose a candidate is where there is one row: clusters of sigma 0.003, 8 x 16384, 423 -> 342 us)
+                const bool its_single = tpk_read_lane(single ? 1 : 0, first) != 0;
+                const int its_origin = tpk_read_lane(origin, first);
                 auto fetch = [&](int c) __attribute__((always_inline)) {
+                    if (its_single)
+                        return points[c + lane < its_total ? its_origin + c + lane : 0];
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     mark64[lane] = 0;
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1140,7 +1159,7 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
                     order();
             }
         };
-        walk(start, size, before, good ? total : 0, MOST);
+        walk(start, size, before, good ? total : 0, MOST, one);
         order();
 
         // ---- the cells outside the block that the ball around the k-th touches (the ends as in nearest_in_grid) ----
@@ -1185,7 +1204,7 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
                 }
             }
             const int before = row_exclusive_sum(size);
-            walk(start, size, before, row_last(before + size, lane), 0);
+            walk(start, size, before, row_last(before + size, lane), 0, false);
         }
         if (__ballot(cnt > k) != 0)
             order();
