@@ -331,8 +331,8 @@ def test_a_block_goes_after_the_device_is_done_with_it(shim):
 
 @pytest.mark.parametrize("threads,parts,fails", [(1, 1, -1), (8, 5, -1), (16, 2, -1), (8, 5, 0), (8, 5, 3)])
 def test_threads_sleep_until_their_part_is_there(shim, threads, parts, fails):
-    """All threads get their part no sooner than it comes, or the error, and take no processor time while they wait (half of
-    one processor would do for a thread that asks for it again and again)."""
+    """All threads get their part no sooner than it comes, or the error, and sleep while it is long in coming: a thread that asks for it
+    again and again takes a processor for as long."""
     shim.parts_waited_for.restype = ctypes.c_double
     shim.parts_waited_for.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.c_int, ctypes.c_void_p]
     right, apart = ctypes.c_int(), 0.1
