@@ -297,15 +297,24 @@ at::Tensor grow_reference_order(const at::Tensor& neighbours, int64_t min_cluste
             check_status(tpk_grow_rows_part(n, nsample, neighbours.data_ptr<int64_t>(), found, static_cast<int>(entry), first, count, h + at_rows,
                                             ws.data_ptr(), ws_bytes, stream),
                          "grow_proximity (rows)");
-            arrivals.part(first + count, event());
+            if (part < points)
+                arrivals.part(first + count, event());
         }
         const int64_t bytes = points * 4;
         host.narrow(0, at_positions, bytes).copy_(staged.narrow(0, at_positions, bytes), /*non_blocking=*/true);
-        arrivals.part(points + 1, event());
-        if (arrivals.wait(1))
-            walk(h + at_rows, 0, pieces, &arrivals);
-        arrivals.wait(points + 1);
-        arrivals.rethrow();
+        if (part < points)
+        {
+            arrivals.part(points + 1, event());
+            if (arrivals.wait(1))
+                walk(h + at_rows, 0, pieces, &arrivals);
+            arrivals.wait(points + 1);
+            arrivals.rethrow();
+        }
+        else
+        {
+            wait(); // (a single part: two events and two waits cost more than there is to overlap)
+            walk(h + at_rows, 0, pieces, nullptr);
+        }
         writes.end();
     }
     else
