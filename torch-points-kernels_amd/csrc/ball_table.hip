@@ -19,12 +19,15 @@
 // before; clearing 3, counting 13, places 4, records 7, against 17 for the windows' ordering), all 212000 of their points as queries 117 ->
 // 61 (nsample 16, radius 0.04), 138 -> 75 (64, 0.1), 2300 -> 272 (64, 0.3: 60 points in a ball of a plane, which the walk over bins
 // left to the scan); 300000 queries of 24 clouds 257 -> 133.  By radius in rooms of 8, nsample 16 / 64:
-//     radius                        0.1                 0.3                   0.6                1                   1.4                2
-//     53000 of 4 clouds, 212000     58 / 59 -> 43 / 46  175 / 402 -> 86 / 92  327 / 678 -> 194 / 311  141 / 393 -> 142 / 331  71 / 182 -> 80 / 217  45 / 101 -> 46 / 93
-//     12500 of 1 cloud, 100000      33 / 34 -> 29 / 31  136 / 375 -> 59 / 74  147 / 310 -> 133 / 198  57 / 184 -> 106 / 227   35 / 77 -> 39 / 148   27 / 46 -> 29 / 48
-//     50000 of 1 cloud, 100000      57 / 58 -> 36 / 38  335 / 1035 -> 101 / 113  289 / 749 -> 211 / 378  112 / 367 -> 138 / 341  62 / 174 -> 60 / 223  44 / 97 -> 42 / 84
-// Still slower are balls of thousands of points, a hundredth of their cloud or more, whose queries are few: a wavefront that serves four
-// waits for the longest of their walks and then of their scans, on a chip that 3125 wavefronts do not fill.
+//     radius                       0.1                     0.3                     0.6                     1                       1.4                     2
+//     53000 of 4 clouds, 212000    57 / 57 -> 43 / 46      275 / 830 -> 85 / 86    305 / 709 -> 254 / 294  164 / 461 -> 163 / 360  83 / 243 -> 85 / 228    54 / 131 -> 51 / 108
+//     12500 of 1 cloud, 100000     32 / 33 -> 30 / 29      160 / 479 -> 52 / 53    176 / 309 -> 152 / 159  82 / 203 -> 114 / 229   46 / 116 -> 53 / 152    31 / 65 -> 33 / 74
+//     50000 of 1 cloud, 100000     53 / 54 -> 35 / 38      415 / 1446 -> 95 / 96   313 / 750 -> 249 / 311  152 / 471 -> 150 / 350  85 / 253 -> 73 / 221    52 / 133 -> 47 / 106
+//     17000 of 1 cloud, 200000     48 / 49 -> 44 / 45      525 / 794 -> 94 / 108   261 / 667 -> 244 / 379  85 / 275 -> 118 / 314   51 / 131 -> 64 / 151    37 / 76 -> 42 / 83
+//     24000 of 12 clouds, 24000    29 / 31 -> 22 / 24      31 / 33 -> 29 / 31      43 / 45 -> 28 / 30      51 / 53 -> 33 / 32      45 / 62 -> 40 / 46      34 / 59 -> 34 / 55
+//     300000 of 24 clouds, 300000  153 / 151 -> 82 / 96    176 / 178 -> 87 / 93    402 / 442 -> 202 / 202  604 / 1491 -> 355 / 606 322 / 991 -> 239 / 599  183 / 549 -> 150 / 359
+// Still slower are balls of a hundredth of their cloud or more with few queries: a wavefront that serves four waits for the longest of their
+// walks and then of their scans, on a chip that 3125 wavefronts do not fill.
 // What bounds it: the counting its atomics, the queries instruction issue - 690 vector instructions per wavefront, 170 per query
 // with 16 hits each, of 1700 clocks a query before.
 // Sorted neighbours (calls against the walk over bins that merged a sorted list, us): 212000 queries of the four scenes 188 -> 69 (16 slots, radius
@@ -46,11 +49,13 @@ constexpr int BT_GROUP = 16;                       // lanes per query
 constexpr int BT_QUERIES = TPK_WAVE / BT_GROUP;    // queries per wavefront
 constexpr int BT_HITS = 2 * TPK_WAVE;              // hits a query holds when a step begins
 constexpr int BT_KEPT = TPK_WAVE;                  // slots of a call whose queries may keep their lowest rows when they hold more
-constexpr int BT_LONG = 8 * BT_HITS;               // candidates from which on a query may be scanned for at once
-constexpr int BT_SAMPLES = 2;                      // of such a query's candidates, per lane, that tell how many of them lie in the ball
-constexpr int BT_HIT_STRIDE = BT_HITS + BT_GROUP + 2; // (the four queries of a wavefront read theirs at the same time: other banks)
+constexpr int BT_LONG = 128;                       // candidates from which on a query may be scanned for at once
+constexpr float BT_MOST_HIT = 0.5f, BT_LEAST_HIT = 1.0f / 64; // of such a query's candidates in the ball, as far as nobody has looked
+constexpr int BT_SAMPLES = 4;                      // of its candidates, per lane, that tell how many of them lie in the ball
+constexpr int BT_HIT_STRIDE = BT_HITS + BT_GROUP + 4; // (the four queries of a wavefront read theirs at the same time: other banks)
 constexpr int BT_COUNT_THREADS = 1024;
 constexpr int BT_COUNT_SLOTS = 2 * BT_COUNT_THREADS; // of the table in LDS: every point of the workgroup may need one
+constexpr int BT_AHEAD = 3;                        // steps whose candidates are requested together (2 and 4: 1 to 3 % slower)
 constexpr unsigned BT_NO_BUCKET = 0xffffffffu;
 constexpr int BT_SCAN_THREADS = 1024;
 constexpr int BT_CHUNK = BT_SCAN_THREADS * 4;      // buckets whose places one workgroup hands out
@@ -224,7 +229,7 @@ __device__ __forceinline__ int rank_among_row(typename HitKey<SORTED>::type mine
 }
 
 // Puts the first cnt hits of every query of the wavefront (int2 (row, distance); cnt is the same in a query's 16 lanes) in ascending order;
-// those that are not among the nsample lowest go.  Up to 16 and 32 hits a query's own lanes rank them, one or two each; above, the
+// those that are not among the nsample lowest go.  (cnt 0: a query whose hits stay as they are.)  Up to 16 and 32 hits a query's own lanes rank them, one or two each; above, the
 // whole wavefront ranks one query's after the other's by lane reads, three instructions per hit.
 template <bool SORTED>
 __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, int nsample)
@@ -266,6 +271,8 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
         {
             int2* const of_g = wave_hits + g * BT_HIT_STRIDE;
             const int count = tpk_read_lane(cnt, g * BT_GROUP);
+            if (count == 0)
+                continue;
             if (count <= TPK_WAVE)
             {
                 const int2 hit = of_g[lane];
@@ -283,18 +290,26 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
             static_assert(PER * TPK_WAVE >= BT_HITS + BT_GROUP, "every hit has a register");
             int2 hit[PER];
             int rank[PER];
+            if (lane < 4)
+                of_g[count + lane] = make_int2(SORTED ? -1 : 0x7fffffff, -1); // (read four at a time; behind all hits)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
             for (int j = 0; j < PER; ++j)
             {
                 hit[j] = of_g[min(j * TPK_WAVE + lane, BT_HIT_STRIDE - 1)];
                 rank[j] = 0;
             }
-            for (int i = 0; i < count; ++i)
+            for (int i = 0; i < count; i += 4)
             {
-                const Key other = K::of(of_g[i]);
+                Key other[4];
 #pragma unroll
-                for (int j = 0; j < PER; ++j)
-                    rank[j] += other < K::of(hit[j]) ? 1 : 0;
+                for (int u = 0; u < 4; ++u)
+                    other[u] = K::of(of_g[i + u]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int j = 0; j < PER; ++j)
+                        rank[j] += other[u] < K::of(hit[j]) ? 1 : 0;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
@@ -307,13 +322,12 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
 }
 
 // Whether a scan of the cloud in index order is likely to take less time than a walk over `candidates` more, for a query with
-// about `hits` hits.  The scan meets nsample of them within rows * nsample / hits rows, 64 a step of `per_step` instructions' time; a step
-// of the walk takes 45 instructions for 16 candidates of each of four queries.  A scan's step has about 10 (25 where it holds hits).  What
-// it counts for is fitted to calls of 12500 to 100000 queries with balls of 60 to 10000 points, where it is not instructions alone: before the
-// walk a step of a scan counts 8, since a long walk by 16 lanes waits for one load after the other; after 128 hits, when most of what is
-// left of a walk is short, 25.  (6 / 16: 100000 points in a room of 8, 12500 queries, radius 0.45 / 1 / 1.4: 137 / 99 / 38 us instead
-// of 107 / 106 / 39; 10 / 10: 103 / 116 / 38, and with 64 slots 170 / 234 / 168 instead of 139 / 227 / 148.)
-constexpr float BT_SCAN_STEP = 8.0f, BT_SCAN_STEP_LATER = 25.0f;
+// about `hits` hits.  The scan meets nsample of them within rows * nsample / hits rows, 64 a step of `per_step` instructions; a step of the
+// walk takes 45 for 16 candidates of each of four queries.  A scan's step counts 14 (9 for the test, 12 more where it holds hits) before the
+// walk, and 25 after 128 hits, when most of what is left of a walk is short.  (8 / 12 / 14 / 16 before the walk: 200000 points in a room of 8,
+// 17000 queries, radius 0.3, nsample 16, 146 / 123 / 94 / 94 us; radius 1, 97 / 114 / 118 / 150; 100000 points, 12500 queries, radius 0.6, 199 /
+// 168 / 152 / 146; radius 1.4, nsample 64, 133 / 136 / 152 / 166.)
+constexpr float BT_SCAN_STEP = 14.0f, BT_SCAN_STEP_LATER = 25.0f;
 __device__ __forceinline__ bool scan_is_shorter(float rows, float nsample, float hits, float candidates, float per_step)
 {
     const float scan = fminf(rows, rows * nsample * __builtin_amdgcn_rcpf(hits)) * (per_step / TPK_WAVE);
@@ -321,66 +335,118 @@ __device__ __forceinline__ bool scan_is_shorter(float rows, float nsample, float
 }
 
 // The support rows s0 .. s1 against those of the wavefront's four queries whose first lanes are set in `which`, as ball_scan_rows does
-// for one: a step's rows are loaded once for all of them.
+// for one: a step's rows are loaded once for all of them.  Hits go to a list in LDS, from there 64 at a time to the outputs: where balls are
+// large most steps have a few, and two stores to memory and their addresses take three times the instructions (300000 queries of 24 rooms,
+// radius 2, nsample 16 / 64: 181 / 440 us stored one by one, 151 / 330 this way).
 __device__ __forceinline__ void bt_scan_rows(const float* __restrict__ x, int s0, int s1, unsigned long long which, float qx, float qy, float qz,
-                                             float radius2, int nsample, int lane, int64_t* __restrict__ idx4, float* __restrict__ dist4 TPK_WORK_PARAM)
+                                             float radius2, int nsample, int lane, int2* wave_hits, int64_t* __restrict__ idx4,
+                                             float* __restrict__ dist4 TPK_WORK_PARAM)
 {
     constexpr int BATCH = 4; // loads of four steps in flight (6: 3 % slower; the next four requested ahead: nothing)
+    static_assert(2 * TPK_WAVE <= BT_HIT_STRIDE, "less than 64 hits wait in a query's list, and a step adds up to 64");
     float x4[BT_QUERIES], y4[BT_QUERIES], z4[BT_QUERIES];
-    int cnt[BT_QUERIES];
+    const unsigned slots = nsample;
+    unsigned cnt[BT_QUERIES];
 #pragma unroll
     for (int g = 0; g < BT_QUERIES; ++g)
     {
         x4[g] = to_vector_register(tpk_read_lane(qx, g * BT_GROUP));
         y4[g] = to_vector_register(tpk_read_lane(qy, g * BT_GROUP));
         z4[g] = to_vector_register(tpk_read_lane(qz, g * BT_GROUP));
-        cnt[g] = which >> (g * BT_GROUP) & 1 ? 0 : nsample;
+        cnt[g] = which >> (g * BT_GROUP) & 1 ? 0 : slots;
     }
-    for (int base = s0; base < s1 && min(min(cnt[0], cnt[1]), min(cnt[2], cnt[3])) < nsample; base += BATCH * TPK_WAVE)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const float none = __builtin_nanf("");
+#pragma unroll
+    for (int g = 0; g < BT_QUERIES; ++g)
+        x4[g] = cnt[g] < slots ? x4[g] : none; // (no row is within reach of a query that is done)
+    for (int base = s0; base < s1 && min(min(cnt[0], cnt[1]), min(cnt[2], cnt[3])) < slots; base += BATCH * TPK_WAVE)
     {
         float px[BATCH], py[BATCH], pz[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
+        const float* __restrict__ const at = x + static_cast<int64_t>(base) * 3;
+        const int last = s1 - 1 - base;
+        if (last >= BATCH * TPK_WAVE - 1)
         {
-            const int64_t pos = min(base + u * TPK_WAVE + lane, s1 - 1);
-            px[u] = x[pos * 3 + 0];
-            py[u] = x[pos * 3 + 1];
-            pz[u] = x[pos * 3 + 2];
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+            {
+                const unsigned word = static_cast<unsigned>(lane) * 3u + u * (TPK_WAVE * 3u);
+                px[u] = at[word + 0u];
+                py[u] = at[word + 1u];
+                pz[u] = at[word + 2u];
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+            {
+                const int row = u * TPK_WAVE + lane;
+                const unsigned word = static_cast<unsigned>(min(row, last)) * 3u;
+                px[u] = row <= last ? at[word + 0u] : none;
+                py[u] = at[word + 1u];
+                pz[u] = at[word + 2u];
+            }
         }
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
         {
-            const int pos = base + u * TPK_WAVE + lane;
-            const unsigned long long rows = __ballot(pos < s1);
+            // (all four at once: a test has to wait for the test in front of it only where there are hits)
+            float d[BT_QUERIES];
+            unsigned long long mask[BT_QUERIES];
 #pragma unroll
             for (int g = 0; g < BT_QUERIES; ++g)
             {
-                if (cnt[g] >= nsample)
-                    continue;
-                const float d = tpk_dist2(x4[g], y4[g], z4[g], px[u], py[u], pz[u]);
+                d[g] = tpk_dist2(x4[g], y4[g], z4[g], px[u], py[u], pz[u]);
                 TPK_WORK_ADD(1);
-                const unsigned long long mask = rows & __ballot(d <= radius2);
-                if (mask == 0)
-                    continue; // (most steps of a long scan)
-                const bool hit = mask >> lane & 1;
-                const int slot = cnt[g] + static_cast<int>(tpk_prefix_count(mask));
-                if (hit && slot < nsample)
+            }
+#pragma unroll
+            for (int g = 0; g < BT_QUERIES; ++g)
+                mask[g] = __ballot(d[g] <= radius2);
+            if (((mask[0] | mask[1]) | (mask[2] | mask[3])) == 0)
+                continue; // (most steps of a long scan)
+            const int pos = base + u * TPK_WAVE + lane;
+#pragma unroll
+            for (int g = 0; g < BT_QUERIES; ++g)
+            {
+                if (mask[g] == 0)
+                    continue;
+                int2* const list = wave_hits + g * BT_HIT_STRIDE;
+                const unsigned waiting = cnt[g] % TPK_WAVE;
+                if (d[g] <= radius2)
+                    list[__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask[g] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask[g]), waiting))] =
+                        make_int2(pos, __float_as_int(d[g]));
+                const unsigned found = __builtin_popcountll(mask[g]);
+                cnt[g] += found;
+                x4[g] = cnt[g] < slots ? x4[g] : none;
+                if (waiting + found < TPK_WAVE)
+                    continue;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const unsigned s = cnt[g] / TPK_WAVE * TPK_WAVE - TPK_WAVE + lane;
+                const int2 hit = list[lane], behind = list[TPK_WAVE + lane];
+                if (s < slots)
                 {
-                    idx4[g * nsample + slot] = pos;
-                    dist4[g * nsample + slot] = d;
+                    idx4[g * slots + s] = hit.x;
+                    dist4[g * slots + s] = __int_as_float(hit.y);
                 }
-                cnt[g] += __builtin_popcountll(mask);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                list[lane] = behind;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             }
         }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int g = 0; g < BT_QUERIES; ++g)
         if (which >> (g * BT_GROUP) & 1)
-            for (int s = cnt[g] + lane; s < nsample; s += TPK_WAVE)
+            for (unsigned s = cnt[g] / TPK_WAVE * TPK_WAVE + lane; s < slots; s += TPK_WAVE)
             {
-                idx4[g * nsample + s] = -1;
-                dist4[g * nsample + s] = -1.0f;
+                const bool found = s < cnt[g];
+                const int2 hit = wave_hits[g * BT_HIT_STRIDE + lane];
+                idx4[g * slots + s] = found ? hit.x : -1;
+                dist4[g * slots + s] = found ? __int_as_float(hit.y) : -1.0f;
             }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
 // SORTED: the nsample (<= 64) NEAREST points with squared distance < radius2, nearest first (equal distances: lower row first), instead
@@ -483,9 +549,18 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
     if constexpr (!SORTED)
     {
         // A run of cells holds 5 to 13 times what the ball itself does, on a surface and in space, but a query beside a surface whose
-        // cells it touches may have a hundredth: of long runs a few candidates at equal distances tell.  (Always an eighth: 12500
-        // queries of 100000 points, radius 0.6, 177 us instead of 133.)
-        const bool asks = total > BT_LONG;
+        // cells it touches may have a hundredth.  Where the scan would be sooner with half of the candidates in the ball, but not with a
+        // sixty-fourth, a few of them at equal distances tell.  (100000 points in a room of 8, 12500 queries: always an eighth, radius 0.6,
+        // 177 us instead of 133; asked from 1024 candidates on, 24000 points of twelve rooms, radius 2, 63 instead of 35; asked whatever
+        // they say, radius 4, 26 instead of 23.)
+        const float rows = static_cast<float>(s1 - s0), slots = static_cast<float>(nsample), candidates = static_cast<float>(total);
+        auto scan_is_sooner = [&](float share, float more) __attribute__((always_inline)) {
+            return scan_is_shorter(rows, slots, candidates * share, more, BT_SCAN_STEP);
+        };
+        const bool may = total > BT_LONG && scan_is_sooner(BT_MOST_HIT, candidates);
+        scan = scan || (may && scan_is_sooner(BT_LEAST_HIT, candidates));
+        const bool asks = may && !scan;
+        total = scan ? 0 : total;
         if (__ballot(asks) != 0)
         {
             int in = 0;
@@ -505,14 +580,17 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
                 }
             }
             const float share = few ? fmaxf(static_cast<float>(in), 0.5f) * (1.0f / (BT_SAMPLES * BT_GROUP)) : 0.125f;
-            const float candidates = static_cast<float>(total);
-            if (asks && scan_is_shorter(static_cast<float>(s1 - s0), static_cast<float>(nsample), candidates * share, candidates, BT_SCAN_STEP))
-            {
-                scan = true;
-                total = 0;
-            }
-            most_total = bt_most(total);
+            // A wavefront walks as long as its longest query: what a query adds to that is what its walk is longer than those of the
+            // queries that walk anyway, shared by the others that would.  (Always a quarter of its own: 100000 points, 50000 queries,
+            // radius 1.4, nsample 16 / 64, 82 / 211 us instead of 71 / 188.)
+            const float others = static_cast<float>(bt_most(asks ? 0 : total));
+            bool walks = asks && !scan_is_sooner(share, candidates);
+            const float together = static_cast<float>(__builtin_popcountll(__ballot(walks && sub == 0)));
+            walks = walks && !scan_is_sooner(share, fmaxf(candidates - others, 0.0f) * (BT_QUERIES / together));
+            scan = scan || (asks && !walks);
+            total = scan ? 0 : total;
         }
+        most_total = bt_most(total);
     }
     auto fetch = [&](int c0) __attribute__((always_inline)) {
         const int c = c0 + sub;
@@ -540,32 +618,36 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
         return record_at(c < total ? at : 0);
     };
     int c0 = 0;
-    float4 ahead = fetch(0);
     for (;;)
     {
-        for (; c0 < most_total; c0 += BT_GROUP)
+        for (bool full = false; c0 < most_total && !full;)
         {
-            const float4 p = ahead;
-            const bool has = c0 + sub < total;
-            if (c0 + BT_GROUP < most_total)
-                ahead = fetch(c0 + BT_GROUP);
-            const float d = tpk_dist2(qx, qy, qz, p.x, p.y, p.z);
-            TPK_WORK_ADD(has ? 1 : 0);
-            const int row = __float_as_int(p.w);
-            const bool near_enough = SORTED ? d < limit || (d == limit && row < limit_row) : d <= radius2;
-            const bool hit = has && near_enough && static_cast<unsigned>(row - s0) < wanted;
-            const unsigned long long all = __ballot(hit);
-            if (all == 0)
-                continue;
-            const unsigned low = static_cast<unsigned>(all) & group_low, high = static_cast<unsigned>(all >> 32) & group_high;
-            const unsigned slot = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, cnt));
-            if (hit)
-                my_hits[slot] = make_int2(row, __float_as_int(d));
-            cnt += __builtin_popcount(low) + __builtin_popcount(high);
-            if (__ballot(cnt > BT_HITS) != 0)
+            float4 p[BT_AHEAD];
+#pragma unroll
+            for (int j = 0; j < BT_AHEAD; ++j)
+                if (j == 0 || c0 + j * BT_GROUP < most_total)
+                    p[j] = fetch(c0 + j * BT_GROUP);
+#pragma unroll
+            for (int j = 0; j < BT_AHEAD; ++j)
             {
+                if (c0 >= most_total || full)
+                    break;
+                const bool has = c0 + sub < total;
+                const float d = tpk_dist2(qx, qy, qz, p[j].x, p[j].y, p[j].z);
+                TPK_WORK_ADD(has ? 1 : 0);
+                const int row = __float_as_int(p[j].w);
+                const bool near_enough = SORTED ? d < limit || (d == limit && row < limit_row) : d <= radius2;
+                const bool hit = has && near_enough && static_cast<unsigned>(row - s0) < wanted;
+                const unsigned long long all = __ballot(hit);
                 c0 += BT_GROUP;
-                break;
+                if (all == 0)
+                    continue;
+                const unsigned low = static_cast<unsigned>(all) & group_low, high = static_cast<unsigned>(all >> 32) & group_high;
+                const unsigned slot = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, cnt));
+                if (hit)
+                    my_hits[slot] = make_int2(row, __float_as_int(d));
+                cnt += __builtin_popcount(low) + __builtin_popcount(high);
+                full = __ballot(cnt > BT_HITS) != 0;
             }
         }
         // Full: the nsample lowest rows are kept and the walk goes on, or the query is scanned for.  (Once rows are kept
@@ -580,8 +662,9 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
             cnt = scan ? 0 : cnt;
         }
         most_total = bt_most(total);
-        order_hits<SORTED>(hits[wave], cnt, lane, nsample);
-        if (cnt >= nsample)
+        const bool ends = c0 >= most_total, ordered = ends || cnt > BT_HITS;
+        order_hits<SORTED>(hits[wave], ordered ? cnt : 0, lane, nsample);
+        if (ordered && cnt >= nsample)
         {
             cnt = nsample;
             const int2 last = my_hits[nsample - 1];
@@ -593,7 +676,7 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
             else
                 wanted = last.x - s0;
         }
-        if (c0 >= most_total)
+        if (ends)
             break;
     }
 
@@ -618,7 +701,7 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
         const int first = tpk_read_lane(s0, from), end = tpk_read_lane(s1, from);
         const unsigned long long with = left & __ballot(s0 == first && s1 == end);
         left &= ~with;
-        bt_scan_rows(x, first, end, with, qx, qy, qz, radius2, nsample, lane, idx4, dist4 TPK_WORK_ARG);
+        bt_scan_rows(x, first, end, with, qx, qy, qz, radius2, nsample, lane, hits[wave], idx4, dist4 TPK_WORK_ARG);
     }
     TPK_WORK_FLUSH
 }
