@@ -100,8 +100,9 @@ int tpk_ball_query_dense_ws_f32(int b, int n, int m, float radius, int nsample,
  * along a space filling curve and a query only visits cells within its radius; queries with
  * more than 16 neighbours in the radius are then answered by a scan in index order that stops
  * after nsample hits.  With workspace == NULL every query scans its whole cloud (same results).
- * A workspace of tpk_ball_query_partial_table_workspace_bytes() bytes or more (0 for sizes not served that way; 28 .. 36
- * bytes per support point and 8 per query) holds a hash table of cells instead, which calls with many queries take (same results).
+ * A workspace of tpk_ball_query_partial_table_workspace_bytes() bytes or more (0 for sizes not served that way; 8 bytes per query and,
+ * from 32768 support points on, 28 .. 36 per point, for fewer 20 per point and a table of 512 KiB) holds a hash table of cells instead,
+ * which calls with many queries take (same results).
  * ------------------------------------------------------------------------------------- */
 size_t tpk_ball_query_partial_workspace_bytes(int64_t size_x, int64_t size_y, int nsample);
 size_t tpk_ball_query_partial_table_workspace_bytes(int64_t size_x, int64_t size_y, int nsample);

@@ -23,6 +23,8 @@ def test_header_declares_the_expected_entry_points():
     names = _declared_symbols()
     for want in (
         "tpk_fps_f32", "tpk_fps_workspace_bytes", "tpk_ball_query_dense_f32", "tpk_ball_query_dense_workspace_bytes", "tpk_ball_query_dense_ws_f32", "tpk_ball_query_partial_workspace_bytes", "tpk_ball_query_partial_f32",
+        "tpk_ball_query_partial_table_workspace_bytes", "tpk_grow_components_workspace_bytes", "tpk_grow_components", "tpk_grow_components_by_size",
+        "tpk_grow_places", "tpk_grow_rows", "tpk_grow_rows_part", "tpk_grow_members", "tpk_region_order_workspace_bytes", "tpk_region_order", "tpk_region_members",
         "tpk_three_nn_workspace_bytes", "tpk_three_nn_f32", "tpk_knn_workspace_bytes", "tpk_knn_f32", "tpk_three_interpolate_f32", "tpk_three_interpolate_grad_f32", "tpk_group_f32",
         "tpk_three_interpolate_lists_f32", "tpk_three_interpolate_grad_lists_f32", "tpk_group_lists", "tpk_group_grad_lists_f32",
         "tpk_group_grad_f32", "tpk_chamfer_fwd_workspace_bytes", "tpk_chamfer_fwd_f32", "tpk_chamfer_fwd_f64", "tpk_chamfer_bwd_f32",

@@ -2378,6 +2378,86 @@ def test_c_abi_pieces_in_the_order_of_their_first_points(dev):
             assert lib.tpk_grow_rows_part(L(n), nsample, P(neighbours), found, entry_bytes, L(12), L(4), P(parts), P(ws), Z(nbytes), S) == -1
 
 
+# (8192 points: the smallest table; 32769 and 40000: 4 buckets per point and nearly 3; 12 points a query, the fewest that take the table)
+@pytest.mark.parametrize("n,m", [(8192, 8192), (32769, 9001), (40000, 30001), (98304, 8192)])
+def test_c_abi_table_of_cells_in_exactly_its_bytes(oracle, dev, n, m):
+    """tpk_ball_query_partial_f32 with as many bytes as tpk_ball_query_partial_table_workspace_bytes says: nothing in front of them or
+    behind is written; with one byte less the call falls back to the walk over bins, with the same results."""
+    import ctypes
+    import os
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip.so"))
+    P, L = lambda t: ctypes.c_void_p(t.data_ptr()), ctypes.c_int64
+    lib.tpk_ball_query_partial_table_workspace_bytes.restype = ctypes.c_size_t
+    nbytes = lib.tpk_ball_query_partial_table_workspace_bytes(L(n), L(m), 8)
+    table = 4 * max(131072, 1 << (2 * n - 1).bit_length())
+    assert 20 * n + 8 * m + table <= nbytes <= 20 * n + 8 * m + table + table // 4096 + 6 * 256
+    g = torch.Generator().manual_seed(n)
+    x, y = torch.rand(n, 3, generator=g), torch.rand(m, 3, generator=g)
+    bx, by = torch.sort(torch.randint(0, 3, (n,), generator=g))[0], torch.sort(torch.randint(0, 4, (m,), generator=g))[0]
+    wi, wd = oracle.ball_query_partial_dense(0.05, 8, x.numpy(), y.numpy(), bx.numpy(), by.numpy())
+    x, y, bx, by = x.to(dev), y.to(dev), bx.to(dev), by.to(dev)
+    guard = 4096
+    buffer = torch.empty(guard + nbytes + guard, dtype=torch.uint8, device=dev)
+    assert buffer.data_ptr() % 256 == 0
+    for given in (nbytes, nbytes - 1):
+        buffer.fill_(0xA5)
+        idx, dist = torch.full((m, 8), 77, dtype=torch.int64, device=dev), torch.full((m, 8), 77.0, device=dev)
+        assert lib.tpk_ball_query_partial_f32(L(n), L(m), ctypes.c_float(0.05), 8, P(x), P(y), P(bx), P(by), P(idx), P(dist),
+                                              ctypes.c_void_p(buffer.data_ptr() + guard), ctypes.c_size_t(given),
+                                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        np.testing.assert_array_equal(_np(idx), wi)
+        np.testing.assert_array_equal(_np(dist), wd)
+        after = _np(buffer)
+        assert (after[:guard] == 0xA5).all() and (after[guard + nbytes:] == 0xA5).all()
+        # the table's last 256 bytes hold its counter of places; the bins take less room
+        assert (after[guard + nbytes - 256:guard + nbytes] != 0xA5).any() == (given == nbytes)
+
+
+@pytest.mark.parametrize("entry_bytes,dtype", [(2, np.uint16), (4, np.uint32)])
+def test_c_abi_members_of_clusters(dev, entry_bytes, dtype):
+    """tpk_grow_members (clusters of one member, of 300, the highest entry 65535) and tpk_region_members with positions of both sizes."""
+    import ctypes
+    import os
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip.so"))
+    P, L = lambda t: ctypes.c_void_p(t.data_ptr()), ctypes.c_int64
+    S = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rng = np.random.default_rng(entry_bytes)
+    n = 100000
+    positions = rng.permutation(n).astype(np.int32)
+    order = rng.permutation(n).astype(np.int32)
+    sizes = np.array([1, 300, 1, 2, 777, 1])
+    bases = np.array([0, 34000, 5, 34000, 70000, 99999])
+    first_entries = np.array([900, 0, 400, 500, 1000, 902])  # (clusters need not lie in the order of their outputs)
+    entries = np.zeros(2000, dtype)
+    want = []
+    for size, base, at in zip(sizes, bases, first_entries):
+        here = rng.integers(0, min(65536, n - base), size)
+        here[0] = min(65535, n - base - 1)
+        entries[at:at + size] = here
+        want += list(positions[base + here])
+    table = np.stack([np.concatenate([[0], np.cumsum(sizes)[:-1]]), first_entries, bases], 1).astype(np.int64)
+    put = lambda a: torch.from_numpy(a.view(np.uint8).reshape(-1).copy()).to(dev)
+    d_table, d_entries, d_positions, d_order = put(table), put(entries), put(positions), put(order)
+    members = torch.full((len(want) + 1,), -7, dtype=torch.int64, device=dev)
+    for with_order in (False, True):
+        expect = order[want] if with_order else np.array(want)
+        members.fill_(-7)
+        assert lib.tpk_grow_members(L(len(want)), L(len(sizes)), P(d_table), entry_bytes, P(d_entries), P(d_positions), P(d_order) if with_order else None,
+                                    P(members), S) == 0
+        assert members.tolist() == list(expect) + [-7]
+        there = put(np.array(want, np.int32 if entry_bytes == 2 else np.int64))
+        members.fill_(-7)
+        assert lib.tpk_region_members(L(len(want)), P(d_order) if with_order else None, 4 if entry_bytes == 2 else 8, P(there), P(members), S) == 0
+        assert members.tolist() == list(expect) + [-7]
+    assert lib.tpk_grow_members(L(0), L(0), None, entry_bytes, None, None, None, None, S) == 0
+    assert lib.tpk_grow_members(L(1), L(1), None, entry_bytes, P(d_entries), P(d_positions), None, P(members), S) == -1
+    assert lib.tpk_grow_members(L(1), L(1), P(d_table), 3, P(d_entries), P(d_positions), None, P(members), S) == -1
+
+
 def test_c_abi_direct_call(oracle, dev):
     """libtpk_hip.so used without the extension: ctypes + raw device pointers + a stream."""
     import ctypes

@@ -1,7 +1,7 @@
 // Ball query, packed layout, over a hash table of cells (several clouds back to back, sorted cloud id per point).
 //
 // Space is cut into cells of 0.55 x 2.2 x 2.2 reaches (the reach: the radius and its rounding), and cell (ix, iy, iz) of a cloud
-// belongs to bucket row(iy, iz, cloud) + ix of a table with 2 .. 4 buckets per support point: the cells a ball touches are
+// belongs to bucket row(iy, iz, cloud) + ix of a table with 2 .. 4 buckets per support point, 131072 at least: the cells a ball touches are
 // at most four runs (two values of iy, two of iz; three each within rounding of an edge) of four or five consecutive buckets.  No
 // bounding box, no windows, no limit on a cloud's size: the launches in front of the queries clear the table, count the points
 // per bucket (the atomic that counts hands out the point's place in its bucket), turn the counts into places, and put the points
