@@ -175,12 +175,6 @@ __global__ void __launch_bounds__(BT_THREADS)
     records[table[bucket] + ranks[i]] = make_float4(px, py, pz, __int_as_float(i));
 }
 
-// The largest of the four queries' values (each the same in the query's lanes).
-__device__ __forceinline__ int bt_most(int v)
-{
-    return max(max(tpk_read_lane(v, 0), tpk_read_lane(v, 16)), max(tpk_read_lane(v, 32), tpk_read_lane(v, 48)));
-}
-
 // (value of the row's lane L)
 template <int L>
 __device__ __forceinline__ int row_lane(int v)
@@ -238,7 +232,7 @@ __device__ __forceinline__ void order_hits(int2* wave_hits, int cnt, int lane, i
     using Key = typename K::type;
     const int group = lane / BT_GROUP, sub = lane % BT_GROUP;
     int2* const hits = wave_hits + group * BT_HIT_STRIDE;
-    const int most = bt_most(cnt);
+    const int most = rows_max(cnt);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if (most <= BT_GROUP)
     {
@@ -535,7 +529,7 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
     float limit = radius2;
     int limit_row = 0;
     const unsigned group_low = group < 2 ? 0xffffu << group_lane : 0, group_high = group < 2 ? 0 : 0xffffu << (group_lane - 32);
-    int most_total = bt_most(total);
+    int most_total = rows_max(total);
     auto record_at = [&](int at) __attribute__((always_inline)) {
         return records[static_cast<uint32_t>(at)];
     };
@@ -583,14 +577,14 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
             // A wavefront walks as long as its longest query: what a query adds to that is what its walk is longer than those of the
             // queries that walk anyway, shared by the others that would.  (Always a quarter of its own: 100000 points, 50000 queries,
             // radius 1.4, nsample 16 / 64, 82 / 211 us instead of 71 / 188.)
-            const float others = static_cast<float>(bt_most(asks ? 0 : total));
+            const float others = static_cast<float>(rows_max(asks ? 0 : total));
             bool walks = asks && !scan_is_sooner(share, candidates);
             const float together = static_cast<float>(__builtin_popcountll(__ballot(walks && sub == 0)));
             walks = walks && !scan_is_sooner(share, fmaxf(candidates - others, 0.0f) * (BT_QUERIES / together));
             scan = scan || (asks && !walks);
             total = scan ? 0 : total;
         }
-        most_total = bt_most(total);
+        most_total = rows_max(total);
     }
     auto fetch = [&](int c0) __attribute__((always_inline)) {
         const int c = c0 + sub;
@@ -661,7 +655,7 @@ __global__ void __launch_bounds__(BT_THREADS, SORTED ? 7 : 8) // (wavefronts per
             total = scan ? 0 : total;
             cnt = scan ? 0 : cnt;
         }
-        most_total = bt_most(total);
+        most_total = rows_max(total);
         const bool ends = c0 >= most_total, ordered = ends || cnt > BT_HITS;
         order_hits<SORTED>(hits[wave], ordered ? cnt : 0, lane, nsample);
         if (ordered && cnt >= nsample)

@@ -865,12 +865,6 @@ __device__ __forceinline__ void order_kept_by_wave(u64* mine, int cnt, int k, in
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// The largest of the four queries' values (each the same in the query's lanes).
-__device__ __forceinline__ int most_of_four(int v)
-{
-    return max(max(tpk_read_lane(v, 0), tpk_read_lane(v, 16)), max(tpk_read_lane(v, 32), tpk_read_lane(v, 48)));
-}
-
 // The smallest, or (LARGEST) the largest of the row's 16 values >= 0.
 template <bool LARGEST>
 __device__ __forceinline__ float row_extreme(float v)
@@ -885,7 +879,7 @@ __device__ __forceinline__ float row_extreme(float v)
     return __int_as_float(s);
 }
 
-template <int PER, int MAX_K>
+template <int PER>
 __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, int m, int k, unsigned blocks_per_cloud, KnnGridLayout layout,
                                                                     const float* __restrict__ query, const unsigned char* __restrict__ workspace,
                                                                     float* __restrict__ dist2, int64_t* __restrict__ idx)
@@ -893,7 +887,7 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
     constexpr int WAVES = KNN_THREADS / TPK_WAVE;
     constexpr int MOST = PER * KNQ_GROUP;                              // a query's candidates
     constexpr int ROOM = KNQ_FULL + TPK_WAVE + 4;
-    static_assert(MOST <= 256 && MAX_K + KNQ_SPARE <= KNQ_FULL, "");
+    static_assert(MOST <= 256 && KNQ_MAX_K + KNQ_SPARE <= KNQ_FULL, "a byte holds a place, the selected keys fit");
     __shared__ u64 keys[WAVES][KNC_ROOM];
     __shared__ u64 kept[WAVES][KNQ_QUERIES][ROOM];
     __shared__ unsigned marks[WAVES][KNQ_QUERIES][MOST / 4];
@@ -1059,7 +1053,7 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
                     mine[at++] = knn_key(d[i], __float_as_int(p[i].w));
         }
         auto order = [&]() __attribute__((always_inline)) {
-            if (most_of_four(cnt) <= 2 * KNQ_GROUP)
+            if (rows_max(cnt) <= 2 * KNQ_GROUP)
                 order_kept<2>(mine, cnt, k, sub);
             else
                 order_kept<(KNQ_FULL + KNQ_GROUP) / KNQ_GROUP>(mine, cnt, k, sub);
@@ -1126,7 +1120,7 @@ __global__ __launch_bounds__(KNN_THREADS, 6) void knn_grid_four_kernel(int n, in
                 reach = first / KNQ_GROUP == group ? its_reach : reach;
             }
             total = total - c0 > KNQ_LONG ? 0 : total;
-            const int most = most_of_four(total);
+            const int most = rows_max(total);
             auto fetch = [&](int c0) __attribute__((always_inline)) {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 mark[sub] = 0;
@@ -1290,7 +1284,7 @@ int launch_knn_grid(int b, int n, int m, int k, int cells, const float* query, c
     const int64_t per_cloud = tpk_ceil_div(n, KNQ_QUERIES * (KNN_THREADS / TPK_WAVE));
     if (k <= KNQ_MAX_K && queries >= KNQ_LEAST && per_cloud * b <= 0x7fffffffLL)
     {
-        auto* const kernel = k <= 8 ? &knn_grid_four_kernel<4, 8> : &knn_grid_four_kernel<8, KNQ_MAX_K>;
+        auto* const kernel = k <= 8 ? &knn_grid_four_kernel<4> : &knn_grid_four_kernel<8>;
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(per_cloud * b)), dim3(KNN_THREADS), 0, stream, n, m, k, static_cast<unsigned>(per_cloud),
                            layout, query, w, dist2, idx);
         return tpk_launch_status();

@@ -240,6 +240,12 @@ __device__ __forceinline__ int row_last(int v, int lane)
     return __builtin_amdgcn_ds_bpermute((lane | 15) * 4, v);
 }
 
+// The largest of the four rows' values (each the same in its row's lanes), in every lane.
+__device__ __forceinline__ int rows_max(int v)
+{
+    return max(max(tpk_read_lane(v, 0), tpk_read_lane(v, 16)), max(tpk_read_lane(v, 32), tpk_read_lane(v, 48)));
+}
+
 // Sum of v over the wavefront, the same value in every lane (row rotations, then the four row
 // totals added in lane order: the result does not depend on which lanes call it).
 __device__ __forceinline__ float wave_sum_f32(float v)
