@@ -65,26 +65,27 @@ int main(int argc, char** argv)
             wrong += idx[q * nsample + s] != (s < static_cast<int>(hits.size()) ? hits[s].second : -1) ||
                      dist[q * nsample + s] != (s < static_cast<int>(hits.size()) ? hits[s].first : -1.f);
     }
-    // buckets that hold points, and those that 1024 consecutive points lie in, added up
+    // buckets that hold points, and those that the consecutive points of a counting workgroup lie in, added up
     CellScale scale;
     scale.reach = bt_reach(radius);
     scale.inverse_x = 1.0f / (BT_WIDTH_X * scale.reach);
     scale.inverse_yz = 1.0f / (BT_WIDTH_YZ * scale.reach);
     const TableLayout l = table_layout(points, queries);
     std::set<uint32_t> all, near;
-    long by_1024 = 0;
+    const size_t together = points < BT_COUNT_MEDIUM ? 256 : points < BT_COUNT_LARGE ? 512 : 1024;
+    long by_group = 0;
     for (size_t i = 0; i < points; ++i)
     {
         const uint32_t bucket = bt_point_bucket(x[i * 3], x[i * 3 + 1], x[i * 3 + 2], bx[i], scale, static_cast<uint32_t>(l.buckets / BT_PARTS - 1));
         all.insert(bucket);
         near.insert(bucket);
-        if (i % 1024 == 1023 || i + 1 == points)
+        if (i % together == together - 1 || i + 1 == points)
         {
-            by_1024 += static_cast<long>(near.size());
+            by_group += static_cast<long>(near.size());
             near.clear();
         }
     }
-    printf("%ld wrong, %ld atomics, %ld buckets, %ld by 1024 points, %ld chunks\n", wrong, emulation::watched, static_cast<long>(all.size()), by_1024,
+    printf("%ld wrong, %ld atomics, %ld buckets, %ld by group, %ld chunks\n", wrong, emulation::watched, static_cast<long>(all.size()), by_group,
            static_cast<long>(l.buckets / BT_CHUNK));
     return wrong == 0 ? 0 : 5;
 }

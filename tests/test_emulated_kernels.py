@@ -49,13 +49,14 @@ def test_dense_ball_query_stays_in_bounds(ball_query_dense, clouds, points, quer
     assert done.returncode == 0, done.stdout + done.stderr
 
 
-# (radius 2: all points of a cloud in a few buckets; 0.02: hardly two in one; 12291 points: the last workgroup counts three)
+# (radius 2: all points of a cloud in a few buckets; 0.02: hardly two in one; 12291 points: the last workgroup counts three; 65537 points: 512 by a
+# workgroup, the last one a single point)
 @pytest.mark.parametrize("clouds,points,queries,nsample,radius,sort", [(1, 12291, 8192, 16, 2.0, 0), (3, 8200, 8195, 5, 0.3, 0), (1, 9000, 8192, 16, 0.02, 0),
-                                                                       (2, 8192, 700, 64, 0.2, 1)])
+                                                                       (2, 8192, 700, 64, 0.2, 1), (1, 65537, 1100, 16, 0.15, 1)])
 def test_packed_ball_query_counts_with_few_atomics(ball_query_packed, clouds, points, queries, nsample, radius, sort):
-    """In bounds and right; and however many points a bucket holds, 1024 consecutive ones that lie in it share one atomic (atomics on
-    one address wait for each other: an atomic per point took 550 us where a ball held a cloud of 100000)."""
+    """In bounds and right; and however many points a bucket holds, those of a workgroup's 256 to 1024 consecutive ones that lie in it share
+    one atomic (atomics on one address wait for each other: an atomic per point took 550 us where a ball held a cloud of 100000)."""
     done = subprocess.run([ball_query_packed] + [str(v) for v in (clouds, points, queries, nsample, radius, sort)], capture_output=True, text=True, timeout=300)
     assert done.returncode == 0, done.stdout + done.stderr
-    wrong, atomics, buckets, by_1024, chunks = (int(v) for v in re.findall(r"(\d+) (?:wrong|atomics|buckets|by 1024|chunks)", done.stdout))
-    assert wrong == 0 and atomics <= by_1024 + chunks
+    wrong, atomics, buckets, by_group, chunks = (int(v) for v in re.findall(r"(\d+) (?:wrong|atomics|buckets|by group|chunks)", done.stdout))
+    assert wrong == 0 and atomics <= by_group + chunks

@@ -54,11 +54,14 @@ constexpr float BT_MOST_HIT = 0.5f, BT_LEAST_HIT = 1.0f / 64; // of such a query
 constexpr int BT_SAMPLES = 4;                      // of its candidates, per lane, that tell how many of them lie in the ball
 constexpr int BT_HIT_STRIDE = BT_HITS + BT_GROUP + 4; // (the four queries of a wavefront read theirs at the same time: other banks)
 constexpr int BT_COUNT_THREADS = 1024;
-constexpr int BT_COUNT_SLOTS = 2 * BT_COUNT_THREADS; // of the table in LDS: every point of the workgroup may need one
 constexpr int BT_AHEAD = 3;                        // steps whose candidates are requested together (2 and 4: 1 to 3 % slower)
 constexpr unsigned BT_NO_BUCKET = 0xffffffffu;
 constexpr int BT_SCAN_THREADS = 1024;
 constexpr int BT_CHUNK = BT_SCAN_THREADS * 4;      // buckets whose places one workgroup hands out
+// Points of a counting workgroup: 256 below 65536 points, 512 below 131072, then 1024.  The more there are, the fewer atomics wait for each other
+// where cells are full; the fewer, the more compute units share a small array.  48000 / 57000 points, radius 0.09: 5.9 / 6.2 us with 256, 7.2 / 7.5
+// with 1024; 100000 points in a room of 8, radius 2: whole call 36 / 34 / 33 us; 212000, radius 0.05: 13.7 with 1024, 14 with 512.
+constexpr int64_t BT_COUNT_MEDIUM = 65536, BT_COUNT_LARGE = 131072;
 constexpr int BT_MOST_X = BT_CHUNK / 2;            // buckets of a run, at most: a run touches two chunks at most
 constexpr float BT_WIDTH_X = 0.55f, BT_WIDTH_YZ = 2.2f; // of a cell, in reaches
 
@@ -84,33 +87,35 @@ __device__ __forceinline__ uint32_t bt_point_bucket(float x, float y, float z, i
 // Bound by the atomics (16 to the nanosecond where they go to different buckets), which wait for each other where they do not, 20 to 60 ns
 // each: the workgroup counts its own points in LDS first and sends one atomic per bucket.  212000 points of four scenes, radius 0.05: 13 us,
 // and 13 with an atomic per point and lanes that share the wavefront's first bucket; 100000 points, radius 0.6 / 2 / 6 in a
-// room of 8: 8 / 4 / 5 us instead of 30 / 130 / 530; a million points 56 instead of 65 and, radius 0.5, 33 instead of 154.  (Workgroups of 512
-// points: 14 / 6 / 6 and 88; atomics at once unless a wavefront's points share the first one's bucket: 8 / 5 / 5 and 53.)
-__global__ void __launch_bounds__(BT_COUNT_THREADS)
+// room of 8: 8 / 4 / 5 us instead of 30 / 130 / 530; a million points 56 instead of 65 and, radius 0.5, 33 instead of 154.  (Atomics at once unless a
+// wavefront's points share the first one's bucket: 8 / 5 / 5 and 53.)
+template <int COUNT_THREADS>
+__global__ void __launch_bounds__(COUNT_THREADS)
     bt_count_kernel(int n, unsigned point_blocks, const float* __restrict__ x, const int64_t* __restrict__ batch_x, CellScale scale, uint32_t part_mask,
                     int* counts, int* __restrict__ ranks, int* __restrict__ placed, CloudRows rows)
 {
-    __shared__ unsigned keys[BT_COUNT_SLOTS];
-    __shared__ int shared_counts[BT_COUNT_SLOTS];
+    constexpr int SLOTS = 2 * COUNT_THREADS; // of the table in LDS: every point of the workgroup may need one
+    __shared__ unsigned keys[SLOTS];
+    __shared__ int shared_counts[SLOTS];
     if (blockIdx.x >= point_blocks)
     {
-        cloud_rows_job(rows, static_cast<int64_t>(blockIdx.x - point_blocks) * (BT_COUNT_THREADS / TPK_WAVE) + threadIdx.x / TPK_WAVE,
+        cloud_rows_job(rows, static_cast<int64_t>(blockIdx.x - point_blocks) * (COUNT_THREADS / TPK_WAVE) + threadIdx.x / TPK_WAVE,
                        threadIdx.x & (TPK_WAVE - 1));
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0)
         *placed = 0;
-    const int i = blockIdx.x * BT_COUNT_THREADS + threadIdx.x;
+    const int i = blockIdx.x * COUNT_THREADS + threadIdx.x;
     const bool has = i < n;
     const int64_t at = has ? i : 0;
     const uint32_t bucket = bt_point_bucket(x[at * 3 + 0], x[at * 3 + 1], x[at * 3 + 2], batch_x[at], scale, part_mask);
-    for (int slot = threadIdx.x; slot < BT_COUNT_SLOTS; slot += BT_COUNT_THREADS)
+    for (int slot = threadIdx.x; slot < SLOTS; slot += COUNT_THREADS)
     {
         keys[slot] = BT_NO_BUCKET;
         shared_counts[slot] = 0;
     }
     __syncthreads();
-    int slot = static_cast<int>(bucket % BT_COUNT_SLOTS), rank = 0;
+    int slot = static_cast<int>(bucket % SLOTS), rank = 0;
     if (has)
     {
         for (;;)
@@ -118,12 +123,12 @@ __global__ void __launch_bounds__(BT_COUNT_THREADS)
             const unsigned there = atomicCAS(&keys[slot], BT_NO_BUCKET, bucket);
             if (there == BT_NO_BUCKET || there == bucket)
                 break;
-            slot = (slot + 1) % BT_COUNT_SLOTS;
+            slot = (slot + 1) % SLOTS;
         }
         rank = atomicAdd(&shared_counts[slot], 1);
     }
     __syncthreads();
-    for (int s = threadIdx.x; s < BT_COUNT_SLOTS; s += BT_COUNT_THREADS)
+    for (int s = threadIdx.x; s < SLOTS; s += COUNT_THREADS)
         if (shared_counts[s] > 0)
             shared_counts[s] = atomicAdd(&counts[keys[s]], shared_counts[s]);
     __syncthreads();
@@ -788,13 +793,17 @@ int tpk_table_ball_query_partial(int64_t size_x, int64_t size_y, float radius, f
     const int n = static_cast<int>(size_x);
 
     const int64_t point_blocks = tpk_ceil_div(size_x, BT_THREADS);
-    const int64_t count_blocks = tpk_ceil_div(size_x, BT_COUNT_THREADS), row_blocks = tpk_ceil_div(size_y, BT_COUNT_THREADS);
+    const int count_threads = size_x < BT_COUNT_MEDIUM ? BT_COUNT_THREADS / 4 : size_x < BT_COUNT_LARGE ? BT_COUNT_THREADS / 2 : BT_COUNT_THREADS;
+    const int64_t count_blocks = tpk_ceil_div(size_x, count_threads), row_blocks = tpk_ceil_div(size_y, count_threads);
     const int64_t query_blocks = tpk_ceil_div(size_y, BT_THREADS / BT_GROUP);
     if (query_blocks > 0x7fffffffLL || count_blocks + row_blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(bt_clear_kernel, dim3(static_cast<unsigned>(tpk_ceil_div(l.buckets / 4, BT_THREADS))), dim3(BT_THREADS), 0, s,
                        l.buckets / 4, reinterpret_cast<int4*>(table));
-    hipLaunchKernelGGL(bt_count_kernel, dim3(static_cast<unsigned>(count_blocks + row_blocks)), dim3(BT_COUNT_THREADS), 0, s, n,
+    auto* const count_kernel = size_x < BT_COUNT_MEDIUM  ? &bt_count_kernel<BT_COUNT_THREADS / 4>
+                               : size_x < BT_COUNT_LARGE ? &bt_count_kernel<BT_COUNT_THREADS / 2>
+                                                         : &bt_count_kernel<BT_COUNT_THREADS>;
+    hipLaunchKernelGGL(count_kernel, dim3(static_cast<unsigned>(count_blocks + row_blocks)), dim3(count_threads), 0, s, n,
                        static_cast<unsigned>(count_blocks), x, batch_x, scale, part_mask, table, ranks, placed, rows);
     hipLaunchKernelGGL(bt_places_kernel, dim3(static_cast<unsigned>(l.buckets / BT_CHUNK)), dim3(BT_SCAN_THREADS), 0, s,
                        reinterpret_cast<int4*>(table), chunk_ends, placed);
