@@ -781,7 +781,8 @@ __global__ __launch_bounds__(KNN_THREADS) void knn_grid_search_kernel(int64_t qu
 // per SIMD instead of six, which spill two registers, 77 to 81 even; seven and eight spill 14 and 33 and take 82 and more.)  k = 32, with 16
 // points a lane, was 8 to 13 % faster in even clouds and 10 to 20 % slower in clusters.
 // Built, measured, dropped: queries that are given up, or have hundreds of points to walk through or are far away, handed to a launch of
-// their own with a wavefront a query (8 x 4099, k = 16, even 30, clusters of sigma 0.003 80 to 105, far 53).
+// their own with a wavefront a query (8 x 4099, k = 16, even 30, clusters of sigma 0.003 80 to 105, far 53); queries that are given up
+// shared among a workgroup's wavefronts, behind a barrier (8 x 16384, k = 4 / 16, even 67 / 79, queries over 3 times the width 136 / 169).
 constexpr int KNQ_MAX_K = 16;
 // Queries from which on: with fewer the four wait for each other while wavefronts' places are empty - at six per SIMD there are 6144, 24576
 // queries -, and what uneven clouds and queries outside lose outweighs what even ones gain.  k = 4 / 16, time over a wavefront a query's, even,
