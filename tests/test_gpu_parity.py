@@ -1044,6 +1044,23 @@ def test_ball_query_packed_scans_of_several_queries(tpk, oracle, dev, sizes, rad
     np.testing.assert_array_equal(_np(dist), wd)
 
 
+# (radius 0.1: about 130 hits and 1000 candidates, thousands near the crowd, walked for by whole wavefronts, whose list is full after 81 hits; with 65
+# slots by sixteen lanes; 0.14: more are scanned for; 0.05: about a hundred candidates)
+@pytest.mark.parametrize("radius,nsample", [(0.1, 64), (0.1, 63), (0.1, 1), (0.1, 16), (0.14, 64), (0.08, 64), (0.1, 65), (0.05, 8)])
+def test_ball_query_packed_walks_by_whole_wavefronts(tpk, oracle, dev, radius, nsample):
+    g = torch.Generator().manual_seed(nsample)
+    n = torch.tensor([33000, 5000])
+    b = torch.arange(2).repeat_interleave(n)
+    x = torch.rand(b.numel(), 3, generator=g)
+    x[30000:33000] = 0.3 + 0.1 * torch.rand(3000, 3, generator=g)  # (crowded cells, the last rows of the cloud)
+    pick = torch.sort(torch.randperm(b.numel(), generator=g)[:8501])[0]
+    y, by = (x[pick] + 0.05 * (torch.rand(8501, 3, generator=g) < 0.1)).contiguous(), b[pick].contiguous()
+    idx, dist = tpk.ball_query(radius, nsample, x.to(dev), y.to(dev), mode="partial_dense", batch_x=b.to(dev), batch_y=by.to(dev))
+    wi, wd = oracle.ball_query_partial_dense(radius, nsample, x.numpy(), y.numpy(), b.numpy(), by.numpy())
+    np.testing.assert_array_equal(_np(idx), wi)
+    np.testing.assert_array_equal(_np(dist), wd)
+
+
 # (a few queries of 65536 points or more walk over bins: radius 0.03 a few bins, 0.3 more than 64 of a window, 1e25 every point; equal points)
 @pytest.mark.parametrize("radius,nsample", [(0.03, 64), (0.1, 16), (0.3, 1), (0.3, 33), (1e25, 5), (0.0, 4)])
 @pytest.mark.parametrize("sizes,queries", [([65536], 1), ([30000, 200, 40001], 500), ([70000], 1093), ([66000], 1031), ([66000], 1032)])
@@ -1061,8 +1078,8 @@ def test_ball_query_packed_sorted_for_few_queries(tpk, oracle, dev, sizes, queri
 
 
 # (most: what the table may take, over bins in the smaller workspace.  Radius 2 and 6 with 16 slots: 1.0 times; an atomic per point and one scan
-# after the other took 5 and 24.  Radius 1.4, a room of which most lies on two planes: 1.1 / 1.3, and 1.8 where long walks of a single query were
-# taken for as short as four together; radius 2 with 64 slots: 1.1, and 2.0.)
+# after the other took 5 and 24.  Radius 1.4, a room of which most lies on two planes: 1.1, and 1.8 where long walks were sixteen lanes' and
+# scans of several queries left the last one with the others' tests; radius 2 with 64 slots: 1.1, and 2.0.)
 @pytest.mark.parametrize("radius,nsample,most", [(2.0, 16, 2.5), (6.0, 16, 2.5), (1.4, 16, 1.5), (2.0, 64, 1.5)])
 def test_ball_query_packed_of_large_balls_is_not_left_behind(dev, radius, nsample, most):
     """Balls that hold a large part of their cloud: the call over the table takes about as long as the one over bins."""
