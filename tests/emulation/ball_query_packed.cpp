@@ -65,7 +65,8 @@ int main(int argc, char** argv)
             wrong += idx[q * nsample + s] != (s < static_cast<int>(hits.size()) ? hits[s].second : -1) ||
                      dist[q * nsample + s] != (s < static_cast<int>(hits.size()) ? hits[s].first : -1.f);
     }
-    // buckets that hold points, and those that the consecutive points of a counting workgroup lie in, added up
+    // buckets that hold points, and those that the consecutive points of a counting workgroup lie in, added up; a point each where hardly two of
+    // them share one
     CellScale scale;
     scale.reach = bt_reach(radius);
     scale.inverse_x = 1.0f / (BT_WIDTH_X * scale.reach);
@@ -81,7 +82,8 @@ int main(int argc, char** argv)
         near.insert(bucket);
         if (i % together == together - 1 || i + 1 == points)
         {
-            by_group += static_cast<long>(near.size());
+            const size_t in_group = i % together + 1;
+            by_group += static_cast<long>(in_group < 64 || near.size() * 4 > in_group * 3 ? in_group : near.size());
             near.clear();
         }
     }

@@ -208,6 +208,16 @@ inline void __syncthreads()
         while (emulation::barrier_turn == turn)
             emulation::yield();
 }
+inline int __syncthreads_or(int p)
+{
+    static int any;
+    __syncthreads();
+    any = 0;
+    __syncthreads();
+    any |= p;
+    __syncthreads();
+    return any;
+}
 inline unsigned long long __ballot(bool p)
 {
     const uint64_t* all = emulation::exchange(p);

@@ -58,6 +58,10 @@ constexpr int BT_ALONE_AHEAD = 3;                  // steps of it whose candidat
 constexpr int BT_HIT_STRIDE = BT_HITS + BT_GROUP + 4; // (the four queries of a wavefront read theirs at the same time: other banks)
 constexpr int BT_COUNT_THREADS = 1024;
 constexpr int BT_AHEAD = 2;                        // steps whose candidates are requested together (3: 300000 queries, radius 0.1, 87 / 110 us instead of 82 / 96)
+// Points of a wavefront that share the buckets of four others, from which on a small array's workgroup counts in LDS first.  (Always: 9000 and
+// 24000 points, radius 0.3 in rooms of 8, counting 6.2 and 6.7 us instead of 3.8 and 5; 2: 24000 points, radius 0.1 to 0.6, calls of 21 to 26 us
+// 0.5 to 1.6 longer; never, see bt_count_kernel.)
+constexpr int BT_SHARED = 4;
 constexpr unsigned BT_NO_BUCKET = 0xffffffffu;
 constexpr int BT_SCAN_THREADS = 1024;
 constexpr int BT_CHUNK = BT_SCAN_THREADS * 4;      // buckets whose places one workgroup hands out
@@ -112,6 +116,23 @@ __global__ void __launch_bounds__(COUNT_THREADS)
     const bool has = i < n;
     const int64_t at = has ? i : 0;
     const uint32_t bucket = bt_point_bucket(x[at * 3 + 0], x[at * 3 + 1], x[at * 3 + 2], batch_x[at], scale, part_mask);
+    if constexpr (COUNT_THREADS < BT_COUNT_THREADS / 2)
+    {
+        // Small arrays: how many of a wavefront's points share the buckets of four of them?
+        int sharing = 0;
+#pragma unroll
+        for (int probe = 0; probe < TPK_WAVE; probe += TPK_WAVE / 4)
+        {
+            const uint32_t of_probe = static_cast<uint32_t>(tpk_read_lane(static_cast<int>(bucket), probe));
+            sharing += __builtin_popcountll(__ballot(has && bucket == of_probe));
+        }
+        if (__syncthreads_or(sharing >= 4 + BT_SHARED) == 0)
+        {
+            if (has)
+                ranks[i] = atomicAdd(&counts[bucket], 1);
+            return;
+        }
+    }
     for (int slot = threadIdx.x; slot < SLOTS; slot += COUNT_THREADS)
     {
         keys[slot] = BT_NO_BUCKET;
