@@ -65,8 +65,8 @@ int main(int argc, char** argv)
             wrong += idx[q * nsample + s] != (s < static_cast<int>(hits.size()) ? hits[s].second : -1) ||
                      dist[q * nsample + s] != (s < static_cast<int>(hits.size()) ? hits[s].first : -1.f);
     }
-    // buckets that hold points, and those that the consecutive points of a counting workgroup lie in, added up; a point each where hardly two of
-    // them share one
+    // Buckets that hold points, and those that the consecutive points of a counting workgroup lie in, added up.  A small array's workgroup may send an
+    // atomic per point where less than 4 of a wavefront's share the buckets of four others - 6 would in 43 buckets, a sixth of 256 points.
     CellScale scale;
     scale.reach = bt_reach(radius);
     scale.inverse_x = 1.0f / (BT_WIDTH_X * scale.reach);
@@ -83,7 +83,7 @@ int main(int argc, char** argv)
         if (i % together == together - 1 || i + 1 == points)
         {
             const size_t in_group = i % together + 1;
-            by_group += static_cast<long>(in_group < 64 || near.size() * 4 > in_group * 3 ? in_group : near.size());
+            by_group += static_cast<long>(together == 256 && (in_group < 64 || near.size() * 6 > in_group) ? in_group : near.size());
             near.clear();
         }
     }

@@ -55,7 +55,7 @@ def test_dense_ball_query_stays_in_bounds(ball_query_dense, clouds, points, quer
                                                                        (2, 8192, 700, 64, 0.2, 1), (1, 65537, 1100, 16, 0.15, 1)])
 def test_packed_ball_query_counts_with_few_atomics(ball_query_packed, clouds, points, queries, nsample, radius, sort):
     """In bounds and right; and however many points a bucket holds, those of a workgroup's 256 to 1024 consecutive ones that lie in it share
-    one atomic, in a small array unless hardly two of them lie in one (atomics on one address wait for each other: an atomic per point took 550 us where a ball held a cloud of 100000)."""
+    one atomic, in a small array where a bucket holds six of them (atomics on one address wait for each other: an atomic per point took 550 us where a ball held a cloud of 100000)."""
     done = subprocess.run([ball_query_packed] + [str(v) for v in (clouds, points, queries, nsample, radius, sort)], capture_output=True, text=True, timeout=300)
     assert done.returncode == 0, done.stdout + done.stderr
     wrong, atomics, buckets, by_group, chunks = (int(v) for v in re.findall(r"(\d+) (?:wrong|atomics|buckets|by group|chunks)", done.stdout))
