@@ -2287,6 +2287,59 @@ def test_cell_search_outliers(tpk, oracle, dev):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
+@pytest.mark.parametrize("n,m", [(513, 600), (1024, 8191), (5000, 16385), (20000, 20000)])
+@pytest.mark.parametrize("kind", ["even", "itself", "nearly itself", "nearly equal", "lattice", "crowded", "scan", "outliers", "far", "one of many", "tiny",
+                                  "not finite"])
+def test_chamfer_on_the_matrix_cores(dev, kind, n, m):
+    """The search over cells against the scan of all pairs, bit for bit: clouds whose queries the products answer, leave to the pass
+    for equal minima (a few of a wavefront, "nearly equal") or to the exact scan (lattices, wide cells, cells far away, units out of range)."""
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_chamfer_fwd_workspace_bytes.restype = ctypes.c_size_t
+    g = torch.Generator().manual_seed(n + m)
+    clouds = [torch.rand(2, count, 3, generator=g) for count in (n, m)]
+    first = lambda count: clouds[1][:, torch.arange(count) % m]
+    if kind == "itself":
+        clouds[0] = first(n).clone()
+    elif kind == "nearly itself":
+        clouds[0] = first(n) + 1e-5 * torch.randn(2, n, 3, generator=g)
+    elif kind == "nearly equal":  # every point has a twin a few units in the last place away
+        clouds[1][:, m // 2 : 2 * (m // 2)] = clouds[1][:, : m // 2] * (1.0 + 2.0 ** -22)
+    elif kind == "lattice":
+        clouds = [torch.floor(c * 16) / 16 for c in clouds]
+    elif kind == "crowded":
+        clouds = [torch.where(torch.rand(c.shape[:2] + (1,), generator=g) < 0.6, c * 1e-3 + 0.4, c) for c in clouds]
+    elif kind == "scan":  # as a laser sees a floor
+        far = [1.5 * (50 / 1.5) ** c[..., 0] for c in clouds]
+        clouds = [torch.stack([r * torch.cos(6.2832 * c[..., 1]), r * torch.sin(6.2832 * c[..., 1]), 0.02 * c[..., 2] - 1.7], 2) for r, c in zip(far, clouds)]
+    elif kind == "outliers":
+        clouds = [torch.where(torch.rand(c.shape[:2] + (1,), generator=g) < 0.05, 100 * (c - 0.5), c) for c in clouds]
+    elif kind == "far":
+        clouds[0] = clouds[0] + torch.tensor([300.0, -2.0, 40.0])
+    elif kind == "one of many":
+        clouds[1][:] = clouds[1][:, :1]
+    elif kind == "tiny":
+        clouds = [c * 1e-17 for c in clouds]
+    elif kind == "not finite":
+        clouds[0][:, 7::97, 1] = float("nan")
+        clouds[1][:, 3::89, 2] = float("inf")
+    a, b = (c.contiguous().to(dev) for c in clouds)
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    results = []
+    for nbytes in (lib.tpk_chamfer_fwd_workspace_bytes(2, n, m), 0):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+        out = [torch.full((2, k), -1, dtype=t, device=dev) for t in (torch.float32, torch.int32) for k in (n, m)]
+        st = lib.tpk_chamfer_fwd_f32(2, n, m, pointer(a), pointer(b), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None)
+        assert st == 0
+        torch.cuda.synchronize()
+        results.append([t.cpu() for t in out])
+    for cells, pairs in zip(*results):
+        assert torch.equal(cells, pairs)
+
+
 def test_chamfer_gradcheck_double(tpk, dev):
     # reference test/test_chamfer_dist.py:20-25
     from torch.autograd import gradcheck

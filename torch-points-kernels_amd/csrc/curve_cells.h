@@ -16,7 +16,11 @@ constexpr int NG_CELL = 64;           // points per cell = lanes of a wavefront
 constexpr int NG_SORT_THREADS = 1024;
 constexpr int CURVE_STAGED = 4096;    // records of a window's part that are put in order in LDS (64 KB)
 constexpr int CURVE_PARTS = CURVE_MAX_POINTS / CURVE_STAGED; // parts of a window, at most
-constexpr int NG_BOX = 10;            // float4 per cell: box of the cell, then of its four runs of 16 points
+constexpr int NG_BOX = 2;             // float4 per cell: lowest and highest corner of its box
+constexpr int NG_RUN_BOXES = 8;       // and of the boxes of its four runs of 16 points, which stand behind the boxes of all cells: the
+                                      // searches read those of 64 cells at a time, a cell per lane (160 bytes apart, with the runs' boxes
+                                      // between them, Chamfer's search lost a third of a wavefront's time on them)
+constexpr int NG_CELL_BOXES = NG_BOX + NG_RUN_BOXES;
 
 // A set of points to be ordered: `total` points in clouds of `cloud_points` consecutive points,
 // every cloud cut into windows of `stride` consecutive points (the last window of a cloud may be
@@ -32,7 +36,7 @@ struct PointSet
     int64_t cloud_points;
     int stride;
     float4* sorted;       // [windows][cells * 64]
-    float4* boxes;        // [windows][cells][NG_BOX]: (lo.xyz, -), (hi.xyz, -) of the cell and of its quarters; or nullptr
+    float4* boxes;        // [windows][cells][NG_BOX]: (lo.xyz, -), (hi.xyz, -) of the cells, then [windows][cells][NG_RUN_BOXES]: of their quarters; or nullptr
     int* bin_ends;        // optional [windows][CURVE_BINS]: end of every bin of the counting sort
     float4* grid;         // optional [windows][2]: origin and scale of the window's 64^3 grid
     int* wide_first;      // optional (with boxes) [windows][cells]: the cells of each of the window's parts (curve_parts()), those
@@ -104,6 +108,7 @@ __device__ __forceinline__ void curve_cells_part(const PointSet& set, int64_t wi
     const int64_t* __restrict__ group = set.group ? set.group + start : nullptr;
     float4* __restrict__ sorted = set.sorted + window * cells * NG_CELL;
     float4* __restrict__ boxes = set.boxes ? set.boxes + window * cells * NG_BOX : nullptr;
+    float4* __restrict__ quarters = set.boxes ? set.boxes + set_windows(set) * cells * NG_BOX + window * cells * NG_RUN_BOXES : nullptr;
     const int tid = threadIdx.x;
     const int lane = tid & (TPK_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / TPK_WAVE);
@@ -395,8 +400,8 @@ __device__ __forceinline__ void curve_cells_part(const PointSet& set, int64_t wi
             for (int r = 0; r < 4; ++r)
             {
                 const int* const run_box = runs + ((c - cell_lo) * 4 + r) * 6;
-                boxes[c * NG_BOX + 2 + r * 2 + 0] = make_float4(as_lo(run_box[0]), as_lo(run_box[1]), as_lo(run_box[2]), 0.f);
-                boxes[c * NG_BOX + 2 + r * 2 + 1] = make_float4(as_hi(run_box[3]), as_hi(run_box[4]), as_hi(run_box[5]), 0.f);
+                quarters[c * NG_RUN_BOXES + r * 2 + 0] = make_float4(as_lo(run_box[0]), as_lo(run_box[1]), as_lo(run_box[2]), 0.f);
+                quarters[c * NG_RUN_BOXES + r * 2 + 1] = make_float4(as_hi(run_box[3]), as_hi(run_box[4]), as_hi(run_box[5]), 0.f);
 #pragma unroll
                 for (int a = 0; a < 3; ++a)
                 {

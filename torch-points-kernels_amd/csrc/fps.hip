@@ -1402,7 +1402,7 @@ CellLayout cell_layout(int b, int n)
     const size_t all = static_cast<size_t>(b) * l.cells;
     l.sorted = 0;
     l.boxes = up(all * NG_CELL * sizeof(float4));
-    l.temp = up(l.boxes + all * NG_BOX * sizeof(float4));
+    l.temp = up(l.boxes + all * NG_CELL_BOXES * sizeof(float4));
     l.coarse = up(l.temp + all * NG_CELL * sizeof(float));
     l.total = fps_coarse_first(b, n) ? up(l.coarse + coarse_layout(static_cast<int64_t>(b) * n).total) : l.coarse;
     return l;

@@ -15,7 +15,8 @@
 // distances" - what a serial first-strictly-smaller scan returns - is enforced explicitly: the
 // scan keeps the minimum and the first group of 8 candidates that reached it, and flags a lane
 // when another group reaches the same value; flagged lanes (duplicated points, lattices) take
-// an extra pass that collects the lowest index among all candidates at that distance.
+// an extra pass that collects the lowest index among all candidates at that distance.  Chamfer's
+// scan runs on the matrix cores and asks for that pass where two candidates are too close to tell.
 //
 // Workspace per cloud: 16 bytes per point (x, y, z, original index) padded to whole cells, and
 // 160 bytes per cell (its box and those of its four runs of 16 points).  The curve ordering works
@@ -64,16 +65,16 @@ struct Nearest
 
 // Scans candidate cell `cell` for the 64 queries of the wavefront.  `stage` is the wavefront's
 // own 64-entry LDS buffer, through which every lane sees every candidate (broadcast reads).
-__device__ __forceinline__ void scan_cell(const float4* __restrict__ cand, const float4* __restrict__ boxes,
+__device__ __forceinline__ void scan_cell(const float4* __restrict__ cand, const float4* __restrict__ runs,
                                           int cell, float4* stage, int lane, float qx, float qy, float qz,
                                           Nearest& s TPK_WORK_PARAM)
 {
     stage[lane] = cand[cell * NG_CELL + lane];
     // (the boxes of the cell's four runs are requested together with its candidates: one wait, not five)
-    float4 quarter[NG_BOX - 2];
+    float4 quarter[NG_RUN_BOXES];
 #pragma unroll
-    for (int i = 0; i < NG_BOX - 2; ++i)
-        quarter[i] = boxes[cell * NG_BOX + 2 + i];
+    for (int i = 0; i < NG_RUN_BOXES; ++i)
+        quarter[i] = runs[cell * NG_RUN_BOXES + i];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); // LDS serves a wavefront's requests in order
 #pragma unroll
     for (int run = 0; run < NG_CELL / (2 * NG_CHUNK); ++run)
@@ -142,10 +143,148 @@ __device__ __forceinline__ void scan_cell_few(const float4* __restrict__ cand, i
     }
 }
 
+// ---- Chamfer's scan on the matrix cores --------------------------------------------------
+// |p - q|^2 = |p|^2 - 2 p.q + |q|^2 is a product over 16 slots once every number is given as two halves, so one
+// v_mfma_f32_32x32x16_f16 forms 32 x 32 distances.  They are not the distances the search returns: they say which
+// eight candidates hold a query's answer, and those are evaluated as ever.  Coordinates are taken relative to the centre of
+// the queries' box and scaled by a power of two; in these units everything the search needs lies within 1024 of the
+// centre along every axis, and candidates further off than 16384 count as that far away.
+//
+// A row of the product: x, y (high halves), x, y (low), z, |p|^2 (high), z, |p|^2 (low), then x, y (high), x, y (low), z, |p|^2
+// (high), 1, 1 against a query's -2x, -2y (high, twice), (-2z, 2^14) (high, twice), -2x, -2y (low, twice), (-2z, 0) (low), |q|^2.
+//
+// The error of a product, in units of 2^-20 (|p| + |q|)^2: two halves hold 22 bits, which costs 2 p.q 0.38 and the squares, formed in
+// float, 0.44; the frame 0.2; the sum of 16 products 0.25 (2^-22 of the sum of their magnitudes: twice the 2^-23.05 that a million
+// products reached, and halves below the normal range are not flushed).  With the two bits that a smallest product gives up for
+// its place that is below 2^-17 (|q|^2 + |p - q|^2), as (|p| + |q|)^2 <= 5 |q|^2 + 5 |p - q|^2, and 2^-6 where a low half is below the normal
+// range.  A query for which the eight and some other candidate are closer together than that (one in 2000 of even clouds, one in
+// 500 on a sphere) goes to the pass for equal minima; where more than MX_PASS of a wavefront's do, the exact scan above answers them, a
+// search of its own that starts with what is known: serving 64 of them one at a time took 2.8 times as long on clouds with outliers.
+//
+// What bounds it: the issue of vector instructions, ~105 for 64 x 64 pairs (22 to form the halves, 60 for the minima) where the
+// exact scan takes ten per candidate.  32 x 16384 points of noisy surfaces: search 121 -> 58 us, whole call 144 -> 86; uniform 143 -> 98, eight
+// clusters 176 -> 89; 8 x 1024 against 16384 109 -> 53, 2 x 60000 159 -> 102, one cloud of 160000 455 -> 281; laser scans of 8 x 16384
+// 266 -> 254, of 2 x 60000 821 -> 917 (cells that are wide for their points' distances leave half of the queries over).
+// Taken back: minima of four candidates (24 more instructions per scan, 12 % slower), whole wavefronts by the exact scan where many
+// queries are left over (laser scans 30 % slower than without the matrix cores).
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+
+constexpr float MX_FAR = 16384.f;          // 2^14: candidates are clamped to this; also the factor |p|^2 and |q|^2 are kept divided by
+constexpr float MX_LIMIT = 134217728.f;    // 2^27: a squared distance that no clamped candidate can have
+constexpr float MX_NEAR = 8.f;             // largest distance of the first cell, in extents of its box and the queries'
+constexpr float MX_ERROR = 0x1p-17f;       // of |q|^2 and of a product (above)
+// A wavefront is left to the exact scan at once where for more than MX_MANY queries two groups of the first cell are within MX_CLOSE
+// errors: normal distributions scaled point by point by e^0 .. e^-12, 8 x 16384: 926 us against 981 with 32 queries (873 without the matrix cores).
+constexpr float MX_CLOSE = 16.f;
+constexpr int MX_MANY = 16;
+constexpr int MX_PASS = 20;                // (12: laser scans of 32 x 4096 106 us against 91, e^-4 2 x 60000 1470 against 930; 32: a tail of slow wavefronts)
+
+// Two halves that add up to v: the rounded value, and what is left of it, rounded.
+// (`minus_one` as a variable: the compiler then takes three instructions for a pair, v_fma_mix among them, instead of nine)
+__device__ __forceinline__ void split_half(float a, float b, float minus_one, half2_t& high, half2_t& low)
+{
+    high = half2_t{static_cast<_Float16>(a), static_cast<_Float16>(b)};
+    low = half2_t{static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high.x), minus_one, a)),
+                  static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high.y), minus_one, b))};
+}
+
+// Operands of two tiles of 32 points, one point per lane: lanes 0 .. 31 of a tile hold slots 0 .. 7 of its points, the others slots 8 .. 15.
+__device__ __forceinline__ void tile_operands(const half2_t (&first)[4], const half2_t (&second)[4], half8_t (&tile)[2])
+{
+    uint4_t t[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        const auto swapped = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, first[i]),
+                                                              __builtin_bit_cast(unsigned, second[i]), false, false);
+        t[0][i] = swapped[0];
+        t[1][i] = swapped[1];
+    }
+    tile[0] = __builtin_bit_cast(half8_t, t[0]);
+    tile[1] = __builtin_bit_cast(half8_t, t[1]);
+}
+
+// v of the two tiles of 32 queries as the products leave them (lane l: query l % 32, the candidates of half l / 32) -> of
+// query `lane` (query 32 j + i stands in lane 32 j + i), of either half of the candidates.
+__device__ __forceinline__ void by_query(int tile0, int tile1, int& half0, int& half1)
+{
+    const auto swapped = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(tile0), static_cast<unsigned>(tile1), false, false);
+    half0 = static_cast<int>(swapped[0]);
+    half1 = static_cast<int>(swapped[1]);
+}
+
+// What a lane knows of one query and half of the candidates: the smallest and the second smallest of the minima of eight
+// candidates (bit patterns; a negative one stands for a distance below the error), the place of the eight in their
+// cell in the two lowest bits, and the smallest one's cell.
+struct MatrixNearest
+{
+    int m1, m2, cell;
+};
+
+__device__ __forceinline__ void take_products(const float16_t& d, int tile, MatrixNearest& s)
+{
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+    {
+        int eight = __float_as_int(d[8 * q]);
+#pragma unroll
+        for (int r = 1; r < 8; ++r)
+            eight = min(eight, __float_as_int(d[8 * q + r]));
+        const int v = (eight & ~3) | (tile * 2 + q);
+        s.m2 = __float_as_int(__builtin_amdgcn_fmed3f(__int_as_float(s.m1), __int_as_float(s.m2), __int_as_float(v)));
+        s.m1 = min(s.m1, v);
+    }
+    // (the second smallest are not looked at before the search ends: without this the compiler keeps what they follow from in
+    // registers beyond the scan, 32 of them)
+    asm volatile("" : "+v"(s.m2));
+}
+
+// Units of a wavefront's search: point * scale + offset.
+struct MatrixFrame
+{
+    float scale, ox, oy, oz, minus_one;
+};
+
+// (`want`: the queries that ask for the cell; a tile of 32 queries, neighbours on the curve, of which none does is left out)
+__device__ __forceinline__ void matrix_scan(const float4* __restrict__ cand, int cell, unsigned long long want, int lane, const MatrixFrame& f,
+                                            const half8_t (&queries)[2], MatrixNearest (&s)[2])
+{
+    const float4 p = cand[cell * NG_CELL + lane];
+    // (a padding candidate, infinitely far away, and one that is not a number count as far away)
+    const float x = __builtin_amdgcn_fmed3f(__builtin_fmaf(p.x, f.scale, f.ox), -MX_FAR, MX_FAR);
+    const float y = __builtin_amdgcn_fmed3f(__builtin_fmaf(p.y, f.scale, f.oy), -MX_FAR, MX_FAR);
+    const float z = __builtin_amdgcn_fmed3f(__builtin_fmaf(p.z, f.scale, f.oz), -MX_FAR, MX_FAR);
+    const float square = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z)) * (1.f / MX_FAR);
+    half2_t xy_high, xy_low, zs_high, zs_low;
+    split_half(x, y, f.minus_one, xy_high, xy_low);
+    split_half(z, square, f.minus_one, zs_high, zs_low);
+    const half2_t scale_slots = half2_t{static_cast<_Float16>(MX_FAR), static_cast<_Float16>(MX_FAR)};
+    half8_t tiles[2];
+    tile_operands({xy_high, xy_low, zs_high, zs_low}, {xy_high, xy_low, zs_high, scale_slots}, tiles);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+    {
+        if (static_cast<unsigned>(want >> (32 * j)) == 0)
+            continue;
+        const int before = s[j].m1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+        {
+            const float16_t d = __builtin_amdgcn_mfma_f32_32x32x16_f16(tiles[i], queries[j], float16_t{}, 0, 0, 0);
+            take_products(d, i, s[j]);
+        }
+        s[j].cell = s[j].m1 != before ? cell : s[j].cell;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // One wavefront = the 64 queries of one cell.  Logical wavefront number (after the die-local
 // block mapping) = cloud * (cells1 + cells2) + cell; the cells of cloud 1 query cloud 2 and
 // write dist1 / idx1, those of cloud 2 the other way round.
-__global__ __launch_bounds__(NG_SCAN_THREADS) void chamfer_grid_kernel(
+__global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
     int n, int m, int cells1, int cells2, int clouds, const float4* __restrict__ sorted1,
     const float4* __restrict__ sorted2, const float4* __restrict__ boxes1,
     const float4* __restrict__ boxes2, float* __restrict__ dist1, float* __restrict__ dist2,
@@ -215,6 +354,8 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void chamfer_grid_kernel(
     const float4* __restrict__ qbox = (second ? boxes2 : boxes1) + static_cast<int64_t>(cloud) * qcells * NG_BOX;
     const float4* __restrict__ cpts = (second ? sorted1 : sorted2) + static_cast<int64_t>(cloud) * ccells * NG_CELL;
     const float4* __restrict__ cbox = (second ? boxes1 : boxes2) + static_cast<int64_t>(cloud) * ccells * NG_BOX;
+    const float4* __restrict__ cruns = (second ? boxes1 : boxes2) + static_cast<int64_t>(clouds) * ccells * NG_BOX +
+                                       static_cast<int64_t>(cloud) * ccells * NG_RUN_BOXES;
     float* __restrict__ dout = (second ? dist2 : dist1) + static_cast<int64_t>(cloud) * qcount;
     int32_t* __restrict__ iout = (second ? idx2 : idx1) + static_cast<int64_t>(cloud) * qcount;
     float4* const stage = stages[wave];
@@ -228,10 +369,14 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void chamfer_grid_kernel(
         return; // a cell without points (the last window of a cloud may have some)
     const float4 qlo = qbox[qcell * NG_BOX + 0], qhi = qbox[qcell * NG_BOX + 1];
 
+    const int groups = (ccells + NG_CELL - 1) / NG_CELL;
+    const bool real = qindex != 0x7FFFFFFF;
+    float best = __builtin_inff();
+    int bi = 0x7FFFFFFF;
     // Box distances to all candidate cells, kept in the wavefront's LDS row (lane l computes
     // cells l, 64 + l, ...); +inf marks a cell that does not exist or has been scanned.
-    const int groups = (ccells + NG_CELL - 1) / NG_CELL;
     unsigned seed_key = 0xFFFFFFFFu;
+#pragma unroll 4 // (the boxes of four groups on their way at a time)
     for (int g = 0; g < groups; ++g)
     {
         const int c = g * NG_CELL + lane;
@@ -249,93 +394,240 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void chamfer_grid_kernel(
         const unsigned key = (static_cast<unsigned>(__float_as_int(centre)) & ~63u) | static_cast<unsigned>(g);
         seed_key = valid && lb < __builtin_inff() && key < seed_key ? key : seed_key;
     }
+    const unsigned lowest = wave_min_u32(seed_key);
+    int seed = static_cast<int>(lowest & 63u) * NG_CELL + __builtin_ctzll(__ballot(seed_key == lowest));
+    if (seed >= ccells) // no lane had a usable key (NaN boxes)
+        seed = 0;
+
+    // The units of the matrix scan: 512 to 1024 for the largest distance, along one axis, from the centre of the queries' box
+    // to their own and the first cell's faces (a query's answer is at most twice that away from its query).  Where the
+    // first cell is far away for its size and that of the queries' box, all its points are about equally distant and
+    // the products could not tell them apart.
+    MatrixFrame frame;
+    bool matrix;
+    {
+        const float4 slo = cbox[seed * NG_BOX + 0], shi = cbox[seed * NG_BOX + 1];
+        const float cx = 0.5f * (qlo.x + qhi.x), cy = 0.5f * (qlo.y + qhi.y), cz = 0.5f * (qlo.z + qhi.z);
+        const float own = fmaxf(fmaxf(qhi.x - cx, qhi.y - cy), qhi.z - cz);
+        const float extent = fmaxf(own, 0.5f * fmaxf(fmaxf(shi.x - slo.x, shi.y - slo.y), shi.z - slo.z));
+        const float radius = fmaxf(fmaxf(fmaxf(fabsf(slo.x - cx), fabsf(shi.x - cx)), fmaxf(fabsf(slo.y - cy), fabsf(shi.y - cy))),
+                                   fmaxf(fmaxf(fabsf(slo.z - cz), fabsf(shi.z - cz)), own));
+        const int exponent = (__float_as_int(radius) >> 23) - 127;
+        frame.scale = __int_as_float((127 + 9 - exponent) << 23);
+        frame.ox = -cx * frame.scale;
+        frame.oy = -cy * frame.scale;
+        frame.oz = -cz * frame.scale;
+        frame.minus_one = to_vector_register(-1.f);
+        matrix = radius >= 8.9e-16f && radius <= 1.1e15f && radius <= MX_NEAR * extent; // (false for what is not a number)
+    }
+    float x = __builtin_fmaf(qx, frame.scale, frame.ox), y = __builtin_fmaf(qy, frame.scale, frame.oy), z = __builtin_fmaf(qz, frame.scale, frame.oz);
+    matrix = matrix && __ballot(real && !(fabsf(x) <= 1100.f && fabsf(y) <= 1100.f && fabsf(z) <= 1100.f)) == 0;
     Nearest s;
-    s.best = qindex == 0x7FFFFFFF ? -1.f : __builtin_inff(); // (a padding lane never asks for a scan)
+    s.best = real ? __builtin_inff() : -1.f; // (a padding lane never asks for a scan)
     s.chunk = 0;
     s.tie = false;
+    bool ask = real; // left to the exact scan
+    bool tie = false; // left to the pass behind it
+    float reach = __builtin_inff();
+    if (matrix)
     {
-        const unsigned lowest = wave_min_u32(seed_key);
-        int seed = static_cast<int>(lowest & 63u) * NG_CELL + __builtin_ctzll(__ballot(seed_key == lowest));
-        if (seed >= ccells) // no lane had a usable key (NaN boxes)
-            seed = 0;
-        scan_cell(cpts, cbox, seed, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
-        if (lane == (seed & (NG_CELL - 1)))
-            lows[seed] = __builtin_inff();
-    }
-
-    // First the cells whose boxes overlap the queries' box - they hold nearly all the answers -
-    // then whatever the worst answer still admits.
-    for (int phase = 0; phase < 2; ++phase)
-        for (int g = 0; g < groups; ++g)
+        x = real ? x : 0.f;
+        y = real ? y : 0.f;
+        z = real ? z : 0.f;
+        const float square = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z));
+        const float own_error = __builtin_fmaf(square, MX_ERROR, 0.0625f);
+        const float unit = 1.f / (frame.scale * frame.scale);
+        const float reach_factor = real ? (1.f + MX_ERROR) * unit : 0.f, reach_error = real ? own_error * unit : -1.f;
+        half8_t queries[2];
         {
-            const float lw = lows[g * NG_CELL + lane];
-            float bound = __int_as_float(wave_max_i32(__float_as_int(s.best)));
-            unsigned long long live =
-                __ballot(lw < __builtin_inff() && (phase == 0 ? lw == 0.f : lw * NG_MARGIN <= bound));
-            while (live != 0)
-            {
-                const int bit = __builtin_ctzll(live);
-                const int c = g * NG_CELL + bit;
-                live &= live - 1;
-                const float lb = point_box_dist2(qx, qy, qz, cbox[c * NG_BOX + 0], cbox[c * NG_BOX + 1]);
-                const unsigned long long want = __ballot(lb * NG_MARGIN <= s.best);
-                // scanned, or no lane can improve here now - and answers only get better: never again
-                if (lane == bit)
-                    lows[c] = __builtin_inff();
-                if (want == 0)
-                    continue;
-                if (__builtin_popcountll(want) <= NG_FEW)
-                    scan_cell_few(cpts, c, want, lane, qx, qy, qz, s TPK_WORK_ARG);
-                else
-                    scan_cell(cpts, cbox, c, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
-                if (phase)
+            half2_t xy_high, xy_low, z_high, z_low, s_high, s_low;
+            split_half(-2.f * x, -2.f * y, frame.minus_one, xy_high, xy_low);
+            split_half(-2.f * z, 0.f, frame.minus_one, z_high, z_low);
+            split_half(square * (1.f / MX_FAR), 0.f, frame.minus_one, s_high, s_low);
+            const half2_t zs = half2_t{z_high.x, static_cast<_Float16>(MX_FAR)};
+            tile_operands({xy_high, xy_high, zs, zs}, {xy_low, xy_low, half2_t{z_low.x, 0}, half2_t{s_high.x, s_low.x}}, queries);
+        }
+        MatrixNearest near[2];
+        near[0].m1 = near[0].m2 = near[1].m1 = near[1].m2 = __float_as_int(__builtin_inff());
+        near[0].cell = near[1].cell = seed;
+        matrix_scan(cpts, seed, ~0ull, lane, frame, queries, near);
+        TPK_WORK_ADD(NG_CELL);
+        // the smallest product of the lane's query, and the squared distance that holds the query's answer for certain
+        auto smallest = [&]() {
+            int a, b;
+            by_query(near[0].m1, near[1].m1, a, b);
+            return __int_as_float(max(min(a, b), 0));
+        };
+        float m = smallest();
+        reach = __builtin_fmaf(m, reach_factor, reach_error);
+        // (where the first cell's second smallest products are near the error already, the search would leave the queries over)
+        int c2, d2;
+        by_query(near[0].m2, near[1].m2, c2, d2);
+        if (__builtin_popcountll(__ballot(real && __int_as_float(min(c2, d2)) < MX_CLOSE * own_error)) <= MX_MANY)
+        {
+            // First the cells whose boxes overlap the queries' box - they hold nearly all the answers - then whatever
+            // the worst answer still admits (a cell is looked at once: answers only get better).
+            for (int phase = 0; phase < 2; ++phase)
+                for (int g = 0; g < groups; ++g)
                 {
-                    bound = __int_as_float(wave_max_i32(__float_as_int(s.best)));
-                    live &= __ballot(lw * NG_MARGIN <= bound);
+                    const float lw = lows[g * NG_CELL + lane];
+                    float bound = __int_as_float(wave_max_i32(__float_as_int(reach)));
+                    unsigned long long live =
+                        __ballot(phase == 0 ? lw == 0.f : lw > 0.f && lw < __builtin_inff() && lw * NG_MARGIN <= bound);
+                    if (g == seed / NG_CELL)
+                        live &= ~(1ull << (seed % NG_CELL));
+                    while (live != 0)
+                    {
+                        const int c = g * NG_CELL + __builtin_ctzll(live);
+                        live &= live - 1;
+                        const float lb = point_box_dist2(qx, qy, qz, cbox[c * NG_BOX + 0], cbox[c * NG_BOX + 1]);
+                        const unsigned long long want = __ballot(lb * NG_MARGIN <= reach);
+                        if (want == 0)
+                            continue;
+                        matrix_scan(cpts, c, want, lane, frame, queries, near);
+                        TPK_WORK_ADD(NG_CELL);
+                        reach = __builtin_fmaf(smallest(), reach_factor, reach_error);
+                        if (phase)
+                        {
+                            bound = __int_as_float(wave_max_i32(__float_as_int(reach)));
+                            live &= __ballot(lw * NG_MARGIN <= bound);
+                        }
+                    }
+                }
+            int a, b, a2, b2, cell_a, cell_b;
+            by_query(near[0].m1, near[1].m1, a, b);
+            by_query(near[0].m2, near[1].m2, a2, b2);
+            by_query(near[0].cell, near[1].cell, cell_a, cell_b);
+            const int m1 = min(a, b);
+            const float m2 = __int_as_float(min(min(a2, b2), max(a, b)));
+            m = __int_as_float(max(m1, 0));
+            ask = real && !(m2 > m + 2.f * __builtin_fmaf(m, MX_ERROR, own_error) && m < MX_LIMIT);
+            const int first = (a <= b ? cell_a : cell_b) * NG_CELL + (m1 & 3) * 16 + (a <= b ? 0 : 4);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) // (rows 0 .. 3 and 8 .. 11 of 16, or those four further on)
+            {
+                const float4 p = cpts[first + (c & 3) + 2 * (c & 4)];
+                const float d = tpk_dist2(p.x, p.y, p.z, qx, qy, qz);
+                const int ci = __float_as_int(p.w);
+                bi = d < best || (d == best && ci < bi) ? ci : bi;
+                best = fminf(d, best);
+            }
+            TPK_WORK_ADD(8);
+        }
+        // (the answer of a query that is left over is below its reach: not equal)
+        reach = m < MX_LIMIT ? reach : __builtin_inff();
+        if (__builtin_popcountll(__ballot(ask)) <= MX_PASS)
+        {
+            tie = ask;
+            ask = false;
+        }
+        s.best = ask ? reach : -1.f;
+    }
+    if (__ballot(ask) != 0)
+    {
+        if (!matrix)
+        {
+            scan_cell(cpts, cruns, seed, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
+            if (lane == (seed & (NG_CELL - 1)))
+                lows[seed] = __builtin_inff();
+        }
+        // (in the same order)
+        for (int phase = 0; phase < 2; ++phase)
+            for (int g = 0; g < groups; ++g)
+            {
+                const float lw = lows[g * NG_CELL + lane];
+                float bound = __int_as_float(wave_max_i32(__float_as_int(s.best)));
+                unsigned long long live =
+                    __ballot(lw < __builtin_inff() && (phase == 0 ? lw == 0.f : lw * NG_MARGIN <= bound));
+                while (live != 0)
+                {
+                    const int bit = __builtin_ctzll(live);
+                    const int c = g * NG_CELL + bit;
+                    live &= live - 1;
+                    const float lb = point_box_dist2(qx, qy, qz, cbox[c * NG_BOX + 0], cbox[c * NG_BOX + 1]);
+                    const unsigned long long want = __ballot(lb * NG_MARGIN <= s.best);
+                    // scanned, or no lane can improve here now - and answers only get better: never again
+                    if (lane == bit)
+                        lows[c] = __builtin_inff();
+                    if (want == 0)
+                        continue;
+                    if (__builtin_popcountll(want) <= NG_FEW)
+                        scan_cell_few(cpts, c, want, lane, qx, qy, qz, s TPK_WORK_ARG);
+                    else
+                        scan_cell(cpts, cruns, c, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
+                    if (phase)
+                    {
+                        bound = __int_as_float(wave_max_i32(__float_as_int(s.best)));
+                        live &= __ballot(lw * NG_MARGIN <= bound);
+                    }
                 }
             }
-        }
 
-    // The index: lowest original index among the candidates of the recorded group that are at
-    // the minimum distance (re-evaluated with the same operations, hence the same bits).
-    int bi = 0x7FFFFFFF;
+        // The index: lowest original index among the candidates of the recorded group that are at
+        // the minimum distance (re-evaluated with the same operations, hence the same bits).
+        best = ask ? s.best : best;
+        bi = ask ? 0x7FFFFFFF : bi;
 #pragma unroll
-    for (int c = 0; c < NG_CHUNK; ++c)
-    {
-        const float4 p = cpts[s.chunk * NG_CHUNK + c];
-        const float d = tpk_dist2(p.x, p.y, p.z, qx, qy, qz);
-        const int ci = __float_as_int(p.w);
-        bi = (d == s.best && ci < bi) ? ci : bi;
+        for (int c = 0; c < NG_CHUNK; ++c)
+        {
+            const float4 p = cpts[s.chunk * NG_CHUNK + c];
+            const float d = tpk_dist2(p.x, p.y, p.z, qx, qy, qz);
+            const int ci = __float_as_int(p.w);
+            bi = (ask && d == best && ci < bi) ? ci : bi;
+        }
+        TPK_WORK_ADD(NG_CHUNK);
+        reach = ask ? best : reach;
+        tie = tie || (ask && s.tie);
     }
-    // Several groups reached a query's minimum (about one query in 10^5 on random clouds, every query on a
-    // lattice): the lowest index over all cells that can hold that distance.  One such query at a time: the
-    // lanes test the boxes of all cells side by side, then the candidates of every cell that passes.
-    for (unsigned long long tied = __ballot(s.tie); tied != 0; tied &= tied - 1)
+    // Several groups reached a query's minimum (about one query in 10^5 on random clouds, every query on a lattice), or
+    // came too close to it for the products to tell (one in 10^3 to 10^4): the nearest candidate, of several the one of lowest index,
+    // over all cells within reach.  One such query at a time: the lanes test the boxes of all cells side by side, then the
+    // candidates of every cell that passes.
+    for (unsigned long long tied = __ballot(tie); tied != 0; tied &= tied - 1)
     {
         const int q = __builtin_ctzll(tied);
         const float ux = tpk_read_lane(qx, q), uy = tpk_read_lane(qy, q), uz = tpk_read_lane(qz, q);
-        const float ub = tpk_read_lane(s.best, q);
+        const float ub = tpk_read_lane(reach, q);
+        float nearest = __builtin_inff();
         int lowest = 0x7FFFFFFF;
+#pragma unroll 4
         for (int g = 0; g < groups; ++g)
         {
             const int c = g * NG_CELL + lane;
             const int cc = c < ccells ? c : 0;
             const float lb = point_box_dist2(ux, uy, uz, cbox[cc * NG_BOX + 0], cbox[cc * NG_BOX + 1]);
-            for (unsigned long long cells = __ballot(c < ccells && lb * NG_MARGIN <= ub); cells != 0; cells &= cells - 1)
+            unsigned long long cells = __ballot(c < ccells && lb * NG_MARGIN <= ub);
+            while (cells != 0)
             {
-                const float4 p = cpts[(g * NG_CELL + __builtin_ctzll(cells)) * NG_CELL + lane];
-                const float d = tpk_dist2(p.x, p.y, p.z, ux, uy, uz);
-                TPK_WORK_ADD(1);
-                lowest = min(lowest, wave_min_i32(d == ub ? __float_as_int(p.w) : 0x7FFFFFFF));
+                float4 p[4]; // (four cells on their way at a time; behind the last, the last one again)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                {
+                    p[u] = cpts[(g * NG_CELL + __builtin_ctzll(cells)) * NG_CELL + lane];
+                    const unsigned long long rest = cells & (cells - 1);
+                    cells = rest != 0 || u == 3 ? rest : cells;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                {
+                    const float d = tpk_dist2(p[u].x, p[u].y, p[u].z, ux, uy, uz);
+                    const int ci = __float_as_int(p[u].w);
+                    lowest = d < nearest || (d == nearest && ci < lowest) ? ci : lowest;
+                    nearest = d < nearest ? d : nearest;
+                }
+                TPK_WORK_ADD(4);
             }
         }
-        bi = lane == q ? min(bi, lowest) : bi;
+        // (distances are >= +0: their bit patterns order like integers)
+        const float least = __int_as_float(wave_min_i32(__float_as_int(nearest)));
+        lowest = wave_min_i32(nearest == least ? lowest : 0x7FFFFFFF);
+        best = lane == q ? least : best;
+        bi = lane == q ? lowest : bi;
     }
-    TPK_WORK_ADD(NG_CHUNK);
     TPK_WORK_FLUSH
-    if (qindex != 0x7FFFFFFF)
+    if (real)
     {
-        dout[qindex] = s.best;
+        dout[qindex] = best;
         iout[qindex] = bi == 0x7FFFFFFF ? 0 : bi;
     }
 }
@@ -360,16 +652,16 @@ __device__ __forceinline__ bool pair_less(float d, int ci, float b, int i)
     return d < b || (d == b && ci < i);
 }
 
-__device__ __forceinline__ void scan_cell3(const float4* __restrict__ cand, const float4* __restrict__ boxes,
+__device__ __forceinline__ void scan_cell3(const float4* __restrict__ cand, const float4* __restrict__ runs,
                                            int cell, float4* stage, int lane, float qx, float qy, float qz,
                                            Nearest3& s TPK_WORK_PARAM)
 {
     stage[lane] = cand[cell * NG_CELL + lane];
     // (the boxes of the cell's four runs are requested together with its candidates: one wait, not five)
-    float4 quarter[NG_BOX - 2];
+    float4 quarter[NG_RUN_BOXES];
 #pragma unroll
-    for (int i = 0; i < NG_BOX - 2; ++i)
-        quarter[i] = boxes[cell * NG_BOX + 2 + i];
+    for (int i = 0; i < NG_RUN_BOXES; ++i)
+        quarter[i] = runs[cell * NG_RUN_BOXES + i];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     bool reached = true;
 #pragma unroll
@@ -493,6 +785,8 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
     const float4* __restrict__ qpts = sorted_unknown + static_cast<int64_t>(cloud) * qcells * NG_CELL;
     const float4* __restrict__ cpts = sorted_known + static_cast<int64_t>(cloud) * ccells * NG_CELL;
     const float4* __restrict__ cbox = boxes_known + static_cast<int64_t>(cloud) * ccells * NG_BOX;
+    const float4* __restrict__ cruns =
+        boxes_known + static_cast<int64_t>(clouds) * ccells * NG_BOX + static_cast<int64_t>(cloud) * ccells * NG_RUN_BOXES;
     dist2 += static_cast<int64_t>(cloud) * n * 3;
     idx += static_cast<int64_t>(cloud) * n * 3;
     float4* const stage = stages[wave];
@@ -532,7 +826,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
         int seed = static_cast<int>(lowest & 63u) * NG_CELL + __builtin_ctzll(__ballot(seed_key == lowest));
         if (seed >= ccells)
             seed = 0;
-        scan_cell3(cpts, cbox, seed, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
+        scan_cell3(cpts, cruns, seed, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
         if (lane == (seed & (NG_CELL - 1)))
             lows[seed] = __builtin_inff();
     }
@@ -553,7 +847,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
                 if (want != 0 && __builtin_popcountll(want) <= NG_FEW3)
                     scan_cell3_few(cpts, c, want, lane, qx, qy, qz, s TPK_WORK_ARG);
                 else if (want != 0)
-                    scan_cell3(cpts, cbox, c, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
+                    scan_cell3(cpts, cruns, c, stage, lane, qx, qy, qz, s TPK_WORK_ARG);
                 if (lane == bit)
                     lows[c] = __builtin_inff(); // scanned, or useless now and ever after
                 if (phase)
@@ -582,7 +876,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
 // is further away than the last kept entry of every lane.
 // ---------------------------------------------------------------------------------------
 template <int K>
-__device__ __forceinline__ void scan_cell_k(const float4* __restrict__ cand, const float4* __restrict__ boxes,
+__device__ __forceinline__ void scan_cell_k(const float4* __restrict__ cand, const float4* __restrict__ runs,
                                             int cell, float4* stage, int lane, float qx, float qy, float qz,
                                             NearestK<K>& s)
 {
@@ -592,12 +886,12 @@ __device__ __forceinline__ void scan_cell_k(const float4* __restrict__ cand, con
     // requested together with the candidates and tested before the scan: one wait, not five.
     unsigned reached = 0;
     {
-        float4 quarter[NG_BOX - 2];
+        float4 quarter[NG_RUN_BOXES];
 #pragma unroll
-        for (int i = 0; i < NG_BOX - 2; ++i)
-            quarter[i] = boxes[cell * NG_BOX + 2 + i];
+        for (int i = 0; i < NG_RUN_BOXES; ++i)
+            quarter[i] = runs[cell * NG_RUN_BOXES + i];
 #pragma unroll
-        for (int run = 0; run < (NG_BOX - 2) / 2; ++run)
+        for (int run = 0; run < NG_RUN_BOXES / 2; ++run)
         {
             const float lb = point_box_dist2(qx, qy, qz, quarter[2 * run], quarter[2 * run + 1]);
             reached |= __ballot(lb * NG_MARGIN <= worst) != 0 ? 1u << run : 0u;
@@ -658,6 +952,8 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void knn_grid_kernel(
     const float4* __restrict__ qpts = sorted_query + static_cast<int64_t>(cloud) * qcells * NG_CELL;
     const float4* __restrict__ cpts = sorted_support + static_cast<int64_t>(cloud) * ccells * NG_CELL;
     const float4* __restrict__ cbox = boxes_support + static_cast<int64_t>(cloud) * ccells * NG_BOX;
+    const float4* __restrict__ cruns =
+        boxes_support + static_cast<int64_t>(clouds) * ccells * NG_BOX + static_cast<int64_t>(cloud) * ccells * NG_RUN_BOXES;
     dist2 += static_cast<int64_t>(cloud) * n * k;
     idx += static_cast<int64_t>(cloud) * n * k;
     float4* const stage = stages[wave];
@@ -702,7 +998,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void knn_grid_kernel(
         int seed = static_cast<int>(lowest & 63u) * NG_CELL + __builtin_ctzll(__ballot(seed_key == lowest));
         if (seed >= ccells)
             seed = 0;
-        scan_cell_k<K>(cpts, cbox, seed, stage, lane, qx, qy, qz, s);
+        scan_cell_k<K>(cpts, cruns, seed, stage, lane, qx, qy, qz, s);
         if (lane == (seed & (NG_CELL - 1)))
             lows[seed] = __builtin_inff();
     }
@@ -720,7 +1016,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void knn_grid_kernel(
                 live &= live - 1;
                 const float lb = point_box_dist2(qx, qy, qz, cbox[c * NG_BOX + 0], cbox[c * NG_BOX + 1]);
                 if (__ballot(lb * NG_MARGIN <= s.worst()) != 0)
-                    scan_cell_k<K>(cpts, cbox, c, stage, lane, qx, qy, qz, s);
+                    scan_cell_k<K>(cpts, cruns, c, stage, lane, qx, qy, qz, s);
                 if (lane == bit)
                     lows[c] = __builtin_inff(); // scanned, or useless now and ever after
                 if (phase)
@@ -1092,9 +1388,9 @@ GridLayout grid_layout(int b, int n, int m, bool wide_first = false)
     l.sorted_b = pos;
     pos = up(pos + static_cast<size_t>(b) * cells_b * NG_CELL * sizeof(float4));
     l.boxes_a = pos;
-    pos = up(pos + static_cast<size_t>(b) * cells_a * NG_BOX * sizeof(float4));
+    pos = up(pos + static_cast<size_t>(b) * cells_a * NG_CELL_BOXES * sizeof(float4));
     l.boxes_b = pos;
-    pos = up(pos + static_cast<size_t>(b) * cells_b * NG_BOX * sizeof(float4));
+    pos = up(pos + static_cast<size_t>(b) * cells_b * NG_CELL_BOXES * sizeof(float4));
     l.wide_a = l.wide_b = pos;
     if (wide_first) // (the Chamfer search: the cells of every window, wide ones first)
     {
@@ -1362,7 +1658,7 @@ SupportLayout support_layout(int b, int m)
     SupportLayout l;
     l.sorted = 0;
     l.boxes = up(static_cast<size_t>(b) * cells * NG_CELL * sizeof(float4));
-    l.runs = l.boxes + up(static_cast<size_t>(b) * cells * NG_BOX * sizeof(float4));
+    l.runs = l.boxes + up(static_cast<size_t>(b) * cells * NG_CELL_BOXES * sizeof(float4));
     l.total = l.runs + up(static_cast<size_t>(b) * ((cells + NG_RUN - 1) / NG_RUN) * 2 * sizeof(float4));
     return l;
 }
