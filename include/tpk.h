@@ -298,6 +298,9 @@ int tpk_group_recording_f32(int b, int c, int n, int npoint, int nsample, const 
  * arguments are kept for callers written against earlier versions and are ignored): the points
  * that chose a point as nearest neighbour are chained to it in LDS.  Clouds of more than about
  * 38000 points scatter with hardware float atomics instead.
+ * tpk_chamfer_fwd_loss_f32: tpk_chamfer_fwd_f32 and tpk_chamfer_loss_f32 in one, without the distances, in
+ * tpk_chamfer_fwd_loss_workspace_bytes() bytes (0: a shape it does not serve, TPK_ERR_UNSUPPORTED); summed in float64, a cell
+ * of neighbouring points at a time, those of a cell in no fixed order.
  * tpk_chamfer_loss_*: *loss = mean(dist1) + mean(dist2) of the whole batch, summed in float64 in a
  * fixed order (`workspace`: tpk_chamfer_loss_workspace_bytes() bytes, 8-byte aligned; NaN where a
  * mean is over nothing).  tpk_chamfer_loss_bwd_*: the backward pass for that loss: grad_loss is one
@@ -307,6 +310,9 @@ size_t tpk_chamfer_fwd_workspace_bytes(int b, int n, int m);
 int tpk_chamfer_fwd_f32(int b, int n, int m, const float* xyz1, const float* xyz2, float* dist1,
                         float* dist2, int32_t* idx1, int32_t* idx2, void* workspace,
                         size_t workspace_bytes, void* stream);
+size_t tpk_chamfer_fwd_loss_workspace_bytes(int b, int n, int m);
+int tpk_chamfer_fwd_loss_f32(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1,
+                             int32_t* idx2, void* workspace, size_t workspace_bytes, void* stream);
 int tpk_chamfer_fwd_f64(int b, int n, int m, const double* xyz1, const double* xyz2,
                         double* dist1, double* dist2, int32_t* idx1, int32_t* idx2,
                         void* stream);

@@ -751,6 +751,19 @@ extern "C" int tpk_chamfer_fwd_f32(int b, int n, int m, const float* xyz1, const
     return chamfer_fwd<float>(b, n, m, xyz1, xyz2, dist1, dist2, idx1, idx2, stream);
 }
 
+extern "C" size_t tpk_chamfer_fwd_loss_workspace_bytes(int b, int n, int m)
+{
+    return tpk_grid_chamfer_loss_workspace_bytes(b, n, m);
+}
+
+extern "C" int tpk_chamfer_fwd_loss_f32(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1,
+                                        int32_t* idx2, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (!xyz1 || !xyz2 || !loss || !idx1 || !idx2)
+        return TPK_ERR_INVALID_ARG;
+    return tpk_grid_chamfer_loss(b, n, m, xyz1, xyz2, loss, idx1, idx2, workspace, workspace_bytes, tpk_stream(stream));
+}
+
 extern "C" int tpk_chamfer_fwd_f64(int b, int n, int m, const double* xyz1, const double* xyz2,
                                    double* dist1, double* dist2, int32_t* idx1, int32_t* idx2,
                                    void* stream)

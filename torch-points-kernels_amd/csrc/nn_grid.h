@@ -14,6 +14,11 @@ int tpk_grid_chamfer_fwd(int b, int n, int m, const float* xyz1, const float* xy
                          float* dist2, int32_t* idx1, int32_t* idx2, void* workspace,
                          size_t workspace_bytes, hipStream_t stream);
 
+// *loss = mean(dist1) + mean(dist2) in their place, summed in float64: same conventions, a workspace of its own (0: not served).
+size_t tpk_grid_chamfer_loss_workspace_bytes(int b, int n, int m);
+int tpk_grid_chamfer_loss(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1, int32_t* idx2, void* workspace,
+                          size_t workspace_bytes, hipStream_t stream);
+
 // three_nn, float32: same conventions.  The workspace ends with one word per cloud
 // (tpk_grid_three_nn_flags: its address, or nullptr when the workspace does not serve the shape); with
 // `flagged` only the clouds whose word is not 0 are searched - a kernel enqueued before has answered the others.

@@ -1249,17 +1249,25 @@ std::vector<at::Tensor> chamfer_loss_forward(const at::Tensor& xyz1, const at::T
     const int b = as_int(xyz1.size(0), "batch size"), n = as_int(xyz1.size(1), "points of xyz1"), m = as_int(xyz2.size(1), "points of xyz2");
     const bool narrow = xyz1.scalar_type() == at::kFloat;
     const size_t total1 = static_cast<size_t>(b) * n, total2 = static_cast<size_t>(b) * m;
+    at::Tensor idx = torch::empty({static_cast<int64_t>(total1 + total2)}, xyz1.options().dtype(at::kInt));
+    at::Tensor loss = torch::empty({}, xyz1.options());
+    int32_t* const idx1 = idx.data_ptr<int32_t>();
+    void* const s = current_stream(xyz1);
+    if (const size_t loss_bytes = narrow ? tpk_chamfer_fwd_loss_workspace_bytes(b, n, m) : 0)
+    {
+        at::Tensor scratch = torch::empty({static_cast<int64_t>(loss_bytes)}, xyz1.options().dtype(at::kByte));
+        check_status(tpk_chamfer_fwd_loss_f32(b, n, m, xyz1.data_ptr<float>(), xyz2.data_ptr<float>(), loss.data_ptr<float>(), idx1, idx1 + total1,
+                                              scratch.data_ptr(), loss_bytes, s),
+                     "chamfer_dist");
+        return {loss, idx};
+    }
     // one scratch: the search's workspace, the sums' workspace, the distances
     const size_t ws_bytes = narrow ? tpk_chamfer_fwd_workspace_bytes(b, n, m) : 0, sum_bytes = tpk_chamfer_loss_workspace_bytes(b, n, m);
     const size_t sums_at = (ws_bytes + 255) & ~static_cast<size_t>(255), dist_at = (sums_at + sum_bytes + 255) & ~static_cast<size_t>(255);
     at::Tensor scratch = torch::empty({static_cast<int64_t>(dist_at + (total1 + total2) * xyz1.element_size())}, xyz1.options().dtype(at::kByte));
-    at::Tensor idx = torch::empty({static_cast<int64_t>(total1 + total2)}, xyz1.options().dtype(at::kInt));
-    at::Tensor loss = torch::empty({}, xyz1.options());
     char* const bytes = static_cast<char*>(scratch.data_ptr());
-    int32_t* const idx1 = idx.data_ptr<int32_t>();
     void* const ws = ws_bytes ? bytes : nullptr;
     void* const sums = sum_bytes ? bytes + sums_at : nullptr;
-    void* const s = current_stream(xyz1);
     if (narrow)
     {
         float* const dist1 = reinterpret_cast<float*>(bytes + dist_at);
