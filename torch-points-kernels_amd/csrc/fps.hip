@@ -473,7 +473,7 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
                         {
 #pragma unroll
                             for (int i = 0; i < PPT; ++i)
-                            {
+                                if (PPT < 8 || __builtin_expect(above[i] != 0ull, 0)) // (a few of sixteen: no branch taken for the others)
                                 {
                                     if (t[i] > floor_bits)
                                     {
@@ -483,7 +483,6 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
                                     }
                                     at += __builtin_popcountll(above[i]);
                                 }
-                            }
                         }
                     }
                 }
@@ -741,12 +740,17 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
         most = wave_max_to_scalar(most);
         const int own_lane = not_hoisted(lane);
         bool several = keyed; // (where there were some there will be more)
+        int held_in = 0;      // the slot that holds the maximum, if one does
         if (!keyed)
         {
             int held = 0;
 #pragma unroll
             for (int i = 0; i < PPT; ++i)
-                held += __builtin_popcountll(__ballot(t[i] == most));
+            {
+                const unsigned long long holds = __ballot(t[i] == most);
+                held += __builtin_popcountll(holds);
+                held_in = PPT >= 8 && holds != 0ull ? i : held_in;
+            }
             several = held > 1;
         }
         if (several && most >= 0)
@@ -794,13 +798,23 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
         }
         else
         {
-#pragma unroll
-            for (int i = 0; i < PPT; ++i)
+            auto offer = [&](int i) __attribute__((always_inline)) {
                 if (t[i] == most)
                 {
                     offers[turn][wave] = make_float4(x[i], y[i], z[i], __int_as_float(most));
                     offer_places[turn][wave] = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
                 }
+            };
+            // (sixteen tests with a branch each, of all wavefronts of a SIMD in turn, were 200 ns of such a sample's 1650; where nothing is
+            // left - most < 0 - any slot that holds it will do)
+            if constexpr (PPT >= 8)
+                with_slot<0, PPT>(held_in, [&](auto chosen) __attribute__((always_inline)) { offer(chosen.value); });
+            else
+            {
+#pragma unroll
+                for (int i = 0; i < PPT; ++i)
+                    offer(i);
+            }
         }
         lds_barrier();
         const float4 offer = offers[turn][lane % WAVES];
