@@ -1195,6 +1195,23 @@ def test_grouping_grad_long_rows(tpk, oracle, dev, N, npoint, nsample, C):
     _assert_scatter_sum_close(_np(f.grad), want, oracle.grouping_operation_grad(gout.abs().numpy(), idx.numpy(), N))
 
 
+@pytest.mark.parametrize("rows", [34, 35, 36, 37, 58, 59, 60, 61, 83, 84, 85, 300])
+def test_grouping_grad_crowded_span(tpk, dev, rows):
+    # one span of targets with about `rows` rows of 64 entries - fewer than a lane holds, as many, and up to several refills more -
+    # beside even ones; small integers, whose sums are exact in any order
+    B, C, N, npoint, nsample = 2, 3, 512, 1024, 32
+    g = torch.Generator().manual_seed(rows)
+    idx = torch.randint(16, N, (B, npoint * nsample), generator=g)
+    for b in range(B):
+        crowd = torch.randperm(npoint * nsample, generator=g)[: 64 * rows - 40 * b]
+        idx[b, crowd] = torch.randint(0, 16, (crowd.numel(),), generator=g) ** 2 // 16 * 2
+    gout = torch.randint(-8, 9, (B, C, npoint, nsample), generator=g).float()
+    f = torch.randn(B, C, N, generator=g).to(dev).requires_grad_(True)
+    tpk.grouping_operation(f, idx.view(B, npoint, nsample).to(dev)).backward(gout.to(dev))
+    want = torch.zeros(B, C, N).scatter_add_(2, idx.view(B, 1, -1).expand(B, C, -1), gout.view(B, C, -1))
+    np.testing.assert_array_equal(_np(f.grad), want.numpy())
+
+
 @pytest.mark.parametrize("B,C,m,n", [(1, 1, 1, 1), (1, 3, 15, 1023), (2, 9, 16, 1024), (2, 5, 17, 1025), (1, 2, 300, 16385), (2, 2, 3000, 32768),
                                      (1, 7, 4096, 32769), (1, 2, 20481, 4097), (16, 64, 1024, 4096)])
 @pytest.mark.parametrize("kind", ["spread", "one target", "last targets", "crowded first", "crowded last", "crowded in turn"])

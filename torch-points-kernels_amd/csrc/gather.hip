@@ -251,6 +251,7 @@ constexpr int GB_STAGE_FLOATS = 32768; // at most this many of them hold the sta
 constexpr int GB_FETCH = GB_STAGE_FLOATS / 4 / G_THREADS; // 16-byte loads per lane that bring in a piece: 8
 constexpr int GB_AHEAD = 8;            // rows of list entries a wavefront has requested ahead of the one it adds
 constexpr int GB_HOLD = 36;            // rows of list entries a lane keeps in registers where a piece's entries are held
+constexpr int GB_REFILL = 24;          // of which are asked for again, so many rows ahead, where a span has more
 constexpr int GB_BUSY_GRID = 128;      // workgroups below which a call takes fewer rows per workgroup
 // The walk that holds a piece's entries in registers: one row per pass, 4-byte entries.
 template <int K, bool WEIGHTED, int R>
@@ -430,7 +431,11 @@ __global__ __launch_bounds__(G_THREADS, 1) void gather_bwd_lists_kernel(
         // piece - for most of the time a piece takes.  Here a piece's entries are all requested before the next
         // piece is, right after the walk of the piece before, and kept in registers: the walk itself then asks
         // memory for nothing, and the next piece is requested at its very beginning, by all wavefronts at once.
-        // (Spans of more than GB_HOLD rows of entries fetch the rest one row at a time.)
+        // The first span of a padded ball query holds three to six times its share of the entries: behind the held rows its
+        // wavefront keeps GB_REFILL rows on their way, in the same registers.  (One row at a time, each a journey to the L2
+        // that the other 15 wavefronts waited for, 16 x 128 rows of 32768 on 4096 targets of a ball query took 279 us, with
+        // 12 rows on their way 133, with 24 127; even lists 78.  Rows refilled while the held ones are walked, two copies of
+        // the walk: 124, but the registers spill and even lists take 82.)
         if (vector_loads)
         {
             struct Span
@@ -509,8 +514,23 @@ __global__ __launch_bounds__(G_THREADS, 1) void gather_bwd_lists_kernel(
                     if (u < cur.steps) // (wave-uniform)
                         take(held[u]);
                 }
-                for (int i = GB_HOLD; i < cur.steps; ++i)
-                    take(entry(cur, i));
+                if (cur.steps > GB_HOLD)
+                {
+#pragma unroll
+                    for (int u = 0; u < GB_REFILL; ++u)
+                        held[u] = entry(cur, GB_HOLD + u);
+                    for (int i0 = GB_HOLD; i0 < cur.steps; i0 += GB_REFILL)
+                    {
+#pragma unroll
+                        for (int u = 0; u < GB_REFILL; ++u)
+                        {
+                            if (i0 + u >= cur.steps) // (wave-uniform)
+                                break;
+                            take(held[u]);
+                            held[u] = entry(cur, i0 + u + GB_REFILL);
+                        }
+                    }
+                }
                 // the first list every lane ended, with what the lanes before carried into it
                 float open[1] = {acc}, carry[1];
                 const bool ended_one = slot != cur.first_slot;
