@@ -289,9 +289,28 @@ inline int __builtin_amdgcn_update_dpp(int old, int v, int control, int rows, in
 // (a fence is where other lanes' accesses to LDS are waited for)
 #define __builtin_amdgcn_fence(...) static_cast<void>(emulation::exchange(0))
 #define __builtin_amdgcn_s_barrier() __syncthreads()
+#define __builtin_amdgcn_sched_barrier(mask) static_cast<void>(0)
 #define __builtin_amdgcn_s_waitcnt(x) static_cast<void>(0)
 inline float __builtin_amdgcn_rcpf(float v) { return 1.0f / v; }
 inline float __builtin_amdgcn_fmed3f(float a, float b, float c) { return fmaxf(fminf(a, b), fminf(fmaxf(a, b), c)); }
+// Chamfer's matrix products of halves are declared for the compiler only: the kernels run here have none.
+#if !defined(__FLT16_MAX__)
+typedef short _Float16;
+#endif
+template <typename V, typename W>
+inline W __builtin_amdgcn_mfma_f32_32x32x16_f16(V, V, W, int, int, int)
+{
+    abort();
+}
+struct emulated_pair
+{
+    unsigned v[2];
+    unsigned operator[](int i) const { return v[i]; }
+};
+inline emulated_pair __builtin_amdgcn_permlane32_swap(unsigned, unsigned, bool, bool)
+{
+    abort();
+}
 inline unsigned __builtin_amdgcn_mbcnt_lo(unsigned mask, unsigned add)
 {
     const int lane = emulation::lane();

@@ -167,10 +167,10 @@ __device__ __forceinline__ void scan_cell_few(const float4* __restrict__ cand, i
 // 266 -> 254, of 2 x 60000 821 -> 917 (cells that are wide for their points' distances leave half of the queries over).
 // Taken back: minima of four candidates (24 more instructions per scan, 12 % slower), whole wavefronts by the exact scan where many
 // queries are left over (laser scans 30 % slower than without the matrix cores).
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half2_t __attribute__((vector_size(4)));
+typedef _Float16 half8_t __attribute__((vector_size(16)));
+typedef float float16_t __attribute__((vector_size(64)));
+typedef unsigned uint4_t __attribute__((vector_size(16)));
 
 constexpr float MX_FAR = 16384.f;          // 2^14: candidates are clamped to this; also the factor |p|^2 and |q|^2 are kept divided by
 constexpr float MX_LIMIT = 134217728.f;    // 2^27: a squared distance that no clamped candidate can have
@@ -187,8 +187,8 @@ constexpr int MX_PASS = 20;                // (12: laser scans of 32 x 4096 106 
 __device__ __forceinline__ void split_half(float a, float b, float minus_one, half2_t& high, half2_t& low)
 {
     high = half2_t{static_cast<_Float16>(a), static_cast<_Float16>(b)};
-    low = half2_t{static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high.x), minus_one, a)),
-                  static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high.y), minus_one, b))};
+    low = half2_t{static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high[0]), minus_one, a)),
+                  static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high[1]), minus_one, b))};
 }
 
 // Operands of two tiles of 32 points, one point per lane: lanes 0 .. 31 of a tile hold slots 0 .. 7 of its points, the others slots 8 .. 15.
@@ -285,10 +285,10 @@ __device__ __forceinline__ void matrix_scan(const float4* __restrict__ cand, int
 template <int CONTROL, int ROWS>
 __device__ __forceinline__ double added_dpp(double v)
 {
-    const long long bits = __double_as_longlong(v);
+    const long long bits = __builtin_bit_cast(long long, v);
     const int low = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits), CONTROL, ROWS, 0xF, false);
     const int high = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits >> 32), CONTROL, ROWS, 0xF, false);
-    return v + __longlong_as_double(static_cast<long long>(high) << 32 | static_cast<unsigned>(low));
+    return v + __builtin_bit_cast(double, static_cast<long long>(high) << 32 | static_cast<unsigned>(low));
 }
 __device__ __forceinline__ double wave_sum_f64(double v)
 {
@@ -468,8 +468,8 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
             split_half(-2.f * x, -2.f * y, frame.minus_one, xy_high, xy_low);
             split_half(-2.f * z, 0.f, frame.minus_one, z_high, z_low);
             split_half(square * (1.f / MX_FAR), 0.f, frame.minus_one, s_high, s_low);
-            const half2_t zs = half2_t{z_high.x, static_cast<_Float16>(MX_FAR)};
-            tile_operands({xy_high, xy_high, zs, zs}, {xy_low, xy_low, half2_t{z_low.x, 0}, half2_t{s_high.x, s_low.x}}, queries);
+            const half2_t zs = half2_t{z_high[0], static_cast<_Float16>(MX_FAR)};
+            tile_operands({xy_high, xy_high, zs, zs}, {xy_low, xy_low, half2_t{z_low[0], 0}, half2_t{s_high[0], s_low[0]}}, queries);
         }
         MatrixNearest near[2];
         near[0].m1 = near[0].m2 = near[1].m1 = near[1].m2 = __float_as_int(__builtin_inff());
