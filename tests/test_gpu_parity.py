@@ -2357,6 +2357,19 @@ def test_chamfer_on_the_matrix_cores(dev, kind, n, m):
         assert torch.equal(cells, pairs)
 
 
+@pytest.mark.parametrize("B,n,m", [(1, 512, 512), (3, 513, 640), (2, 16385, 520), (2048, 512, 512), (2049, 512, 512), (600, 700, 1100)])
+def test_chamfer_loss_from_the_searchs_sums(tpk, dev, B, n, m):
+    """The loss of float32 clouds that the search over cells serves: padding in a cloud's last cell, cells without points behind a whole
+    window, as many wavefronts as leave sums (32768) and one cloud more, whose distances are stored and read again."""
+    g = torch.Generator(device=dev).manual_seed(B + n + m)
+    a, b = (torch.rand(B, k, 3, generator=g, device=dev) for k in (n, m))
+    loss = tpk.chamfer_dist.chamfer_dist(a, b)
+    d1, d2 = tpk.ChamferFunction.apply(a, b)
+    want = float(d1.double().mean() + d2.double().mean())
+    # (sums in float64 on either side: their rounding is far below the one rounding of the result)
+    assert abs(float(loss) - want) <= 2.0 ** -23 * want
+
+
 def test_chamfer_gradcheck_double(tpk, dev):
     # reference test/test_chamfer_dist.py:20-25
     from torch.autograd import gradcheck
