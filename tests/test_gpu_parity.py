@@ -2184,6 +2184,42 @@ def test_chamfer_backward_skewed_indices(tpk, dev, dtype):
         _assert_scatter_sum_close(_np(gb), wb.astype(np.float32), mb.astype(np.float32), "chamfer backward, skewed indices, xyz2")
 
 
+@pytest.mark.parametrize("B", [1, 56, 57, 113, 114, 227, 228])
+@pytest.mark.parametrize("kind", ["even", "crowded", "lattice", "not finite"])
+def test_three_nn_cells_shared_by_wavefronts(dev, kind, B):
+    """The search over cells against the scan of all pairs, bit for bit, where 8, 4, 2 or one wavefront share a cell's queries: either side of 4096
+    wavefronts of every number, a last cell of one query (most of its wavefronts have none), and one call of several windows."""
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_three_nn_workspace_bytes.restype = ctypes.c_size_t
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    for n, m in [(513, 600)] + ([(16449, 9001)] if B == 1 else []):
+        g = torch.Generator().manual_seed(B + n)
+        clouds = [torch.rand(B, count, 3, generator=g) for count in (n, m)]
+        if kind == "crowded":
+            clouds = [torch.where(torch.rand(c.shape[:2] + (1,), generator=g) < 0.9, c * 0.02 + 0.4, c) for c in clouds]
+        elif kind == "lattice":
+            clouds = [torch.floor(c * 6) / 6 for c in clouds]
+        elif kind == "not finite":
+            clouds[0][:, 7::97, 1] = float("nan")
+            clouds[1][:, 3::89, 2] = float("inf")
+        unknown, known = (c.contiguous().to(dev) for c in clouds)
+        results = []
+        for nbytes in (lib.tpk_three_nn_workspace_bytes(B, n, m), 0):
+            ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+            out = [torch.full((B, n, 3), -1, dtype=t, device=dev) for t in (torch.float32, torch.int32)]
+            st = lib.tpk_three_nn_f32(B, n, m, pointer(unknown), pointer(known), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None)
+            assert st == 0
+            torch.cuda.synchronize()
+            results.append([t.cpu() for t in out])
+        assert lib.tpk_three_nn_workspace_bytes(B, n, m) > 0
+        for cells, pairs in zip(*results):
+            assert torch.equal(cells, pairs)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("B,n,m", [(1, 1, 1), (2, 4096, 1), (1, 4096, 4096), (1, 4097, 4096), (3, 2731, 2000), (1, 40000, 700), (2, 0, 5)])
 def test_chamfer_loss_as_one_node(tpk, dev, dtype, B, n, m):

@@ -839,10 +839,19 @@ __device__ __forceinline__ void scan_cell3_few(const float4* __restrict__ cand, 
     }
 }
 
+// Where the queries' cells are too few to fill the chip, the search lasts as long as its slowest wavefront, one whose 64 queries lie far
+// apart and ask for many cells, one after the other.  The queries of a cell are then shared by 2, 4 or 8 wavefronts, whose boxes
+// are smaller and which scan fewer cells each, as long as these are no more than four per SIMD: beyond, the scans that
+// several of them repeat cost more than the tail (16 x 16384 queries on as many points 110 us whole, in halves 119; on 4096, eight
+// clusters, 120 and 124).  us, whole -> as here, even / eight clusters / sphere: 1 x 16384 on as many 91 -> 54 / 256 -> 114 / 89 -> 52; 2 x 16384 91 -> 60 /
+// 256 -> 112 / 94 -> 59; 4 x 16384 91 -> 66 / 255 -> 167 / 93 -> 67; 8 x 16384 91 -> 80 / 256 -> 215 / 96 -> 90; 2 x 60000 216 -> 157 / 548 -> 458 /
+// 184 -> 157; clusters handed over by the grid in LDS, 1 x 4096 106 -> 63, 8 x 4096 128 -> 101, 4 x 8264 on 4132 106 -> 97, 16 x 2000 85 -> 79.
+constexpr int64_t NG_PARTED_WAVES = 4096;
+constexpr int NG_MOST_PARTS = 3; // log2: 8 queries per wavefront
 __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
     int n, int m, int qcells, int ccells, int clouds, const float4* __restrict__ sorted_unknown,
     const float4* __restrict__ sorted_known, const float4* __restrict__ boxes_known, float* __restrict__ dist2,
-    int32_t* __restrict__ idx, bool root, const int* __restrict__ only)
+    int32_t* __restrict__ idx, bool root, const int* __restrict__ only, int log2_parts)
 {
     __shared__ float4 stages[NG_SCAN_THREADS / TPK_WAVE][NG_CELL];
     extern __shared__ float lows_all[]; // [wavefronts][candidate cells, in whole groups of 64]
@@ -851,12 +860,14 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TPK_WAVE);
     const int64_t task = static_cast<int64_t>(xcd_local_block(blockIdx.x, gridDim.x)) *
                              (NG_SCAN_THREADS / TPK_WAVE) + wave;
-    if (task >= static_cast<int64_t>(qcells) * clouds)
+    const int64_t cell_task = task >> log2_parts;
+    if (cell_task >= static_cast<int64_t>(qcells) * clouds)
         return; // (no workgroup barrier anywhere in this kernel)
-    const int cloud = static_cast<int>(task / qcells);
+    const int cloud = static_cast<int>(cell_task / qcells);
     if (only && only[cloud] == 0)
         return; // (a cloud that another kernel has answered)
-    const int qcell = static_cast<int>(task - static_cast<int64_t>(cloud) * qcells);
+    const int qcell = static_cast<int>(cell_task - static_cast<int64_t>(cloud) * qcells);
+    const int part = static_cast<int>(task) & ((1 << log2_parts) - 1);
     const float4* __restrict__ qpts = sorted_unknown + static_cast<int64_t>(cloud) * qcells * NG_CELL;
     const float4* __restrict__ cpts = sorted_known + static_cast<int64_t>(cloud) * ccells * NG_CELL;
     const float4* __restrict__ cbox = boxes_known + static_cast<int64_t>(cloud) * ccells * NG_BOX;
@@ -870,7 +881,8 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
 
     const float4 query = qpts[qcell * NG_CELL + lane];
     const float qx = query.x, qy = query.y, qz = query.z;
-    const int qindex = __float_as_int(query.w); // 0x7FFFFFFF: padding, nothing to store
+    // 0x7FFFFFFF: padding, nothing to store; so are the queries of the cell's other parts here
+    const int qindex = ((lane << log2_parts) / TPK_WAVE) == part ? __float_as_int(query.w) : 0x7FFFFFFF;
     if (__ballot(qindex != 0x7FFFFFFF) == 0)
         return; // a cell without points (the last window of a cloud may have some)
     float4 qlo, qhi;
@@ -878,6 +890,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void three_nn_grid_kernel(
 
     const int groups = (ccells + NG_CELL - 1) / NG_CELL;
     unsigned seed_key = 0xFFFFFFFFu;
+#pragma unroll 4 // (the boxes of four groups on their way at a time: clusters 2 x 60000 551 -> 533 us, 16 x 16384 263 -> 258)
     for (int g = 0; g < groups; ++g)
     {
         const int c = g * NG_CELL + lane;
@@ -1609,14 +1622,17 @@ int tpk_grid_three_nn(int b, int n, int m, const float* unknown, const float* kn
             return st;
     }
     const int qcells = grid_cells(n), ccells = grid_cells(m);
-    const int64_t waves = static_cast<int64_t>(qcells) * b;
+    int64_t waves = static_cast<int64_t>(qcells) * b;
+    int log2_parts = 0;
+    for (; log2_parts < NG_MOST_PARTS && waves * 2 <= NG_PARTED_WAVES; ++log2_parts)
+        waves *= 2;
     const int64_t blocks = tpk_ceil_div(waves, NG_SCAN_THREADS / TPK_WAVE);
     if (blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
     const size_t lds = static_cast<size_t>(NG_SCAN_THREADS / TPK_WAVE) * ((ccells + NG_CELL - 1) / NG_CELL * NG_CELL) *
                        sizeof(float);
     hipLaunchKernelGGL(three_nn_grid_kernel, dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), lds, s, n,
-                       m, qcells, ccells, b, a.sorted, c.sorted, c.boxes, dist2, idx, root, only);
+                       m, qcells, ccells, b, a.sorted, c.sorted, c.boxes, dist2, idx, root, only, log2_parts);
     return tpk_launch_status();
 }
 
