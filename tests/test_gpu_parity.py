@@ -2393,6 +2393,47 @@ def test_chamfer_on_the_matrix_cores(dev, kind, n, m):
         assert torch.equal(cells, pairs)
 
 
+@pytest.mark.parametrize("B", [1, 28, 29, 113, 114])
+@pytest.mark.parametrize("kind", ["even", "nearly equal", "lattice", "scan", "not finite"])
+def test_chamfer_cells_shared_by_wavefronts(tpk, dev, kind, B):
+    """Four, two or one wavefront for a cell's queries, either side of the cells (512, 2048) at which that changes, with a last cell of one query:
+    the distances and indices of the scan of all pairs, bit for bit, and the loss of those distances."""
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_chamfer_fwd_workspace_bytes.restype = ctypes.c_size_t
+    n = m = 513
+    g = torch.Generator().manual_seed(B)
+    clouds = [torch.rand(B, count, 3, generator=g) for count in (n, m)]
+    if kind == "nearly equal":  # every point has a twin a few units in the last place away
+        clouds[1][:, m // 2 : 2 * (m // 2)] = clouds[1][:, : m // 2] * (1.0 + 2.0 ** -22)
+    elif kind == "lattice":
+        clouds = [torch.floor(c * 6) / 6 for c in clouds]
+    elif kind == "scan":
+        far = [1.5 * (50 / 1.5) ** c[..., 0] for c in clouds]
+        clouds = [torch.stack([r * torch.cos(6.2832 * c[..., 1]), r * torch.sin(6.2832 * c[..., 1]), 0.02 * c[..., 2] - 1.7], 2) for r, c in zip(far, clouds)]
+    elif kind == "not finite":
+        clouds[0][:, 7::97, 1] = float("nan")
+        clouds[1][:, 3::89, 2] = float("inf")
+    a, b = (c.contiguous().to(dev) for c in clouds)
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    results = []
+    for nbytes in (lib.tpk_chamfer_fwd_workspace_bytes(B, n, m), 0):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+        out = [torch.full((B, k), -1, dtype=t, device=dev) for t in (torch.float32, torch.int32) for k in (n, m)]
+        st = lib.tpk_chamfer_fwd_f32(B, n, m, pointer(a), pointer(b), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None)
+        assert st == 0
+        torch.cuda.synchronize()
+        results.append([t.cpu() for t in out])
+    for cells, pairs in zip(*results):
+        assert torch.equal(cells, pairs)
+    want = float(results[1][0].double().mean() + results[1][1].double().mean())
+    loss = float(tpk.chamfer_dist.chamfer_dist(a, b))
+    assert loss == want or abs(loss - want) <= 2.0 ** -23 * want  # (summed in float64: one rounding)
+
+
 @pytest.mark.parametrize("B,n,m", [(1, 512, 512), (3, 513, 640), (2, 16385, 520), (2048, 512, 512), (2049, 512, 512), (600, 700, 1100)])
 def test_chamfer_loss_from_the_searchs_sums(tpk, dev, B, n, m):
     """The loss of float32 clouds that the search over cells serves: padding in a cloud's last cell, cells without points behind a whole

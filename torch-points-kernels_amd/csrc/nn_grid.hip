@@ -300,15 +300,15 @@ __device__ __forceinline__ double wave_sum_f64(double v)
     return added_dpp<0x143, 0xC>(v); // row_bcast:31 into rows 2 and 3
 }
 
-// One wavefront = the 64 queries of one cell.  Logical wavefront number (after the die-local
-// block mapping) = cloud * (cells1 + cells2) + cell; the cells of cloud 1 query cloud 2 and
+// One wavefront = the 64 queries of one cell, or a half or a quarter of them.  Logical wavefront number (after the
+// die-local block mapping) = cloud * (cells1 + cells2) + cell, times the parts; the cells of cloud 1 query cloud 2 and
 // write dist1 / idx1, those of cloud 2 the other way round.
 __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
     int n, int m, int cells1, int cells2, int clouds, const float4* __restrict__ sorted1,
     const float4* __restrict__ sorted2, const float4* __restrict__ boxes1,
     const float4* __restrict__ boxes2, float* __restrict__ dist1, float* __restrict__ dist2,
     int32_t* __restrict__ idx1, int32_t* __restrict__ idx2, const int* __restrict__ wide1,
-    const int* __restrict__ wide2, int window_cells, int part_cells, double* __restrict__ sums)
+    const int* __restrict__ wide2, int window_cells, int part_cells, double* __restrict__ sums, int log2_parts)
 {
     __shared__ float4 stages[NG_SCAN_THREADS / TPK_WAVE][NG_CELL];
     extern __shared__ float lows_all[]; // [wavefronts][largest number of candidate cells, in whole groups of 64]
@@ -316,8 +316,10 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
     const int lane = threadIdx.x & (TPK_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TPK_WAVE);
     const int per_cloud = cells1 + cells2;
-    const int64_t task = static_cast<int64_t>(xcd_local_block(blockIdx.x, gridDim.x)) *
-                             (NG_SCAN_THREADS / TPK_WAVE) + wave;
+    const int64_t number = static_cast<int64_t>(xcd_local_block(blockIdx.x, gridDim.x)) *
+                               (NG_SCAN_THREADS / TPK_WAVE) + wave;
+    const int64_t task = number >> log2_parts;
+    const int part = static_cast<int>(number) & ((1 << log2_parts) - 1);
     if (task >= static_cast<int64_t>(per_cloud) * clouds)
         return; // (no workgroup barrier anywhere in this kernel)
     int cloud = static_cast<int>(task / per_cloud);
@@ -383,15 +385,18 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
 
     const float4 query = qpts[qcell * NG_CELL + lane];
     const float qx = query.x, qy = query.y, qz = query.z;
-    const int qindex = __float_as_int(query.w); // 0x7FFFFFFF: padding, nothing to store
-    double* const sum = sums + static_cast<int64_t>(cloud) * per_cloud + r;
+    // 0x7FFFFFFF: padding, nothing to store; so are the queries of the cell's other parts here
+    const int qindex = ((lane << log2_parts) / TPK_WAVE) == part ? __float_as_int(query.w) : 0x7FFFFFFF;
+    double* const sum = sums + ((static_cast<int64_t>(cloud) * per_cloud + r) << log2_parts) + part;
     if (__ballot(qindex != 0x7FFFFFFF) == 0) // a cell without points (the last window of a cloud may have some)
     {
         if (sums && lane == 0)
             *sum = 0.0;
         return;
     }
-    const float4 qlo = qbox[qcell * NG_BOX + 0], qhi = qbox[qcell * NG_BOX + 1];
+    float4 qlo = qbox[qcell * NG_BOX + 0], qhi = qbox[qcell * NG_BOX + 1];
+    if (log2_parts > 0)
+        query_box(qx, qy, qz, qindex != 0x7FFFFFFF, qlo, qhi);
 
     const int groups = (ccells + NG_CELL - 1) / NG_CELL;
     const bool real = qindex != 0x7FFFFFFF;
@@ -474,7 +479,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         MatrixNearest near[2];
         near[0].m1 = near[0].m2 = near[1].m1 = near[1].m2 = __float_as_int(__builtin_inff());
         near[0].cell = near[1].cell = seed;
-        matrix_scan(cpts, seed, ~0ull, lane, frame, queries, near);
+        matrix_scan(cpts, seed, __ballot(real), lane, frame, queries, near);
         TPK_WORK_ADD(NG_CELL);
         // the smallest product of the lane's query, and the squared distance that holds the query's answer for certain
         auto smallest = [&]() {
@@ -1505,6 +1510,17 @@ size_t tpk_grid_chamfer_workspace_bytes(int b, int n, int m)
 }
 
 namespace {
+// log2 of the wavefronts that share a cell's queries, as in three_nn's search, to fewer wavefronts: a scan on the matrix cores costs 32
+// queries what it costs 16, and a wavefront's set-up is a larger part of it.  Pass without gradients, us, whole / halves / quarters / eighths:
+// 1 x 16384 points, noisy sphere 44.5 / 39.4 / 37.5 / 38.7, eight clusters 74.6 / 70.1 / 64.1 / 59.5; 2 x 16384 46.6 / 43.0 / 43.6 / 48.1, 78.1 / 70.8 /
+// 66.7 / 68.6; 4 x 16384 49.3 / 48.1 / 52.0, 81.5 / 73.6 / 77.5, even 47.6 / 49.6 / 53.9; 8 x 16384 50.3 / 54.1, 82.2 / 80.7; laser scans of
+// 1, 2, 4 x 16384 132.9 -> 96.0, 136.9 -> 106.8, 144.0 -> 131.8 as here.
+int chamfer_parts(int b, int n, int m)
+{
+    const int64_t cells = static_cast<int64_t>(grid_cells(n) + grid_cells(m)) * b;
+    return cells <= 512 ? 2 : cells <= 2048 ? 1 : 0;
+}
+
 // sums: nullptr, or where the wavefronts' sums go, instead of the distances
 int grid_chamfer(int b, int n, int m, const float* xyz1, const float* xyz2, float* dist1, float* dist2, int32_t* idx1, int32_t* idx2,
                  void* workspace, double* sums, hipStream_t s)
@@ -1527,7 +1543,8 @@ int grid_chamfer(int b, int n, int m, const float* xyz1, const float* xyz2, floa
     if (st != TPK_OK)
         return st;
     const int cells1 = grid_cells(n), cells2 = grid_cells(m);
-    const int64_t waves = static_cast<int64_t>(cells1 + cells2) * b;
+    const int log2_parts = chamfer_parts(b, n, m);
+    const int64_t waves = static_cast<int64_t>(cells1 + cells2) * b << log2_parts;
     const int64_t blocks = tpk_ceil_div(waves, NG_SCAN_THREADS / TPK_WAVE);
     if (blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
@@ -1535,7 +1552,7 @@ int grid_chamfer(int b, int n, int m, const float* xyz1, const float* xyz2, floa
                        ((std::max(cells1, cells2) + NG_CELL - 1) / NG_CELL * NG_CELL) * sizeof(float);
     hipLaunchKernelGGL(chamfer_grid_kernel, dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), lds, s, n,
                        m, cells1, cells2, b, a.sorted, c.sorted, a.boxes, c.boxes, dist1, dist2, idx1, idx2, a.wide_first,
-                       c.wide_first, window_cells, static_cast<int>(tpk_ceil_div(set_cells(a), curve_parts(a, c))), sums);
+                       c.wide_first, window_cells, static_cast<int>(tpk_ceil_div(set_cells(a), curve_parts(a, c))), sums, log2_parts);
     return tpk_launch_status();
 }
 } // namespace
@@ -1556,7 +1573,7 @@ size_t tpk_grid_chamfer_loss_workspace_bytes(int b, int n, int m)
     if (!grid_supported(b, n, m))
         return 0;
     const int64_t waves = static_cast<int64_t>(grid_cells(n) + grid_cells(m)) * b;
-    return waves <= CT_MOST ? grid_layout(b, n, m, true).total + static_cast<size_t>(waves) * sizeof(double) : 0;
+    return waves <= CT_MOST ? grid_layout(b, n, m, true).total + (static_cast<size_t>(waves) << chamfer_parts(b, n, m)) * sizeof(double) : 0;
 }
 
 int tpk_grid_chamfer_loss(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1, int32_t* idx2, void* workspace,
@@ -1571,7 +1588,7 @@ int tpk_grid_chamfer_loss(int b, int n, int m, const float* xyz1, const float* x
     const int st = grid_chamfer(b, n, m, xyz1, xyz2, nullptr, nullptr, idx1, idx2, workspace, sums, s);
     if (st != TPK_OK)
         return st;
-    const int cells1 = grid_cells(n), per_cloud = cells1 + grid_cells(m);
+    const int log2_parts = chamfer_parts(b, n, m), cells1 = grid_cells(n) << log2_parts, per_cloud = cells1 + (grid_cells(m) << log2_parts);
     hipLaunchKernelGGL(chamfer_cells_loss_kernel, dim3(1), dim3(CT_THREADS), 0, s, per_cloud * b, per_cloud, cells1,
                        static_cast<double>(b) * n, static_cast<double>(b) * m, sums, loss);
     return tpk_launch_status();
