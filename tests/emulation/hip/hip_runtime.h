@@ -293,23 +293,101 @@ inline int __builtin_amdgcn_update_dpp(int old, int v, int control, int rows, in
 #define __builtin_amdgcn_s_waitcnt(x) static_cast<void>(0)
 inline float __builtin_amdgcn_rcpf(float v) { return 1.0f / v; }
 inline float __builtin_amdgcn_fmed3f(float a, float b, float c) { return fmaxf(fminf(a, b), fminf(fmaxf(a, b), c)); }
-// Chamfer's matrix products of halves are declared for the compiler only: the kernels run here have none.
-#if !defined(__FLT16_MAX__)
-typedef short _Float16;
-#endif
-template <typename V, typename W>
-inline W __builtin_amdgcn_mfma_f32_32x32x16_f16(V, V, W, int, int, int)
+// A product of nought and infinity is a NaN of either sign, as the hardware likes: here of the one that orders above everything as an integer.
+namespace emulation {
+inline float fused(float a, float b, float c)
 {
-    abort();
+    const float v = fmaf(a, b, c);
+    return v != v ? __builtin_nanf("") : v;
 }
-struct emulated_pair
+// Halves, rounded to nearest even, those below the normal range kept.  (The sources' vectors of them become these.)
+struct Half
+{
+    uint16_t bits;
+    Half() = default;
+    Half(float v)
+    {
+        const double size = fabs(static_cast<double>(v));
+        int exponent = -14;
+        if (size >= 0x1p-14 && size < 65536.0)
+            exponent = ilogb(size);
+        const double unit = ldexp(1.0, exponent - 10), rounded = nearbyint(size / unit);
+        int magnitude = 0x7C00;
+        if (size < 65520.0)
+            magnitude = static_cast<int>(rounded) + (exponent + 14) * 1024; // (a carry out of the mantissa is the next exponent)
+        bits = static_cast<uint16_t>(v != v ? 0x7E00 : magnitude | (std::signbit(v) ? 0x8000 : 0));
+    }
+    operator float() const
+    {
+        const int exponent = bits >> 10 & 31, mantissa = bits & 1023;
+        const double size = exponent == 31 ? (mantissa ? NAN : INFINITY)
+                            : exponent == 0 ? mantissa * 0x1p-24 : ldexp(1024 + mantissa, exponent - 25);
+        return static_cast<float>(bits >> 15 ? -size : size);
+    }
+};
+template <int N>
+struct Halves
+{
+    Half v[N];
+    Half operator[](int i) const { return v[i]; }
+};
+// How far a matrix product may be from the sum of its products, in units of the sum of their magnitudes.
+inline double product_error;
+inline uint64_t product_noise = 1;
+} // namespace emulation
+#define __builtin_fmaf emulation::fused
+#define _Float16 emulation::Half
+// Lane l of the operands: row (column) l % 32, slots 8 (l / 32) .. 8 (l / 32) + 7; of the result: column l % 32, rows r % 4 + 8 (r / 4) + 4 (l / 32).
+template <typename V, typename W>
+inline W __builtin_amdgcn_mfma_f32_32x32x16_f16(const V& a, const V& b, W c, int, int, int)
+{
+    static float as_float[1 << 16];
+    static bool made = false;
+    for (int i = 0; i < (1 << 16) && !made; ++i)
+    {
+        const uint16_t bits = static_cast<uint16_t>(i);
+        as_float[i] = __builtin_bit_cast(emulation::Half, bits);
+    }
+    made = true;
+    uint16_t row[emulation::WAVE][8], own[16];
+    for (int part = 0; part < 2; ++part)
+    {
+        uint64_t four;
+        memcpy(&four, reinterpret_cast<const char*>(&a) + part * 8, 8);
+        const uint64_t* all = emulation::exchange(four);
+        for (int l = 0; l < emulation::WAVE; ++l)
+            memcpy(&row[l][part * 4], &all[l], 8);
+        memcpy(&four, reinterpret_cast<const char*>(&b) + part * 8, 8);
+        all = emulation::exchange(four);
+        for (int l = 0; l < 2; ++l)
+            memcpy(&own[l * 8 + part * 4], &all[emulation::lane() % 32 + 32 * l], 8);
+    }
+    for (int r = 0; r < 16; ++r)
+    {
+        const int at = r % 4 + 8 * (r / 4) + 4 * (emulation::lane() / 32);
+        double sum = c[r], magnitudes = 0.0;
+        for (int k = 0; k < 16; ++k)
+        {
+            const double product = static_cast<double>(as_float[row[at + 32 * (k / 8)][k % 8]]) * as_float[own[k]];
+            sum += product;
+            magnitudes += fabs(product);
+        }
+        emulation::product_noise = emulation::product_noise * 6364136223846793005ull + 1442695040888963407ull;
+        c[r] = static_cast<float>(sum + (emulation::product_noise >> 63 ? 1.0 : -1.0) * emulation::product_error * magnitudes);
+    }
+    return c;
+}
+struct EmulatedPair
 {
     unsigned v[2];
     unsigned operator[](int i) const { return v[i]; }
 };
-inline emulated_pair __builtin_amdgcn_permlane32_swap(unsigned, unsigned, bool, bool)
+// The lanes 32 .. 63 of the first and the lanes 0 .. 31 of the second change places.
+inline EmulatedPair __builtin_amdgcn_permlane32_swap(unsigned first, unsigned second, bool, bool)
 {
-    abort();
+    const uint64_t* all = emulation::exchange(static_cast<uint64_t>(second) << 32 | first);
+    const int lane = emulation::lane();
+    return {{lane < 32 ? first : static_cast<unsigned>(all[lane - 32] >> 32), lane < 32 ? static_cast<unsigned>(all[lane + 32]) : second}};
 }
 inline unsigned __builtin_amdgcn_mbcnt_lo(unsigned mask, unsigned add)
 {

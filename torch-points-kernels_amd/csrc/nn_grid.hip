@@ -466,7 +466,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         const float square = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z));
         const float own_error = __builtin_fmaf(square, MX_ERROR, 0.0625f);
         const float unit = 1.f / (frame.scale * frame.scale);
-        const float reach_factor = real ? (1.f + MX_ERROR) * unit : 0.f, reach_error = real ? own_error * unit : -1.f;
+        const float reach_factor = (1.f + MX_ERROR) * unit, reach_error = own_error * unit;
         half8_t queries[2];
         {
             half2_t xy_high, xy_low, z_high, z_low, s_high, s_low;
@@ -481,14 +481,16 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         near[0].cell = near[1].cell = seed;
         matrix_scan(cpts, seed, __ballot(real), lane, frame, queries, near);
         TPK_WORK_ADD(NG_CELL);
-        // the smallest product of the lane's query, and the squared distance that holds the query's answer for certain
+        // The smallest product of the lane's query, and the squared distance that holds the query's answer for certain.  (A tile
+        // without a query is never scanned: its m1 stay infinite.  No lane without a query may reach for anything.)
         auto smallest = [&]() {
             int a, b;
             by_query(near[0].m1, near[1].m1, a, b);
             return __int_as_float(max(min(a, b), 0));
         };
         float m = smallest();
-        reach = __builtin_fmaf(m, reach_factor, reach_error);
+        auto reach_of = [&](float product) { return real ? __builtin_fmaf(product, reach_factor, reach_error) : -1.f; };
+        reach = reach_of(m);
         // (where the first cell's second smallest products are near the error already, the search would leave the queries over)
         int c2, d2;
         by_query(near[0].m2, near[1].m2, c2, d2);
@@ -515,7 +517,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
                             continue;
                         matrix_scan(cpts, c, want, lane, frame, queries, near);
                         TPK_WORK_ADD(NG_CELL);
-                        reach = __builtin_fmaf(smallest(), reach_factor, reach_error);
+                        reach = reach_of(smallest());
                         if (phase)
                         {
                             bound = __int_as_float(wave_max_i32(__float_as_int(reach)));
