@@ -298,9 +298,9 @@ int tpk_group_recording_f32(int b, int c, int n, int npoint, int nsample, const 
  * arguments are kept for callers written against earlier versions and are ignored): the points
  * that chose a point as nearest neighbour are chained to it in LDS.  Clouds of more than about
  * 38000 points scatter with hardware float atomics instead.
- * tpk_chamfer_fwd_loss_f32: tpk_chamfer_fwd_f32 and tpk_chamfer_loss_f32 in one, without the distances, in
- * tpk_chamfer_fwd_loss_workspace_bytes() bytes (0: a shape it does not serve, TPK_ERR_UNSUPPORTED); summed in float64, a cell
- * of neighbouring points at a time, those of a cell in no fixed order.
+ * tpk_chamfer_fwd_loss_f32: tpk_chamfer_fwd_f32 and tpk_chamfer_loss_f32 in one, the distances in the workspace, 256-byte aligned, of
+ * tpk_chamfer_fwd_loss_workspace_bytes() bytes (0: a shape it does not serve, TPK_ERR_UNSUPPORTED: clouds below 512 points, more
+ * than 32768 cells of 64 points of both clouds); the loss those two calls return, bit for bit.
  * tpk_chamfer_loss_*: *loss = mean(dist1) + mean(dist2) of the whole batch, summed in float64 in a
  * fixed order (`workspace`: tpk_chamfer_loss_workspace_bytes() bytes, 8-byte aligned; NaN where a
  * mean is over nothing).  tpk_chamfer_loss_bwd_*: the backward pass for that loss: grad_loss is one

@@ -27,7 +27,7 @@ def test_header_declares_the_expected_entry_points():
         "tpk_grow_places", "tpk_grow_rows", "tpk_grow_rows_part", "tpk_grow_members", "tpk_region_order_workspace_bytes", "tpk_region_order", "tpk_region_members",
         "tpk_three_nn_workspace_bytes", "tpk_three_nn_f32", "tpk_knn_workspace_bytes", "tpk_knn_f32", "tpk_three_interpolate_f32", "tpk_three_interpolate_grad_f32", "tpk_group_f32",
         "tpk_three_interpolate_lists_f32", "tpk_three_interpolate_grad_lists_f32", "tpk_group_lists", "tpk_group_grad_lists_f32",
-        "tpk_group_grad_f32", "tpk_chamfer_fwd_workspace_bytes", "tpk_chamfer_fwd_f32", "tpk_chamfer_fwd_f64", "tpk_chamfer_bwd_f32",
+        "tpk_group_grad_f32", "tpk_chamfer_fwd_workspace_bytes", "tpk_chamfer_fwd_f32", "tpk_chamfer_fwd_f64", "tpk_chamfer_fwd_loss_workspace_bytes", "tpk_chamfer_fwd_loss_f32", "tpk_chamfer_bwd_f32",
         "tpk_chamfer_bwd_f64", "tpk_grow_proximity_workspace_bytes", "tpk_grow_proximity", "tpk_instance_iou", "tpk_gridding_f32", "tpk_gridding_f64", "tpk_gridding_grad_f32",
         "tpk_gridding_grad_f64", "tpk_cubic_feature_sampling_f32", "tpk_cubic_feature_sampling_f64",
         "tpk_cubic_feature_sampling_grad_f32", "tpk_cubic_feature_sampling_grad_f64", "tpk_ball_query_sorted_dense_workspace_bytes",
@@ -59,6 +59,30 @@ def test_sorted_packed_ball_query_builds_no_table_for_few_queries():
         got, bins, with_table = sizes[0](L(n), L(m)), sizes[1](L(n), L(m), 64), sizes[2](L(n), L(m), 64)
         assert bins < with_table
         assert (got >= with_table) == table and got >= bins, (n, m)
+
+
+def test_chamfer_loss_in_one_call_refuses_what_it_does_not_serve():
+    """tpk_chamfer_fwd_loss_f32 takes the search's shapes up to 32768 cells of 64 points, in a workspace that also holds the distances;
+    a missing, short or misaligned one and missing arrays are refused before anything is launched."""
+    lib = ctypes.CDLL(LIB)
+    for name in ("tpk_chamfer_fwd_workspace_bytes", "tpk_chamfer_fwd_loss_workspace_bytes", "tpk_chamfer_loss_workspace_bytes"):
+        getattr(lib, name).restype = ctypes.c_size_t
+    size, search, shares = lib.tpk_chamfer_fwd_loss_workspace_bytes, lib.tpk_chamfer_fwd_workspace_bytes, lib.tpk_chamfer_loss_workspace_bytes
+    for b, n, m in ((1, 511, 600), (1, 600, 511), (0, 600, 600), (-1, 600, 600), (2049, 512, 512), (1, 200000, 600)):
+        assert size(b, n, m) == 0, (b, n, m)
+    up = lambda v: (v + 255) // 256 * 256
+    for b, n, m in ((1, 512, 512), (2048, 512, 512), (3, 700, 20000), (32, 16384, 16384)):
+        assert size(b, n, m) == up(up(search(b, n, m)) + 4 * b * (n + m)) + shares(b, n, m), (b, n, m)
+    INVALID, UNSUPPORTED, WORKSPACE = -1, -2, -3
+    p, ws = ctypes.c_void_p(4096), ctypes.c_void_p(1 << 20)  # (never reached)
+    need = size(1, 600, 700)
+    call = lambda b, n, m, arrays, workspace, nbytes: lib.tpk_chamfer_fwd_loss_f32(b, n, m, *arrays, workspace, ctypes.c_size_t(nbytes), None)
+    for missing in range(5):
+        assert call(1, 600, 700, [p] * missing + [None] + [p] * (4 - missing), ws, need) == INVALID
+    assert call(1, 511, 700, [p] * 5, ws, need) == UNSUPPORTED
+    assert call(1, 600, 700, [p] * 5, None, need) == WORKSPACE
+    assert call(1, 600, 700, [p] * 5, ws, need - 1) == WORKSPACE
+    assert call(1, 600, 700, [p] * 5, ctypes.c_void_p((1 << 20) + 128), need) == WORKSPACE
 
 
 def test_counting_build_exports_the_same_abi_plus_its_reader():

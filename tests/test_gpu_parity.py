@@ -2437,7 +2437,7 @@ def test_chamfer_cells_shared_by_wavefronts(tpk, dev, kind, B):
 @pytest.mark.parametrize("B,n,m", [(1, 512, 512), (3, 513, 640), (2, 16385, 520), (2048, 512, 512), (2049, 512, 512), (600, 700, 1100)])
 def test_chamfer_loss_from_the_searchs_sums(tpk, dev, B, n, m):
     """The loss of float32 clouds that the search over cells serves: padding in a cloud's last cell, cells without points behind a whole
-    window, as many wavefronts as leave sums (32768) and one cloud more, whose distances are stored and read again."""
+    window, as many cells (32768) as the call for the loss alone takes and one cloud more."""
     g = torch.Generator(device=dev).manual_seed(B + n + m)
     a, b = (torch.rand(B, k, 3, generator=g, device=dev) for k in (n, m))
     loss = tpk.chamfer_dist.chamfer_dist(a, b)
@@ -2445,6 +2445,45 @@ def test_chamfer_loss_from_the_searchs_sums(tpk, dev, B, n, m):
     want = float(d1.double().mean() + d2.double().mean())
     # (sums in float64 on either side: their rounding is far below the one rounding of the result)
     assert abs(float(loss) - want) <= 2.0 ** -23 * want
+
+
+def test_chamfer_loss_is_summed_in_a_fixed_order(tpk, dev):
+    """One distance of 1, one of half of its last place and four that are lost one by one beside it and not together: whether the loss is
+    rounded up tells in which order it was summed, and that order depends on the sizes only.  (The sum of every cell of neighbouring points by
+    itself, the points of a cell in no fixed order, gave another loss in a part of these clouds.)"""
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    for f in ("tpk_chamfer_fwd_workspace_bytes", "tpk_chamfer_loss_workspace_bytes", "tpk_chamfer_fwd_loss_workspace_bytes"):
+        getattr(lib, f).restype = ctypes.c_size_t
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    room = lambda nbytes: torch.zeros(max(nbytes, 1), dtype=torch.uint8, device=dev)
+    n = 1024
+    at = torch.arange(n)
+    lattice = torch.stack([torch.zeros(n), 4.0 * (at % 32), 4.0 * (at // 32)], 1)
+    rounded_up = 0
+    for seed in range(200):
+        g = torch.Generator().manual_seed(seed)
+        chosen = torch.randperm(n, generator=g)[:6]
+        moved = lattice.clone()
+        moved[chosen, 0] = torch.tensor([1.0, 2.0**-12, 2.0**-27, 2.0**-27, 2.0**-27, 2.0**-27])
+        a, b = lattice[None].contiguous().to(dev), moved[None].contiguous().to(dev)
+        d = [torch.empty(1, n, device=dev) for _ in range(2)]
+        i = [torch.empty(1, n, dtype=torch.int32, device=dev) for _ in range(2)]
+        want, one_call = torch.empty((), device=dev), torch.empty((), device=dev)
+        search, shares, both = (int(getattr(lib, "tpk_chamfer_%s_workspace_bytes" % k)(1, n, n)) for k in ("fwd", "loss", "fwd_loss"))
+        ws, sums, ws2 = room(search), room(shares), room(both)
+        size = ctypes.c_size_t
+        assert lib.tpk_chamfer_fwd_f32(1, n, n, pointer(a), pointer(b), *(pointer(t) for t in d + i), pointer(ws), size(search), None) == 0
+        assert lib.tpk_chamfer_loss_f32(1, n, n, pointer(d[0]), pointer(d[1]), pointer(want), pointer(sums), size(shares), None) == 0
+        assert lib.tpk_chamfer_fwd_loss_f32(1, n, n, pointer(a), pointer(b), pointer(one_call), *(pointer(t) for t in i), pointer(ws2), size(both), None) == 0
+        torch.cuda.synchronize()
+        loss = tpk.chamfer_dist.chamfer_dist(a, b)
+        assert float(loss) == float(want) == float(one_call), seed
+        rounded_up += float(want) > 2.0 * 2.0**-10
+    assert 0 < rounded_up < 200  # (so that the order decides)
 
 
 def test_chamfer_gradcheck_double(tpk, dev):

@@ -751,19 +751,6 @@ extern "C" int tpk_chamfer_fwd_f32(int b, int n, int m, const float* xyz1, const
     return chamfer_fwd<float>(b, n, m, xyz1, xyz2, dist1, dist2, idx1, idx2, stream);
 }
 
-extern "C" size_t tpk_chamfer_fwd_loss_workspace_bytes(int b, int n, int m)
-{
-    return tpk_grid_chamfer_loss_workspace_bytes(b, n, m);
-}
-
-extern "C" int tpk_chamfer_fwd_loss_f32(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1,
-                                        int32_t* idx2, void* workspace, size_t workspace_bytes, void* stream)
-{
-    if (!xyz1 || !xyz2 || !loss || !idx1 || !idx2)
-        return TPK_ERR_INVALID_ARG;
-    return tpk_grid_chamfer_loss(b, n, m, xyz1, xyz2, loss, idx1, idx2, workspace, workspace_bytes, tpk_stream(stream));
-}
-
 extern "C" int tpk_chamfer_fwd_f64(int b, int n, int m, const double* xyz1, const double* xyz2,
                                    double* dist1, double* dist2, int32_t* idx1, int32_t* idx2,
                                    void* stream)
@@ -809,6 +796,50 @@ extern "C" size_t tpk_chamfer_loss_workspace_bytes(int b, int n, int m)
         return 0;
     const int blocks = mean_blocks(static_cast<int64_t>(b) * n + static_cast<int64_t>(b) * m);
     return blocks > 1 ? blocks * sizeof(double) : 0;
+}
+
+namespace {
+// The search's workspace, the distances, the shares of their means (of 0 bytes: a shape tpk_chamfer_fwd_loss_f32 does not serve).
+struct LossLayout
+{
+    size_t search, dist, shares, total;
+};
+LossLayout loss_layout(int b, int n, int m)
+{
+    constexpr int64_t MOST_CELLS = 32768; // of 64 points; callers of larger ones have their own room for distances
+    LossLayout l{};
+    const size_t search = tpk_grid_chamfer_workspace_bytes(b, n, m);
+    if (search == 0 || tpk_grid_chamfer_cells(b, n, m) > MOST_CELLS)
+        return l;
+    const size_t points = static_cast<size_t>(b) * (static_cast<size_t>(n) + static_cast<size_t>(m));
+    l.search = search;
+    l.dist = (search + 255) & ~static_cast<size_t>(255);
+    l.shares = (l.dist + points * sizeof(float) + 255) & ~static_cast<size_t>(255);
+    l.total = l.shares + tpk_chamfer_loss_workspace_bytes(b, n, m);
+    return l;
+}
+} // namespace
+
+extern "C" size_t tpk_chamfer_fwd_loss_workspace_bytes(int b, int n, int m)
+{
+    return loss_layout(b, n, m).total;
+}
+
+extern "C" int tpk_chamfer_fwd_loss_f32(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1,
+                                        int32_t* idx2, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (!xyz1 || !xyz2 || !loss || !idx1 || !idx2)
+        return TPK_ERR_INVALID_ARG;
+    const LossLayout l = loss_layout(b, n, m);
+    if (l.total == 0)
+        return TPK_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+        return TPK_ERR_WORKSPACE;
+    char* const bytes = static_cast<char*>(workspace);
+    float* const dist1 = reinterpret_cast<float*>(bytes + l.dist);
+    float* const dist2 = dist1 + static_cast<size_t>(b) * n;
+    const int st = tpk_grid_chamfer_fwd(b, n, m, xyz1, xyz2, dist1, dist2, idx1, idx2, workspace, l.search, tpk_stream(stream));
+    return st != TPK_OK ? st : chamfer_loss<float>(b, n, m, dist1, dist2, loss, bytes + l.shares, l.total - l.shares, stream);
 }
 
 extern "C" int tpk_chamfer_loss_f32(int b, int n, int m, const float* dist1, const float* dist2, float* loss,

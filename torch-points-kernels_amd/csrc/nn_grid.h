@@ -7,17 +7,13 @@
 // Bytes of workspace tpk_grid_chamfer_fwd needs for b pairs of n- and m-point clouds; 0 when it
 // does not serve that shape (callers then use the all-pairs scan).
 size_t tpk_grid_chamfer_workspace_bytes(int b, int n, int m);
+int64_t tpk_grid_chamfer_cells(int b, int n, int m); // cells of 64 queries, both directions (of a shape it serves)
 
 // Chamfer forward, both directions, float32.  TPK_ERR_UNSUPPORTED when the shape is not served,
 // TPK_ERR_WORKSPACE when the workspace is missing, too small or not 256-byte aligned.
 int tpk_grid_chamfer_fwd(int b, int n, int m, const float* xyz1, const float* xyz2, float* dist1,
                          float* dist2, int32_t* idx1, int32_t* idx2, void* workspace,
                          size_t workspace_bytes, hipStream_t stream);
-
-// *loss = mean(dist1) + mean(dist2) in their place, summed in float64: same conventions, a workspace of its own (0: not served).
-size_t tpk_grid_chamfer_loss_workspace_bytes(int b, int n, int m);
-int tpk_grid_chamfer_loss(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1, int32_t* idx2, void* workspace,
-                          size_t workspace_bytes, hipStream_t stream);
 
 // three_nn, float32: same conventions.  The workspace ends with one word per cloud
 // (tpk_grid_three_nn_flags: its address, or nullptr when the workspace does not serve the shape); with

@@ -281,25 +281,6 @@ __device__ __forceinline__ void matrix_scan(const float4* __restrict__ cand, int
     }
 }
 
-// Sum over the wavefront, in its last lane.
-template <int CONTROL, int ROWS>
-__device__ __forceinline__ double added_dpp(double v)
-{
-    const long long bits = __builtin_bit_cast(long long, v);
-    const int low = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits), CONTROL, ROWS, 0xF, false);
-    const int high = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits >> 32), CONTROL, ROWS, 0xF, false);
-    return v + __builtin_bit_cast(double, static_cast<long long>(high) << 32 | static_cast<unsigned>(low));
-}
-__device__ __forceinline__ double wave_sum_f64(double v)
-{
-    v = added_dpp<0xB1, 0xF>(v);  // quad_perm [1,0,3,2]
-    v = added_dpp<0x4E, 0xF>(v);  // quad_perm [2,3,0,1]
-    v = added_dpp<0x141, 0xF>(v); // row_half_mirror
-    v = added_dpp<0x140, 0xF>(v); // row_mirror
-    v = added_dpp<0x142, 0xA>(v); // row_bcast:15 into rows 1 and 3
-    return added_dpp<0x143, 0xC>(v); // row_bcast:31 into rows 2 and 3
-}
-
 // One wavefront = the 64 queries of one cell, or a half or a quarter of them.  Logical wavefront number (after the
 // die-local block mapping) = cloud * (cells1 + cells2) + cell, times the parts; the cells of cloud 1 query cloud 2 and
 // write dist1 / idx1, those of cloud 2 the other way round.
@@ -308,7 +289,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
     const float4* __restrict__ sorted2, const float4* __restrict__ boxes1,
     const float4* __restrict__ boxes2, float* __restrict__ dist1, float* __restrict__ dist2,
     int32_t* __restrict__ idx1, int32_t* __restrict__ idx2, const int* __restrict__ wide1,
-    const int* __restrict__ wide2, int window_cells, int part_cells, double* __restrict__ sums, int log2_parts)
+    const int* __restrict__ wide2, int window_cells, int part_cells, int log2_parts)
 {
     __shared__ float4 stages[NG_SCAN_THREADS / TPK_WAVE][NG_CELL];
     extern __shared__ float lows_all[]; // [wavefronts][largest number of candidate cells, in whole groups of 64]
@@ -387,13 +368,8 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
     const float qx = query.x, qy = query.y, qz = query.z;
     // 0x7FFFFFFF: padding, nothing to store; so are the queries of the cell's other parts here
     const int qindex = ((lane << log2_parts) / TPK_WAVE) == part ? __float_as_int(query.w) : 0x7FFFFFFF;
-    double* const sum = sums + ((static_cast<int64_t>(cloud) * per_cloud + r) << log2_parts) + part;
-    if (__ballot(qindex != 0x7FFFFFFF) == 0) // a cell without points (the last window of a cloud may have some)
-    {
-        if (sums && lane == 0)
-            *sum = 0.0;
-        return;
-    }
+    if (__ballot(qindex != 0x7FFFFFFF) == 0)
+        return; // a cell without points (the last window of a cloud may have some)
     float4 qlo = qbox[qcell * NG_BOX + 0], qhi = qbox[qcell * NG_BOX + 1];
     if (log2_parts > 0)
         query_box(qx, qy, qz, qindex != 0x7FFFFFFF, qlo, qhi);
@@ -655,62 +631,10 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         bi = lane == q ? lowest : bi;
     }
     TPK_WORK_FLUSH
-    if (sums) // (the loss alone: nobody wants the distances)
-    {
-        const double all = wave_sum_f64(real ? static_cast<double>(best) : 0.0);
-        if (lane == TPK_WAVE - 1)
-            *sum = all;
-    }
     if (real)
     {
-        if (!sums)
-            dout[qindex] = best;
+        dout[qindex] = best;
         iout[qindex] = bi == 0x7FFFFFFF ? 0 : bi;
-    }
-}
-
-// Mean of the distances of both directions, added, from what the wavefronts of the search left: a workgroup, as the
-// sums are few (16384 for 32 pairs of 16384 points, of 4.2 MB of distances that are never written); 5 us, latency.  The loss of those and its
-// gradient 101.6 -> 100.1 us: a launch and the scattered stores of the distances less, 25 instructions per wavefront of the search more.
-constexpr int CT_THREADS = 1024;
-constexpr int64_t CT_MOST = 32768; // sums
-__global__ __launch_bounds__(CT_THREADS) void chamfer_cells_loss_kernel(int count, int per_cloud, int cells1, double total1, double total2,
-                                                                       const double* __restrict__ sums, float* __restrict__ loss)
-{
-    __shared__ double of_wave[2][CT_THREADS / TPK_WAVE];
-    constexpr int BATCH = 16; // loads in flight per lane
-    double first = 0.0, second = 0.0;
-    for (int at = threadIdx.x; at < count; at += BATCH * CT_THREADS)
-    {
-        double v[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-            v[u] = at + u * CT_THREADS < count ? sums[at + u * CT_THREADS] : 0.0;
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-        {
-            const bool in_second = (at + u * CT_THREADS) % per_cloud >= cells1;
-            first += in_second ? 0.0 : v[u];
-            second += in_second ? v[u] : 0.0;
-        }
-    }
-    first = wave_sum_f64(first);
-    second = wave_sum_f64(second);
-    if (threadIdx.x % TPK_WAVE == TPK_WAVE - 1)
-    {
-        of_wave[0][threadIdx.x / TPK_WAVE] = first;
-        of_wave[1][threadIdx.x / TPK_WAVE] = second;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        first = second = 0.0;
-        for (int w = 0; w < CT_THREADS / TPK_WAVE; ++w)
-        {
-            first += of_wave[0][w];
-            second += of_wave[1][w];
-        }
-        *loss = static_cast<float>(first / total1 + second / total2);
     }
 }
 
@@ -1511,6 +1435,11 @@ size_t tpk_grid_chamfer_workspace_bytes(int b, int n, int m)
     return grid_supported(b, n, m) ? grid_layout(b, n, m, true).total : 0;
 }
 
+int64_t tpk_grid_chamfer_cells(int b, int n, int m)
+{
+    return static_cast<int64_t>(grid_cells(n) + grid_cells(m)) * b;
+}
+
 namespace {
 // log2 of the wavefronts that share a cell's queries, as in three_nn's search, to fewer wavefronts: a scan on the matrix cores costs 32
 // queries what it costs 16, and a wavefront's set-up is a larger part of it.  Pass without gradients, us, whole / halves / quarters / eighths:
@@ -1519,15 +1448,20 @@ namespace {
 // 1, 2, 4 x 16384 132.9 -> 96.0, 136.9 -> 106.8, 144.0 -> 131.8 as here.
 int chamfer_parts(int b, int n, int m)
 {
-    const int64_t cells = static_cast<int64_t>(grid_cells(n) + grid_cells(m)) * b;
+    const int64_t cells = tpk_grid_chamfer_cells(b, n, m);
     return cells <= 512 ? 2 : cells <= 2048 ? 1 : 0;
 }
+} // namespace
 
-// sums: nullptr, or where the wavefronts' sums go, instead of the distances
-int grid_chamfer(int b, int n, int m, const float* xyz1, const float* xyz2, float* dist1, float* dist2, int32_t* idx1, int32_t* idx2,
-                 void* workspace, double* sums, hipStream_t s)
+int tpk_grid_chamfer_fwd(int b, int n, int m, const float* xyz1, const float* xyz2, float* dist1,
+                         float* dist2, int32_t* idx1, int32_t* idx2, void* workspace,
+                         size_t workspace_bytes, hipStream_t s)
 {
+    if (!grid_supported(b, n, m) || static_cast<int64_t>(b) * 2 > 0x7fffffffLL)
+        return TPK_ERR_UNSUPPORTED;
     const GridLayout l = grid_layout(b, n, m, true);
+    if (!workspace || workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+        return TPK_ERR_WORKSPACE;
     char* w = static_cast<char*>(workspace);
     PointSet a{xyz1, nullptr, static_cast<int64_t>(b) * n, n, grid_stride(n), reinterpret_cast<float4*>(w + l.sorted_a),
                reinterpret_cast<float4*>(w + l.boxes_a), nullptr, nullptr, nullptr};
@@ -1546,7 +1480,7 @@ int grid_chamfer(int b, int n, int m, const float* xyz1, const float* xyz2, floa
         return st;
     const int cells1 = grid_cells(n), cells2 = grid_cells(m);
     const int log2_parts = chamfer_parts(b, n, m);
-    const int64_t waves = static_cast<int64_t>(cells1 + cells2) * b << log2_parts;
+    const int64_t waves = tpk_grid_chamfer_cells(b, n, m) << log2_parts;
     const int64_t blocks = tpk_ceil_div(waves, NG_SCAN_THREADS / TPK_WAVE);
     if (blocks > 0x7fffffffLL)
         return TPK_ERR_UNSUPPORTED;
@@ -1554,45 +1488,7 @@ int grid_chamfer(int b, int n, int m, const float* xyz1, const float* xyz2, floa
                        ((std::max(cells1, cells2) + NG_CELL - 1) / NG_CELL * NG_CELL) * sizeof(float);
     hipLaunchKernelGGL(chamfer_grid_kernel, dim3(static_cast<unsigned>(blocks)), dim3(NG_SCAN_THREADS), lds, s, n,
                        m, cells1, cells2, b, a.sorted, c.sorted, a.boxes, c.boxes, dist1, dist2, idx1, idx2, a.wide_first,
-                       c.wide_first, window_cells, static_cast<int>(tpk_ceil_div(set_cells(a), curve_parts(a, c))), sums, log2_parts);
-    return tpk_launch_status();
-}
-} // namespace
-
-int tpk_grid_chamfer_fwd(int b, int n, int m, const float* xyz1, const float* xyz2, float* dist1,
-                         float* dist2, int32_t* idx1, int32_t* idx2, void* workspace,
-                         size_t workspace_bytes, hipStream_t s)
-{
-    if (!grid_supported(b, n, m) || static_cast<int64_t>(b) * 2 > 0x7fffffffLL)
-        return TPK_ERR_UNSUPPORTED;
-    if (!workspace || workspace_bytes < grid_layout(b, n, m, true).total || (reinterpret_cast<uintptr_t>(workspace) & 255u))
-        return TPK_ERR_WORKSPACE;
-    return grid_chamfer(b, n, m, xyz1, xyz2, dist1, dist2, idx1, idx2, workspace, nullptr, s);
-}
-
-size_t tpk_grid_chamfer_loss_workspace_bytes(int b, int n, int m)
-{
-    if (!grid_supported(b, n, m))
-        return 0;
-    const int64_t waves = static_cast<int64_t>(grid_cells(n) + grid_cells(m)) * b;
-    return waves <= CT_MOST ? grid_layout(b, n, m, true).total + (static_cast<size_t>(waves) << chamfer_parts(b, n, m)) * sizeof(double) : 0;
-}
-
-int tpk_grid_chamfer_loss(int b, int n, int m, const float* xyz1, const float* xyz2, float* loss, int32_t* idx1, int32_t* idx2, void* workspace,
-                          size_t workspace_bytes, hipStream_t s)
-{
-    const size_t need = tpk_grid_chamfer_loss_workspace_bytes(b, n, m);
-    if (need == 0)
-        return TPK_ERR_UNSUPPORTED;
-    if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u))
-        return TPK_ERR_WORKSPACE;
-    double* const sums = reinterpret_cast<double*>(static_cast<char*>(workspace) + grid_layout(b, n, m, true).total);
-    const int st = grid_chamfer(b, n, m, xyz1, xyz2, nullptr, nullptr, idx1, idx2, workspace, sums, s);
-    if (st != TPK_OK)
-        return st;
-    const int log2_parts = chamfer_parts(b, n, m), cells1 = grid_cells(n) << log2_parts, per_cloud = cells1 + (grid_cells(m) << log2_parts);
-    hipLaunchKernelGGL(chamfer_cells_loss_kernel, dim3(1), dim3(CT_THREADS), 0, s, per_cloud * b, per_cloud, cells1,
-                       static_cast<double>(b) * n, static_cast<double>(b) * m, sums, loss);
+                       c.wide_first, window_cells, static_cast<int>(tpk_ceil_div(set_cells(a), curve_parts(a, c))), log2_parts);
     return tpk_launch_status();
 }
 

@@ -1253,14 +1253,6 @@ std::vector<at::Tensor> chamfer_loss_forward(const at::Tensor& xyz1, const at::T
     at::Tensor loss = torch::empty({}, xyz1.options());
     int32_t* const idx1 = idx.data_ptr<int32_t>();
     void* const s = current_stream(xyz1);
-    if (const size_t loss_bytes = narrow ? tpk_chamfer_fwd_loss_workspace_bytes(b, n, m) : 0)
-    {
-        at::Tensor scratch = torch::empty({static_cast<int64_t>(loss_bytes)}, xyz1.options().dtype(at::kByte));
-        check_status(tpk_chamfer_fwd_loss_f32(b, n, m, xyz1.data_ptr<float>(), xyz2.data_ptr<float>(), loss.data_ptr<float>(), idx1, idx1 + total1,
-                                              scratch.data_ptr(), loss_bytes, s),
-                     "chamfer_dist");
-        return {loss, idx};
-    }
     // one scratch: the search's workspace, the sums' workspace, the distances
     const size_t ws_bytes = narrow ? tpk_chamfer_fwd_workspace_bytes(b, n, m) : 0, sum_bytes = tpk_chamfer_loss_workspace_bytes(b, n, m);
     const size_t sums_at = (ws_bytes + 255) & ~static_cast<size_t>(255), dist_at = (sums_at + sum_bytes + 255) & ~static_cast<size_t>(255);
