@@ -157,14 +157,13 @@ __device__ __forceinline__ void scan_cell_few(const float4* __restrict__ cand, i
 // float, 0.44; the frame 0.2; the sum of 16 products 0.25 (2^-22 of the sum of their magnitudes: twice the 2^-23.05 that a million
 // products reached, and halves below the normal range are not flushed).  With the two bits that a smallest product gives up for
 // its place that is below 2^-17 (|q|^2 + |p - q|^2), as (|p| + |q|)^2 <= 5 |q|^2 + 5 |p - q|^2, and 2^-6 where a low half is below the normal
-// range.  A query for which the eight and some other candidate are closer together than that (one in 2000 of even clouds, one in
-// 500 on a sphere) goes to the pass for equal minima; where more than MX_PASS of a wavefront's do, the exact scan above answers them, a
-// search of its own that starts with what is known: serving 64 of them one at a time took 2.8 times as long on clouds with outliers.
+// range.  A query for which the eight and some other candidate are closer together than that (of 32 x 16384 points one in 3600 of even clouds, one
+// in 1200 on a sphere) goes to the pass for equal minima; where many of a wavefront's do, the exact scan above answers them, a search of
+// its own that starts with what is known: serving 64 of them one at a time took 2.8 times as long on clouds with outliers.
 //
 // What bounds it: the issue of vector instructions, ~105 for 64 x 64 pairs (22 to form the halves, 60 for the minima) where the
 // exact scan takes ten per candidate.  32 x 16384 points of noisy surfaces: search 121 -> 58 us, whole call 144 -> 86; uniform 143 -> 98, eight
-// clusters 176 -> 89; 8 x 1024 against 16384 109 -> 53, 2 x 60000 159 -> 102, one cloud of 160000 455 -> 281; laser scans of 8 x 16384
-// 266 -> 254, of 2 x 60000 821 -> 917 (cells that are wide for their points' distances leave half of the queries over).
+// clusters 176 -> 89; 8 x 1024 against 16384 109 -> 53, 2 x 60000 159 -> 102, one cloud of 160000 455 -> 281.
 // Taken back: minima of four candidates (24 more instructions per scan, 12 % slower), whole wavefronts by the exact scan where many
 // queries are left over (laser scans 30 % slower than without the matrix cores).
 typedef _Float16 half2_t __attribute__((vector_size(4)));
@@ -176,11 +175,26 @@ constexpr float MX_FAR = 16384.f;          // 2^14: candidates are clamped to th
 constexpr float MX_LIMIT = 134217728.f;    // 2^27: a squared distance that no clamped candidate can have
 constexpr float MX_NEAR = 8.f;             // largest distance of the first cell, in extents of its box and the queries'
 constexpr float MX_ERROR = 0x1p-17f;       // of |q|^2 and of a product (above)
-// A wavefront is left to the exact scan at once where for more than MX_MANY queries two groups of the first cell are within MX_CLOSE
-// errors: normal distributions scaled point by point by e^0 .. e^-12, 8 x 16384: 926 us against 981 with 32 queries (873 without the matrix cores).
+// Who answers the queries that the products cannot: the pass for equal minima costs a query a look at all boxes and at the cells within its
+// reach, the exact scan costs a wavefront its whole search again.  us, before the matrix cores / products with an exact scan of more than 20 queries,
+// whatever the search was like / as here.
+// - Left to the exact scan at once: more than MX_MANY queries for which two groups of the first cell are within MX_CLOSE errors of nothing, or too
+//   close to each other.  Points with twins a few units in the last place away 32 x 16384 147 / 176 / 152, points on a line 8 x 16384 144 / 171 / 162.
+// - Given up behind the overlapping cells: more than MX_MOST too close to each other, and those not blind, that is, with a smallest product above its
+//   error (the blind go on: what they learn shortens the exact scan).  Twins in other windows 2 x 60000 170 / 244 / 188.
+// - One by one, up to MX_PASS, and more of them where a query has MX_SCANS scans of the search to itself and half are not blind: wide cells, whose
+//   search is long and whose queries are few and far apart.  Laser scans 2 x 60000 868 / 944 / 815, 2 x 100000 2110 / 1990 / 1960.  (All such
+//   wavefronts, blind or not: 670 and 1640, but clouds with outliers 2 x 60000 2900 instead of 2690.)
+// The reach of those left over ends at the best of their eight: clouds with outliers 32 x 4096 270 / 232 / 213, scaled point by point by e^0 .. e^-12
+// 8 x 16384 890 / 960 / 933.  Still behind the search without products: these, twins, lines, and outliers in small calls (8 x 8192 on 2048 327 / 390 / 387).
+// Taken back: giving up inside the overlapping cells (outliers and lines 5 to 10 % faster, every call 3 %, by what each scan has to keep).
 constexpr float MX_CLOSE = 16.f;
-constexpr int MX_MANY = 16;
-constexpr int MX_PASS = 20;                // (12: laser scans of 32 x 4096 106 us against 91, e^-4 2 x 60000 1470 against 930; 32: a tail of slow wavefronts)
+constexpr int MX_MANY = 8;                 // (of 64; 16: twins 156, line 171)
+constexpr int MX_MOST = 32;
+constexpr int MX_SCANS = 8;                // (4: outliers 8 x 16384 1027 instead of 910)
+// (12: laser scans of 32 x 4096 106 us against 91, e^-4 2 x 60000 1470 against 930; 32: a tail of slow wavefronts.  Not less in wavefronts that share a
+// cell: halves with 10, laser scans of 2 x 16384 223 against 151, 8 x 8192 on 2048 144 against 93.)
+constexpr int MX_PASS = 20;
 
 // Two halves that add up to v: the rounded value, and what is left of it, rounded.
 // (`minus_one` as a variable: the compiler then takes three instructions for a pair, v_fma_mix among them, instead of nine)
@@ -434,6 +448,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
     bool ask = real; // left to the exact scan
     bool tie = false; // left to the pass behind it
     float reach = __builtin_inff();
+    int scans = 0; // behind the first cell's
     if (matrix)
     {
         x = real ? x : 0.f;
@@ -467,14 +482,36 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         float m = smallest();
         auto reach_of = [&](float product) { return real ? __builtin_fmaf(product, reach_factor, reach_error) : -1.f; };
         reach = reach_of(m);
-        // (where the first cell's second smallest products are near the error already, the search would leave the queries over)
-        int c2, d2;
-        by_query(near[0].m2, near[1].m2, c2, d2);
-        if (__builtin_popcountll(__ballot(real && __int_as_float(min(c2, d2)) < MX_CLOSE * own_error)) <= MX_MANY)
+        // The second smallest, and whether the smallest is surely further from it than both err.
+        auto second_smallest = [&]() {
+            int a, b, a2, b2;
+            by_query(near[0].m1, near[1].m1, a, b);
+            by_query(near[0].m2, near[1].m2, a2, b2);
+            return __int_as_float(min(min(a2, b2), max(a, b)));
+        };
+        auto clear = [&](float second) { return second > m + 2.f * __builtin_fmaf(m, MX_ERROR, own_error) && m < MX_LIMIT; };
+        // Where the first cell's second smallest products are near the error already, or near the smallest, the search would leave the queries
+        // over.  (A wavefront that shares its cell has half of the queries at most and keeps to the first test: it would give few back.)
+        float m2 = second_smallest();
+        const bool alone = log2_parts == 0;
+        const int close = __builtin_popcountll(__ballot(real && (m2 < MX_CLOSE * own_error || (alone && !clear(m2)))));
+        if (close <= (alone ? MX_MANY : 2 * MX_MANY))
         {
             // First the cells whose boxes overlap the queries' box - they hold nearly all the answers - then whatever
             // the worst answer still admits (a cell is looked at once: answers only get better).
+            bool given_up = false;
             for (int phase = 0; phase < 2; ++phase)
+            {
+                if (phase == 1)
+                {
+                    m = smallest();
+                    m2 = second_smallest();
+                    const unsigned long long unclear = __ballot(real && !clear(m2)), blind = unclear & __ballot(m < own_error);
+                    const int count = __builtin_popcountll(unclear);
+                    given_up = count > MX_MOST && count * MX_SCANS > scans && 2 * __builtin_popcountll(blind) <= count;
+                    if (given_up)
+                        break;
+                }
                 for (int g = 0; g < groups; ++g)
                 {
                     const float lw = lows[g * NG_CELL + lane];
@@ -494,6 +531,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
                         matrix_scan(cpts, c, want, lane, frame, queries, near);
                         TPK_WORK_ADD(NG_CELL);
                         reach = reach_of(smallest());
+                        ++scans;
                         if (phase)
                         {
                             bound = __int_as_float(wave_max_i32(__float_as_int(reach)));
@@ -501,29 +539,31 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
                         }
                     }
                 }
-            int a, b, a2, b2, cell_a, cell_b;
-            by_query(near[0].m1, near[1].m1, a, b);
-            by_query(near[0].m2, near[1].m2, a2, b2);
-            by_query(near[0].cell, near[1].cell, cell_a, cell_b);
-            const int m1 = min(a, b);
-            const float m2 = __int_as_float(min(min(a2, b2), max(a, b)));
-            m = __int_as_float(max(m1, 0));
-            ask = real && !(m2 > m + 2.f * __builtin_fmaf(m, MX_ERROR, own_error) && m < MX_LIMIT);
-            const int first = (a <= b ? cell_a : cell_b) * NG_CELL + (m1 & 3) * 16 + (a <= b ? 0 : 4);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) // (rows 0 .. 3 and 8 .. 11 of 16, or those four further on)
-            {
-                const float4 p = cpts[first + (c & 3) + 2 * (c & 4)];
-                const float d = tpk_dist2(p.x, p.y, p.z, qx, qy, qz);
-                const int ci = __float_as_int(p.w);
-                bi = d < best || (d == best && ci < bi) ? ci : bi;
-                best = fminf(d, best);
             }
-            TPK_WORK_ADD(8);
+            m = smallest();
+            m2 = second_smallest();
+            ask = real && (given_up || !clear(m2));
         }
-        // (the answer of a query that is left over is below its reach: not equal)
+        // The eight of the smallest product: the answer of a query that is not left over, and no further away than it for one that is.
+        int a, b, cell_a, cell_b;
+        by_query(near[0].m1, near[1].m1, a, b);
+        by_query(near[0].cell, near[1].cell, cell_a, cell_b);
+        const int first = (a <= b ? cell_a : cell_b) * NG_CELL + (min(a, b) & 3) * 16 + (a <= b ? 0 : 4);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) // (rows 0 .. 3 and 8 .. 11 of 16, or those four further on)
+        {
+            const float4 p = cpts[first + (c & 3) + 2 * (c & 4)];
+            const float d = tpk_dist2(p.x, p.y, p.z, qx, qy, qz);
+            const int ci = __float_as_int(p.w);
+            bi = d < best || (d == best && ci < bi) ? ci : bi;
+            best = fminf(d, best);
+        }
+        TPK_WORK_ADD(8);
+        // The answer of a query that is left over is below its reach, not equal, and no more than the best of the eight.
         reach = m < MX_LIMIT ? reach : __builtin_inff();
-        if (__builtin_popcountll(__ballot(ask)) <= MX_PASS)
+        reach = fminf(reach, __int_as_float(min(__float_as_int(best), 0x7F7FFFFF) + 1));
+        const int left = __builtin_popcountll(__ballot(ask)), blind = __builtin_popcountll(__ballot(ask && m < own_error));
+        if (left <= MX_PASS || (left * MX_SCANS <= scans && 2 * blind <= left))
         {
             tie = ask;
             ask = false;
@@ -597,33 +637,45 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         const float ub = tpk_read_lane(reach, q);
         float nearest = __builtin_inff();
         int lowest = 0x7FFFFFFF;
-        for (int g = 0; g < groups; ++g)
-        {
-            const int c = g * NG_CELL + lane;
-            const int cc = c < ccells ? c : 0;
-            const float lb = point_box_dist2(ux, uy, uz, cbox[cc * NG_BOX + 0], cbox[cc * NG_BOX + 1]);
-            unsigned long long cells = __ballot(c < ccells && lb * NG_MARGIN <= ub);
-            while (cells != 0)
+        auto look = [&](auto batch, int g0) __attribute__((always_inline)) {
+            constexpr int BATCH = batch.value; // groups whose boxes are on their way at a time
+            unsigned long long cells[BATCH];
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
             {
-                float4 p[4]; // (four cells on their way at a time; behind the last, the last one again)
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                {
-                    p[u] = cpts[(g * NG_CELL + __builtin_ctzll(cells)) * NG_CELL + lane];
-                    const unsigned long long rest = cells & (cells - 1);
-                    cells = rest != 0 || u == 3 ? rest : cells;
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                {
-                    const float d = tpk_dist2(p[u].x, p[u].y, p[u].z, ux, uy, uz);
-                    const int ci = __float_as_int(p[u].w);
-                    lowest = d < nearest || (d == nearest && ci < lowest) ? ci : lowest;
-                    nearest = d < nearest ? d : nearest;
-                }
-                TPK_WORK_ADD(4);
+                const int c = (g0 + u) * NG_CELL + lane;
+                const int cc = c < ccells ? c : 0;
+                const float lb = point_box_dist2(ux, uy, uz, cbox[cc * NG_BOX + 0], cbox[cc * NG_BOX + 1]);
+                cells[u] = __ballot(c < ccells && lb * NG_MARGIN <= ub);
             }
-        }
+#pragma unroll
+            for (int v = 0; v < BATCH; ++v)
+                while (cells[v] != 0)
+                {
+                    float4 p[4]; // (four cells on their way at a time; behind the last, the last one again)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                    {
+                        p[u] = cpts[((g0 + v) * NG_CELL + __builtin_ctzll(cells[v])) * NG_CELL + lane];
+                        const unsigned long long rest = cells[v] & (cells[v] - 1);
+                        cells[v] = rest != 0 || u == 3 ? rest : cells[v];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                    {
+                        const float d = tpk_dist2(p[u].x, p[u].y, p[u].z, ux, uy, uz);
+                        const int ci = __float_as_int(p[u].w);
+                        lowest = d < nearest || (d == nearest && ci < lowest) ? ci : lowest;
+                        nearest = d < nearest ? d : nearest;
+                    }
+                    TPK_WORK_ADD(4);
+                }
+        };
+        int g0 = 0;
+        for (; g0 + 4 <= groups; g0 += 4)
+            look(std::integral_constant<int, 4>{}, g0);
+        for (; g0 < groups; ++g0)
+            look(std::integral_constant<int, 1>{}, g0);
         // (distances are >= +0: their bit patterns order like integers)
         const float least = __int_as_float(wave_min_i32(__float_as_int(nearest)));
         lowest = wave_min_i32(nearest == least ? lowest : 0x7FFFFFFF);
