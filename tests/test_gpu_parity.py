@@ -2393,10 +2393,10 @@ def test_chamfer_on_the_matrix_cores(dev, kind, n, m):
         assert torch.equal(cells, pairs)
 
 
-@pytest.mark.parametrize("B", [1, 28, 29, 113, 114])
+@pytest.mark.parametrize("B", [1, 28, 29, 42, 43, 113, 114])
 @pytest.mark.parametrize("kind", ["even", "nearly equal", "lattice", "scan", "not finite"])
 def test_chamfer_cells_shared_by_wavefronts(tpk, dev, kind, B):
-    """Four, two or one wavefront for a cell's queries, either side of the cells (512, 2048) at which that changes, with a last cell of one query:
+    """Four, two or one wavefront for a cell's queries, either side of the cells (512; 2048, or 32768 times the pairs) at which that changes, with a last cell of one query:
     the distances and indices of the scan of all pairs, bit for bit, and the loss of those distances."""
     import ctypes
     import os

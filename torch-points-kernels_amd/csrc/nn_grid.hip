@@ -1494,14 +1494,21 @@ int64_t tpk_grid_chamfer_cells(int b, int n, int m)
 
 namespace {
 // log2 of the wavefronts that share a cell's queries, as in three_nn's search, to fewer wavefronts: a scan on the matrix cores costs 32
-// queries what it costs 16, and a wavefront's set-up is a larger part of it.  Pass without gradients, us, whole / halves / quarters / eighths:
-// 1 x 16384 points, noisy sphere 44.5 / 39.4 / 37.5 / 38.7, eight clusters 74.6 / 70.1 / 64.1 / 59.5; 2 x 16384 46.6 / 43.0 / 43.6 / 48.1, 78.1 / 70.8 /
-// 66.7 / 68.6; 4 x 16384 49.3 / 48.1 / 52.0, 81.5 / 73.6 / 77.5, even 47.6 / 49.6 / 53.9; 8 x 16384 50.3 / 54.1, 82.2 / 80.7; laser scans of
-// 1, 2, 4 x 16384 132.9 -> 96.0, 136.9 -> 106.8, 144.0 -> 131.8 as here.
+// queries what it costs 16, and a wavefront's set-up is a larger part of it.  Sharing shortens the wavefronts the call would wait for, which takes
+// large clouds, and is paid in wavefronts, so that few cells are shared, and in calls of many pairs fewer.  Forward, us, whole / halves / quarters:
+//   512 cells of 64 queries: 1 x 16384 even 41 / 37 / 36, eight clusters 60 / 55 / 47, laser scan 226 / 130 / 92; 4 x 4096 34 / 30 / 28, 44 / 38 / 38,
+//     102 / 53 / 47; 32 x 512 20.9 / 20.6 / 21.3, 21.1 / 20.6 / 21.3, 24.8 / 22.6 / 22.7
+//   1024: 2 x 16384 42 / 38 / 40, 81 / 68 / 56, 227 / 130 / 101; 32 x 1024 24.5 / 25.1 / 28, 24.5 / 24.1 / 27, 32 / 29 / 31; 64 x 512 21.3 / 22.3 / 25,
+//     21.2 / 21.8 / 25, 25.9 / 24.3 / 27
+//   2048: 4 x 16384 44 / 44 / 52, 82 / 73 / 62, 268 / 137 / 152; 16 x 4096 34.9 / 35.7 / 41, 41 / 38 / 40, 96 / 59 / 72; 32 x 2048 31 / 33 / 37,
+//     30.9 / 31.4 / 38, 49 / 46 / 58; 64 x 1024 26.9 / 29.5 / 36, 26.3 / 27.5 / 33, 36 / 34 / 40
+//   4096: 8 x 16384 51 / 56 / 69, 83 / 75 / 74, 285 / 181 / 227; 32 x 4096 41 / 45 / 56, 42 / 43 / 54, 97 / 81 / 104
+constexpr int64_t CHAMFER_QUARTERED_CELLS = 512, CHAMFER_HALVED_CELLS = 2048;
+constexpr int64_t CHAMFER_HALVED_PAIR_CELLS = 32768; // cells times pairs of clouds: 32 pairs of 1024 cells, 16 of 2048
 int chamfer_parts(int b, int n, int m)
 {
     const int64_t cells = tpk_grid_chamfer_cells(b, n, m);
-    return cells <= 512 ? 2 : cells <= 2048 ? 1 : 0;
+    return cells <= CHAMFER_QUARTERED_CELLS ? 2 : cells <= CHAMFER_HALVED_CELLS && cells * b <= CHAMFER_HALVED_PAIR_CELLS ? 1 : 0;
 }
 } // namespace
 
