@@ -30,6 +30,8 @@ for _p in (ROOT, os.path.join(ROOT, "torch-points-kernels_amd")):
 PEAK_HBM_GBS = 8000.0
 PEAK_FP32_TFLOPS = 157.3  # published fp32 figure (vector = matrix); it counts every lane-op as an FMA (2 flop)
 
+PEAK_FP16_TFLOPS = 2500.0  # dense matrix products of halves
+
 PROFILES = os.path.join(ROOT, "profiles")
 TRAFFIC_FILE = os.path.join(PROFILES, "all_ops_baseline_configs_hbm_traffic.txt")
 VALU_FILE = os.path.join(PROFILES, "distance_scans_valu_utilisation.txt")
@@ -246,8 +248,8 @@ def _all_pairs_entry(call, pairs, steps, warmup, valu_kernel):
 COUNT_WORK = True  # --no-count: leave the counting build out (profiler runs: its kernels carry the same names)
 
 
-def _executed(call):
-    """Pair evaluations executed by call(lib, stream) -> status."""
+def _executed(call, products=None):
+    """Pair evaluations executed by call(lib, stream) -> status; the pairs of its matrix products are added to the list `products`."""
     import ctypes
 
     import torch
@@ -255,11 +257,13 @@ def _executed(call):
     if not COUNT_WORK:
         return 0
     lib = _counting_lib()
-    n = ctypes.c_ulonglong(0)
+    n, formed = ctypes.c_ulonglong(0), ctypes.c_ulonglong(0)
     assert lib.tpk_work_read_reset(ctypes.byref(n)) == 0
     st = call(lib, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     assert st == 0, "counting call failed with status %d" % st
-    assert lib.tpk_work_read_reset(ctypes.byref(n)) == 0
+    assert lib.tpk_work_read_reset_both(ctypes.byref(n), ctypes.byref(formed)) == 0
+    if products is not None:
+        products.append(int(formed.value))
     return int(n.value)
 
 
@@ -666,14 +670,21 @@ def bench_others(dev, steps, warmup, with_cpu):
     ci2 = torch.empty(cb, cm, dtype=torch.int32, device=dev)
     ws_bytes = _counting_lib().tpk_chamfer_fwd_workspace_bytes(cb, cn, cm)
     ws = _ws(ws_bytes, dev)
+    formed = []
     executed = _executed(lambda lib, st: lib.tpk_chamfer_fwd_f32(
         cb, cn, cm, _p(a), _p(b), _p(cd1), _p(cd2), _p(ci1), _p(ci2), _p(ws) if ws_bytes else None,
-        ctypes.c_size_t(ws_bytes), st))
+        ctypes.c_size_t(ws_bytes), st), formed)
     e = {"workload": "configs[4]: Chamfer forward B=32 16384x16384 (both directions)", "metric": "pairs/s",
          "value": pairs / (wall * 1e-3), "kernel_ms": ev, "wall_ms": wall,
          "roofline": _roof_flops(executed, pairs, 8, ev, "chamfer_fwd"), "pairs": pairs}
-    e["roofline"]["note"] += PRUNED_NOTE + ("; most of its pairs are formed by matrix products of halves, which choose the few "
-                                            "that are evaluated in fp32, and are counted like those")
+    e["roofline"]["note"] = ("fp32 evaluations of the few pairs that matrix products of halves choose (achieved and frac: those evaluations "
+                             "alone, unfused, x 8 flop / kernel time); matrix_products: the pairs formed by the products, in tiles of 32 x 32 and "
+                             "16 slots, x 32 flop / the same time, of the dense fp16 peak; algorithmic_rate = the pairs a brute-force scan "
+                             "tests x 8 flop / the same time" + PRUNED_NOTE)
+    if formed:
+        rate = formed[0] * 32 / (ev * 1e-3) / 1e12
+        e["roofline"]["matrix_products"] = {"pairs": formed[0], "achieved": rate, "peak": PEAK_FP16_TFLOPS, "unit": "TFLOP/s",
+                                            "frac": rate / PEAK_FP16_TFLOPS}
     e["all_pairs_kernel"] = _all_pairs_entry(lambda lib, st: lib.tpk_chamfer_fwd_f32(
         cb, cn, cm, _p(a), _p(b), _p(cd1), _p(cd2), _p(ci1), _p(ci2), None, ctypes.c_size_t(0), st), pairs, 3, 1,
         "chamfer_fwd_kernel<float, 4>")
@@ -772,6 +783,8 @@ def _compact_op(e):
         row["frac"] = _sig(r.get("frac"), 3)
         if "algorithmic_rate" in r:
             row["alg_frac"] = _sig(r["algorithmic_rate"] / r["peak"], 3)
+        if "matrix_products" in r:  # (of the fp16 peak; frac is that of the fp32 evaluations alone)
+            row["products_frac"] = _sig(r["matrix_products"]["frac"], 3)
         if r.get("traffic") and e.get("algorithmic_bytes"):
             row["traffic_x"] = _sig(r["traffic"] / e["algorithmic_bytes"], 3)
     ag = e.get("as_autograd_runs_it")

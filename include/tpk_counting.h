@@ -1,10 +1,12 @@
 /*
- * tpk_counting.h - the one extra entry point of libtpk_hip_counting.so.
+ * tpk_counting.h - the two extra entry points of libtpk_hip_counting.so.
  *
  * libtpk_hip_counting.so is libtpk_hip.so (same sources, same C ABI: tpk.h) with the distance
  * scans compiled -DTPK_COUNT_WORK: furthest point sampling, the ball queries, three_nn and the
  * Chamfer forward pass count the pair evaluations their lanes EXECUTE (one count = one lane
- * forming one squared distance; for furthest point sampling one running minimum updated).  It is
+ * forming one squared distance; for furthest point sampling one running minimum updated).  Chamfer's
+ * search also counts the pairs it forms in matrix products of halves, to choose those it evaluates,
+ * by themselves: one count per pair of a tile of 32 x 32 that is multiplied.  It is
  * a measuring instrument for benchmarks - executed work divided by time, for kernels that skip
  * most of the pairs a brute-force scan would test - and slower than the shipping library (an
  * atomic add per lane at the end of every kernel).  It has no counterpart in the reference.
@@ -19,6 +21,9 @@ extern "C" {
 /* Waits for the device, stores the pair evaluations counted on the current device since the last
  * call in *pairs and sets the counters back to zero.  Returns TPK_OK or a hipError_t. */
 int tpk_work_read_reset(unsigned long long* pairs);
+
+/* The same, and in *products the pairs formed by matrix products since the last call of either. */
+int tpk_work_read_reset_both(unsigned long long* pairs, unsigned long long* products);
 
 #ifdef __cplusplus
 }

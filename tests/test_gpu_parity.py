@@ -2896,6 +2896,43 @@ def test_counting_build_counts_executed_pairs(oracle, dev):
     assert lib.tpk_work_read_reset(ctypes.byref(count)) == 0 and count.value == 0
 
 
+def test_counting_build_counts_matrix_products_by_themselves(dev):
+    """Chamfer's search: the eight evaluated per lane and the few cells of single queries are evaluations, the tiles multiplied are not; a
+    tile without a query is neither (64 pairs of 513 points, whose last cells hold one query)."""
+    import ctypes
+    import os
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip_counting.so"))
+    lib.tpk_chamfer_fwd_workspace_bytes.restype = ctypes.c_size_t
+    pairs, products = ctypes.c_ulonglong(0), ctypes.c_ulonglong(0)
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr())
+    both = (ctypes.byref(pairs), ctypes.byref(products))
+
+    def run(a, b):
+        B, n, m = a.shape[0], a.shape[1], b.shape[1]
+        out = [torch.empty(B, k, dtype=t, device=dev) for t in (torch.float32, torch.int32) for k in (n, m)]
+        nbytes = lib.tpk_chamfer_fwd_workspace_bytes(B, n, m)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        assert lib.tpk_work_read_reset_both(*both) == 0
+        assert lib.tpk_chamfer_fwd_f32(B, n, m, pointer(a), pointer(b), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None) == 0
+        assert lib.tpk_work_read_reset_both(*both) == 0
+        return int(pairs.value), int(products.value)
+
+    g = torch.Generator().manual_seed(3)
+    a, b = (torch.rand(8, 16384, 3, generator=g).to(dev) for _ in range(2))
+    evaluated, formed = run(a, b)
+    queries = 2 * 8 * 16384
+    assert 8 * queries <= evaluated <= 12 * queries  # (one query in 3600 takes up to a few dozen cells of 64)
+    assert formed % 2048 == 0 and queries * 64 <= formed <= queries * 16384 // 8
+    a = torch.rand(64, 513, 3, generator=g).to(dev)
+    evaluated, formed = run(a, a[:, :, [1, 2, 0]].contiguous())
+    assert 64 * 2 * 9 * 64 * 8 <= evaluated and formed % 2048 == 0
+    assert formed <= 64 * 2 * (512 + 32) * 576
+    lib.tpk_work_read_reset_both(*both)
+    assert pairs.value == 0 and products.value == 0
+
+
 def _knn_steps(oracle, dev, support, query, k, workspace="grid"):
     """Steps of 64 points per query that the counting build takes; the answers are checked on the way.  workspace: the size the
     grid in memory wants, or the one for curve-ordered cells."""

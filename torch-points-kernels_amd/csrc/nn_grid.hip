@@ -264,7 +264,7 @@ struct MatrixFrame
 
 // (`want`: the queries that ask for the cell; a tile of 32 queries, neighbours on the curve, of which none does is left out)
 __device__ __forceinline__ void matrix_scan(const float4* __restrict__ cand, int cell, unsigned long long want, int lane, const MatrixFrame& f,
-                                            const half8_t (&queries)[2], MatrixNearest (&s)[2])
+                                            const half8_t (&queries)[2], MatrixNearest (&s)[2] TPK_PRODUCTS_PARAM)
 {
     const float4 p = cand[cell * NG_CELL + lane];
     // (a padding candidate, infinitely far away, and one that is not a number count as far away)
@@ -283,6 +283,7 @@ __device__ __forceinline__ void matrix_scan(const float4* __restrict__ cand, int
     {
         if (static_cast<unsigned>(want >> (32 * j)) == 0)
             continue;
+        TPK_PRODUCTS_ADD(32); // (32 queries and 64 candidates, counted by 64 lanes)
         const int before = s[j].m1;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -377,6 +378,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
     float4* const stage = stages[wave];
     float* const lows = lows_all + wave * ((max(cells1, cells2) + NG_CELL - 1) / NG_CELL * NG_CELL);
     TPK_WORK_DECL
+    TPK_PRODUCTS_DECL
 
     const float4 query = qpts[qcell * NG_CELL + lane];
     const float qx = query.x, qy = query.y, qz = query.z;
@@ -470,8 +472,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         MatrixNearest near[2];
         near[0].m1 = near[0].m2 = near[1].m1 = near[1].m2 = __float_as_int(__builtin_inff());
         near[0].cell = near[1].cell = seed;
-        matrix_scan(cpts, seed, __ballot(real), lane, frame, queries, near);
-        TPK_WORK_ADD(NG_CELL);
+        matrix_scan(cpts, seed, __ballot(real), lane, frame, queries, near TPK_PRODUCTS_ARG);
         // The smallest product of the lane's query, and the squared distance that holds the query's answer for certain.  (A tile
         // without a query is never scanned: its m1 stay infinite.  No lane without a query may reach for anything.)
         auto smallest = [&]() {
@@ -528,8 +529,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
                         const unsigned long long want = __ballot(lb * NG_MARGIN <= reach);
                         if (want == 0)
                             continue;
-                        matrix_scan(cpts, c, want, lane, frame, queries, near);
-                        TPK_WORK_ADD(NG_CELL);
+                        matrix_scan(cpts, c, want, lane, frame, queries, near TPK_PRODUCTS_ARG);
                         reach = reach_of(smallest());
                         ++scans;
                         if (phase)
@@ -652,6 +652,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
             for (int v = 0; v < BATCH; ++v)
                 while (cells[v] != 0)
                 {
+                    TPK_WORK_ADD(min(4, __builtin_popcountll(cells[v])));
                     float4 p[4]; // (four cells on their way at a time; behind the last, the last one again)
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
@@ -668,7 +669,6 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
                         lowest = d < nearest || (d == nearest && ci < lowest) ? ci : lowest;
                         nearest = d < nearest ? d : nearest;
                     }
-                    TPK_WORK_ADD(4);
                 }
         };
         int g0 = 0;
@@ -683,6 +683,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         bi = lane == q ? lowest : bi;
     }
     TPK_WORK_FLUSH
+    TPK_PRODUCTS_FLUSH
     if (real)
     {
         dout[qindex] = best;

@@ -45,23 +45,31 @@ extern "C" void tpk_work_register(int (*read_reset)(unsigned long long*))
     work_readers().push_back(read_reset);
 }
 
-// Waits for the device, returns the pair evaluations counted since the last call in *pairs and
-// sets the counters back to zero.
-extern "C" int tpk_work_read_reset(unsigned long long* pairs)
+// Wait for the device, return the pair evaluations - and the pairs formed by matrix products - counted since the last
+// call of either and set the counters back to zero.
+extern "C" int tpk_work_read_reset_both(unsigned long long* pairs, unsigned long long* products)
 {
     hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess)
         return static_cast<int>(e);
-    unsigned long long total = 0;
+    unsigned long long total[2] = {0, 0};
     for (auto reader : work_readers())
     {
-        unsigned long long part = 0;
-        const int st = reader(&part);
+        unsigned long long part[2] = {0, 0};
+        const int st = reader(part);
         if (st != 0)
             return st;
-        total += part;
+        total[0] += part[0];
+        total[1] += part[1];
     }
-    *pairs = total;
+    *pairs = total[0];
+    *products = total[1];
     return TPK_OK;
+}
+
+extern "C" int tpk_work_read_reset(unsigned long long* pairs)
+{
+    unsigned long long products;
+    return tpk_work_read_reset_both(pairs, &products);
 }
 #endif

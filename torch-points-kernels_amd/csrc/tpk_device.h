@@ -273,18 +273,19 @@ __device__ __forceinline__ void lds_barrier()
 // (libtpk_hip_counting.so): there the distance scans add up the pair evaluations their lanes
 // execute (one count = one lane forming one squared distance, or one running minimum updated by
 // furthest point sampling), so that a benchmark can divide EXECUTED work by time.  Every
-// translation unit has its own device counter, registered with the reader in status.hip.  In the
-// shipping build all of this expands to nothing.
+// translation unit has its own device counter, registered with the reader in status.hip.  A second one counts
+// the pairs that matrix products form (Chamfer's search), which are not evaluations.  In the shipping build
+// all of this expands to nothing.
 // ---------------------------------------------------------------------------------------------
 #ifdef TPK_COUNT_WORK
 namespace {
-__device__ unsigned long long tpk_work_cell;
+__device__ unsigned long long tpk_work_cell[2]; // evaluations, pairs of matrix products
 int tpk_work_cell_read_reset(unsigned long long* out)
 {
-    const unsigned long long zero = 0;
-    hipError_t e = hipMemcpyFromSymbol(out, HIP_SYMBOL(tpk_work_cell), sizeof(*out));
+    const unsigned long long zero[2] = {0, 0};
+    hipError_t e = hipMemcpyFromSymbol(out, HIP_SYMBOL(tpk_work_cell), sizeof(zero));
     if (e == hipSuccess)
-        e = hipMemcpyToSymbol(HIP_SYMBOL(tpk_work_cell), &zero, sizeof(zero));
+        e = hipMemcpyToSymbol(HIP_SYMBOL(tpk_work_cell), zero, sizeof(zero));
     return static_cast<int>(e);
 }
 } // namespace
@@ -297,13 +298,23 @@ struct TpkWorkRegistration
 } // namespace
 #define TPK_WORK_DECL unsigned long long tpk_work = 0;
 #define TPK_WORK_ADD(n) (tpk_work += static_cast<unsigned long long>(n))
-#define TPK_WORK_FLUSH atomicAdd(&tpk_work_cell, tpk_work);
+#define TPK_WORK_FLUSH atomicAdd(&tpk_work_cell[0], tpk_work);
 #define TPK_WORK_PARAM , unsigned long long& tpk_work
 #define TPK_WORK_ARG , tpk_work
+#define TPK_PRODUCTS_DECL unsigned long long tpk_products = 0;
+#define TPK_PRODUCTS_ADD(n) (tpk_products += static_cast<unsigned long long>(n))
+#define TPK_PRODUCTS_FLUSH atomicAdd(&tpk_work_cell[1], tpk_products);
+#define TPK_PRODUCTS_PARAM , unsigned long long& tpk_products
+#define TPK_PRODUCTS_ARG , tpk_products
 #else
 #define TPK_WORK_DECL
 #define TPK_WORK_ADD(n) ((void)0)
 #define TPK_WORK_FLUSH
 #define TPK_WORK_PARAM
 #define TPK_WORK_ARG
+#define TPK_PRODUCTS_DECL
+#define TPK_PRODUCTS_ADD(n) ((void)0)
+#define TPK_PRODUCTS_FLUSH
+#define TPK_PRODUCTS_PARAM
+#define TPK_PRODUCTS_ARG
 #endif
