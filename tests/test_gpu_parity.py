@@ -2220,6 +2220,30 @@ def test_three_nn_cells_shared_by_wavefronts(dev, kind, B):
             assert torch.equal(cells, pairs)
 
 
+@pytest.mark.parametrize("kind", ["even", "crowded", "lattice", "not finite"])
+def test_three_nn_whole_wavefronts_over_windows(dev, kind):
+    """The same with all 64 queries of a cell in one wavefront, on clouds of two windows of both kinds (those of 513 points above have one)."""
+    B, n, m = 5, 20000, 17000
+    assert 2 * B * _cells(n) > _search_limit("NG_PARTED_WAVES") and m > 8192
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_three_nn_workspace_bytes.restype = ctypes.c_size_t
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr())
+    unknown, known = (c.to(dev) for c in _chamfer_clouds(kind, B, n, m))
+    nbytes = lib.tpk_three_nn_workspace_bytes(B, n, m)
+    assert nbytes > 0
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+    out, want = ([torch.full((B, n, 3), -1, dtype=t, device=dev) for t in (torch.float32, torch.int32)] for _ in range(2))
+    assert lib.tpk_three_nn_f32(B, n, m, pointer(unknown), pointer(known), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None) == 0
+    assert lib.tpk_three_nn_all_pairs_f32(B, n, m, pointer(unknown), pointer(known), *(pointer(t) for t in want), None) == 0
+    torch.cuda.synchronize()
+    for cells, pairs in zip(out, want):
+        assert torch.equal(cells, pairs)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("B,n,m", [(1, 1, 1), (2, 4096, 1), (1, 4096, 4096), (1, 4097, 4096), (3, 2731, 2000), (1, 40000, 700), (2, 0, 5)])
 def test_chamfer_loss_as_one_node(tpk, dev, dtype, B, n, m):
@@ -2340,25 +2364,14 @@ def test_cell_search_outliers(tpk, oracle, dev):
         np.testing.assert_array_equal(_np(dist2), wd)
 
 
-@pytest.mark.parametrize("n,m", [(513, 600), (1024, 8191), (5000, 16385), (20000, 20000)])
-@pytest.mark.parametrize("kind", ["even", "itself", "nearly itself", "nearly equal", "lattice", "crowded", "scan", "outliers", "far", "one of many", "tiny",
-                                  "not finite"])
-def test_chamfer_on_the_matrix_cores(dev, kind, n, m):
-    """The search over cells against the scan of all pairs, bit for bit: clouds whose queries the products answer, leave to the pass
-    for equal minima (a few of a wavefront, "nearly equal") or to the exact scan (lattices, wide cells, cells far away, units out of range)."""
-    import ctypes
-    import os
-
-    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
-                                   "torch_points_kernels", "libtpk_hip.so"))
-    lib.tpk_chamfer_fwd_workspace_bytes.restype = ctypes.c_size_t
+def _chamfer_clouds(kind, B, n, m):
     g = torch.Generator().manual_seed(n + m)
-    clouds = [torch.rand(2, count, 3, generator=g) for count in (n, m)]
+    clouds = [torch.rand(B, count, 3, generator=g) for count in (n, m)]
     first = lambda count: clouds[1][:, torch.arange(count) % m]
     if kind == "itself":
         clouds[0] = first(n).clone()
     elif kind == "nearly itself":
-        clouds[0] = first(n) + 1e-5 * torch.randn(2, n, 3, generator=g)
+        clouds[0] = first(n) + 1e-5 * torch.randn(B, n, 3, generator=g)
     elif kind == "nearly equal":  # every point has a twin a few units in the last place away
         clouds[1][:, m // 2 : 2 * (m // 2)] = clouds[1][:, : m // 2] * (1.0 + 2.0 ** -22)
     elif kind == "lattice":
@@ -2379,18 +2392,62 @@ def test_chamfer_on_the_matrix_cores(dev, kind, n, m):
     elif kind == "not finite":
         clouds[0][:, 7::97, 1] = float("nan")
         clouds[1][:, 3::89, 2] = float("inf")
-    a, b = (c.contiguous().to(dev) for c in clouds)
+    return [c.contiguous() for c in clouds]
+
+
+def _chamfer_over_cells_is_that_of_all_pairs(dev, clouds):
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd",
+                                   "torch_points_kernels", "libtpk_hip.so"))
+    lib.tpk_chamfer_fwd_workspace_bytes.restype = ctypes.c_size_t
+    a, b = (c.to(dev) for c in clouds)
+    B, n, m = a.shape[0], a.shape[1], b.shape[1]
     pointer = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
     results = []
-    for nbytes in (lib.tpk_chamfer_fwd_workspace_bytes(2, n, m), 0):
+    for nbytes in (lib.tpk_chamfer_fwd_workspace_bytes(B, n, m), 0):
         ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
-        out = [torch.full((2, k), -1, dtype=t, device=dev) for t in (torch.float32, torch.int32) for k in (n, m)]
-        st = lib.tpk_chamfer_fwd_f32(2, n, m, pointer(a), pointer(b), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None)
+        out = [torch.full((B, k), -1, dtype=t, device=dev) for t in (torch.float32, torch.int32) for k in (n, m)]
+        st = lib.tpk_chamfer_fwd_f32(B, n, m, pointer(a), pointer(b), *(pointer(t) for t in out), pointer(ws), ctypes.c_size_t(nbytes), None)
         assert st == 0
         torch.cuda.synchronize()
         results.append([t.cpu() for t in out])
+    assert lib.tpk_chamfer_fwd_workspace_bytes(B, n, m) > 0
     for cells, pairs in zip(*results):
         assert torch.equal(cells, pairs)
+
+
+CHAMFER_KINDS = ["even", "itself", "nearly itself", "nearly equal", "lattice", "crowded", "scan", "outliers", "far", "one of many", "tiny", "not finite"]
+
+
+@pytest.mark.parametrize("n,m", [(513, 600), (1024, 8191), (5000, 16385), (20000, 20000)])
+@pytest.mark.parametrize("kind", CHAMFER_KINDS)
+def test_chamfer_on_the_matrix_cores(dev, kind, n, m):
+    """The search over cells against the scan of all pairs, bit for bit: clouds whose queries the products answer, leave to the pass
+    for equal minima (a few of a wavefront, "nearly equal") or to the exact scan (lattices, wide cells, cells far away, units out of range)."""
+    _chamfer_over_cells_is_that_of_all_pairs(dev, _chamfer_clouds(kind, 2, n, m))
+
+
+def _search_limit(name):
+    import os
+    import re
+
+    source = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "torch-points-kernels_amd", "csrc", "nn_grid.hip")
+    return int(re.search(r"\b%s = (\d+)" % name, open(source).read()).group(1))
+
+
+def _cells(n):
+    return -(-n // 64) if n <= 16384 else -(-n // 16384) * 256
+
+
+@pytest.mark.parametrize("B,n,m", [(5, 20000, 20000), (16, 5000, 16385), (2, 60000, 50000)])
+@pytest.mark.parametrize("kind", CHAMFER_KINDS)
+def test_chamfer_whole_wavefronts_on_the_matrix_cores(dev, kind, B, n, m):
+    """The same where a wavefront has all 64 queries of its cell, as in large calls: the limits on those left over count 64 of them, searches of
+    several groups of cells and several windows are given up, and long ones serve many single queries (scans of 60000 points)."""
+    assert B * (_cells(n) + _cells(m)) > _search_limit("CHAMFER_HALVED_CELLS")
+    _chamfer_over_cells_is_that_of_all_pairs(dev, _chamfer_clouds(kind, B, n, m))
 
 
 @pytest.mark.parametrize("B", [1, 28, 29, 42, 43, 113, 114])
