@@ -625,6 +625,28 @@ def test_fps_ties_origin_skip_and_exhaustion(tpk, oracle, dev):
     assert (tpk.furthest_point_sample(tiny.to(dev), 10) == 0).all()
 
 
+@pytest.mark.parametrize("n", [300, 1024, 4096, 8192, 12000, 16384])
+def test_fps_points_at_infinity(tpk, oracle, dev, n):
+    """300 points at infinity along one axis or another, 40 others, the rest too near to the origin to be sampled: one sample for every axis (the
+    distances of the others along it are NaN from then on), and behind them those of the cloud without these points.  Their
+    wavefronts have had equal maxima and hold points that never take part, in any of their registers."""
+    count = min(300, n // 3)
+    for seed in range(12):
+        g = torch.Generator().manual_seed(seed)
+        xyz = torch.rand(1, n, 3, generator=g) * 0.01
+        order = torch.randperm(n - 1, generator=g) + 1
+        xyz[0, 0] = 0.9
+        for axis in range(3):
+            xyz[0, order[axis:count:3], axis] = float("inf")
+        xyz[0, order[count : count + 40]] = torch.rand(40, 3, generator=g) + 0.5
+        without = xyz.clone()
+        without[0, order[:count]] = 0.001
+        out = _np(tpk.furthest_point_sample(xyz.to(dev), 43))[0]
+        axes = [int(np.argmax(np.isinf(xyz[0, i].numpy()))) if np.isinf(xyz[0, i].numpy()).any() else -1 for i in out[1:4]]
+        assert out[0] == 0 and sorted(axes) == [0, 1, 2], seed
+        np.testing.assert_array_equal(out[4:], oracle.furthest_point_sample(without.numpy(), 40)[0][1:])
+
+
 def test_fps_ties_large_cloud(tpk, oracle, dev):
     # the same tie cases at cloud sizes served by the kernel that sorts the cloud along a space
     # filling curve (slots no longer in index order: the tie key has to be applied explicitly)

@@ -740,8 +740,10 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
         most = wave_max_to_scalar(most);
         const int own_lane = not_hoisted(lane);
         bool several = keyed; // (where there were some there will be more)
-        int held_in = 0;      // the slot that holds the maximum, if one does
-        if (!keyed)
+        int held_in = 0;      // a slot that holds the maximum
+        // (A wavefront whose points have all been at infinity with a sample is keyed and has nothing left: the distance there is a NaN, whose
+        // bits lie below 0 and above those of -1, the minimum of points that take no part.)
+        if (!keyed || most < 0)
         {
             int held = 0;
 #pragma unroll
@@ -805,8 +807,9 @@ __global__ __launch_bounds__(WAVES* TPK_WAVE) void fps_pool_kernel(
                     offer_places[turn][wave] = sorted_position<WAVES, GS>(i / GS, wave, i % GS, own_lane);
                 }
             };
-            // (sixteen tests with a branch each, of all wavefronts of a SIMD in turn, were 200 ns of such a sample's 1650; where nothing is
-            // left - most < 0 - any slot that holds it will do)
+            // (sixteen tests with a branch each, of all wavefronts of a SIMD in turn, were 100 ns of such a sample's 1650: 16 x 16384 points, 4096
+            // samples, even 601 -> 594 us, clusters 727 -> 724, a laser scan 868 -> 858, 4 x 16384 on a sphere 367 -> 361; where nothing is left
+            // any slot that holds the maximum will do)
             if constexpr (PPT >= 8)
                 with_slot<0, PPT>(held_in, [&](auto chosen) __attribute__((always_inline)) { offer(chosen.value); });
             else
