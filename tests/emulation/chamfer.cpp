@@ -52,6 +52,8 @@ int main(int argc, char** argv)
                     p[a] = p[a - 3 * (counts[1] / 2)] * (1.f + 0x1p-22f);
             else if (kind == "far" && s == 0)
                 p[0] += 300.f;
+            else if (kind == "not a number" && i % 15 == 3)
+                p[1] = -__builtin_nanf("");
         }
     }
     const size_t bytes = tpk_grid_chamfer_workspace_bytes(b, n, m);

@@ -71,7 +71,7 @@ def chamfer(tmp_path_factory):
 # (530 points: a last cell of 18, whose second 32 queries are none; wavefronts that share a cell have half of their queries at most; 1032 points:
 # a second tile of products without queries in the last cell of every part; 58 pairs of 18 cells: wavefronts with all queries of a cell)
 @pytest.mark.parametrize("clouds,n,m,kind", [shape + (kind,) for shape in [(1, 530, 1032), (2, 1032, 700)]
-                                             for kind in ("even", "lattice", "scan", "outliers", "scaled", "twins", "far")]
+                                             for kind in ("even", "lattice", "scan", "outliers", "scaled", "twins", "far", "not a number")]
                          + [(58, 514, 513, "outliers"), (58, 514, 513, "twins")])
 def test_chamfer_finds_the_nearest(chamfer, clouds, n, m, kind):
     """The search's answers where the matrix products err by as much as its bound assumes and a NaN has the sign that orders above everything."""

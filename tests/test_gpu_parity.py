@@ -2414,6 +2414,9 @@ def _chamfer_clouds(kind, B, n, m):
     elif kind == "not finite":
         clouds[0][:, 7::97, 1] = float("nan")
         clouds[1][:, 3::89, 2] = float("inf")
+    elif kind == "not a number":  # with the sign the device gives it
+        for c, first, step in zip(clouds, (3, 5), (17, 13)):
+            c.view(torch.int32)[:, first::step, 1] = -4194304
     return [c.contiguous() for c in clouds]
 
 
@@ -2440,7 +2443,7 @@ def _chamfer_over_cells_is_that_of_all_pairs(dev, clouds):
         assert torch.equal(cells, pairs)
 
 
-CHAMFER_KINDS = ["even", "itself", "nearly itself", "nearly equal", "lattice", "crowded", "scan", "outliers", "far", "one of many", "tiny", "not finite"]
+CHAMFER_KINDS = ["even", "itself", "nearly itself", "nearly equal", "lattice", "crowded", "scan", "outliers", "far", "one of many", "tiny", "not finite", "not a number"]
 
 
 @pytest.mark.parametrize("n,m", [(513, 600), (1024, 8191), (5000, 16385), (20000, 20000)])

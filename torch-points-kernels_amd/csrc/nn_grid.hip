@@ -125,8 +125,9 @@ __device__ __forceinline__ void scan_cell_few(const float4* __restrict__ cand, i
         TPK_WORK_ADD(1);
         const float ux = tpk_read_lane(qx, q), uy = tpk_read_lane(qy, q), uz = tpk_read_lane(qz, q);
         const float d = tpk_dist2(p.x, p.y, p.z, ux, uy, uz); // (a padding candidate lies at infinity)
-        // distances are >= +0: their bit patterns order like integers (a NaN sorts above infinity)
-        const float mn = __int_as_float(wave_min_i32(__float_as_int(d)));
+        // distances are >= +0: their bit patterns order like unsigned integers (a NaN of either sign sorts above infinity; what the
+        // device itself makes of 0 / 0 or infinity minus infinity has the sign set)
+        const float mn = __int_as_float(static_cast<int>(wave_min_u32(static_cast<unsigned>(__float_as_int(d)))));
         const unsigned long long at = __ballot(d == mn);
         if (at == 0)
             continue; // nothing but NaN
