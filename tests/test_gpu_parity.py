@@ -2266,6 +2266,28 @@ def test_three_nn_whole_wavefronts_over_windows(dev, kind):
         assert torch.equal(cells, pairs)
 
 
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("n", [700, 9000, 20000, 50000])
+def test_sorted_ball_query_beside_points_that_are_not_numbers(tpk, dev, n, sign):
+    """Support points without a number along one axis, of either sign, hide none of the others: the boxes of their cells have no side there, and
+    the boxes of sixteen cells must not be taken from the other cells alone."""
+    g = torch.Generator().manual_seed(n)
+    xyz = torch.rand(1, n, 3, generator=g)
+    query = xyz[:, torch.randperm(n, generator=g)[:300]].clone()
+    xyz.view(torch.int32)[0, 4::29, 1] = 0x7FC00000 if sign > 0 else -4194304
+    radius, nsample = float(np.float32((10.0 / (4.19 * n)) ** (1.0 / 3.0))), 24
+    idx, dist = (_np(t)[0] for t in tpk.ball_query(radius, nsample, xyz.to(dev), query.to(dev), sort=True))
+    d = (query[0][:, None] - xyz[0][None]) ** 2  # (float32, every operation rounded on its own)
+    d = ((d[..., 0] + d[..., 1]) + d[..., 2]).numpy()
+    limit = np.float32(radius) * np.float32(radius)
+    for q in range(300):
+        hits = np.nonzero(d[q] < limit)[0]
+        hits = hits[np.lexsort((hits, d[q][hits]))][:nsample]
+        np.testing.assert_array_equal(idx[q, : len(hits)], hits)
+        np.testing.assert_array_equal(dist[q, : len(hits)], d[q][hits])
+        assert (dist[q, len(hits) :] == -1).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("B,n,m", [(1, 1, 1), (2, 4096, 1), (1, 4096, 4096), (1, 4097, 4096), (3, 2731, 2000), (1, 40000, 700), (2, 0, 5)])
 def test_chamfer_loss_as_one_node(tpk, dev, dtype, B, n, m):

@@ -1738,11 +1738,14 @@ __global__ __launch_bounds__(NG_SCAN_THREADS) void run_boxes_kernel(int64_t tota
     const float4* __restrict__ cbox = boxes + cloud * ccells * NG_BOX;
     const float inf = __builtin_inff();
     float4 lo = make_float4(inf, inf, inf, 0.f), hi = make_float4(-inf, -inf, -inf, 0.f);
+    // (an empty cell: lo = +inf, hi = -inf; a side that is not a number, of a cell with such a point, says nothing of the cell's others)
+    auto lower = [=](float v, float side) { return side != side ? -inf : fminf(v, side); };
+    auto higher = [=](float v, float side) { return side != side ? inf : fmaxf(v, side); };
     for (int c = r * NG_RUN; c < ccells && c < (r + 1) * NG_RUN; ++c)
     {
-        const float4 a = cbox[c * NG_BOX + 0], b = cbox[c * NG_BOX + 1]; // (an empty cell: lo = +inf, hi = -inf)
-        lo = make_float4(fminf(lo.x, a.x), fminf(lo.y, a.y), fminf(lo.z, a.z), 0.f);
-        hi = make_float4(fmaxf(hi.x, b.x), fmaxf(hi.y, b.y), fmaxf(hi.z, b.z), 0.f);
+        const float4 a = cbox[c * NG_BOX + 0], b = cbox[c * NG_BOX + 1];
+        lo = make_float4(lower(lo.x, a.x), lower(lo.y, a.y), lower(lo.z, a.z), 0.f);
+        hi = make_float4(higher(hi.x, b.x), higher(hi.y, b.y), higher(hi.z, b.z), 0.f);
     }
     run_boxes[t * 2 + 0] = lo;
     run_boxes[t * 2 + 1] = hi;
