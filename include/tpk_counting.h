@@ -1,5 +1,5 @@
 /*
- * tpk_counting.h - the two extra entry points of libtpk_hip_counting.so.
+ * tpk_counting.h - the three extra entry points of libtpk_hip_counting.so.
  *
  * libtpk_hip_counting.so is libtpk_hip.so (same sources, same C ABI: tpk.h) with the distance
  * scans compiled -DTPK_COUNT_WORK: furthest point sampling, the ball queries, three_nn and the
@@ -14,6 +14,8 @@
 #ifndef TPK_COUNTING_H
 #define TPK_COUNTING_H
 
+#include <stdint.h>
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -24,6 +26,11 @@ int tpk_work_read_reset(unsigned long long* pairs);
 
 /* The same, and in *products the pairs formed by matrix products since the last call of either. */
 int tpk_work_read_reset_both(unsigned long long* pairs, unsigned long long* products);
+
+/* `count` (at most 2^20) products of 32 x 16 halves by 16 x 32 on the matrix cores, for a test of the error that Chamfer's search
+ * allows them: of product i, a holds row r's slots 8 h .. 8 h + 7 as its vector of 8 halves number 64 i + 32 h + r, b column c's
+ * likewise (16-byte aligned), d (count, 32, 32) the float32 sums. */
+int tpk_matrix_product(int64_t count, const void* a, const void* b, float* d, void* stream);
 
 #ifdef __cplusplus
 }

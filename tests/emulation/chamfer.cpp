@@ -12,7 +12,7 @@ int main(int argc, char** argv)
     const int b = atoi(argv[1]), n = atoi(argv[2]), m = atoi(argv[3]);
     const std::string kind = argv[4];
     report_accesses_out_of_bounds();
-    emulation::product_error = 0x1p-22;
+    emulation::product_error = 14 * 0x1p-24;
     std::mt19937 random(atoi(argv[5]));
     std::uniform_real_distribution<float> even(0.f, 1.f);
     std::normal_distribution<float> normal(0.f, 1.f);

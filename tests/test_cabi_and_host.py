@@ -91,11 +91,12 @@ def test_counting_build_exports_the_same_abi_plus_its_reader():
     path = LIB.replace("libtpk_hip.so", "libtpk_hip_counting.so")
     assert os.path.exists(path), "libtpk_hip_counting.so is not built (run torch-points-kernels_amd/build.py)"
     lib = ctypes.CDLL(path)
-    for name in _declared_symbols() + ["tpk_work_read_reset", "tpk_work_read_reset_both"]:
+    extra = ["tpk_work_read_reset", "tpk_work_read_reset_both", "tpk_matrix_product"]
+    for name in _declared_symbols() + extra:
         assert hasattr(lib, name), name
-    assert not hasattr(ctypes.CDLL(LIB), "tpk_work_read_reset")
+    assert not any(hasattr(ctypes.CDLL(LIB), name) for name in extra)
     text = open(os.path.join(ROOT, "include", "tpk_counting.h")).read()
-    assert "tpk_work_read_reset" in text and "tpk_work_read_reset_both" in text
+    assert all(name in text for name in extra)
 
 
 def test_library_exports_every_declared_symbol():

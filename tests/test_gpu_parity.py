@@ -3037,6 +3037,51 @@ def test_counting_build_counts_matrix_products_by_themselves(dev):
     assert pairs.value == 0 and products.value == 0
 
 
+@pytest.mark.parametrize("kind", ["even", "magnitudes", "as the search has them", "below the normal range", "just cut off"])
+def test_matrix_products_err_as_little_as_chamfers_bound_assumes(dev, kind):
+    """14 x 2^-24 of the sum of the products' magnitudes, and halves below the normal range count: what the search's bound takes the matrix
+    cores to do (its host run errs by as much).  float64 holds every product and, for the comparison, every sum."""
+    import ctypes
+    import os
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(root, "torch-points-kernels_amd", "torch_points_kernels", "libtpk_hip_counting.so"))
+    g = torch.Generator().manual_seed(11)
+    count = 1024
+    a, b = (torch.randn(count, 32, 16, generator=g) for _ in range(2))
+    if kind == "magnitudes":
+        a, b = (v * torch.exp2(torch.rand(v.shape, generator=g) * 26 - 13) for v in (a, b))
+    elif kind == "as the search has them":  # a point's high halves, low halves 2^-11 of them, squares; nearly cancelling sums
+        p, q = (1000 * (torch.rand(count, 32, 3, generator=g) - 0.5) for _ in range(2))
+        q = torch.where(torch.rand(count, 32, 1, generator=g) < 0.5, p + torch.randn(p.shape, generator=g), q)
+        high = lambda v: v.half().float()
+        low = lambda v: (v - high(v)).half().float()
+        sq = lambda v: (v * v).sum(2, keepdim=True) / 16384
+        far = torch.full((count, 32, 2), 16384.0)
+        nought = torch.zeros(count, 32, 1)
+        xy, z, xy2, z2 = p[..., :2], p[..., 2:], -2 * q[..., :2], -2 * q[..., 2:]
+        a = torch.cat([high(xy), low(xy), high(z), high(sq(p)), low(z), low(sq(p)), high(xy), low(xy), high(z), high(sq(p)), far], 2)
+        b = torch.cat([high(xy2), high(xy2), high(z2), far[..., :1], high(z2), far[..., :1], low(xy2), low(xy2), low(z2), nought, high(sq(q)), low(sq(q))], 2)
+    elif kind == "below the normal range":
+        a = torch.randint(-1023, 1024, a.shape, generator=g) * 2.0**-24
+    elif kind == "just cut off":  # one or two large terms, the others about 2^-24 of them, of both signs: the largest error found
+        order = torch.argsort(torch.rand(count, 1, 16, generator=g), 2)
+        large = (order < torch.randint(1, 3, (count, 1, 1), generator=g)).expand(-1, 32, -1)
+        sign = torch.where(torch.rand(a.shape, generator=g) < 0.5, -1.0, 1.0)
+        small = 1.9990234375 * torch.exp2(12.0 - torch.randint(23, 26, a.shape, generator=g))
+        a, b = sign * torch.where(large, torch.ones(()), small), torch.where(large, 1.0, 2.0**-12)
+    a, b = a.half(), b.half()
+    assert torch.isfinite(a).all() and torch.isfinite(b).all()
+    lanes = lambda v: v.view(count, 32, 2, 8).transpose(1, 2).contiguous().to(dev)  # halves of the slots, then rows
+    da, db, d = lanes(a), lanes(b), torch.empty(count, 32, 32, device=dev)
+    st = lib.tpk_matrix_product(ctypes.c_int64(count), ctypes.c_void_p(da.data_ptr()), ctypes.c_void_p(db.data_ptr()), ctypes.c_void_p(d.data_ptr()), None)
+    assert st == 0
+    torch.cuda.synchronize()
+    terms = a.double()[:, :, None, :] * b.double()[:, None, :, :]
+    error = (d.cpu().double() - terms.sum(3)).abs()
+    assert (error <= 14 * 2.0**-24 * terms.abs().sum(3)).all(), float((error / terms.abs().sum(3).clamp_min(1e-300)).max())
+
+
 def _knn_steps(oracle, dev, support, query, k, workspace="grid"):
     """Steps of 64 points per query that the counting build takes; the answers are checked on the way.  workspace: the size the
     grid in memory wants, or the one for curve-ordered cells."""

@@ -151,16 +151,22 @@ __device__ __forceinline__ void scan_cell_few(const float4* __restrict__ cand, i
 // the queries' box and scaled by a power of two; in these units everything the search needs lies within 1024 of the
 // centre along every axis, and candidates further off than 16384 count as that far away.
 //
-// A row of the product: x, y (high halves), x, y (low), z, |p|^2 (high), z, |p|^2 (low), then x, y (high), x, y (low), z, |p|^2
-// (high), 1, 1 against a query's -2x, -2y (high, twice), (-2z, 2^14) (high, twice), -2x, -2y (low, twice), (-2z, 0) (low), |q|^2.
+// A candidate's row of the product: x, y (high halves), x, y (low), z, |p|^2 (high), z, |p|^2 (low), then x, y (high), x, y (low), z, |p|^2
+// (high), 2^14, 2^14; against a query's -2x, -2y (high, twice), (-2z, 2^14) (high, twice), -2x, -2y (low, twice), (-2z, 0) (low), |q|^2 (high, low).
+// The squares are kept divided by 2^14.
 //
 // The error of a product, in units of 2^-20 (|p| + |q|)^2: two halves hold 22 bits, which costs 2 p.q 0.38 and the squares, formed in
-// float, 0.44; the frame 0.2; the sum of 16 products 0.25 (2^-22 of the sum of their magnitudes: twice the 2^-23.05 that a million
-// products reached, and halves below the normal range are not flushed).  With the two bits that a smallest product gives up for
-// its place that is below 2^-17 (|q|^2 + |p - q|^2), as (|p| + |q|)^2 <= 5 |q|^2 + 5 |p - q|^2, and 2^-6 where a low half is below the normal
-// range.  A query for which the eight and some other candidate are closer together than that (of 32 x 16384 points one in 3600 of even clouds, one
-// in 1200 on a sphere) goes to the pass for equal minima; where many of a wavefront's do, the exact scan above answers them, a search of
-// its own that starts with what is known: serving 64 of them one at a time took 2.8 times as long on clouds with outliers.
+// float, 0.44; the frame 0.13; the sum of 16 products 0.88, 14 x 2^-24 of the sum of their magnitudes.  (Terms are cut off at about 2^-24 of the
+// largest: random sums are off by up to 2.3 of these 14, sums made for it - one large term, the others just below the cut, of both signs - by 9.)
+// As (|p| + |q|)^2 <= 4.4 |q|^2 + 11 |p - q|^2, that is 1.82 x 2^-20 times it: below MX_ERROR of |q|^2 and, with 0.4 for the two bits that a smallest
+// product gives up for its place and 0.3 for the rounding of the distances themselves, MX_ERROR_NEAR of |p - q|^2.  Where a low half is below the
+// normal range the products are off by less than 2^-8 more (2^-25 of a slot, against at most 2 x 1100 or 2^14); 2^-4 is allowed for it.
+// What the unit's sums are off by, and that halves below the normal range count, is not documented but measured, and tested on the device
+// (tpk_matrix_product, counting build); the search is run on the host with sums that far off.
+//
+// A query for which the eight and some other candidate are closer together than that (of 32 x 16384 points one in 3200 of even clouds, one in
+// 1200 on a sphere) goes to the pass for equal minima; where many of a wavefront's do, the exact scan above answers
+// them, a search of its own that starts with what is known: serving 64 of them one at a time took 2.8 times as long on clouds with outliers.
 //
 // What bounds it: the issue of vector instructions, ~105 for 64 x 64 pairs (22 to form the halves, 60 for the minima) where the
 // exact scan takes ten per candidate.  32 x 16384 points of noisy surfaces: search 121 -> 58 us, whole call 144 -> 86; uniform 143 -> 98, eight
@@ -175,7 +181,8 @@ typedef unsigned uint4_t __attribute__((vector_size(16)));
 constexpr float MX_FAR = 16384.f;          // 2^14: candidates are clamped to this; also the factor |p|^2 and |q|^2 are kept divided by
 constexpr float MX_LIMIT = 134217728.f;    // 2^27: a squared distance that no clamped candidate can have
 constexpr float MX_NEAR = 8.f;             // largest distance of the first cell, in extents of its box and the queries'
-constexpr float MX_ERROR = 0x1p-17f;       // of |q|^2 and of a product (above)
+constexpr float MX_ERROR = 0x1p-17f;       // of |q|^2, 8 x 2^-20 (above)
+constexpr float MX_ERROR_NEAR = 0x1.8p-16f; // and of a product, 24 x 2^-20
 // Who answers the queries that the products cannot: the pass for equal minima costs a query a look at all boxes and at the cells within its
 // reach, the exact scan costs a wavefront its whole search again.  us, before the matrix cores / products with an exact scan of more than 20 queries,
 // whatever the search was like / as here.
@@ -256,6 +263,19 @@ __device__ __forceinline__ void take_products(const float16_t& d, int tile, Matr
     // registers beyond the scan, 32 of them)
     asm volatile("" : "+v"(s.m2));
 }
+
+#ifdef TPK_COUNT_WORK
+// One product per wavefront, for a test of what the bound above assumes of the unit.
+__global__ __launch_bounds__(TPK_WAVE) void matrix_product_kernel(const uint4* __restrict__ a, const uint4* __restrict__ b, float* __restrict__ d)
+{
+    const int lane = threadIdx.x;
+    const int64_t at = static_cast<int64_t>(blockIdx.x) * TPK_WAVE + lane;
+    const float16_t sums = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a[at]), __builtin_bit_cast(half8_t, b[at]), float16_t{}, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        d[(static_cast<int64_t>(blockIdx.x) * 32 + r % 4 + 8 * (r / 4) + 4 * (lane / 32)) * 32 + lane % 32] = sums[r];
+}
+#endif
 
 // Units of a wavefront's search: point * scale + offset.
 struct MatrixFrame
@@ -460,7 +480,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         const float square = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z));
         const float own_error = __builtin_fmaf(square, MX_ERROR, 0.0625f);
         const float unit = 1.f / (frame.scale * frame.scale);
-        const float reach_factor = (1.f + MX_ERROR) * unit, reach_error = own_error * unit;
+        const float reach_factor = (1.f + MX_ERROR_NEAR) * unit, reach_error = own_error * unit;
         half8_t queries[2];
         {
             half2_t xy_high, xy_low, z_high, z_low, s_high, s_low;
@@ -491,7 +511,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
             by_query(near[0].m2, near[1].m2, a2, b2);
             return __int_as_float(min(min(a2, b2), max(a, b)));
         };
-        auto clear = [&](float second) { return second > m + 2.f * __builtin_fmaf(m, MX_ERROR, own_error) && m < MX_LIMIT; };
+        auto clear = [&](float second) { return second > m + 2.f * __builtin_fmaf(m, MX_ERROR_NEAR, own_error) && m < MX_LIMIT; };
         // Where the first cell's second smallest products are near the error already, or near the smallest, the search would leave the queries
         // over.  (A wavefront that shares its cell has half of the queries at most and keeps to the first test: it would give few back.)
         float m2 = second_smallest();
@@ -628,7 +648,7 @@ __global__ __launch_bounds__(NG_SCAN_THREADS, 8) void chamfer_grid_kernel(
         tie = tie || (ask && s.tie);
     }
     // Several groups reached a query's minimum (about one query in 10^5 on random clouds, every query on a lattice), or
-    // came too close to it for the products to tell (one in 10^3 to 10^4): the nearest candidate, of several the one of lowest index,
+    // came too close to it for the products to tell (one in 1200 to 5500): the nearest candidate, of several the one of lowest index,
     // over all cells within reach.  One such query at a time: the lanes test the boxes of all cells side by side, then the
     // candidates of every cell that passes.
     for (unsigned long long tied = __ballot(tie); tied != 0; tied &= tied - 1)
@@ -1483,6 +1503,21 @@ bool grid_supported(int b, int n, int m)
 }
 
 } // namespace
+
+#ifdef TPK_COUNT_WORK
+extern "C" int tpk_matrix_product(int64_t count, const void* a, const void* b, float* d, void* stream)
+{
+    if (count < 0 || (count > 0 && (!a || !b || !d)))
+        return TPK_ERR_INVALID_ARG;
+    if (count == 0)
+        return TPK_OK;
+    if (count > (1 << 20) || ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u))
+        return TPK_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(matrix_product_kernel, dim3(static_cast<unsigned>(count)), dim3(TPK_WAVE), 0, tpk_stream(stream),
+                       static_cast<const uint4*>(a), static_cast<const uint4*>(b), d);
+    return tpk_launch_status();
+}
+#endif
 
 size_t tpk_grid_chamfer_workspace_bytes(int b, int n, int m)
 {
