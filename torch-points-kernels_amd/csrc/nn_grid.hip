@@ -169,8 +169,8 @@ __device__ __forceinline__ void scan_cell_few(const float4* __restrict__ cand, i
 // them, a search of its own that starts with what is known: serving 64 of them one at a time took 2.8 times as long on clouds with outliers.
 //
 // What bounds it: the issue of vector instructions, ~105 for 64 x 64 pairs (22 to form the halves, 60 for the minima) where the
-// exact scan takes ten per candidate.  32 x 16384 points of noisy surfaces: search 121 -> 58 us, whole call 144 -> 86; uniform 143 -> 98, eight
-// clusters 176 -> 89; 8 x 1024 against 16384 109 -> 53, 2 x 60000 159 -> 102, one cloud of 160000 455 -> 281.
+// exact scan takes ten per candidate.  32 x 16384 points, forward, with the ordering: a noisy sphere 116 -> 80 us (surfaces, with what else a
+// pass does 122 -> 65 for the search alone), uniform 140 -> 98, eight clusters 182 -> 94; 2 x 60000 uniform 154 -> 101.
 // Taken back: minima of four candidates (24 more instructions per scan, 12 % slower), whole wavefronts by the exact scan where many
 // queries are left over (laser scans 30 % slower than without the matrix cores).
 typedef _Float16 half2_t __attribute__((vector_size(4)));
