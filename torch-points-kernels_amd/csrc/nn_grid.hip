@@ -195,7 +195,8 @@ constexpr float MX_ERROR_NEAR = 0x1.8p-16f; // and of a product, 24 x 2^-20
 //   wavefronts, blind or not: 670 and 1640, but clouds with outliers 2 x 60000 2900 instead of 2690.)
 // The reach of those left over ends at the best of their eight: clouds with outliers 32 x 4096 270 / 232 / 213, scaled point by point by e^0 .. e^-12
 // 8 x 16384 890 / 960 / 933.  Still behind the search without products: these, twins, lines, and outliers in small calls (8 x 8192 on 2048 327 / 390 / 387).
-// Taken back: giving up inside the overlapping cells (outliers and lines 5 to 10 % faster, every call 3 %, by what each scan has to keep).
+// Taken back: giving up inside the overlapping cells, after 8, 16, 32 .. scans (outliers and lines 5 to 10 % faster, every call 3 % slower, by what each
+// scan has to keep) or between groups of 64 cells (a line 2 x 60000 480 -> 439, outliers 2 x 16384 695 -> 623, every call 1 % slower).
 constexpr float MX_CLOSE = 16.f;
 constexpr int MX_MANY = 8;                 // (of 64; 16: twins 156, line 171)
 constexpr int MX_MOST = 32;
